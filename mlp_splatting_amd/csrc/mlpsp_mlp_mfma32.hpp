@@ -122,39 +122,94 @@ __device__ __forceinline__ void request_layer2(const float* __restrict__ W2, con
   }
 }
 
-// max(x, +0): v_max_f32 yields the same bits as x > 0 ? x : 0 for every x (NaN -> 0, -0 -> +0).  Written
-// as a builtin, not as inline assembly: the compiler must see the instruction to keep the wait states
-// between a matrix-core result and its first reader.
-__device__ __forceinline__ float relu_f32(float x) { return __builtin_fmaxf(x, 0.f); }
+// max(x, +0): the same bits as x > 0 ? x : 0 for every x (NaN -> 0, -0 -> +0).  v_med3_f32 with 0 and +inf is one
+// instruction; fmaxf() is two, because the compiler quiets a possible signalling NaN first (128 of the 1,150 vector
+// instructions of a hit step).  The infinity is hidden from the compiler, which would turn a median with it into that
+// maximum.  A builtin, not inline assembly: the compiler must see the instruction to keep the wait states between a
+// matrix-core result and its first reader.
+__device__ __forceinline__ float relu_limit() {
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return inf;
+}
+__device__ __forceinline__ float relu_f32(float x, float inf) { return __builtin_amdgcn_fmed3f(x, 0.f, inf); }
 
-// The encoding of the ray direction (input components 0..2) does not depend on the primitive: its 18
-// sin/cos pairs are computed once per pixel and kept in B-operand position (after the half-wave swap).
-struct DirOperands {
-  float b0[18], b1[18];
-};
-__device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz, const float* __restrict__ freq,
-                                                 const float* __restrict__ att, DirOperands& d) {
-  const float x3[3] = {rdx, rdy, rdz};
+// det_sincos() for |x| <= 65536, the same bits: no range check, the quadrant's signs by exclusive-or.
+__device__ __forceinline__ void det_sincos_in_range(float x, float& s_out, float& c_out) {
+  const float kf = __builtin_rintf(x * 0.636619772f);
+  float r = fmaf(kf, -1.5703125f, x);
+  r = fmaf(kf, -4.83751297e-04f, r);
+  r = fmaf(kf, -7.54978995e-08f, r);
+  const float z = r * r;
+  float ps = 2.75573192e-06f;
+  ps = fmaf(ps, z, -1.98412698e-04f);
+  ps = fmaf(ps, z, 8.33333333e-03f);
+  ps = fmaf(ps, z, -1.66666667e-01f);
+  const float s = fmaf(r * z, ps, r);
+  float pc = -2.75573192e-07f;
+  pc = fmaf(pc, z, 2.48015873e-05f);
+  pc = fmaf(pc, z, -1.38888889e-03f);
+  pc = fmaf(pc, z, 4.16666667e-02f);
+  const float c = fmaf(z * z, pc, fmaf(z, -0.5f, 1.0f));
+  const uint32_t q = (uint32_t)(int)kf;
+  const bool odd = (q & 1u) != 0u;
+  const uint32_t turn = q << 30;             // bit 31: the sine's sign; one more quarter turn: the cosine's
+  s_out = bits_to_float(float_to_bits(odd ? c : s) ^ (turn & 0x80000000u));
+  c_out = bits_to_float(float_to_bits(odd ? s : c) ^ ((turn + 0x40000000u) & 0x80000000u));
+}
+// The six (sin, cos) pairs of one input component, bit for bit det_sincos((x freq_f) att_f).  One test covers the
+// range of all six (a NaN fails it too); phases beyond it, which no scene has in earnest, are put right behind a branch
+// that the whole wavefront skips.
+__device__ __forceinline__ void encode_component(float x, const float* __restrict__ freq, const float* __restrict__ att,
+                                                 float s[6], float c[6]) {
+  float phase[6];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
+  for (int f = 0; f < 6; ++f) phase[f] = (x * freq[f]) * att[f];
+  const float reach = ((__builtin_fabsf(phase[0]) + __builtin_fabsf(phase[1])) +
+                       (__builtin_fabsf(phase[2]) + __builtin_fabsf(phase[3]))) +
+                      (__builtin_fabsf(phase[4]) + __builtin_fabsf(phase[5]));
+#pragma unroll
+  for (int f = 0; f < 6; ++f) det_sincos_in_range(phase[f], s[f], c[f]);
+  if (__ballot(!(reach <= 65536.0f)) != 0ull) {
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
-      float s, co;
-      det_sincos((x3[c] * freq[f]) * att[f], s, co);
-      half_swap(s, co);
-      d.b0[c * 6 + f] = s;
-      d.b1[c * 6 + f] = co;
+      float again = x;                       // (or the six comparisons are made ahead of the branch)
+      asm volatile("" : "+v"(again));
+      const bool ok = __builtin_fabsf((again * freq[f]) * att[f]) <= 65536.0f;
+      s[f] = ok ? s[f] : __builtin_nanf("");
+      c[f] = ok ? c[f] : __builtin_nanf("");
     }
   }
 }
 
+// The encoding of the ray direction (input components 0..2) does not depend on the primitive: its 18 sin/cos pairs are
+// computed once per pixel and parked in LDS in B-operand position (after the half-wave swap), four instructions' worth
+// per 16-byte read.  Written and read by one wavefront: no barrier.  (36 registers less than keeping them: a fourth
+// wavefront per SIMD.)
+struct DirOperands {
+  mf32x4 q[9][64];       // [i]: blocks 0 and 1 of pairs 2i and 2i + 1 = (b0[2i], b1[2i], b0[2i+1], b1[2i+1])
+};
+__device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz, const float* __restrict__ freq,
+                                                 const float* __restrict__ att, DirOperands& d) {
+  const int lane = threadIdx.x & 63;
+  const float x3[3] = {rdx, rdy, rdz};
+  for (int c = 0; c < 3; ++c) {
+    float s[6], co[6];
+    encode_component(c == 0 ? x3[0] : c == 1 ? x3[1] : x3[2], freq, att, s, co);
+#pragma unroll
+    for (int f = 0; f < 6; ++f) half_swap(s[f], co[f]);
+#pragma unroll
+    for (int f = 0; f < 6; f += 2) d.q[3 * c + f / 2][lane] = mf32x4{s[f], co[f], s[f + 1], co[f + 1]};
+  }
+}
+
 // All 64 lanes must be active.  x6 is the lane's own pixel's input (components 0..2 enter through dir,
-// which encode_direction() made from them); out is the lane's own pixel's output.  `w1`, `w2` = the primitive's
-// operands as request_layer1() and request_layer2() loaded them.
+// which encode_direction() made from them); out is the lane's own pixel's output.  `w1` = the primitive's layer-1
+// operands as request_layer1() loaded them; layer2(w2) requests those of layer 2.
 // REC selects the record kernels' layer-2 rounding (bias added after a chain started at zero); MASKS fills
 // masks[0..1] with the ReLU masks of the lane's pixel.
-template <bool REC = false, bool MASKS = REC, int HID = 32>
-__device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, const MlpLayer2<HID>& w2, const float x6[6],
+template <bool REC = false, bool MASKS = REC, int HID = 32, typename RequestLayer2>
+__device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, RequestLayer2&& layer2, const float x6[6],
                                                      const float* __restrict__ freq, const float* __restrict__ att,
                                                      const float* __restrict__ W3, const float* __restrict__ b3, int p,
                                                      const DirOperands& dir, float out[4], uint32_t* masks = nullptr) {
@@ -162,6 +217,7 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, c
   constexpr int H = HID, R = H / 2;   // R: accumulator registers in use (hidden units 2i + g)
   const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
   const bool row_used = mfma32_hidden_row(m) < H;          // (always, with 32 hidden units)
+  const float inf = relu_limit();
 
   // A operands: lane (m, g) supplies row hid, k = g of every instruction.
   float a1[36];
@@ -172,42 +228,53 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, c
     a1[4 * q + 2] = row_used ? w1.a1[q][2] : 0.f;
     a1[4 * q + 3] = row_used ? w1.a1[q][3] : 0.f;
   }
-  float a2[16] = {}, bias1[16] = {}, bias2[16] = {};
-  interleave<H>(w2.a2, a2);
+  float bias1[16] = {};
   interleave<H>(w1.b1, bias1);
-  interleave<H>(w2.b2, bias2);
-  if constexpr (H != 32) {
-#pragma unroll
-    for (int i = 0; i < R; ++i) a2[i] = row_used ? a2[i] : 0.f;
-  }
 
   mf32x16 d0, d1;
 #pragma unroll
   for (int i = 0; i < 16; ++i) d0[i] = d1[i] = (i < R) ? bias1[i] : 0.f;
+  // (the lane index is made opaque so that the reads stay here and are not hoisted out of the primitive loop)
+  int ll = lane;
+  asm volatile("" : "+v"(ll));
 #pragma unroll
-  for (int j = 0; j < 18; ++j) {
-    d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], dir.b0[j], d0, 0, 0, 0);
-    d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], dir.b1[j], d1, 0, 0, 0);
+  for (int i = 0; i < 9; ++i) {
+    const mf32x4 q = dir.q[i][ll];
+    d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i], q[0], d0, 0, 0, 0);
+    d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i], q[1], d1, 0, 0, 0);
+    d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i + 1], q[2], d0, 0, 0, 0);
+    d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i + 1], q[3], d1, 0, 0, 0);
   }
+  MlpLayer2<HID> w2;
 #pragma unroll
   for (int c = 3; c < 6; ++c) {
+    // (layer 2's operands are requested behind five sixths of layer 1, and not before: 32 registers)
+    if (c == 5) layer2(w2);
+    float sn[6], cs[6];
+    encode_component(x6[c], freq, att, sn, cs);
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
-      float s, co;
-      det_sincos((x6[c] * freq[f]) * att[f], s, co);
+      float s = sn[f], co = cs[f];
       half_swap(s, co);   // s: (sin, cos) of pixels 0..31, co: (sin, cos) of pixels 32..63
       d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[c * 6 + f], s, d0, 0, 0, 0);
       d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[c * 6 + f], co, d1, 0, 0, 0);
     }
   }
 
+  float a2[16] = {}, bias2[16] = {};
+  interleave<H>(w2.a2, a2);
+  interleave<H>(w2.b2, bias2);
+  if constexpr (H != 32) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) a2[i] = row_used ? a2[i] : 0.f;
+  }
   mf32x16 e0, e1;
 #pragma unroll
   for (int i = 0; i < 16; ++i) e0[i] = e1[i] = (REC || i >= R) ? 0.f : bias2[i];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    e0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d0[i]), e0, 0, 0, 0);
-    e1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d1[i]), e1, 0, 0, 0);
+    e0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d0[i], inf), e0, 0, 0, 0);
+    e1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d1[i], inf), e1, 0, 0, 0);
   }
   if constexpr (REC) {
 #pragma unroll
@@ -224,7 +291,7 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, c
   uint32_t m2 = 0u;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    float even = relu_f32(e0[i]), odd = relu_f32(e1[i]);
+    float even = relu_f32(e0[i], inf), odd = relu_f32(e1[i], inf);
     half_swap(even, odd);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -278,6 +345,7 @@ __device__ __forceinline__ void mlp_half_mfma32_with(const MlpLayer1<HID>& w1, c
   constexpr int H = HID, R = H / 2;
   const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
   const bool row_used = mfma32_hidden_row(m) < H;
+  const float inf = relu_limit();
   float a1[36];
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
@@ -301,18 +369,18 @@ __device__ __forceinline__ void mlp_half_mfma32_with(const MlpLayer1<HID>& w1, c
   for (int j = 0; j < 18; ++j) d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], dir[j], d, 0, 0, 0);
 #pragma unroll
   for (int c = 3; c < 6; ++c) {
+    float sn[6], cs[6];
+    encode_component(x6[c], freq, att, sn, cs);
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
-      float s, co;
-      det_sincos((x6[c] * freq[f]) * att[f], s, co);
-      d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[c * 6 + f], g ? co : s, d, 0, 0, 0);
+      d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[c * 6 + f], g ? cs[f] : sn[f], d, 0, 0, 0);
     }
   }
   mf32x16 e;
 #pragma unroll
   for (int i = 0; i < 16; ++i) e[i] = (i >= R) ? 0.f : bias2[i];
 #pragma unroll
-  for (int i = 0; i < R; ++i) e = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d[i]), e, 0, 0, 0);
+  for (int i = 0; i < R; ++i) e = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d[i], inf), e, 0, 0, 0);
 
   const float* __restrict__ w3 = W3 + (size_t)p * (4 * H);
   const float* __restrict__ bb3 = b3 + (size_t)p * 4;
@@ -321,7 +389,7 @@ __device__ __forceinline__ void mlp_half_mfma32_with(const MlpLayer1<HID>& w1, c
   for (int i = 0; i < R; ++i) {
     // register i of lane (n, g) is hidden unit 2i + g of pixel n: after the swap `even` holds the g = 0 lane's
     // value and `odd` the g = 1 lane's, on both lanes
-    float even = relu_f32(e[i]), odd = even;
+    float even = relu_f32(e[i], inf), odd = even;
     half_swap(even, odd);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -342,10 +410,12 @@ __device__ __forceinline__ void mlp_wave_mfma32(const float x6[6], const float* 
                                                 const float* __restrict__ b3, int p, const DirOperands& dir,
                                                 float out[4], uint32_t* masks = nullptr) {
   MlpLayer1<HID> w1;
-  MlpLayer2<HID> w2;
   request_layer1<HID>(W1, b1, p, w1);
-  request_layer2<HID>(W2, b2, p, w2);
-  mlp_wave_mfma32_with<REC, MASKS, HID>(w1, w2, x6, freq, att, W3, b3, p, dir, out, masks);
+  const auto layer2 = [&](MlpLayer2<HID>& w2) {
+    __builtin_amdgcn_sched_barrier(0);
+    request_layer2<HID>(W2, b2, p, w2);
+  };
+  mlp_wave_mfma32_with<REC, MASKS, HID>(w1, layer2, x6, freq, att, W3, b3, p, dir, out, masks);
 }
 
 }  // namespace mlpsp

@@ -10,6 +10,7 @@
 #include "mlpsp_mlp_mfma32.hpp"
 #include "mlpsp_render_f32.hpp"
 #include "mlpsp_record_stage.hpp"
+#include <type_traits>
 
 // records of a pixel staged in LDS before they are written (mlpsp_record_stage.hpp); 8x8 tiles on the matrix-core
 // path only -- the scalar shapes keep the direct stores
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(64) void records_kernel(
   float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
   int used = 0;
   bool over = false;
-  DirOperands dir;
+  __shared__ typename std::conditional<MF, DirOperands, char>::type dir;
   if constexpr (MF) encode_direction(rdx, rdy, rdz, freq, att, dir);
   for (int i = start; i < end; ++i) {
     const int p = __builtin_amdgcn_readfirstlane(order[i]);

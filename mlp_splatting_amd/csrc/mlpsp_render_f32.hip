@@ -47,6 +47,12 @@ MLPSP_API int mlpsp_render_tilecenter_f32(const float* rays_o_dev, const float* 
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,         \
                      num_frequencies, W1, b1, W2, b2, W3, b3, num_primitives, hidden, g, wpt, per_xcd, (int)items, threshold,           \
                      out_rgb_dev, out_alpha_dev, out_t_dev, ctr, 0.f, 0.f, HitPool{})
+#define MLPSP_F32_MF_LAUNCH(HT)                                                                                   \
+  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<HT, 0>), dim3(f32_mf_grid(g, wpt)), block, 0, s, rays_o_dev,  \
+                     rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev,        \
+                     att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, \
+                     out_t_dev, ctr, 0.f, 0.f, HitPool{}, (const float*)nullptr, (float*)nullptr, (float*)nullptr,   \
+                     (int32_t*)nullptr, (float*)nullptr, (int32_t*)nullptr)
 #define MLPSP_F32_AHEAD_LAUNCH(HT, HALF, UNITS)                                                                   \
   hipLaunchKernelGGL((render_tilecenter_f32_ahead_kernel<HT, HALF>), dim3((unsigned)(ceil_div_units(UNITS) * kNumXcd)), block, 0, s, \
                      rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev,    \
@@ -61,13 +67,14 @@ MLPSP_API int mlpsp_render_tilecenter_f32(const float* rays_o_dev, const float* 
     } else if (mode == 1) {
       if (hidden == 32) MLPSP_F32_AHEAD_LAUNCH(32, false, items);
       else MLPSP_F32_AHEAD_LAUNCH(16, false, items);
-    } else if (hidden == 32) MLPSP_F32_LAUNCH(32, 6, false, true);
-    else MLPSP_F32_LAUNCH(16, 6, false, true);
+    } else if (hidden == 32) MLPSP_F32_MF_LAUNCH(32);
+    else MLPSP_F32_MF_LAUNCH(16);
   }
   else if (hidden == 32 && num_frequencies == 6) MLPSP_F32_LAUNCH(32, 6);
   else if (hidden == 16 && num_frequencies == 6) MLPSP_F32_LAUNCH(16, 6);
   else MLPSP_F32_LAUNCH(0, 0);
 #undef MLPSP_F32_AHEAD_LAUNCH
+#undef MLPSP_F32_MF_LAUNCH
 #undef MLPSP_F32_LAUNCH
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
@@ -107,13 +114,20 @@ MLPSP_API int mlpsp_render_tilecenter_stats_f32(const float* rays_o_dev, const f
                      (int)items, threshold, out_rgb_dev, out_alpha_dev, (float*)nullptr,                         \
                      (unsigned long long*)nullptr, 0.f, 0.f, HitPool{}, gt_rgb_dev, stat_sum_w_dev,              \
                      stat_max_w_dev, stat_hits_dev, stat_sum_werr_dev, stat_contrib_dev)
+#define MLPSP_STATS_MF_LAUNCH(HT)                                                                                \
+  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<HT, 0, true>), dim3(f32_mf_grid(g, wpt)), block, 0, s,       \
+                     rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev,     \
+                     freq_dev, att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev,    \
+                     out_alpha_dev, (float*)nullptr, (unsigned long long*)nullptr, 0.f, 0.f, HitPool{}, gt_rgb_dev, \
+                     stat_sum_w_dev, stat_max_w_dev, stat_hits_dev, stat_sum_werr_dev, stat_contrib_dev)
   if (use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    if (hidden == 32) MLPSP_STATS_LAUNCH(32, 6, true);
-    else MLPSP_STATS_LAUNCH(16, 6, true);
+    if (hidden == 32) MLPSP_STATS_MF_LAUNCH(32);
+    else MLPSP_STATS_MF_LAUNCH(16);
   }
   else if (hidden == 32 && num_frequencies == 6) MLPSP_STATS_LAUNCH(32, 6);
   else if (hidden == 16 && num_frequencies == 6) MLPSP_STATS_LAUNCH(16, 6);
   else MLPSP_STATS_LAUNCH(0, 0);
+#undef MLPSP_STATS_MF_LAUNCH
 #undef MLPSP_STATS_LAUNCH
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;

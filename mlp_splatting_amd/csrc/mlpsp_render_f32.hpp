@@ -7,6 +7,7 @@
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
+#include "mlpsp_walk_f32.hpp"
 
 namespace mlpsp {
 
@@ -29,9 +30,8 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// MF: the 72->32->32->4 MLP runs on the matrix cores for all 64 pixels at once (mlp_wave_mfma32, same bits);
-// requires HT == 32 or 16, FT == 6 and 16-byte aligned weight arrays.
-template <int HT, int FT, int EMIT, bool STATS = false, bool MF = false>
+// This kernel evaluates the MLP on the vector ALU (shapes and alignments the matrix-core kernel below does not take).
+template <int HT, int FT, int EMIT, bool STATS = false>
 __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
@@ -78,8 +78,6 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
     }
   }
   HitEmitter em = hit_emitter_begin(hp, wslot, start, tile);
-  DirOperands dir;
-  if constexpr (MF) encode_direction(rdx, rdy, rdz, freq, att, dir);
 
   for (int i = start; i < end; ++i) {
     const int p = __builtin_amdgcn_readfirstlane(order[i]);
@@ -97,12 +95,10 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
       float w_stat = 0.f;
       if constexpr (EMIT > 0) rs = hit_emitter_next(hp, em, (int)threadIdx.x);
       float* __restrict__ rec = reinterpret_cast<float*>(hp.records + (size_t)(rs < 0 ? 0 : rs) * hp.record_bytes);
-      // (lanes that did not hit carry no hit point; the matrix-core evaluation runs on all 64 lanes)
-      const float x6[6] = {rdx, rdy, rdz, hit ? h.dx : 0.f, hit ? h.dy : 0.f, hit ? h.dz : 0.f};
+      const float x6[6] = {rdx, rdy, rdz, h.dx, h.dy, h.dz};
       float o[4];
-      if constexpr (MF) mlp_wave_mfma32<false, false, HT>(x6, freq, att, W1, b1, W2, b2, W3, b3, p, dir, o);
       if (hit) {
-        if constexpr (!MF) mlp_eval<HT, FT>(x6, freq, att, F, H, mlp, p, o);
+        mlp_eval<HT, FT>(x6, freq, att, F, H, mlp, p, o);
         const float w = blend_step(acc, o[0], o[1], o[2], o[3], h.decay, h.t);
         w_stat = w;
         if constexpr (EMIT > 0) {
@@ -158,6 +154,117 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
   }
 }
 
+// The 72->{32,16}->{32,16}->4 MLP of a hit on the matrix cores for all 64 pixels at once (mlp_wave_mfma32, same bits);
+// needs 16-byte aligned weight arrays.
+//
+// What bounds it: v_mfma_f32_32x32x2 and vector instructions do NOT run beside one another on this chip, neither in one
+// wavefront nor across the wavefronts of a SIMD (a probe of four wavefronts per SIMD: 8 MFMAs 516 clocks, 64
+// independent FMAs 183, the two interleaved 691), so a hit step costs the sum: 104 x 64 clocks of matrix work plus 2.9
+// for every vector instruction, and every instruction removed shows: the walk of mlpsp_walk_f32.hpp, sin/cos pairs without
+// their range selects, a one-instruction ReLU (1,575 -> 1,360 vector instructions per hit step) and super-blocks of
+// tiles dealt to the XCDs instead of bands of image rows took the 200,000-primitive 1200x680 frame from 4.33 to
+// 3.93 ms and a 30,000-primitive 333x251 feature frame from 1.77 to 1.47.  Three wavefronts per SIMD: four would need
+// 10 KB of LDS per wavefront, and two less registers, and measured within 1 % of three.
+template <int HT, int EMIT, bool STATS = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_tilecenter_f32_mf_kernel(
+    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
+    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
+    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
+    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
+    float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
+    float temp, HitPool hp, const float* __restrict__ gt_rgb, float* __restrict__ stat_sum_w,
+    float* __restrict__ stat_max_w, int32_t* __restrict__ stat_hits, float* __restrict__ stat_sum_werr,
+    int32_t* __restrict__ stat_contrib) {
+  __shared__ DirOperands s_dir;
+  __shared__ WalkLds s_walk;
+  const int unit = (int)(blockIdx.x / kNumXcd), wslot = unit % waves_per_tile;
+  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
+  if (tile < 0) return;
+  const int lane = (int)threadIdx.x, slot = wslot * 64 + lane;
+  const int tx = tile % g.ntx, ty = tile / g.ntx;
+  const int x = tx * g.TW + slot % g.TW, y = ty * g.TH + slot / g.TW;
+  const bool valid = (slot < g.TW * g.TH) && (x < g.W) && (y < g.H);
+  const int pix = valid ? (y * g.W + x) : 0;
+  const Float3 ro = valid ? load3(rays_o, pix) : Float3{0.f, 0.f, 0.f}, rd = valid ? load3(rays_d, pix) : Float3{0.f, 0.f, 0.f};
+  const int start = offsets[tile], end = offsets[tile + 1];
+
+  PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
+  unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
+  Float3 gt = {0.f, 0.f, 0.f};
+  if constexpr (STATS) {
+    if (valid) gt = load3(gt_rgb, pix);
+  }
+  HitEmitter em = hit_emitter_begin(hp, wslot, start, tile);
+  encode_direction(rd.x, rd.y, rd.z, freq, att, s_dir);
+
+  walk_tile_f32(
+      order, start, end, N, prims, valid, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, thr, s_walk,
+      [&]() { return valid && (acc.trans >= kTransmittanceFloor); },
+      [&](int p, bool hit, const HitInfo& h, unsigned long long mask) {
+        ++n_proc;
+        if (mask == 0ull) return true;
+        ++n_proc_hit;
+        n_hits += __popcll(mask);
+        int rs = -1;
+        if constexpr (EMIT > 0) rs = hit_emitter_next(hp, em, lane);
+        // (lanes that did not hit carry no hit point; the matrix-core evaluation runs on all 64 lanes)
+        const float x6[6] = {rd.x, rd.y, rd.z, hit ? h.dx : 0.f, hit ? h.dy : 0.f, hit ? h.dz : 0.f};
+        float o[4];
+        mlp_wave_mfma32<false, false, HT>(x6, freq, att, W1, b1, W2, b2, W3, b3, p, s_dir, o);
+        float w = 0.f;
+        if (hit) w = blend_step(acc, o[0], o[1], o[2], o[3], h.decay, h.t);
+        if constexpr (EMIT > 0) {
+          if (rs >= 0) {
+            float* __restrict__ rec = reinterpret_cast<float*>(hp.records + (size_t)rs * hp.record_bytes);
+            rec[lane] = hit ? w : -1.f;
+            if constexpr (EMIT > 1) {
+              if (hit) {          // the gates of a missed pixel are never read
+                const PrimRecord& P = prims[p];
+                float gates[4];
+                tetra_gates(h.qlx, h.qly, h.qlz, P.lgx, P.lgy, P.lgz, beta, temp, gates);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) rec[(k + 1) * 64 + lane] = gates[k];
+              }
+            }
+            if (lane == 0) hp.hit_ids[rs] = p;
+          }
+        }
+        if constexpr (STATS) {
+          const bool contrib = hit && (w > 1e-1f);
+          float lerr = 0.f;
+          if (contrib) lerr = w * ((fabsf(acc.cr - gt.x) + fabsf(acc.cg - gt.y)) + fabsf(acc.cb - gt.z));
+          const float s_w = wave_sum(w), m_w = wave_max(w), s_err = wave_sum(lerr);
+          const int n_hit = __popcll(__ballot(hit && (w > 1e-8f))), n_con = __popcll(__ballot(contrib));
+          if (lane == 0) {
+            atomicAdd(stat_sum_w + p, s_w);
+            atomicMax(reinterpret_cast<int*>(stat_max_w + p), __float_as_int(m_w));   // weights are >= 0
+            atomicAdd(stat_hits + p, n_hit);
+            if (stat_sum_werr) atomicAdd(stat_sum_werr + p, s_err);
+            if (stat_contrib) atomicAdd(stat_contrib + p, n_con);
+          }
+        }
+        return __ballot(valid && (acc.trans >= kTransmittanceFloor)) != 0ull;
+      });
+
+  if (valid) {
+    store3(out_rgb, pix, acc.cr, acc.cg, acc.cb);
+    out_alpha[pix] = 1.f - acc.trans;
+    if (out_t) out_t[pix] = acc.t_acc / (acc.w_acc > 1e-8f ? acc.w_acc : 1.f);
+  }
+  if constexpr (EMIT > 0) {
+    if (lane == 0) hp.item_hits[tile * waves_per_tile + wslot] = em.count;
+  }
+  if (counters && lane == 0) {
+    atomicAdd(counters + 1, (unsigned long long)n_proc);
+    atomicAdd(counters + 2, (unsigned long long)n_proc_hit);
+    atomicAdd(counters + 3, (unsigned long long)n_hits);
+  }
+}
+inline unsigned f32_mf_grid(const TileGeom& g, int waves_per_tile) {
+  return superblock_grid(g.ntx, g.nty) * (unsigned)waves_per_tile;
+}
+
 // The same walk (image only, matrix-core evaluation) for launches too small to fill the chip: a few hundred tiles on
 // a thousand SIMDs leave every wavefront alone on its SIMD, where nothing hides the chain id -> geometry record ->
 // hit test -> weight rows -> MLP, and the launch lasts as long as its longest tile.  Two things shorten that chain.
@@ -203,7 +310,7 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_ahead_kernel(
 
   PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
-  DirOperands dir;
+  __shared__ DirOperands dir;
   float dir_half[18];
   if constexpr (HALF) encode_direction_half(rdx, rdy, rdz, freq, att, dir_half);
   else encode_direction(rdx, rdy, rdz, freq, att, dir);
@@ -242,7 +349,7 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_ahead_kernel(
           MlpLayer2<HT> w2;
           request_layer2<HT>(W2, b2, p, w2);
           if constexpr (HALF) mlp_half_mfma32_with<HT>(w, w2, x6, freq, att, W3, b3, p, dir_half, o);
-          else mlp_wave_mfma32_with<false, false, HT>(w, w2, x6, freq, att, W3, b3, p, dir, o);
+          else mlp_wave_mfma32_with<false, false, HT>(w, [&](MlpLayer2<HT>& to) { to = w2; }, x6, freq, att, W3, b3, p, dir, o);
           if (hit) blend_step(acc, o[0], o[1], o[2], o[3], h.decay, h.t);
         }
         if (__ballot(valid && (acc.trans >= kTransmittanceFloor)) == 0ull) {

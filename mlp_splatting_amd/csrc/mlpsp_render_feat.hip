@@ -175,10 +175,17 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
                      num_frequencies, W1, b1, W2, b2, W3, b3, num_primitives, hidden, g, wpt, per_xcd, (int)items, threshold,          \
                      out_rgb_dev, out_alpha_dev, (float*)nullptr, (unsigned long long*)nullptr, gating_beta,      \
                      gating_temp, hp)
+#define MLPSP_EMIT_MF_LAUNCH(EM)                                                                                  \
+  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<32, EM>), dim3(f32_mf_grid(g, wpt)), block, 0, s, rays_o_dev, \
+                     rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev,        \
+                     att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, \
+                     (float*)nullptr, (unsigned long long*)nullptr, gating_beta, gating_temp, hp,                   \
+                     (const float*)nullptr, (float*)nullptr, (float*)nullptr, (int32_t*)nullptr, (float*)nullptr,   \
+                     (int32_t*)nullptr)
   const bool gated = feat_slots > 1;
   if (hidden == 32 && use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    if (gated) MLPSP_EMIT_LAUNCH(32, 6, 2, false, true);
-    else MLPSP_EMIT_LAUNCH(32, 6, 1, false, true);
+    if (gated) MLPSP_EMIT_MF_LAUNCH(2);
+    else MLPSP_EMIT_MF_LAUNCH(1);
   } else if (hidden == 32 && num_frequencies == 6) {
     if (gated) MLPSP_EMIT_LAUNCH(32, 6, 2);
     else MLPSP_EMIT_LAUNCH(32, 6, 1);
@@ -186,6 +193,7 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
     if (gated) MLPSP_EMIT_LAUNCH(0, 0, 2);
     else MLPSP_EMIT_LAUNCH(0, 0, 1);
   }
+#undef MLPSP_EMIT_MF_LAUNCH
 #undef MLPSP_EMIT_LAUNCH
   MLPSP_LAUNCH_CHECK();
   const dim3 agrid((unsigned)(per_xcd * kNumXcd), (unsigned)ceil_div(feat_channels, 512)), ablock(256);
