@@ -516,6 +516,60 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
                              int segment, int num_primitives, float* partial_dev, float* grad_positions_dev,
                              float* grad_log_scales_dev, float* grad_quats_dev, mlpsp_stream_t stream);
 
+/* Training steps: a differentiable frame of 8x8 tiles with the 72->32->32->4 MLP in one traversal.  The forward keeps
+ * one STEP per (tile, primitive that hits one of its pixels) -- 64 lanes = the tile's pixels, laid out in planes of 64 --
+ * instead of one record per pixel and hit, and the backward works on steps from end to end: no per-record sort, gather or
+ * scattered store.  Same arithmetic as the record entry points above (the pipeline of np_tile_kernels.cu:2925-3206,
+ * scannet/cuda/training_wmma.cuh:62-253, primitive_records.cuh:3-46, scannet/primitive_gemm.py:101-183); sums are formed
+ * in a fixed order that does not depend on scheduling.
+ *
+ * mlpsp_train_forward_f32 / _mfma: image, alpha and the steps of the lists order_dev (num_pairs entries, sorted by
+ *   mlpsp_sort_tiles with the t* key).  render_order as in mlpsp_records_count; max_hits as there.  workspace_dev:
+ *   mlpsp_train_workspace_bytes(num_pairs, width, height, pool_steps) bytes, 256-byte aligned (pool_steps < 0: the worst
+ *   case).  Its first three int32 words are for the caller to read: {chunks of 16 steps the frame needs, status bits
+ *   (1 = non-finite operand, activation or output of the reduced-precision MLP, 2 = a live pixel reached max_hits), steps}.
+ *   If 16 times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
+ *   the caller repeats the call with a pool of that size.
+ * mlpsp_train_list_steps: primitive, pool slot and tile of every step, in tile order (num_steps = the third word).
+ * mlpsp_train_reverse: reverse compositing; d4_dev [num_steps, 64, 4] = adjoints of the four pre-activation outputs,
+ *   falloff_dev [num_steps, 64] = dL/d(decay) * decay.
+ * mlpsp_train_group: sorted_prim_dev / permutation_dev (int64) = the stable sort of step_prim_dev; fills the index part of
+ *   scratch_dev (mlpsp_train_scratch_bytes(num_steps, num_primitives) bytes, 256-byte aligned).
+ * mlpsp_train_gradients: the nine gradients, written whole, from a scratch_dev that mlpsp_train_group has filled.
+ *   precision, scale: as mlpsp_grouped_vjp; nonfinite_dev[0] becomes 1 if a weight gradient is not finite. */
+size_t mlpsp_train_workspace_bytes(int64_t num_pairs, int width, int height, int64_t pool_steps);
+int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
+                            const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
+                            const float* freq_dev, const float* att_dev, const float* W1, const float* b1,
+                            const float* W2, const float* b2, const float* W3, const float* b3, int num_primitives,
+                            int width, int height, float threshold, int max_hits, int render_order,
+                            void* workspace_dev, size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev,
+                            mlpsp_stream_t stream);
+int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
+                             const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
+                             const float* freq_dev, const float* att_dev, const void* packed_dev, int num_primitives,
+                             int width, int height, float threshold, int max_hits, int use_bf16, void* workspace_dev,
+                             size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev, mlpsp_stream_t stream);
+int mlpsp_train_list_steps(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
+                           const void* workspace_dev, size_t workspace_bytes, int32_t* step_prim_dev,
+                           int32_t* step_slot_dev, int32_t* step_tile_dev, mlpsp_stream_t stream);
+int mlpsp_train_reverse(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
+                        const void* workspace_dev, size_t workspace_bytes, const float* grad_rgb_dev,
+                        const float* grad_t_dev, float* d4_dev, float* falloff_dev, mlpsp_stream_t stream);
+size_t mlpsp_train_scratch_bytes(int64_t num_steps, int num_primitives);
+int mlpsp_train_group(const int32_t* sorted_prim_dev, const int64_t* permutation_dev, const int32_t* step_slot_dev,
+                      const int32_t* step_tile_dev, int64_t num_steps, int num_primitives, void* scratch_dev,
+                      size_t scratch_bytes, mlpsp_stream_t stream);
+int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int64_t num_pairs, int width, int height,
+                          const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,
+                          const float* falloff_dev, const float* rays_d_dev, const float* freq_dev,
+                          const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2,
+                          const float* W3, const float* log_scales_dev, const float* quats_dev, int num_primitives,
+                          int precision, float scale, void* scratch_dev, size_t scratch_bytes, float* gW1_dev,
+                          float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev, float* gb3_dev,
+                          float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev,
+                          int32_t* nonfinite_dev, mlpsp_stream_t stream);
+
 /* Streamed feature L1 loss over saved records = _stream_l1 (scannet/record_feature_loss.py:34-63, launched at
  * :66-89): for every pixel of the low-resolution target [target_height, target_width, channels] (f32, or fp16 if
  * target_is_half) the feature of its four bilinear source pixels is blended from their record lists

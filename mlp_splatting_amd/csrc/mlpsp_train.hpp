@@ -1,0 +1,113 @@
+// Training steps: what a differentiable frame keeps between its forward and its backward pass.
+//
+// The forward writes one STEP per (8x8 tile, primitive that hits one of its pixels): 64 lanes = the tile's pixels, in
+// planes of 64 so that every access of a wavefront is contiguous.  A lane that the primitive did not hit holds zeros,
+// which are neutral everywhere below (weight 0, adjoints 0); 58 of 64 lanes hit at the 200,000-primitive 1200x680
+// frame.  Everything downstream works on steps: the reverse walk goes through a tile's steps last to first, and the
+// per-primitive gradient sums need an ordering of 0.65 M steps instead of one of 38 M per-pixel records -- whose sort,
+// gathers and scattered stores were a third of a training step (the per-pixel records of mlpsp_records_* stay for
+// callers that take records in their hands).
+//
+//   plane A  float4[64]  R, G, B, sigma_raw
+//   plane B  float4[64]  T before the hit, alpha, decay, sigma logit
+//   plane C  float4[64]  hit offset centre - point (MLP inputs 3..5), ReLU mask of layer 1 (bits)
+//   plane D  uint32[64]  ReLU mask of layer 2
+//
+// How many steps a tile will have is known only when it is done, so steps come from a pool in chunks of 16 (as the hit
+// records of mlpsp_hitrec.hpp), two chunks per atomic.  The draw goes on when the pool is exhausted, so that the caller
+// learns how many chunks the frame needs.
+//
+// Workspace: head int32[64] {chunks drawn, status bits, steps in all} | tile_steps int32[T] | tile_base int32[T + 1] |
+// chunk_table int32[P / 16 + T + 1] | ids int32[pool] | records
+#pragma once
+#include "mlpsp_device.hpp"
+#include "mlpsp_host.hpp"
+
+namespace mlpsp {
+
+constexpr int kStepBytes = 3328;
+constexpr int kStepPlaneB = 1024, kStepPlaneC = 2048, kStepPlaneD = 3072;
+constexpr int kStepChunk = 16, kStepGrab = 2;
+constexpr int kTrainNumeric = 1, kTrainCapacity = 2;   // status bits
+
+struct StepPool {
+  int32_t* head;
+  int32_t* tile_steps;
+  int32_t* tile_base;
+  int32_t* chunk_table;
+  int32_t* ids;
+  unsigned char* records;
+  int pool_chunks;
+};
+
+inline size_t step_align(size_t v) { return (v + 255) & ~(size_t)255; }
+inline size_t step_tables_bytes(int64_t num_pairs, int64_t num_tiles) {
+  return step_align(64 * 4) + step_align((size_t)num_tiles * 4) + step_align((size_t)(num_tiles + 1) * 4) +
+         step_align((size_t)(num_pairs / kStepChunk + num_tiles + 1) * 4);
+}
+inline size_t step_pool_bytes(int64_t num_pairs, int64_t num_tiles, int64_t pool_steps) {
+  const size_t chunks = (size_t)((pool_steps + kStepChunk - 1) / kStepChunk);
+  return step_tables_bytes(num_pairs, num_tiles) + step_align(chunks * kStepChunk * 4) + chunks * kStepChunk * (size_t)kStepBytes;
+}
+inline StepPool step_pool_carve(void* workspace, size_t bytes, int64_t num_pairs, int64_t num_tiles) {
+  StepPool sp{};
+  unsigned char* p = (unsigned char*)workspace;
+  sp.head = (int32_t*)p;
+  p += step_align(64 * 4);
+  sp.tile_steps = (int32_t*)p;
+  p += step_align((size_t)num_tiles * 4);
+  sp.tile_base = (int32_t*)p;
+  p += step_align((size_t)(num_tiles + 1) * 4);
+  sp.chunk_table = (int32_t*)p;
+  p += step_align((size_t)(num_pairs / kStepChunk + num_tiles + 1) * 4);
+  const size_t left = bytes - step_tables_bytes(num_pairs, num_tiles);
+  size_t chunks = left / ((size_t)kStepChunk * (kStepBytes + 4));
+  while (chunks > 0 && step_align(chunks * kStepChunk * 4) + chunks * kStepChunk * (size_t)kStepBytes > left) --chunks;
+  if (chunks > 0x7fffffffull / kStepChunk) chunks = 0x7fffffffull / kStepChunk;
+  sp.pool_chunks = (int)chunks;
+  sp.ids = (int32_t*)p;
+  sp.records = p + step_align(chunks * kStepChunk * 4);
+  return sp;
+}
+
+#if defined(__HIPCC__)
+// Wave-uniform writer state of one tile.
+struct StepWriter {
+  int table_base, count, chunk;
+};
+__device__ __forceinline__ StepWriter step_writer_begin(int list_start, int tile) {
+  return StepWriter{(list_start >> 4) + tile, 0, 0};
+}
+// Slot of the tile's next step, or -1 if the pool is exhausted.  Call with the whole wavefront active.
+__device__ __forceinline__ int step_writer_next(const StepPool& sp, StepWriter& w, int lane) {
+  constexpr int kGroup = kStepChunk * kStepGrab;
+  if ((w.count & (kGroup - 1)) == 0) {
+    int c = 0;
+    if (lane == 0) c = atomicAdd(sp.head, kStepGrab);
+    w.chunk = __builtin_amdgcn_readfirstlane(c);
+  }
+  const bool fits = w.chunk + kStepGrab <= sp.pool_chunks;
+  const int within = w.count & (kGroup - 1);
+  if (fits && (within & (kStepChunk - 1)) == 0 && lane == 0)
+    sp.chunk_table[w.table_base + (w.count >> 4)] = w.chunk + (within >> 4);
+  ++w.count;
+  return fits ? w.chunk * kStepChunk + within : -1;
+}
+__device__ __forceinline__ int step_slot(const int32_t* __restrict__ chunk_table, int table_base, int m) {
+  return chunk_table[table_base + (m >> 4)] * kStepChunk + (m & (kStepChunk - 1));
+}
+// One lane's part of a step.
+__device__ __forceinline__ void step_store(const StepPool& sp, int slot, int lane, int p, bool hit, float R, float G,
+                                           float B, float sigma_raw, float trans, float alpha, float decay, float logit,
+                                           float dx, float dy, float dz, uint32_t mask1, uint32_t mask2) {
+  unsigned char* __restrict__ rec = sp.records + (size_t)slot * kStepBytes;
+  float4* __restrict__ a = reinterpret_cast<float4*>(rec);
+  a[lane] = hit ? make_float4(R, G, B, sigma_raw) : make_float4(0.f, 0.f, 0.f, 0.f);
+  a[64 + lane] = hit ? make_float4(trans, alpha, decay, logit) : make_float4(0.f, 0.f, 0.f, 0.f);
+  a[128 + lane] = hit ? make_float4(dx, dy, dz, __uint_as_float(mask1)) : make_float4(0.f, 0.f, 0.f, 0.f);
+  reinterpret_cast<uint32_t*>(rec + kStepPlaneD)[lane] = hit ? mask2 : 0u;
+  if (lane == 0) sp.ids[slot] = p;
+}
+#endif
+
+}  // namespace mlpsp

@@ -270,27 +270,26 @@ class _TileRenderAutogradFn(torch.autograd.Function):
                 W1, b1, W2, b2, W3, b3)
         dims = (int(Wimg), int(Himg), int(TW), int(TH), float(threshold))
         # a training step: nothing derived from the parameters may be reused from, or kept for, another call
-        records = None
+        frame = None
         with _uncached(ext):
             if mode == 0:
                 rgb, alpha = ext.render_tiles_forward(*args, *dims)
             elif mode == 1:
                 matches = getattr(ext, "records_forward_matches_render", None)
                 if (dims[2] == dims[3] and callable(matches) and matches(freq, W1, b1, W2, b2, dims[2])
+                        and positions.shape[0] > 0 and W3.dtype == torch.float32 and b3.dtype == torch.float32
                         and os.environ.get("MLPSP_AUTOGRAD_KEEP_RECORDS", "1") != "0"):
-                    # the records forward in the render kernels' rounding IS this forward (same bits), and its
-                    # records serve the backward: one traversal of the frame less per step
-                    placeholders = [torch.zeros_like(rays_o), torch.zeros(rays_o.shape[0], device=rays_o.device)]
-                    records = ext.render_tiles_training_records(list(args) + placeholders, dims[0], dims[1], dims[2],
-                                                                dims[4], 1.5, 2.0, render_order=True)
-                    rgb, alpha = records[0], records[1]
+                    # the training forward in the render kernels' rounding IS this forward (same bits), and its steps
+                    # serve the backward: the frame is traversed once
+                    rgb, alpha, frame = ext.train_forward(args, dims[0], dims[1], dims[4])
+                    ext.refuse_overflow(frame)
                 else:
                     rgb, alpha = ext.render_tiles_forward_tilecenter(*args, *dims)
             else:
                 raise ValueError("Unsupported tile mode for backward")
         rgb = _add_background(rgb, alpha, bg_color)
-        ctx.save_for_backward(*args, *(records[2:] if records is not None else ()))
-        ctx.has_records = records is not None
+        ctx.save_for_backward(*args, *(() if frame is None else (frame.workspace,)))
+        ctx.frame = None if frame is None else frame.with_workspace(None)
         ctx.dims, ctx.mode, ctx.bg_color = dims, int(mode), bg_color
         return rgb
 
@@ -313,9 +312,11 @@ class _TileRenderAutogradFn(torch.autograd.Function):
                 records = ext.render_tiles_per_pixel_records(args, *ctx.dims, 1.5, 2.0)
                 gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.backward_from_records(
                     records, args[2], args[3], args[4], args[7], args[8], *args[9:15], grad_out_rgb, grad_t_end)
-        elif ctx.has_records:
-            gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.backward_from_records(
-                [None, None, *kept], args[2], args[3], args[4], args[7], args[8], *args[9:15], grad_out_rgb, grad_t_end)
+        elif ctx.frame is not None:
+            frame = ctx.frame.with_workspace(kept[0])
+            groups = ops.train_group(frame, args[6], args[2].shape[0])
+            gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.backward_from_steps(frame, groups, args, grad_out_rgb,
+                                                                               grad_t_end)
         else:
             gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.render_tiles_backward_tilecenter_full(
                 *args, grad_out_rgb, grad_t_end, *ctx.dims)

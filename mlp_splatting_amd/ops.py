@@ -785,3 +785,98 @@ def geometry_gradients(csr_offsets, record_indices, x6_sorted, falloff_adjoint, 
                                                     _ptr(gp), _ptr(gs), _ptr(gq), _stream(dev)),
                "mlpsp_geometry_gradients")
     return gp, gs, gq
+
+
+class TrainFrame:
+    """What a differentiable frame keeps between its forward and its backward: the workspace of its steps (one step per
+    tile and primitive that hits it) and their number.  ``steps`` is what the backward's launches are sized by."""
+    __slots__ = ("workspace", "pairs", "width", "height", "steps", "status", "chunks")
+
+    def __init__(self, workspace, pairs, width, height, chunks, status, steps):
+        self.workspace, self.pairs, self.width, self.height = workspace, pairs, width, height
+        self.chunks, self.status, self.steps = chunks, status, steps
+
+    def with_workspace(self, workspace):
+        """The same frame around ``workspace`` (None: to keep the numbers while autograd keeps the tensor)."""
+        return TrainFrame(workspace, self.pairs, self.width, self.height, self.chunks, self.status, self.steps)
+
+
+def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W, H, threshold, max_hits, pool_steps,
+                  render_order=True, packed=None, bf16=False):
+    """Forward of a differentiable frame -> (rgb, alpha, :class:`TrainFrame`); one read-back (12 bytes).  ``ws``: the six
+    f32 weight tensors (exact MLP); ``packed``: their matrix-core operand copy instead.  ``pool_steps``: steps to make
+    room for; a frame that needs more is repeated once with what it asked for."""
+    dev = rays_o.device
+    lib = _lib.load()
+    pairs, n = int(order.numel()), records.numel() // _lib.PRIM_RECORD_BYTES
+    rgb = torch.empty(W * H, 3, dtype=torch.float32, device=dev)
+    alpha = torch.empty(W * H, 1, dtype=torch.float32, device=dev)
+    for _ in range(2):
+        nbytes = lib.mlpsp_train_workspace_bytes(pairs, W, H, int(pool_steps))
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        head = (_ptr(rays_o), _ptr(rays_d), _ptr(records), _ptr(order), _ptr(tile_offsets), pairs, _ptr(freq), _ptr(att))
+        if packed is None:
+            code = lib.mlpsp_train_forward_f32(*head, *[_ptr(w) for w in ws], n, W, H, float(threshold), int(max_hits),
+                                               1 if render_order else 0, _ptr(workspace), nbytes, _ptr(rgb), _ptr(alpha),
+                                               _stream(dev))
+        else:
+            code = lib.mlpsp_train_forward_mfma(*head, _ptr(packed), n, W, H, float(threshold), int(max_hits),
+                                                1 if bf16 else 0, _ptr(workspace), nbytes, _ptr(rgb), _ptr(alpha),
+                                                _stream(dev))
+        _check(code, "mlpsp_train_forward")
+        chunks, status, steps = workspace[:12].view(torch.int32).tolist()
+        if chunks * 16 <= pool_steps or pool_steps < 0:
+            break
+        pool_steps = chunks * 16
+    return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps)
+
+
+class TrainGroups:
+    """The steps of a frame sorted by primitive: ``prim`` the sorted primitives, ``scratch`` the index and row buffer of
+    the gradient kernels, ``slot`` / ``tile`` of the steps in tile order."""
+    __slots__ = ("prim", "perm", "slot", "tile", "scratch")
+
+
+def train_group(frame, tile_offsets, n):
+    dev = frame.workspace.device
+    lib = _lib.load()
+    S = frame.steps
+    listed = torch.empty(3, max(S, 1), dtype=torch.int32, device=dev)
+    groups = TrainGroups()
+    keys, groups.slot, groups.tile = listed[0, :S], listed[1], listed[2]
+    _check(lib.mlpsp_train_list_steps(_ptr(tile_offsets), frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
+                                      frame.workspace.numel(), _ptr(listed[0]), _ptr(listed[1]), _ptr(listed[2]),
+                                      _stream(dev)), "mlpsp_train_list_steps")
+    groups.prim, groups.perm = torch.sort(keys, stable=True)
+    nbytes = lib.mlpsp_train_scratch_bytes(S, n)
+    groups.scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    _check(lib.mlpsp_train_group(_ptr(groups.prim), _ptr(groups.perm), _ptr(listed[1]), _ptr(listed[2]), S, n,
+                                 _ptr(groups.scratch), nbytes, _stream(dev)), "mlpsp_train_group")
+    return groups
+
+
+def train_reverse(frame, tile_offsets, grad_rgb, grad_t):
+    """(d4 [S, 64, 4], falloff adjoint [S, 64]) of a frame's steps."""
+    dev = frame.workspace.device
+    d4 = torch.empty(max(frame.steps, 1), 64, 4, dtype=torch.float32, device=dev)
+    falloff = torch.empty(max(frame.steps, 1), 64, dtype=torch.float32, device=dev)
+    _check(_lib.load().mlpsp_train_reverse(_ptr(tile_offsets), frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
+                                           frame.workspace.numel(), _ptr(grad_rgb), _ptr(grad_t), _ptr(d4), _ptr(falloff),
+                                           _stream(dev)), "mlpsp_train_reverse")
+    return d4, falloff
+
+
+def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scales, quats, precision, scale):
+    """([gW1, gb1, gW2, gb2, gW3, gb3, grad_positions, grad_log_scales, grad_quats], non-finite flag int32 [1])."""
+    dev = rays_d.device
+    n = log_scales.shape[0]
+    grads = [torch.empty_like(w) for w in ws[:6]]
+    geo = [torch.empty_like(log_scales), torch.empty_like(log_scales), torch.empty_like(quats)]
+    flag = torch.empty(1, dtype=torch.int32, device=dev)
+    code = _lib.load().mlpsp_train_gradients(
+        _ptr(groups.prim), frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
+        frame.workspace.numel(), _ptr(d4), _ptr(falloff), _ptr(rays_d), _ptr(freq), _ptr(att), *[_ptr(w) for w in ws[:5]],
+        _ptr(log_scales), _ptr(quats), n, int(precision), float(scale), _ptr(groups.scratch), groups.scratch.numel(),
+        *[_ptr(g) for g in grads], *[_ptr(g) for g in geo], _ptr(flag), _stream(dev))
+    _check(code, "mlpsp_train_gradients")
+    return grads + geo, flag

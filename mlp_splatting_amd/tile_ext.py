@@ -82,6 +82,7 @@ class TileExt:
         self._binned = None
         self._queue_capacity = 0          # candidate-buffer estimate of render_frame_queued (0: not seeded yet)
         self._queue_scratch_scale = 1
+        self._steps_per_tile = 96         # room the differentiable frame makes for its steps (see train_forward)
 
     # ------------------------------------------------------------------------------------------
     # derived-tensor caches (geometry records, matrix-core operand copies)
@@ -579,6 +580,60 @@ class TileExt:
         forward pass for the backward instead of traversing the frame again."""
         return (int(tile) == 8 and freq.numel() == 6 and tuple(W1.shape[1:]) == (32, 72) and tuple(W2.shape[1:]) == (32, 32)
                 and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (W1, b1, W2, b2)))
+
+    # ------------------------------------------------------------------------------------------
+    # a differentiable frame in training steps (no counterpart in the reference; what its record entry points, reverse
+    # walk and grouped gradients compute, with the step -- tile x primitive -- as the unit of storage)
+    # ------------------------------------------------------------------------------------------
+    def train_forward(self, x, width, height, threshold, *, render_order=True, precision=None,
+                      name="render_tiles_mlp_records"):
+        """(rgb, alpha, ops.TrainFrame) of an 8x8-tile frame with the 72->32->32->4 MLP.  ``x``: the 15 scene tensors.
+        ``precision`` None: exact f32 (with ``render_order`` the bits of ``render_tiles_forward_tilecenter``, see
+        :meth:`records_forward_matches_render`); "float16" / "bfloat16": the matrix cores.  The frame's ``status`` bits
+        (1 numeric, 2 hit capacity) are the caller's to judge."""
+        width, height = int(width), int(height)
+        _chk(width > 0 and height > 0 and x[0].shape[0] == width * height, "B must equal W*H for tile renderer")
+        self._check_base(*x[:9])
+        for t in x:
+            _chk(t.is_cuda and t.is_contiguous() and t.device == x[0].device, "Inputs must be contiguous CUDA tensors")
+        n = x[2].shape[0]
+        n_tiles = ops.num_tiles(width, height, 8, 8)
+        with torch.cuda.device(x[0].device), self.uncached():
+            self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
+            rec = self._records(x[2], x[3], x[4])
+            order = x[5]
+            if x[5].numel() > 0:
+                order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
+                                          self.max_tile_prims, cull_threshold=float(threshold))
+            packed = None if precision is None else self._packed_weights(list(x[9:15]), precision == "bfloat16")
+            with self._lock:
+                pool = n_tiles * self._steps_per_tile
+            rgb, alpha, frame = ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height,
+                                                  float(threshold), self.max_hits, pool, render_order=render_order,
+                                                  packed=packed, bf16=precision == "bfloat16")
+            with self._lock:      # a quarter more than this frame needed, in whole chunks, for the next one
+                self._steps_per_tile = max(16, -(-frame.chunks * 20 // n_tiles))
+        return rgb, alpha, frame
+
+    def refuse_overflow(self, frame, name="render_tiles_mlp_records"):
+        """Raise the reference's hit-capacity error (np_tile_kernels.cu:4601-4609) if the frame's status says so."""
+        if frame.status & 2:
+            raise RuntimeError(f"{name}: tile-center backward hit capacity {int(self.max_hits)} reached before "
+                               "transmittance termination; refusing to return truncated gradients")
+
+    @staticmethod
+    def backward_from_steps(frame, groups, x, grad_rgb, grad_t, dtype=torch.float32):
+        """The nine gradients of :meth:`render_tiles_backward_tilecenter_full` from a frame's steps; ``x``: the scene
+        tensors of the forward, ``groups``: ``ops.train_group`` of the frame.  Non-finite policy of
+        ``primitive_gemm.grouped_weight_gradients``."""
+        from . import primitive_gemm
+        with torch.cuda.device(x[0].device), torch.no_grad():
+            d4, falloff = ops.train_reverse(frame, x[6], grad_rgb, grad_t)
+
+            def launch(operand_dtype, scale):
+                return ops.train_gradients(frame, groups, d4, falloff, x[1], x[7], x[8], x[9:15], x[3], x[4],
+                                           primitive_gemm._PRECISION_CODE[operand_dtype], scale)
+            return primitive_gemm._checked_grouped_vjp(launch, dtype, 4096.0 if dtype == torch.float16 else 1.0)
 
     def training_wmma_safety_stats(self):
         """[calls, frame_fallbacks, fp32_nonfinite_failures, count_emit_failures, capacity_failures] of
