@@ -527,7 +527,8 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  *   mlpsp_sort_tiles with the t* key).  render_order as in mlpsp_records_count; max_hits as there.  workspace_dev:
  *   mlpsp_train_workspace_bytes(num_pairs, width, height, pool_steps) bytes, 256-byte aligned (pool_steps < 0: the worst
  *   case).  Its first three int32 words are for the caller to read: {chunks of 16 steps the frame needs, status bits
- *   (1 = non-finite operand, activation or output of the reduced-precision MLP, 2 = a live pixel reached max_hits), steps}.
+ *   (1 = non-finite offset, activation, output or colour -- not reported by the f32 forward in the render's order --,
+ *   2 = a live pixel reached max_hits), steps}.
  *   If 16 times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
  *   the caller repeats the call with a pool of that size.
  * mlpsp_train_list_steps: primitive, pool slot and tile of every step, in tile order (num_steps = the third word).
@@ -536,7 +537,13 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  * mlpsp_train_group: sorted_prim_dev / permutation_dev (int64) = the stable sort of step_prim_dev; fills the index part of
  *   scratch_dev (mlpsp_train_scratch_bytes(num_steps, num_primitives) bytes, 256-byte aligned).
  * mlpsp_train_gradients: the nine gradients, written whole, from a scratch_dev that mlpsp_train_group has filled.
- *   precision, scale: as mlpsp_grouped_vjp; nonfinite_dev[0] becomes 1 if a weight gradient is not finite. */
+ *   precision, scale: as mlpsp_grouped_vjp; nonfinite_dev[0] becomes 1 if a weight gradient is not finite.
+ *
+ * mlpsp_train_feature_l1 / _gradients: the streamed feature L1 loss of mlpsp_stream_feature_l1 and its attribute gradient
+ *   (mlpsp_feature_attribute_gradients, times the loss adjoint loss_adjoint_dev[0]) from the steps; arguments as there, beta
+ *   and temp as in the record forward.  mlpsp_train_feature_bytes returns the size of kept_dev (what the gradients need,
+ *   256-byte aligned) and fills share_bytes (shares_dev, scratch of the loss), loss_partials (floats; their sum is the loss)
+ *   and row_bytes (rows_dev, scratch of the gradients); 0 = invalid shape.  scratch_dev: filled by mlpsp_train_group. */
 size_t mlpsp_train_workspace_bytes(int64_t num_pairs, int width, int height, int64_t pool_steps);
 int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
                             const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
@@ -569,6 +576,19 @@ int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int
                           float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev, float* gb3_dev,
                           float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev,
                           int32_t* nonfinite_dev, mlpsp_stream_t stream);
+
+size_t mlpsp_train_feature_bytes(int width, int height, int target_width, int target_height, int channels, int slots,
+                                 int64_t num_steps, size_t* share_bytes, int64_t* loss_partials, size_t* row_bytes);
+int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
+                           const void* workspace_dev, size_t workspace_bytes, int64_t num_steps,
+                           const void* prim_records_dev, const float* attributes_dev, const void* target_dev,
+                           int target_is_half, int target_width, int target_height, int channels, int slots, float beta,
+                           float temp, void* kept_dev, size_t kept_bytes, float* shares_dev, float* loss_partials_dev,
+                           mlpsp_stream_t stream);
+int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int width, int height,
+                                  int target_width, int target_height, int channels, int slots, const void* kept_dev,
+                                  size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes, int num_primitives,
+                                  const float* loss_adjoint_dev, float* rows_dev, float* out_dev, mlpsp_stream_t stream);
 
 /* Streamed feature L1 loss over saved records = _stream_l1 (scannet/record_feature_loss.py:34-63, launched at
  * :66-89): for every pixel of the low-resolution target [target_height, target_width, channels] (f32, or fp16 if

@@ -70,6 +70,27 @@ inline StepPool step_pool_carve(void* workspace, size_t bytes, int64_t num_pairs
   return sp;
 }
 
+// The steps sorted by primitive: first sorted position of every primitive [N + 1]; pool slot, tile and number in tile order
+// of the sorted steps [S].  Every buffer that holds them begins with them.
+struct StepSort {
+  int32_t *first, *slot, *tile, *ord;
+  size_t bytes;
+};
+inline StepSort step_sort(void* base, int64_t S, int N) {
+  StepSort t{};
+  unsigned char* p = (unsigned char*)base;
+  t.first = (int32_t*)p;
+  p += step_align(((size_t)N + 1) * 4);
+  t.slot = (int32_t*)p;
+  p += step_align((size_t)S * 4);
+  t.tile = (int32_t*)p;
+  p += step_align((size_t)S * 4);
+  t.ord = (int32_t*)p;
+  p += step_align((size_t)S * 4);
+  t.bytes = (size_t)(p - (unsigned char*)base);
+  return t;
+}
+
 #if defined(__HIPCC__)
 // Wave-uniform writer state of one tile.
 struct StepWriter {

@@ -601,28 +601,18 @@ inline int train_chunk_steps(int64_t S) {
   return per >= 16 ? 16 : per <= 4 ? 4 : (int)per;
 }
 
-struct TrainScratch {
-  int32_t *first, *slot, *tile, *ord;
+// The sorted steps, then head and tail rows of every chunk.
+struct TrainScratch : StepSort {
   float* rows;
   int chunk_steps, num_chunks;
-  size_t bytes;
 };
 inline TrainScratch train_scratch(void* base, int64_t S, int N) {
   TrainScratch t{};
-  unsigned char* p = (unsigned char*)base;
-  t.first = (int32_t*)p;
-  p += step_align(((size_t)N + 1) * 4);
-  t.slot = (int32_t*)p;
-  p += step_align((size_t)S * 4);
-  t.tile = (int32_t*)p;
-  p += step_align((size_t)S * 4);
-  t.ord = (int32_t*)p;
-  p += step_align((size_t)S * 4);
-  t.rows = (float*)p;
+  static_cast<StepSort&>(t) = step_sort(base, S, N);
+  t.rows = (float*)((unsigned char*)base + t.bytes);
   t.chunk_steps = train_chunk_steps(S);
   t.num_chunks = (int)((S + t.chunk_steps - 1) / t.chunk_steps);
-  p += step_align((size_t)2 * t.num_chunks * kRowFloats * 4);
-  t.bytes = (size_t)(p - (unsigned char*)base);
+  t.bytes += step_align((size_t)2 * t.num_chunks * kRowFloats * 4);
   return t;
 }
 

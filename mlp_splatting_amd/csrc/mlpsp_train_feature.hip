@@ -1,0 +1,513 @@
+// libmlpsp_hip: streamed feature L1 loss over the training steps of a frame (mlpsp_train.hpp) and its gradient with
+// respect to the feature attributes: what the reference's _stream_l1, _feature_vjp and _feature_reduce
+// (scannet/record_feature_loss.py:12-162) compute from per-pixel records.
+//
+// The value of target pixel t and channel c is  sum over steps, slots  k[t][step][slot] attr[primitive][slot][c]  with
+//   k[t][step][slot] = sum over the (up to) four bilinear taps q of t:  weight_q  T alpha(step, q)  gate_slot(step, q),
+// and the gradient of the attributes is the transposed product  sum over t  k[t][step][slot] sign(t, c).  So the taps are
+// gathered once, into k -- per step and tile one number for each of the tile's targets and slots, 64 bytes where a
+// target is a quarter of the image's resolution --, and what runs over the channels is a product of small matrices, not
+// four walks over four pixels' record lists.  Both directions use the same k, in f32.
+//
+//   train_feature_blend_kernel  k of a tile's steps (kept for the backward); the tile's share of its targets' values
+//   train_feature_join_kernel   the shares of a target (its taps lie in one, two or four tiles), residual, sign, loss
+//   train_attr_kernel           steps sorted by primitive, in chunks as in mlpsp_train_backward.hip
+//   train_attr_finish_kernel    rows of primitives that span chunks; zeros of those without a step
+//
+// All are bound by memory traffic: attribute rows out of L2 in the blend (8 KB per step at 512 channels, four slots), sign
+// rows (2 KB) in the gradient, the zeros of the gradient (8 KB per primitive) in the last.  At 200,000 primitives,
+// 1200x680, a 300x170 target of 512 channels: 0.56, 0.07, 0.44 and 0.32 ms; the record kernels took 4.95 ms for the
+// loss and 8.1 ms for the gradient.
+#include "mlpsp_device.hpp"
+#include "mlpsp_host.hpp"
+#include "mlpsp_train.hpp"
+
+namespace mlpsp {
+
+// Bilinear source pixels of low-resolution index i (F.interpolate, align_corners=False): the same on host and device.
+struct Taps {
+  int i0, i1;
+  float w;      // of i1
+};
+__host__ __device__ inline Taps feature_taps(int i, float scale, int size) {
+  float v = ((float)i + .5f) * scale - .5f;
+  v = v > 0.f ? v : 0.f;
+  Taps t;
+  t.i0 = (int)v;
+  if (t.i0 > size - 1) t.i0 = size - 1;
+  t.i1 = t.i0 + 1 < size ? t.i0 + 1 : size - 1;
+  t.w = v - (float)t.i0;
+  return t;
+}
+// Targets with a tap in [8 tile, 8 tile + 7]: the first one and their number (taps never decrease with i).
+struct AxisSpan {
+  int lo, n;
+};
+__host__ __device__ inline AxisSpan feature_axis_span(int tile, float scale, int size, int targets) {
+  int lo = (int)((8.f * (float)tile - .5f) / scale) - 3;
+  if (lo < 0) lo = 0;
+  while (lo < targets && feature_taps(lo, scale, size).i1 < 8 * tile) ++lo;
+  int hi = lo;
+  while (hi < targets && feature_taps(hi, scale, size).i0 <= 8 * tile + 7) ++hi;
+  return AxisSpan{lo, hi - lo};
+}
+
+constexpr int kFeatWaves = 4;       // wavefronts of a blend workgroup, 256 channels each, at most
+
+struct FeatShape {
+  int W, H, ntx, nty, WF, HF, C, Cp, slots, NT;   // Cp: C rounded up to 4; NT: targets per tile, rounded up to 4
+  float sx, sy;
+  int64_t T;
+};
+inline bool feat_shape(int width, int height, int wf, int hf, int channels, int slots, FeatShape& f) {
+  f.T = checked_num_tiles(width, height, 8, 8);
+  if (f.T <= 0 || f.T > 2147483647LL - 8 || wf <= 0 || hf <= 0 || wf > width || hf > height || channels <= 0 ||
+      channels > (1 << 20) || (slots != 1 && slots != 4 && slots != 5) || (int64_t)wf * hf > 2147483647LL)
+    return false;
+  f.W = width, f.H = height, f.WF = wf, f.HF = hf, f.C = channels, f.slots = slots;
+  f.ntx = ceil_div(width, 8), f.nty = ceil_div(height, 8);
+  f.Cp = (channels + 3) & ~3;
+  f.sx = (float)width / (float)wf, f.sy = (float)height / (float)hf;
+  int nx = 0, ny = 0;
+  for (int t = 0; t < f.ntx; ++t) { const int n = feature_axis_span(t, f.sx, width, wf).n; nx = n > nx ? n : nx; }
+  for (int t = 0; t < f.nty; ++t) { const int n = feature_axis_span(t, f.sy, height, hf).n; ny = n > ny ? n : ny; }
+  f.NT = (nx * ny + 3) & ~3;
+  return true;
+}
+// Kept for the backward: spans int32[2 (ntx + nty)] | groups of four targets of every tile int32[T] | signs int8[T][NT][Cp]
+// | k float[S][NT / 4][slots][4].  Scratch of the forward: shares float[T][NT][Cp].
+struct FeatKept {
+  int2 *columns, *rows;
+  int32_t* groups;
+  int8_t* signs;
+  float* k;
+  size_t bytes;
+};
+inline FeatKept feat_kept(void* base, const FeatShape& f, int64_t S) {
+  FeatKept o{};
+  unsigned char* p = (unsigned char*)base;
+  o.columns = (int2*)p;
+  p += step_align((size_t)f.ntx * 8);
+  o.rows = (int2*)p;
+  p += step_align((size_t)f.nty * 8);
+  o.groups = (int32_t*)p;
+  p += step_align((size_t)f.T * 4);
+  o.signs = (int8_t*)p;
+  p += step_align((size_t)f.T * f.NT * f.Cp);
+  o.k = (float*)p;
+  p += step_align((size_t)S * f.NT * f.slots * 4);
+  o.bytes = (size_t)(p - (unsigned char*)base);
+  return o;
+}
+
+__global__ __launch_bounds__(256) void feature_span_kernel(FeatShape f, FeatKept o) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i < f.ntx) {
+    const AxisSpan s = feature_axis_span(i, f.sx, f.W, f.WF);
+    o.columns[i] = make_int2(s.lo, s.n);
+  }
+  if (i < f.nty) {
+    const AxisSpan s = feature_axis_span(i, f.sy, f.H, f.HF);
+    o.rows[i] = make_int2(s.lo, s.n);
+  }
+  if (i < f.T)
+    o.groups[i] = (feature_axis_span(i % f.ntx, f.sx, f.W, f.WF).n * feature_axis_span(i / f.ntx, f.sy, f.H, f.HF).n + 3) >> 2;
+}
+
+// Four consecutive channels of an attribute row: one load where the rows are 16-byte aligned (VEC), else four, those past
+// the last channel clamped to it (what they yield is never used).
+template <bool VEC>
+__device__ __forceinline__ float4 four_channels(const float* __restrict__ row, int c, int C) {
+  if constexpr (VEC) {
+    return *reinterpret_cast<const float4*>(row + min(c, C - 4));
+  } else {
+    return make_float4(row[min(c, C - 1)], row[min(c + 1, C - 1)], row[min(c + 2, C - 1)], row[min(c + 3, C - 1)]);
+  }
+}
+// Lanes per step, as a power of two: a row of up to 64, 128 or 256 channels takes 16, 32 or 64 lanes (four channels each),
+// and the 4, 2 or 1 lane groups of a wavefront take steps in turn.
+inline int lanes_per_row_log2(int Cp) { return Cp <= 64 ? 4 : Cp <= 128 ? 5 : 6; }
+
+// One workgroup = one tile, four of its targets (blockIdx.y), up to 1,024 channels (blockIdx.z).  Sixteen steps at a time
+// (a chunk of the pool): every group of 16 lanes computes k of one step -- lane = (target, tap), the taps' sum two DPP
+// adds --, then every lane adds the sixteen steps to its four channels.
+template <int SLOTS, bool VEC>
+__global__ __launch_bounds__(64 * kFeatWaves) void train_feature_blend_kernel(
+    FeatShape f, FeatKept o, const int32_t* __restrict__ offsets, const int32_t* __restrict__ tile_base,
+    const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ ids, const unsigned char* __restrict__ records,
+    const PrimRecord* __restrict__ prims, const float* __restrict__ attr, int lpr_log2, float beta, float temp,
+    float* __restrict__ shares) {
+  __shared__ __attribute__((aligned(16))) float s_k[2][kStepChunk][SLOTS][4];
+  __shared__ int s_p[2][kStepChunk];
+  const int tile = superblock_tile(blockIdx.x, f.ntx, f.nty);
+  if (tile < 0) return;
+  const int group = blockIdx.y, tx = tile % f.ntx, ty = tile / f.ntx, tid = threadIdx.x, lane = tid & 63;
+  const int2 col = o.columns[tx], row = o.rows[ty];
+  const int nt = col.y * row.y;
+  if (group * 4 >= nt) return;
+  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = (offsets[tile] >> 4) + tile;
+
+  // this lane's target and tap
+  const int q = tid & 3, j = (tid >> 2) & 3, t = group * 4 + j;
+  float weight = 0.f;
+  int px = 0;
+  if (t < nt) {
+    const Taps x = feature_taps(col.x + t % col.y, f.sx, f.W), y = feature_taps(row.x + t / col.y, f.sy, f.H);
+    const int xx = (q & 1) ? x.i1 : x.i0, yy = (q & 2) ? y.i1 : y.i0;
+    const float w = ((q & 1) ? x.w : 1.f - x.w) * ((q & 2) ? y.w : 1.f - y.w);
+    if ((xx >> 3) == tx && (yy >> 3) == ty) {
+      weight = w;
+      px = (yy & 7) * 8 + (xx & 7);
+    }
+  }
+  const int lpr = 1 << lpr_log2, sub = lane >> lpr_log2, nsub = 64 >> lpr_log2;
+  const int c = (blockIdx.z * (int)(blockDim.x >> 6) + (tid >> 6)) * 256 + (lane & (lpr - 1)) * 4;
+  const bool channels = c < f.C;
+  float4 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+
+  for (int m = 0; m < count; m += kStepChunk) {
+    const int first = chunk_table[table + (m >> 4)] * kStepChunk, n = min(kStepChunk, count - m), buf = (m >> 4) & 1;
+    for (int i = tid >> 4; i < n; i += (int)(blockDim.x >> 4)) {
+      const int p = ids[first + i];
+      float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+      if (weight != 0.f) {
+        const unsigned char* __restrict__ rec = records + (size_t)(first + i) * kStepBytes;
+        const float2 ta = *reinterpret_cast<const float2*>(rec + kStepPlaneB + px * 16);
+        v[4] = weight * (ta.x * ta.y);
+        if constexpr (SLOTS != 1) {
+          const float4 d = *reinterpret_cast<const float4*>(rec + kStepPlaneC + px * 16);
+          const PrimRecord& P = prims[p];
+          const Vec3 ql = quat_rotate_conj(P.qw, P.qx, P.qy, P.qz, Vec3{d.x, d.y, d.z});
+          float g[4];
+          tetra_gates(ql.x, ql.y, ql.z, P.lgx, P.lgy, P.lgz, beta, temp, g);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) v[s] = v[4] * g[s];
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 5; ++s) {
+        v[s] += __shfl_xor(v[s], 1);
+        v[s] += __shfl_xor(v[s], 2);
+      }
+      float* __restrict__ keep = o.k + (((size_t)(base + m + i) * (f.NT >> 2) + group) * SLOTS) * 4 + j;
+      const bool writes = blockIdx.z == 0;
+      if constexpr (SLOTS != 1) {
+        const float mine = (q & 2) ? ((q & 1) ? v[3] : v[2]) : ((q & 1) ? v[1] : v[0]);
+        const int s = q + (SLOTS == 5 ? 1 : 0);
+        s_k[buf][i][s][j] = mine;
+        if (writes) keep[s * 4] = mine;
+      }
+      if (SLOTS != 4 && q == 0) {
+        s_k[buf][i][0][j] = v[4];
+        if (writes) keep[0] = v[4];
+      }
+      if ((tid & 15) == 0) s_p[buf][i] = p;
+    }
+    __syncthreads();
+    if (channels) {
+#pragma unroll 4
+      for (int i = sub; i < n; i += nsub) {
+        const float* __restrict__ src = attr + (size_t)s_p[buf][i] * SLOTS * f.C;
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+          const float4 a = four_channels<VEC>(src + (size_t)s * f.C, c, f.C);
+          const float4 k = *reinterpret_cast<const float4*>(&s_k[buf][i][s][0]);
+          acc[0].x = fmaf(k.x, a.x, acc[0].x), acc[0].y = fmaf(k.x, a.y, acc[0].y);
+          acc[0].z = fmaf(k.x, a.z, acc[0].z), acc[0].w = fmaf(k.x, a.w, acc[0].w);
+          acc[1].x = fmaf(k.y, a.x, acc[1].x), acc[1].y = fmaf(k.y, a.y, acc[1].y);
+          acc[1].z = fmaf(k.y, a.z, acc[1].z), acc[1].w = fmaf(k.y, a.w, acc[1].w);
+          acc[2].x = fmaf(k.z, a.x, acc[2].x), acc[2].y = fmaf(k.z, a.y, acc[2].y);
+          acc[2].z = fmaf(k.z, a.z, acc[2].z), acc[2].w = fmaf(k.z, a.w, acc[2].w);
+          acc[3].x = fmaf(k.w, a.x, acc[3].x), acc[3].y = fmaf(k.w, a.y, acc[3].y);
+          acc[3].z = fmaf(k.w, a.z, acc[3].z), acc[3].w = fmaf(k.w, a.w, acc[3].w);
+        }
+      }
+    }
+  }
+  for (int d = lpr; d < 64; d <<= 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      acc[i].x += __shfl_xor(acc[i].x, d);
+      acc[i].y += __shfl_xor(acc[i].y, d);
+      acc[i].z += __shfl_xor(acc[i].z, d);
+      acc[i].w += __shfl_xor(acc[i].w, d);
+    }
+  }
+  if (channels && sub == 0) {
+    float* __restrict__ dst = shares + ((size_t)tile * f.NT + group * 4) * f.Cp + c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(dst + (size_t)i * f.Cp) = acc[i];
+  }
+}
+
+// One lane = four channels of one target.  loss: one partial per workgroup, already divided by the number of residuals.
+template <typename T>
+__global__ __launch_bounds__(256) void train_feature_join_kernel(FeatShape f, FeatKept o, const float* __restrict__ shares,
+                                                                 const T* __restrict__ target, float* __restrict__ loss) {
+  __shared__ float s_part[4];
+  const int quads = f.Cp >> 2;
+  const long long at = (long long)blockIdx.x * 256 + threadIdx.x;
+  float part = 0.f;
+  if (at < (long long)f.WF * f.HF * quads) {
+    const int pix = (int)(at / quads), c = (int)(at - (long long)pix * quads) * 4;
+    const int ix = pix % f.WF, iy = pix / f.WF;
+    const Taps x = feature_taps(ix, f.sx, f.W), y = feature_taps(iy, f.sy, f.H);
+    const int x0 = x.i0 >> 3, x1 = x.i1 >> 3, y0 = y.i0 >> 3, y1 = y.i1 >> 3;
+    const auto place = [&](int tx, int ty) {
+      const int2 col = o.columns[tx], row = o.rows[ty];
+      return ((size_t)(ty * f.ntx + tx) * f.NT + (iy - row.x) * col.y + (ix - col.x)) * f.Cp + c;
+    };
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int ty = y0; ty <= y1; ++ty)
+      for (int tx = x0; tx <= x1; ++tx) {
+        const float4 s = *reinterpret_cast<const float4*>(shares + place(tx, ty));
+        v[0] += s.x, v[1] += s.y, v[2] += s.z, v[3] += s.w;
+      }
+    const T* __restrict__ want = target + (size_t)pix * f.C;
+    uint32_t signs = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (c + k < f.C) {
+        const float delta = v[k] - (float)want[c + k];
+        signs |= (uint32_t)(uint8_t)(int8_t)((delta > 0.f) - (delta < 0.f)) << (8 * k);
+        part += __builtin_fabsf(delta);
+      }
+    }
+    for (int ty = y0; ty <= y1; ++ty)
+      for (int tx = x0; tx <= x1; ++tx) *reinterpret_cast<uint32_t*>(o.signs + place(tx, ty)) = signs;
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) part += __shfl_xor(part, d);
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = part;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    loss[blockIdx.x] = ((s_part[0] + s_part[1]) + (s_part[2] + s_part[3])) / (float)((long long)f.HF * f.WF * f.C);
+}
+
+// One wavefront = one chunk of the sorted steps x 256 channels: sum over the steps' targets of k[slot][target] sign.
+template <int SLOTS, bool VEC>
+__global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o, const int32_t* __restrict__ prim,
+                                                         const int32_t* __restrict__ first, const int32_t* __restrict__ step_tile,
+                                                         const int32_t* __restrict__ step_ord, int S, int chunk_steps,
+                                                         int num_chunks, int lpr_log2, const float* __restrict__ adjoint,
+                                                         float* __restrict__ rows, float* __restrict__ out) {
+  const int chunk = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  if (chunk >= num_chunks) return;
+  const int chunk_end = min(S, (chunk + 1) * chunk_steps);
+  const int lpr = 1 << lpr_log2, sub = lane >> lpr_log2, nsub = 64 >> lpr_log2;
+  const int c = (int)blockIdx.y * 256 + (lane & (lpr - 1)) * 4;
+  const bool channels = c < f.C;
+  const int cs = channels ? c : 0;
+  const float norm = (float)((long long)f.WF * f.HF * f.C), scale = adjoint[0];
+  const size_t k_stride = (size_t)f.NT * SLOTS;
+  for (int pos = chunk * chunk_steps; pos < chunk_end;) {
+    const int p = __builtin_amdgcn_readfirstlane(prim[pos]);
+    const int all_end = first[p + 1], end = min(all_end, chunk_end);
+    const bool goes_on = all_end > chunk_end, complete = first[p] == pos && !goes_on;
+    float4 acc[SLOTS];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s) acc[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = pos + sub; i < end; i += nsub) {
+      const int tile = step_tile[i], groups = o.groups[tile];
+      const float* __restrict__ k = o.k + (size_t)step_ord[i] * k_stride;
+      const int8_t* __restrict__ sg = o.signs + (size_t)tile * f.NT * f.Cp + cs;
+      for (int g = 0; g < groups; ++g, k += 4 * SLOTS, sg += 4 * f.Cp) {
+        int word[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) word[t] = *reinterpret_cast<const int*>(sg + t * f.Cp);
+        float4 kk[SLOTS];
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) kk[s] = *reinterpret_cast<const float4*>(k + 4 * s);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float s0 = (float)(int8_t)word[t], s1 = (float)(int8_t)(word[t] >> 8), s2 = (float)(int8_t)(word[t] >> 16),
+                      s3 = (float)(word[t] >> 24);
+#pragma unroll
+          for (int s = 0; s < SLOTS; ++s) {
+            const float v = t == 0 ? kk[s].x : t == 1 ? kk[s].y : t == 2 ? kk[s].z : kk[s].w;
+            acc[s].x = fmaf(v, s0, acc[s].x);
+            acc[s].y = fmaf(v, s1, acc[s].y);
+            acc[s].z = fmaf(v, s2, acc[s].z);
+            acc[s].w = fmaf(v, s3, acc[s].w);
+          }
+        }
+      }
+    }
+    for (int d = lpr; d < 64; d <<= 1) {
+#pragma unroll
+      for (int s = 0; s < SLOTS; ++s) {
+        acc[s].x += __shfl_xor(acc[s].x, d);
+        acc[s].y += __shfl_xor(acc[s].y, d);
+        acc[s].z += __shfl_xor(acc[s].z, d);
+        acc[s].w += __shfl_xor(acc[s].w, d);
+      }
+    }
+    if (channels && sub == 0) {
+      if (complete) {
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+          float* __restrict__ dst = out + ((size_t)p * SLOTS + s) * f.C + c;
+          const float4 v = make_float4(acc[s].x / norm * scale, acc[s].y / norm * scale, acc[s].z / norm * scale,
+                                       acc[s].w / norm * scale);
+          if constexpr (VEC) {
+            *reinterpret_cast<float4*>(dst) = v;
+          } else {
+            dst[0] = v.x;
+            if (c + 1 < f.C) dst[1] = v.y;
+            if (c + 2 < f.C) dst[2] = v.z;
+            if (c + 3 < f.C) dst[3] = v.w;
+          }
+        }
+      } else {
+        float* __restrict__ dst = rows + ((size_t)(goes_on ? num_chunks + chunk : chunk) * SLOTS) * f.Cp + c;
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) *reinterpret_cast<float4*>(dst + (size_t)s * f.Cp) = acc[s];
+      }
+    }
+    pos = end;
+  }
+}
+
+// One workgroup per primitive, lane = four channels of one slot.
+template <bool VEC>
+__global__ __launch_bounds__(256) void train_attr_finish_kernel(FeatShape f, const int32_t* __restrict__ first, int chunk_steps,
+                                                                int num_chunks, const float* __restrict__ adjoint,
+                                                                const float* __restrict__ rows, float* __restrict__ out) {
+  const int p = blockIdx.x, begin = first[p], end = first[p + 1];
+  const int cf = begin / chunk_steps, cl = begin < end ? (end - 1) / chunk_steps : cf;
+  if (begin < end && cf == cl) return;
+  const float norm = (float)((long long)f.WF * f.HF * f.C), scale = adjoint[0];
+  const int quads = f.Cp >> 2;
+  for (int i = threadIdx.x; i < quads * f.slots; i += 256) {
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (begin < end) {
+#pragma unroll 8
+      for (int c = cf; c <= cl; ++c) {
+        const float4 v = reinterpret_cast<const float4*>(rows + ((size_t)(c < cl ? num_chunks + c : c) * f.slots) * f.Cp)[i];
+        acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w;
+      }
+      acc = make_float4(acc.x / norm * scale, acc.y / norm * scale, acc.z / norm * scale, acc.w / norm * scale);
+    }
+    if constexpr (VEC) {
+      reinterpret_cast<float4*>(out + (size_t)p * f.slots * f.C)[i] = acc;
+    } else {
+      const int s = i / quads, c = (i - s * quads) * 4;
+      float* __restrict__ dst = out + ((size_t)p * f.slots + s) * f.C + c;
+      dst[0] = acc.x;
+      if (c + 1 < f.C) dst[1] = acc.y;
+      if (c + 2 < f.C) dst[2] = acc.z;
+      if (c + 3 < f.C) dst[3] = acc.w;
+    }
+  }
+}
+
+// Steps per wavefront of the gradient: 64, fewer where that would leave fewer than sixteen wavefronts for each SIMD.
+inline int attr_chunk_steps(int64_t S, int C) {
+  const int64_t per = S * ceil_div(C, 256) / 16384;
+  return per >= 64 ? 64 : per <= 4 ? 4 : (int)per;
+}
+
+}  // namespace mlpsp
+
+using namespace mlpsp;
+
+MLPSP_API size_t mlpsp_train_feature_bytes(int width, int height, int target_width, int target_height, int channels, int slots,
+                                           int64_t num_steps, size_t* share_bytes, int64_t* loss_partials, size_t* row_bytes) {
+  FeatShape f;
+  if (!feat_shape(width, height, target_width, target_height, channels, slots, f) || num_steps < 0 || num_steps > 2147483647LL)
+    return 0;
+  if (share_bytes) *share_bytes = (size_t)f.T * f.NT * f.Cp * 4;
+  if (loss_partials) *loss_partials = ((int64_t)f.WF * f.HF * (f.Cp >> 2) + 255) / 256;
+  if (row_bytes) {
+    const int per = attr_chunk_steps(num_steps, channels);
+    *row_bytes = (size_t)2 * ((num_steps + per - 1) / per) * slots * f.Cp * 4;
+  }
+  return feat_kept(nullptr, f, num_steps).bytes;
+}
+
+MLPSP_API int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
+                                     const void* workspace_dev, size_t workspace_bytes, int64_t num_steps,
+                                     const void* prim_records_dev, const float* attributes_dev, const void* target_dev,
+                                     int target_is_half, int target_width, int target_height, int channels, int slots,
+                                     float beta, float temp, void* kept_dev, size_t kept_bytes, float* shares_dev,
+                                     float* loss_partials_dev, mlpsp_stream_t stream) {
+  FeatShape f;
+  if (!feat_shape(width, height, target_width, target_height, channels, slots, f) || num_pairs < 0 ||
+      num_pairs > 2147483647LL || num_steps < 0 || num_steps > 2147483647LL)
+    return MLPSP_E_ARGUMENT;
+  if (!workspace_dev || workspace_bytes < step_tables_bytes(num_pairs, f.T)) return MLPSP_E_SCRATCH;
+  const FeatKept o = feat_kept(kept_dev, f, num_steps);
+  if (!kept_dev || reinterpret_cast<uintptr_t>(kept_dev) % 256 != 0 || kept_bytes < o.bytes) return MLPSP_E_SCRATCH;
+  if (!tile_offsets_dev || !target_dev || !shares_dev || !loss_partials_dev || ((uintptr_t)shares_dev & 15u) ||
+      (num_steps > 0 && (!prim_records_dev || !attributes_dev || (uintptr_t)prim_records_dev % 128 != 0)))
+    return MLPSP_E_ARGUMENT;
+  const StepPool sp = step_pool_carve(const_cast<void*>(workspace_dev), workspace_bytes, num_pairs, f.T);
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(feature_span_kernel, dim3((unsigned)((f.T + 255) / 256)), dim3(256), 0, s, f, o);
+  MLPSP_LAUNCH_CHECK();
+  const int waves = min(kFeatWaves, ceil_div(channels, 256));
+  const dim3 grid(superblock_grid(f.ntx, f.nty), (unsigned)(f.NT >> 2), (unsigned)ceil_div(channels, 256 * waves));
+  const bool vec = channels % 4 == 0 && ((uintptr_t)attributes_dev & 15u) == 0;
+  if (f.NT > 0) {
+#define MLPSP_BLEND(SL, VEC)                                                                                            \
+  hipLaunchKernelGGL((train_feature_blend_kernel<SL, VEC>), grid, dim3(64 * waves), 0, s, f, o, tile_offsets_dev, sp.tile_base, \
+                     sp.chunk_table, sp.ids, sp.records, (const PrimRecord*)prim_records_dev, attributes_dev,            \
+                     lanes_per_row_log2(f.Cp), beta, temp, shares_dev)
+    if (slots == 1) { if (vec) MLPSP_BLEND(1, true); else MLPSP_BLEND(1, false); }
+    else if (slots == 4) { if (vec) MLPSP_BLEND(4, true); else MLPSP_BLEND(4, false); }
+    else { if (vec) MLPSP_BLEND(5, true); else MLPSP_BLEND(5, false); }
+#undef MLPSP_BLEND
+    MLPSP_LAUNCH_CHECK();
+  }
+  const dim3 join((unsigned)(((int64_t)f.WF * f.HF * (f.Cp >> 2) + 255) / 256));
+  if (target_is_half)
+    hipLaunchKernelGGL(train_feature_join_kernel<_Float16>, join, dim3(256), 0, s, f, o, shares_dev,
+                       (const _Float16*)target_dev, loss_partials_dev);
+  else
+    hipLaunchKernelGGL(train_feature_join_kernel<float>, join, dim3(256), 0, s, f, o, shares_dev, (const float*)target_dev,
+                       loss_partials_dev);
+  MLPSP_LAUNCH_CHECK();
+  return MLPSP_OK;
+}
+
+MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int width, int height,
+                                            int target_width, int target_height, int channels, int slots,
+                                            const void* kept_dev, size_t kept_bytes, const void* scratch_dev,
+                                            size_t scratch_bytes, int num_primitives, const float* loss_adjoint_dev,
+                                            float* rows_dev, float* out_dev, mlpsp_stream_t stream) {
+  FeatShape f;
+  if (!feat_shape(width, height, target_width, target_height, channels, slots, f) || num_steps < 0 ||
+      num_steps > 2147483647LL || num_primitives < 0)
+    return MLPSP_E_ARGUMENT;
+  const FeatKept o = feat_kept(const_cast<void*>(kept_dev), f, num_steps);
+  if (!kept_dev || kept_bytes < o.bytes) return MLPSP_E_SCRATCH;
+  const StepSort t = step_sort(const_cast<void*>(scratch_dev), num_steps, num_primitives);
+  if (!scratch_dev || scratch_bytes < t.bytes) return MLPSP_E_SCRATCH;
+  if (num_primitives == 0) return MLPSP_OK;
+  if (!loss_adjoint_dev || !out_dev || (num_steps > 0 && (!sorted_prim_dev || !rows_dev || ((uintptr_t)rows_dev & 15u))))
+    return MLPSP_E_ARGUMENT;
+  hipStream_t s = (hipStream_t)stream;
+  const bool vec = channels % 4 == 0 && ((uintptr_t)out_dev & 15u) == 0;
+  const int per = attr_chunk_steps(num_steps, channels), chunks = (int)((num_steps + per - 1) / per);
+  if (chunks > 0) {
+    const dim3 grid((unsigned)ceil_div(chunks, 4), (unsigned)ceil_div(channels, 256));
+#define MLPSP_ATTR(SL, VEC)                                                                                              \
+  hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, sorted_prim_dev, t.first, t.tile, t.ord,  \
+                     (int)num_steps, per, chunks, lanes_per_row_log2(f.Cp), loss_adjoint_dev, rows_dev, out_dev)
+    if (slots == 1) { if (vec) MLPSP_ATTR(1, true); else MLPSP_ATTR(1, false); }
+    else if (slots == 4) { if (vec) MLPSP_ATTR(4, true); else MLPSP_ATTR(4, false); }
+    else { if (vec) MLPSP_ATTR(5, true); else MLPSP_ATTR(5, false); }
+#undef MLPSP_ATTR
+    MLPSP_LAUNCH_CHECK();
+  }
+  if (vec)
+    hipLaunchKernelGGL(train_attr_finish_kernel<true>, dim3((unsigned)num_primitives), dim3(256), 0, s, f, t.first, per, chunks,
+                       loss_adjoint_dev, rows_dev, out_dev);
+  else
+    hipLaunchKernelGGL(train_attr_finish_kernel<false>, dim3((unsigned)num_primitives), dim3(256), 0, s, f, t.first, per,
+                       chunks, loss_adjoint_dev, rows_dev, out_dev);
+  MLPSP_LAUNCH_CHECK();
+  return MLPSP_OK;
+}

@@ -22,8 +22,8 @@ struct TrainOut {
 
 __device__ __forceinline__ bool train_not_finite(float v) { return !(__builtin_fabsf(v) <= 3.4028235e38f); }
 
-// T = float: the MLP in exact f32 (REC: layer 2 rounded as the record kernels do); _Float16 / __bf16: reduced operands,
-// with the numeric checks of the reduced-precision record forward.
+// T = float: the MLP in exact f32 (REC: layer 2 rounded as the record kernels do); _Float16 / __bf16: reduced operands.
+// All but the exact forward in the render's order report what is not finite, as the reduced-precision record forward does.
 template <typename T> struct TrainLds { DirWords dir; };
 template <> struct TrainLds<float> { DirOperands dir; };
 
@@ -36,6 +36,7 @@ __device__ __forceinline__ void train_forward_body(
     const float* __restrict__ b3, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx, int nty,
     float thr, int max_hits, const StepPool& sp, TrainOut out, TrainLds<T>& s, WalkLds& s_walk) {
   constexpr bool F32 = sizeof(T) == 4;
+  constexpr bool CHECKED = !F32 || REC;
   const int tile = superblock_tile(blockIdx.x, ntx, nty);
   if (tile < 0) return;
   const int l = threadIdx.x;
@@ -67,9 +68,9 @@ __device__ __forceinline__ void train_forward_body(
           const float x6[6] = {rd.x, rd.y, rd.z, dx, dy, dz};
           mlp_wave_mfma32<REC, true, 32>(x6, freq, att, W1, b1, W2, b2, W3, b3, p, s.dir, o, mk);
         } else {
-          bad |= hit && (train_not_finite((dx + dy) + dz) || train_not_finite(h.decay));
           bad |= mlp_wave_mfma16<T, true, true>(packed + (size_t)p * kPackStride, mask, l, dx, dy, dz, kf, s.dir, o, mk);
         }
+        if constexpr (CHECKED) bad |= hit && (train_not_finite((dx + dy) + dz) || train_not_finite(h.decay));
         const int slot = step_writer_next(sp, writer, l);
         float R = 0.f, G = 0.f, Bc = 0.f, sigma_raw = 0.f, alpha = 0.f;
         const float before = trans;
@@ -79,7 +80,7 @@ __device__ __forceinline__ void train_forward_body(
           Bc = sigmoid(o[2]);
           sigma_raw = softplus(o[3]);
           alpha = 1.f - det_exp(-(sigma_raw * h.decay));
-          if constexpr (!F32)
+          if constexpr (CHECKED)
             bad |= train_not_finite((o[0] + o[1]) + (o[2] + o[3])) || train_not_finite((R + G) + (Bc + sigma_raw)) ||
                    train_not_finite(alpha);
           const float weight = trans * alpha;
@@ -88,14 +89,14 @@ __device__ __forceinline__ void train_forward_body(
           cb = fmaf(weight, Bc, cb);
           trans = trans * (1.f - alpha);
           ++used;
-          if constexpr (!F32) bad |= train_not_finite(trans);
+          if constexpr (CHECKED) bad |= train_not_finite(trans);
         }
         if (slot >= 0) step_store(sp, slot, l, p, hit, R, G, Bc, sigma_raw, before, alpha, h.decay, o[3], dx, dy, dz, mk[0], mk[1]);
         const bool live = valid && (trans >= kTransmittanceFloor);
         over |= live && (used >= max_hits);      // np_tile_kernels.cu:3166-3168: refused, never truncated silently
         return __ballot(live) != 0ull;
       });
-  if constexpr (!F32) bad |= train_not_finite((cr + cg) + cb);
+  if constexpr (CHECKED) bad |= train_not_finite((cr + cg) + cb);
   if (l == 0) sp.tile_steps[tile] = writer.count;
   int bits = 0;
   if (__ballot(over) != 0ull) bits |= kTrainCapacity;

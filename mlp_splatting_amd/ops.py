@@ -789,12 +789,13 @@ def geometry_gradients(csr_offsets, record_indices, x6_sorted, falloff_adjoint, 
 
 class TrainFrame:
     """What a differentiable frame keeps between its forward and its backward: the workspace of its steps (one step per
-    tile and primitive that hits it) and their number.  ``steps`` is what the backward's launches are sized by."""
-    __slots__ = ("workspace", "pairs", "width", "height", "steps", "status", "chunks")
+    tile and primitive that hits it) and their number.  ``steps`` is what the backward's launches are sized by;
+    ``geometry`` the primitives' records, for the feature loss."""
+    __slots__ = ("workspace", "pairs", "width", "height", "steps", "status", "chunks", "geometry")
 
-    def __init__(self, workspace, pairs, width, height, chunks, status, steps):
+    def __init__(self, workspace, pairs, width, height, chunks, status, steps, geometry=None):
         self.workspace, self.pairs, self.width, self.height = workspace, pairs, width, height
-        self.chunks, self.status, self.steps = chunks, status, steps
+        self.chunks, self.status, self.steps, self.geometry = chunks, status, steps, geometry
 
     def with_workspace(self, workspace):
         """The same frame around ``workspace`` (None: to keep the numbers while autograd keeps the tensor)."""
@@ -808,7 +809,7 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
     room for; a frame that needs more is repeated once with what it asked for."""
     dev = rays_o.device
     lib = _lib.load()
-    pairs, n = int(order.numel()), records.numel() // _lib.PRIM_RECORD_BYTES
+    pairs, n = int(order.numel()), ws[0].shape[0]
     rgb = torch.empty(W * H, 3, dtype=torch.float32, device=dev)
     alpha = torch.empty(W * H, 1, dtype=torch.float32, device=dev)
     for _ in range(2):
@@ -828,7 +829,7 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
         if chunks * 16 <= pool_steps or pool_steps < 0:
             break
         pool_steps = chunks * 16
-    return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps)
+    return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps, records)
 
 
 class TrainGroups:
@@ -872,6 +873,8 @@ def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scale
     n = log_scales.shape[0]
     grads = [torch.empty_like(w) for w in ws[:6]]
     geo = [torch.empty_like(log_scales), torch.empty_like(log_scales), torch.empty_like(quats)]
+    if n == 0:
+        return grads + geo, torch.zeros(1, dtype=torch.int32, device=dev)
     flag = torch.empty(1, dtype=torch.int32, device=dev)
     code = _lib.load().mlpsp_train_gradients(
         _ptr(groups.prim), frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
@@ -880,3 +883,46 @@ def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scale
         *[_ptr(g) for g in grads], *[_ptr(g) for g in geo], _ptr(flag), _stream(dev))
     _check(code, "mlpsp_train_gradients")
     return grads + geo, flag
+
+
+class TrainFeature:
+    """What the streamed feature loss of a frame keeps for its gradient: residual signs and the taps' coefficients."""
+    __slots__ = ("kept", "target_size", "channels", "slots", "shares", "partials", "row_bytes")
+
+    def __init__(self, frame, target_height, target_width, channels, slots):
+        shares, partials, rows = C.c_size_t(), C.c_int64(), C.c_size_t()
+        self.kept = _lib.load().mlpsp_train_feature_bytes(
+            frame.width, frame.height, target_width, target_height, channels, slots, frame.steps, C.addressof(shares),
+            C.addressof(partials), C.addressof(rows))
+        if self.kept == 0:
+            raise RuntimeError("mlpsp_train_feature_bytes: invalid shape")
+        self.target_size, self.channels, self.slots = (target_width, target_height), channels, slots
+        self.shares, self.partials, self.row_bytes = shares.value, partials.value, rows.value
+
+
+def train_feature_l1(frame, tile_offsets, attributes, target, beta, temp):
+    """(loss, :class:`TrainFeature`, its buffer) of the steps of ``frame``; ``target`` [h, w, C] f32 or fp16, contiguous."""
+    dev = target.device
+    hf, wf, channels = target.shape
+    feature = TrainFeature(frame, hf, wf, channels, attributes.shape[1] if attributes.ndim == 3 else 1)
+    kept = torch.empty(feature.kept, dtype=torch.uint8, device=dev)
+    shares = torch.empty(feature.shares, dtype=torch.uint8, device=dev)
+    partials = torch.empty(feature.partials, dtype=torch.float32, device=dev)
+    _check(_lib.load().mlpsp_train_feature_l1(
+        _ptr(tile_offsets), frame.pairs, frame.width, frame.height, _ptr(frame.workspace), frame.workspace.numel(),
+        frame.steps, _ptr(frame.geometry), _ptr(attributes), _ptr(target), int(target.dtype == torch.float16),
+        wf, hf, channels, feature.slots, float(beta), float(temp), _ptr(kept), feature.kept, _ptr(shares), _ptr(partials),
+        _stream(dev)), "mlpsp_train_feature_l1")
+    return partials.sum(), feature, kept
+
+
+def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoint):
+    """d / d attributes of the loss of :func:`train_feature_l1` times ``loss_adjoint`` (f32 device scalar)."""
+    dev = kept.device
+    rows = torch.empty(feature.row_bytes, dtype=torch.uint8, device=dev)
+    out = torch.empty_like(attributes)
+    _check(_lib.load().mlpsp_train_feature_gradients(
+        _ptr(groups.prim), frame.steps, frame.width, frame.height, *feature.target_size, feature.channels, feature.slots,
+        _ptr(kept), feature.kept, _ptr(groups.scratch), groups.scratch.numel(), attributes.shape[0], _ptr(loss_adjoint),
+        _ptr(rows), _ptr(out), _stream(dev)), "mlpsp_train_feature_gradients")
+    return out

@@ -586,11 +586,11 @@ class TileExt:
     # walk and grouped gradients compute, with the step -- tile x primitive -- as the unit of storage)
     # ------------------------------------------------------------------------------------------
     def train_forward(self, x, width, height, threshold, *, render_order=True, precision=None,
-                      name="render_tiles_mlp_records"):
+                      name="render_tiles_mlp_records", accept=None):
         """(rgb, alpha, ops.TrainFrame) of an 8x8-tile frame with the 72->32->32->4 MLP.  ``x``: the 15 scene tensors.
         ``precision`` None: exact f32 (with ``render_order`` the bits of ``render_tiles_forward_tilecenter``, see
         :meth:`records_forward_matches_render`); "float16" / "bfloat16": the matrix cores.  The frame's ``status`` bits
-        (1 numeric, 2 hit capacity) are the caller's to judge."""
+        (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called once the lists are validated."""
         width, height = int(width), int(height)
         _chk(width > 0 and height > 0 and x[0].shape[0] == width * height, "B must equal W*H for tile renderer")
         self._check_base(*x[:9])
@@ -600,6 +600,8 @@ class TileExt:
         n_tiles = ops.num_tiles(width, height, 8, 8)
         with torch.cuda.device(x[0].device), self.uncached():
             self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
+            if accept is not None:
+                accept()
             rec = self._records(x[2], x[3], x[4])
             order = x[5]
             if x[5].numel() > 0:
@@ -613,6 +615,33 @@ class TileExt:
                                                   packed=packed, bf16=precision == "bfloat16")
             with self._lock:      # a quarter more than this frame needed, in whole chunks, for the next one
                 self._steps_per_tile = max(16, -(-frame.chunks * 20 // n_tiles))
+        return rgb, alpha, frame
+
+    def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision):
+        """:meth:`train_forward` on the matrix cores under the contract and policy of
+        :meth:`render_tiles_training_records_wmma`: non-finite inputs are refused, a numeric overflow discards the
+        reduced-precision pass and repeats the frame in f32, hit capacity raises; same counters."""
+        width, height = int(width), int(height)
+        self._check_training_wmma(x, width, height, 8, threshold, beta, temp, precision)
+
+        def accept():
+            self._refuse_nonfinite(x)
+            self._count_training_mfma(0)
+        rgb, alpha, frame = self.train_forward(x, width, height, threshold, precision=precision, accept=accept,
+                                               name="render_tiles_training_records_wmma")
+        if frame.status & 2:
+            self._count_training_mfma(4)
+            raise RuntimeError(f"Training WMMA hit capacity {self.max_hits} exceeded; refusing truncated records")
+        if frame.status & 1:
+            self._count_training_mfma(1)
+            warnings.warn("Training WMMA numeric overflow: discarding both mixed passes and rerunning the whole "
+                          "FP32 record forward")
+            del frame
+            rgb, alpha, frame = self.train_forward(x, width, height, threshold, render_order=False)
+            self.refuse_overflow(frame)
+            if frame.status & 1:
+                self._count_training_mfma(2)
+                raise RuntimeError("Training WMMA scalar FP32 fallback records are nonfinite")
         return rgb, alpha, frame
 
     def refuse_overflow(self, frame, name="render_tiles_mlp_records"):
@@ -646,17 +675,12 @@ class TileExt:
         with self._lock:
             self._training_mfma_stats[index] += 1
 
-    def render_tiles_training_records_wmma(self, x, width, height, tile, threshold, beta, temp, precision):
-        """The records of :meth:`render_tiles_training_records` with the MLP on the matrix cores in ``precision``
-        ("float16" or "bfloat16") and everything else in the same f32 expressions (wrapper and policy of
-        training_wmma.cuh:267-357): non-finite inputs are refused, a numeric overflow of the reduced-precision
-        pass discards it and repeats the whole frame with the scalar f32 record forward, hit capacity and a
-        count/emit disagreement raise."""
+    def _check_training_wmma(self, x, width, height, tile, threshold, beta, temp, precision):
+        """Argument contract of the reduced-precision training forward (training_wmma.cuh:267-312): shapes and types.
+        ``x``: the 15 scene tensors, and the two adjoint placeholders where the entry point takes them."""
         import math
-        _chk(len(x) == 17, "Training WMMA requires 15 scene inputs and two RGB/T adjoint placeholders")
         _chk(int(tile) == 8, "Training WMMA requires tile8")
         _chk(precision in ("float16", "bfloat16"), "Training WMMA precision must be float16 or bfloat16")
-        width, height = int(width), int(height)
         _chk(0 < width <= 2147483647 and 0 < height <= 2147483647 and width <= 2147483647 // height,
              "Training WMMA image dimensions exceed int32 pixel indexing")
         thr32 = torch.tensor(float(threshold), dtype=torch.float32).item()
@@ -676,12 +700,28 @@ class TileExt:
         _chk(x[7].dim() == 1 and x[7].numel() == 6 and x[8].shape == x[7].shape)
         _chk(tuple(x[9].shape) == (n, 32, 72) and tuple(x[10].shape) == (n, 32) and tuple(x[11].shape) == (n, 32, 32))
         _chk(x[12].shape == x[10].shape and tuple(x[13].shape) == (n, 4, 32) and tuple(x[14].shape) == (n, 4))
-        _chk(x[15].shape == x[0].shape and x[16].dim() == 1 and x[16].numel() == pixels)
+        if len(x) == 17:
+            _chk(x[15].shape == x[0].shape and x[16].dim() == 1 and x[16].numel() == pixels)
+
+    @staticmethod
+    def _refuse_nonfinite(x):
+        nonfinite = ops.all_finite_flag([t for i, t in enumerate(x) if i not in (5, 6)])
+        _chk(int(nonfinite.item()) == 0, "Training WMMA input is nonfinite; refusing unsafe forward/fallback")
+
+    def render_tiles_training_records_wmma(self, x, width, height, tile, threshold, beta, temp, precision):
+        """The records of :meth:`render_tiles_training_records` with the MLP on the matrix cores in ``precision``
+        ("float16" or "bfloat16") and everything else in the same f32 expressions (wrapper and policy of
+        training_wmma.cuh:267-357): non-finite inputs are refused, a numeric overflow of the reduced-precision
+        pass discards it and repeats the whole frame with the scalar f32 record forward, hit capacity and a
+        count/emit disagreement raise."""
+        _chk(len(x) == 17, "Training WMMA requires 15 scene inputs and two RGB/T adjoint placeholders")
+        width, height = int(width), int(height)
+        self._check_training_wmma(x, width, height, tile, threshold, beta, temp, precision)
+        n = x[2].shape[0]
         name = "render_tiles_training_records_wmma"
         with torch.cuda.device(x[0].device), self.uncached():
             self._validate(x[5], x[6], ops.num_tiles(width, height, 8, 8), self.max_tile_prims, n, name)
-            nonfinite = ops.all_finite_flag([t for i, t in enumerate(x) if i not in (5, 6)])
-            _chk(int(nonfinite.item()) == 0, "Training WMMA input is nonfinite; refusing unsafe forward/fallback")
+            self._refuse_nonfinite(x)
             self._count_training_mfma(0)
             bf16 = precision == "bfloat16"
             rec = self._records(x[2], x[3], x[4])

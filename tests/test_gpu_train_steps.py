@@ -69,3 +69,49 @@ def test_reduced_forward_steps_are_those_of_its_records(device, oracle_mod, prec
     got = ext.backward_from_steps(frame, ops.train_group(frame, base[6], 300), base, g_rgb, g_t)
     for i, (g, w) in enumerate(zip(got, want)):
         assert float((g - w).norm()) <= 1e-4 * float(w.norm()), i
+
+
+#                target, channels, slots
+@pytest.mark.parametrize("wf,hf,channels,slots", [
+    (33, 17, 5, 4),        # a target for every pixel: nine taps to a tile and axis, shared between tiles
+    (8, 4, 64, 4), (8, 4, 67, 5), (8, 4, 516, 1),     # a quarter; one, two and four lane groups; more than one wavefront
+    (13, 7, 130, 5),       # a ratio that is no whole number
+    (3, 2, 256, 4),        # more pixels than a tile between two targets: tiles without one
+    (1, 1, 3, 1)])
+@pytest.mark.parametrize("half", [False, True])
+def test_feature_loss_of_steps_is_that_of_records(device, oracle_mod, wf, hf, channels, slots, half):
+    from mlp_splatting_amd import ops, primitive_csr, record_feature_loss
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr, base = _scene(device, oracle_mod, 300, 33, 17, 1.0, False)
+    ext = TileExt()
+    gen = torch.Generator(device=device).manual_seed(7)
+    attributes = torch.randn(300, slots, channels, device=device, generator=gen)
+    attributes = attributes[:, 0].contiguous() if slots == 1 else attributes
+    target = torch.randn(hf, wf, channels, device=device, generator=gen)
+    target = target.half() if half else target
+    x = base + [torch.zeros_like(base[0]), torch.zeros(33 * 17, device=device)]
+    records = ext.render_tiles_training_records(x, 33, 17, 8, fr.thr, 1.5, 2.0)
+    want_loss, signs, _ = record_feature_loss.streaming_feature_l1(records, attributes, target, 33, 17)
+    csr = primitive_csr.group_records(records[2], records[3], records[3].new_zeros(records[2].numel(), 4), 300, records[5])
+    want = record_feature_loss.feature_weight_gradients(records, csr, signs, attributes, 33, 17, mixed=False)
+    _, _, frame = ext.train_forward(base, 33, 17, fr.thr, render_order=False)
+    loss, feature, kept = ops.train_feature_l1(frame, base[6], attributes, target, 1.5, 2.0)
+    got = ops.train_feature_gradients(frame, ops.train_group(frame, base[6], 300), feature, kept, attributes,
+                                      torch.tensor(0.75, device=device))
+    torch.testing.assert_close(loss, want_loss, rtol=1e-6, atol=0)
+    assert got.shape == want.shape
+    torch.testing.assert_close(got, want * 0.75, rtol=1e-4, atol=2e-6 * float(want.abs().max()))
+
+
+def test_feature_training_step_of_an_empty_scene(device, oracle_mod):
+    from mlp_splatting_amd.record_training import Frame as TrainingFrame, feature_training_step
+    fr, base = _scene(device, oracle_mod, 40, 33, 17, 1.0, False)
+    empty = [t[:0].clone() if i in (2, 3, 4, *range(9, 15)) else t for i, t in enumerate(base)]
+    empty[5], empty[6] = empty[5][:0].clone(), torch.zeros_like(empty[6])
+    leaves = [t.requires_grad_() if i in (2, 3, 4, *range(9, 15)) else t for i, t in enumerate(empty)]
+    attributes = torch.zeros(0, 4, 16, device=device, requires_grad=True)
+    target = torch.ones(4, 8, 16, device=device)
+    rgb, loss = feature_training_step(leaves, attributes, target, TrainingFrame(33, 17, fr.thr, 1.5, 2.0))
+    assert float(rgb.detach().abs().max()) == 0.0 and float(loss.detach()) == 1.0
+    (rgb.sum() + loss).backward()
+    assert attributes.grad.shape == attributes.shape
