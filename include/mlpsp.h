@@ -565,7 +565,7 @@ int mlpsp_train_reverse(const int32_t* tile_offsets_dev, int64_t num_pairs, int 
                         const float* grad_t_dev, float* d4_dev, float* falloff_dev, mlpsp_stream_t stream);
 size_t mlpsp_train_scratch_bytes(int64_t num_steps, int num_primitives);
 int mlpsp_train_group(const int32_t* sorted_prim_dev, const int64_t* permutation_dev, const int32_t* step_slot_dev,
-                      const int32_t* step_tile_dev, int64_t num_steps, int num_primitives, void* scratch_dev,
+                      const int32_t* step_tile_dev, int64_t num_steps, int num_primitives, int width, void* scratch_dev,
                       size_t scratch_bytes, mlpsp_stream_t stream);
 int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int64_t num_pairs, int width, int height,
                           const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,

@@ -31,16 +31,16 @@ __global__ __launch_bounds__(64) void grouped_vjp16_kernel(
     const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, int segment,
     float* __restrict__ partial) {
-  __shared__ __attribute__((aligned(16))) int32_t s_mask[2][32];
+  __shared__ __attribute__((aligned(16))) Vjp16Operands<T> w;
+  __shared__ __attribute__((aligned(16))) Vjp16Masks s_mask;
   const int lane = threadIdx.x, n = lane & 31, g = lane >> 5;
   const long long group = blockIdx.x;
   const long long p = group_prim[group];
   const long long begin = group_start[group];
   const long long seg_end = begin + segment, list_end = offsets[p + 1];
   const long long end = seg_end < list_end ? seg_end : list_end;
-  Vjp16Operands<T> w;
-  w.select(n, g);
-  w.load(W1, b1, W2, b2, W3, p, n, g);
+  w.select(lane);
+  w.load(W1, b1, W2, b2, W3, (size_t)p, lane);
   float kf[6];
 #pragma unroll
   for (int f = 0; f < 6; ++f) kf[f] = (freq[f] * att[f]) * 0.159154943f;
@@ -55,8 +55,12 @@ __global__ __launch_bounds__(64) void grouped_vjp16_kernel(
     for (int c = 0; c < 3; ++c) x[c] = live ? x6[rec * 6 + 3 * g + c] : 0.f;
     float4 d3 = make_float4(0.f, 0.f, 0.f, 0.f);
     if (live && g == 0) d3 = *reinterpret_cast<const float4*>(grad4 + rec * 4);
-    if constexpr (SAVED) s_mask[g][n] = live ? masks[rec * 2 + g] : 0;      // group 0 fetches layer 1, group 1 layer 2
-    vjp16_block<T, SAVED>(w, sum, x, d3, live, s_mask, kf, b1 + p * 32, b2 + p * 32, scale, n, g);
+    uint2 words = make_uint2(0u, 0u);
+    if constexpr (SAVED) {
+      if (live) words = make_uint2((uint32_t)masks[rec * 2], (uint32_t)masks[rec * 2 + 1]);
+      s_mask.put(g, n, g ? words.y : words.x);
+    }
+    vjp16_block<T, SAVED>(w, sum, x, d3, live, s_mask, words.y, kf, scale, lane);
   }
   vjp16_store(sum, packed_grad_rows(partial + group * kGradFloats), 1.f / scale, lane);
 }

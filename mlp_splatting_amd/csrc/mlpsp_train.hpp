@@ -70,10 +70,12 @@ inline StepPool step_pool_carve(void* workspace, size_t bytes, int64_t num_pairs
   return sp;
 }
 
-// The steps sorted by primitive: first sorted position of every primitive [N + 1]; pool slot, tile and number in tile order
-// of the sorted steps [S].  Every buffer that holds them begins with them.
+// The steps sorted by primitive: first sorted position of every primitive [N + 1]; of the sorted steps [S] pool slot,
+// number in tile order, tile and pixel number of the tile's first pixel -- one 16-byte read.  Every buffer that holds them
+// begins with them.
 struct StepSort {
-  int32_t *first, *slot, *tile, *ord;
+  int32_t* first;
+  int4* step;
   size_t bytes;
 };
 inline StepSort step_sort(void* base, int64_t S, int N) {
@@ -81,12 +83,8 @@ inline StepSort step_sort(void* base, int64_t S, int N) {
   unsigned char* p = (unsigned char*)base;
   t.first = (int32_t*)p;
   p += step_align(((size_t)N + 1) * 4);
-  t.slot = (int32_t*)p;
-  p += step_align((size_t)S * 4);
-  t.tile = (int32_t*)p;
-  p += step_align((size_t)S * 4);
-  t.ord = (int32_t*)p;
-  p += step_align((size_t)S * 4);
+  t.step = (int4*)p;
+  p += step_align((size_t)S * 16);
   t.bytes = (size_t)(p - (unsigned char*)base);
   return t;
 }

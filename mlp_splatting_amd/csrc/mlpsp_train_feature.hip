@@ -289,10 +289,9 @@ __global__ __launch_bounds__(256) void train_feature_join_kernel(FeatShape f, Fe
 // One wavefront = one chunk of the sorted steps x 256 channels: sum over the steps' targets of k[slot][target] sign.
 template <int SLOTS, bool VEC>
 __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o, const int32_t* __restrict__ prim,
-                                                         const int32_t* __restrict__ first, const int32_t* __restrict__ step_tile,
-                                                         const int32_t* __restrict__ step_ord, int S, int chunk_steps,
-                                                         int num_chunks, int lpr_log2, const float* __restrict__ adjoint,
-                                                         float* __restrict__ rows, float* __restrict__ out) {
+                                                         const int32_t* __restrict__ first, const int4* __restrict__ step, int S,
+                                                         int chunk_steps, int num_chunks, int lpr_log2,
+                                                         const float* __restrict__ adjoint, float* __restrict__ rows, float* __restrict__ out) {
   const int chunk = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
   if (chunk >= num_chunks) return;
   const int chunk_end = min(S, (chunk + 1) * chunk_steps);
@@ -310,8 +309,9 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) acc[s] = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int i = pos + sub; i < end; i += nsub) {
-      const int tile = step_tile[i], groups = o.groups[tile];
-      const float* __restrict__ k = o.k + (size_t)step_ord[i] * k_stride;
+      const int4 at = step[i];
+      const int tile = at.z, groups = o.groups[tile];
+      const float* __restrict__ k = o.k + (size_t)at.y * k_stride;
       const int8_t* __restrict__ sg = o.signs + (size_t)tile * f.NT * f.Cp + cs;
       for (int g = 0; g < groups; ++g, k += 4 * SLOTS, sg += 4 * f.Cp) {
         int word[4];
@@ -494,7 +494,7 @@ MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int6
   if (chunks > 0) {
     const dim3 grid((unsigned)ceil_div(chunks, 4), (unsigned)ceil_div(channels, 256));
 #define MLPSP_ATTR(SL, VEC)                                                                                              \
-  hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, sorted_prim_dev, t.first, t.tile, t.ord,  \
+  hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, sorted_prim_dev, t.first, t.step,         \
                      (int)num_steps, per, chunks, lanes_per_row_log2(f.Cp), loss_adjoint_dev, rows_dev, out_dev)
     if (slots == 1) { if (vec) MLPSP_ATTR(1, true); else MLPSP_ATTR(1, false); }
     else if (slots == 4) { if (vec) MLPSP_ATTR(4, true); else MLPSP_ATTR(4, false); }

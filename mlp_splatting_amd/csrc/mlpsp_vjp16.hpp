@@ -28,9 +28,11 @@ constexpr int kGradFloats = 3524;   // W1 2304 | b1 32 | W2 1024 | b2 32 | W3 12
 //  (2) A tile that no product yields in the needed orientation (the encoding, the output adjoints) is
 //      transposed by the matrix core itself: mfma(X, I) with a 0/1 selection operand I returns X unit-major,
 //      exactly (one non-zero term per sum).
-// Per block of 32 records: 32 MFMAs (34 without saved masks) against 20 for a formulation that transposes
-// through LDS, and no LDS traffic except the 64 mask words: 11.3 -> 2.8 ms for 38.6 M records, with one
-// wavefront per SIMD (342 registers; capped at 256 the compiler spills 84 and the kernel takes 4.5 ms).
+// Per block of 32 records: 30 MFMAs of 32 clocks and 8 small ones (32 without saved masks) against 20 for a formulation
+// that transposes through LDS.  The 4x32 gradient of W3 and the bias gradient of layer 2 are 4x4x4 products: their 4 rows
+// would fill an eighth of a 32x32 tile.  Bound by the ~350 vector instructions of a block: a wavefront that is alone on its
+// SIMD issues them at half the rate, so the weight operands lie in LDS and two wavefronts fit (252 registers; with the
+// operands in registers 342 and one wavefront).  648,000 steps of 64 records: 3.18 -> 2.06 ms.
 //
 // k-slot order of the encoding (both the X operand of layer 1 and W1's operand): lane group g owns input
 // components 3g..3g+2; its slot q = 8 s + j of K-step s (q < 36) is pair t = q / 2 = 6 c + f (component
@@ -92,42 +94,48 @@ __device__ __forceinline__ Pack8 active_tile(const Pack8& h) {
     for (int d = 0; d < 4; ++d) r.s[s][d] = active_halves(h.s[s][d]);
   return r;
 }
-// AND-masks of a unit-major tile from saved mask words: w[i] = the mask word of the record in register i,
-// bit = this lane's unit
-__device__ __forceinline__ Pack8 mask_tile_unit_major(const int32_t w[16], int bit) {
+// 0xFFFF in each half whose bit 15 - up is set, 0 in the other
+__device__ __forceinline__ unsigned spread_bit(unsigned halves, vu16x2 up) {
+  typedef short vi16x2 __attribute__((ext_vector_type(2)));
+  const vu16x2 top = __builtin_bit_cast(vu16x2, halves) << up;
+  return __builtin_bit_cast(unsigned, (vi16x2)(__builtin_bit_cast(vi16x2, top) >> (vi16x2){15, 15}));
+}
+// Mask words of the block's records, split in halves: half h of the word of record m at [h][m].  A lane that looks at
+// unit n takes the half that holds bit n, four consecutive records in one 8-byte read, already paired as the packed
+// tiles pair them.
+struct Vjp16Masks {
+  unsigned short half[2][2][32];     // [layer][half][record]
+  __device__ __forceinline__ void put(int layer, int record, uint32_t word) {
+    half[layer][0][record] = (unsigned short)word;
+    half[layer][1][record] = (unsigned short)(word >> 16);
+  }
+};
+__device__ __forceinline__ Pack8 mask_tile_unit_major(const unsigned short (*half)[32], int n, int g) {
+  const unsigned short* __restrict__ src = half[n >> 4] + 4 * g;
+  const unsigned short shift = (unsigned short)(15 - (n & 15));
+  const vu16x2 up = {shift, shift};
+  Pack8 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint2 v = *reinterpret_cast<const uint2*>(src + 8 * q);
+    r.s[q >> 1][2 * (q & 1)] = spread_bit(v.x, up);
+    r.s[q >> 1][2 * (q & 1) + 1] = spread_bit(v.y, up);
+  }
+  return r;
+}
+// ... and of a record-major tile whose register i holds unit hidden_unit(i, g): the two units of a pair are bits k and
+// k + 16 of this lane's word
+__device__ __forceinline__ Pack8 mask_tile_record_major(uint32_t word, int g) {
+  const unsigned mine = (word >> (8 * g)) & 0x00ff00ffu;
   Pack8 r;
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const int i = 8 * s + 2 * d;
-      const unsigned lo = (unsigned)__builtin_amdgcn_sbfe(w[i], bit, 1), hi = (unsigned)__builtin_amdgcn_sbfe(w[i + 1], bit, 1);
-      r.s[s][d] = (lo & 0xFFFFu) | (hi << 16);
+      const unsigned short shift = (unsigned short)(15 - (4 * s + d));
+      r.s[s][d] = spread_bit(mine, vu16x2{shift, shift});
     }
   return r;
-}
-// ... and of a record-major tile: `word` = the mask word of this lane's record, register i is unit d_row(i, g)
-__device__ __forceinline__ Pack8 mask_tile_record_major(int32_t word, int g) {
-  const int shifted = word >> (4 * g);
-  Pack8 r;
-#pragma unroll
-  for (int s = 0; s < 2; ++s)
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int i = 8 * s + 2 * d, u = 8 * (i / 4) + (i % 4);      // d_row(i, 0); i is even, so i + 1 is unit u + 1
-      const unsigned lo = (unsigned)__builtin_amdgcn_sbfe(shifted, u, 1), hi = (unsigned)__builtin_amdgcn_sbfe(shifted, u + 1, 1);
-      r.s[s][d] = (lo & 0xFFFFu) | (hi << 16);
-    }
-  return r;
-}
-template <typename T>
-__device__ __forceinline__ float sum_tile(const Pack8& r) {
-  float t = 0.f;
-#pragma unroll
-  for (int s = 0; s < 2; ++s)
-#pragma unroll
-    for (int d = 0; d < 4; ++d) t += Unpack<T>::lo(r.s[s][d]) + Unpack<T>::hi(r.s[s][d]);
-  return t;
 }
 template <typename T>
 __device__ __forceinline__ vf32x16 mma2(const Pack8& a, const Pack8& b, vf32x16 acc) {
@@ -141,32 +149,34 @@ __device__ __forceinline__ vf32x16 splat16(float v) {
   return r;
 }
 
-// The primitive's weights as operands, one unit (n) per lane, and the selection operands.
+// The primitive's weights as operands, one unit (n) per lane, and the selection operands, in LDS: they change per primitive
+// and are read once per block (15 reads of 16 bytes), which leaves the registers to the sums and the tiles.
 template <typename T>
 struct Vjp16Operands {
-  u32x4 w1op[5], w3op, out_sel, k_sel[2];
-  Pack8 w2op, w2top;     // W2[n][u] and W2[u][n] over the units u = d_row(8 s + j, g) of this lane's k-slots
-  float bias1, bias2;
-  unsigned one_lo;
+  u32x4 w1[5][64], w2[2][64], w2t[2][64];  // w2: W2[n][u] over the units u = d_row(8 s + j, g) of a lane's k-slots; w2t:
+                                           // W2[u][n] over u = hidden_unit(8 s + j, g)
+  u32x4 k_sel[2][64];                      // returns K-step 2c + h of the encoding as columns 32c + n
+  u32x2 w3u[64], w3r[64];                  // W3 column of unit n, of unit hidden_unit_of_row(n) (k-slots: the four outputs)
+  float bias1[32], bias2[32];
 
-  __device__ __forceinline__ void select(int n, int g) {
-    // out_sel returns the output adjoints unit-major (column n = output n < 4); k_sel[h] returns K-step 2c + h of the
-    // encoding as columns 32c + n
-    const unsigned one_hi = Ops<T>::pack2(0.f, 1.f);
-    one_lo = Ops<T>::pack2(1.f, 0.f);
-    out_sel = k_sel[0] = k_sel[1] = u32x4{0u, 0u, 0u, 0u};
-    if (g == 0 && n < 4) out_sel[n >> 1] = (n & 1) ? one_hi : one_lo;
-    const unsigned v = (n & 1) ? one_hi : one_lo;
+  // What is the same for every primitive.
+  __device__ __forceinline__ void select(int lane) {
+    const int n = lane & 31, g = lane >> 5;
+    const unsigned v = (n & 1) ? Ops<T>::pack2(0.f, 1.f) : Ops<T>::pack2(1.f, 0.f);
     const bool mine = ((n >> 3) & 1) == g;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      u32x4 k;
 #pragma unroll
-      for (int d = 0; d < 4; ++d) k_sel[h][d] = (mine && (n >> 4) == h && ((n & 7) >> 1) == d) ? v : 0u;
+      for (int d = 0; d < 4; ++d) k[d] = (mine && (n >> 4) == h && ((n & 7) >> 1) == d) ? v : 0u;
+      k_sel[h][lane] = k;
+    }
   }
 
   __device__ __forceinline__ void load(const float* __restrict__ W1, const float* __restrict__ b1,
                                        const float* __restrict__ W2, const float* __restrict__ b2,
-                                       const float* __restrict__ W3, long long p, int n, int g) {
+                                       const float* __restrict__ W3, size_t p, int lane) {
+    const int n = lane & 31, g = lane >> 5;
     {
       const float* __restrict__ row = W1 + p * 2304 + n * 72 + 18 * g;
       float ws[18], wc[18];
@@ -179,12 +189,15 @@ struct Vjp16Operands {
         wc[t + 1] = c.y;
       }
 #pragma unroll
-      for (int s = 0; s < 5; ++s)
+      for (int s = 0; s < 5; ++s) {
+        u32x4 v;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           const int t = 4 * s + d;
-          w1op[s][d] = t < 18 ? Ops<T>::pack2(ws[t], wc[t]) : 0u;
+          v[d] = t < 18 ? Ops<T>::pack2(ws[t], wc[t]) : 0u;
         }
+        w1[s][lane] = v;
+      }
     }
     {
       const float* __restrict__ row = W2 + p * 1024 + n * 32;
@@ -193,43 +206,74 @@ struct Vjp16Operands {
       for (int s = 0; s < 2; ++s) {
         const float4 lo = *reinterpret_cast<const float4*>(row + 16 * s + 4 * g);
         const float4 hi = *reinterpret_cast<const float4*>(row + 16 * s + 8 + 4 * g);
-        w2op.s[s] = u32x4{Ops<T>::pack2(lo.x, lo.y), Ops<T>::pack2(lo.z, lo.w), Ops<T>::pack2(hi.x, hi.y), Ops<T>::pack2(hi.z, hi.w)};
+        w2[s][lane] = u32x4{Ops<T>::pack2(lo.x, lo.y), Ops<T>::pack2(lo.z, lo.w), Ops<T>::pack2(hi.x, hi.y), Ops<T>::pack2(hi.z, hi.w)};
         float c[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) c[j] = col[(16 * s + 8 * (j / 4) + 4 * g + j % 4) * 32];
-        w2top.s[s] = u32x4{Ops<T>::pack2(c[0], c[1]), Ops<T>::pack2(c[2], c[3]), Ops<T>::pack2(c[4], c[5]), Ops<T>::pack2(c[6], c[7])};
+        for (int j = 0; j < 8; ++j) c[j] = col[hidden_unit(8 * s + j, g) * 32];
+        w2t[s][lane] = u32x4{Ops<T>::pack2(c[0], c[1]), Ops<T>::pack2(c[2], c[3]), Ops<T>::pack2(c[4], c[5]), Ops<T>::pack2(c[6], c[7])};
       }
     }
-    // W3^T: k-slots = the four outputs (group 0, slots 0..3)
-    w3op = u32x4{0u, 0u, 0u, 0u};
-    if (g == 0) {
-      const float* __restrict__ col = W3 + p * 128 + n;
-      w3op[0] = Ops<T>::pack2(col[0], col[32]);
-      w3op[1] = Ops<T>::pack2(col[64], col[96]);
+    // W3^T: k-slots = the four outputs (group 0, slots 0..3; group 1's are zero)
+    {
+      const float* __restrict__ u = W3 + p * 128 + n;
+      const float* __restrict__ r = W3 + p * 128 + hidden_unit_of_row(n);
+      w3u[lane] = g ? u32x2{0u, 0u} : u32x2{Ops<T>::pack2(u[0], u[32]), Ops<T>::pack2(u[64], u[96])};
+      w3r[lane] = g ? u32x2{0u, 0u} : u32x2{Ops<T>::pack2(r[0], r[32]), Ops<T>::pack2(r[64], r[96])};
     }
-    bias1 = b1[p * 32 + n];
-    bias2 = b2[p * 32 + n];
+    if (g == 0) {
+      bias1[n] = b1[p * 32 + n];
+      bias2[n] = b2[p * 32 + n];
+    }
   }
 };
 
 struct Vjp16Sums {
-  vf32x16 gw1[3], gw2, gw3;
-  float gb2, gb3[4];
+  vf32x16 gw1[3], gw2;
+  f32x4 gw3, gb2;
+  float gb3[4];
   __device__ __forceinline__ void clear() {
-    gw1[0] = gw1[1] = gw1[2] = gw2 = gw3 = splat16(0.f);
-    gb2 = gb3[0] = gb3[1] = gb3[2] = gb3[3] = 0.f;
+    gw1[0] = gw1[1] = gw1[2] = gw2 = splat16(0.f);
+    gw3 = gb2 = f32x4{0.f, 0.f, 0.f, 0.f};
+    gb3[0] = gb3[1] = gb3[2] = gb3[3] = 0.f;
   }
 };
 
+// The four 4x4x4 products over the records of two packed unit-major tiles: every group of four lanes is a block of its
+// own, row l % 4 of a against column l % 4 of b.
+template <typename T>
+__device__ __forceinline__ f32x4 mma4(const Pack8& a, const Pack8& b, f32x4 acc) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int s = q >> 1, d = 2 * (q & 1);
+    acc = Ops<T>::mfma4(u32x2{a.s[s][d], a.s[s][d + 1]}, u32x2{b.s[s][d], b.s[s][d + 1]}, acc);
+  }
+  return acc;
+}
+
+// The bias of a record-major tile: register i holds unit d_row(i, g) (rows), or of a row order of the caller's
+__device__ __forceinline__ vf32x16 bias_rows(const float* bias, int g) {
+  vf32x16 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(bias + 8 * q + 4 * g);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[4 * q + k] = v[k];
+  }
+  return r;
+}
+
 // One block of 32 records.  Lane (n, g): record n; x = its three inputs of group g, d3 = the record's output adjoints
-// (lanes of group 0; zeros in group 1); SAVED: s_mask[g][n] holds mask word g of record n already.  b1r, b2r: the
-// primitive's bias rows in global memory (L1-resident).
+// (lanes of group 0; zeros in group 1); SAVED: `masks` holds the mask words of the block's records, mask2 is that of
+// record n and layer 2.
 template <typename T, bool SAVED>
 __device__ __forceinline__ void vjp16_block(const Vjp16Operands<T>& w, Vjp16Sums& sum, const float x[3], float4 d3,
-                                            bool live, const int32_t (*s_mask)[32], const float kf[6],
-                                            const float* __restrict__ b1r, const float* __restrict__ b2r, float scale,
-                                            int n, int g) {
+                                            bool live, const Vjp16Masks& masks, uint32_t mask2, const float kf[6],
+                                            float scale, int lane) {
+  // (opaque: the operands are to be read here, not kept in registers from block to block)
+  asm volatile("" : "+v"(lane));
+  const int n = lane & 31, g = lane >> 5;
   const vf32x16 zero = splat16(0.f);
+  const unsigned one_lo = Ops<T>::pack2(1.f, 0.f), one_hi = Ops<T>::pack2(0.f, 1.f);
   // ---- encoding, record-major
   u32x4 enc[5];
 #pragma unroll
@@ -241,7 +285,7 @@ __device__ __forceinline__ void vjp16_block(const Vjp16Operands<T>& w, Vjp16Sums
         const float rev = x[t / 6] * kf[t % 6];
         enc[s][d] = live ? Ops<T>::pack2(__builtin_amdgcn_sinf(rev), __builtin_amdgcn_cosf(rev)) : 0u;
       } else if (t == 18) {
-        enc[s][d] = (live && g == 0) ? w.one_lo : 0u;      // the constant input (k = 68): bias gradient of layer 1
+        enc[s][d] = (live && g == 0) ? one_lo : 0u;      // the constant input (k = 68): bias gradient of layer 1
       } else {
         enc[s][d] = 0u;
       }
@@ -255,76 +299,54 @@ __device__ __forceinline__ void vjp16_block(const Vjp16Operands<T>& w, Vjp16Sums
   sum.gb3[3] += Unpack<T>::hi(d3op[1]);
 
   // ---- layer 1 in both orientations
-  vf32x16 a_rec, a_unit = splat16(w.bias1);
-  {
-    // record-major: register i is unit d_row(i, g); its bias comes from global memory (L1-resident)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 v = *reinterpret_cast<const float4*>(b1r + 8 * q + 4 * g);
-      a_rec[4 * q] = v.x;
-      a_rec[4 * q + 1] = v.y;
-      a_rec[4 * q + 2] = v.z;
-      a_rec[4 * q + 3] = v.w;
-    }
-  }
+  vf32x16 a_rec = bias_rows(w.bias1, g), a_unit = splat16(w.bias1[n]);
 #pragma unroll
   for (int s = 0; s < 5; ++s) {
-    a_rec = Ops<T>::mfma(w.w1op[s], enc[s], a_rec);
-    a_unit = Ops<T>::mfma(enc[s], w.w1op[s], a_unit);
+    const u32x4 w1 = w.w1[s][lane];
+    a_rec = Ops<T>::mfma(w1, enc[s], a_rec);
+    a_unit = Ops<T>::mfma(enc[s], w1, a_unit);
   }
   const Pack8 h1_rec = relu_tile(pack_tile<T>(a_rec));
   const Pack8 h1_unit = relu_tile(pack_tile<T>(a_unit));
   // ---- layer 2: unit-major for the W3 gradient; record-major only to learn which units are active
-  const Pack8 h2_unit = relu_tile(pack_tile<T>(mma2<T>(h1_rec, w.w2op, splat16(w.bias2))));
+  const Pack8 w2 = {{w.w2[0][lane], w.w2[1][lane]}};
+  const Pack8 h2_unit = relu_tile(pack_tile<T>(mma2<T>(h1_rec, w2, splat16(w.bias2[n]))));
   Pack8 act1_unit, act2_unit, act2_rec;
   if constexpr (SAVED) {
-    int32_t words[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int4 v = *reinterpret_cast<const int4*>(&s_mask[0][8 * q + 4 * g]);
-      words[4 * q] = v.x;
-      words[4 * q + 1] = v.y;
-      words[4 * q + 2] = v.z;
-      words[4 * q + 3] = v.w;
-    }
-    act1_unit = mask_tile_unit_major(words, n);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int4 v = *reinterpret_cast<const int4*>(&s_mask[1][8 * q + 4 * g]);
-      words[4 * q] = v.x;
-      words[4 * q + 1] = v.y;
-      words[4 * q + 2] = v.z;
-      words[4 * q + 3] = v.w;
-    }
-    act2_unit = mask_tile_unit_major(words, n);
-    act2_rec = mask_tile_record_major(s_mask[1][n], g);
+    act1_unit = mask_tile_unit_major(masks.half[0], n, g);
+    act2_unit = mask_tile_unit_major(masks.half[1], n, g);
+    act2_rec = mask_tile_record_major(mask2, g);
   } else {
+    // rows of the product = units hidden_unit(i, g), as mask_tile_record_major has them
+    const int m = (lane & 32) | hidden_unit_of_row(n);
+    const Pack8 w2r = {{w.w2[0][m], w.w2[1][m]}};
     vf32x16 a2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 v = *reinterpret_cast<const float4*>(b2r + 8 * q + 4 * g);
-      a2[4 * q] = v.x;
-      a2[4 * q + 1] = v.y;
-      a2[4 * q + 2] = v.z;
-      a2[4 * q + 3] = v.w;
-    }
+    for (int i = 0; i < 16; ++i) a2[i] = w.bias2[hidden_unit(i, 0) + 8 * g];
     act1_unit = active_tile(h1_unit);
     act2_unit = active_tile(h2_unit);
-    act2_rec = active_tile(relu_tile(pack_tile<T>(mma2<T>(w.w2op, h1_rec, a2))));
+    act2_rec = active_tile(relu_tile(pack_tile<T>(mma2<T>(w2r, h1_rec, a2))));
   }
-  // ---- backward: D2 in both orientations, D1 unit-major, the output adjoints unit-major
-  const Pack8 d2_rec = and_tile(pack_tile<T>(Ops<T>::mfma(w.w3op, d3op, zero)), act2_rec);
-  const Pack8 d2_unit = and_tile(pack_tile<T>(Ops<T>::mfma(d3op, w.w3op, zero)), act2_unit);
-  const Pack8 d1_unit = and_tile(pack_tile<T>(mma2<T>(d2_rec, w.w2top, zero)), act1_unit);
-  const Pack8 d3_unit = pack_tile<T>(Ops<T>::mfma(d3op, w.out_sel, zero));
-  sum.gb2 += sum_tile<T>(d2_unit);
+  // ---- backward: D2 in both orientations, D1 unit-major, the output adjoints unit-major (column n = output n % 4)
+  const u32x2 w3r = w.w3r[lane], w3u = w.w3u[lane];
+  const unsigned pick = (n & 1) ? one_hi : one_lo;
+  const u32x4 out_sel = {(g == 0 && !(n & 2)) ? pick : 0u, (g == 0 && (n & 2)) ? pick : 0u, 0u, 0u};
+  const Pack8 d2_rec = and_tile(pack_tile<T>(Ops<T>::mfma(u32x4{w3r[0], w3r[1], 0u, 0u}, d3op, zero)), act2_rec);
+  const Pack8 d2_unit = and_tile(pack_tile<T>(Ops<T>::mfma(d3op, u32x4{w3u[0], w3u[1], 0u, 0u}, zero)), act2_unit);
+  const Pack8 d3_unit = pack_tile<T>(Ops<T>::mfma(d3op, out_sel, zero));
+  const Pack8 w2t = {{w.w2t[0][lane], w.w2t[1][lane]}};
+  const Pack8 d1_unit = and_tile(pack_tile<T>(mma2<T>(d2_rec, w2t, zero)), act1_unit);
   // ---- weight gradients: contraction over the records in the k-slots of the unit-major tiles
+  Pack8 ones;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) ones.s[0][d] = ones.s[1][d] = Ops<T>::kOneWord;
+  sum.gb2 = mma4<T>(ones, d2_unit, sum.gb2);
+  sum.gw3 = mma4<T>(d3_unit, h2_unit, sum.gw3);
   sum.gw2 = mma2<T>(d2_unit, h1_unit, sum.gw2);
-  sum.gw3 = mma2<T>(d3_unit, h2_unit, sum.gw3);
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    vf32x16 e = Ops<T>::mfma(enc[2 * c], w.k_sel[0], zero);
-    if (c < 2) e = Ops<T>::mfma(enc[2 * c + 1], w.k_sel[1], e);
+    vf32x16 e = Ops<T>::mfma(enc[2 * c], w.k_sel[0][lane], zero);
+    if (c < 2) e = Ops<T>::mfma(enc[2 * c + 1], w.k_sel[1][lane], e);
     sum.gw1[c] = mma2<T>(d1_unit, pack_tile<T>(e), sum.gw1[c]);
   }
 }
@@ -360,9 +382,13 @@ __device__ __forceinline__ bool vjp16_store(Vjp16Sums& sum, const GradRows& out,
       else if (feature[c] == -2) put(out.b1 + row, sum.gw1[c][i] * inv);
     }
     put(out.W2 + row * 32 + n, sum.gw2[i] * inv);
-    if (row < 4) put(out.W3 + row * 32 + n, sum.gw3[i] * inv);
   }
-  const float gb2 = sum.gb2 + __shfl_xor(sum.gb2, 32);
+#pragma unroll
+  for (int o = 0; o < 4; ++o) {
+    const float v = sum.gw3[o] + __shfl_xor(sum.gw3[o], 32);
+    if (g == 0) put(out.W3 + o * 32 + n, v * inv);
+  }
+  const float gb2 = sum.gb2[0] + __shfl_xor(sum.gb2[0], 32);
   if (g == 0) put(out.b2 + n, gb2 * inv);
 #pragma unroll
   for (int o = 0; o < 4; ++o) {

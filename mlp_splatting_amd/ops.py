@@ -851,7 +851,7 @@ def train_group(frame, tile_offsets, n):
     groups.prim, groups.perm = torch.sort(keys, stable=True)
     nbytes = lib.mlpsp_train_scratch_bytes(S, n)
     groups.scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    _check(lib.mlpsp_train_group(_ptr(groups.prim), _ptr(groups.perm), _ptr(listed[1]), _ptr(listed[2]), S, n,
+    _check(lib.mlpsp_train_group(_ptr(groups.prim), _ptr(groups.perm), _ptr(listed[1]), _ptr(listed[2]), S, n, frame.width,
                                  _ptr(groups.scratch), nbytes, _stream(dev)), "mlpsp_train_group")
     return groups
 
