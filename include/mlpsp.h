@@ -404,6 +404,12 @@ int mlpsp_pack_mfma_weights(const float* W1, const float* b1, const float* W2, c
 int mlpsp_pack_mfma_weights_half(const void* W1, const void* b1, const void* W2, const void* b2, const void* W3,
                                  const void* b3, int num_primitives, int use_bf16, void* packed_dev,
                                  mlpsp_stream_t stream);
+/* mlpsp_pack_mfma_weights of the primitives that order_dev names (negative entries: none) alone: a training step, whose
+ * weights are new in every call, converts what its frame reads.  wanted_dev: num_primitives bytes of scratch; the blocks
+ * of other primitives are not written. */
+int mlpsp_pack_mfma_weights_listed(const float* W1, const float* b1, const float* W2, const float* b2, const float* W3,
+                                   const float* b3, int num_primitives, int use_bf16, const int32_t* order_dev,
+                                   int64_t num_pairs, unsigned char* wanted_dev, void* packed_dev, mlpsp_stream_t stream);
 int mlpsp_render_tilecenter_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
                                  const int32_t* order_dev, const int32_t* tile_offsets_dev, const float* freq_dev,
                                  const float* att_dev, const void* packed_dev, int num_primitives, int use_bf16,

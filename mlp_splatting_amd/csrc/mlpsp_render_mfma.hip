@@ -31,9 +31,10 @@ template <typename T, typename S>
 __global__ __launch_bounds__(64) void pack_mfma_weights_kernel(const S* __restrict__ W1, const S* __restrict__ b1,
                                                                const S* __restrict__ W2, const S* __restrict__ b2,
                                                                const S* __restrict__ W3, const S* __restrict__ b3,
-                                                               int N, unsigned char* __restrict__ out) {
+                                                               int N, const unsigned char* __restrict__ wanted,
+                                                               unsigned char* __restrict__ out) {
   const int p = blockIdx.x;
-  if (p >= N) return;
+  if (p >= N || (wanted && !wanted[p])) return;
   const int l = threadIdx.x, m = l & 31, g = l >> 5;
   unsigned char* blk = out + (size_t)p * kPackStride;
   // accumulator row m holds hidden unit hidden_unit_of_row(m), for both hidden layers
@@ -83,6 +84,16 @@ __global__ __launch_bounds__(64) void pack_mfma_weights_kernel(const S* __restri
   const unsigned long long any = __ballot(bad);
   if (l == 0) *reinterpret_cast<int32_t*>(blk + kOffFlag) = any ? 1 : 0;
   if (l < (kPackStride - kOffFlag - 4) / 4) reinterpret_cast<unsigned*>(blk + kOffFlag + 4)[l] = 0u;   // unused tail
+}
+
+// wanted[p] = 1 for the primitives of a list (negative entries: culled).  Most lists name a primitive in tile after tile: a
+// plain store of the same byte by whoever comes.
+__global__ __launch_bounds__(256) void mark_listed_kernel(const int32_t* __restrict__ order, long long num_pairs, int N,
+                                                          unsigned char* __restrict__ wanted) {
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < num_pairs; i += (long long)gridDim.x * 256) {
+    const int p = order[i];
+    if (p >= 0 && p < N) wanted[p] = 1;
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -808,17 +819,17 @@ MLPSP_API size_t mlpsp_mfma_pack_bytes(int num_primitives) {
 namespace {
 template <typename S>
 int pack_weights_from(const S* W1, const S* b1, const S* W2, const S* b2, const S* W3, const S* b3, int num_primitives,
-                      int use_bf16, void* packed_dev, hipStream_t s) {
+                      int use_bf16, const unsigned char* wanted, void* packed_dev, hipStream_t s) {
   if (num_primitives < 0) return MLPSP_E_ARGUMENT;
   if (num_primitives == 0) return MLPSP_OK;
   if (!W1 || !b1 || !W2 || !b2 || !W3 || !b3 || !packed_dev) return MLPSP_E_ARGUMENT;
   if (reinterpret_cast<uintptr_t>(packed_dev) % 128 != 0) return MLPSP_E_ARGUMENT;
   if (use_bf16)
     hipLaunchKernelGGL((pack_mfma_weights_kernel<__bf16, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
-                       b3, num_primitives, (unsigned char*)packed_dev);
+                       b3, num_primitives, wanted, (unsigned char*)packed_dev);
   else
     hipLaunchKernelGGL((pack_mfma_weights_kernel<_Float16, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
-                       b3, num_primitives, (unsigned char*)packed_dev);
+                       b3, num_primitives, wanted, (unsigned char*)packed_dev);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }
@@ -827,15 +838,31 @@ int pack_weights_from(const S* W1, const S* b1, const S* W2, const S* b2, const 
 MLPSP_API int mlpsp_pack_mfma_weights(const float* W1, const float* b1, const float* W2, const float* b2,
                                       const float* W3, const float* b3, int num_primitives, int use_bf16,
                                       void* packed_dev, mlpsp_stream_t stream) {
-  return pack_weights_from<float>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, packed_dev, (hipStream_t)stream);
+  return pack_weights_from<float>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, nullptr, packed_dev, (hipStream_t)stream);
 }
 
 MLPSP_API int mlpsp_pack_mfma_weights_half(const void* W1, const void* b1, const void* W2, const void* b2,
                                            const void* W3, const void* b3, int num_primitives, int use_bf16,
                                            void* packed_dev, mlpsp_stream_t stream) {
   typedef const _Float16* H;
-  return pack_weights_from<_Float16>((H)W1, (H)b1, (H)W2, (H)b2, (H)W3, (H)b3, num_primitives, use_bf16, packed_dev,
+  return pack_weights_from<_Float16>((H)W1, (H)b1, (H)W2, (H)b2, (H)W3, (H)b3, num_primitives, use_bf16, nullptr, packed_dev,
                                      (hipStream_t)stream);
+}
+
+MLPSP_API int mlpsp_pack_mfma_weights_listed(const float* W1, const float* b1, const float* W2, const float* b2,
+                                             const float* W3, const float* b3, int num_primitives, int use_bf16,
+                                             const int32_t* order_dev, int64_t num_pairs, unsigned char* wanted_dev,
+                                             void* packed_dev, mlpsp_stream_t stream) {
+  if (num_primitives < 0 || num_pairs < 0) return MLPSP_E_ARGUMENT;
+  if (num_primitives == 0 || num_pairs == 0) return MLPSP_OK;
+  if (!order_dev || !wanted_dev) return MLPSP_E_ARGUMENT;
+  hipStream_t s = (hipStream_t)stream;
+  MLPSP_HIP_TRY(hipMemsetAsync(wanted_dev, 0, (size_t)num_primitives, s));
+  const int64_t blocks = (num_pairs + 1023) / 1024;
+  hipLaunchKernelGGL(mark_listed_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, order_dev,
+                     (long long)num_pairs, num_primitives, wanted_dev);
+  MLPSP_LAUNCH_CHECK();
+  return pack_weights_from<float>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, wanted_dev, packed_dev, s);
 }
 
 namespace {

@@ -607,7 +607,7 @@ class TileExt:
             if x[5].numel() > 0:
                 order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
                                           self.max_tile_prims, cull_threshold=float(threshold))
-            packed = None if precision is None else self._packed_weights(list(x[9:15]), precision == "bfloat16")
+            packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
             with self._lock:
                 pool = n_tiles * self._steps_per_tile
             rgb, alpha, frame = ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height,
