@@ -127,6 +127,60 @@ __device__ __forceinline__ void step_store(const StepPool& sp, int slot, int lan
   reinterpret_cast<uint32_t*>(rec + kStepPlaneD)[lane] = hit ? mask2 : 0u;
   if (lane == 0) sp.ids[slot] = p;
 }
+// Zero rows of the primitives that have no step, in every gradient tensor: a wavefront takes eight primitives, so that a
+// row of a few floats fills its stores too.  Bound by the stores (6.3 TB/s for a plain fill on this card).
+struct ZeroRows {
+  float* base[9];
+  int len[9];        // floats per primitive
+  int count;
+  void add(float* p, int floats) {
+    base[count] = p;
+    len[count++] = floats;
+  }
+};
+static __global__ __launch_bounds__(256) void zero_rows_kernel(const int32_t* __restrict__ first, int N, ZeroRows z) {
+  const int p0 = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * 8, lane = threadIdx.x & 63;
+  if (p0 >= N) return;
+  const int p = min(p0 + (lane & 7), N - 1);
+  const unsigned empty = (unsigned)__ballot(lane < 8 && p0 + lane < N && first[p] == first[p + 1]);
+  if (empty == 0u) return;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int a = 0; a < z.count; ++a) {
+    float* __restrict__ dst = z.base[a] + (size_t)p0 * z.len[a];
+    const bool quads = (z.len[a] & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
+    const int n = quads ? z.len[a] >> 2 : z.len[a];          // items per primitive
+    if (n >= 64) {
+      for (unsigned todo = empty; todo; todo &= todo - 1u) {
+        const size_t at = (size_t)__builtin_ctz(todo) * n;
+        for (int i = lane; i < n; i += 64) {
+          if (quads) reinterpret_cast<float4*>(dst)[at + i] = zero;
+          else dst[at + i] = 0.f;
+        }
+      }
+    } else {
+      for (int i = lane; i < 8 * n; i += 64) {
+        if (!((empty >> (i / n)) & 1u)) continue;
+        if (quads) reinterpret_cast<float4*>(dst)[i] = zero;
+        else dst[i] = 0.f;
+      }
+    }
+  }
+}
+inline void launch_zero_rows(const int32_t* first, int N, const ZeroRows& z, hipStream_t s) {
+  hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)((N + 31) / 32)), dim3(256), 0, s, first, N, z);
+}
+// The primitive whose steps begin in chunk `chunk` and go on in the next (at most one): its number, or -1.
+struct SpanningRun {
+  int p, last_chunk;
+};
+__device__ __forceinline__ SpanningRun spanning_run(const int32_t* __restrict__ prim, const int32_t* __restrict__ first, int S,
+                                                    int chunk, int chunk_steps) {
+  const int chunk_end = (chunk + 1) * chunk_steps;
+  if (chunk_end >= S) return SpanningRun{-1, 0};
+  const int p = prim[chunk_end - 1], begin = first[p], end = first[p + 1];
+  if (begin < chunk * chunk_steps || end <= chunk_end) return SpanningRun{-1, 0};
+  return SpanningRun{p, (end - 1) / chunk_steps};
+}
 #endif
 
 }  // namespace mlpsp

@@ -5,8 +5,8 @@
 // The steps are sorted by primitive (by the caller: a stable sort of S keys, S = 0.65 M at the 200,000-primitive
 // 1200x680 frame) and cut into chunks of equal length.  A wavefront walks one chunk; where the primitive changes it
 // writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
-// (the primitive goes on in the next chunk) or head row (it ended here).  One more launch adds the rows of the primitives
-// that span chunks and writes the zeros of those without a step.  No atomics, a fixed order of every sum.
+// (the primitive goes on in the next chunk) or head row (it ended here).  Two more launches add the rows of the primitives
+// that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.52 (1.9), sort and grouping
 // 0.22 (sort 1.7, gathers 2.85), geometry 0.21 (1.1), weight gradients 7.5 (13.5), joining rows and zeros 0.9 (0.8).
@@ -538,33 +538,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 }
 
 // ---------------------------------------------------------------------------------------------
-// One workgroup per primitive: zeros where it has no step, nothing where one chunk held all of them, else the sum of its
-// rows (tail of the first chunk, tails in between, head of the last).  Bound by the zeros: 14 KB per primitive.
+// One workgroup per chunk and quarter of a row: the sum of the rows of the primitive whose steps begin in the chunk and go
+// on in the next (its tail row here, tails in between, the head row of its last chunk); nothing if there is none.  What
+// lasts is a primitive with steps in most tiles, hundreds of rows one after the other: sixteen of them are in flight, and
+// its columns are shared out (one workgroup and eight in flight: 0.35 ms at 650,000 steps; now 0.21).
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void train_finish_kernel(const int32_t* __restrict__ first, int chunk_steps, int num_chunks,
-                                                           const float* __restrict__ rows, const float* __restrict__ quats,
-                                                           GradRows grads, GeoGrads geo, int32_t* __restrict__ nonfinite) {
-  const int p = blockIdx.x, begin = first[p], end = first[p + 1], t = threadIdx.x;
-  const int cf = begin / chunk_steps, cl = begin < end ? (end - 1) / chunk_steps : cf;
-  if (begin < end && cf == cl) return;
-  const size_t np = (size_t)p;
+__global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, int chunk_steps, int num_chunks,
+                                                         const float* __restrict__ rows, const float* __restrict__ quats,
+                                                         GradRows grads, GeoGrads geo, int32_t* __restrict__ nonfinite) {
+  const int t = threadIdx.x, cf = blockIdx.x, k = blockIdx.y * 256 + t;
+  const SpanningRun run = spanning_run(ix.prim, ix.first, S, cf, chunk_steps);
+  if (run.p < 0) return;
+  const int cl = run.last_chunk;
+  const size_t np = (size_t)run.p;
   __shared__ float s_geo[16][kGeoFloats];
   bool bad = false;
   const auto row = [&](int c) { return rows + (size_t)(c < cl ? num_chunks + c : c) * kRowFloats; };
-  for (int k = t; k < kGradFloats / 4; k += 256) {
+  if (k < kGradFloats / 4) {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (begin < end) {
-#pragma unroll 8
-      for (int c = cf; c <= cl; ++c) {
-        const float4 v = reinterpret_cast<const float4*>(row(c))[k];
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-      }
-      bad |= !(__builtin_fabsf(acc.x) <= 3.4028235e38f) || !(__builtin_fabsf(acc.y) <= 3.4028235e38f) ||
-             !(__builtin_fabsf(acc.z) <= 3.4028235e38f) || !(__builtin_fabsf(acc.w) <= 3.4028235e38f);
+#pragma unroll 16
+    for (int c = cf; c <= cl; ++c) {
+      const float4 v = reinterpret_cast<const float4*>(row(c))[k];
+      acc.x += v.x;
+      acc.y += v.y;
+      acc.z += v.z;
+      acc.w += v.w;
     }
+    bad |= !(__builtin_fabsf(acc.x) <= 3.4028235e38f) || !(__builtin_fabsf(acc.y) <= 3.4028235e38f) ||
+           !(__builtin_fabsf(acc.z) <= 3.4028235e38f) || !(__builtin_fabsf(acc.w) <= 3.4028235e38f);
     // float4 ranges of the parts: [0,576) W1, [576,584) b1, [584,840) W2, [840,848) b2, [848,880) W3, 880 b3
     float4* dst;
     if (k < 576) dst = reinterpret_cast<float4*>(grads.W1) + np * 576 + k;
@@ -576,12 +577,7 @@ __global__ __launch_bounds__(256) void train_finish_kernel(const int32_t* __rest
     *dst = acc;
   }
   if (__ballot(bad) != 0ull && (t & 63) == 0) atomicOr(nonfinite, 1);
-  if (begin == end) {
-    if (t < 3) geo.pos[np * 3 + t] = 0.f;
-    else if (t < 6) geo.scale[np * 3 + t - 3] = 0.f;
-    else if (t < 10) geo.quat[np * 4 + t - 6] = 0.f;
-    return;
-  }
+  if (blockIdx.y != 3) return;         // (the last quarter is the shortest)
   float v = 0.f;
   for (int c = cf + (t >> 4); c <= cl; c += 16) v += (t & 15) < 15 ? row(c)[kGradFloats + (t & 15)] : 0.f;
   s_geo[t >> 4][t & 15] = v;
@@ -704,9 +700,21 @@ MLPSP_API int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_
     hipLaunchKernelGGL(train_geometry_kernel, dim3((unsigned)((t.num_chunks + 3) / 4)), dim3(256), 0, s, ix, S, t.chunk_steps,
                        t.num_chunks, sp.records, falloff_dev, log_scales_dev, quats_dev, t.rows, geo);
     MLPSP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)t.num_chunks, 4), dim3(256), 0, s, ix, S, t.chunk_steps, t.num_chunks,
+                       t.rows, quats_dev, grads, geo, nonfinite_dev);
+    MLPSP_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(train_finish_kernel, dim3((unsigned)num_primitives), dim3(256), 0, s, t.first, t.chunk_steps,
-                     t.num_chunks, t.rows, quats_dev, grads, geo, nonfinite_dev);
+  ZeroRows zero{};
+  zero.add(gW1_dev, 2304);
+  zero.add(gb1_dev, 32);
+  zero.add(gW2_dev, 1024);
+  zero.add(gb2_dev, 32);
+  zero.add(gW3_dev, 128);
+  zero.add(gb3_dev, 4);
+  zero.add(grad_positions_dev, 3);
+  zero.add(grad_log_scales_dev, 3);
+  zero.add(grad_quats_dev, 4);
+  launch_zero_rows(t.first, num_primitives, zero, s);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }

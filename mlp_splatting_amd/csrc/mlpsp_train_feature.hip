@@ -12,10 +12,10 @@
 //   train_feature_blend_kernel  k of a tile's steps (kept for the backward); the tile's share of its targets' values
 //   train_feature_join_kernel   the shares of a target (its taps lie in one, two or four tiles), residual, sign, loss
 //   train_attr_kernel           steps sorted by primitive, in chunks as in mlpsp_train_backward.hip
-//   train_attr_finish_kernel    rows of primitives that span chunks; zeros of those without a step
+//   train_attr_join_kernel      rows of primitives that span chunks
 //
 // All are bound by memory traffic: attribute rows out of L2 in the blend (8 KB per step at 512 channels, four slots), sign
-// rows (2 KB) in the gradient, the zeros of the gradient (8 KB per primitive) in the last.  At 200,000 primitives,
+// rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each).  At 200,000 primitives,
 // 1200x680, a 300x170 target of 512 channels: 0.56, 0.07, 0.44 and 0.32 ms; the record kernels took 4.95 ms for the
 // loss and 8.1 ms for the gradient.
 #include "mlpsp_device.hpp"
@@ -370,31 +370,31 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
   }
 }
 
-// One workgroup per primitive, lane = four channels of one slot.
+// One workgroup per chunk, lane = four channels of one slot: the rows of the primitive that begins in it and goes on.
 template <bool VEC>
-__global__ __launch_bounds__(256) void train_attr_finish_kernel(FeatShape f, const int32_t* __restrict__ first, int chunk_steps,
-                                                                int num_chunks, const float* __restrict__ adjoint,
-                                                                const float* __restrict__ rows, float* __restrict__ out) {
-  const int p = blockIdx.x, begin = first[p], end = first[p + 1];
-  const int cf = begin / chunk_steps, cl = begin < end ? (end - 1) / chunk_steps : cf;
-  if (begin < end && cf == cl) return;
+__global__ __launch_bounds__(256) void train_attr_join_kernel(FeatShape f, const int32_t* __restrict__ prim,
+                                                              const int32_t* __restrict__ first, int S, int chunk_steps,
+                                                              int num_chunks, const float* __restrict__ adjoint,
+                                                              const float* __restrict__ rows, float* __restrict__ out) {
+  const int cf = blockIdx.x;
+  const SpanningRun run = spanning_run(prim, first, S, cf, chunk_steps);
+  if (run.p < 0) return;
+  const int cl = run.last_chunk;
   const float norm = (float)((long long)f.WF * f.HF * f.C), scale = adjoint[0];
   const int quads = f.Cp >> 2;
   for (int i = threadIdx.x; i < quads * f.slots; i += 256) {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (begin < end) {
 #pragma unroll 8
-      for (int c = cf; c <= cl; ++c) {
-        const float4 v = reinterpret_cast<const float4*>(rows + ((size_t)(c < cl ? num_chunks + c : c) * f.slots) * f.Cp)[i];
-        acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w;
-      }
-      acc = make_float4(acc.x / norm * scale, acc.y / norm * scale, acc.z / norm * scale, acc.w / norm * scale);
+    for (int c = cf; c <= cl; ++c) {
+      const float4 v = reinterpret_cast<const float4*>(rows + ((size_t)(c < cl ? num_chunks + c : c) * f.slots) * f.Cp)[i];
+      acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w;
     }
+    acc = make_float4(acc.x / norm * scale, acc.y / norm * scale, acc.z / norm * scale, acc.w / norm * scale);
     if constexpr (VEC) {
-      reinterpret_cast<float4*>(out + (size_t)p * f.slots * f.C)[i] = acc;
+      reinterpret_cast<float4*>(out + (size_t)run.p * f.slots * f.C)[i] = acc;
     } else {
       const int s = i / quads, c = (i - s * quads) * 4;
-      float* __restrict__ dst = out + ((size_t)p * f.slots + s) * f.C + c;
+      float* __restrict__ dst = out + ((size_t)run.p * f.slots + s) * f.C + c;
       dst[0] = acc.x;
       if (c + 1 < f.C) dst[1] = acc.y;
       if (c + 2 < f.C) dst[2] = acc.z;
@@ -501,13 +501,17 @@ MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int6
     else { if (vec) MLPSP_ATTR(5, true); else MLPSP_ATTR(5, false); }
 #undef MLPSP_ATTR
     MLPSP_LAUNCH_CHECK();
+    if (vec)
+      hipLaunchKernelGGL(train_attr_join_kernel<true>, dim3((unsigned)chunks), dim3(256), 0, s, f, sorted_prim_dev, t.first,
+                         (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
+    else
+      hipLaunchKernelGGL(train_attr_join_kernel<false>, dim3((unsigned)chunks), dim3(256), 0, s, f, sorted_prim_dev, t.first,
+                         (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
+    MLPSP_LAUNCH_CHECK();
   }
-  if (vec)
-    hipLaunchKernelGGL(train_attr_finish_kernel<true>, dim3((unsigned)num_primitives), dim3(256), 0, s, f, t.first, per, chunks,
-                       loss_adjoint_dev, rows_dev, out_dev);
-  else
-    hipLaunchKernelGGL(train_attr_finish_kernel<false>, dim3((unsigned)num_primitives), dim3(256), 0, s, f, t.first, per,
-                       chunks, loss_adjoint_dev, rows_dev, out_dev);
+  ZeroRows zero{};
+  zero.add(out_dev, slots * channels);
+  launch_zero_rows(t.first, num_primitives, zero, s);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }
