@@ -434,10 +434,12 @@ int mlpsp_render_tilecenter_mfma(const float* rays_o_dev, const float* rays_d_de
  * (for timing the two launches apart; 1 and 2 need feat_slots != 0).  MLPSP_STAGE_STATUS_IS_CLEAR may be or-ed in:
  * the caller vouches that the 16 words at status_dev are zero already (it read them back as zero after the previous
  * call on this buffer), and the call queues no clear of them -- one launch less between the sort and the render
- * of a frame.
+ * of a frame.  MLPSP_STAGE_FRAMES_OVERLAP may be or-ed in: another frame is queued on another stream beside this one (the
+ * launch is then laid out for throughput alone; the results are the same).
  * tile_ends_dev: NULL, or the ends of lists that lie in segments (see mlpsp_sort_tiles); num_pairs is then the
  * number of entries of order_dev, gaps included. */
 #define MLPSP_STAGE_STATUS_IS_CLEAR 4
+#define MLPSP_STAGE_FRAMES_OVERLAP 8
 size_t mlpsp_mfma_feat_pack_bytes(int num_primitives, int feat_slots, int feat_channels);
 int mlpsp_pack_mfma_feat(const float* feat_attr_dev, int num_primitives, int feat_slots, int feat_channels,
                          void* packed_feat_dev, int32_t* status_dev, mlpsp_stream_t stream);

@@ -9,6 +9,7 @@
 // or cross-lane traffic between the layers).  (Measured alternatives that did not pay on gfx950: a
 // 4096-entry LDS sin/cos table -- same kernel time, 2x the image error; persistent wavefronts with a tile
 // work queue -- 6 % slower than one wavefront per tile.)
+#include <type_traits>
 #include "mlpsp_device.hpp"
 #include "mlpsp_hitrec.hpp"
 #include "mlpsp_mfma16.hpp"
@@ -423,6 +424,7 @@ __device__ __forceinline__ void render_tile_mfma(
         }
         live = valid && (acc.trans >= kTransmittanceFloor);
         if (__ballot(live) == 0ull) {
+          fast_arrived(q);       // (the next entry's line may still be landing in these registers)
           finished = true;
           break;
         }
@@ -448,23 +450,265 @@ __device__ __forceinline__ void render_tile_mfma(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// A tile's wavefronts as a team: what an entry contributes does not depend on the entries in front of it, only the weight
+// it gets does.  Wavefront k tests and evaluates entries k, k + TEAM, ... of the list; after every round of TEAM entries
+// each wavefront goes through their opacities in list order -- so all of them know the transmittance and when the tile is
+// done --, and wavefront 0 adds up the colours, in the order and with the roundings of the single wavefront: same bits.
+//
+// A tile is a serial chain of 40 to 170 entries of two microseconds each; an image of few tiles lasts as long as its longest
+// chain, with the chip mostly idle.  320x240, 20,000 primitives, bf16: 166 -> 127 us with three wavefronts per tile (all of
+// them resident); then the SIMDs' issue slots are two thirds busy and the rest is the spread of the tiles.  Requesting the
+// next entry's weights a round ahead changes nothing there.  The price is the second pass over the opacities and up to
+// TEAM - 1 entries evaluated behind the last one that counts.
+// ---------------------------------------------------------------------------------------------
+// (orders LDS alone: requests to memory stay in flight across it)
+__device__ __forceinline__ void team_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+template <int TEAM>
+struct TeamRound {
+  float alpha[TEAM][64];
+  float colour[TEAM - 1][3][64];      // of wavefronts 1..: wavefront 0 has its own in registers
+};
+
+template <int TEAM>
+struct TeamLds {
+  DirWords dir;
+  OriginLds<0> org;
+  TeamRound<TEAM> round[2];
+};
+
+template <typename T, int TEAM>
+__device__ __forceinline__ void render_tile_team(
+    const int tile, const int k, const int l, TeamLds<TEAM>& lds, const SinCosTable* table, const float* __restrict__ rays_o,
+    const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims, const int32_t* __restrict__ order,
+    const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends, const float* __restrict__ freq,
+    const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx, float thr,
+    float* __restrict__ out_rgb, float* __restrict__ out_alpha, int32_t* __restrict__ status,
+    unsigned long long* __restrict__ counters) {
+  DirWords& s_dir = lds.dir;
+  OriginLds<0>& s_org = lds.org;
+  TeamRound<TEAM>(&s_round)[2] = lds.round;
+  float kf[3];
+  phase_scales(freq, att, l >> 5, kf);
+  float kfm[3] = {kf[0], kf[1], kf[2]};
+  float input_limit = 3.4028235e38f;
+  if constexpr (RenderTable<T>::kUse) {
+    float kmax = fmaxf(fmaxf(__builtin_fabsf(kf[0]), __builtin_fabsf(kf[1])), __builtin_fabsf(kf[2]));
+    kmax = fmaxf(kmax, __shfl_xor(kmax, 32));
+    input_limit = kSinCosRange / fmaxf(kmax, 1e-30f);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) kfm[j] = kf[j] * (4.0f * (float)kSinCosEntries);
+  }
+  unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
+  bool bad = false;
+  const int tx = tile % ntx, ty = tile / ntx;
+  const int x = tx * 8 + (l & 7), y = ty * 8 + (l >> 3);
+  const bool valid = (x < W) && (y < H);
+  const int pix = valid ? (y * W + x) : 0;
+  const Float3 ray_o = valid ? load3(rays_o, pix) : Float3{0.f, 0.f, 0.f};
+  const Float3 ray_d = valid ? load3(rays_d, pix) : Float3{0.f, 0.f, 0.f};
+  const float rox = ray_o.x, roy = ray_o.y, roz = ray_o.z;
+  const float rdx = ray_d.x, rdy = ray_d.y, rdz = ray_d.z;
+  if (k == 0) encode_direction_words<T>(rdx, rdy, rdz, kf, l, s_dir);
+  const unsigned long long in_image = __ballot(valid);
+  const int lane0 = in_image ? (int)__builtin_ctzll(in_image) : 0;
+  const float ox = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(rox), lane0)),
+              oy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(roy), lane0)),
+              oz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(roz), lane0));
+  const float reach = 4e-6f * __builtin_sqrtf(fmaxf(-2.f * __logf(thr), 0.f));
+  const bool one_origin = __ballot(valid && !(rox == ox && roy == oy && roz == oz)) == 0ull;
+  const int start = offsets[tile], end = ends[tile];
+  float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
+  bool live = valid;
+  int buf = 0;
+  const unsigned char* __restrict__ fast_half = reinterpret_cast<const unsigned char*>(prims) + 64;
+  bool finished = false;
+  for (int base = start; base < end && !finished; base += 64) {
+    const int id_lane = (base + l < end) ? order[base + l] : -1;
+    unsigned long long todo = __ballot(id_lane >= 0 && id_lane < N);
+    if (todo == 0ull) continue;
+    // the entries' origin terms, shared out (the barriers of the last round and of this batch are around them)
+    if (one_origin && l % TEAM == k && id_lane >= 0 && id_lane < N) {
+      const FastRec& F = *reinterpret_cast<const FastRec*>(fast_half + (size_t)id_lane * sizeof(PrimRecord));
+      const OriginTerms o = origin_terms(ox, oy, oz, F.cx, F.cy, F.cz, F.r);
+      *reinterpret_cast<f32x4*>(&s_org.e[l][0]) = f32x4{o.vx, o.vy, o.vz, o.vlx};
+      *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, band_for(o, thr, reach), 0.f};
+    }
+    const int rounds = ((int)__builtin_popcountll(todo) + TEAM - 1) / TEAM;
+    for (int i = 0; i < k; ++i) todo &= todo - 1ull;
+    FastRegs q;
+    int j = 0, p = 0;
+    if (todo != 0ull) {
+      j = (int)__builtin_ctzll(todo);
+      p = __builtin_amdgcn_readlane(id_lane, j);
+      fast_request(fast_half + (size_t)p * sizeof(PrimRecord), q);
+    }
+    team_barrier();
+    for (int r = 0; r < rounds; ++r) {
+      float alpha = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+      bool hit = false, hit_bad = false;
+      const bool mine = todo != 0ull;
+      if (mine) {
+        const FastRec R = fast_arrived(q);
+        OriginTerms ot;
+        float band;
+        if (one_origin) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(&s_org.e[j][0]);
+          const f32x4 b = *reinterpret_cast<const f32x4*>(&s_org.e[j][4]);
+          ot = OriginTerms{a[0], a[1], a[2], a[3], b[0], b[1]};
+          band = b[2];
+        } else {
+          ot = origin_terms(rox, roy, roz, R.cx, R.cy, R.cz, R.r);
+          band = band_for(ot, thr, reach);
+        }
+        HitInfo h;
+        bool unsure;
+        hit = hit_fast(ot, rdx, rdy, rdz, R.r, thr, band, h, unsure) && live;
+        asm volatile("" : "+v"(h.dx), "+v"(h.dy), "+v"(h.dz), "+v"(h.decay));   // R is used up here
+        const int p_now = p;
+#pragma unroll
+        for (int i = 0; i < TEAM; ++i) todo &= todo - 1ull;
+        if (todo != 0ull) {
+          j = (int)__builtin_ctzll(todo);
+          p = __builtin_amdgcn_readlane(id_lane, j);
+          fast_request(fast_half + (size_t)p * sizeof(PrimRecord), q);
+        }
+        if (__ballot(unsure && live) != 0ull) {   // rare
+          if (unsure && live) {
+            const PrimRecord P = prims[p_now];
+            HitInfo exact;
+            hit = hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, exact);
+          }
+        }
+        const unsigned long long mask = __ballot(hit);
+        ++n_proc;
+        if (mask != 0ull) {
+          const unsigned char* __restrict__ blk = packed + (size_t)p_now * kPackStride;
+          hit_bad = !((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit);
+          if ((unsigned)mask != 0u && (unsigned)(mask >> 32) != 0u)
+            hit_bad |= mlp_pair_mfma16<T, Ops<T>::kCheckHidden, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm,
+                                                                                     s_dir, o, table);
+          else
+            hit_bad |= mlp_wave_mfma16<T, Ops<T>::kCheckHidden, false, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz,
+                                                                                            kfm, s_dir, o, nullptr, table);
+          if (hit) {
+            hit_bad |= !(max3_abs(o[0], o[1], o[2]) <= 3.4028235e38f) || !(__builtin_fabsf(o[3]) <= 3.4028235e38f);
+            alpha = 1.f - fast_exp(-(fast_softplus(o[3]) * h.decay));
+#pragma unroll
+            for (int c = 0; c < 3; ++c) o[c] = fast_sigmoid(o[c]);
+          }
+        }
+      }
+      TeamRound<TEAM>& round = s_round[buf];
+      buf ^= 1;
+      // (a lane without a hit: opacity 0, which changes neither the transmittance nor a colour; NaN where the lane hit and
+      // its opacity is NaN, as for a single wavefront)
+      round.alpha[k][l] = hit ? alpha : 0.f;
+      if (k > 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) round.colour[k - 1][c][l] = hit ? o[c] : 0.f;
+      }
+      team_barrier();
+#pragma unroll
+      for (int i = 0; i < TEAM; ++i) {
+        const float a = i == k ? (hit ? alpha : 0.f) : round.alpha[i][l];
+        const bool open = valid && trans >= kTransmittanceFloor;
+        if (i == k) {                          // (an entry behind the last one that counts leaves no trace)
+          bad |= hit && open && hit_bad;
+          const unsigned long long blended = __ballot(hit && open);
+          n_proc_hit += blended != 0ull;
+          n_hits += __popcll(blended);
+        }
+        if (open) {
+          if (k == 0) {
+            const float w = trans * a;
+            cr = fmaf(w, i == 0 ? o[0] : round.colour[i > 0 ? i - 1 : 0][0][l], cr);
+            cg = fmaf(w, i == 0 ? o[1] : round.colour[i > 0 ? i - 1 : 0][1][l], cg);
+            cb = fmaf(w, i == 0 ? o[2] : round.colour[i > 0 ? i - 1 : 0][2][l], cb);
+          }
+          trans = trans * (1.f - a);
+        }
+      }
+      live = valid && (trans >= kTransmittanceFloor);
+      if (__ballot(live) == 0ull) {
+        if (todo != 0ull) fast_arrived(q);      // (the next entry's line may still be landing in these registers)
+        finished = true;
+        break;
+      }
+    }
+    if (!finished) team_barrier();             // the origin terms are free again
+  }
+  if (k == 0 && valid) {
+    store3(out_rgb, pix, cr, cg, cb);
+    out_alpha[pix] = 1.f - trans;
+  }
+  if (__ballot(bad) != 0ull && l == 0) atomicExch(status, 1);
+  if (counters && l == 0) {
+    atomicAdd(counters + 1, (unsigned long long)n_proc);
+    atomicAdd(counters + 2, (unsigned long long)n_proc_hit);
+    atomicAdd(counters + 3, (unsigned long long)n_hits);
+  }
+}
+
+// Every tile by a team of TEAM wavefronts.
+template <typename T, int TEAM>
+__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_team_mfma_kernel(
+    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends,
+    const float* __restrict__ freq, const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W,
+    int H, int ntx, int num_tiles, float thr, float* __restrict__ out_rgb, float* __restrict__ out_alpha,
+    int32_t* __restrict__ status, unsigned long long* __restrict__ counters) {
+  __shared__ __attribute__((aligned(16))) TeamLds<TEAM> lds;
+  __shared__ RenderTable<T> s_table;
+  const int tile = superblock_tile(blockIdx.x, ntx, num_tiles / ntx);
+  if (tile < 0) return;
+  const SinCosTable* table = nullptr;
+  if constexpr (RenderTable<T>::kUse) {      // (ready behind the first barrier of the walk)
+    fill_sincos_table<T>(s_table.t);
+    table = &s_table.t;
+  }
+  render_tile_team<T, TEAM>(tile, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)threadIdx.x & 63, lds, table,
+                            rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr, out_rgb,
+                            out_alpha, status, counters);
+}
+
 // Four wavefronts = four tiles per workgroup: they share nothing but the sin/cos table, which they fill together
 // (sixteen transcendentals per thread) before each goes its own way.
 #ifndef MLPSP_RENDER_WAVES
 #define MLPSP_RENDER_WAVES 4
 #endif
 constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
-template <typename T, int SP>
+// Tiles at the end of the launch that get a workgroup each (RGB only): as many as there are workgroups on the chip, so
+// that what is left when the queue is empty are teams, which finish a tile in a third of the time.  Frame, in us, without
+// and with it: 3,150 tiles 277 -> 266, 4,860 tiles 502 -> 479; at 12,750 tiles 661 either way.  Not where another frame
+// follows on the heels of this one: its wavefronts take the places that the last tiles leave.
+constexpr int kLastRound = 1024;
+// MIXED: the workgroups from `body` on (per XCD) take one tile each, as a team.
+template <typename T, int SP, bool MIXED>
 __global__ __launch_bounds__(64 * kRenderWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_tilecenter_mfma_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends,
     const float* __restrict__ freq,
     const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx,
-    int per_xcd, int num_tiles, float thr, float* __restrict__ out_rgb, float* __restrict__ out_alpha,
+    int body, int num_tiles, float thr, float* __restrict__ out_rgb, float* __restrict__ out_alpha,
     int32_t* __restrict__ status, unsigned long long* __restrict__ counters, int slots, float beta, float temp,
     HitPool hp) {
-  __shared__ DirWords s_dir[kRenderWaves];
-  __shared__ __attribute__((aligned(16))) OriginLds<SP> s_org[kRenderWaves];
+  struct TileLds {
+    DirWords dir[kRenderWaves];
+    __attribute__((aligned(16))) OriginLds<SP> org[kRenderWaves];
+  };
+  struct NoTeam {};
+  union Lds {
+    TileLds tiles;
+    typename std::conditional<MIXED, TeamLds<kRenderWaves>, NoTeam>::type team;
+  };
+  __shared__ __attribute__((aligned(16))) Lds lds;
+  DirWords(&s_dir)[kRenderWaves] = lds.tiles.dir;
+  OriginLds<SP>(&s_org)[kRenderWaves] = lds.tiles.org;
   __shared__ RenderTable<T> s_table;
   const SinCosTable* table = nullptr;
   if constexpr (RenderTable<T>::kUse) {
@@ -474,9 +718,18 @@ __global__ __launch_bounds__(64 * kRenderWaves) __attribute__((amdgpu_waves_per_
   }
   // 8x8 super-blocks of tiles dealt to the XCDs in turn: neighbouring tiles, which share most primitives (their
   // records and weight blocks), run on one L2.  Workgroup b runs on XCD b % 8 and takes four consecutive slots of it.
-  const int wave = (int)threadIdx.x >> 6;
-  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), (int)(blockIdx.x / kNumXcd) * kRenderWaves + wave, ntx,
-                                      num_tiles / ntx);
+  const int wave = (int)threadIdx.x >> 6, xcd = (int)(blockIdx.x % kNumXcd), unit = (int)(blockIdx.x / kNumXcd);
+  if constexpr (MIXED) {
+    if (unit >= body) {
+      const int tile = superblock_tile_of(xcd, body * kRenderWaves + (unit - body), ntx, num_tiles / ntx);
+      if (tile >= 0)
+        render_tile_team<T, kRenderWaves>(tile, __builtin_amdgcn_readfirstlane(wave), (int)threadIdx.x & 63, lds.team, table,
+                                          rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr,
+                                          out_rgb, out_alpha, status, counters);
+      return;
+    }
+  }
+  const int tile = superblock_tile_of(xcd, unit * kRenderWaves + wave, ntx, num_tiles / ntx);
   if (tile < 0) return;
   render_tile_mfma<T, SP>(tile, (int)threadIdx.x & 63, s_dir[wave], s_org[wave], table, rays_o, rays_d, prims, order, offsets,
                           ends, freq, att, packed, N, W, H, ntx, thr, out_rgb, out_alpha, status, counters, slots, beta, temp,
@@ -870,14 +1123,17 @@ constexpr int kGemmNcb = MLPSP_GEMM_NCB;   // 32-channel accumulator tiles per w
 constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 inline int feat_pad(int slots) { return slots == 5 ? 8 : 4; }
 
-template <typename E, int SP>
+template <typename E, int SP, bool MIXED>
 void launch_mfma(dim3 grid, hipStream_t s, const float* rays_o, const float* rays_d, const void* prims, const int32_t* order,
                  const int32_t* offsets, const int32_t* ends, const float* freq, const float* att, const void* packed, int N, int W, int H,
-                 int ntx, int per_xcd, int T, float thr, float* rgb, float* alpha, int32_t* status,
+                 int ntx, int T, float thr, float* rgb, float* alpha, int32_t* status,
                  unsigned long long* ctr, int slots, float beta, float temp, const HitPool& hp) {
-  hipLaunchKernelGGL((render_tilecenter_mfma_kernel<E, SP>), dim3(grid.x / kRenderWaves), dim3(64 * kRenderWaves), 0, s, rays_o, rays_d,
+  const int per_xcd = (int)(grid.x / kNumXcd);       // slots
+  int body = per_xcd / kRenderWaves;                 // workgroups with a tile per wavefront
+  if (MIXED) body = max(0, per_xcd - kLastRound / kNumXcd) / kRenderWaves;
+  hipLaunchKernelGGL((render_tilecenter_mfma_kernel<E, SP, MIXED>), dim3(kNumXcd * (body + per_xcd - body * kRenderWaves)), dim3(64 * kRenderWaves), 0, s, rays_o, rays_d,
                      (const PrimRecord*)prims, order, offsets, ends, freq, att, (const unsigned char*)packed, N, W, H, ntx,
-                     per_xcd, T, thr, rgb, alpha, status, ctr, slots, beta, temp, hp);
+                     body, T, thr, rgb, alpha, status, ctr, slots, beta, temp, hp);
 }
 }  // namespace
 
@@ -935,7 +1191,8 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
                                                 int64_t* counters_dev, int stage, const int32_t* tile_ends_dev,
                                                 mlpsp_stream_t stream) {
   const int64_t T = checked_num_tiles(width, height, 8, 8);
-  if (stage < 0 || (stage & ~(3 | MLPSP_STAGE_STATUS_IS_CLEAR)) != 0) return MLPSP_E_ARGUMENT;
+  if (stage < 0 || (stage & ~(3 | MLPSP_STAGE_STATUS_IS_CLEAR | MLPSP_STAGE_FRAMES_OVERLAP)) != 0) return MLPSP_E_ARGUMENT;
+  const bool overlapped = (stage & MLPSP_STAGE_FRAMES_OVERLAP) != 0;
   const bool status_is_clear = (stage & MLPSP_STAGE_STATUS_IS_CLEAR) != 0;
   stage &= 3;
   if (stage > 2 || (stage != 0 && feat_slots == 0)) return MLPSP_E_ARGUMENT;
@@ -964,15 +1221,31 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
   const dim3 grid(superblock_grid(ntx, ceil_div(height, 8)));
   auto* ctr = reinterpret_cast<unsigned long long*>(counters_dev);
   const int sp = feat_slots ? feat_pad(feat_slots) : 0;
-#define MLPSP_MFMA_GO(TT, SP)                                                                                     \
-  launch_mfma<TT, SP>(grid, s, rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev,   \
-                      att_dev, packed_dev, num_primitives, width, height, ntx, per_xcd, (int)T, threshold,        \
+  // An image with fewer tiles than half the wavefronts the chip holds at four per SIMD: as many wavefronts per tile as
+  // fit at once (a second round of workgroups would cost what the larger team gains).  Frame, bf16, in us with 1 / 2 / 3 /
+  // 4 / 8 wavefronts per tile: 300 tiles 187 / 161 / 150 / 142 / 130, 972 tiles 235 / 207 / 192 / 180 / 190, 1,200 tiles
+  // 236 / 209 / 196 / 202 / 209, 1,610 tiles 234 / 219 / 231 / 220 / 241, 2,214 tiles 242 / 245 / 251 / 249 / 277.
+  const int64_t team = 4096 / T;
+  const bool mixed = T <= 2 * 4096 && !overlapped;     // (see kLastRound)
+#define MLPSP_MFMA_TEAM(TT, TEAM)                                                                                       \
+  hipLaunchKernelGGL((render_team_mfma_kernel<TT, TEAM>), dim3(grid.x), dim3(64 * TEAM), 0, s, rays_o_dev, rays_d_dev,      \
+                     (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev, att_dev,             \
+                     (const unsigned char*)packed_dev, num_primitives, width, height, ntx, (int)T, threshold, out_rgb_dev,  \
+                     out_alpha_dev, status_dev, ctr)
+#define MLPSP_MFMA_GO(TT, SP, MIXED)                                                                              \
+  launch_mfma<TT, SP, MIXED>(grid, s, rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev,   \
+                      att_dev, packed_dev, num_primitives, width, height, ntx, (int)T, threshold,                 \
                       out_rgb_dev, out_alpha_dev, status_dev, ctr, feat_slots, gating_beta, gating_temp, hp)
 #define MLPSP_MFMA_SP(TT)                 \
   do {                                    \
-    if (sp == 0) MLPSP_MFMA_GO(TT, 0);    \
-    else if (sp == 4) MLPSP_MFMA_GO(TT, 4); \
-    else MLPSP_MFMA_GO(TT, 8);            \
+    if (sp == 0 && team >= 8) MLPSP_MFMA_TEAM(TT, 8); \
+    else if (sp == 0 && team >= 4) MLPSP_MFMA_TEAM(TT, 4); \
+    else if (sp == 0 && team == 3) MLPSP_MFMA_TEAM(TT, 3); \
+    else if (sp == 0 && team == 2) MLPSP_MFMA_TEAM(TT, 2); \
+    else if (sp == 0 && mixed) MLPSP_MFMA_GO(TT, 0, true); \
+    else if (sp == 0) MLPSP_MFMA_GO(TT, 0, false); \
+    else if (sp == 4) MLPSP_MFMA_GO(TT, 4, false); \
+    else MLPSP_MFMA_GO(TT, 8, false);            \
   } while (0)
   if (stage != 2) {
     if (use_bf16) MLPSP_MFMA_SP(__bf16);

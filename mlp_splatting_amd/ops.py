@@ -637,13 +637,14 @@ def pack_mfma_weights_listed(ws, order, bf16):
 
 def render_tilecenter_mfma(rays_o, rays_d, records, order, tile_offsets, freq, att, W1, b1, W2, b2, W3, b3, W, H,
                            threshold, bf16=True, counters=None, packed=None, check=True, status=None,
-                           status_is_clear=False, tile_ends=None):
+                           status_is_clear=False, tile_ends=None, overlapped=False):
     """Matrix-core tile-centre forward (8x8 tiles) -> (rgb, alpha, nonfinite).
 
     ``nonfinite`` is a bool when ``check`` (one 4-byte readback) or the int32 device flag otherwise.  ``status``: an
     int32 [16] device tensor for the flag words (word 0 = non-finite), allocated here when omitted.
     ``status_is_clear``: the caller read all 16 words of ``status`` back as zero after the previous call that used
-    it, so no clear is queued in front of the kernel.  ``tile_ends``: as in :func:`sort_tiles`.
+    it, so no clear is queued in front of the kernel.  ``tile_ends``: as in :func:`sort_tiles`.  ``overlapped``: another
+    frame is in flight on another stream.
     """
     dev = rays_o.device
     if freq.numel() != 6:
@@ -656,10 +657,11 @@ def render_tilecenter_mfma(rays_o, rays_d, records, order, tile_offsets, freq, a
     flag = status if status is not None else torch.empty(16, dtype=torch.int32, device=dev)
     if not (flag.is_cuda and flag.dtype == torch.int32 and flag.numel() == 16 and flag.is_contiguous()):
         raise ValueError("status must be a contiguous int32 [16] tensor on the device")
-    if (status_is_clear and status is not None) or tile_ends is not None:
+    if (status_is_clear and status is not None) or tile_ends is not None or overlapped:
         # (the RGB entry point is the feature entry point without features; only that one takes the stage word and
         # the ends of lists in segments)
-        stage = _lib.STAGE_STATUS_IS_CLEAR if (status_is_clear and status is not None) else 0
+        stage = ((_lib.STAGE_STATUS_IS_CLEAR if (status_is_clear and status is not None) else 0)
+                 | (_lib.STAGE_FRAMES_OVERLAP if overlapped else 0))
         code = _lib.load().mlpsp_render_tilecenter_mfma_feat(
             _ptr(rays_o), _ptr(rays_d), _ptr(records), _ptr(order), _ptr(tile_offsets), 0, _ptr(freq), _ptr(att),
             _ptr(packed), W1.shape[0], int(bool(bf16)), None, 0, 0, 0.0, 0.0, W, H, float(threshold), None, 0, _ptr(rgb),

@@ -442,7 +442,8 @@ class TileExt:
                     rgb, alpha, _ = ops.render_tilecenter_mfma(rays_o, unit_dirs, rec, order, offsets, freq, att, *ws,
                                                                width, height, threshold, bf16=(precision == "bf16"),
                                                                packed=packed, check=False, status=status,
-                                                               status_is_clear=flags_clear, tile_ends=ends)
+                                                               status_is_clear=flags_clear, tile_ends=ends,
+                                                               overlapped=defer)
                 else:
                     packed_feat, bad_attr = self._packed_feat(feat[0])
                     if bad_attr:

@@ -362,3 +362,23 @@ def test_feature_attributes_beyond_fp16_fall_back_to_the_exact_kernel(device, or
     exact = ext.render_tiles_forward_tilecenter_with_feat(*x, fa, 1.0, 4.0, fr.W, fr.H, 8, 8, fr.thr)
     assert all(torch.equal(a, b) for a, b in zip(out, exact))
     assert ext.rgb_wmma_safety_stats() == [calls0 + 1, fb0 + 1]
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("width,height", [(9, 7), (160, 128), (256, 192), (320, 256), (400, 256), (400, 344)])
+def test_teams_of_wavefronts_give_the_bits_of_one_wavefront(device, oracle_mod, bf16, width, height):
+    """The RGB render takes 8, 4, 3 or 2 wavefronts per tile, or teams for its last tiles only, by the number of tiles;
+    the render with a feature channel always one.  Image and alpha are the same bits."""
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=1500, hidden=32, width=width, height=height)
+    cand, off = fr.oracle_lists(oracle_mod)
+    sc = fr.scene
+    t = lambda a: to_dev(a, device)
+    rgb, alpha, bad = _mfma(fr, device, cand, off, bf16)
+    rec = ops.prepare_primitives(t(sc.positions), t(sc.log_scales), t(sc.quats))
+    ro, rd, c, o = t(fr.rays_o), t(fr.rays_d), t(cand), t(off)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8)
+    one = ops.render_tilecenter_mfma_feat(ro, rd, rec, order, o, t(sc.freq), t(sc.att), *[t(w) for w in sc.mlp()],
+                                          torch.zeros(1500, 4, device=device), 1.5, 2.0, fr.W, fr.H, fr.thr, bf16=bf16)
+    assert not bad and float(alpha.max()) > 0.2
+    assert torch.equal(rgb, one[0]) and torch.equal(alpha, one[1])
