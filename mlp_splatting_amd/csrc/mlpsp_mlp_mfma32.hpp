@@ -315,92 +315,6 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, R
   }
 }
 
-// One column block: the 32 pixels of HALF a wavefront's usual share, every pixel on two lanes (n, g = 0 / 1) that
-// hold the same pixel state.  Half the matrix instructions of mlp_wave_mfma32_with() per wavefront -- what a launch
-// too small to fill the chip wants, whose time is the time of one wavefront's chain.  Lane (n, g) supplies k = g of
-// every B operand itself (the sine for g = 0, the cosine for g = 1: no swap), the layer-2 results of a pixel are
-// split over its two lanes as before and one swap per pair brings both to both.  dir[j]: the direction half of the
-// encoding in that form (encode_direction_half).  Same chain, same bits.
-__device__ __forceinline__ void encode_direction_half(float rdx, float rdy, float rdz, const float* __restrict__ freq,
-                                                      const float* __restrict__ att, float dir[18]) {
-  const int g = (threadIdx.x & 63) >> 5;
-  const float x3[3] = {rdx, rdy, rdz};
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      float s, co;
-      det_sincos((x3[c] * freq[f]) * att[f], s, co);
-      dir[c * 6 + f] = g ? co : s;
-    }
-  }
-}
-template <int HID>
-__device__ __forceinline__ void mlp_half_mfma32_with(const MlpLayer1<HID>& w1, const MlpLayer2<HID>& w2,
-                                                     const float x6[6], const float* __restrict__ freq,
-                                                     const float* __restrict__ att, const float* __restrict__ W3,
-                                                     const float* __restrict__ b3, int p, const float dir[18],
-                                                     float out[4]) {
-  static_assert(HID == 32 || HID == 16, "hidden width of the matrix-core f32 evaluation");
-  constexpr int H = HID, R = H / 2;
-  const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
-  const bool row_used = mfma32_hidden_row(m) < H;
-  const float inf = relu_limit();
-  float a1[36];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    a1[4 * q + 0] = row_used ? w1.a1[q][0] : 0.f;
-    a1[4 * q + 1] = row_used ? w1.a1[q][1] : 0.f;
-    a1[4 * q + 2] = row_used ? w1.a1[q][2] : 0.f;
-    a1[4 * q + 3] = row_used ? w1.a1[q][3] : 0.f;
-  }
-  float a2[16] = {}, bias1[16] = {}, bias2[16] = {};
-  interleave<H>(w2.a2, a2);
-  interleave<H>(w1.b1, bias1);
-  interleave<H>(w2.b2, bias2);
-  if constexpr (H != 32) {
-#pragma unroll
-    for (int i = 0; i < R; ++i) a2[i] = row_used ? a2[i] : 0.f;
-  }
-  mf32x16 d;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) d[i] = (i < R) ? bias1[i] : 0.f;
-#pragma unroll
-  for (int j = 0; j < 18; ++j) d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], dir[j], d, 0, 0, 0);
-#pragma unroll
-  for (int c = 3; c < 6; ++c) {
-    float sn[6], cs[6];
-    encode_component(x6[c], freq, att, sn, cs);
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      d = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[c * 6 + f], g ? cs[f] : sn[f], d, 0, 0, 0);
-    }
-  }
-  mf32x16 e;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) e[i] = (i >= R) ? 0.f : bias2[i];
-#pragma unroll
-  for (int i = 0; i < R; ++i) e = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d[i], inf), e, 0, 0, 0);
-
-  const float* __restrict__ w3 = W3 + (size_t)p * (4 * H);
-  const float* __restrict__ bb3 = b3 + (size_t)p * 4;
-  float acc[4] = {bb3[0], bb3[1], bb3[2], bb3[3]};
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    // register i of lane (n, g) is hidden unit 2i + g of pixel n: after the swap `even` holds the g = 0 lane's
-    // value and `odd` the g = 1 lane's, on both lanes
-    float even = relu_f32(e[i], inf), odd = even;
-    half_swap(even, odd);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      acc[k] = fmaf(w3[k * H + 2 * i], even, acc[k]);
-      acc[k] = fmaf(w3[k * H + 2 * i + 1], odd, acc[k]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) out[k] = acc[k];
-}
-
 // The same with the operands requested here.
 template <bool REC = false, bool MASKS = REC, int HID = 32>
 __device__ __forceinline__ void mlp_wave_mfma32(const float x6[6], const float* __restrict__ freq,

@@ -47,34 +47,26 @@ MLPSP_API int mlpsp_render_tilecenter_f32(const float* rays_o_dev, const float* 
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,         \
                      num_frequencies, W1, b1, W2, b2, W3, b3, num_primitives, hidden, g, wpt, per_xcd, (int)items, threshold,           \
                      out_rgb_dev, out_alpha_dev, out_t_dev, ctr, 0.f, 0.f, HitPool{})
-#define MLPSP_F32_MF_LAUNCH(HT)                                                                                   \
-  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<HT, 0>), dim3(f32_mf_grid(g, wpt)), block, 0, s, rays_o_dev,  \
-                     rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev,        \
-                     att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, \
-                     out_t_dev, ctr, 0.f, 0.f, HitPool{}, (const float*)nullptr, (float*)nullptr, (float*)nullptr,   \
-                     (int32_t*)nullptr, (float*)nullptr, (int32_t*)nullptr)
-#define MLPSP_F32_AHEAD_LAUNCH(HT, HALF, UNITS)                                                                   \
-  hipLaunchKernelGGL((render_tilecenter_f32_ahead_kernel<HT, HALF>), dim3((unsigned)(ceil_div_units(UNITS) * kNumXcd)), block, 0, s, \
-                     rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev,    \
-                     freq_dev, att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, ceil_div_units(UNITS),    \
-                     (int)(UNITS), threshold, out_rgb_dev, out_alpha_dev, out_t_dev, ctr)
-  const auto ceil_div_units = [](int64_t units) { return (int)((units + kNumXcd - 1) / kNumXcd); };
+#define MLPSP_F32_ARGS                                                                                            \
+  rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, \
+      b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, out_t_dev, ctr, 0.f, 0.f, HitPool{}
+#define MLPSP_F32_GO(HT)                                                                                          \
+  do {                                                                                                            \
+    if (plan.twelve)                                                                                              \
+      hipLaunchKernelGGL((render_team_f32_kernel<HT, 0, 12>), dim3(plan.grid), dim3(768), 0, s, MLPSP_F32_ARGS);    \
+    else                                                                                                          \
+      hipLaunchKernelGGL((render_mixed_f32_kernel<HT, 0>), dim3(plan.grid), dim3(256), 0, s, MLPSP_F32_ARGS, plan.body); \
+  } while (0)
   if (use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    const int mode = ahead_mode(items, num_primitives, ctr != nullptr);
-    if (mode == 2) {
-      if (hidden == 32) MLPSP_F32_AHEAD_LAUNCH(32, true, 2 * items);
-      else MLPSP_F32_AHEAD_LAUNCH(16, true, 2 * items);
-    } else if (mode == 1) {
-      if (hidden == 32) MLPSP_F32_AHEAD_LAUNCH(32, false, items);
-      else MLPSP_F32_AHEAD_LAUNCH(16, false, items);
-    } else if (hidden == 32) MLPSP_F32_MF_LAUNCH(32);
-    else MLPSP_F32_MF_LAUNCH(16);
+    const PlanF32 plan = plan_f32(g, wpt, items);
+    if (hidden == 32) MLPSP_F32_GO(32);
+    else MLPSP_F32_GO(16);
   }
   else if (hidden == 32 && num_frequencies == 6) MLPSP_F32_LAUNCH(32, 6);
   else if (hidden == 16 && num_frequencies == 6) MLPSP_F32_LAUNCH(16, 6);
   else MLPSP_F32_LAUNCH(0, 0);
-#undef MLPSP_F32_AHEAD_LAUNCH
-#undef MLPSP_F32_MF_LAUNCH
+#undef MLPSP_F32_GO
+#undef MLPSP_F32_ARGS
 #undef MLPSP_F32_LAUNCH
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
@@ -115,11 +107,12 @@ MLPSP_API int mlpsp_render_tilecenter_stats_f32(const float* rays_o_dev, const f
                      (unsigned long long*)nullptr, 0.f, 0.f, HitPool{}, gt_rgb_dev, stat_sum_w_dev,              \
                      stat_max_w_dev, stat_hits_dev, stat_sum_werr_dev, stat_contrib_dev)
 #define MLPSP_STATS_MF_LAUNCH(HT)                                                                                \
-  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<HT, 0, true>), dim3(f32_mf_grid(g, wpt)), block, 0, s,       \
+  hipLaunchKernelGGL((render_stats_f32_kernel<HT>), dim3(superblock_grid(g.ntx, g.nty) * (unsigned)wpt), block, 0, s, \
                      rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev,     \
                      freq_dev, att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev,    \
-                     out_alpha_dev, (float*)nullptr, (unsigned long long*)nullptr, 0.f, 0.f, HitPool{}, gt_rgb_dev, \
-                     stat_sum_w_dev, stat_max_w_dev, stat_hits_dev, stat_sum_werr_dev, stat_contrib_dev)
+                     out_alpha_dev, (float*)nullptr, (unsigned long long*)nullptr, 0.f, 0.f, HitPool{},            \
+                     StatsF32{gt_rgb_dev, stat_sum_w_dev, stat_max_w_dev, stat_hits_dev, stat_sum_werr_dev,        \
+                              stat_contrib_dev})
   if (use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
     if (hidden == 32) MLPSP_STATS_MF_LAUNCH(32);
     else MLPSP_STATS_MF_LAUNCH(16);

@@ -7,6 +7,7 @@
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
+#include "mlpsp_team.hpp"
 #include "mlpsp_walk_f32.hpp"
 
 namespace mlpsp {
@@ -165,23 +166,30 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
 // tiles dealt to the XCDs instead of bands of image rows took the 200,000-primitive 1200x680 frame from 4.33 to
 // 3.93 ms and a 30,000-primitive 333x251 feature frame from 1.77 to 1.47.  Three wavefronts per SIMD: four would need
 // 10 KB of LDS per wavefront, and two less registers, and measured within 1 % of three.
-template <int HT, int EMIT, bool STATS = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_tilecenter_f32_mf_kernel(
+struct ItemF32Lds {
+  DirOperands dir;
+  WalkLds walk;
+};
+struct StatsF32 {
+  const float* gt_rgb;
+  float *sum_w, *max_w;
+  int32_t* hits;
+  float* sum_werr;
+  int32_t* contrib;
+};
+template <int HT, int EMIT, bool STATS>
+__device__ __forceinline__ void render_item_f32(
+    const int tile, const int wslot, const int lane, ItemF32Lds& lds,
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
     const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
     const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
     float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
-    float temp, HitPool hp, const float* __restrict__ gt_rgb, float* __restrict__ stat_sum_w,
-    float* __restrict__ stat_max_w, int32_t* __restrict__ stat_hits, float* __restrict__ stat_sum_werr,
-    int32_t* __restrict__ stat_contrib) {
-  __shared__ DirOperands s_dir;
-  __shared__ WalkLds s_walk;
-  const int unit = (int)(blockIdx.x / kNumXcd), wslot = unit % waves_per_tile;
-  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
-  if (tile < 0) return;
-  const int lane = (int)threadIdx.x, slot = wslot * 64 + lane;
+    float temp, HitPool hp, const StatsF32& stats) {
+  DirOperands& s_dir = lds.dir;
+  WalkLds& s_walk = lds.walk;
+  const int slot = wslot * 64 + lane;
   const int tx = tile % g.ntx, ty = tile / g.ntx;
   const int x = tx * g.TW + slot % g.TW, y = ty * g.TH + slot / g.TW;
   const bool valid = (slot < g.TW * g.TH) && (x < g.W) && (y < g.H);
@@ -193,7 +201,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
   Float3 gt = {0.f, 0.f, 0.f};
   if constexpr (STATS) {
-    if (valid) gt = load3(gt_rgb, pix);
+    if (valid) gt = load3(stats.gt_rgb, pix);
   }
   HitEmitter em = hit_emitter_begin(hp, wslot, start, tile);
   encode_direction(rd.x, rd.y, rd.z, freq, att, s_dir);
@@ -237,11 +245,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
           const float s_w = wave_sum(w), m_w = wave_max(w), s_err = wave_sum(lerr);
           const int n_hit = __popcll(__ballot(hit && (w > 1e-8f))), n_con = __popcll(__ballot(contrib));
           if (lane == 0) {
-            atomicAdd(stat_sum_w + p, s_w);
-            atomicMax(reinterpret_cast<int*>(stat_max_w + p), __float_as_int(m_w));   // weights are >= 0
-            atomicAdd(stat_hits + p, n_hit);
-            if (stat_sum_werr) atomicAdd(stat_sum_werr + p, s_err);
-            if (stat_contrib) atomicAdd(stat_contrib + p, n_con);
+            atomicAdd(stats.sum_w + p, s_w);
+            atomicMax(reinterpret_cast<int*>(stats.max_w + p), __float_as_int(m_w));   // weights are >= 0
+            atomicAdd(stats.hits + p, n_hit);
+            if (stats.sum_werr) atomicAdd(stats.sum_werr + p, s_err);
+            if (stats.contrib) atomicAdd(stats.contrib + p, n_con);
           }
         }
         return __ballot(valid && (acc.trans >= kTransmittanceFloor)) != 0ull;
@@ -261,135 +269,215 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
     atomicAdd(counters + 3, (unsigned long long)n_hits);
   }
 }
-inline unsigned f32_mf_grid(const TileGeom& g, int waves_per_tile) {
-  return superblock_grid(g.ntx, g.nty) * (unsigned)waves_per_tile;
-}
-
-// The same walk (image only, matrix-core evaluation) for launches too small to fill the chip: a few hundred tiles on
-// a thousand SIMDs leave every wavefront alone on its SIMD, where nothing hides the chain id -> geometry record ->
-// hit test -> weight rows -> MLP, and the launch lasts as long as its longest tile.  Two things shorten that chain.
-// (1) The ids of a tile are read 64 at a time (one per lane), and the NEXT entry's geometry record and layer-1
-// operands are requested before the current entry is tested and evaluated, whether or not that entry will hit:
-// registers are plentiful when one wavefront has the SIMD to itself.  (Layer 2's operands are requested as an
-// evaluation begins: they arrive behind layer 1's instructions.)  (2) HALF: two wavefronts share a 64-pixel item,
-// each takes 32 of its pixels -- every pixel on two lanes that carry the same state -- and evaluates one column block,
-// half the matrix instructions (mlp_half_mfma32_with).  Pixels are independent (a pixel below the transmittance floor
-// never blends again, so a wavefront that stops early stops nothing its pixels would still have done).
-// Same arithmetic in the same order either way: same bits.  Work counters are kept per 64-pixel item: the caller
-// does not ask for them with HALF.
-template <int HT, bool HALF>
-__global__ __launch_bounds__(64) void render_tilecenter_f32_ahead_kernel(
+// The pruning statistics beside the image: one wavefront per item.
+template <int HT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_stats_f32_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
     const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
-    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, int per_xcd, int num_items, float thr,
-    float* __restrict__ out_rgb, float* __restrict__ out_alpha, float* __restrict__ out_t,
-    unsigned long long* __restrict__ counters) {
-  // (with HALF, num_items and per_xcd count half items)
-  const int unit = (blockIdx.x % kNumXcd) * per_xcd + blockIdx.x / kNumXcd;
-  if (unit >= num_items) return;
-  const int item = HALF ? unit >> 1 : unit;
-  const int tile = item / waves_per_tile, wslot = item % waves_per_tile;
-  const int lane = (int)threadIdx.x;
-  const int slot = HALF ? wslot * 64 + (unit & 1) * 32 + (lane & 31) : wslot * 64 + lane;
-  const bool writer = !HALF || lane < 32;
+    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
+    float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
+    float temp, HitPool hp, StatsF32 stats) {
+  __shared__ ItemF32Lds s;
+  const int unit = (int)(blockIdx.x / kNumXcd);
+  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
+  if (tile < 0) return;
+  render_item_f32<HT, 0, true>(tile, unit % waves_per_tile, (int)threadIdx.x, s, rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, N, g, waves_per_tile, thr, out_rgb, out_alpha, out_t, counters,
+      beta, temp, hp, stats);
+}
+
+// The same item by a team of wavefronts (mlpsp_team.hpp).  Wavefront 0 adds up
+// image and depth, in list order and with the roundings of the single wavefront; each wavefront writes the record of its
+// own entry.
+template <int TEAM>
+struct TeamF32Lds {
+  DirOperands dir;
+  TeamWalkLds<TEAM> walk;
+  float pay[2][TEAM][5][64];        // opacity, colour, ray parameter
+  int chunk;
+};
+template <int HT, int EMIT, int TEAM>
+__device__ __forceinline__ void render_team_item_f32(
+    const int tile, const int wslot, const int k, const int lane, TeamF32Lds<TEAM>& s,
+    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
+    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
+    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
+    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
+    float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
+    float temp, HitPool hp) {
+  const int slot = wslot * 64 + lane;
   const int tx = tile % g.ntx, ty = tile / g.ntx;
-  const int lx = slot % g.TW, ly = slot / g.TW;
-  const int x = tx * g.TW + lx, y = ty * g.TH + ly;
+  const int x = tx * g.TW + slot % g.TW, y = ty * g.TH + slot / g.TW;
   const bool valid = (slot < g.TW * g.TH) && (x < g.W) && (y < g.H);
   const int pix = valid ? (y * g.W + x) : 0;
-  const float rox = valid ? rays_o[pix * 3 + 0] : 0.f;
-  const float roy = valid ? rays_o[pix * 3 + 1] : 0.f;
-  const float roz = valid ? rays_o[pix * 3 + 2] : 0.f;
-  const float rdx = valid ? rays_d[pix * 3 + 0] : 0.f;
-  const float rdy = valid ? rays_d[pix * 3 + 1] : 0.f;
-  const float rdz = valid ? rays_d[pix * 3 + 2] : 0.f;
-  const int start = offsets[tile];
-  const int end = offsets[tile + 1];
-
+  const Float3 ro = valid ? load3(rays_o, pix) : Float3{0.f, 0.f, 0.f}, rd = valid ? load3(rays_d, pix) : Float3{0.f, 0.f, 0.f};
+  const int start = offsets[tile], end = offsets[tile + 1];
   PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
-  __shared__ DirOperands dir;
-  float dir_half[18];
-  if constexpr (HALF) encode_direction_half(rdx, rdy, rdz, freq, att, dir_half);
-  else encode_direction(rdx, rdy, rdz, freq, att, dir);
+  TeamSlots slots{wslot * hp.table_stride + (start >> 4) + tile, 0, 0};
+  if (k == 0) encode_direction(rd.x, rd.y, rd.z, freq, att, s.dir);
 
-  bool done = false;
-  for (int base = start; base < end && !done; base += 64) {
-    const int n = min(64, end - base);
-    const int idv = lane < n ? order[base + lane] : -1;
-    // entry 0 of this stretch: nothing to hide its requests behind
-    int p = __builtin_amdgcn_readlane(idv, 0);
-    bool ok = p >= 0 && p < N;
-    PrimRecord P = prims[ok ? p : 0];
-    MlpLayer1<HT> w;
-    request_layer1<HT>(W1, b1, ok ? p : 0, w);
-    for (int k = 0; k < n; ++k) {
-      // the next entry's record and operands, under way while this one is worked on (an id outside [0, N) and the
-      // entry after the last one request primitive 0 and are not used)
-      const int q = __builtin_amdgcn_readlane(idv, min(k + 1, 63));
-      const bool ok_next = k + 1 < n && q >= 0 && q < N;
-      const int p_next = ok_next ? q : 0;
-      const PrimRecord P_next = prims[p_next];
-      MlpLayer1<HT> w_next;
-      request_layer1<HT>(W1, b1, p_next, w_next);
-      if (ok) {
-        HitInfo h;
-        const bool live = valid && (acc.trans >= kTransmittanceFloor);
-        const bool hit = live && hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, h);
-        const unsigned long long hit_mask = __ballot(hit);
-        ++n_proc;
-        if (hit_mask != 0ull) {
-          ++n_proc_hit;
-          n_hits += __popcll(hit_mask);
-          // (lanes that did not hit carry no hit point; the matrix-core evaluation runs on all 64 lanes)
-          const float x6[6] = {rdx, rdy, rdz, hit ? h.dx : 0.f, hit ? h.dy : 0.f, hit ? h.dz : 0.f};
-          float o[4];
-          MlpLayer2<HT> w2;
-          request_layer2<HT>(W2, b2, p, w2);
-          if constexpr (HALF) mlp_half_mfma32_with<HT>(w, w2, x6, freq, att, W3, b3, p, dir_half, o);
-          else mlp_wave_mfma32_with<false, false, HT>(w, [&](MlpLayer2<HT>& to) { to = w2; }, x6, freq, att, W3, b3, p, dir, o);
-          if (hit) blend_step(acc, o[0], o[1], o[2], o[3], h.decay, h.t);
+  int p_mine = 0;
+  float gates[4];
+  walk_team_f32<TEAM>(
+      order, start, end, N, prims, valid, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, thr, s.walk, k, lane,
+      [&]() { return valid && (acc.trans >= kTransmittanceFloor); },
+      [&](int p, bool hit, const HitInfo& h, unsigned long long, int buf) {
+        p_mine = p;
+        const float x6[6] = {rd.x, rd.y, rd.z, hit ? h.dx : 0.f, hit ? h.dy : 0.f, hit ? h.dz : 0.f};
+        float o[4];
+        mlp_wave_mfma32<false, false, HT>(x6, freq, att, W1, b1, W2, b2, W3, b3, p, s.dir, o);
+        float(&pay)[5][64] = s.pay[buf][k];
+        if (hit) {
+          const float sigma = softplus(o[3]) * h.decay;
+          pay[0][lane] = 1.f - det_exp(-sigma);
+          pay[1][lane] = sigmoid(o[0]);
+          pay[2][lane] = sigmoid(o[1]);
+          pay[3][lane] = sigmoid(o[2]);
+          pay[4][lane] = h.t;
+          if constexpr (EMIT > 1) {
+            const PrimRecord& P = prims[p];
+            tetra_gates(h.qlx, h.qly, h.qlz, P.lgx, P.lgy, P.lgz, beta, temp, gates);
+          }
         }
-        if (__ballot(valid && (acc.trans >= kTransmittanceFloor)) == 0ull) {
-          done = true;
-          break;
+      },
+      [&](const unsigned long long* masks, int entries, int buf) {
+        int kept = 0, mine = -1;
+        float w_mine = -1.f;
+#pragma unroll
+        for (int i = 0; i < TEAM; ++i) {
+          if (i == k && i < entries) n_proc += __ballot(valid && acc.trans >= kTransmittanceFloor) != 0ull;
+          const unsigned long long m = masks[i];
+          const unsigned long long um = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m) |
+                                        ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32);
+          if (um == 0ull) continue;
+          const bool hit = ((um >> lane) & 1ull) && (acc.trans >= kTransmittanceFloor);
+          const unsigned long long blended = __ballot(hit);
+          if (blended == 0ull) continue;           // (behind the last entry that counts)
+          const float(&pay)[5][64] = s.pay[buf][i];
+          const float alpha = pay[0][lane], w = acc.trans * alpha;
+          if (i == k) {
+            ++n_proc_hit;
+            n_hits += __popcll(blended);
+            mine = kept;
+            w_mine = hit ? w : -1.f;
+          }
+          ++kept;
+          if (hit) {
+            if (k == 0) {
+              acc.w_acc = fmaf(1.f, w, acc.w_acc);
+              acc.t_acc = fmaf(w, pay[4][lane], acc.t_acc);
+              acc.cr = fmaf(w, pay[1][lane], acc.cr);
+              acc.cg = fmaf(w, pay[2][lane], acc.cg);
+              acc.cb = fmaf(w, pay[3][lane], acc.cb);
+            }
+            acc.trans = acc.trans * (1.f - alpha);
+          }
         }
-      }
-      p = p_next;
-      ok = ok_next;
-      P = P_next;
-      w = w_next;
-    }
-  }
+        if constexpr (EMIT > 0) {
+          const int rs = team_slot<kHitGrab, true>(slots, kept, mine, k, lane, hp.counters, hp.chunk_table, hp.pool_chunks, s.chunk);
+          if (rs >= 0) {
+            float* __restrict__ rec = reinterpret_cast<float*>(hp.records + (size_t)rs * hp.record_bytes);
+            rec[lane] = w_mine;
+            if constexpr (EMIT > 1) {
+              if (w_mine >= 0.f) {          // the gates of a missed pixel are never read
+#pragma unroll
+                for (int c = 0; c < 4; ++c) rec[(c + 1) * 64 + lane] = gates[c];
+              }
+            }
+            if (lane == 0) hp.hit_ids[rs] = p_mine;
+          }
+        }
+        return __ballot(valid && (acc.trans >= kTransmittanceFloor)) != 0ull;
+      });
 
-  if (valid && writer) {
-    out_rgb[pix * 3 + 0] = acc.cr;
-    out_rgb[pix * 3 + 1] = acc.cg;
-    out_rgb[pix * 3 + 2] = acc.cb;
+  if (k == 0 && valid) {
+    store3(out_rgb, pix, acc.cr, acc.cg, acc.cb);
     out_alpha[pix] = 1.f - acc.trans;
     if (out_t) out_t[pix] = acc.t_acc / (acc.w_acc > 1e-8f ? acc.w_acc : 1.f);
   }
-  if (!HALF && counters && lane == 0) {
+  if constexpr (EMIT > 0) {
+    if (k == 0 && lane == 0) hp.item_hits[tile * waves_per_tile + wslot] = slots.count;
+  }
+  if (counters && lane == 0) {
     atomicAdd(counters + 1, (unsigned long long)n_proc);
     atomicAdd(counters + 2, (unsigned long long)n_proc_hit);
     atomicAdd(counters + 3, (unsigned long long)n_hits);
   }
 }
 
-// Which of the two kernels above a launch of `items` 64-pixel items takes: 2 = two wavefronts per item (at most one
-// wavefront per SIMD of the chip's 1,024, and no work counters asked for), 1 = one wavefront per item with the next
-// entry requested ahead (at most 1,024 items), 0 = neither (the kernel for launches that fill the chip).
-// MLPSP_F32_AHEAD=0 / 1 / 2 in the environment overrides the size rule (comparison runs, tests); 2 still needs a
-// launch without counters.
-constexpr int kAheadItems = 1024;
-inline int ahead_mode(int64_t items, int num_primitives, bool counters) {
-  if (num_primitives <= 0) return 0;
-  int mode = items * 2 <= kAheadItems ? 2 : items <= kAheadItems ? 1 : 0;
+template <int HT, int EMIT, int TEAM>
+__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_team_f32_kernel(
+    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
+    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
+    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
+    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
+    float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
+    float temp, HitPool hp) {
+  __shared__ TeamF32Lds<TEAM> s;
+  const int unit = (int)(blockIdx.x / kNumXcd);
+  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
+  if (tile < 0) return;
+  render_team_item_f32<HT, EMIT, TEAM>(tile, unit % waves_per_tile, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6),
+                                       (int)threadIdx.x & 63, s, rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, N, g, waves_per_tile, thr, out_rgb, out_alpha, out_t, counters,
+      beta, temp, hp);
+}
+
+// A wavefront per item, four items to a workgroup, but for the last ones: the workgroups from `body` on (per XCD) take one
+// item each, as a team.
+template <int HT, int EMIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_mixed_f32_kernel(
+    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
+    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
+    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
+    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
+    const float* __restrict__ b3, int N, TileGeom g, int waves_per_tile, float thr, float* __restrict__ out_rgb,
+    float* __restrict__ out_alpha, float* __restrict__ out_t, unsigned long long* __restrict__ counters, float beta,
+    float temp, HitPool hp, int body) {
+  union Lds {
+    ItemF32Lds item[4];
+    TeamF32Lds<4> team;
+  };
+  __shared__ Lds s;
+  const int unit = (int)(blockIdx.x / kNumXcd), xcd = (int)(blockIdx.x % kNumXcd);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  const bool alone = unit < body;
+  const int item = alone ? unit * 4 + wave : body * 4 + (unit - body);
+  const int tile = superblock_tile_of(xcd, item / waves_per_tile, g.ntx, g.nty);
+  if (tile < 0) return;
+  if (alone)
+    render_item_f32<HT, EMIT, false>(tile, item % waves_per_tile, lane, s.item[wave], rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, N, g, waves_per_tile, thr, out_rgb, out_alpha, out_t, counters,
+      beta, temp, hp, StatsF32{});
+  else
+    render_team_item_f32<HT, EMIT, 4>(tile, item % waves_per_tile, wave, lane, s.team, rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, N, g, waves_per_tile, thr, out_rgb, out_alpha, out_t, counters,
+      beta, temp, hp);
+}
+
+// Launch of `items` 64-pixel items on the matrix cores.  An evaluation keeps its SIMD's matrix core busy, so a team is a
+// multiple of four, one wavefront on each SIMD of a CU (3, 6 and 8 were slower than 4, 2 as well); twelve where the items
+// are no more than the CUs.  Else the mixed kernel with a team for each of the last 1,024 items -- for all of them up to
+// 1,280 --, which shortens the tail of the launch: what is left when the queue is empty lasts a third as long.  Frame in us,
+// one wavefront per item / teams of four / mixed: 96 items 690 / 315 (of twelve 264), 300 items hidden 16 495 / 268, 588
+// items 780 / 512, 1,200 items 1,020 / 744 / 785, 1,610 items 980 / 901 / 841, 2,214 items 1,086 / 1,070 / 985, 4,860 items
+// 1,840 / 2,128 / 1,766, 12,750 items 4,034 / 5,065 / 3,945; with 768 and 1,536 instead of 1,024 items 4,020 and 3,955.
+// MLPSP_F32_AHEAD=0 / 1 / 2 in the environment: a wavefront per item throughout / four / twelve (comparison runs, tests).
+struct PlanF32 {
+  bool twelve;
+  int body;          // workgroups per XCD with an item per wavefront (mixed kernel)
+  unsigned grid;
+};
+inline PlanF32 plan_f32(const TileGeom& g, int waves_per_tile, int64_t items) {
+  const unsigned slots = superblock_grid(g.ntx, g.nty) * (unsigned)waves_per_tile;
   const char* e = getenv("MLPSP_F32_AHEAD");
-  if (e && e[0] >= '0' && e[0] <= '2' && items * 2 <= 2147483647LL - 8) mode = e[0] - '0';
-  return (mode == 2 && counters) ? 1 : mode;
+  const int forced = e && e[0] >= '0' && e[0] <= '2' ? e[0] - '0' : -1;
+  if (forced == 2 || (forced < 0 && items <= 256)) return PlanF32{true, 0, slots};
+  const int per_xcd = (int)(slots / kNumXcd);
+  const int teams = forced == 0 ? 0 : forced == 1 || items <= 1280 ? per_xcd : min(per_xcd, 1024 / kNumXcd);
+  const int body = forced == 0 ? (per_xcd + 3) / 4 : (per_xcd - teams) / 4;
+  return PlanF32{false, body, (unsigned)(kNumXcd * (body + max(0, per_xcd - 4 * body)))};
 }
 
 // Whether the matrix-core f32 evaluation applies: the 72->32->32->4 or 72->16->16->4 shape, weight arrays that can be

@@ -175,17 +175,22 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
                      num_frequencies, W1, b1, W2, b2, W3, b3, num_primitives, hidden, g, wpt, per_xcd, (int)items, threshold,          \
                      out_rgb_dev, out_alpha_dev, (float*)nullptr, (unsigned long long*)nullptr, gating_beta,      \
                      gating_temp, hp)
-#define MLPSP_EMIT_MF_LAUNCH(EM)                                                                                  \
-  hipLaunchKernelGGL((render_tilecenter_f32_mf_kernel<32, EM>), dim3(f32_mf_grid(g, wpt)), block, 0, s, rays_o_dev, \
-                     rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev,        \
-                     att_dev, W1, b1, W2, b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, \
-                     (float*)nullptr, (unsigned long long*)nullptr, gating_beta, gating_temp, hp,                   \
-                     (const float*)nullptr, (float*)nullptr, (float*)nullptr, (int32_t*)nullptr, (float*)nullptr,   \
-                     (int32_t*)nullptr)
+#define MLPSP_EMIT_ARGS                                                                                           \
+  rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, \
+      b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, (float*)nullptr,                   \
+      (unsigned long long*)nullptr, gating_beta, gating_temp, hp
+#define MLPSP_EMIT_GO(EM)                                                                                         \
+  do {                                                                                                            \
+    if (plan.twelve)                                                                                              \
+      hipLaunchKernelGGL((render_team_f32_kernel<32, EM, 12>), dim3(plan.grid), dim3(768), 0, s, MLPSP_EMIT_ARGS);  \
+    else                                                                                                          \
+      hipLaunchKernelGGL((render_mixed_f32_kernel<32, EM>), dim3(plan.grid), dim3(256), 0, s, MLPSP_EMIT_ARGS, plan.body); \
+  } while (0)
   const bool gated = feat_slots > 1;
   if (hidden == 32 && use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    if (gated) MLPSP_EMIT_MF_LAUNCH(2);
-    else MLPSP_EMIT_MF_LAUNCH(1);
+    const PlanF32 plan = plan_f32(g, wpt, items);
+    if (gated) MLPSP_EMIT_GO(2);
+    else MLPSP_EMIT_GO(1);
   } else if (hidden == 32 && num_frequencies == 6) {
     if (gated) MLPSP_EMIT_LAUNCH(32, 6, 2);
     else MLPSP_EMIT_LAUNCH(32, 6, 1);
@@ -193,7 +198,8 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
     if (gated) MLPSP_EMIT_LAUNCH(0, 0, 2);
     else MLPSP_EMIT_LAUNCH(0, 0, 1);
   }
-#undef MLPSP_EMIT_MF_LAUNCH
+#undef MLPSP_EMIT_GO
+#undef MLPSP_EMIT_ARGS
 #undef MLPSP_EMIT_LAUNCH
   MLPSP_LAUNCH_CHECK();
   const dim3 agrid((unsigned)(per_xcd * kNumXcd), (unsigned)ceil_div(feat_channels, 512)), ablock(256);

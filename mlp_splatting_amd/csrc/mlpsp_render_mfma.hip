@@ -14,6 +14,7 @@
 #include "mlpsp_hitrec.hpp"
 #include "mlpsp_mfma16.hpp"
 #include "mlpsp_host.hpp"
+#include "mlpsp_team.hpp"
 
 // 32-channel accumulator tiles per wavefront of the feature GEMM: a block of four wavefronts covers 128 x this many
 // channels of a tile (2: three blocks per CU instead of two, a few percent faster than 4 on 512 channels)
@@ -462,12 +463,6 @@ __device__ __forceinline__ void render_tile_mfma(
 // next entry's weights a round ahead changes nothing there.  The price is the second pass over the opacities and up to
 // TEAM - 1 entries evaluated behind the last one that counts.
 // ---------------------------------------------------------------------------------------------
-// (orders LDS alone: requests to memory stay in flight across it)
-__device__ __forceinline__ void team_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 template <int TEAM>
 struct TeamRound {
   float alpha[TEAM][64];
@@ -550,7 +545,7 @@ __device__ __forceinline__ void render_tile_team(
     team_barrier();
     for (int r = 0; r < rounds; ++r) {
       float alpha = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-      bool hit = false, hit_bad = false;
+      bool hit = false, hit_bad = false, mlp_bad = false;     // mlp_bad: of any lane's pixel
       const bool mine = todo != 0ull;
       if (mine) {
         const FastRec R = fast_arrived(q);
@@ -585,16 +580,15 @@ __device__ __forceinline__ void render_tile_team(
           }
         }
         const unsigned long long mask = __ballot(hit);
-        ++n_proc;
         if (mask != 0ull) {
           const unsigned char* __restrict__ blk = packed + (size_t)p_now * kPackStride;
           hit_bad = !((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit);
           if ((unsigned)mask != 0u && (unsigned)(mask >> 32) != 0u)
-            hit_bad |= mlp_pair_mfma16<T, Ops<T>::kCheckHidden, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm,
-                                                                                     s_dir, o, table);
+            mlp_bad = mlp_pair_mfma16<T, Ops<T>::kCheckHidden, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm,
+                                                                                    s_dir, o, table);
           else
-            hit_bad |= mlp_wave_mfma16<T, Ops<T>::kCheckHidden, false, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz,
-                                                                                            kfm, s_dir, o, nullptr, table);
+            mlp_bad = mlp_wave_mfma16<T, Ops<T>::kCheckHidden, false, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz,
+                                                                                           kfm, s_dir, o, nullptr, table);
           if (hit) {
             hit_bad |= !(max3_abs(o[0], o[1], o[2]) <= 3.4028235e38f) || !(__builtin_fabsf(o[3]) <= 3.4028235e38f);
             alpha = 1.f - fast_exp(-(fast_softplus(o[3]) * h.decay));
@@ -618,8 +612,9 @@ __device__ __forceinline__ void render_tile_team(
         const float a = i == k ? (hit ? alpha : 0.f) : round.alpha[i][l];
         const bool open = valid && trans >= kTransmittanceFloor;
         if (i == k) {                          // (an entry behind the last one that counts leaves no trace)
-          bad |= hit && open && hit_bad;
+          n_proc += mine && __ballot(open) != 0ull;
           const unsigned long long blended = __ballot(hit && open);
+          bad |= (hit && open && hit_bad) || (blended != 0ull && mlp_bad);
           n_proc_hit += blended != 0ull;
           n_hits += __popcll(blended);
         }

@@ -5,11 +5,13 @@
 //
 // Geometry, order, activations and compositing are the f32 expressions of the render (f32 MLP: its bits with
 // `render_order`, the record kernels' rounding of layer 2 without).  Bound by the MLP; the steps add 3.3 KB of contiguous
-// stores per hit step.  200,000 primitives, 1200x680, f32: 4.7 ms, against 4.4 + 6.6 ms of the record forward's two walks.
+// stores per hit step.  200,000 primitives, 1200x680, f32: 4.5 ms, against 4.4 + 6.6 ms of the record forward's two walks;
+// 20,000 primitives, 320x240: 1.15 ms with a wavefront per tile, 0.88 with teams.
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mfma16.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
+#include "mlpsp_team.hpp"
 #include "mlpsp_train.hpp"
 #include "mlpsp_walk_f32.hpp"
 
@@ -24,113 +26,270 @@ __device__ __forceinline__ bool train_not_finite(float v) { return !(__builtin_f
 
 // T = float: the MLP in exact f32 (REC: layer 2 rounded as the record kernels do); _Float16 / __bf16: reduced operands.
 // All but the exact forward in the render's order report what is not finite, as the reduced-precision record forward does.
-template <typename T> struct TrainLds { DirWords dir; };
-template <> struct TrainLds<float> { DirOperands dir; };
+template <typename T> struct TrainDir { typedef DirWords type; };
+template <> struct TrainDir<float> { typedef DirOperands type; };
 
+struct TrainScene {
+  const float *rays_o, *rays_d;
+  const PrimRecord* prims;
+  const int32_t *order, *offsets;
+  const float *freq, *att, *W1, *b1, *W2, *b2, *W3, *b3;
+  const unsigned char* packed;
+  int N, W, H, ntx, nty;
+  float thr;
+  int max_hits;
+};
+template <typename T>
+struct TrainItemLds {
+  typename TrainDir<T>::type dir;
+  WalkLds walk;
+};
+template <typename T, int TEAM>
+struct TrainTeamLds {
+  typename TrainDir<T>::type dir;
+  TeamWalkLds<TEAM> walk;
+  float pay[2][TEAM][4][64];       // opacity, colour
+  int chunk;
+};
+
+// A lane's pixel and the encoding of its ray.
+struct TrainPixel {
+  bool valid;
+  int pix;
+  Float3 ro, rd;
+  float kf[3];
+};
+__device__ __forceinline__ TrainPixel train_pixel(const TrainScene& c, int tile, int l) {
+  TrainPixel t;
+  const int x = (tile % c.ntx) * 8 + (l & 7), y = (tile / c.ntx) * 8 + (l >> 3);
+  t.valid = (x < c.W) && (y < c.H);
+  t.pix = t.valid ? (y * c.W + x) : 0;
+  t.ro = t.valid ? load3(c.rays_o, t.pix) : Float3{0.f, 0.f, 0.f};
+  t.rd = t.valid ? load3(c.rays_d, t.pix) : Float3{0.f, 0.f, 0.f};
+  t.kf[0] = t.kf[1] = t.kf[2] = 0.f;
+  return t;
+}
+template <typename T>
+__device__ __forceinline__ void train_encode(const TrainScene& c, const TrainPixel& t, int l, typename TrainDir<T>::type& dir) {
+  if constexpr (sizeof(T) == 4) encode_direction(t.rd.x, t.rd.y, t.rd.z, c.freq, c.att, dir);
+  else encode_direction_words<T>(t.rd.x, t.rd.y, t.rd.z, t.kf, l, dir);
+}
+// What an entry computes for a lane's pixel; zeros in the lanes that it does not hit, but for the masks.
+struct TrainEntry {
+  float R, G, B, sigma_raw, alpha, decay, logit, dx, dy, dz;
+  uint32_t mask[2];
+};
+// bad: this lane's pixel yields something that is not finite; mlp_bad: some pixel's hidden layers do.
 template <typename T, bool REC>
-__device__ __forceinline__ void train_forward_body(
-    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
-    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
-    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
-    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
-    const float* __restrict__ b3, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx, int nty,
-    float thr, int max_hits, const StepPool& sp, TrainOut out, TrainLds<T>& s, WalkLds& s_walk) {
+__device__ __forceinline__ TrainEntry train_entry(const TrainScene& c, const TrainPixel& t, int p, bool hit, const HitInfo& h,
+                                                  unsigned long long mask, int l, const typename TrainDir<T>::type& dir,
+                                                  bool& bad, bool& mlp_bad) {
   constexpr bool F32 = sizeof(T) == 4;
-  constexpr bool CHECKED = !F32 || REC;
-  const int tile = superblock_tile(blockIdx.x, ntx, nty);
-  if (tile < 0) return;
-  const int l = threadIdx.x;
-  const int x = (tile % ntx) * 8 + (l & 7), y = (tile / ntx) * 8 + (l >> 3);
-  const bool valid = (x < W) && (y < H);
-  const int pix = valid ? (y * W + x) : 0;
-  const Float3 ro = valid ? load3(rays_o, pix) : Float3{0.f, 0.f, 0.f}, rd = valid ? load3(rays_d, pix) : Float3{0.f, 0.f, 0.f};
-  float kf[3] = {0.f, 0.f, 0.f};
+  TrainEntry e{};
+  e.dx = hit ? h.dx : 0.f;
+  e.dy = hit ? h.dy : 0.f;
+  e.dz = hit ? h.dz : 0.f;
+  e.decay = h.decay;
+  float o[4];
+  bad = mlp_bad = false;
   if constexpr (F32) {
-    encode_direction(rd.x, rd.y, rd.z, freq, att, s.dir);
+    const float x6[6] = {t.rd.x, t.rd.y, t.rd.z, e.dx, e.dy, e.dz};
+    mlp_wave_mfma32<REC, true, 32>(x6, c.freq, c.att, c.W1, c.b1, c.W2, c.b2, c.W3, c.b3, p, dir, o, e.mask);
   } else {
-    phase_scales(freq, att, l >> 5, kf);
-    encode_direction_words<T>(rd.x, rd.y, rd.z, kf, l, s.dir);
+    mlp_bad = mlp_wave_mfma16<T, true, true>(c.packed + (size_t)p * kPackStride, mask, l, e.dx, e.dy, e.dz, t.kf, dir, o, e.mask);
   }
-  const int start = offsets[tile], end = offsets[tile + 1];
+  e.logit = o[3];
+  if (hit) {
+    e.R = sigmoid(o[0]);
+    e.G = sigmoid(o[1]);
+    e.B = sigmoid(o[2]);
+    e.sigma_raw = softplus(o[3]);
+    e.alpha = 1.f - det_exp(-(e.sigma_raw * h.decay));
+    if constexpr (!F32 || REC)
+      bad = train_not_finite((e.dx + e.dy) + e.dz) || train_not_finite(h.decay) ||
+            train_not_finite((o[0] + o[1]) + (o[2] + o[3])) || train_not_finite((e.R + e.G) + (e.B + e.sigma_raw)) ||
+            train_not_finite(e.alpha);
+  }
+  return e;
+}
+__device__ __forceinline__ void train_store(const StepPool& sp, int slot, int l, int p, bool hit, float before, const TrainEntry& e) {
+  if (slot >= 0)
+    step_store(sp, slot, l, p, hit, e.R, e.G, e.B, e.sigma_raw, before, e.alpha, e.decay, e.logit, e.dx, e.dy, e.dz, e.mask[0], e.mask[1]);
+}
+__device__ __forceinline__ void train_status(const StepPool& sp, bool over, bool bad, int l) {
+  int bits = 0;
+  if (__ballot(over) != 0ull) bits |= kTrainCapacity;
+  if (__ballot(bad) != 0ull) bits |= kTrainNumeric;
+  if (bits != 0 && l == 0) atomicOr(sp.head + 1, bits);
+}
+
+// One tile by one wavefront.
+template <typename T, bool REC>
+__device__ __forceinline__ void train_tile(const int tile, const int l, TrainItemLds<T>& s, const TrainScene& c,
+                                           const StepPool& sp, const TrainOut& out) {
+  constexpr bool CHECKED = sizeof(T) != 4 || REC;
+  TrainPixel t = train_pixel(c, tile, l);
+  if constexpr (sizeof(T) != 4) phase_scales(c.freq, c.att, l >> 5, t.kf);
+  train_encode<T>(c, t, l, s.dir);
+  const int start = c.offsets[tile], end = c.offsets[tile + 1];
   float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
   int used = 0;
   bool over = false, bad = false;
   StepWriter writer = step_writer_begin(start, tile);
   walk_tile_f32(
-      order, start, end, N, prims, valid, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, thr, s_walk,
-      [&]() { return valid && (trans >= kTransmittanceFloor) && (used < max_hits); },
+      c.order, start, end, c.N, c.prims, t.valid, t.ro.x, t.ro.y, t.ro.z, t.rd.x, t.rd.y, t.rd.z, c.thr, s.walk,
+      [&]() { return t.valid && (trans >= kTransmittanceFloor) && (used < c.max_hits); },
       [&](int p, bool hit, const HitInfo& h, unsigned long long mask) {
         if (mask == 0ull) return true;
-        const float dx = hit ? h.dx : 0.f, dy = hit ? h.dy : 0.f, dz = hit ? h.dz : 0.f;
-        float o[4];
-        uint32_t mk[2] = {0u, 0u};
-        if constexpr (F32) {
-          const float x6[6] = {rd.x, rd.y, rd.z, dx, dy, dz};
-          mlp_wave_mfma32<REC, true, 32>(x6, freq, att, W1, b1, W2, b2, W3, b3, p, s.dir, o, mk);
-        } else {
-          bad |= mlp_wave_mfma16<T, true, true>(packed + (size_t)p * kPackStride, mask, l, dx, dy, dz, kf, s.dir, o, mk);
-        }
-        if constexpr (CHECKED) bad |= hit && (train_not_finite((dx + dy) + dz) || train_not_finite(h.decay));
+        bool lane_bad, mlp_bad;
+        const TrainEntry e = train_entry<T, REC>(c, t, p, hit, h, mask, l, s.dir, lane_bad, mlp_bad);
+        if constexpr (CHECKED) bad |= lane_bad | mlp_bad;
         const int slot = step_writer_next(sp, writer, l);
-        float R = 0.f, G = 0.f, Bc = 0.f, sigma_raw = 0.f, alpha = 0.f;
         const float before = trans;
         if (hit) {
-          R = sigmoid(o[0]);
-          G = sigmoid(o[1]);
-          Bc = sigmoid(o[2]);
-          sigma_raw = softplus(o[3]);
-          alpha = 1.f - det_exp(-(sigma_raw * h.decay));
-          if constexpr (CHECKED)
-            bad |= train_not_finite((o[0] + o[1]) + (o[2] + o[3])) || train_not_finite((R + G) + (Bc + sigma_raw)) ||
-                   train_not_finite(alpha);
-          const float weight = trans * alpha;
-          cr = fmaf(weight, R, cr);
-          cg = fmaf(weight, G, cg);
-          cb = fmaf(weight, Bc, cb);
-          trans = trans * (1.f - alpha);
+          const float weight = trans * e.alpha;
+          cr = fmaf(weight, e.R, cr);
+          cg = fmaf(weight, e.G, cg);
+          cb = fmaf(weight, e.B, cb);
+          trans = trans * (1.f - e.alpha);
           ++used;
           if constexpr (CHECKED) bad |= train_not_finite(trans);
         }
-        if (slot >= 0) step_store(sp, slot, l, p, hit, R, G, Bc, sigma_raw, before, alpha, h.decay, o[3], dx, dy, dz, mk[0], mk[1]);
-        const bool live = valid && (trans >= kTransmittanceFloor);
-        over |= live && (used >= max_hits);      // np_tile_kernels.cu:3166-3168: refused, never truncated silently
+        train_store(sp, slot, l, p, hit, before, e);
+        const bool live = t.valid && (trans >= kTransmittanceFloor);
+        over |= live && (used >= c.max_hits);      // np_tile_kernels.cu:3166-3168: refused, never truncated silently
         return __ballot(live) != 0ull;
       });
   if constexpr (CHECKED) bad |= train_not_finite((cr + cg) + cb);
   if (l == 0) sp.tile_steps[tile] = writer.count;
-  int bits = 0;
-  if (__ballot(over) != 0ull) bits |= kTrainCapacity;
-  if (__ballot(bad) != 0ull) bits |= kTrainNumeric;
-  if (bits != 0 && l == 0) atomicOr(sp.head + 1, bits);
-  if (valid) {
-    store3(out.rgb, pix, cr, cg, cb);
-    out.alpha[pix] = 1.f - trans;
+  train_status(sp, over, bad, l);
+  if (t.valid) {
+    store3(out.rgb, t.pix, cr, cg, cb);
+    out.alpha[t.pix] = 1.f - trans;
   }
 }
 
-template <bool REC>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void train_forward_f32_kernel(
-    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
-    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
-    const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
-    const float* __restrict__ W2, const float* __restrict__ b2, const float* __restrict__ W3,
-    const float* __restrict__ b3, int N, int W, int H, int ntx, int nty, float thr, int max_hits, StepPool sp, TrainOut out) {
-  __shared__ TrainLds<float> s;
-  __shared__ WalkLds s_walk;
-  train_forward_body<float, REC>(rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, nullptr, N, W, H,
-                                 ntx, nty, thr, max_hits, sp, out, s, s_walk);
+// One tile by a team (mlpsp_team.hpp): wavefront 0 adds up the colours, each wavefront writes the step of its own entry.
+template <typename T, bool REC, int TEAM>
+__device__ __forceinline__ void train_tile_team(const int tile, const int k, const int l, TrainTeamLds<T, TEAM>& s,
+                                                const TrainScene& c, const StepPool& sp, const TrainOut& out) {
+  constexpr bool CHECKED = sizeof(T) != 4 || REC;
+  TrainPixel t = train_pixel(c, tile, l);
+  if constexpr (sizeof(T) != 4) phase_scales(c.freq, c.att, l >> 5, t.kf);
+  if (k == 0) train_encode<T>(c, t, l, s.dir);
+  const int start = c.offsets[tile], end = c.offsets[tile + 1];
+  float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
+  int used = 0, p_mine = 0;
+  bool over = false, bad = false, lane_bad = false, mlp_bad = false;
+  TeamSlots slots{(start >> 4) + tile, 0, 0};
+  TrainEntry e{};
+  walk_team_f32<TEAM>(
+      c.order, start, end, c.N, c.prims, t.valid, t.ro.x, t.ro.y, t.ro.z, t.rd.x, t.rd.y, t.rd.z, c.thr, s.walk, k, l,
+      [&]() { return t.valid && (trans >= kTransmittanceFloor) && (used < c.max_hits); },
+      [&](int p, bool hit, const HitInfo& h, unsigned long long mask, int buf) {
+        p_mine = p;
+        e = train_entry<T, REC>(c, t, p, hit, h, mask, l, s.dir, lane_bad, mlp_bad);
+        s.pay[buf][k][0][l] = e.alpha;
+        s.pay[buf][k][1][l] = e.R;
+        s.pay[buf][k][2][l] = e.G;
+        s.pay[buf][k][3][l] = e.B;
+      },
+      [&](const unsigned long long* masks, int, int buf) {
+        int kept = 0, mine = -1;
+        float before = 0.f;
+        bool hit_mine = false;
+#pragma unroll
+        for (int i = 0; i < TEAM; ++i) {
+          const unsigned long long m = masks[i];
+          const unsigned long long um = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m) |
+                                        ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32);
+          if (um == 0ull) continue;
+          const bool hit = ((um >> l) & 1ull) && (trans >= kTransmittanceFloor) && (used < c.max_hits);
+          if (__ballot(hit) == 0ull) continue;           // (behind the last entry that counts)
+          const float alpha = s.pay[buf][i][0][l];
+          if (i == k) {
+            mine = kept;
+            before = trans;
+            hit_mine = hit;
+          }
+          ++kept;
+          if (hit) {
+            if (k == 0) {
+              const float weight = trans * alpha;
+              cr = fmaf(weight, s.pay[buf][i][1][l], cr);
+              cg = fmaf(weight, s.pay[buf][i][2][l], cg);
+              cb = fmaf(weight, s.pay[buf][i][3][l], cb);
+            }
+            trans = trans * (1.f - alpha);
+            ++used;
+            if constexpr (CHECKED) bad |= train_not_finite(trans);
+          }
+          over |= t.valid && (trans >= kTransmittanceFloor) && (used >= c.max_hits);
+        }
+        if constexpr (CHECKED) bad |= (hit_mine && lane_bad) || (mine >= 0 && mlp_bad);
+        const int slot = team_slot<kStepGrab, false>(slots, kept, mine, k, l, sp.head, sp.chunk_table, sp.pool_chunks, s.chunk);
+        train_store(sp, slot, l, p_mine, hit_mine, before, e);
+        return __ballot(t.valid && (trans >= kTransmittanceFloor)) != 0ull;
+      });
+  if constexpr (CHECKED) bad |= train_not_finite((cr + cg) + cb);
+  if (k == 0 && l == 0) sp.tile_steps[tile] = slots.count;
+  train_status(sp, over, bad, l);
+  if (k == 0 && t.valid) {
+    store3(out.rgb, t.pix, cr, cg, cb);
+    out.alpha[t.pix] = 1.f - trans;
+  }
 }
 
+// A wavefront per tile, four tiles to a workgroup, but for the last ones: the workgroups from `body` on (per XCD) take a tile
+// each, as a team.
+constexpr int kTrainTeam = 4;
+template <typename T, bool REC>
+__device__ __forceinline__ void train_forward_body(const TrainScene& c, const StepPool& sp, const TrainOut& out, int body) {
+  union Lds {
+    TrainItemLds<T> item[kTrainTeam];
+    TrainTeamLds<T, kTrainTeam> team;
+  };
+  __shared__ Lds s;
+  const int unit = (int)(blockIdx.x / kNumXcd), xcd = (int)(blockIdx.x % kNumXcd);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = (int)threadIdx.x & 63;
+  const bool alone = unit < body;
+  const int tile = superblock_tile_of(xcd, alone ? unit * kTrainTeam + wave : body * kTrainTeam + (unit - body), c.ntx, c.nty);
+  if (tile < 0) return;
+  if (alone) train_tile<T, REC>(tile, l, s.item[wave], c, sp, out);
+  else train_tile_team<T, REC, kTrainTeam>(tile, wave, l, s.team, c, sp, out);
+}
+// (The kernels take their pointers one by one, __restrict__: as members of an argument structure the output layer's weights,
+// the same for all lanes, would be read through the vector memory path behind the stores of the steps.)
+#define MLPSP_TRAIN_PARAMS                                                                                             \
+  const float *__restrict__ rays_o, const float *__restrict__ rays_d, const PrimRecord *__restrict__ prims,             \
+      const int32_t *__restrict__ order, const int32_t *__restrict__ offsets, const float *__restrict__ freq,           \
+      const float *__restrict__ att
+#define MLPSP_TRAIN_TAIL int N, int W, int H, int ntx, int nty, float thr, int max_hits, StepPool sp, TrainOut out, int body
+template <bool REC>
+__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(3, 3))) void train_forward_f32_kernel(
+    MLPSP_TRAIN_PARAMS, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
+    const float* __restrict__ b2, const float* __restrict__ W3, const float* __restrict__ b3, MLPSP_TRAIN_TAIL) {
+  const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, nullptr, N, W, H, ntx, nty, thr, max_hits};
+  train_forward_body<float, REC>(c, sp, out, body);
+}
 template <typename T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_mfma_kernel(
-    const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
-    const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
-    const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx, int nty, float thr,
-    int max_hits, StepPool sp, TrainOut out) {
-  __shared__ TrainLds<T> s;
-  __shared__ WalkLds s_walk;
-  train_forward_body<T, false>(rays_o, rays_d, prims, order, offsets, freq, att, nullptr, nullptr, nullptr, nullptr, nullptr,
-                               nullptr, packed, N, W, H, ntx, nty, thr, max_hits, sp, out, s, s_walk);
+__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_mfma_kernel(
+    MLPSP_TRAIN_PARAMS, const unsigned char* __restrict__ packed, MLPSP_TRAIN_TAIL) {
+  const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, packed,
+                     N, W, H, ntx, nty, thr, max_hits};
+  train_forward_body<T, false>(c, sp, out, body);
+}
+#undef MLPSP_TRAIN_PARAMS
+#undef MLPSP_TRAIN_TAIL
+// As many teams at the end as there are workgroups on the chip; all tiles where they are hardly more.
+struct TrainPlan {
+  int body;
+  unsigned grid;
+};
+inline TrainPlan train_plan(int ntx, int nty, int64_t T) {
+  const int per_xcd = (int)(superblock_grid(ntx, nty) / kNumXcd);
+  const int teams = T <= 1280 ? per_xcd : min(per_xcd, 1024 / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
+  return TrainPlan{body, (unsigned)(kNumXcd * (body + per_xcd - kTrainTeam * body))};
 }
 
 // tile_base = exclusive sums of tile_steps, head[2] = their total; one workgroup (12,750 tiles: 6 us).
@@ -235,12 +394,12 @@ MLPSP_API int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays
   if (((uintptr_t)W1 | (uintptr_t)b1 | (uintptr_t)W2 | (uintptr_t)b2) & 15u) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(hipMemsetAsync(f.sp.head, 0, 64 * sizeof(int32_t), s));
-  const dim3 grid(superblock_grid(f.ntx, f.nty)), block(64);
-#define MLPSP_TRAIN_LAUNCH(REC)                                                                                       \
-  hipLaunchKernelGGL((train_forward_f32_kernel<REC>), grid, block, 0, s, rays_o_dev, rays_d_dev,                      \
-                     (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, b2, \
-                     W3, b3, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp,                    \
-                     TrainOut{out_rgb_dev, out_alpha_dev})
+  const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
+#define MLPSP_TRAIN_LAUNCH(REC)                                                                                        \
+  hipLaunchKernelGGL(train_forward_f32_kernel<REC>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \
+                     (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, b2,  \
+                     W3, b3, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp,                      \
+                     TrainOut{out_rgb_dev, out_alpha_dev}, plan.body)
   if (render_order) MLPSP_TRAIN_LAUNCH(false);
   else MLPSP_TRAIN_LAUNCH(true);
 #undef MLPSP_TRAIN_LAUNCH
@@ -264,12 +423,12 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
   if (((uintptr_t)prim_records_dev % 128) != 0 || ((uintptr_t)packed_dev % 16) != 0) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(hipMemsetAsync(f.sp.head, 0, 64 * sizeof(int32_t), s));
-  const dim3 grid(superblock_grid(f.ntx, f.nty)), block(64);
-#define MLPSP_TRAIN_LAUNCH(T)                                                                                         \
-  hipLaunchKernelGGL((train_forward_mfma_kernel<T>), grid, block, 0, s, rays_o_dev, rays_d_dev,                       \
-                     (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,              \
-                     (const unsigned char*)packed_dev, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, \
-                     f.sp, TrainOut{out_rgb_dev, out_alpha_dev})
+  const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
+#define MLPSP_TRAIN_LAUNCH(T)                                                                                          \
+  hipLaunchKernelGGL(train_forward_mfma_kernel<T>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \
+                     (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,                \
+                     (const unsigned char*)packed_dev, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp, \
+                     TrainOut{out_rgb_dev, out_alpha_dev}, plan.body)
   if (use_bf16) MLPSP_TRAIN_LAUNCH(__bf16);
   else MLPSP_TRAIN_LAUNCH(_Float16);
 #undef MLPSP_TRAIN_LAUNCH
