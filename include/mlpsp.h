@@ -76,6 +76,12 @@ int mlpsp_prepare_primitives(const float* positions_dev, const float* log_scales
  * launch.  rays_d_dev, unit_dirs_dev: num_rays x 3 floats, contiguous; they may be the same buffer. */
 int mlpsp_normalize_rays(const float* rays_d_dev, long long num_rays, float* unit_dirs_dev, mlpsp_stream_t stream);
 
+/* quats / max(|quats|, 1e-12) per row of four, the bits of torch.nn.functional.normalize(quats, dim=-1), and the gradient of
+ * that with respect to quats from the adjoint of the unit quaternions.  16-byte aligned arrays of num_quats x 4 floats. */
+int mlpsp_normalize_quats(const float* quats_dev, int64_t num_quats, float* unit_quats_dev, mlpsp_stream_t stream);
+int mlpsp_normalize_quats_backward(const float* quats_dev, const float* grad_unit_dev, int64_t num_quats,
+                                   float* grad_quats_dev, mlpsp_stream_t stream);
+
 /* Tile-list validation = validate_tile_candidate_capacity (np_tile_kernels.cu:4485-4589).
  * capacity 0 = no cap (per-pixel and presorted entry points).  status_dev: 2 int32 of device
  * scratch.  BLOCKS: one 8-byte device-to-host copy, then returns the status mask;
@@ -538,11 +544,10 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  *   2 = a live pixel reached max_hits), steps}.
  *   If 16 times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
  *   the caller repeats the call with a pool of that size.
- * mlpsp_train_list_steps: primitive, pool slot and tile of every step, in tile order (num_steps = the third word).
  * mlpsp_train_reverse: reverse compositing; d4_dev [num_steps, 64, 4] = adjoints of the four pre-activation outputs,
  *   falloff_dev [num_steps, 64] = dL/d(decay) * decay.
- * mlpsp_train_group: sorted_prim_dev / permutation_dev (int64) = the stable sort of step_prim_dev; fills the index part of
- *   scratch_dev (mlpsp_train_scratch_bytes(num_steps, num_primitives) bytes, 256-byte aligned).
+ * mlpsp_train_group: the steps (num_steps = the third word) sorted by primitive, into the index part of scratch_dev
+ *   (mlpsp_train_scratch_bytes(num_steps, num_primitives) bytes, 256-byte aligned; all of it is scratch of the call).
  * mlpsp_train_gradients: the nine gradients, written whole, from a scratch_dev that mlpsp_train_group has filled.
  *   precision, scale: as mlpsp_grouped_vjp; nonfinite_dev[0] becomes 1 if a weight gradient is not finite.
  *
@@ -564,17 +569,14 @@ int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, c
                              const float* freq_dev, const float* att_dev, const void* packed_dev, int num_primitives,
                              int width, int height, float threshold, int max_hits, int use_bf16, void* workspace_dev,
                              size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev, mlpsp_stream_t stream);
-int mlpsp_train_list_steps(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
-                           const void* workspace_dev, size_t workspace_bytes, int32_t* step_prim_dev,
-                           int32_t* step_slot_dev, int32_t* step_tile_dev, mlpsp_stream_t stream);
 int mlpsp_train_reverse(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
                         const void* workspace_dev, size_t workspace_bytes, const float* grad_rgb_dev,
                         const float* grad_t_dev, float* d4_dev, float* falloff_dev, mlpsp_stream_t stream);
 size_t mlpsp_train_scratch_bytes(int64_t num_steps, int num_primitives);
-int mlpsp_train_group(const int32_t* sorted_prim_dev, const int64_t* permutation_dev, const int32_t* step_slot_dev,
-                      const int32_t* step_tile_dev, int64_t num_steps, int num_primitives, int width, void* scratch_dev,
+int mlpsp_train_group(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height, const void* workspace_dev,
+                      size_t workspace_bytes, int64_t num_steps, int num_primitives, void* scratch_dev,
                       size_t scratch_bytes, mlpsp_stream_t stream);
-int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int64_t num_pairs, int width, int height,
+int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int width, int height,
                           const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,
                           const float* falloff_dev, const float* rays_d_dev, const float* freq_dev,
                           const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2,
@@ -592,7 +594,7 @@ int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t num_pairs, i
                            int target_is_half, int target_width, int target_height, int channels, int slots, float beta,
                            float temp, void* kept_dev, size_t kept_bytes, float* shares_dev, float* loss_partials_dev,
                            mlpsp_stream_t stream);
-int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int width, int height,
+int mlpsp_train_feature_gradients(int64_t num_steps, int width, int height,
                                   int target_width, int target_height, int channels, int slots, const void* kept_dev,
                                   size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes, int num_primitives,
                                   const float* loss_adjoint_dev, float* rows_dev, float* out_dev, mlpsp_stream_t stream);

@@ -96,17 +96,18 @@ SIGNATURES = {
     "mlpsp_records_reverse_adjoints": (_i, [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "mlpsp_geometry_gradients": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _i, _vp, _vp, _vp, _vp,
                                       _vp]),
+    "mlpsp_normalize_quats": (_i, [_vp, _i64, _vp, _vp]),
+    "mlpsp_normalize_quats_backward": (_i, [_vp, _vp, _i64, _vp, _vp]),
     "mlpsp_train_workspace_bytes": (_sz, [_i64, _i, _i, _i64]),
     "mlpsp_train_forward_f32": (_i, [_vp] * 5 + [_i64] + [_vp] * 8 + [_i, _i, _i, _f, _i, _i, _vp, _sz, _vp, _vp, _vp]),
     "mlpsp_train_forward_mfma": (_i, [_vp] * 5 + [_i64] + [_vp] * 3 + [_i, _i, _i, _f, _i, _i, _vp, _sz, _vp, _vp, _vp]),
-    "mlpsp_train_list_steps": (_i, [_vp, _i64, _i, _i, _vp, _sz, _vp, _vp, _vp, _vp]),
     "mlpsp_train_reverse": (_i, [_vp, _i64, _i, _i, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "mlpsp_train_scratch_bytes": (_sz, [_i64, _i]),
-    "mlpsp_train_group": (_i, [_vp, _vp, _vp, _vp, _i64, _i, _i, _vp, _sz, _vp]),
-    "mlpsp_train_gradients": (_i, [_vp, _i64, _i64, _i, _i, _vp, _sz] + [_vp] * 12 + [_i, _i, _f, _vp, _sz] + [_vp] * 11),
+    "mlpsp_train_group": (_i, [_vp, _i64, _i, _i, _vp, _sz, _i64, _i, _vp, _sz, _vp]),
+    "mlpsp_train_gradients": (_i, [_i64, _i64, _i, _i, _vp, _sz] + [_vp] * 12 + [_i, _i, _f, _vp, _sz] + [_vp] * 11),
     "mlpsp_train_feature_bytes": (_sz, [_i] * 6 + [_i64, _vp, _vp, _vp]),
     "mlpsp_train_feature_l1": (_i, [_vp, _i64, _i, _i, _vp, _sz, _i64, _vp, _vp, _vp] + [_i] * 5 + [_f, _f, _vp, _sz, _vp, _vp, _vp]),
-    "mlpsp_train_feature_gradients": (_i, [_vp, _i64] + [_i] * 6 + [_vp, _sz, _vp, _sz, _i] + [_vp] * 4),
+    "mlpsp_train_feature_gradients": (_i, [_i64] + [_i] * 6 + [_vp, _sz, _vp, _sz, _i] + [_vp] * 4),
     "mlpsp_records_reverse": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _vp, _vp, _vp, _vp, _vp]),
 }
 

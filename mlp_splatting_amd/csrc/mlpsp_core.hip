@@ -94,6 +94,34 @@ __global__ __launch_bounds__(256) void normalize_rays_kernel(const float* __rest
   store3(out, i, ux, uy, uz);
 }
 
+// q / max(|q|, 1e-12) per quaternion, as torch.nn.functional.normalize(quats, dim=-1) rounds it on this device (the squares
+// summed in pairs), and its gradient (g - u (u.g)) / |q| with u the unit quaternion.  One launch each in place of the
+// library's three and twelve, a twentieth of a small training step between them.
+__device__ __forceinline__ float quat_norm(const float4& q) {
+  return sqrtf((q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w));
+}
+__global__ __launch_bounds__(256) void normalize_quats_kernel(const float4* __restrict__ q, long long n, float4* __restrict__ out) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float4 v = q[i];
+  const float norm = quat_norm(v), den = norm < 1e-12f ? 1e-12f : norm;
+  out[i] = make_float4(v.x / den, v.y / den, v.z / den, v.w / den);
+}
+__global__ __launch_bounds__(256) void normalize_quats_backward_kernel(const float4* __restrict__ q, const float4* __restrict__ g,
+                                                                       long long n, float4* __restrict__ out) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const float4 v = q[i], d = g[i];
+  const float norm = quat_norm(v);
+  if (norm < 1e-12f) {          // the norm is a constant there
+    out[i] = make_float4(d.x / 1e-12f, d.y / 1e-12f, d.z / 1e-12f, d.w / 1e-12f);
+    return;
+  }
+  const float4 u = make_float4(v.x / norm, v.y / norm, v.z / norm, v.w / norm);
+  const float along = (u.x * d.x + u.y * d.y) + (u.z * d.z + u.w * d.w);
+  out[i] = make_float4((d.x - u.x * along) / norm, (d.y - u.y * along) / norm, (d.z - u.z * along) / norm, (d.w - u.w * along) / norm);
+}
+
 // The per-frame preparations that depend on nothing but the rays (and the scene), in one launch: blocks
 // [0, ray_blocks) write the unit directions (normalize_rays_kernel's statements), the next tile_blocks blocks the
 // tiles' ray pyramids for the sort (a wavefront per tile, from the directions as given: it does not wait for the unit
@@ -181,6 +209,30 @@ MLPSP_API int mlpsp_normalize_rays(const float* rays_d_dev, long long num_rays, 
   if (num_rays > 2147483647LL * 256) return MLPSP_E_ARGUMENT;
   hipLaunchKernelGGL(normalize_rays_kernel, dim3((unsigned)((num_rays + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                      rays_d_dev, num_rays, unit_dirs_dev);
+  MLPSP_LAUNCH_CHECK();
+  return MLPSP_OK;
+}
+
+MLPSP_API int mlpsp_normalize_quats(const float* quats_dev, int64_t num_quats, float* unit_quats_dev, mlpsp_stream_t stream) {
+  if (num_quats < 0 || num_quats > 2147483647LL * 256) return MLPSP_E_ARGUMENT;
+  if (num_quats == 0) return MLPSP_OK;
+  if (!quats_dev || !unit_quats_dev || (((uintptr_t)quats_dev | (uintptr_t)unit_quats_dev) & 15u)) return MLPSP_E_ARGUMENT;
+  hipLaunchKernelGGL(normalize_quats_kernel, dim3((unsigned)((num_quats + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                     (const float4*)quats_dev, (long long)num_quats, (float4*)unit_quats_dev);
+  MLPSP_LAUNCH_CHECK();
+  return MLPSP_OK;
+}
+
+MLPSP_API int mlpsp_normalize_quats_backward(const float* quats_dev, const float* grad_unit_dev, int64_t num_quats,
+                                             float* grad_quats_dev, mlpsp_stream_t stream) {
+  if (num_quats < 0 || num_quats > 2147483647LL * 256) return MLPSP_E_ARGUMENT;
+  if (num_quats == 0) return MLPSP_OK;
+  if (!quats_dev || !grad_unit_dev || !grad_quats_dev ||
+      (((uintptr_t)quats_dev | (uintptr_t)grad_unit_dev | (uintptr_t)grad_quats_dev) & 15u))
+    return MLPSP_E_ARGUMENT;
+  hipLaunchKernelGGL(normalize_quats_backward_kernel, dim3((unsigned)((num_quats + 255) / 256)), dim3(256), 0,
+                     (hipStream_t)stream, (const float4*)quats_dev, (const float4*)grad_unit_dev, (long long)num_quats,
+                     (float4*)grad_quats_dev);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }

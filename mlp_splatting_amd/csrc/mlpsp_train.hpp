@@ -70,11 +70,11 @@ inline StepPool step_pool_carve(void* workspace, size_t bytes, int64_t num_pairs
   return sp;
 }
 
-// The steps sorted by primitive: first sorted position of every primitive [N + 1]; of the sorted steps [S] pool slot,
-// number in tile order, tile and pixel number of the tile's first pixel -- one 16-byte read.  Every buffer that holds them
-// begins with them.
+// The steps sorted by primitive: first sorted position of every primitive [N + 1]; of the sorted steps [S] the primitive, and
+// pool slot, number in tile order, tile and pixel number of the tile's first pixel -- one 16-byte read.  Every buffer that
+// holds them begins with them.
 struct StepSort {
-  int32_t* first;
+  int32_t *first, *prim;
   int4* step;
   size_t bytes;
 };
@@ -83,6 +83,8 @@ inline StepSort step_sort(void* base, int64_t S, int N) {
   unsigned char* p = (unsigned char*)base;
   t.first = (int32_t*)p;
   p += step_align(((size_t)N + 1) * 4);
+  t.prim = (int32_t*)p;
+  p += step_align((size_t)S * 4);
   t.step = (int4*)p;
   p += step_align((size_t)S * 16);
   t.bytes = (size_t)(p - (unsigned char*)base);

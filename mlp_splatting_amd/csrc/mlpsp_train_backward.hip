@@ -2,8 +2,7 @@
 // and MLP weight gradients per primitive.  Counterpart of the reference's reverse walk (primitive_records.cuh:3-46) and
 // grouped gradient kernels (scannet/primitive_gemm.py:101-183) in one pipeline whose unit is a step, not a record.
 //
-// The steps are sorted by primitive (by the caller: a stable sort of S keys, S = 0.65 M at the 200,000-primitive
-// 1200x680 frame) and cut into chunks of equal length.  A wavefront walks one chunk; where the primitive changes it
+// The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal length.  A wavefront walks one chunk; where the primitive changes it
 // writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
 // (the primitive goes on in the next chunk) or head row (it ended here).  Two more launches add the rows of the primitives
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
@@ -68,33 +67,147 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// steps grouped by primitive
+// steps sorted by primitive: a stable radix sort of the S primitive numbers in tile order, in digits of equal width (two of
+// nine bits at 200,000 primitives).  A wavefront takes an eighth of its block's steps in rounds of 64, whose equal digits are
+// found with a ballot per bit.  Eight launches, 75 us at 650,000 steps; the library's sort took 22 launches and 200 us with
+// the gather behind it.
 // ---------------------------------------------------------------------------------------------
-struct StepIndex {
-  const int32_t* prim;    // [S] sorted
-  const int32_t* first;   // [N + 1] first sorted position of every primitive
-  const int4* step;       // [S] pool slot, number in tile order, tile, first pixel of the tile
-};
+constexpr int kSortBlock = 512, kSortBits = 10;
+// Steps of a block: 8,192, a quarter of that where this would leave a chip of 256 CUs fewer than 32 blocks (16 rounds one
+// after the other took 33 us at 80,000 steps); the sums over blocks x digits grow with the blocks.
+inline int sort_keys(int64_t S) { return S >= 32 * 8192 ? 8192 : 2048; }
 
-__global__ __launch_bounds__(256) void step_group_kernel(const int32_t* __restrict__ prim, const long long* __restrict__ perm,
-                                                         const int32_t* __restrict__ step_slot_of,
-                                                         const int32_t* __restrict__ step_tile, int S, int N, int W, int ntx,
-                                                         int32_t* __restrict__ first, int4* __restrict__ step) {
-  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (i < S) {
-    const int o = (int)perm[i], tile = step_tile[o];
-    step[i] = make_int4(step_slot_of[o], o, tile, (tile / ntx) * 8 * W + (tile % ntx) * 8);
-  }
-  if (i <= N) {
-    int lo = 0, hi = S;        // first position whose key is >= i
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (prim[mid] < i) lo = mid + 1;
-      else hi = mid;
-    }
-    first[i] = lo;
+// keys and particulars of the steps in tile order
+__global__ __launch_bounds__(256) void step_list_kernel(const int32_t* __restrict__ offsets, const int32_t* __restrict__ tile_base,
+                                                        const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ ids,
+                                                        int T, int W, int ntx, int32_t* __restrict__ keys, int4* __restrict__ info) {
+  const int tile = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  if (tile >= T) return;
+  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = (offsets[tile] >> 4) + tile;
+  const int pixel = (tile / ntx) * 8 * W + (tile % ntx) * 8;
+  for (int m = lane; m < count; m += 64) {
+    const int slot = step_slot(chunk_table, table, m);
+    keys[base + m] = ids[slot];
+    info[base + m] = make_int4(slot, base + m, tile, pixel);
   }
 }
+
+__global__ __launch_bounds__(kSortBlock) void step_hist_kernel(const int32_t* __restrict__ keys, int S, int share, int shift,
+                                                               int bits, int blocks, int32_t* __restrict__ hist) {
+  __shared__ int s_count[1 << kSortBits];
+  const int R = 1 << bits;
+  for (int d = threadIdx.x; d < R; d += kSortBlock) s_count[d] = 0;
+  __syncthreads();
+  const int end = min(S, (int)(blockIdx.x + 1) * share);
+  for (int i = (int)blockIdx.x * share + threadIdx.x; i < end; i += kSortBlock)
+    atomicAdd(&s_count[(keys[i] >> shift) & (R - 1)], 1);
+  __syncthreads();
+  for (int d = threadIdx.x; d < R; d += kSortBlock) hist[d * blocks + blockIdx.x] = s_count[d];
+}
+
+// exclusive sums of n counts, in place; one workgroup
+__global__ __launch_bounds__(1024) void step_sums_kernel(int32_t* __restrict__ v, int n) {
+  __shared__ int s_wave[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int carry = 0;
+  for (int base = 0; base < n; base += 4096) {
+    const int i = base + 4 * t;
+    int x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = i + k < n ? v[i + k] : 0;
+    const int mine = (x[0] + x[1]) + (x[2] + x[3]);
+    int incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(incl, d);
+      if (lane >= d) incl += u;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    int before = carry, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      before += w < wave ? s_wave[w] : 0;
+      total += s_wave[w];
+    }
+    carry += total;
+    int run = before + incl - mine;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (i + k < n) v[i + k] = run;
+      run += x[k];
+    }
+    __syncthreads();
+  }
+}
+
+// order: numbers of the keys (null: their places).  The last digit's pass writes the sorted primitives and particulars.
+template <bool LAST>
+__global__ __launch_bounds__(kSortBlock) void step_scatter_kernel(const int32_t* __restrict__ keys, const int32_t* __restrict__ order,
+                                                                  int S, int share, int shift, int bits, int blocks,
+                                                                  const int32_t* __restrict__ sums, const int4* __restrict__ info,
+                                                                  int32_t* __restrict__ out_keys, int32_t* __restrict__ out_order,
+                                                                  int4* __restrict__ out_step) {
+  constexpr int kWaves = kSortBlock / 64;
+  __shared__ int s_at[kWaves][1 << kSortBits];
+  const int R = 1 << bits, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int d = threadIdx.x; d < R; d += kSortBlock) {
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s_at[w][d] = 0;
+  }
+  __syncthreads();
+  const int begin = (int)blockIdx.x * share + wave * (share / kWaves), end = min(S, begin + share / kWaves);
+  for (int i = begin + lane; i < end; i += 64) atomicAdd(&s_at[wave][(keys[i] >> shift) & (R - 1)], 1);
+  __syncthreads();
+  for (int d = threadIdx.x; d < R; d += kSortBlock) {
+    int run = sums[d * blocks + blockIdx.x];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int c = s_at[w][d];
+      s_at[w][d] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+  for (int base = begin; base < end; base += 64) {
+    const int i = base + lane;
+    const bool valid = i < end;
+    const int key = valid ? keys[i] : 0, digit = (key >> shift) & (R - 1);
+    unsigned long long same = __ballot(valid);
+    for (int b = 0; b < bits; ++b) {
+      const bool set = (digit >> b) & 1;
+      const unsigned long long m = __ballot(set);
+      same &= set ? m : ~m;
+    }
+    if (!valid) continue;
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    const int at = s_at[wave][digit] + rank;
+    if (rank == 0) s_at[wave][digit] = at + (int)__popcll(same);
+    const int number = order ? order[i] : i;
+    out_keys[at] = key;
+    if constexpr (LAST) out_step[at] = info[number];
+    else out_order[at] = number;
+  }
+}
+
+// first[p] = first sorted position whose primitive is >= p
+__global__ __launch_bounds__(256) void step_first_kernel(const int32_t* __restrict__ prim, int S, int N, int32_t* __restrict__ first) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i > N) return;
+  int lo = 0, hi = S;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (prim[mid] < i) lo = mid + 1;
+    else hi = mid;
+  }
+  first[i] = lo;
+}
+
+struct StepIndex {
+  const int32_t* prim;    // of StepSort
+  const int32_t* first;
+  const int4* step;
+};
 
 constexpr int kGeoFloats = 16;                            // 15 geometry sums, one pad
 constexpr int kRowFloats = kGradFloats + kGeoFloats;      // of a head or tail row
@@ -642,22 +755,65 @@ MLPSP_API size_t mlpsp_train_scratch_bytes(int64_t num_steps, int num_primitives
   return train_scratch(nullptr, num_steps, num_primitives).bytes;
 }
 
-MLPSP_API int mlpsp_train_group(const int32_t* sorted_prim_dev, const int64_t* permutation_dev, const int32_t* step_slot_dev,
-                                const int32_t* step_tile_dev, int64_t num_steps, int num_primitives, int width,
+MLPSP_API int mlpsp_train_group(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
+                                const void* workspace_dev, size_t workspace_bytes, int64_t num_steps, int num_primitives,
                                 void* scratch_dev, size_t scratch_bytes, mlpsp_stream_t stream) {
-  if (width <= 0 || num_steps < 0 || num_steps > 2147483647LL || num_primitives < 0) return MLPSP_E_ARGUMENT;
-  if (num_steps > 0 && (!sorted_prim_dev || !permutation_dev || !step_slot_dev || !step_tile_dev)) return MLPSP_E_ARGUMENT;
+  const int64_t T = checked_num_tiles(width, height, 8, 8);
+  if (T <= 0 || T > 2147483647LL - 8 || num_pairs < 0 || num_pairs > 2147483647LL || num_steps < 0 ||
+      num_steps > 2147483647LL - 8192 || num_primitives < 0 || !tile_offsets_dev)
+    return MLPSP_E_ARGUMENT;
+  if (!workspace_dev || workspace_bytes < step_tables_bytes(num_pairs, T)) return MLPSP_E_SCRATCH;
   const TrainScratch t = train_scratch(scratch_dev, num_steps, num_primitives);
   if (!scratch_dev || reinterpret_cast<uintptr_t>(scratch_dev) % 256 != 0 || scratch_bytes < t.bytes) return MLPSP_E_SCRATCH;
-  const int64_t items = num_steps > (int64_t)num_primitives + 1 ? num_steps : (int64_t)num_primitives + 1;
-  hipLaunchKernelGGL(step_group_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                     sorted_prim_dev, (const long long*)permutation_dev, step_slot_dev, step_tile_dev, (int)num_steps,
-                     num_primitives, width, ceil_div(width, 8), t.first, t.step);
+  const StepPool sp = step_pool_carve(const_cast<void*>(workspace_dev), workspace_bytes, num_pairs, T);
+  hipStream_t s = (hipStream_t)stream;
+  const int S = (int)num_steps;
+  if (S > 0) {
+    int bits = 1;
+    while (bits < 31 && (1 << bits) < num_primitives) ++bits;
+    const int passes = (bits + kSortBits - 1) / kSortBits, width_bits = (bits + passes - 1) / passes;
+    const int share = sort_keys(S), blocks = (S + share - 1) / share;
+    // (the rows are written after the sort: its buffers lie there)
+    unsigned char* p = (unsigned char*)t.rows;
+    int4* info = (int4*)p;
+    p += step_align((size_t)S * 16);
+    int32_t *keys[2], *order[2];
+    for (int k = 0; k < 2; ++k) {
+      keys[k] = (int32_t*)p;
+      p += step_align((size_t)S * 4);
+      order[k] = (int32_t*)p;
+      p += step_align((size_t)S * 4);
+    }
+    int32_t* hist = (int32_t*)p;
+    p += (size_t)blocks * (1 << width_bits) * 4;
+    if ((size_t)(p - (unsigned char*)scratch_dev) > t.bytes) return MLPSP_E_SCRATCH;      // (cannot be: 4 KB of rows per step)
+    hipLaunchKernelGGL(step_list_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, tile_offsets_dev, sp.tile_base,
+                       sp.chunk_table, sp.ids, (int)T, width, ceil_div(width, 8), keys[0], info);
+    MLPSP_LAUNCH_CHECK();
+    for (int pass = 0; pass < passes; ++pass) {
+      const int32_t *in = keys[pass & 1], *numbers = pass == 0 ? nullptr : order[pass & 1];
+      hipLaunchKernelGGL(step_hist_kernel, dim3((unsigned)blocks), dim3(kSortBlock), 0, s, in, S, share, pass * width_bits,
+                         width_bits, blocks, hist);
+      MLPSP_LAUNCH_CHECK();
+      hipLaunchKernelGGL(step_sums_kernel, dim3(1), dim3(1024), 0, s, hist, blocks << width_bits);
+      MLPSP_LAUNCH_CHECK();
+      if (pass + 1 == passes)
+        hipLaunchKernelGGL(step_scatter_kernel<true>, dim3((unsigned)blocks), dim3(kSortBlock), 0, s, in, numbers, S, share,
+                           pass * width_bits, width_bits, blocks, hist, info, t.prim, (int32_t*)nullptr, t.step);
+      else
+        hipLaunchKernelGGL(step_scatter_kernel<false>, dim3((unsigned)blocks), dim3(kSortBlock), 0, s, in, numbers, S, share,
+                           pass * width_bits, width_bits, blocks, hist, info, keys[(pass + 1) & 1], order[(pass + 1) & 1],
+                           (int4*)nullptr);
+      MLPSP_LAUNCH_CHECK();
+    }
+  }
+  hipLaunchKernelGGL(step_first_kernel, dim3((unsigned)((num_primitives + 256) / 256)), dim3(256), 0, s, t.prim, S, num_primitives,
+                     t.first);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }
 
-MLPSP_API int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int64_t num_pairs, int width,
+MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int width,
                                     int height, const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,
                                     const float* falloff_dev, const float* rays_d_dev, const float* freq_dev,
                                     const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2,
@@ -675,7 +831,7 @@ MLPSP_API int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_
   if (!scratch_dev || reinterpret_cast<uintptr_t>(scratch_dev) % 256 != 0 || scratch_bytes < t.bytes) return MLPSP_E_SCRATCH;
   if (!rays_d_dev || !freq_dev || !att_dev || !W1 || !b1 || !W2 || !b2 || !W3 || !log_scales_dev || !quats_dev || !gW1_dev ||
       !gb1_dev || !gW2_dev || !gb2_dev || !gW3_dev || !gb3_dev || !grad_positions_dev || !grad_log_scales_dev ||
-      !grad_quats_dev || !nonfinite_dev || (num_steps > 0 && (!sorted_prim_dev || !d4_dev || !falloff_dev)))
+      !grad_quats_dev || !nonfinite_dev || (num_steps > 0 && (!d4_dev || !falloff_dev)))
     return MLPSP_E_ARGUMENT;
   if (((uintptr_t)W1 | (uintptr_t)b1 | (uintptr_t)W2 | (uintptr_t)b2 | (uintptr_t)d4_dev | (uintptr_t)gW1_dev |
        (uintptr_t)gb1_dev | (uintptr_t)gW2_dev | (uintptr_t)gb2_dev | (uintptr_t)gW3_dev | (uintptr_t)gb3_dev) & 15u)
@@ -683,7 +839,7 @@ MLPSP_API int mlpsp_train_gradients(const int32_t* sorted_prim_dev, int64_t num_
   const StepPool sp = step_pool_carve(const_cast<void*>(workspace_dev), workspace_bytes, num_pairs, T);
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(hipMemsetAsync(nonfinite_dev, 0, sizeof(int32_t), s));
-  const StepIndex ix{sorted_prim_dev, t.first, t.step};
+  const StepIndex ix{t.prim, t.first, t.step};
   const GradRows grads{gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
   const GeoGrads geo{grad_positions_dev, grad_log_scales_dev, grad_quats_dev};
   const int S = (int)num_steps;

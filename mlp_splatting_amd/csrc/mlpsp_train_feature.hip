@@ -472,7 +472,7 @@ MLPSP_API int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t nu
   return MLPSP_OK;
 }
 
-MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int64_t num_steps, int width, int height,
+MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int height,
                                             int target_width, int target_height, int channels, int slots,
                                             const void* kept_dev, size_t kept_bytes, const void* scratch_dev,
                                             size_t scratch_bytes, int num_primitives, const float* loss_adjoint_dev,
@@ -486,7 +486,7 @@ MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int6
   const StepSort t = step_sort(const_cast<void*>(scratch_dev), num_steps, num_primitives);
   if (!scratch_dev || scratch_bytes < t.bytes) return MLPSP_E_SCRATCH;
   if (num_primitives == 0) return MLPSP_OK;
-  if (!loss_adjoint_dev || !out_dev || (num_steps > 0 && (!sorted_prim_dev || !rows_dev || ((uintptr_t)rows_dev & 15u))))
+  if (!loss_adjoint_dev || !out_dev || (num_steps > 0 && (!rows_dev || ((uintptr_t)rows_dev & 15u))))
     return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   const bool vec = channels % 4 == 0 && ((uintptr_t)out_dev & 15u) == 0;
@@ -494,7 +494,7 @@ MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int6
   if (chunks > 0) {
     const dim3 grid((unsigned)ceil_div(chunks, 4), (unsigned)ceil_div(channels, 256));
 #define MLPSP_ATTR(SL, VEC)                                                                                              \
-  hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, sorted_prim_dev, t.first, t.step,         \
+  hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, t.prim, t.first, t.step,         \
                      (int)num_steps, per, chunks, lanes_per_row_log2(f.Cp), loss_adjoint_dev, rows_dev, out_dev)
     if (slots == 1) { if (vec) MLPSP_ATTR(1, true); else MLPSP_ATTR(1, false); }
     else if (slots == 4) { if (vec) MLPSP_ATTR(4, true); else MLPSP_ATTR(4, false); }
@@ -502,10 +502,10 @@ MLPSP_API int mlpsp_train_feature_gradients(const int32_t* sorted_prim_dev, int6
 #undef MLPSP_ATTR
     MLPSP_LAUNCH_CHECK();
     if (vec)
-      hipLaunchKernelGGL(train_attr_join_kernel<true>, dim3((unsigned)chunks), dim3(256), 0, s, f, sorted_prim_dev, t.first,
+      hipLaunchKernelGGL(train_attr_join_kernel<true>, dim3((unsigned)chunks), dim3(256), 0, s, f, t.prim, t.first,
                          (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
     else
-      hipLaunchKernelGGL(train_attr_join_kernel<false>, dim3((unsigned)chunks), dim3(256), 0, s, f, sorted_prim_dev, t.first,
+      hipLaunchKernelGGL(train_attr_join_kernel<false>, dim3((unsigned)chunks), dim3(256), 0, s, f, t.prim, t.first,
                          (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
     MLPSP_LAUNCH_CHECK();
   }

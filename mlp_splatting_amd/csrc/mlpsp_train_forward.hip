@@ -325,22 +325,6 @@ __global__ __launch_bounds__(1024) void step_scan_kernel(const int32_t* __restri
   }
 }
 
-// Steps in tile order: primitive, pool slot and tile of each.
-__global__ __launch_bounds__(256) void step_list_kernel(const int32_t* __restrict__ offsets, const int32_t* __restrict__ tile_base,
-                                                        const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ ids,
-                                                        int T, int32_t* __restrict__ step_prim,
-                                                        int32_t* __restrict__ step_slot_of, int32_t* __restrict__ step_tile) {
-  const int tile = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  if (tile >= T) return;
-  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = (offsets[tile] >> 4) + tile;
-  for (int m = lane; m < count; m += 64) {
-    const int slot = step_slot(chunk_table, table, m);
-    step_prim[base + m] = ids[slot];
-    step_slot_of[base + m] = slot;
-    step_tile[base + m] = tile;
-  }
-}
-
 }  // namespace mlpsp
 
 using namespace mlpsp;
@@ -434,17 +418,4 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
 #undef MLPSP_TRAIN_LAUNCH
   MLPSP_LAUNCH_CHECK();
   return train_scan(f, s);
-}
-
-MLPSP_API int mlpsp_train_list_steps(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
-                                     const void* workspace_dev, size_t workspace_bytes, int32_t* step_prim_dev,
-                                     int32_t* step_slot_dev, int32_t* step_tile_dev, mlpsp_stream_t stream) {
-  TrainFrame f;
-  const int rc = train_frame(width, height, num_pairs, const_cast<void*>(workspace_dev), workspace_bytes, f);
-  if (rc != MLPSP_OK) return rc;
-  if (!tile_offsets_dev || !step_prim_dev || !step_slot_dev || !step_tile_dev) return MLPSP_E_ARGUMENT;
-  hipLaunchKernelGGL(step_list_kernel, dim3((unsigned)((f.T + 3) / 4)), dim3(256), 0, (hipStream_t)stream, tile_offsets_dev,
-                     f.sp.tile_base, f.sp.chunk_table, f.sp.ids, (int)f.T, step_prim_dev, step_slot_dev, step_tile_dev);
-  MLPSP_LAUNCH_CHECK();
-  return MLPSP_OK;
 }

@@ -817,11 +817,19 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         if ext is not None and callable(getattr(ext, "invalidate_caches", None)):
             ext.invalidate_caches()
 
+    def _forget_parameters(self):
+        """:meth:`invalidate_render_caches` for a grad-mode forward: the frequency tables, which come from the encoder's
+        buffers and not from parameters, stay."""
+        tables = self.__dict__.get("_mlpsp_cache", {}).get("frequency_tables")
+        self.invalidate_render_caches()
+        if tables is not None:
+            self.__dict__["_mlpsp_cache"] = {"frequency_tables": tables}
+
     def _forward_csr_training(self, ray_o, ray_d, score_threshold, bg_color, view_matrix, proj_matrix,
                               culled_prim_indices, tile_offsets, return_feature, feature_target, device):
         """(rgb, streamed feature L1 loss) through the record-based training function
         (scannet/cumodel.py:1098-1108)."""
-        self.invalidate_render_caches()
+        self._forget_parameters()
         W, H = self.image_size
         ts = int(self.tile_size)
         use_tilecenter = self._resolve_tile_order_mode() == "tilecenter"
@@ -834,7 +842,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
                 ray_o, ray_d, score_threshold, view_matrix, proj_matrix, culled_prim_indices, tile_offsets, device)
             freq, att = self._frequency_tables(device)
         base = [ray_o.contiguous(), unit_dirs, self.positions.contiguous(), self.log_scales.contiguous(),
-                F.normalize(self.quats, dim=-1).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
+                ops.unit_quats(self.quats).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
                 self.W1.contiguous(), self.b1.contiguous(), self.W2.contiguous(), self.b2.contiguous(),
                 self.W3.contiguous(), self.b3.contiguous()]
         frame = Frame(int(W), int(H), float(score_threshold), float(self.feature_gating_beta),
@@ -846,7 +854,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
                                 culled_prim_indices, tile_offsets, return_feature, device):
         """RGB with autograd (scannet/cumodel.py:1110-1131): tile lists and encodings are constants, positions,
         log-scales, normalised quaternions and MLP weights carry gradients."""
-        self.invalidate_render_caches()
+        self._forget_parameters()
         W, H = self.image_size
         ts = int(self.tile_size)
         with torch.no_grad():
@@ -857,7 +865,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         mode = 1 if self._resolve_tile_order_mode() == "tilecenter" else 0
         rgb = _TileRenderAutogradFn.apply(
             ray_o.contiguous(), unit_dirs, self.positions.contiguous(), self.log_scales.contiguous(),
-            F.normalize(self.quats, dim=-1).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
+            ops.unit_quats(self.quats).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
             self.W1.contiguous(), self.b1.contiguous(), self.W2.contiguous(), self.b2.contiguous(),
             self.W3.contiguous(), self.b3.contiguous(), int(W), int(H), ts, ts, float(score_threshold), mode,
             self._background(bg_color, ray_o))
@@ -870,7 +878,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         """(rgb, feature image) with autograd (scannet/cumodel.py:1128-1160), in either order."""
         fn = (_TileRenderWithFeatAutogradFn if self._resolve_tile_order_mode() == "tilecenter"
               else _TileRenderWithFeatPerPixelAutogradFn)
-        self.invalidate_render_caches()
+        self._forget_parameters()
         W, H = self.image_size
         ts = int(self.tile_size)
         with torch.no_grad():
@@ -880,7 +888,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             freq, att = self._frequency_tables(device)
         return fn.apply(
             ray_o.contiguous(), unit_dirs, self.positions.contiguous(), self.log_scales.contiguous(),
-            F.normalize(self.quats, dim=-1).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
+            ops.unit_quats(self.quats).contiguous(), culled_prim_indices, tile_offsets.to(torch.int32), freq, att,
             self.W1.contiguous(), self.b1.contiguous(), self.W2.contiguous(), self.b2.contiguous(),
             self.W3.contiguous(), self.b3.contiguous(), self.feat_attr.contiguous(), float(self.feature_gating_beta),
             float(self.feature_gating_temp), int(W), int(H), ts, ts, float(score_threshold),

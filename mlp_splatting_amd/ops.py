@@ -66,6 +66,41 @@ def normalize_rays(rays_d):
     return out
 
 
+class _UnitQuats(torch.autograd.Function):
+    """``F.normalize(quats, dim=-1)`` of float32 [N, 4]: the same bits in one launch, and its gradient in one."""
+    @staticmethod
+    def forward(ctx, quats):
+        quats = quats.detach()
+        ctx.save_for_backward(quats)
+        ctx.set_materialize_grads(False)
+        out = torch.empty_like(quats)
+        with torch.cuda.device(quats.device):
+            _check(_lib.load().mlpsp_normalize_quats(_ptr(quats), quats.shape[0], _ptr(out), _stream(quats.device)),
+                   "mlpsp_normalize_quats")
+        return out
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, grad):
+        if grad is None:
+            return None
+        quats, = ctx.saved_tensors
+        grad, out = grad.contiguous(), torch.empty_like(quats)
+        grad = grad.clone() if grad.data_ptr() % 16 else grad
+        with torch.cuda.device(quats.device):
+            _check(_lib.load().mlpsp_normalize_quats_backward(_ptr(quats), _ptr(grad), quats.shape[0], _ptr(out),
+                                                              _stream(quats.device)), "mlpsp_normalize_quats_backward")
+        return out
+
+
+def unit_quats(quats):
+    """``F.normalize(quats, dim=-1)``, differentiable once."""
+    if (quats.is_cuda and quats.dtype == torch.float32 and quats.dim() == 2 and quats.shape[1] == 4
+            and quats.is_contiguous() and quats.data_ptr() % 16 == 0):
+        return _UnitQuats.apply(quats)
+    return torch.nn.functional.normalize(quats, dim=-1)
+
+
 def frame_prologue(rays_o, rays_d, W, H, TW=8, TH=8, records=None):
     """(unit directions, tile pyramids, frame records | None) of a W x H frame in one launch: what
     :func:`normalize_rays` returns; the per-tile ray pyramids :func:`sort_tiles` takes as ``tile_pyramids``; and, with
@@ -846,28 +881,15 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
     return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps, records)
 
 
-class TrainGroups:
-    """The steps of a frame sorted by primitive: ``prim`` the sorted primitives, ``scratch`` the index and row buffer of
-    the gradient kernels, ``slot`` / ``tile`` of the steps in tile order."""
-    __slots__ = ("prim", "perm", "slot", "tile", "scratch")
-
-
 def train_group(frame, tile_offsets, n):
-    dev = frame.workspace.device
+    """The steps of ``frame`` sorted by primitive: the scratch buffer of the gradient kernels, its index part filled."""
     lib = _lib.load()
-    S = frame.steps
-    listed = torch.empty(3, max(S, 1), dtype=torch.int32, device=dev)
-    groups = TrainGroups()
-    keys, groups.slot, groups.tile = listed[0, :S], listed[1], listed[2]
-    _check(lib.mlpsp_train_list_steps(_ptr(tile_offsets), frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
-                                      frame.workspace.numel(), _ptr(listed[0]), _ptr(listed[1]), _ptr(listed[2]),
-                                      _stream(dev)), "mlpsp_train_list_steps")
-    groups.prim, groups.perm = torch.sort(keys, stable=True)
-    nbytes = lib.mlpsp_train_scratch_bytes(S, n)
-    groups.scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    _check(lib.mlpsp_train_group(_ptr(groups.prim), _ptr(groups.perm), _ptr(listed[1]), _ptr(listed[2]), S, n, frame.width,
-                                 _ptr(groups.scratch), nbytes, _stream(dev)), "mlpsp_train_group")
-    return groups
+    nbytes = lib.mlpsp_train_scratch_bytes(frame.steps, n)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=frame.workspace.device)
+    _check(lib.mlpsp_train_group(_ptr(tile_offsets), frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
+                                 frame.workspace.numel(), frame.steps, n, _ptr(scratch), nbytes, _stream(scratch.device)),
+           "mlpsp_train_group")
+    return scratch
 
 
 def train_reverse(frame, tile_offsets, grad_rgb, grad_t):
@@ -891,9 +913,8 @@ def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scale
         return grads + geo, torch.zeros(1, dtype=torch.int32, device=dev)
     flag = torch.empty(1, dtype=torch.int32, device=dev)
     code = _lib.load().mlpsp_train_gradients(
-        _ptr(groups.prim), frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace),
-        frame.workspace.numel(), _ptr(d4), _ptr(falloff), _ptr(rays_d), _ptr(freq), _ptr(att), *[_ptr(w) for w in ws[:5]],
-        _ptr(log_scales), _ptr(quats), n, int(precision), float(scale), _ptr(groups.scratch), groups.scratch.numel(),
+        frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace), frame.workspace.numel(), _ptr(d4), _ptr(falloff), _ptr(rays_d), _ptr(freq), _ptr(att), *[_ptr(w) for w in ws[:5]],
+        _ptr(log_scales), _ptr(quats), n, int(precision), float(scale), _ptr(groups), groups.numel(),
         *[_ptr(g) for g in grads], *[_ptr(g) for g in geo], _ptr(flag), _stream(dev))
     _check(code, "mlpsp_train_gradients")
     return grads + geo, flag
@@ -936,7 +957,7 @@ def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoi
     rows = torch.empty(feature.row_bytes, dtype=torch.uint8, device=dev)
     out = torch.empty_like(attributes)
     _check(_lib.load().mlpsp_train_feature_gradients(
-        _ptr(groups.prim), frame.steps, frame.width, frame.height, *feature.target_size, feature.channels, feature.slots,
-        _ptr(kept), feature.kept, _ptr(groups.scratch), groups.scratch.numel(), attributes.shape[0], _ptr(loss_adjoint),
+        frame.steps, frame.width, frame.height, *feature.target_size, feature.channels, feature.slots,
+        _ptr(kept), feature.kept, _ptr(groups), groups.numel(), attributes.shape[0], _ptr(loss_adjoint),
         _ptr(rows), _ptr(out), _stream(dev)), "mlpsp_train_feature_gradients")
     return out

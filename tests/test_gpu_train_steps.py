@@ -115,3 +115,19 @@ def test_feature_training_step_of_an_empty_scene(device, oracle_mod):
     assert float(rgb.detach().abs().max()) == 0.0 and float(loss.detach()) == 1.0
     (rgb.sum() + loss).backward()
     assert attributes.grad.shape == attributes.shape
+
+
+def test_unit_quaternions_are_those_of_torch(device):
+    from mlp_splatting_amd import ops
+    gen = torch.Generator(device=device).manual_seed(2)
+    q = torch.randn(5000, 4, device=device, generator=gen)
+    q[:3] *= torch.tensor([[0.0], [1e-20], [1e18]], device=device)
+    g = torch.randn(5000, 4, device=device, generator=gen)
+    grads = []
+    for f in (ops.unit_quats, lambda t: torch.nn.functional.normalize(t, dim=-1)):
+        leaf = q.clone().requires_grad_()
+        u = f(leaf)
+        u.backward(g)
+        grads.append((u.detach(), leaf.grad))
+    assert torch.equal(grads[0][0], grads[1][0])
+    torch.testing.assert_close(grads[0][1], grads[1][1], rtol=1e-5, atol=1e-6)
