@@ -8,10 +8,9 @@
 //      the primitives that hit and per pixel the weight w and the four gates (hit records,
 //      mlpsp_hitrec.hpp): float[K][64] with K = 5 (w, g0..g3) or 1 (w), w = -1 where the primitive missed;
 //   2. feat_accumulate_kernel turns the roles around: lane = channel.  A 256-thread block owns one
-//      64-pixel item; wavefront v owns channels [128v, 128v+128) of all 64 pixels in 128 accumulator
-//      VGPRs.  Per record the attribute rows are two coalesced loads per slot, the per-pixel weight and
-//      gates are wave-uniform scalar operands, a pixel the primitive missed costs one scalar branch, and
-//      every output row is written exactly once.
+//      64-pixel item, a wavefront 128 channels of 32 or 16 of its pixels.  Per record the attribute rows
+//      are two coalesced loads per slot, the per-pixel weight and gates are wave-uniform scalar operands, a
+//      pixel the primitive missed costs one scalar branch, and every output row is written exactly once.
 #include "mlpsp_device.hpp"
 #include "mlpsp_hitrec.hpp"
 #include "mlpsp_host.hpp"
@@ -22,32 +21,41 @@ namespace mlpsp {
 
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-// SLOTS = 1, 4 or 5; mix as np_tile_kernels.cu:6037-6070.
-template <int SLOTS>
+// SLOTS = 1, 4 or 5; mix as np_tile_kernels.cu:6037-6070.  PX: pixels per wavefront, 16 or 32; 64 / PX wavefronts share
+// 128 channels.  Bound by latency: a record is its slot, then its rows and weights, then two to ten operations per hit.
+// Few pixels per wavefront mean more wavefronts (all four of a block have channels at 128 already) on smaller
+// accumulators (58 to 73 registers at 16 pixels, 150 at 64), at the price of fetching the rows 64 / PX times.
+// 333x251, 30,000 primitives, 67 channels: 433 us with 64 pixels and one slot fetch per record, 187 us with 16.
+// Fetching the next record's rows ahead gained nothing at either size.
+template <int SLOTS, int PX>
 __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __restrict__ feat_attr, int C, HitPool hp,
                                                               const int32_t* __restrict__ offsets, TileGeom g,
-                                                              int waves_per_tile, int per_xcd, int num_items,
-                                                              float* __restrict__ out_feat) {
-  const int item = (blockIdx.x % kNumXcd) * per_xcd + blockIdx.x / kNumXcd;
-  if (item >= num_items) return;
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int c0 = ((int)blockIdx.y * 4 + wave) * 128;
+                                                              int waves_per_tile, float* __restrict__ out_feat) {
+  constexpr int kShare = 64 / PX;
+  // (the render's mapping: what a tile's wavefront wrote lies in this XCD's L2)
+  const int unit = (int)(blockIdx.x / kNumXcd), wslot = unit % waves_per_tile;
+  const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
+  if (tile < 0) return;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int c0 = ((int)blockIdx.y * (4 / kShare) + wave / kShare) * 128, px0 = (wave % kShare) * PX;
   if (c0 >= C) return;
-  const int tile = item / waves_per_tile, wslot = item % waves_per_tile;
-  const int hits = hp.item_hits[item];
+  const int hits = hp.item_hits[tile * waves_per_tile + wslot];
   const int table_base = wslot * hp.table_stride + (offsets[tile] >> 4) + tile;
   const int ca = c0 + l, cb = c0 + 64 + l;
   const bool has_a = ca < C, has_b = cb < C;
   constexpr bool GATED = SLOTS > 1;
-  constexpr int K = GATED ? 5 : 1;
 
-  float acc[64][2];
+  float acc[PX][2];
 #pragma unroll
-  for (int px = 0; px < 64; ++px) acc[px][0] = acc[px][1] = 0.f;
+  for (int px = 0; px < PX; ++px) acc[px][0] = acc[px][1] = 0.f;
 
+  int slots = 0, ids = 0;               // of 64 records, one per lane
   for (int m = 0; m < hits; ++m) {
-    const int rs = __builtin_amdgcn_readfirstlane(hit_slot(hp, table_base, m));
-    const int p = __builtin_amdgcn_readfirstlane(hp.hit_ids[rs]);
+    if ((m & 63) == 0) {
+      slots = m + l < hits ? hit_slot(hp, table_base, m + l) : 0;
+      ids = m + l < hits ? hp.hit_ids[slots] : 0;
+    }
+    const int rs = __builtin_amdgcn_readlane(slots, m & 63), p = __builtin_amdgcn_readlane(ids, m & 63);
     const float* __restrict__ rows = feat_attr + (size_t)p * SLOTS * C;
     float ra[SLOTS], rb[SLOTS];
 #pragma unroll
@@ -55,11 +63,11 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
       ra[s] = has_a ? rows[(size_t)s * C + ca] : 0.f;
       rb[s] = has_b ? rows[(size_t)s * C + cb] : 0.f;
     }
-    const float* __restrict__ rec = reinterpret_cast<const float*>(hp.records + (size_t)rs * hp.record_bytes);
+    const float* __restrict__ rec = reinterpret_cast<const float*>(hp.records + (size_t)rs * hp.record_bytes) + px0;
     // weights and gates of 8 pixels at a time: wave-uniform 32-byte scalar loads, issued unconditionally
     // so that their latency overlaps the previous group's arithmetic
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < PX / 8; ++q) {
       const f32x8 w8 = *reinterpret_cast<const f32x8*>(rec + 8 * q);
       f32x8 g8[4];
       if constexpr (GATED) {
@@ -106,8 +114,8 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
 
   const int tx = tile % g.ntx, ty = tile / g.ntx;
 #pragma unroll
-  for (int px = 0; px < 64; ++px) {
-    const int slot = wslot * 64 + px;
+  for (int px = 0; px < PX; ++px) {
+    const int slot = wslot * 64 + px0 + px;
     const int x = tx * g.TW + slot % g.TW, y = ty * g.TH + slot / g.TW;
     if (slot < g.TW * g.TH && x < g.W && y < g.H) {
       float* __restrict__ dst = out_feat + (size_t)(y * g.W + x) * C;
@@ -115,7 +123,6 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
       if (has_b) dst[cb] = acc[px][1];
     }
   }
-  (void)K;
 }
 
 }  // namespace mlpsp
@@ -202,13 +209,21 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
 #undef MLPSP_EMIT_ARGS
 #undef MLPSP_EMIT_LAUNCH
   MLPSP_LAUNCH_CHECK();
-  const dim3 agrid((unsigned)(per_xcd * kNumXcd), (unsigned)ceil_div(feat_channels, 512)), ablock(256);
-#define MLPSP_ACC_LAUNCH(SL)                                                                                     \
-  hipLaunchKernelGGL((feat_accumulate_kernel<SL>), agrid, ablock, 0, s, feat_attr_dev, feat_channels, hp,        \
-                     tile_offsets_dev, g, wpt, per_xcd, (int)items, out_feat_dev)
-  if (feat_slots == 4) MLPSP_ACC_LAUNCH(4);
-  else if (feat_slots == 5) MLPSP_ACC_LAUNCH(5);
-  else MLPSP_ACC_LAUNCH(1);
+#define MLPSP_ACC_LAUNCH(SL, PX)                                                                                    \
+  hipLaunchKernelGGL((feat_accumulate_kernel<SL, PX>), dim3(superblock_grid(g.ntx, g.nty) * (unsigned)wpt,            \
+                     (unsigned)ceil_div(feat_channels, 8 * PX)), dim3(256), 0, s, feat_attr_dev, feat_channels, hp,   \
+                     tile_offsets_dev, g, wpt, out_feat_dev)
+  // 16 pixels per wavefront unless the rows are long and the launch fills the chip anyway: whole frames in us with 32 / 16
+  // pixels, 333x251 (1,344 items) 67 channels 1250 / 1185, 512 channels 1545 / 1521; 640x480 (4,800 items) 64 channels
+  // 2685 / 2515, 256 channels 2920 / 2945, 512 channels 3630 / 3795 (4240 with 64 pixels).
+  const bool sixteen = feat_channels <= 128 || items <= 2048;
+  if (feat_slots == 4) {
+    if (sixteen) MLPSP_ACC_LAUNCH(4, 16); else MLPSP_ACC_LAUNCH(4, 32);
+  } else if (feat_slots == 5) {
+    if (sixteen) MLPSP_ACC_LAUNCH(5, 16); else MLPSP_ACC_LAUNCH(5, 32);
+  } else {
+    if (sixteen) MLPSP_ACC_LAUNCH(1, 16); else MLPSP_ACC_LAUNCH(1, 32);
+  }
 #undef MLPSP_ACC_LAUNCH
   MLPSP_LAUNCH_CHECK();
   // status_dev[0] = 1 if the record pool was too small (the feature image is then incomplete)

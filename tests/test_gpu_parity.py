@@ -700,6 +700,28 @@ def test_feature_render_is_bit_exact(device, oracle_mod, slots, channels):
     _assert_bits(feat, want["feat"], "feat")
 
 
+@pytest.mark.parametrize("slots,channels", [(4, 129), (5, 256), (1, 257)])
+def test_feature_pixels_per_wavefront_give_the_same_bits(device, oracle_mod, slots, channels):
+    """Over 2048 tiles and 128 channels a wavefront takes 32 pixels; the same channels in pieces take it 16."""
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=900, width=421, height=317, feature_dim=channels, feature_slots=max(slots, 4))
+    sc = fr.scene
+    fa = sc.feat_attr if slots > 1 else np.ascontiguousarray(sc.feat_attr[:, 0])
+    cand, off = fr.oracle_lists(oracle_mod)
+    rec = ops.prepare_primitives(_t(sc.positions, device), _t(sc.log_scales, device), _t(sc.quats, device))
+    ro, rd, c, o = _t(fr.rays_o, device), _t(fr.rays_d, device), _t(cand, device), _t(off, device)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8)
+
+    def feature(rows):
+        return ops.render_tilecenter_feat_f32(ro, rd, rec, order, o, _t(sc.freq, device), _t(sc.att, device),
+                                              *[_t(w, device) for w in sc.mlp()], _t(np.ascontiguousarray(rows), device),
+                                              1.3, 2.2, fr.W, fr.H, 8, 8, fr.thr)[2].cpu().numpy()
+    whole = feature(fa)
+    assert np.abs(whole).max() > 1e-3
+    for first in range(0, channels, 100):
+        _assert_bits(whole[:, first:first + 100], feature(fa[..., first:first + 100]), "feat")
+
+
 @pytest.mark.parametrize("with_feat", [False, True])
 def test_per_pixel_render_is_bit_exact(device, oracle_mod, with_feat):
     from mlp_splatting_amd import ops
