@@ -11,6 +11,11 @@
 
 namespace mlpsp {
 
+// A set of lanes as a scalar mask, and back: a condition made of several comparisons is put together by the scalar unit
+// (__ballot(a) & __ballot(b)), where __ballot(a && b) takes the vector unit two more instructions, and a branch on
+// lane_in(mask) none.
+__device__ __forceinline__ bool lane_in(unsigned long long mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
 constexpr float kTransmittanceFloor = 1e-3f;  // pixel stops once T < 1e-3 (np_tile_kernels.cu:2026)
 constexpr float kInvalidKey = 1e30f;          // sort key of primitives behind the ray (np_tile_kernels.cu:514-517)
 

@@ -269,18 +269,19 @@ __device__ __forceinline__ f32x4 layer3_small(u32x4 a, u32x4 b, f32x4 c) {
 // lane's own hit offset (inputs 3..5; lanes that did not hit pass anything finite).  o[k] = output k of THIS
 // lane's pixel, output bias included.
 // CHECK: report pre-activations outside the operand type's range.  MASKS: also return the pixel's two
-// 32-bit ReLU masks (bit u = hidden unit u active) in mk.  Returns true if a stored weight was flagged
-// non-finite when packed or (CHECK) a pre-activation of a hit pixel is out of range.
-// Vector-memory instructions per call: 7 (W1, W2) + 1 (b2 words) + 2 (W3); the output bias and the flag are
-// wave-uniform scalar loads.
+// 32-bit ReLU masks (bit u = hidden unit u active) in mk.  Returns a mask of lanes that is not empty if a stored weight
+// was flagged non-finite when packed or (CHECK) a pre-activation of a hit pixel is out of range.
+// Vector-memory instructions per call: 7 (W1, W2) + 2 (W3); the output bias and the flag are wave-uniform scalar loads.
+// (Half the bias as the addend that lanes l and l ^ 32 both start the output layer from saves four additions and costs
+// four registers: spills, 648 instead of 615 us for the render with feature coefficients.)
 // LUT: the position words come from the workgroup's sin/cos table; kf then holds the phase scales times
 // 4 kSinCosEntries.
 template <typename T, bool CHECK, bool MASKS, bool LUT = false>
-__device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict__ blk, unsigned long long mask, int l,
+__device__ __forceinline__ unsigned long long mlp_wave_mfma16(const unsigned char* __restrict__ blk, unsigned long long mask, int l,
                                                 float dx, float dy, float dz, const float kf[3], const DirWords& dir,
                                                 float o[4], unsigned mk[2], const SinCosTable* table = nullptr) {
   const int g = l >> 5;
-  bool bad = false;
+  unsigned long long bad = 0ull;
   // Addresses of the weight loads: wave-uniform base in scalar registers + zero-extended 32-bit lane offset +
   // immediate, the form the global loads take as they are, so that no address is computed per lane and hit.  The
   // compiler picks that form only if it sees the zero extension next to the load; the lane index is therefore made
@@ -303,7 +304,7 @@ __device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict_
   for (int s = 0; s < 2; ++s) a3[s] = *reinterpret_cast<const u32x4*>(hi + (kOffW3 - 4096) + s * 128 + row16);
   const f32x4 b3v = *reinterpret_cast<const f32x4*>(blk + kOffB3);
   const int wflag = *reinterpret_cast<const int32_t*>(blk + kOffFlag);
-  bad |= (wflag != 0);
+  bad |= wflag != 0 ? 1ull : 0ull;
   // the constant operand word that multiplies the (hi, lo) bias words: k-slots of lane group 0 only
   const unsigned one_word = g ? 0u : Ops<T>::kOneWord;
 
@@ -317,7 +318,7 @@ __device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict_
     const unsigned half_mask = (unsigned)(mask >> (32 * b));
     if (half_mask != 0u) {   // wave-uniform: skip a 32-pixel block nobody hits
       const float xin[3] = {b ? hx.blk1 : hx.blk0, b ? hy.blk1 : hy.blk0, b ? hz.blk1 : hz.blk0};
-      const bool col_active = (half_mask >> (l & 31)) & 1u;
+      const unsigned long long columns = ((unsigned long long)half_mask << 32) | half_mask;   // both lane groups
       // layer 1: 18 (sin, cos) words per lane + the bias word, 5 K-steps; words 0..8 come from LDS.  (The lane
       // index is made opaque so that the loads stay here and are not hoisted out of the primitive loop into
       // registers.)
@@ -351,7 +352,7 @@ __device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict_
         }
         d1 = Ops<T>::mfma(a1[s], bw, d1);
       }
-      if constexpr (CHECK) bad |= col_active && out_of_range_in<T>(d1);
+      if constexpr (CHECK) bad |= columns & __ballot(out_of_range_in<T>(d1));
       // layer 2: the bias K-step first (its operands are ready), then the D registers of layer 1, rectified and
       // rounded, as the B operand
       // (its B operand is constant, three zero words and the (1, 1) word: the compiler keeps it in four registers
@@ -368,7 +369,7 @@ __device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict_
         }
         d2 = Ops<T>::mfma(a2[s], bw, d2);
       }
-      if constexpr (CHECK) bad |= col_active && out_of_range_in<T>(d2);
+      if constexpr (CHECK) bad |= columns & __ballot(out_of_range_in<T>(d2));
       // output layer: this lane's half of the four sums of its column (layer3_small)
       f32x4 d3 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -412,11 +413,11 @@ __device__ __forceinline__ bool mlp_wave_mfma16(const unsigned char* __restrict_
 // independent MFMA of block 1, and the operand preparation of one block sits behind the MFMA of the other.
 // No ReLU masks (render only).
 template <typename T, bool CHECK, bool LUT = false>
-__device__ __forceinline__ bool mlp_pair_mfma16(const unsigned char* __restrict__ blk, unsigned long long mask, int l,
+__device__ __forceinline__ unsigned long long mlp_pair_mfma16(const unsigned char* __restrict__ blk, unsigned long long mask, int l,
                                                 float dx, float dy, float dz, const float kf[3], const DirWords& dir,
                                                 float o[4], const SinCosTable* table = nullptr) {
   const int g = l >> 5;
-  bool bad = false;
+  unsigned long long bad = 0ull;
   // Addresses of the weight loads: wave-uniform base in scalar registers + zero-extended 32-bit lane offset +
   // immediate, the form the global loads take as they are, so that no address is computed per lane and hit.  The
   // compiler picks that form only if it sees the zero extension next to the load; the lane index is therefore made
@@ -437,12 +438,14 @@ __device__ __forceinline__ bool mlp_pair_mfma16(const unsigned char* __restrict_
   for (int s = 0; s < 2; ++s) a3[s] = *reinterpret_cast<const u32x4*>(hi + (kOffW3 - 4096) + s * 128 + row16);
   const f32x4 b3v = *reinterpret_cast<const f32x4*>(blk + kOffB3);
   const int wflag = *reinterpret_cast<const int32_t*>(blk + kOffFlag);
-  bad |= (wflag != 0);
+  bad |= wflag != 0 ? 1ull : 0ull;
   const unsigned one_word = g ? 0u : Ops<T>::kOneWord;
   const HalfPair hx = both_halves(dx), hy = both_halves(dy), hz = both_halves(dz);
   const float xin[2][3] = {{hx.blk0, hy.blk0, hz.blk0}, {hx.blk1, hy.blk1, hz.blk1}};
   const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   f32x16 d1[2] = {zero16, zero16};
+  const unsigned long long lo = mask & 0xffffffffull, up = mask >> 32;
+  const unsigned long long columns[2] = {lo | (lo << 32), up | (up << 32)};     // the lanes that hold a hit pixel's column
   // The wavefront asks for issue priority while it walks its MFMA chains (the other wavefronts of the SIMD are
   // mostly in vector work, which also issues beside an MFMA): 0.7 % off the kernel, measured against priority 0
   // on one device; raising it earlier, over the weight loads, or for the walk instead, gains nothing.
@@ -480,8 +483,8 @@ __device__ __forceinline__ bool mlp_pair_mfma16(const unsigned char* __restrict_
     }
   }
   if constexpr (CHECK) {
-    bad |= ((mask >> (l & 31)) & 1ull) && out_of_range_in<T>(d1[0]);
-    bad |= ((mask >> (32 + (l & 31))) & 1ull) && out_of_range_in<T>(d1[1]);
+    bad |= columns[0] & __ballot(out_of_range_in<T>(d1[0]));
+    bad |= columns[1] & __ballot(out_of_range_in<T>(d1[1]));
   }
   const unsigned z0 = 0u, z1 = 0u, z2 = 0u;
   // the bias tile of layer 2 (every column the same) is computed once and is the addend of both blocks' first K-step
@@ -498,8 +501,8 @@ __device__ __forceinline__ bool mlp_pair_mfma16(const unsigned char* __restrict_
     }
   }
   if constexpr (CHECK) {
-    bad |= ((mask >> (l & 31)) & 1ull) && out_of_range_in<T>(d2[0]);
-    bad |= ((mask >> (32 + (l & 31))) & 1ull) && out_of_range_in<T>(d2[1]);
+    bad |= columns[0] & __ballot(out_of_range_in<T>(d2[0]));
+    bad |= columns[1] & __ballot(out_of_range_in<T>(d2[1]));
   }
   f32x4 d3[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll

@@ -106,44 +106,52 @@ __global__ __launch_bounds__(256) void mark_listed_kernel(const int32_t* __restr
 // operand rounding of this path).  Same formulas as np_tile_kernels.cu:75-83, 2092-2103.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
 __device__ __forceinline__ float fast_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.0f + fast_exp(-x)); }
-__device__ __forceinline__ float fast_softplus(float x) {
-  const float e = fast_exp(x);
-  const float mid = __builtin_amdgcn_logf(1.0f + e) * 0.693147181f;
-  float y = (x < -20.f) ? e : mid;
-  y = (x > 20.f) ? x : y;
-  return y;
+// exp(-softplus(x) decay), what an entry lets through.  softplus(x) = max(x, 0) + log(1 + exp(-|x|)) needs no case of its
+// own where exp(x) overflows or 1 + exp(x) rounds to 1, and in units of log 2 -- y = x log2 e -- no scaling between its
+// logarithm and the next exponential.
+__device__ __forceinline__ float fast_keep(float x, float decay) {
+  const float y = x * 1.44269504f;
+  const float e = __builtin_amdgcn_exp2f(-__builtin_fabsf(y));
+  return __builtin_amdgcn_exp2f(-((__builtin_amdgcn_logf(1.0f + e) + fmaxf(y, 0.f)) * decay));
 }
 __device__ __forceinline__ float fast_blend_step(PixelAcc& a, float o0, float o1, float o2, float o3, float decay) {
-  const float sigma = fast_softplus(o3) * decay;
-  const float alpha = 1.f - fast_exp(-sigma);
-  const float w = a.trans * alpha;
+  const float keep = fast_keep(o3, decay);
+  const float w = fmaf(-a.trans, keep, a.trans);
   a.cr = fmaf(w, fast_sigmoid(o0), a.cr);
   a.cg = fmaf(w, fast_sigmoid(o1), a.cg);
   a.cb = fmaf(w, fast_sigmoid(o2), a.cb);
-  a.trans = a.trans * (1.f - alpha);
+  a.trans = a.trans * keep;
   return w;
 }
-// tetrahedral gates (np_tile_kernels.cu:97-124) with the native exp/rcp.  qs = local hit offset divided by the
+// tetrahedral gates (np_tile_kernels.cu:97-124) with the native exp/rcp, times w.  qs = local hit offset divided by the
 // scales (what hit_fast() returns); u = q / (beta s + 1e-6) = qs k with k = s / (beta s + 1e-6), which depends on
-// the primitive alone (gate_factor).
+// the primitive alone (gate_factor); here k comes multiplied by `t` = temp log2 e, and u is clamped at |t| instead of 1,
+// so that the four sums are the exponents of 2 as they stand.  They add up to zero: one of them is not negative, and
+// the sum of the exponentials is at least 1.  BIG: |t| where they would overflow without the largest taken off first.
+// A lane that did not hit has w = 0 and any qs: the median with two numbers is a number.
 __device__ __forceinline__ float gate_factor(float lg, float beta) {
   const float s = fast_exp(lg);
   return s * __builtin_amdgcn_rcpf(beta * s + 1e-6f);
 }
-__device__ __forceinline__ void fast_tetra_gates(float qsx, float qsy, float qsz, float kx, float ky, float kz,
-                                                 float temp, float g[4]) {
-  const float ux = fminf(1.f, fmaxf(-1.f, qsx * kx));
-  const float uy = fminf(1.f, fmaxf(-1.f, qsy * ky));
-  const float uz = fminf(1.f, fmaxf(-1.f, qsz * kz));
-  const float l0 = temp * ((ux + uy) + uz), l1 = temp * ((ux - uy) - uz);
-  const float l2 = temp * ((-ux + uy) - uz), l3 = temp * ((-ux - uy) + uz);
-  const float lm = fmaxf(fmaxf(l0, l1), fmaxf(l2, l3));
-  const float e0 = fast_exp(l0 - lm), e1 = fast_exp(l1 - lm), e2 = fast_exp(l2 - lm), e3 = fast_exp(l3 - lm);
-  const float inv = __builtin_amdgcn_rcpf(fmaxf(((e0 + e1) + e2) + e3, 1e-8f));
-  g[0] = e0 * inv;
-  g[1] = e1 * inv;
-  g[2] = e2 * inv;
-  g[3] = e3 * inv;
+constexpr float kGateExponents = 40.f;      // |t| up to which 2^(3 |t|), four of them added, is far from overflow
+template <bool BIG>
+__device__ __forceinline__ void fast_tetra_gates(float w, float qsx, float qsy, float qsz, const f32x4& k, float t, float g[4]) {
+  const float ux = __builtin_amdgcn_fmed3f(qsx * k[0], -t, t);
+  const float uy = __builtin_amdgcn_fmed3f(qsy * k[1], -t, t);
+  const float uz = __builtin_amdgcn_fmed3f(qsz * k[2], -t, t);
+  const float s = ux + uy, d = ux - uy;
+  float l[4] = {s + uz, d - uz, -d - uz, uz - s};
+  if constexpr (BIG) {
+    const float lm = fmaxf(fmaxf(l[0], l[1]), fmaxf(l[2], l[3]));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) l[j] -= lm;
+  }
+  float e[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) e[j] = __builtin_amdgcn_exp2f(l[j]);
+  const float share = w * __builtin_amdgcn_rcpf(((e[0] + e[1]) + e[2]) + e[3]);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) g[j] = e[j] * share;
 }
 
 // The second half of a PrimRecord (mlpsp_device.hpp): one 64-byte line per primitive.
@@ -185,9 +193,9 @@ __device__ __forceinline__ FastRec fast_arrived(FastRegs& q) {
 //
 // The hit decision itself is a hard threshold, and a primitive that barely hits still contributes up to a
 // few 1e-3 to a pixel, so a decision that differs from the exact path's would show as isolated pixel
-// errors well above the rounding noise of this path.  unsure = the fast quantities are too close to one of
+// errors well above the rounding noise of this path.  unsure = the lanes whose fast quantities are too close to one of
 // the three decision boundaries (decay within `band` of thr, t or denom near zero) to be trusted; the
-// caller then takes the decision -- only the decision -- from hit_rot().
+// caller then takes the decision -- only the decision -- from hit_rot().  The others hit where t and decay say so.
 //
 // How wide the band has to be: with u = 2^-24, vl and dl carry about 4 u |vl| and 4 u |dl| of rounding (entries of
 // r rounded, three-term sums), t = numer / denom about 24 u |vl| / |dl|, so ql = vl - t dl is off by up to
@@ -215,8 +223,11 @@ __device__ __forceinline__ OriginTerms origin_terms(float ox, float oy, float oz
   o.vlz = fmaf(r[6], o.vx, fmaf(r[7], o.vy, r[8] * o.vz));
   return o;
 }
-__device__ __forceinline__ bool hit_fast(const OriginTerms& o, float rdx, float rdy, float rdz, const float r[9],
-                                         float thr, float band, HitInfo& h, bool& unsure) {
+struct HitMasks {
+  unsigned long long hit, unsure;
+};
+__device__ __forceinline__ HitMasks hit_fast(const OriginTerms& o, float rdx, float rdy, float rdz, const float r[9],
+                                             float thr_lo, float thr_hi, HitInfo& h) {
   const float dlx = fmaf(r[0], rdx, fmaf(r[1], rdy, r[2] * rdz));
   const float dly = fmaf(r[3], rdx, fmaf(r[4], rdy, r[5] * rdz));
   const float dlz = fmaf(r[6], rdx, fmaf(r[7], rdy, r[8] * rdz));
@@ -232,11 +243,12 @@ __device__ __forceinline__ bool hit_fast(const OriginTerms& o, float rdx, float 
   h.qlz = fmaf(-t, dlz, o.vlz);
   const float r2 = fmaf(h.qlx, h.qlx, fmaf(h.qly, h.qly, h.qlz * h.qlz));
   h.decay = __builtin_amdgcn_exp2f(r2 * -0.72134752f);
-  unsure = (__builtin_fabsf(h.decay - thr) <= band) || !(__builtin_fabsf(t) >= 1e-4f) || !(denom >= 1e-18f);
-  return !(denom <= 1e-20f) && !(t <= 0.f) && (h.decay > thr);
+  const unsigned long long above = __ballot(h.decay > thr_hi), below = __ballot(h.decay < thr_lo);
+  const unsigned long long sure = (above | below) & __ballot(__builtin_fabsf(t) >= 1e-4f) & __ballot(denom >= 1e-18f);
+  return HitMasks{above & __ballot(t > 0.f) & sure, ~sure};
 }
 
-// LDS of one wavefront: the OriginTerms of the 64 list entries it is walking and the width of their decision
+// LDS of one wavefront: the OriginTerms of the 64 list entries it is walking and the ends of their decision
 // band (one address register for the two reads of a step); with a gated feature channel also the entries' three
 // gate factors, which a hit would otherwise have to fetch from the primitive's record -- a load that nothing but
 // the gates waits for, at the end of the step.
@@ -286,7 +298,8 @@ __device__ __forceinline__ void render_tile_mfma(
     for (int j = 0; j < 3; ++j) kfm[j] = kf[j] * (4.0f * (float)kSinCosEntries);
   }
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
-  bool bad = false;
+  unsigned long long bad = 0ull;       // lanes (or any bit) with something this path cannot represent
+  float largest = 0.f;                 // output of the MLP at this lane's hits, in magnitude
   const int tx = tile % ntx, ty = tile / ntx;
   const int x = tx * 8 + (l & 7), y = ty * 8 + (l >> 3);
   const bool valid = (x < W) && (y < H);
@@ -309,13 +322,15 @@ __device__ __forceinline__ void render_tile_mfma(
   const float ox = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(rox), lane0)),
               oy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(roy), lane0)),
               oz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(roz), lane0));
-  const float reach = 4e-6f * __builtin_sqrtf(fmaxf(-2.f * __logf(thr), 0.f));   // see band_for()
+  const float radius = __builtin_sqrtf(fmaxf(-2.f * __logf(thr), 0.f));     // of the threshold's ellipsoid, in scales
+  const float reach = 4e-6f * radius;   // see band_for()
+  const float gate_t = temp * 1.44269504f;
   const bool one_origin = __ballot(valid && !(rox == ox && roy == oy && roz == oz)) == 0ull;
 
   const int start = offsets[tile], end = ends[tile];
   PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
   HitEmitter em = hit_emitter_begin(hp, 0, start, tile);
-  bool live = valid;
+  unsigned long long live = in_image;
   const unsigned char* __restrict__ fast_half = reinterpret_cast<const unsigned char*>(prims) + 64;
 
   // The tile's list is read 64 entries at a time, one coalesced load; a lane's entry is broadcast with
@@ -327,17 +342,26 @@ __device__ __forceinline__ void render_tile_mfma(
     const int id_lane = (base + l < end) ? order[base + l] : -1;
     unsigned long long todo = __ballot(id_lane >= 0 && id_lane < N);
     if (todo == 0ull) continue;
+    // A hit lies within `radius` of the largest scale from the centre: only where that is beyond the inputs' limit for
+    // one of the 64 entries (or not known) are their hits' inputs looked at one by one.
+    bool reaches = !one_origin || !(thr > 0.f);
     if (one_origin && id_lane >= 0 && id_lane < N) {
       const FastRec& F = *reinterpret_cast<const FastRec*>(fast_half + (size_t)id_lane * sizeof(PrimRecord));
       const OriginTerms o = origin_terms(ox, oy, oz, F.cx, F.cy, F.cz, F.r);
+      float inverse2 = 3.4028235e38f;          // the smallest of the inverse scales, squared
+#pragma unroll
+      for (int k = 0; k < 9; k += 3)
+        inverse2 = fminf(inverse2, fmaf(F.r[k], F.r[k], fmaf(F.r[k + 1], F.r[k + 1], F.r[k + 2] * F.r[k + 2])));
+      reaches |= !(2.f * radius <= input_limit * __builtin_amdgcn_sqrtf(inverse2));    // (2: sum of three magnitudes)
       *reinterpret_cast<f32x4*>(&s_org.e[l][0]) = f32x4{o.vx, o.vy, o.vz, o.vlx};
-      *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, band_for(o, thr, reach), 0.f};
+      *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, thr - band_for(o, thr, reach), thr + band_for(o, thr, reach)};
     }
+    const bool look = __ballot(reaches) != 0ull;
     if constexpr (SP > 0) {
       if (slots > 1 && id_lane >= 0 && id_lane < N) {
         const PrimRecord& P = prims[id_lane];
         *reinterpret_cast<f32x4*>(&s_org.e[l][8]) =
-            f32x4{gate_factor(P.lgx, beta), gate_factor(P.lgy, beta), gate_factor(P.lgz, beta), 0.f};
+            f32x4{gate_t * gate_factor(P.lgx, beta), gate_t * gate_factor(P.lgy, beta), gate_t * gate_factor(P.lgz, beta), 0.f};
       }
     }
     int j = (int)__builtin_ctzll(todo);
@@ -351,19 +375,22 @@ __device__ __forceinline__ void render_tile_mfma(
       // while they are being loaded.
       const FastRec R = fast_arrived(q);
       OriginTerms ot;
-      float band;
+      float thr_lo, thr_hi;
       if (one_origin) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(&s_org.e[j][0]);
         const f32x4 b = *reinterpret_cast<const f32x4*>(&s_org.e[j][4]);
         ot = OriginTerms{a[0], a[1], a[2], a[3], b[0], b[1]};
-        band = b[2];
+        thr_lo = b[2];
+        thr_hi = b[3];
       } else {
         ot = origin_terms(rox, roy, roz, R.cx, R.cy, R.cz, R.r);
-        band = band_for(ot, thr, reach);
+        const float band = band_for(ot, thr, reach);
+        thr_lo = thr - band;
+        thr_hi = thr + band;
       }
       HitInfo h;
-      bool unsure;
-      bool hit = hit_fast(ot, rdx, rdy, rdz, R.r, thr, band, h, unsure) && live;
+      const HitMasks test = hit_fast(ot, rdx, rdy, rdz, R.r, thr_lo, thr_hi, h);
+      unsigned long long mask = test.hit & live;
       asm volatile("" : "+v"(h.t), "+v"(h.qlx), "+v"(h.qly), "+v"(h.qlz), "+v"(h.decay));   // R is used up here
 
       const bool more = todo != 0ull;
@@ -376,20 +403,23 @@ __device__ __forceinline__ void render_tile_mfma(
         // the loop, when the compiler has long given them to something else)
         fast_request(fast_half + (size_t)p_next * sizeof(PrimRecord), q);
       }
-      if (__ballot(unsure && live) != 0ull) {   // rare
-        if (unsure && live) {
+      const unsigned long long unsure = test.unsure & live;
+      if (unsure != 0ull) {   // rare
+        bool exact_hit = false;
+        if (lane_in(unsure)) {
           const PrimRecord P = prims[p];
           HitInfo exact;
-          hit = hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, exact);
+          exact_hit = hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, exact);
         }
+        mask |= unsure & __ballot(exact_hit);
       }
-      const unsigned long long mask = __ballot(hit);
       ++n_proc;
       if (mask != 0ull) {
         ++n_proc_hit;
         n_hits += __popcll(mask);
         const unsigned char* __restrict__ blk = packed + (size_t)p * kPackStride;
-        bad |= hit && !((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit);
+        if (look)
+          bad |= mask & __ballot(!((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit));
         float o[4];
         if ((unsigned)mask != 0u && (unsigned)(mask >> 32) != 0u)
           bad |= mlp_pair_mfma16<T, Ops<T>::kCheckHidden, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm, s_dir, o,
@@ -398,33 +428,36 @@ __device__ __forceinline__ void render_tile_mfma(
           bad |= mlp_wave_mfma16<T, Ops<T>::kCheckHidden, false, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm,
                                                                                       s_dir, o, nullptr, table);
         float w = 0.f;
-        if (hit) {
-          bad |= !(max3_abs(o[0], o[1], o[2]) <= 3.4028235e38f) || !(__builtin_fabsf(o[3]) <= 3.4028235e38f);
+        if (lane_in(mask)) {
+          // (infinities show here, NaN in the sums below)
+          asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(o[0]), "v"(o[1]));
+          asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(o[2]), "v"(o[3]));
           w = fast_blend_step(acc, o[0], o[1], o[2], o[3], h.decay);
         }
         if constexpr (SP > 0) {
-          float gt[4] = {0.f, 0.f, 0.f, 0.f};
+          float gt[4] = {0.f, 0.f, 0.f, 0.f};       // w times the gates
           if (slots > 1) {
             const f32x4 k = *reinterpret_cast<const f32x4*>(&s_org.e[j][8]);
-            if (hit) fast_tetra_gates(h.qlx, h.qly, h.qlz, k[0], k[1], k[2], temp, gt);
+            if (__builtin_fabsf(gate_t) <= kGateExponents) fast_tetra_gates<false>(w, h.qlx, h.qly, h.qlz, k, gate_t, gt);
+            else fast_tetra_gates<true>(w, h.qlx, h.qly, h.qlz, k, gate_t, gt);
           }
           const int rs = hit_emitter_next(hp, em, l);
           if (rs >= 0) {
             unsigned* __restrict__ coef = reinterpret_cast<unsigned*>(hp.records + (size_t)rs * hp.record_bytes);
             if constexpr (SP == 4) {
-              const unsigned c01 = (slots > 1) ? Ops<_Float16>::pack2(w * gt[0], w * gt[1]) : Ops<_Float16>::pack2(w, 0.f);
-              const unsigned c23 = Ops<_Float16>::pack2(w * gt[2], w * gt[3]);
+              const unsigned c01 = (slots > 1) ? Ops<_Float16>::pack2(gt[0], gt[1]) : Ops<_Float16>::pack2(w, 0.f);
+              const unsigned c23 = Ops<_Float16>::pack2(gt[2], gt[3]);
               *reinterpret_cast<uint2*>(coef + l * 2) = make_uint2(c01, c23);
             } else {
-              const u32x4 c = {Ops<_Float16>::pack2(w, w * gt[0]), Ops<_Float16>::pack2(w * gt[1], w * gt[2]),
-                               Ops<_Float16>::pack2(w * gt[3], 0.f), 0u};
+              const u32x4 c = {Ops<_Float16>::pack2(w, gt[0]), Ops<_Float16>::pack2(gt[1], gt[2]),
+                               Ops<_Float16>::pack2(gt[3], 0.f), 0u};
               *reinterpret_cast<u32x4*>(coef + l * 4) = c;
             }
             if (l == 0) hp.hit_ids[rs] = p;
           }
         }
-        live = valid && (acc.trans >= kTransmittanceFloor);
-        if (__ballot(live) == 0ull) {
+        live = in_image & __ballot(acc.trans >= kTransmittanceFloor);
+        if (live == 0ull) {
           fast_arrived(q);       // (the next entry's line may still be landing in these registers)
           finished = true;
           break;
@@ -443,7 +476,9 @@ __device__ __forceinline__ void render_tile_mfma(
   if constexpr (SP > 0) {
     if (l == 0) hp.item_hits[tile] = em.count;
   }
-  if (__ballot(bad) != 0ull && l == 0) atomicExch(status, 1);
+  bad |= __ballot(!(largest <= 3.4028235e38f)) |
+         __ballot(!(__builtin_fabsf((acc.cr + acc.cg) + (acc.cb + acc.trans)) <= 3.4028235e38f));
+  if (bad != 0ull && l == 0) atomicExch(status, 1);
   if (counters && l == 0) {
     atomicAdd(counters + 1, (unsigned long long)n_proc);
     atomicAdd(counters + 2, (unsigned long long)n_proc_hit);
@@ -465,7 +500,7 @@ __device__ __forceinline__ void render_tile_mfma(
 // ---------------------------------------------------------------------------------------------
 template <int TEAM>
 struct TeamRound {
-  float alpha[TEAM][64];
+  float keep[TEAM][64];               // 1 - opacity
   float colour[TEAM - 1][3][64];      // of wavefronts 1..: wavefront 0 has its own in registers
 };
 
@@ -499,7 +534,7 @@ __device__ __forceinline__ void render_tile_team(
     for (int j = 0; j < 3; ++j) kfm[j] = kf[j] * (4.0f * (float)kSinCosEntries);
   }
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
-  bool bad = false;
+  unsigned long long bad = 0ull;
   const int tx = tile % ntx, ty = tile / ntx;
   const int x = tx * 8 + (l & 7), y = ty * 8 + (l >> 3);
   const bool valid = (x < W) && (y < H);
@@ -518,7 +553,7 @@ __device__ __forceinline__ void render_tile_team(
   const bool one_origin = __ballot(valid && !(rox == ox && roy == oy && roz == oz)) == 0ull;
   const int start = offsets[tile], end = ends[tile];
   float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
-  bool live = valid;
+  unsigned long long live = in_image;
   int buf = 0;
   const unsigned char* __restrict__ fast_half = reinterpret_cast<const unsigned char*>(prims) + 64;
   bool finished = false;
@@ -531,7 +566,7 @@ __device__ __forceinline__ void render_tile_team(
       const FastRec& F = *reinterpret_cast<const FastRec*>(fast_half + (size_t)id_lane * sizeof(PrimRecord));
       const OriginTerms o = origin_terms(ox, oy, oz, F.cx, F.cy, F.cz, F.r);
       *reinterpret_cast<f32x4*>(&s_org.e[l][0]) = f32x4{o.vx, o.vy, o.vz, o.vlx};
-      *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, band_for(o, thr, reach), 0.f};
+      *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, thr - band_for(o, thr, reach), thr + band_for(o, thr, reach)};
     }
     const int rounds = ((int)__builtin_popcountll(todo) + TEAM - 1) / TEAM;
     for (int i = 0; i < k; ++i) todo &= todo - 1ull;
@@ -544,25 +579,28 @@ __device__ __forceinline__ void render_tile_team(
     }
     team_barrier();
     for (int r = 0; r < rounds; ++r) {
-      float alpha = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-      bool hit = false, hit_bad = false, mlp_bad = false;     // mlp_bad: of any lane's pixel
+      float keep = 1.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+      unsigned long long mask = 0ull, hit_bad = 0ull, mlp_bad = 0ull;     // mlp_bad: of any lane's pixel
       const bool mine = todo != 0ull;
       if (mine) {
         const FastRec R = fast_arrived(q);
         OriginTerms ot;
-        float band;
+        float thr_lo, thr_hi;
         if (one_origin) {
           const f32x4 a = *reinterpret_cast<const f32x4*>(&s_org.e[j][0]);
           const f32x4 b = *reinterpret_cast<const f32x4*>(&s_org.e[j][4]);
           ot = OriginTerms{a[0], a[1], a[2], a[3], b[0], b[1]};
-          band = b[2];
+          thr_lo = b[2];
+          thr_hi = b[3];
         } else {
           ot = origin_terms(rox, roy, roz, R.cx, R.cy, R.cz, R.r);
-          band = band_for(ot, thr, reach);
+          const float band = band_for(ot, thr, reach);
+          thr_lo = thr - band;
+          thr_hi = thr + band;
         }
         HitInfo h;
-        bool unsure;
-        hit = hit_fast(ot, rdx, rdy, rdz, R.r, thr, band, h, unsure) && live;
+        const HitMasks test = hit_fast(ot, rdx, rdy, rdz, R.r, thr_lo, thr_hi, h);
+        mask = test.hit & live;
         asm volatile("" : "+v"(h.dx), "+v"(h.dy), "+v"(h.dz), "+v"(h.decay));   // R is used up here
         const int p_now = p;
 #pragma unroll
@@ -572,64 +610,64 @@ __device__ __forceinline__ void render_tile_team(
           p = __builtin_amdgcn_readlane(id_lane, j);
           fast_request(fast_half + (size_t)p * sizeof(PrimRecord), q);
         }
-        if (__ballot(unsure && live) != 0ull) {   // rare
-          if (unsure && live) {
+        const unsigned long long unsure = test.unsure & live;
+        if (unsure != 0ull) {   // rare
+          bool exact_hit = false;
+          if (lane_in(unsure)) {
             const PrimRecord P = prims[p_now];
             HitInfo exact;
-            hit = hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, exact);
+            exact_hit = hit_rot(rox, roy, roz, rdx, rdy, rdz, P, thr, exact);
           }
+          mask |= unsure & __ballot(exact_hit);
         }
-        const unsigned long long mask = __ballot(hit);
         if (mask != 0ull) {
           const unsigned char* __restrict__ blk = packed + (size_t)p_now * kPackStride;
-          hit_bad = !((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit);
           if ((unsigned)mask != 0u && (unsigned)(mask >> 32) != 0u)
             mlp_bad = mlp_pair_mfma16<T, Ops<T>::kCheckHidden, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz, kfm,
                                                                                     s_dir, o, table);
           else
             mlp_bad = mlp_wave_mfma16<T, Ops<T>::kCheckHidden, false, RenderTable<T>::kUse>(blk, mask, l, h.dx, h.dy, h.dz,
                                                                                            kfm, s_dir, o, nullptr, table);
-          if (hit) {
-            hit_bad |= !(max3_abs(o[0], o[1], o[2]) <= 3.4028235e38f) || !(__builtin_fabsf(o[3]) <= 3.4028235e38f);
-            alpha = 1.f - fast_exp(-(fast_softplus(o[3]) * h.decay));
+          hit_bad = __ballot(!((__builtin_fabsf(h.dx) + __builtin_fabsf(h.dy)) + __builtin_fabsf(h.dz) <= input_limit)) |
+                    __ballot(!(max3_abs(o[0], o[1], o[2]) <= 3.4028235e38f)) | __ballot(!(__builtin_fabsf(o[3]) <= 3.4028235e38f));
+          // (a lane without a hit: nothing held back, which changes neither the transmittance nor a colour; NaN where the
+          // lane hit and its opacity is NaN, as for a single wavefront)
+          if (lane_in(mask)) keep = fast_keep(o[3], h.decay);
 #pragma unroll
-            for (int c = 0; c < 3; ++c) o[c] = fast_sigmoid(o[c]);
-          }
+          for (int c = 0; c < 3; ++c) o[c] = lane_in(mask) ? fast_sigmoid(o[c]) : 0.f;
         }
       }
       TeamRound<TEAM>& round = s_round[buf];
       buf ^= 1;
-      // (a lane without a hit: opacity 0, which changes neither the transmittance nor a colour; NaN where the lane hit and
-      // its opacity is NaN, as for a single wavefront)
-      round.alpha[k][l] = hit ? alpha : 0.f;
+      round.keep[k][l] = keep;
       if (k > 0) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) round.colour[k - 1][c][l] = hit ? o[c] : 0.f;
+        for (int c = 0; c < 3; ++c) round.colour[k - 1][c][l] = o[c];
       }
       team_barrier();
 #pragma unroll
       for (int i = 0; i < TEAM; ++i) {
-        const float a = i == k ? (hit ? alpha : 0.f) : round.alpha[i][l];
-        const bool open = valid && trans >= kTransmittanceFloor;
+        const float let = i == k ? keep : round.keep[i][l];
+        const unsigned long long open = in_image & __ballot(trans >= kTransmittanceFloor);
         if (i == k) {                          // (an entry behind the last one that counts leaves no trace)
-          n_proc += mine && __ballot(open) != 0ull;
-          const unsigned long long blended = __ballot(hit && open);
-          bad |= (hit && open && hit_bad) || (blended != 0ull && mlp_bad);
+          n_proc += mine && open != 0ull;
+          const unsigned long long blended = mask & open;
+          bad |= (blended & hit_bad) | (blended != 0ull ? mlp_bad : 0ull);
           n_proc_hit += blended != 0ull;
           n_hits += __popcll(blended);
         }
-        if (open) {
+        if (lane_in(open)) {
           if (k == 0) {
-            const float w = trans * a;
+            const float w = fmaf(-trans, let, trans);
             cr = fmaf(w, i == 0 ? o[0] : round.colour[i > 0 ? i - 1 : 0][0][l], cr);
             cg = fmaf(w, i == 0 ? o[1] : round.colour[i > 0 ? i - 1 : 0][1][l], cg);
             cb = fmaf(w, i == 0 ? o[2] : round.colour[i > 0 ? i - 1 : 0][2][l], cb);
           }
-          trans = trans * (1.f - a);
+          trans = trans * let;
         }
       }
-      live = valid && (trans >= kTransmittanceFloor);
-      if (__ballot(live) == 0ull) {
+      live = in_image & __ballot(trans >= kTransmittanceFloor);
+      if (live == 0ull) {
         if (todo != 0ull) fast_arrived(q);      // (the next entry's line may still be landing in these registers)
         finished = true;
         break;
@@ -641,7 +679,9 @@ __device__ __forceinline__ void render_tile_team(
     store3(out_rgb, pix, cr, cg, cb);
     out_alpha[pix] = 1.f - trans;
   }
-  if (__ballot(bad) != 0ull && l == 0) atomicExch(status, 1);
+  // (a NaN among the outputs of a hit, which the largest of them does not show)
+  bad |= __ballot(!(__builtin_fabsf((cr + cg) + (cb + trans)) <= 3.4028235e38f));
+  if (bad != 0ull && l == 0) atomicExch(status, 1);
   if (counters && l == 0) {
     atomicAdd(counters + 1, (unsigned long long)n_proc);
     atomicAdd(counters + 2, (unsigned long long)n_proc_hit);

@@ -382,3 +382,44 @@ def test_teams_of_wavefronts_give_the_bits_of_one_wavefront(device, oracle_mod, 
                                           torch.zeros(1500, 4, device=device), 1.5, 2.0, fr.W, fr.H, fr.thr, bf16=bf16)
     assert not bad and float(alpha.max()) > 0.2
     assert torch.equal(rgb, one[0]) and torch.equal(alpha, one[1])
+
+
+@pytest.mark.parametrize("temp", [-2.2, 27.0, 60.0])
+def test_feature_gates_at_temperatures_on_both_sides_of_the_exponents_range(device, oracle_mod, temp):
+    # up to 40 / log2(e) the four exponentials are taken as they stand, beyond it the largest is taken off first
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=600, hidden=32, width=40, height=24, feature_dim=24, feature_slots=4)
+    sc = fr.scene
+    cand, off = fr.oracle_lists(oracle_mod)
+    want = oracle_mod.render_tilecenter(*fr.base_numpy(cand, off), *fr.dims, feat_attr=sc.feat_attr, beta=1.3, temp=temp)
+    t = lambda a: to_dev(a, device)
+    rec = ops.prepare_primitives(t(sc.positions), t(sc.log_scales), t(sc.quats))
+    ro, rd, c, o = t(fr.rays_o), t(fr.rays_d), t(cand), t(off)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8, cull_threshold=fr.thr)
+    _, _, feat, nonfinite = ops.render_tilecenter_mfma_feat(ro, rd, rec, order, o, t(sc.freq), t(sc.att),
+                                                            *[t(w) for w in sc.mlp()], t(sc.feat_attr), 1.3, temp, fr.W,
+                                                            fr.H, fr.thr, bf16=False)
+    scale = float(np.abs(want["feat"]).max())
+    assert not nonfinite and scale > 1e-2
+    assert np.abs(feat.cpu().numpy() - want["feat"]).max() <= TOL[False] * max(1.0, scale)
+
+
+@pytest.mark.parametrize("width,height", [(32, 24), (1024, 640)])
+@pytest.mark.parametrize("row,value", [(0, 3e38), (3, 3e38), (3, -3e38), (1, None)])
+def test_outputs_beyond_f32_are_reported(device, oracle_mod, width, height, row, value):
+    # infinite or NaN outputs of finite weights: on images of teams and of single wavefronts
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=300, hidden=32, width=width, height=height)
+    sc = fr.scene
+    cand, off = fr.oracle_lists(oracle_mod)
+    t = lambda a: to_dev(a, device)
+    rec = ops.prepare_primitives(t(sc.positions), t(sc.log_scales), t(sc.quats))
+    ro, rd, c, o = t(fr.rays_o), t(fr.rays_d), t(cand), t(off)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8, cull_threshold=fr.thr)
+    render = lambda: ops.render_tilecenter_mfma(ro, rd, rec, order, o, t(sc.freq), t(sc.att), *[t(w) for w in sc.mlp()],
+                                                fr.W, fr.H, fr.thr, bf16=True)[2]
+    assert not render()
+    W1, b1, W2, b2, W3, b3 = sc.mlp()
+    b2[:] = 10.0                       # every hidden unit is active
+    W3[:, row] = value if value is not None else np.where(np.arange(32) % 3, 3e38, -3e38)
+    assert render()
