@@ -840,15 +840,21 @@ class TrainFrame:
     """What a differentiable frame keeps between its forward and its backward: the workspace of its steps (one step per
     tile and primitive that hits it) and their number.  ``steps`` is what the backward's launches are sized by;
     ``geometry`` the primitives' records, for the feature loss."""
-    __slots__ = ("workspace", "pairs", "width", "height", "steps", "status", "chunks", "geometry")
+    __slots__ = ("workspace", "pairs", "width", "height", "steps", "status", "chunks", "geometry", "nbytes")
 
     def __init__(self, workspace, pairs, width, height, chunks, status, steps, geometry=None):
         self.workspace, self.pairs, self.width, self.height = workspace, pairs, width, height
         self.chunks, self.status, self.steps, self.geometry = chunks, status, steps, geometry
+        self.nbytes = 0 if workspace is None else workspace.numel()
 
     def with_workspace(self, workspace):
         """The same frame around ``workspace`` (None: to keep the numbers while autograd keeps the tensor)."""
-        return TrainFrame(workspace, self.pairs, self.width, self.height, self.chunks, self.status, self.steps)
+        if workspace is not None and not (workspace.is_cuda and workspace.dtype == torch.uint8 and workspace.dim() == 1
+                                          and workspace.is_contiguous() and workspace.numel() == self.nbytes):
+            raise RuntimeError("the saved steps of this frame must come back as they were saved")
+        frame = TrainFrame(workspace, self.pairs, self.width, self.height, self.chunks, self.status, self.steps)
+        frame.nbytes = self.nbytes
+        return frame
 
 
 def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W, H, threshold, max_hits, pool_steps,
@@ -881,8 +887,15 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
     return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps, records)
 
 
+def _check_step_offsets(frame, tile_offsets):
+    if not (tile_offsets.is_cuda and tile_offsets.dtype == torch.int32 and tile_offsets.is_contiguous()
+            and tile_offsets.numel() == num_tiles(frame.width, frame.height, 8, 8) + 1):
+        raise RuntimeError("tile_offsets must be the contiguous CUDA int32 vector of the frame's forward")
+
+
 def train_group(frame, tile_offsets, n):
     """The steps of ``frame`` sorted by primitive: the scratch buffer of the gradient kernels, its index part filled."""
+    _check_step_offsets(frame, tile_offsets)
     lib = _lib.load()
     nbytes = lib.mlpsp_train_scratch_bytes(frame.steps, n)
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=frame.workspace.device)
@@ -894,6 +907,7 @@ def train_group(frame, tile_offsets, n):
 
 def train_reverse(frame, tile_offsets, grad_rgb, grad_t):
     """(d4 [S, 64, 4], falloff adjoint [S, 64]) of a frame's steps."""
+    _check_step_offsets(frame, tile_offsets)
     dev = frame.workspace.device
     d4 = torch.empty(max(frame.steps, 1), 64, 4, dtype=torch.float32, device=dev)
     falloff = torch.empty(max(frame.steps, 1), 64, dtype=torch.float32, device=dev)
@@ -953,6 +967,11 @@ def train_feature_l1(frame, tile_offsets, attributes, target, beta, temp):
 
 def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoint):
     """d / d attributes of the loss of :func:`train_feature_l1` times ``loss_adjoint`` (f32 device scalar)."""
+    for t in (attributes, loss_adjoint):
+        if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
+            raise RuntimeError("feature attributes and the loss adjoint must be contiguous float32 CUDA tensors")
+    if loss_adjoint.numel() != 1 or attributes[0:1].numel() != (feature.slots * feature.channels if len(attributes) else 0):
+        raise RuntimeError("feature attributes and the loss adjoint do not match the loss they belong to")
     dev = kept.device
     rows = torch.empty(feature.row_bytes, dtype=torch.uint8, device=dev)
     out = torch.empty_like(attributes)

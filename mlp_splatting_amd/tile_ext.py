@@ -547,19 +547,7 @@ class TileExt:
         # any_tile: the backward entry points, whose reference kernels take any square tile of up to 256 pixels
         _chk(width > 0 and height > 0 and (tile in (8, 16) or (any_tile and 0 < tile * tile <= 256)),
              "the records forward supports 8x8 and 16x16 tiles")
-        for i, t in enumerate(x):
-            _chk(t.is_cuda and t.is_contiguous(), "Inputs must be contiguous CUDA tensors")
-            _chk(t.device == x[0].device, "Inputs must share a device")
-            _chk(t.dtype == (torch.int32 if i in (5, 6) else torch.float32),
-                 "Records path requires FP32 inputs and int32 tile lists")
-        pixels, n = width * height, x[2].shape[0]
-        _chk(tuple(x[0].shape) == (pixels, 3) and x[1].shape == x[0].shape)
-        _chk(x[2].dim() == 2 and x[2].shape[1] == 3 and x[3].shape == x[2].shape and tuple(x[4].shape) == (n, 4))
-        _chk(x[7].dim() == 1 and x[8].shape == x[7].shape and x[9].dim() == 3 and x[9].shape[0] == n)
-        h, inp, f = x[9].shape[1], x[9].shape[2], x[7].numel()
-        _chk(0 < h <= 32 and f > 0 and inp == 12 * f)
-        _chk(tuple(x[10].shape) == (n, h) and tuple(x[11].shape) == (n, h, h) and x[12].shape == x[10].shape)
-        _chk(tuple(x[13].shape) == (n, 4, h) and tuple(x[14].shape) == (n, 4))
+        pixels, n = width * height, self._check_training_f32(x, width, height)
         _chk(x[15].shape == x[0].shape and x[16].dim() == 1 and x[16].numel() == pixels)
         with torch.cuda.device(x[0].device), self.uncached():
             self._validate(x[5], x[6], ops.num_tiles(width, height, tile, tile), self.max_tile_prims, n, name)
@@ -572,6 +560,26 @@ class TileExt:
                                        float(threshold), float(beta), float(temp), self.max_hits, name,
                                        render_order=bool(render_order), counts_only=counts_only)
             return out if counts_only else list(out)
+
+    @staticmethod
+    def _check_training_f32(x, width, height):
+        """Argument contract of the exact training forwards (np_tile_kernels.cu:6897-6998): types and shapes of the 15
+        scene tensors, and of the two adjoint placeholders where the entry point takes them.  Returns the primitive
+        count."""
+        for i, t in enumerate(x):
+            _chk(t.is_cuda and t.is_contiguous(), "Inputs must be contiguous CUDA tensors")
+            _chk(t.device == x[0].device, "Inputs must share a device")
+            _chk(t.dtype == (torch.int32 if i in (5, 6) else torch.float32),
+                 "Records path requires FP32 inputs and int32 tile lists")
+        n = x[2].shape[0] if x[2].dim() == 2 else -1
+        _chk(tuple(x[0].shape) == (width * height, 3) and x[1].shape == x[0].shape)
+        _chk(x[2].dim() == 2 and x[2].shape[1] == 3 and x[3].shape == x[2].shape and tuple(x[4].shape) == (n, 4))
+        _chk(x[7].dim() == 1 and x[8].shape == x[7].shape and x[9].dim() == 3 and x[9].shape[0] == n)
+        h, inp, f = x[9].shape[1], x[9].shape[2], x[7].numel()
+        _chk(0 < h <= 32 and f > 0 and inp == 12 * f)
+        _chk(tuple(x[10].shape) == (n, h) and tuple(x[11].shape) == (n, h, h) and x[12].shape == x[10].shape)
+        _chk(tuple(x[13].shape) == (n, 4, h) and tuple(x[14].shape) == (n, 4))
+        return n
 
     @staticmethod
     def records_forward_matches_render(freq, W1, b1, W2, b2, tile):
@@ -594,10 +602,9 @@ class TileExt:
         (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called once the lists are validated."""
         width, height = int(width), int(height)
         _chk(width > 0 and height > 0 and x[0].shape[0] == width * height, "B must equal W*H for tile renderer")
-        self._check_base(*x[:9])
-        for t in x:
-            _chk(t.is_cuda and t.is_contiguous() and t.device == x[0].device, "Inputs must be contiguous CUDA tensors")
-        n = x[2].shape[0]
+        _chk(len(x) == 15, "Expected 15 scene inputs")
+        n = self._check_training_f32(x, width, height)
+        _chk(x[7].numel() == 6 and tuple(x[9].shape[1:]) == (32, 72), "training steps require the 72->32->32->4 MLP")
         n_tiles = ops.num_tiles(width, height, 8, 8)
         with torch.cuda.device(x[0].device), self.uncached():
             self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
@@ -651,12 +658,19 @@ class TileExt:
             raise RuntimeError(f"{name}: tile-center backward hit capacity {int(self.max_hits)} reached before "
                                "transmittance termination; refusing to return truncated gradients")
 
-    @staticmethod
-    def backward_from_steps(frame, groups, x, grad_rgb, grad_t, dtype=torch.float32):
+    @classmethod
+    def backward_from_steps(cls, frame, groups, x, grad_rgb, grad_t, dtype=torch.float32):
         """The nine gradients of :meth:`render_tiles_backward_tilecenter_full` from a frame's steps; ``x``: the scene
         tensors of the forward, ``groups``: ``ops.train_group`` of the frame.  Non-finite policy of
         ``primitive_gemm.grouped_weight_gradients``."""
         from . import primitive_gemm
+        # (what saved-tensor hooks hand back is a tensor of their making: it is held to the forward's contract again)
+        cls._check_training_f32(x, frame.width, frame.height)
+        pixels = frame.width * frame.height
+        for t in (grad_rgb, grad_t):
+            _chk(t.is_cuda and t.is_contiguous() and t.device == x[0].device and t.dtype == torch.float32,
+                 "The image adjoints must be contiguous FP32 CUDA tensors")
+        _chk(tuple(grad_rgb.shape) == (pixels, 3) and grad_t.dim() == 1 and grad_t.numel() == pixels)
         with torch.cuda.device(x[0].device), torch.no_grad():
             d4, falloff = ops.train_reverse(frame, x[6], grad_rgb, grad_t)
 

@@ -131,3 +131,16 @@ def test_unit_quaternions_are_those_of_torch(device):
         grads.append((u.detach(), leaf.grad))
     assert torch.equal(grads[0][0], grads[1][0])
     torch.testing.assert_close(grads[0][1], grads[1][1], rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("backend", ["scalar", "wmma_fp16"])
+def test_feature_training_step_refuses_weights_stored_in_half_precision(device, oracle_mod, monkeypatch, backend):
+    from mlp_splatting_amd.record_training import Frame as TrainingFrame, feature_training_step
+    monkeypatch.setenv("MLPSP_CSR_FORWARD_BACKEND", backend)
+    fr, base = _scene(device, oracle_mod, 40, 33, 17, 1.0, False)
+    target, attributes = torch.zeros(4, 8, 16, device=device), torch.zeros(40, 4, 16, device=device)
+    half = [t.half() if i >= 9 else t for i, t in enumerate(base)]
+    short = [t[:39].contiguous() if i in (11, 13) else t for i, t in enumerate(base)]
+    for bad, text in ((half, "requires FP32 inputs"), (short, None)):
+        with pytest.raises(RuntimeError, match=text):
+            feature_training_step(bad, attributes, target, TrainingFrame(33, 17, fr.thr, 1.5, 2.0))
