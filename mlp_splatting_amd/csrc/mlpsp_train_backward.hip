@@ -50,19 +50,24 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
       b = src[64];
     }
     const float R = va.x, G = va.y, B = va.z, sigma_raw = va.w, trans = vb.x, alpha = vb.y, decay = vb.z;
+    // A lane that the primitive missed holds zeros (a hit's transmittance is at least the floor), and its adjoint may be
+    // anything -- the derivative of a root at a black pixel is infinite --: zeros come of it, not 0 inf.
+    const bool hit = trans != 0.f;
     const float dotg = (g.x * R + g.y * G) + g.z * B;
     const float grad_alpha = trans * (dotg - next);
-    next = next * (1.f - alpha) + dotg * alpha;
+    next = hit ? next * (1.f - alpha) + dotg * alpha : next;
     const float grad_sigma = grad_alpha * det_exp(-sigma_raw * decay);
     const float grad_decay = grad_sigma * sigma_raw;
-    float4 d;
-    d.x = g.x * (trans * alpha) * R * (1.f - R);
-    d.y = g.y * (trans * alpha) * G * (1.f - G);
-    d.z = g.z * (trans * alpha) * B * (1.f - B);
-    d.w = grad_sigma * decay * sigmoid(vb.w);
+    float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (hit) {
+      d.x = g.x * (trans * alpha) * R * (1.f - R);
+      d.y = g.y * (trans * alpha) * G * (1.f - G);
+      d.z = g.z * (trans * alpha) * B * (1.f - B);
+      d.w = grad_sigma * decay * sigmoid(vb.w);
+    }
     const size_t at = (size_t)(base + m) * 64 + l;
     d4[at] = d;
-    falloff[at] = grad_decay * decay;
+    falloff[at] = hit ? grad_decay * decay : 0.f;
   }
 }
 

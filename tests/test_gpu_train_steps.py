@@ -144,3 +144,79 @@ def test_feature_training_step_refuses_weights_stored_in_half_precision(device, 
     for bad, text in ((half, "requires FP32 inputs"), (short, None)):
         with pytest.raises(RuntimeError, match=text):
             feature_training_step(bad, attributes, target, TrainingFrame(33, 17, fr.thr, 1.5, 2.0))
+
+
+def _frame_with_holes(device, oracle_mod):
+    """Small primitives: tiles where some pixels are hit and others by nothing at all."""
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr, base = _scene(device, oracle_mod, 300, 33, 17, 0.35, False)
+    ext = TileExt()
+    x = base + [torch.zeros_like(base[0]), torch.zeros(33 * 17, device=device)]
+    records = ext.render_tiles_training_records(x, 33, 17, 8, fr.thr, 1.5, 2.0, render_order=True)
+    empty = records[7].diff() == 0
+    pixel = torch.arange(33 * 17, device=device)
+    tile = (pixel // 33) // 8 * 5 + (pixel % 33) // 8
+    beside_hits = torch.isin(tile[empty], tile[~empty])
+    assert int(beside_hits.sum()) > 20 and int((~empty).sum()) > 20
+    return fr, base, ext, records, empty
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+def test_pixels_that_nothing_hits_contribute_nothing_whatever_their_adjoint(device, oracle_mod, value, dtype):
+    from mlp_splatting_amd import ops
+    fr, base, ext, records, empty = _frame_with_holes(device, oracle_mod)
+    _, _, frame = ext.train_forward(base, 33, 17, fr.thr)
+    groups = ops.train_group(frame, base[6], 300)
+    torch.manual_seed(5)
+    g_rgb, g_t = torch.randn(33 * 17, 3, device=device), torch.randn(33 * 17, device=device)
+    g_rgb[empty], g_t[empty] = 0.0, 0.0
+    want = ext.backward_from_steps(frame, groups, base, g_rgb, g_t, dtype=dtype)
+    for rgb_too, t_too in ((True, False), (False, True), (True, True)):
+        b_rgb, b_t = g_rgb.clone(), g_t.clone()
+        if rgb_too:
+            b_rgb[empty] = value
+        if t_too:
+            b_t[empty] = value
+        got = ext.backward_from_steps(frame, groups, base, b_rgb, b_t, dtype=dtype)
+        for g, w in zip(got, want):
+            assert torch.equal(g, w) and bool(torch.isfinite(g).all())
+
+
+def test_a_pixel_with_hits_and_a_non_finite_adjoint_is_refused_as_by_the_record_pipeline(device, oracle_mod):
+    from mlp_splatting_amd import ops
+    fr, base, ext, records, empty = _frame_with_holes(device, oracle_mod)
+    _, _, frame = ext.train_forward(base, 33, 17, fr.thr)
+    g_rgb, g_t = torch.zeros(33 * 17, 3, device=device), torch.zeros(33 * 17, device=device)
+    g_rgb[(~empty).nonzero()[0]] = float("inf")
+    with pytest.raises(FloatingPointError):
+        ext.backward_from_records(records, base[2], base[3], base[4], base[7], base[8], *base[9:15], g_rgb, g_t)
+    with pytest.raises(FloatingPointError):
+        ext.backward_from_steps(frame, ops.train_group(frame, base[6], 300), base, g_rgb, g_t)
+
+
+@pytest.mark.parametrize("background", [None, 0.5])
+def test_a_loss_whose_derivative_is_infinite_at_black_pixels_trains(device, background):
+    """rgb ** (1 / 2.2) at an empty pixel on black: an infinite adjoint, which ends there."""
+    from mlp_splatting_amd import synthetic as syn
+    from mlp_splatting_amd.cumodel import NeuralPrimitiveSceneTileCUDA
+    sc = syn.make_scene(300, 32, seed=0, log_scale_mean=-4.0)
+    scene = NeuralPrimitiveSceneTileCUDA(num_primitives=300, hidden_dim=32).to(device)
+    with torch.no_grad():
+        for name, value in zip(("positions", "log_scales", "quats", "W1", "b1", "W2", "b2", "W3", "b3"),
+                               (sc.positions, sc.log_scales, sc.quats, *sc.mlp())):
+            getattr(scene, name).copy_(to_dev(value, device))
+    width, height, focal = 64, 48, 60.0
+    scene.set_image_size(width, height)
+    c2w = syn.look_at((0.2, -0.1, -3.0), (0.0, 0.0, 0.0))
+    ro, rd = (to_dev(a, device) for a in syn.pinhole_rays(width, height, focal, c2w))
+    args = dict(score_threshold=5e-3, view_matrix=to_dev(syn.view_matrix(c2w), device),
+                proj_matrix=to_dev(syn.projection_matrix(focal, width, height), device))
+    rgb = scene(ro, rd, bg_color=None if background is None else (0.0, background, 0.0), **args)
+    empty = (rgb == 0).any(-1)
+    assert 20 < int(empty.sum()) < width * height - 20
+    rgb.retain_grad()
+    (rgb ** (1 / 2.2)).mean().backward()
+    assert not bool(torch.isfinite(rgb.grad[empty]).all())
+    for parameter in (scene.positions, scene.log_scales, scene.quats, scene.W1, scene.b3):
+        assert bool(torch.isfinite(parameter.grad).all()) and float(parameter.grad.abs().max()) > 0
