@@ -18,6 +18,7 @@
 // rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each).  At 200,000 primitives,
 // 1200x680, a 300x170 target of 512 channels: 0.56, 0.07, 0.44 and 0.32 ms; the record kernels took 4.95 ms for the
 // loss and 8.1 ms for the gradient.
+#include <type_traits>
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_train.hpp"
@@ -164,68 +165,85 @@ __global__ __launch_bounds__(64 * kFeatWaves) void train_feature_blend_kernel(
   const int c = (blockIdx.z * (int)(blockDim.x >> 6) + (tid >> 6)) * 256 + (lane & (lpr - 1)) * 4;
   const bool channels = c < f.C;
   float4 acc[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 
-  for (int m = 0; m < count; m += kStepChunk) {
-    const int first = chunk_table[table + (m >> 4)] * kStepChunk, n = min(kStepChunk, count - m), buf = (m >> 4) & 1;
-    for (int i = tid >> 4; i < n; i += (int)(blockDim.x >> 4)) {
-      const int p = ids[first + i];
-      float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-      if (weight != 0.f) {
-        const unsigned char* __restrict__ rec = records + (size_t)(first + i) * kStepBytes;
-        const float2 ta = *reinterpret_cast<const float2*>(rec + kStepPlaneB + px * 16);
-        v[4] = weight * (ta.x * ta.y);
+  // A target of the tile that does not sample a step has a coefficient of 0, and 0 a = 0 unless the attribute a is infinite
+  // or NaN: then the sums below are not finite, and the tile's are formed again without those products (SELECT), so that
+  // such an attribute stays with the targets that sample it.
+  const auto blend = [&](auto select) {
+    constexpr bool SELECT = decltype(select)::value;
+    const auto add = [](float k, float a, float& sum) {
+      const float v = fmaf(k, a, sum);
+      sum = SELECT && k == 0.f ? sum : v;
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int m = 0; m < count; m += kStepChunk) {
+      const int first = chunk_table[table + (m >> 4)] * kStepChunk, n = min(kStepChunk, count - m), buf = (m >> 4) & 1;
+      for (int i = tid >> 4; i < n; i += (int)(blockDim.x >> 4)) {
+        const int p = ids[first + i];
+        float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        if (weight != 0.f) {
+          const unsigned char* __restrict__ rec = records + (size_t)(first + i) * kStepBytes;
+          const float2 ta = *reinterpret_cast<const float2*>(rec + kStepPlaneB + px * 16);
+          v[4] = weight * (ta.x * ta.y);
+          if constexpr (SLOTS != 1) {
+            const float4 d = *reinterpret_cast<const float4*>(rec + kStepPlaneC + px * 16);
+            const PrimRecord& P = prims[p];
+            const Vec3 ql = quat_rotate_conj(P.qw, P.qx, P.qy, P.qz, Vec3{d.x, d.y, d.z});
+            float g[4];
+            tetra_gates(ql.x, ql.y, ql.z, P.lgx, P.lgy, P.lgz, beta, temp, g);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[s] = v[4] * g[s];
+          }
+        }
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+          v[s] += __shfl_xor(v[s], 1);
+          v[s] += __shfl_xor(v[s], 2);
+        }
+        float* __restrict__ keep = o.k + (((size_t)(base + m + i) * (f.NT >> 2) + group) * SLOTS) * 4 + j;
+        const bool writes = blockIdx.z == 0;
         if constexpr (SLOTS != 1) {
-          const float4 d = *reinterpret_cast<const float4*>(rec + kStepPlaneC + px * 16);
-          const PrimRecord& P = prims[p];
-          const Vec3 ql = quat_rotate_conj(P.qw, P.qx, P.qy, P.qz, Vec3{d.x, d.y, d.z});
-          float g[4];
-          tetra_gates(ql.x, ql.y, ql.z, P.lgx, P.lgy, P.lgz, beta, temp, g);
-#pragma unroll
-          for (int s = 0; s < 4; ++s) v[s] = v[4] * g[s];
+          const float mine = (q & 2) ? ((q & 1) ? v[3] : v[2]) : ((q & 1) ? v[1] : v[0]);
+          const int s = q + (SLOTS == 5 ? 1 : 0);
+          s_k[buf][i][s][j] = mine;
+          if (writes) keep[s * 4] = mine;
         }
+        if (SLOTS != 4 && q == 0) {
+          s_k[buf][i][0][j] = v[4];
+          if (writes) keep[0] = v[4];
+        }
+        if ((tid & 15) == 0) s_p[buf][i] = p;
       }
-#pragma unroll
-      for (int s = 0; s < 5; ++s) {
-        v[s] += __shfl_xor(v[s], 1);
-        v[s] += __shfl_xor(v[s], 2);
-      }
-      float* __restrict__ keep = o.k + (((size_t)(base + m + i) * (f.NT >> 2) + group) * SLOTS) * 4 + j;
-      const bool writes = blockIdx.z == 0;
-      if constexpr (SLOTS != 1) {
-        const float mine = (q & 2) ? ((q & 1) ? v[3] : v[2]) : ((q & 1) ? v[1] : v[0]);
-        const int s = q + (SLOTS == 5 ? 1 : 0);
-        s_k[buf][i][s][j] = mine;
-        if (writes) keep[s * 4] = mine;
-      }
-      if (SLOTS != 4 && q == 0) {
-        s_k[buf][i][0][j] = v[4];
-        if (writes) keep[0] = v[4];
-      }
-      if ((tid & 15) == 0) s_p[buf][i] = p;
-    }
-    __syncthreads();
-    if (channels) {
+      __syncthreads();
+      if (channels) {
 #pragma unroll 4
-      for (int i = sub; i < n; i += nsub) {
-        const float* __restrict__ src = attr + (size_t)s_p[buf][i] * SLOTS * f.C;
+        for (int i = sub; i < n; i += nsub) {
+          const float* __restrict__ src = attr + (size_t)s_p[buf][i] * SLOTS * f.C;
 #pragma unroll
-        for (int s = 0; s < SLOTS; ++s) {
-          const float4 a = four_channels<VEC>(src + (size_t)s * f.C, c, f.C);
-          const float4 k = *reinterpret_cast<const float4*>(&s_k[buf][i][s][0]);
-          acc[0].x = fmaf(k.x, a.x, acc[0].x), acc[0].y = fmaf(k.x, a.y, acc[0].y);
-          acc[0].z = fmaf(k.x, a.z, acc[0].z), acc[0].w = fmaf(k.x, a.w, acc[0].w);
-          acc[1].x = fmaf(k.y, a.x, acc[1].x), acc[1].y = fmaf(k.y, a.y, acc[1].y);
-          acc[1].z = fmaf(k.y, a.z, acc[1].z), acc[1].w = fmaf(k.y, a.w, acc[1].w);
-          acc[2].x = fmaf(k.z, a.x, acc[2].x), acc[2].y = fmaf(k.z, a.y, acc[2].y);
-          acc[2].z = fmaf(k.z, a.z, acc[2].z), acc[2].w = fmaf(k.z, a.w, acc[2].w);
-          acc[3].x = fmaf(k.w, a.x, acc[3].x), acc[3].y = fmaf(k.w, a.y, acc[3].y);
-          acc[3].z = fmaf(k.w, a.z, acc[3].z), acc[3].w = fmaf(k.w, a.w, acc[3].w);
+          for (int s = 0; s < SLOTS; ++s) {
+            const float4 a = four_channels<VEC>(src + (size_t)s * f.C, c, f.C);
+            const float4 k = *reinterpret_cast<const float4*>(&s_k[buf][i][s][0]);
+            add(k.x, a.x, acc[0].x), add(k.x, a.y, acc[0].y);
+            add(k.x, a.z, acc[0].z), add(k.x, a.w, acc[0].w);
+            add(k.y, a.x, acc[1].x), add(k.y, a.y, acc[1].y);
+            add(k.y, a.z, acc[1].z), add(k.y, a.w, acc[1].w);
+            add(k.z, a.x, acc[2].x), add(k.z, a.y, acc[2].y);
+            add(k.z, a.z, acc[2].z), add(k.z, a.w, acc[2].w);
+            add(k.w, a.x, acc[3].x), add(k.w, a.y, acc[3].y);
+            add(k.w, a.z, acc[3].z), add(k.w, a.w, acc[3].w);
+          }
         }
       }
     }
-  }
+  };
+  blend(std::false_type{});
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    finite &= __builtin_fabsf(acc[i].x) <= 3.4028235e38f && __builtin_fabsf(acc[i].y) <= 3.4028235e38f &&
+              __builtin_fabsf(acc[i].z) <= 3.4028235e38f && __builtin_fabsf(acc[i].w) <= 3.4028235e38f;
+  if (__syncthreads_or(!finite)) blend(std::true_type{});
   for (int d = lpr; d < 64; d <<= 1) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -220,3 +220,40 @@ def test_a_loss_whose_derivative_is_infinite_at_black_pixels_trains(device, back
     assert not bool(torch.isfinite(rgb.grad[empty]).all())
     for parameter in (scene.positions, scene.log_scales, scene.quats, scene.W1, scene.b3):
         assert bool(torch.isfinite(parameter.grad).all()) and float(parameter.grad.abs().max()) > 0
+
+
+@pytest.mark.parametrize("channels,slots", [(8, 4), (67, 5), (300, 1)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, value, channels, slots):
+    """A primitive that hits a tile, but none of the pixels that the tile's targets take: its attributes reach no target."""
+    from mlp_splatting_amd import ops
+    fr, base, ext, records, empty = _frame_with_holes(device, oracle_mod)
+    wf, hf = 8, 4
+    taps = []
+    for size, low in ((33, wf), (17, hf)):
+        at = ((torch.arange(low, device=device) + 0.5) * (size / low) - 0.5).clamp_min(0).long()
+        taps.append(torch.cat([at, (at + 1).clamp_max(size - 1)]).unique())
+    sampled = torch.zeros(17, 33, dtype=torch.bool, device=device)
+    sampled[taps[1][:, None], taps[0][None, :]] = True
+    pixel = torch.repeat_interleave(torch.arange(33 * 17, device=device), records[7].diff())
+    is_hit, is_sampled = torch.zeros(300, dtype=torch.bool, device=device), torch.zeros(300, dtype=torch.bool, device=device)
+    is_hit[records[2].long()] = True
+    is_sampled[records[2].long()[sampled.reshape(-1)[pixel]]] = True
+    others = is_hit & ~is_sampled
+    assert int(others.sum()) > 5 and int(is_sampled.sum()) > 5
+    gen = torch.Generator(device=device).manual_seed(11)
+    attributes = torch.randn(300, slots, channels, device=device, generator=gen)
+    attributes[others] = 0.0
+    target = torch.randn(hf, wf, channels, device=device, generator=gen)
+    _, _, frame = ext.train_forward(base, 33, 17, fr.thr, render_order=False)
+    groups, one, results = ops.train_group(frame, base[6], 300), torch.ones((), device=device), []
+    for fill in (0.0, value):
+        attributes[others] = fill
+        used = attributes[:, 0].contiguous() if slots == 1 else attributes
+        loss, feature, kept = ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)
+        results.append((loss, ops.train_feature_gradients(frame, groups, feature, kept, used, one)))
+    assert torch.equal(results[0][0], results[1][0]) and bool(torch.isfinite(results[1][0]))
+    assert torch.equal(results[0][1], results[1][1]) and bool(torch.isfinite(results[1][1]).all())
+    attributes[is_sampled] = value
+    used = attributes[:, 0].contiguous() if slots == 1 else attributes
+    assert not bool(torch.isfinite(ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)[0]))
