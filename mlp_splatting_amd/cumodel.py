@@ -314,10 +314,9 @@ class _TileRenderAutogradFn(torch.autograd.Function):
                     records, args[2], args[3], args[4], args[7], args[8], *args[9:15], grad_out_rgb, grad_t_end)
         elif ctx.frame is not None:
             frame = ctx.frame.with_workspace(kept[0])
-            with torch.cuda.device(args[0].device):
-                groups = ops.train_group(frame, args[6], args[2].shape[0])
-                gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.backward_from_steps(frame, groups, args, grad_out_rgb,
-                                                                                   grad_t_end)
+            groups = ops.train_group(frame, args[6], args[2].shape[0])
+            gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.backward_from_steps(frame, groups, args, grad_out_rgb,
+                                                                               grad_t_end)
         else:
             gW1, gb1, gW2, gb2, gW3, gb3, gp, gs, gq = ext.render_tiles_backward_tilecenter_full(
                 *args, grad_out_rgb, grad_t_end, *ctx.dims)

@@ -547,8 +547,7 @@ class TileExt:
         # any_tile: the backward entry points, whose reference kernels take any square tile of up to 256 pixels
         _chk(width > 0 and height > 0 and (tile in (8, 16) or (any_tile and 0 < tile * tile <= 256)),
              "the records forward supports 8x8 and 16x16 tiles")
-        pixels, n = width * height, self._check_training_f32(x, width, height)
-        _chk(x[15].shape == x[0].shape and x[16].dim() == 1 and x[16].numel() == pixels)
+        n = self._check_training_f32(x, width, height)
         with torch.cuda.device(x[0].device), self.uncached():
             self._validate(x[5], x[6], ops.num_tiles(width, height, tile, tile), self.max_tile_prims, n, name)
             rec = self._records(x[2], x[3], x[4])
@@ -566,19 +565,20 @@ class TileExt:
         """Argument contract of the exact training forwards (np_tile_kernels.cu:6897-6998): types and shapes of the 15
         scene tensors, and of the two adjoint placeholders where the entry point takes them.  Returns the primitive
         count."""
-        for i, t in enumerate(x):
-            _chk(t.is_cuda and t.is_contiguous(), "Inputs must be contiguous CUDA tensors")
-            _chk(t.device == x[0].device, "Inputs must share a device")
-            _chk(t.dtype == (torch.int32 if i in (5, 6) else torch.float32),
-                 "Records path requires FP32 inputs and int32 tile lists")
-        n = x[2].shape[0] if x[2].dim() == 2 else -1
-        _chk(tuple(x[0].shape) == (width * height, 3) and x[1].shape == x[0].shape)
-        _chk(x[2].dim() == 2 and x[2].shape[1] == 3 and x[3].shape == x[2].shape and tuple(x[4].shape) == (n, 4))
-        _chk(x[7].dim() == 1 and x[8].shape == x[7].shape and x[9].dim() == 3 and x[9].shape[0] == n)
-        h, inp, f = x[9].shape[1], x[9].shape[2], x[7].numel()
-        _chk(0 < h <= 32 and f > 0 and inp == 12 * f)
-        _chk(tuple(x[10].shape) == (n, h) and tuple(x[11].shape) == (n, h, h) and x[12].shape == x[10].shape)
-        _chk(tuple(x[13].shape) == (n, 4, h) and tuple(x[14].shape) == (n, 4))
+        index, f32, i32 = x[0].get_device(), torch.float32, torch.int32
+        for i, t in enumerate(x):       # (twice in a training step, whose host time shows where the frame is small)
+            if index < 0 or t.get_device() != index or not t.is_contiguous() or t.dtype is not (i32 if i in (5, 6) else f32):
+                _chk(t.is_cuda and t.is_contiguous(), "Inputs must be contiguous CUDA tensors")
+                _chk(t.device == x[0].device, "Inputs must share a device")
+                raise RuntimeError("Records path requires FP32 inputs and int32 tile lists")
+        pixels, n, f = width * height, x[2].shape[0] if x[2].dim() == 2 else -1, x[7].numel()
+        h = x[9].shape[1] if x[9].dim() == 3 else -1
+        _chk(0 < h <= 32 and f > 0)
+        want = ((pixels, 3), (pixels, 3), (n, 3), (n, 3), (n, 4), None, None, (f,), (f,), (n, h, 12 * f), (n, h), (n, h, h),
+                (n, h), (n, 4, h), (n, 4), (pixels, 3), (pixels,))
+        for t, shape in zip(x, want):
+            if shape is not None and t.shape != shape:
+                raise RuntimeError("Expected condition to be true")
         return n
 
     @staticmethod
@@ -606,7 +606,7 @@ class TileExt:
         n = self._check_training_f32(x, width, height)
         _chk(x[7].numel() == 6 and tuple(x[9].shape[1:]) == (32, 72), "training steps require the 72->32->32->4 MLP")
         n_tiles = ops.num_tiles(width, height, 8, 8)
-        with torch.cuda.device(x[0].device), self.uncached():
+        with _on_device(x[0].device), self.uncached():
             self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
             if accept is not None:
                 accept()
@@ -667,11 +667,10 @@ class TileExt:
         # (what saved-tensor hooks hand back is a tensor of their making: it is held to the forward's contract again)
         cls._check_training_f32(x, frame.width, frame.height)
         pixels = frame.width * frame.height
-        for t in (grad_rgb, grad_t):
-            _chk(t.is_cuda and t.is_contiguous() and t.device == x[0].device and t.dtype == torch.float32,
-                 "The image adjoints must be contiguous FP32 CUDA tensors")
-        _chk(tuple(grad_rgb.shape) == (pixels, 3) and grad_t.dim() == 1 and grad_t.numel() == pixels)
-        with torch.cuda.device(x[0].device), torch.no_grad():
+        for t, shape in ((grad_rgb, (pixels, 3)), (grad_t, (pixels,))):
+            _chk(t.get_device() == x[0].get_device() and t.is_contiguous() and t.dtype is torch.float32 and t.shape == shape,
+                 "The image adjoints must be contiguous FP32 CUDA tensors [B, 3] and [B]")
+        with _on_device(x[0].device), torch.no_grad():
             d4, falloff = ops.train_reverse(frame, x[6], grad_rgb, grad_t)
 
             def launch(operand_dtype, scale):

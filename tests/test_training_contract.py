@@ -4,7 +4,7 @@ import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
-from mlp_splatting_amd import ops
+from mlp_splatting_amd import ops, tile_ext
 from mlp_splatting_amd.tile_ext import TileExt
 
 W, H, N = 20, 12, 7
@@ -41,6 +41,7 @@ def ext(monkeypatch):
         def __exit__(self, *_a):
             pass
     monkeypatch.setattr(torch.cuda, "device", NoDevice)
+    monkeypatch.setattr(tile_ext, "_on_device", NoDevice)
     return ext
 
 
