@@ -539,10 +539,10 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  * mlpsp_train_forward_f32 / _mfma: image, alpha and the steps of the lists order_dev (num_pairs entries, sorted by
  *   mlpsp_sort_tiles with the t* key).  render_order as in mlpsp_records_count; max_hits as there.  workspace_dev:
  *   mlpsp_train_workspace_bytes(num_pairs, width, height, pool_steps) bytes, 256-byte aligned (pool_steps < 0: the worst
- *   case).  Its first three int32 words are for the caller to read: {chunks of 16 steps the frame needs, status bits
+ *   case).  Its first three int32 words are for the caller to read: {chunks of MLPSP_STEP_CHUNK steps the frame needs, status bits
  *   (1 = non-finite offset, activation, output or colour -- not reported by the f32 forward in the render's order --,
  *   2 = a live pixel reached max_hits), steps}.
- *   If 16 times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
+ *   If MLPSP_STEP_CHUNK times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
  *   the caller repeats the call with a pool of that size.
  * mlpsp_train_reverse: reverse compositing; d4_dev [num_steps, 64, 4] = adjoints of the four pre-activation outputs,
  *   falloff_dev [num_steps, 64] = dL/d(decay) * decay.
@@ -556,6 +556,7 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  *   and temp as in the record forward.  mlpsp_train_feature_bytes returns the size of kept_dev (what the gradients need,
  *   256-byte aligned) and fills share_bytes (shares_dev, scratch of the loss), loss_partials (floats; their sum is the loss)
  *   and row_bytes (rows_dev, scratch of the gradients); 0 = invalid shape.  scratch_dev: filled by mlpsp_train_group. */
+#define MLPSP_STEP_CHUNK 8
 size_t mlpsp_train_workspace_bytes(int64_t num_pairs, int width, int height, int64_t pool_steps);
 int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
                             const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,

@@ -21,6 +21,7 @@ PIXEL_HIT_CAPACITY = 256
 PRIM_RECORD_BYTES = 128
 MFMA_PACK_BYTES = 7808
 VERSION = 303      # MLPSP_VERSION of include/mlpsp.h: the interface this binding was written against
+STEP_CHUNK = 8
 STAGE_STATUS_IS_CLEAR = 4
 STAGE_FRAMES_OVERLAP = 8
 

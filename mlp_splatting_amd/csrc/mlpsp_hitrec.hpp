@@ -24,6 +24,11 @@ namespace mlpsp {
 constexpr int kHitChunk = 16;
 constexpr int kHitGrab = 4;      // chunks a wavefront draws from the pool per atomic
 
+struct HitGroups {               // as mlpsp_team.hpp takes them
+  static constexpr int kLog2 = 4;
+  __host__ __device__ static constexpr int slots(int) { return kHitChunk * kHitGrab; }
+};
+
 struct HitPool {
   int32_t* counters;
   int32_t* item_hits;

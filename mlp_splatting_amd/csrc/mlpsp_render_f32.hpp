@@ -316,7 +316,7 @@ __device__ __forceinline__ void render_team_item_f32(
   const int start = offsets[tile], end = offsets[tile + 1];
   PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
-  TeamSlots slots{wslot * hp.table_stride + (start >> 4) + tile, 0, 0};
+  TeamSlots slots{wslot * hp.table_stride + (start >> 4) + tile, 0, 0, 0, 0};
   if (k == 0) encode_direction(rd.x, rd.y, rd.z, freq, att, s.dir);
 
   int p_mine = 0;
@@ -377,7 +377,7 @@ __device__ __forceinline__ void render_team_item_f32(
           }
         }
         if constexpr (EMIT > 0) {
-          const int rs = team_slot<kHitGrab, true>(slots, kept, mine, k, lane, hp.counters, hp.chunk_table, hp.pool_chunks, s.chunk);
+          const int rs = team_slot<HitGroups, true>(slots, kept, mine, k, lane, hp.counters, hp.chunk_table, hp.pool_chunks, s.chunk);
           if (rs >= 0) {
             float* __restrict__ rec = reinterpret_cast<float*>(hp.records + (size_t)rs * hp.record_bytes);
             rec[lane] = w_mine;

@@ -80,30 +80,35 @@ __device__ __forceinline__ void walk_team_f32(const int32_t* __restrict__ order,
   }
 }
 
-// Slots of a pool that hands out chunks of 16 in groups (mlpsp_hitrec.hpp, mlpsp_train.hpp), drawn by a team: the entries of
-// a round that are kept get consecutive numbers in list order; a round that begins a new group lets wavefront 0 draw it
-// (one atomic and one barrier per group).
+// Slots of a pool that hands out chunks in groups (mlpsp_hitrec.hpp, mlpsp_train.hpp), drawn by a team: the entries of a
+// round that are kept get consecutive numbers in list order; a round that begins a new group lets wavefront 0 draw it (one
+// atomic and one barrier per group).  GROUPS: kLog2, of the slots of a chunk, and slots(n), of the group that begins at
+// number n; no fewer than a team has wavefronts, so that a round begins one chunk and one group at most.
 struct TeamSlots {
   int table_base, count, chunk;      // chunk: first of the current group, -1 once the pool is exhausted
+  int begin, end;                    // the numbers of the current group
 };
 // kept: entries of the round that are kept; mine: rank of this wavefront's entry among them, -1 if it is not.  Returns its
 // slot, -1 if there is none.  Called by the whole team.  STOPS: nothing is counted once the pool is exhausted
 // (counters[1] = 1 says so); else the draws go on.
-template <int GRAB, bool STOPS>
+template <typename GROUPS, bool STOPS>
 __device__ __forceinline__ int team_slot(TeamSlots& w, int kept, int mine, int k, int l, int32_t* __restrict__ counters,
                                          int32_t* __restrict__ chunk_table, int pool_chunks, int& s_chunk) {
-  constexpr int kGroup = 16 * GRAB;
+  constexpr int kLog2 = GROUPS::kLog2, kChunk = 1 << kLog2;
   if (kept == 0 || (STOPS && w.chunk < 0)) return -1;
   const int before = w.count, after = before + kept;
-  const int group = (before + kGroup - 1) & ~(kGroup - 1), entry = (before + 15) & ~15;   // next beginnings at or behind `before`
-  const int old_chunk = w.chunk;
+  const int group = w.end, entry = (before + kChunk - 1) & ~(kChunk - 1);   // next beginnings at or behind `before`
+  const int old_chunk = w.chunk, old_begin = w.begin;
   w.count = after;
   if (group < after) {
+    const int draw = GROUPS::slots(group) >> kLog2;
     team_barrier();                  // (the number drawn before has been read by all)
-    if (k == 0 && l == 0) s_chunk = atomicAdd(counters, GRAB);
+    if (k == 0 && l == 0) s_chunk = atomicAdd(counters, draw);
     team_barrier();
     w.chunk = __builtin_amdgcn_readfirstlane(s_chunk);
-    if (w.chunk + GRAB > pool_chunks) {
+    w.begin = group;
+    w.end = group + (draw << kLog2);
+    if (w.chunk + draw > pool_chunks) {
       w.chunk = -1;
       if (STOPS) {
         w.count = group;
@@ -113,12 +118,12 @@ __device__ __forceinline__ int team_slot(TeamSlots& w, int kept, int mine, int k
   }
   const auto chunk_of = [&](int number) {
     const int c = number >= group ? w.chunk : old_chunk;
-    return c < 0 ? -1 : c + ((number & (kGroup - 1)) >> 4);
+    return c < 0 ? -1 : c + ((number - (number >= group ? group : old_begin)) >> kLog2);
   };
-  if (entry < after && k == 0 && l == 0 && chunk_of(entry) >= 0) chunk_table[w.table_base + (entry >> 4)] = chunk_of(entry);
+  if (entry < after && k == 0 && l == 0 && chunk_of(entry) >= 0) chunk_table[w.table_base + (entry >> kLog2)] = chunk_of(entry);
   if (mine < 0) return -1;
   const int chunk = chunk_of(before + mine);
-  return chunk < 0 ? -1 : chunk * 16 + ((before + mine) & 15);
+  return chunk < 0 ? -1 : (chunk << kLog2) + ((before + mine) & (kChunk - 1));
 }
 
 }  // namespace mlpsp

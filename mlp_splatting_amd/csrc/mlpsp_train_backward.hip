@@ -36,7 +36,7 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
   const int pix = valid ? (y * W + x) : 0;
   const Float3 g = valid ? load3(grgb, pix) : Float3{0.f, 0.f, 0.f};
   float next = valid ? gt[pix] : 0.f;
-  const int table = (offsets[tile] >> 4) + tile;
+  const int table = step_table(offsets[tile], tile);
   const auto planes = [&](int m) {
     return reinterpret_cast<const float4*>(records + (size_t)step_slot(chunk_table, table, m) * kStepBytes) + l;
   };
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void step_list_kernel(const int32_t* __restric
                                                         int T, int W, int ntx, int32_t* __restrict__ keys, int4* __restrict__ info) {
   const int tile = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
   if (tile >= T) return;
-  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = (offsets[tile] >> 4) + tile;
+  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = step_table(offsets[tile], tile);
   const int pixel = (tile / ntx) * 8 * W + (tile % ntx) * 8;
   for (int m = lane; m < count; m += 64) {
     const int slot = step_slot(chunk_table, table, m);

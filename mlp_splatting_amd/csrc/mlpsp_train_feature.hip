@@ -53,6 +53,7 @@ __host__ __device__ inline AxisSpan feature_axis_span(int tile, float scale, int
   return AxisSpan{lo, hi - lo};
 }
 
+constexpr int kBlendSteps = 16;     // steps per round of a blend workgroup
 constexpr int kFeatWaves = 4;       // wavefronts of a blend workgroup, 256 channels each, at most
 
 struct FeatShape {
@@ -129,8 +130,8 @@ __device__ __forceinline__ float4 four_channels(const float* __restrict__ row, i
 // and the 4, 2 or 1 lane groups of a wavefront take steps in turn.
 inline int lanes_per_row_log2(int Cp) { return Cp <= 64 ? 4 : Cp <= 128 ? 5 : 6; }
 
-// One workgroup = one tile, four of its targets (blockIdx.y), up to 1,024 channels (blockIdx.z).  Sixteen steps at a time
-// (a chunk of the pool): every group of 16 lanes computes k of one step -- lane = (target, tap), the taps' sum two DPP
+// One workgroup = one tile, four of its targets (blockIdx.y), up to 1,024 channels (blockIdx.z).  Sixteen steps at a time:
+// every group of 16 lanes computes k of one step -- lane = (target, tap), the taps' sum two DPP
 // adds --, then every lane adds the sixteen steps to its four channels.
 template <int SLOTS, bool VEC>
 __global__ __launch_bounds__(64 * kFeatWaves) void train_feature_blend_kernel(
@@ -138,15 +139,15 @@ __global__ __launch_bounds__(64 * kFeatWaves) void train_feature_blend_kernel(
     const int32_t* __restrict__ chunk_table, const int32_t* __restrict__ ids, const unsigned char* __restrict__ records,
     const PrimRecord* __restrict__ prims, const float* __restrict__ attr, int lpr_log2, float beta, float temp,
     float* __restrict__ shares) {
-  __shared__ __attribute__((aligned(16))) float s_k[2][kStepChunk][SLOTS][4];
-  __shared__ int s_p[2][kStepChunk];
+  __shared__ __attribute__((aligned(16))) float s_k[2][kBlendSteps][SLOTS][4];
+  __shared__ int s_p[2][kBlendSteps];
   const int tile = superblock_tile(blockIdx.x, f.ntx, f.nty);
   if (tile < 0) return;
   const int group = blockIdx.y, tx = tile % f.ntx, ty = tile / f.ntx, tid = threadIdx.x, lane = tid & 63;
   const int2 col = o.columns[tx], row = o.rows[ty];
   const int nt = col.y * row.y;
   if (group * 4 >= nt) return;
-  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = (offsets[tile] >> 4) + tile;
+  const int base = tile_base[tile], count = tile_base[tile + 1] - base, table = step_table(offsets[tile], tile);
 
   // this lane's target and tap
   const int q = tid & 3, j = (tid >> 2) & 3, t = group * 4 + j;
@@ -177,13 +178,13 @@ __global__ __launch_bounds__(64 * kFeatWaves) void train_feature_blend_kernel(
     };
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int m = 0; m < count; m += kStepChunk) {
-      const int first = chunk_table[table + (m >> 4)] * kStepChunk, n = min(kStepChunk, count - m), buf = (m >> 4) & 1;
+    for (int m = 0; m < count; m += kBlendSteps) {
+      const int n = min(kBlendSteps, count - m), buf = (m / kBlendSteps) & 1;
       for (int i = tid >> 4; i < n; i += (int)(blockDim.x >> 4)) {
-        const int p = ids[first + i];
+        const int slot = step_slot(chunk_table, table, m + i), p = ids[slot];
         float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
         if (weight != 0.f) {
-          const unsigned char* __restrict__ rec = records + (size_t)(first + i) * kStepBytes;
+          const unsigned char* __restrict__ rec = records + (size_t)slot * kStepBytes;
           const float2 ta = *reinterpret_cast<const float2*>(rec + kStepPlaneB + px * 16);
           v[4] = weight * (ta.x * ta.y);
           if constexpr (SLOTS != 1) {

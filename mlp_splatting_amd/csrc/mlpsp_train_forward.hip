@@ -181,7 +181,7 @@ __device__ __forceinline__ void train_tile_team(const int tile, const int k, con
   float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
   int used = 0, p_mine = 0;
   bool over = false, bad = false, lane_bad = false, mlp_bad = false;
-  TeamSlots slots{(start >> 4) + tile, 0, 0};
+  TeamSlots slots{step_table(start, tile), 0, 0, 0, 0};
   TrainEntry e{};
   walk_team_f32<TEAM>(
       c.order, start, end, c.N, c.prims, t.valid, t.ro.x, t.ro.y, t.ro.z, t.rd.x, t.rd.y, t.rd.z, c.thr, s.walk, k, l,
@@ -227,7 +227,7 @@ __device__ __forceinline__ void train_tile_team(const int tile, const int k, con
           over |= t.valid && (trans >= kTransmittanceFloor) && (used >= c.max_hits);
         }
         if constexpr (CHECKED) bad |= (hit_mine && lane_bad) || (mine >= 0 && mlp_bad);
-        const int slot = team_slot<kStepGrab, false>(slots, kept, mine, k, l, sp.head, sp.chunk_table, sp.pool_chunks, s.chunk);
+        const int slot = team_slot<StepGroups, false>(slots, kept, mine, k, l, sp.head, sp.chunk_table, sp.pool_chunks, s.chunk);
         train_store(sp, slot, l, p_mine, hit_mine, before, e);
         return __ballot(t.valid && (trans >= kTransmittanceFloor)) != 0ull;
       });
@@ -243,6 +243,7 @@ __device__ __forceinline__ void train_tile_team(const int tile, const int k, con
 // A wavefront per tile, four tiles to a workgroup, but for the last ones: the workgroups from `body` on (per XCD) take a tile
 // each, as a team.
 constexpr int kTrainTeam = 4;
+static_assert(kTrainTeam <= kStepChunk, "a round of a team begins one chunk at most");
 template <typename T, bool REC>
 __device__ __forceinline__ void train_forward_body(const TrainScene& c, const StepPool& sp, const TrainOut& out, int body) {
   union Lds {
@@ -356,7 +357,9 @@ int train_scan(const TrainFrame& f, hipStream_t s) {
 MLPSP_API size_t mlpsp_train_workspace_bytes(int64_t num_pairs, int width, int height, int64_t pool_steps) {
   const int64_t T = checked_num_tiles(width, height, 8, 8);
   if (T <= 0 || num_pairs < 0) return 0;
-  const int64_t worst = num_pairs + (int64_t)(kStepChunk * kStepGrab - 1) * T + kStepChunk * kStepGrab;
+  // k steps of a tile take up to k + 31 slots, and no more than the larger of a chunk and 2 k
+  const int64_t full = num_pairs + (int64_t)(StepGroups::kMost - 1) * T, sparse = 2 * num_pairs + (int64_t)kStepChunk * T;
+  const int64_t worst = (full < sparse ? full : sparse) + StepGroups::kMost;
   if (pool_steps < 0 || pool_steps > worst) pool_steps = worst;
   return step_pool_bytes(num_pairs, T, pool_steps);
 }

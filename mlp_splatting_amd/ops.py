@@ -881,9 +881,10 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
                                                 _stream(dev))
         _check(code, "mlpsp_train_forward")
         chunks, status, steps = workspace[:12].view(torch.int32).tolist()
-        if chunks * 16 <= pool_steps or pool_steps < 0:
+        if chunks * _lib.STEP_CHUNK <= pool_steps or pool_steps < 0:
             break
-        pool_steps = chunks * 16
+        pool_steps = chunks * _lib.STEP_CHUNK
+        del workspace                       # (too small: its memory is free for the next)
     return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps, records)
 
 

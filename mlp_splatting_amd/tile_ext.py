@@ -82,7 +82,7 @@ class TileExt:
         self._binned = None
         self._queue_capacity = 0          # candidate-buffer estimate of render_frame_queued (0: not seeded yet)
         self._queue_scratch_scale = 1
-        self._steps_per_tile = 96         # room the differentiable frame makes for its steps (see train_forward)
+        self._steps_per_tile = None       # room the differentiable frame makes for its steps (see train_forward)
 
     # ------------------------------------------------------------------------------------------
     # derived-tensor caches (geometry records, matrix-core operand copies)
@@ -616,13 +616,20 @@ class TileExt:
                 order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
                                           self.max_tile_prims, cull_threshold=float(threshold))
             packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
+            # Room for the steps: for the first frame as its lists suggest (a step per 13 entries at the 200,000-primitive
+            # 1200x680 frame, per three or four where primitives are small), then as the frames before needed.  A frame
+            # that needs more is repeated; the bound on what its lists can need is never exceeded.
             with self._lock:
-                pool = n_tiles * self._steps_per_tile
+                room = self._steps_per_tile
+            if room is None:
+                room = min(96.0, 0.5 * x[5].numel() / n_tiles + _lib.STEP_CHUNK)
+            pool = int(n_tiles * room)
             rgb, alpha, frame = ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height,
                                                   float(threshold), self.max_hits, pool, render_order=render_order,
                                                   packed=packed, bf16=precision == "bfloat16")
-            with self._lock:      # a quarter more than this frame needed, in whole chunks, for the next one
-                self._steps_per_tile = max(16, -(-frame.chunks * 20 // n_tiles))
+            needed = 1.25 * frame.chunks * _lib.STEP_CHUNK / n_tiles
+            with self._lock:      # a quarter more than was needed; an eighth less with every frame that needs less
+                self._steps_per_tile = max(needed, 0.875 * (self._steps_per_tile or 0.0))
         return rgb, alpha, frame
 
     def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision):

@@ -50,6 +50,7 @@ def test_status_constants_agree_with_the_header():
     assert int(consts["TILE_CAPACITY_MAX"]) == _lib.TILE_CAPACITY_MAX
     assert int(consts["PIXEL_HIT_CAPACITY"]) == _lib.PIXEL_HIT_CAPACITY == 256
     assert int(consts["PRIM_RECORD_BYTES"]) == _lib.PRIM_RECORD_BYTES
+    assert int(consts["STEP_CHUNK"]) == _lib.STEP_CHUNK
     assert int(consts["VERSION"]) == _lib.VERSION == _lib.load().mlpsp_version()
 
 

@@ -257,3 +257,62 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
     attributes[is_sampled] = value
     used = attributes[:, 0].contiguous() if slots == 1 else attributes
     assert not bool(torch.isfinite(ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)[0]))
+
+
+@pytest.mark.parametrize("width,height", [(61, 40), (328, 325)])       # every tile by a team; most by one wavefront
+def test_tiles_of_every_length_take_the_chunks_they_need(device, width, height):
+    """Lists of 0 to 97 primitives that all hit their tile: the steps, and the pool's chunks, of one tile beside another at
+    and around the ends of the groups that a tile draws; image and gradients as the records give them."""
+    import numpy as np
+    from mlp_splatting_amd import _lib, ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    n, tiles = 97, ((width + 7) // 8) * ((height + 7) // 8)
+    lengths = np.array([1, 8, 9, 0, 7, 16, 17, 31, 32, 33, 2, 63, 64, 65, 96, 97, 15, 4])[np.arange(tiles) % 18]
+    sc = syn.make_scene(n, 32, seed=3, log_scale_mean=1.2)
+    sc.positions[:, 2] += 6.0
+    sc.b3[:, 3] = -6.0
+    c2w = syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0))
+    ro, rd = syn.pinhole_rays(width, height, float(width), c2w)
+    cand = np.concatenate([np.arange(k) for k in lengths]).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats, cand, off, sc.freq,
+                                        sc.att, *sc.mlp())]
+    ext = TileExt()
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0, render_order=True)
+    rgb, alpha, frame = ext.train_forward(base, width, height, 1e-3)
+    assert frame.status == 0 and torch.equal(rgb, records[0]) and torch.equal(alpha, records[1])
+    # (the primitives of a tile that hit it, as the records have them: the lists but for a few at the image's border)
+    pixel = torch.repeat_interleave(torch.arange(width * height, device=device), records[7].diff())
+    tile = (pixel // width) // 8 * ((width + 7) // 8) + (pixel % width) // 8
+    steps = torch.bincount((tile * n + records[2]).unique() // n, minlength=tiles).cpu().numpy()
+    assert (steps <= lengths).all() and (steps == lengths).mean() > 0.9
+    assert frame.steps == steps.sum()
+    ends = np.array([0, 8, 16, *range(32, 129, 32)])
+    assert frame.chunks * _lib.STEP_CHUNK == ends[np.searchsorted(ends, steps)].sum()
+    torch.manual_seed(6)
+    g_rgb, g_t = torch.randn(width * height, 3, device=device), torch.randn(width * height, device=device)
+    want = ext.backward_from_records(records, base[2], base[3], base[4], base[7], base[8], *base[9:15], g_rgb, g_t)
+    got = ext.backward_from_steps(frame, ops.train_group(frame, base[6], n), base, g_rgb, g_t)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert float((g - w).norm()) <= 1e-4 * float(w.norm()), i      # (up to 107,000 records of a primitive, f32 sums)
+    # the same frame from a pool that is too small at first
+    ext._steps_per_tile = 3.0
+    again, _, frame = ext.train_forward(base, width, height, 1e-3)
+    assert torch.equal(again, rgb) and frame.steps == steps.sum()
+    for g, w in zip(ext.backward_from_steps(frame, ops.train_group(frame, base[6], n), base, g_rgb, g_t), got):
+        assert torch.equal(g, w)
+
+
+def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
+    """Storage follows the steps, not the tiles: a tile with a hit takes a chunk, and the first frame reserves no more than
+    its lists can need."""
+    from mlp_splatting_amd import _lib
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr, base = _scene(device, oracle_mod, 300, 160, 120, 0.2, False)
+    _, _, frame = TileExt().train_forward(base, 160, 120, fr.thr)
+    assert frame.steps > 50
+    slots = frame.chunks * _lib.STEP_CHUNK
+    assert slots <= 2 * frame.steps + _lib.STEP_CHUNK * min(frame.steps, 300)
+    pairs = base[5].numel()
+    assert frame.nbytes <= (2 * pairs + _lib.STEP_CHUNK * 300 + 32) * 3400 + 65536
