@@ -20,7 +20,7 @@ TILE_CAPACITY_MAX = 2048
 PIXEL_HIT_CAPACITY = 256
 PRIM_RECORD_BYTES = 128
 MFMA_PACK_BYTES = 7808
-VERSION = 303      # MLPSP_VERSION of include/mlpsp.h: the interface this binding was written against
+VERSION = 400      # MLPSP_VERSION of include/mlpsp.h: the interface this binding was written against
 STEP_CHUNK = 8
 STAGE_STATUS_IS_CLEAR = 4
 STAGE_FRAMES_OVERLAP = 8
@@ -132,6 +132,13 @@ def load():
             f"libmlpsp_hip.so not found at {LIB_PATH}; build it with `make -C {CSRC_DIR}` "
             "(there is no CPU or PyTorch fallback for the renderer)")
     lib = C.CDLL(LIB_PATH)
+    try:         # first of all: a library of another version has other functions, or the same with other arguments
+        found = lib.mlpsp_version()
+    except AttributeError:
+        found = "unknown"
+    if found != VERSION:
+        raise RuntimeError(f"libmlpsp_hip.so is version {found}, this binding expects {VERSION}: "
+                           f"rebuild the library (`make -C {CSRC_DIR}`)")
     for name, (restype, argtypes) in SIGNATURES.items():
         try:
             fn = getattr(lib, name)
@@ -139,9 +146,6 @@ def load():
             raise RuntimeError(f"libmlpsp_hip.so does not export {name}; rebuild the library") from exc
         fn.restype = restype
         fn.argtypes = argtypes
-    if lib.mlpsp_version() != VERSION:
-        raise RuntimeError(f"libmlpsp_hip.so is version {lib.mlpsp_version()}, this binding expects {VERSION}: "
-                           f"rebuild the library (`make -C {CSRC_DIR}`)")
     _lib = lib
     return lib
 

@@ -83,3 +83,32 @@ def test_product_sources_never_reach_into_the_oracle():
                 text = open(os.path.join(dirpath, f)).read()
                 assert not re.search(r"^\s*(import|from)\s+oracle\b", text, flags=re.M), f
                 assert "oracle/" not in text and "mlpsp_oracle" not in text, f
+
+
+def _interface_digest():
+    """Of the header's declarations and constants, the version itself left out."""
+    import hashlib
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "mlpsp.h")).read(), flags=re.S)
+    text = re.sub(r"#define\s+MLPSP_VERSION\s+\d+", "", text)
+    return hashlib.sha256(" ".join(text.split()).encode()).hexdigest()[:16]
+
+
+def test_a_changed_interface_has_a_version_of_its_own():
+    """Whoever adds, drops or changes a declaration of include/mlpsp.h raises MLPSP_VERSION (and _lib.VERSION), and puts the
+    digest of the new interface here."""
+    from mlp_splatting_amd import _lib
+    assert (_lib.VERSION, _interface_digest()) == (400, "c51b72a39265e9ec")
+
+
+@pytest.mark.parametrize("version", [303, None])
+def test_a_library_of_another_version_is_refused_by_its_version(monkeypatch, version):
+    """Before any function is looked up that it may not have."""
+    from mlp_splatting_amd import _lib
+
+    class Older:
+        if version is not None:
+            mlpsp_version = staticmethod(lambda: version)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib.C, "CDLL", lambda path: Older())
+    with pytest.raises(RuntimeError, match=f"is version {version or 'unknown'}, this binding expects {_lib.VERSION}"):
+        _lib.load()
