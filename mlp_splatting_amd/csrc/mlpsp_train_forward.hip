@@ -282,14 +282,23 @@ __global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu
 }
 #undef MLPSP_TRAIN_PARAMS
 #undef MLPSP_TRAIN_TAIL
-// As many teams at the end as there are workgroups on the chip; all tiles where they are hardly more.
+// A team for each of the last 1,024 tiles, and for every tile of an image of up to 2,048: the launch then ends with tiles that
+// last a third as long.  Forward in us, f32 / fp16 operands, a wavefront per tile, 1,024 teams, teams throughout:
+//     300 tiles    641 / 245        294 / 125        294 / 125
+//   1,200         1,242 / 426        992 / 369        877 / 303
+//   1,530                            818 / 322        754 / 272
+//   1,900                          1,097 / 393      1,010 / 332
+//   2,214         1,194 / 424      1,049 / 361      1,093 / 370
+//   4,800         1,783 / 639      1,666 / 572      2,091 / 671
+//  12,750         4,211 / 1,356    3,977 / 1,307    5,396 / 1,695
+// 768 and 1,536 teams are within 3 % of 1,024 from 3,000 tiles on.
 struct TrainPlan {
   int body;
   unsigned grid;
 };
 inline TrainPlan train_plan(int ntx, int nty, int64_t T) {
   const int per_xcd = (int)(superblock_grid(ntx, nty) / kNumXcd);
-  const int teams = T <= 1280 ? per_xcd : min(per_xcd, 1024 / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
+  const int teams = T <= 2048 ? per_xcd : min(per_xcd, 1024 / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
   return TrainPlan{body, (unsigned)(kNumXcd * (body + per_xcd - kTrainTeam * body))};
 }
 

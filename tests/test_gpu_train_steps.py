@@ -259,7 +259,8 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
     assert not bool(torch.isfinite(ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)[0]))
 
 
-@pytest.mark.parametrize("width,height", [(61, 40), (328, 325)])       # every tile by a team; most by one wavefront
+# every tile by a team (40 and 1,681 tiles), then most by one wavefront (2,050 tiles, in rows of 50 and one of 2,050)
+@pytest.mark.parametrize("width,height", [(61, 40), (328, 325), (400, 325), (16397, 5)])
 def test_tiles_of_every_length_take_the_chunks_they_need(device, width, height):
     """Lists of 0 to 97 primitives that all hit their tile: the steps, and the pool's chunks, of one tile beside another at
     and around the ends of the groups that a tile draws; image and gradients as the records give them."""
