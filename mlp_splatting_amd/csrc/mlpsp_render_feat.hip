@@ -213,10 +213,17 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
   hipLaunchKernelGGL((feat_accumulate_kernel<SL, PX>), dim3(superblock_grid(g.ntx, g.nty) * (unsigned)wpt,            \
                      (unsigned)ceil_div(feat_channels, 8 * PX)), dim3(256), 0, s, feat_attr_dev, feat_channels, hp,   \
                      tile_offsets_dev, g, wpt, out_feat_dev)
-  // 16 pixels per wavefront unless the rows are long and the launch fills the chip anyway: whole frames in us with 32 / 16
-  // pixels, 333x251 (1,344 items) 67 channels 1250 / 1185, 512 channels 1545 / 1521; 640x480 (4,800 items) 64 channels
-  // 2685 / 2515, 256 channels 2920 / 2945, 512 channels 3630 / 3795 (4240 with 64 pixels).
-  const bool sixteen = feat_channels <= 128 || items <= 2048;
+  // 16 pixels per wavefront unless the rows are long and the launch fills the chip anyway: four times the wavefronts for
+  // four times the row fetches.  Render and product in us with 16 / 32 pixels (runs differ by about 1 %):
+  //    items   64 channels      128           192           256           384           512
+  //    1,200   1,019 / 1,111  1,010 / 1,109  1,114 / 1,134  1,108 / 1,137  1,203 / 1,287  1,304 / 1,342
+  //    2,640   1,428 / 1,537  1,441 / 1,545  1,637 / 1,673  1,651 / 1,693  1,869 / 1,948  2,083 / 2,085
+  //    3,500   1,821 / 1,928  1,821 / 1,927  2,118 / 2,132  2,103 / 2,134  2,438 / 2,496  2,741 / 2,659
+  //    4,800   2,360 / 2,525  2,417 / 2,552  2,815 / 2,775  2,812 / 2,778  3,268 / 3,329  3,713 / 3,560
+  //    8,190   3,569 / 3,763  3,542 / 3,759  4,337 / 4,135  4,321 / 4,153  5,078 / 5,051  5,764 / 5,439
+  //   12,750   5,408 / 5,678  5,464 / 5,659  6,602 / 6,404  6,667 / 6,380  7,847 / 7,722  8,970 / 8,389
+  // (384 channels are one and a half of the 256 that a workgroup of 32-pixel wavefronts takes.)
+  const bool sixteen = feat_channels <= 128 || items <= 3072;
   if (feat_slots == 4) {
     if (sixteen) MLPSP_ACC_LAUNCH(4, 16); else MLPSP_ACC_LAUNCH(4, 32);
   } else if (feat_slots == 5) {

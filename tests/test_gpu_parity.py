@@ -700,11 +700,13 @@ def test_feature_render_is_bit_exact(device, oracle_mod, slots, channels):
     _assert_bits(feat, want["feat"], "feat")
 
 
+# 2,120 tiles; 3,300, where more than 128 channels take 32 pixels per wavefront
+@pytest.mark.parametrize("width,height", [(421, 317), (521, 397)])
 @pytest.mark.parametrize("slots,channels", [(4, 129), (5, 256), (1, 257)])
-def test_feature_pixels_per_wavefront_give_the_same_bits(device, oracle_mod, slots, channels):
-    """Over 2048 tiles and 128 channels a wavefront takes 32 pixels; the same channels in pieces take it 16."""
+def test_feature_pixels_per_wavefront_give_the_same_bits(device, oracle_mod, slots, channels, width, height):
+    """Over 3,072 tiles and 128 channels a wavefront takes 32 pixels; the same channels in pieces take it 16."""
     from mlp_splatting_amd import ops
-    fr = Frame("cfg1_5k_160x120", n=900, width=421, height=317, feature_dim=channels, feature_slots=max(slots, 4))
+    fr = Frame("cfg1_5k_160x120", n=900, width=width, height=height, feature_dim=channels, feature_slots=max(slots, 4))
     sc = fr.scene
     fa = sc.feat_attr if slots > 1 else np.ascontiguousarray(sc.feat_attr[:, 0])
     cand, off = fr.oracle_lists(oracle_mod)
