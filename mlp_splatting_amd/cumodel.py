@@ -579,7 +579,9 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         hit = cache.get(name)
         if hit is None or hit[0] != key:
             with torch.inference_mode(False), torch.no_grad():
-                hit = (key, build())
+                # (the sources are kept with the value: an address names a tensor only while its memory is not free for
+                # another, whose address, version and shape would match)
+                hit = (key, build(), tuple(sources))
             cache[name] = hit
         return hit[1]
 

@@ -512,3 +512,19 @@ def test_harness_renders_times_and_scores_a_view(device, oracle_mod):
     assert q["per_view_psnr_db"][0] == float("inf") and abs(q["per_view_psnr_db"][1] - 20.0) < 1e-4
     st = harness.timing_stats([harness.render_view(scene, *frame)[1] for _ in range(5)])
     assert st["samples"] == 5 and st["mean_ms"] > 0 and st["std_ms"] >= 0
+
+
+def test_derived_tensors_follow_a_replaced_tensor_at_a_recycled_address(device):
+    """What is cached belongs to the tensor it was made from, not to whatever lies at its address later."""
+    from mlp_splatting_amd.cumodel import NeuralPrimitiveSceneTileCUDA
+    scene = NeuralPrimitiveSceneTileCUDA(num_primitives=4).to(device)
+    weights, parameters = scene.encoder._buffers, scene._parameters
+    plain = scene._frequency_tables(device)[1].clone()
+    for step in range(1, 5):
+        # (the allocator hands a freed block to the next tensor of its size)
+        weights["runtime_frequency_weights"] = None
+        weights["runtime_frequency_weights"] = torch.full((6,), 0.1 * step, device=device)
+        torch.testing.assert_close(scene._frequency_tables(device)[1], plain * 0.1 * step)
+        parameters["quats"] = None
+        parameters["quats"] = torch.nn.Parameter(torch.full((4, 4), 1.0, device=device).cumsum(1) ** step)
+        torch.testing.assert_close(scene._unit_quats(), torch.nn.functional.normalize(scene.quats.detach(), dim=-1))
