@@ -41,7 +41,7 @@ def _loss_geometry(attributes, target, record_tensors, width, height):
              "feature master attributes must be contiguous FP32"),
             (target.dtype in (torch.float16, torch.float32), "feature target must be FP16 or FP32"),
             (on_one_gpu, "feature tensors and records must share a CUDA device"),
-            (slots in (1, 4, 5) and shape_ok and attributes.shape[-1] == target.shape[-1],
+            (attributes.ndim in (2, 3) and slots in (1, 4, 5) and shape_ok and attributes.shape[-1] == target.shape[-1],
              "feature shape does not match the 1/4/5-slot renderer"),
             (shape_ok and target.shape[0] <= height and target.shape[1] <= width,
              "streamed feature loss supports downsampling only")):

@@ -144,3 +144,15 @@ def test_the_backward_takes_the_offsets_attributes_and_adjoint_of_its_forward(mo
         for bad in (one.double(), torch.empty(2, device="cuda"), one.cpu()):
             with pytest.raises(RuntimeError):
                 ops.train_feature_gradients(frame, kept, Feature, kept, attributes, bad)
+
+
+@pytest.mark.parametrize("shape", [(6,), (N, 2, 2, 6)])
+def test_the_streamed_loss_refuses_attributes_that_are_no_rows_of_channels(shape):
+    """One axis would be read as [N, C] past its end."""
+    from mlp_splatting_amd.record_feature_loss import _loss_geometry
+    with FakeTensorMode():
+        image, target = torch.empty(W * H, 3, device="cuda"), torch.empty(2, 3, 6, device="cuda")
+        assert _loss_geometry(torch.empty(N, 6, device="cuda"), target, (image,), W, H) == (2, 3, 6, 1)
+        assert _loss_geometry(torch.empty(N, 5, 6, device="cuda"), target, (image,), W, H) == (2, 3, 6, 5)
+        with pytest.raises(ValueError, match="1/4/5-slot renderer"):
+            _loss_geometry(torch.empty(shape, device="cuda"), target, (image,), W, H)
