@@ -1238,8 +1238,8 @@ MLPSP_API int mlpsp_bin_legacy_count(const float* positions_dev, const float* lo
   const BinScratch b = carve(scratch_dev, scratch_bytes, num_primitives, num_views, g.nsx * g.nsy, g.NC);
   counts_out[0] = counts_out[1] = 0;
   if (num_primitives == 0) {
-    MLPSP_HIP_TRY(hipMemsetAsync(tile_offsets_dev, 0, (size_t)(T + 1) * sizeof(int32_t), s));
-    MLPSP_HIP_TRY(hipMemsetAsync(b.totals, 0, 4 * sizeof(long long), s));
+    MLPSP_HIP_TRY(clear_async(tile_offsets_dev, (size_t)(T + 1) * sizeof(int32_t), s));
+    MLPSP_HIP_TRY(clear_async(b.totals, 4 * sizeof(long long), s));
     return MLPSP_OK;
   }
   const int erc = enqueue_bin_count(positions_dev, log_scales_dev, num_primitives, view_matrices_host, num_views,
@@ -1275,8 +1275,8 @@ int bin_legacy_async_impl(const float* positions_dev, const float* log_scales_de
   const BinGeom g = make_geom(num_primitives, num_views, width, height, tile);
   const BinScratch b = carve(scratch_dev, scratch_bytes, num_primitives, num_views, g.nsx * g.nsy, g.NC);
   if (num_primitives == 0) {
-    MLPSP_HIP_TRY(hipMemsetAsync(tile_offsets_dev, 0, (size_t)(T + 1) * sizeof(int32_t), s));
-    MLPSP_HIP_TRY(hipMemsetAsync(counts_dev, 0, 4 * sizeof(int64_t), s));
+    MLPSP_HIP_TRY(clear_async(tile_offsets_dev, (size_t)(T + 1) * sizeof(int32_t), s));
+    MLPSP_HIP_TRY(clear_async(counts_dev, 4 * sizeof(int64_t), s));
     return MLPSP_OK;
   }
   const int erc = enqueue_bin_count(positions_dev, log_scales_dev, num_primitives, view_matrices_host, num_views,
@@ -1332,9 +1332,9 @@ MLPSP_API int mlpsp_bin_segments_async_device_matrices(const float* positions_de
   const BinGeom g = make_geom(num_primitives, 1, width, height, tile);
   const BinScratch b = carve(scratch_dev, scratch_bytes, num_primitives, 1, g.nsx * g.nsy, g.NC);
   if (num_primitives == 0) {        // every list empty: [0, 0)
-    MLPSP_HIP_TRY(hipMemsetAsync(tile_offsets_dev, 0, (size_t)(T + 1) * sizeof(int32_t), s));
-    MLPSP_HIP_TRY(hipMemsetAsync(tile_ends_dev, 0, (size_t)T * sizeof(int32_t), s));
-    MLPSP_HIP_TRY(hipMemsetAsync(counts_dev, 0, 4 * sizeof(int64_t), s));
+    MLPSP_HIP_TRY(clear_async(tile_offsets_dev, (size_t)(T + 1) * sizeof(int32_t), s));
+    MLPSP_HIP_TRY(clear_async(tile_ends_dev, (size_t)T * sizeof(int32_t), s));
+    MLPSP_HIP_TRY(clear_async(counts_dev, 4 * sizeof(int64_t), s));
     return MLPSP_OK;
   }
   const int erc = enqueue_bin_count(positions_dev, log_scales_dev, num_primitives, nullptr, 1, nullptr, nullptr, width,

@@ -288,7 +288,7 @@ MLPSP_API int mlpsp_validate_tile_lists(const int32_t* tile_offsets_dev, const i
     return MLPSP_E_ARGUMENT;
   if (num_candidates > 0 && !candidates_dev) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(status_dev, 0, 2 * sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(status_dev, 2 * sizeof(int32_t), s));
   const int64_t work = num_tiles > num_candidates ? num_tiles : num_candidates;
   int64_t blocks = (work + 255) / 256;
   if (blocks > 4096) blocks = 4096;

@@ -304,7 +304,7 @@ MLPSP_API int mlpsp_reduce_partials(const float* partial_dev, const int64_t* gro
                                     float* out_dev, int32_t* nonfinite_dev, mlpsp_stream_t stream) {
   if (!nonfinite_dev || num_primitives < 0) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(nonfinite_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(nonfinite_dev, sizeof(int32_t), s));
   ReduceDest dest{};
   dest.packed = out_dev;
   return segment_reduce<false>(partial_dev, group_primitives_dev, group_offsets_dev, num_groups, num_primitives,
@@ -317,7 +317,7 @@ MLPSP_API int mlpsp_reduce_partials_split(const float* partial_dev, const int64_
                                           float* gb3_dev, int32_t* nonfinite_dev, mlpsp_stream_t stream) {
   if (!nonfinite_dev || num_primitives < 0) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(nonfinite_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(nonfinite_dev, sizeof(int32_t), s));
   ReduceDest dest{};
   float* parts[6] = {gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
   for (int i = 0; i < 6; ++i) dest.part[i] = parts[i];

@@ -21,6 +21,25 @@
 
 namespace mlpsp {
 
+// Zeros in place of hipMemsetAsync: as a node of a captured graph a memset has left wrong contents on replays after the
+// first, and every entry point but those that read back may be captured.  W: the widest word that pointer and size allow.
+template <typename W>
+__global__ __launch_bounds__(256) void clear_kernel(W* __restrict__ p, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = W{};
+}
+inline hipError_t clear_async(void* dev, size_t bytes, hipStream_t s) {
+  if (bytes == 0) return hipSuccess;
+  const auto launch = [&](auto* p) {
+    const size_t n = bytes / sizeof(*p), blocks = (n + 255) / 256;
+    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, s, p, n);
+    return hipGetLastError();
+  };
+  const uintptr_t bits = (uintptr_t)dev | (uintptr_t)bytes;
+  if ((bits & 15) == 0) return launch((uint4*)dev);
+  if ((bits & 3) == 0) return launch((uint32_t*)dev);
+  return launch((unsigned char*)dev);
+}
+
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // tiles_x * tiles_y with the overflow checks of np_tile_kernels.cu:4542-4551; 0 if unusable.

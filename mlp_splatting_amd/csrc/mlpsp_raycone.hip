@@ -172,7 +172,7 @@ MLPSP_API int mlpsp_bin_raycone_count(const float* rays_o_dev, const float* rays
   const RayconeScratch sc = rc_carve(scratch_dev, (int)T);
   const int ntx = ceil_div(width, tile);
   const float mult = (float)sqrt(-2.0 * log((double)threshold));
-  MLPSP_HIP_TRY(hipMemsetAsync(scratch_dev, 0, 256, s));
+  MLPSP_HIP_TRY(clear_async(scratch_dev, 256, s));
   hipLaunchKernelGGL(raycone_tiles_kernel, dim3(ceil_div((int)T, 256)), dim3(256), 0, s, rays_o_dev, rays_d_dev, width,
                      height, tile, ntx, (int)T, sc.cones, sc.flags);
   MLPSP_LAUNCH_CHECK();

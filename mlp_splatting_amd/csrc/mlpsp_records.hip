@@ -207,7 +207,7 @@ MLPSP_API int mlpsp_records_count(const float* rays_o_dev, const float* rays_d_d
                                   int32_t* overflow_dev, mlpsp_stream_t stream) {
   if (!counts_dev || !overflow_dev) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(overflow_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(overflow_dev, sizeof(int32_t), s));
   return records_launch(false, rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,
                         num_frequencies, W1, b1, W2, b2, W3, b3, num_primitives, hidden, width, height, tile_w, tile_h,
                         threshold, max_hits, render_order, 0.f, 0.f, counts_dev, overflow_dev, RecordOut{}, s);

@@ -301,7 +301,7 @@ MLPSP_API int mlpsp_all_finite(const float* const* arrays_dev, const int64_t* le
     ++in.count;
   }
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(flag_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(flag_dev, sizeof(int32_t), s));
   if (in.count == 0) return MLPSP_OK;
   const long long want = (largest / 4 + 255) / 256;
   const unsigned blocks = (unsigned)(want < 1 ? 1 : (want > 8192 ? 8192 : want));

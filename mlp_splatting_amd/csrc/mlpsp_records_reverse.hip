@@ -176,9 +176,9 @@ MLPSP_API int mlpsp_records_reverse(const int32_t* ids_dev, const int64_t* pixel
   hipStream_t s = (hipStream_t)stream;
   if (num_primitives > 0) {
     if (!grad_positions_dev || !grad_log_scales_dev || !grad_quats_dev) return MLPSP_E_ARGUMENT;
-    MLPSP_HIP_TRY(hipMemsetAsync(grad_positions_dev, 0, sizeof(float) * 3 * (size_t)num_primitives, s));
-    MLPSP_HIP_TRY(hipMemsetAsync(grad_log_scales_dev, 0, sizeof(float) * 3 * (size_t)num_primitives, s));
-    MLPSP_HIP_TRY(hipMemsetAsync(grad_quats_dev, 0, sizeof(float) * 4 * (size_t)num_primitives, s));
+    MLPSP_HIP_TRY(clear_async(grad_positions_dev, sizeof(float) * 3 * (size_t)num_primitives, s));
+    MLPSP_HIP_TRY(clear_async(grad_log_scales_dev, sizeof(float) * 3 * (size_t)num_primitives, s));
+    MLPSP_HIP_TRY(clear_async(grad_quats_dev, sizeof(float) * 4 * (size_t)num_primitives, s));
   }
   if (num_pixels == 0) return MLPSP_OK;
   if (!pixel_offsets_dev || !grad_rgb_dev || !grad_t_dev) return MLPSP_E_ARGUMENT;

@@ -172,7 +172,7 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
   const int rec_bytes = 64 * 4 * (feat_slots > 1 ? 5 : 1);
   const HitPool hp = hitpool_carve(workspace_dev, workspace_bytes, num_pairs, T, wpt, rec_bytes);
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(hp.counters, 0, 64 * sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(hp.counters, 64 * sizeof(int32_t), s));
   const int per_xcd = (int)((items + kNumXcd - 1) / kNumXcd);
   TileGeom g{width, height, tile_w, tile_h, ceil_div(width, tile_w), ceil_div(height, tile_h)};
   const dim3 grid((unsigned)(per_xcd * kNumXcd)), block(64);

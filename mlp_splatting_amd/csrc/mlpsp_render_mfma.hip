@@ -1145,7 +1145,7 @@ MLPSP_API int mlpsp_pack_mfma_weights_listed(const float* W1, const float* b1, c
   if (num_primitives == 0 || num_pairs == 0) return MLPSP_OK;
   if (!order_dev || !wanted_dev) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(wanted_dev, 0, (size_t)num_primitives, s));
+  MLPSP_HIP_TRY(clear_async(wanted_dev, (size_t)num_primitives, s));
   const int64_t blocks = (num_pairs + 1023) / 1024;
   hipLaunchKernelGGL(mark_listed_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, order_dev,
                      (long long)num_pairs, num_primitives, wanted_dev);
@@ -1184,7 +1184,7 @@ int pack_feat_from(const S* feat_attr_dev, int num_primitives, int feat_slots, i
   if (num_primitives < 0 || feat_channels <= 0 || feat_channels > 512 ||
       !(feat_slots == 1 || feat_slots == 4 || feat_slots == 5) || !status_dev)
     return MLPSP_E_ARGUMENT;
-  MLPSP_HIP_TRY(hipMemsetAsync(status_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(status_dev, sizeof(int32_t), s));
   if (num_primitives == 0) return MLPSP_OK;
   if (!feat_attr_dev || !packed_feat_dev || reinterpret_cast<uintptr_t>(packed_feat_dev) % 16 != 0) return MLPSP_E_ARGUMENT;
   const size_t total = (size_t)num_primitives * feat_channels;
@@ -1247,9 +1247,9 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
         workspace_bytes < hitpool_min_bytes(num_pairs, T, 1))
       return MLPSP_E_SCRATCH;
     hp = hitpool_carve(workspace_dev, workspace_bytes, num_pairs, T, 1, 64 * 2 * feat_pad(feat_slots));
-    if (stage != 2) MLPSP_HIP_TRY(hipMemsetAsync(hp.counters, 0, 64 * sizeof(int32_t), s));
+    if (stage != 2) MLPSP_HIP_TRY(clear_async(hp.counters, 64 * sizeof(int32_t), s));
   }
-  if (stage != 2 && !status_is_clear) MLPSP_HIP_TRY(hipMemsetAsync(status_dev, 0, 16 * sizeof(int32_t), s));
+  if (stage != 2 && !status_is_clear) MLPSP_HIP_TRY(clear_async(status_dev, 16 * sizeof(int32_t), s));
   const int per_xcd = (int)((T + kNumXcd - 1) / kNumXcd);
   const int ntx = ceil_div(width, 8);
   const int32_t* ends = tile_ends_dev ? tile_ends_dev : tile_offsets_dev + 1;

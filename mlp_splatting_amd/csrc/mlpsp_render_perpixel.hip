@@ -322,7 +322,7 @@ MLPSP_API int mlpsp_render_per_pixel_f32(
   int32_t* flag = reinterpret_cast<int32_t*>(workspace_dev);
   float* ws_t = reinterpret_cast<float*>(static_cast<char*>(workspace_dev) + 256);
   int32_t* ws_k = reinterpret_cast<int32_t*>(ws_t + (size_t)items * 64 * kHitCap);
-  MLPSP_HIP_TRY(hipMemsetAsync(flag, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(flag, sizeof(int32_t), s));
   TileGeom g{width, height, tile_w, tile_h, ceil_div(width, tile_w), ceil_div(height, tile_h)};
   MlpPtrs m{W1, b1, W2, b2, W3, b3};
   const dim3 grid((unsigned)items), block(64);
@@ -378,7 +378,7 @@ int records_per_pixel_launch(const float* rays_o_dev, const float* rays_d_dev, c
   int32_t* flag = reinterpret_cast<int32_t*>(workspace_dev);
   float* ws_t = reinterpret_cast<float*>(static_cast<char*>(workspace_dev) + 256);
   int32_t* ws_k = reinterpret_cast<int32_t*>(ws_t + (size_t)items * 64 * kHitCap);
-  MLPSP_HIP_TRY(hipMemsetAsync(flag, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(flag, sizeof(int32_t), s));
   TileGeom g{width, height, tile_w, tile_h, ceil_div(width, tile_w), ceil_div(height, tile_h)};
   MlpPtrs m{W1, b1, W2, b2, W3, b3};
   const dim3 grid((unsigned)items), block(64);

@@ -843,7 +843,7 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
     return MLPSP_E_ARGUMENT;
   const StepPool sp = step_pool_carve(const_cast<void*>(workspace_dev), workspace_bytes, num_pairs, T);
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(nonfinite_dev, 0, sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(nonfinite_dev, sizeof(int32_t), s));
   const StepIndex ix{t.prim, t.first, t.step};
   const GradRows grads{gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
   const GeoGrads geo{grad_positions_dev, grad_log_scales_dev, grad_quats_dev};

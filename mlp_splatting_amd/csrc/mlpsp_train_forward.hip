@@ -389,7 +389,7 @@ MLPSP_API int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays
   if (num_primitives > 0 && (!prim_records_dev || !W1 || !b1 || !W2 || !b2 || !W3 || !b3)) return MLPSP_E_ARGUMENT;
   if (((uintptr_t)W1 | (uintptr_t)b1 | (uintptr_t)W2 | (uintptr_t)b2) & 15u) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(f.sp.head, 0, 64 * sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(f.sp.head, 64 * sizeof(int32_t), s));
   const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
 #define MLPSP_TRAIN_LAUNCH(REC)                                                                                        \
   hipLaunchKernelGGL(train_forward_f32_kernel<REC>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \
@@ -418,7 +418,7 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
   if (num_primitives > 0 && (!prim_records_dev || !packed_dev)) return MLPSP_E_ARGUMENT;
   if (((uintptr_t)prim_records_dev % 128) != 0 || ((uintptr_t)packed_dev % 16) != 0) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
-  MLPSP_HIP_TRY(hipMemsetAsync(f.sp.head, 0, 64 * sizeof(int32_t), s));
+  MLPSP_HIP_TRY(clear_async(f.sp.head, 64 * sizeof(int32_t), s));
   const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
 #define MLPSP_TRAIN_LAUNCH(T)                                                                                          \
   hipLaunchKernelGGL(train_forward_mfma_kernel<T>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \

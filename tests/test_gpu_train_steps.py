@@ -317,3 +317,43 @@ def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
     assert slots <= 2 * frame.steps + _lib.STEP_CHUNK * min(frame.steps, 300)
     pairs = base[5].numel()
     assert frame.nbytes <= (2 * pairs + _lib.STEP_CHUNK * 300 + 32) * 3400 + 65536
+
+
+def test_captured_launches_replay_like_eager_ones(device, oracle_mod):
+    """The launches between two read-backs of a training step, and a matrix-core render, as a captured graph: every replay,
+    with eager work in between, gives what the eager calls give, and flags that one replay raised are down in the next."""
+    from mlp_splatting_amd import _lib, ops
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr, base = _scene(device, oracle_mod, 300, 33, 17, 1.0, False)
+    ext, mlp = TileExt(), base[9:15]
+    _, alpha, frame = ext.train_forward(base, 33, 17, fr.thr)
+    rec = ops.prepare_primitives(*base[2:5])
+    order, _ = ops.sort_tiles(base[0], base[1], rec, base[5], base[6], 33, 17, 8, 8, _lib.KEY_TSTAR)
+    packed = ops.pack_mfma_weights(*mlp)
+    g_rgb, g_t = torch.zeros(33 * 17, 3, device=device), torch.zeros(33 * 17, device=device)
+
+    def launches():
+        groups = ops.train_group(frame, base[6], 300)
+        d4, falloff = ops.train_reverse(frame, base[6], g_rgb, g_t)
+        grads, flag = ops.train_gradients(frame, groups, d4, falloff, base[1], base[7], base[8], mlp, base[3], base[4], 0, 1.0)
+        image = ops.render_tilecenter_mfma(base[0], base[1], rec, order, base[6], base[7], base[8], *mlp, 33, 17, fr.thr,
+                                           packed=packed, check=False)
+        return [*grads, flag, *image]
+    launches()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = launches()
+    hit = int((alpha.reshape(-1) > 0).nonzero()[0])
+    gen = torch.Generator(device=device).manual_seed(8)
+    for replay in range(5):
+        g_rgb.copy_(torch.randn(33 * 17, 3, device=device, generator=gen))
+        g_t.copy_(torch.randn(33 * 17, device=device, generator=gen))
+        if replay % 2:
+            g_rgb[hit] = float("inf")
+        want = launches()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert int(captured[9]) == int(want[9]) == replay % 2 and not int(captured[12][0])
+        for got, expected in zip(captured[:9] + captured[10:12], want[:9] + want[10:12]):
+            assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(expected))
