@@ -85,6 +85,8 @@ class _UnitQuats(torch.autograd.Function):
         if grad is None:
             return None
         quats, = ctx.saved_tensors
+        if not (quats.is_cuda and quats.dtype == torch.float32 and quats.is_contiguous() and quats.shape == grad.shape):
+            raise RuntimeError("the saved quaternions must come back as they were saved")
         grad, out = grad.contiguous(), torch.empty_like(quats)
         grad = grad.clone() if grad.data_ptr() % 16 else grad
         with torch.cuda.device(quats.device):
