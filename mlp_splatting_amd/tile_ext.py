@@ -628,8 +628,10 @@ class TileExt:
                                                   float(threshold), self.max_hits, pool, render_order=render_order,
                                                   packed=packed, bf16=precision == "bfloat16")
             needed = 1.25 * frame.chunks * _lib.STEP_CHUNK / n_tiles
-            with self._lock:      # a quarter more than was needed; an eighth less with every frame that needs less
-                self._steps_per_tile = max(needed, 0.875 * (self._steps_per_tile or 0.0))
+            # A quarter more than was needed, a sixty-fourth less with every frame that needs less: a training set's cameras
+            # come in any order, and room for the largest of them is to be there when it comes round again.
+            with self._lock:
+                self._steps_per_tile = max(needed, (self._steps_per_tile or 0.0) * (63 / 64))
         return rgb, alpha, frame
 
     def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision):

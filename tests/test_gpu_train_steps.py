@@ -357,3 +357,25 @@ def test_captured_launches_replay_like_eager_ones(device, oracle_mod):
         assert int(captured[9]) == int(want[9]) == replay % 2 and not int(captured[12][0])
         for got, expected in zip(captured[:9] + captured[10:12], want[:9] + want[10:12]):
             assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(expected))
+
+
+def test_cameras_that_come_round_again_are_not_rendered_twice(device, oracle_mod, monkeypatch):
+    """Room for the steps is kept for the largest of the frames, whatever lies between its turns."""
+    from mlp_splatting_amd import ops
+    from mlp_splatting_amd.tile_ext import TileExt
+    lib, asked = ops._lib.load(), []
+
+    class Counting:
+        def __getattr__(self, name):
+            if name == "mlpsp_train_workspace_bytes":
+                asked.append(name)
+            return getattr(lib, name)
+    frames = [_scene(device, oracle_mod, n, 160, 120, scale, False) for n, scale in ((300, 0.3), (1500, 1.0), (300, 0.2))]
+    ext = TileExt()
+    monkeypatch.setattr(ops._lib, "load", lambda: Counting())
+    for turn in range(4):
+        for fr, base in (*frames, frames[0], frames[2]):
+            ext.train_forward(base, 160, 120, fr.thr)
+        if turn == 0:
+            asked.clear()
+    assert len(asked) == 3 * 5
