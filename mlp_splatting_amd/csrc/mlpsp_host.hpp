@@ -62,8 +62,8 @@ constexpr int kNumXcd = 8;
 // Workgroup b belongs to XCD b % 8; it is that XCD's j-th workgroup, j = b / 8, and takes tile j % side^2 of the XCD's
 // (j / side^2)-th super-block.  Tiles outside the image return -1.
 // A side is 8 tiles (16 measured 7 to 10 % slower, 4 within 1 %), or fewer on an image that has fewer than eight
-// super-blocks of that size for every XCD (2 at the least: the render takes four slots at a time): 40x30 tiles are 20 super-blocks of 8x8, three for some XCDs and two for the
-// others, but 80 of 4x4.
+// super-blocks of that size for every XCD (2 at the least: the render takes four slots at a time): 40x30 tiles are 20
+// super-blocks of 8x8, three for some XCDs and two for the others, but 80 of 4x4.
 constexpr int kSuperLog2 = 3;
 
 __host__ __device__ inline int superblock_log2(int ntx, int nty) {

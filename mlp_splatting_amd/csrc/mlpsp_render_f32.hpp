@@ -162,10 +162,11 @@ __global__ __launch_bounds__(64) void render_tilecenter_f32_kernel(
 // wavefront nor across the wavefronts of a SIMD (a probe of four wavefronts per SIMD: 8 MFMAs 516 clocks, 64
 // independent FMAs 183, the two interleaved 691), so a hit step costs the sum: 104 x 64 clocks of matrix work plus 2.9
 // for every vector instruction, and every instruction removed shows: the walk of mlpsp_walk_f32.hpp, sin/cos pairs without
-// their range selects, a one-instruction ReLU (1,575 -> 1,360 vector instructions per hit step) and super-blocks of
-// tiles dealt to the XCDs instead of bands of image rows took the 200,000-primitive 1200x680 frame from 4.33 to
-// 3.93 ms and a 30,000-primitive 333x251 feature frame from 1.77 to 1.47.  Three wavefronts per SIMD: four would need
-// 10 KB of LDS per wavefront, and two less registers, and measured within 1 % of three.
+// their range selects, a one-instruction ReLU (1,575 -> 1,360 vector instructions per hit step, 106 of them MFMAs) and
+// super-blocks of tiles dealt to the XCDs instead of bands of image rows took the 200,000-primitive 1200x680 frame from 4.33 to 3.93
+// ms and a 30,000-primitive 333x251 feature frame from 1.77 to 1.47.  The sum is 10,400 of the 13,500 clocks that a hit step
+// takes; the rest are waits of the three wavefronts per SIMD: four would need 10 KB of LDS per wavefront, and two less
+// registers, and measured within 1 % of three.
 struct ItemF32Lds {
   DirOperands dir;
   WalkLds walk;
@@ -287,9 +288,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
       beta, temp, hp, stats);
 }
 
-// The same item by a team of wavefronts (mlpsp_team.hpp).  Wavefront 0 adds up
-// image and depth, in list order and with the roundings of the single wavefront; each wavefront writes the record of its
-// own entry.
+// The same item by a team of wavefronts (mlpsp_team.hpp).  Wavefront 0 adds up image and depth, in list order and with the
+// roundings of the single wavefront; each wavefront writes the record of its own entry.
 template <int TEAM>
 struct TeamF32Lds {
   DirOperands dir;

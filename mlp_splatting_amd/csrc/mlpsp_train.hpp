@@ -16,10 +16,12 @@
 //
 // How many steps a tile will have is known only when it is done, so steps come from a pool in chunks, one atomic for a
 // group of them: a group per chunk at first, up to 32 steps in the end, so that a tile with a single hit takes one chunk
-// and a long one few atomics.
-// (Training step of 50,000 small primitives, 2400x1360, 45 % of the pixels hit: 7.6 GiB with 32 steps from the start, 1.7 now;
-// the full frames take what they did, in the same time, and chunks of four are no better than of eight.)  The draw goes on when the pool is exhausted, so that the caller
-// learns how many chunks the frame needs.
+// and a long one few atomics.  (Training step of 50,000 small primitives, 2400x1360, 45 % of the pixels hit: 7.6 GiB with
+// 32 steps from the start, 1.7 now; full frames take what they did, in the same time, and chunks of four are no better
+// than of eight.)  The draw goes on when the pool is exhausted, so that the caller learns how many chunks the frame needs.
+//
+// A step is as large for five hits as for 64.  A primitive of few hits per tile is small on the screen, though, and hits
+// few tiles: its steps are bounded by a few times the 28 KB of its weights and their gradients.
 //
 // Workspace: head int32[64] {chunks drawn, status bits, steps in all} | tile_steps int32[T] | tile_base int32[T + 1] |
 // chunk_table int32[P / chunk + T + 1] | ids int32[pool] | records

@@ -2,13 +2,13 @@
 // and MLP weight gradients per primitive.  Counterpart of the reference's reverse walk (primitive_records.cuh:3-46) and
 // grouped gradient kernels (scannet/primitive_gemm.py:101-183) in one pipeline whose unit is a step, not a record.
 //
-// The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal length.  A wavefront walks one chunk; where the primitive changes it
-// writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
+// The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal
+// length.  A wavefront walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
 // (the primitive goes on in the next chunk) or head row (it ended here).  Two more launches add the rows of the primitives
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
-// Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.52 (1.9), sort and grouping
-// 0.22 (sort 1.7, gathers 2.85), geometry 0.21 (1.1), weight gradients 7.5 (13.5), joining rows and zeros 0.9 (0.8).
+// Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
+// 0.14 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients 6.8 (12.8), joining rows 0.20 and zeros 0.48 (0.8).
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -74,8 +74,8 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
 // ---------------------------------------------------------------------------------------------
 // steps sorted by primitive: a stable radix sort of the S primitive numbers in tile order, in digits of equal width (two of
 // nine bits at 200,000 primitives).  A wavefront takes an eighth of its block's steps in rounds of 64, whose equal digits are
-// found with a ballot per bit.  Eight launches, 75 us at 650,000 steps; the library's sort took 22 launches and 200 us with
-// the gather behind it.
+// found with a ballot per bit.  Eight launches, 140 us at 650,000 steps (the two sums over blocks x digits, one workgroup
+// each, 50 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSortBlock = 512, kSortBits = 10;
 // Steps of a block: 8,192, a quarter of that where this would leave a chip of 256 CUs fewer than 32 blocks (16 rounds one

@@ -16,7 +16,7 @@
 //
 // All are bound by memory traffic: attribute rows out of L2 in the blend (8 KB per step at 512 channels, four slots), sign
 // rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each).  At 200,000 primitives,
-// 1200x680, a 300x170 target of 512 channels: 0.56, 0.07, 0.44 and 0.32 ms; the record kernels took 4.95 ms for the
+// 1200x680, a 300x170 target of 512 channels: 0.45, 0.06, 0.42 and 0.28 ms; the record kernels took 4.95 ms for the
 // loss and 8.1 ms for the gradient.
 #include <type_traits>
 #include "mlpsp_device.hpp"

@@ -5,8 +5,8 @@
 //
 // Geometry, order, activations and compositing are the f32 expressions of the render (f32 MLP: its bits with
 // `render_order`, the record kernels' rounding of layer 2 without).  Bound by the MLP; the steps add 3.3 KB of contiguous
-// stores per hit step.  200,000 primitives, 1200x680, f32: 4.5 ms, against 4.4 + 6.6 ms of the record forward's two walks;
-// 20,000 primitives, 320x240: 1.15 ms with a wavefront per tile, 0.88 with teams.
+// stores per hit step.  200,000 primitives, 1200x680, f32: 3.9 ms, against 4.0 + 6.0 of the record forward's two walks;
+// 20,000 primitives, 320x240: 1.24 ms with a wavefront per tile, 0.87 with teams (see train_plan).
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mfma16.hpp"

@@ -44,8 +44,8 @@ __device__ __forceinline__ bool hit_rot_from(const wf32x4 q[3], Vec3 vl, float r
 }
 
 // can(): may this lane still take a hit?  step(p, hit, h, mask): called for every entry that was tested, with the
-// ballot of its hits; returns false when the walk is over.  Call with all 64 lanes of a wavefront that is alone in its
-// workgroup (its LDS operations are in order: no barrier).
+// ballot of its hits; returns false when the walk is over.  Call with all 64 lanes of a wavefront, and with an `s` that no
+// other wavefront of its workgroup touches (a wavefront's LDS operations are in order: no barrier).
 template <typename Can, typename Step>
 __device__ __forceinline__ void walk_tile_f32(const int32_t* __restrict__ order, int start, int end, int N,
                                               const PrimRecord* __restrict__ prims, bool valid, float rox, float roy,

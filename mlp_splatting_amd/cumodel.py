@@ -9,8 +9,8 @@ the API: culling is the sparse HIP binning instead of a dense [tiles x primitive
 expression, and the extension object is ``tile_ext.TileExt`` on ``libmlpsp_hip.so``.
 
 ``forward`` renders without a graph under ``torch.no_grad()``; in grad mode with parameters that require
-grad it goes through ``_TileRenderAutogradFn`` (RGB) or, with a feature target, through the record-based
-training step of ``record_training``.  The dense feature-image backward of the reference is not provided.
+grad it goes through ``_TileRenderAutogradFn`` (RGB), ``_TileRenderWithFeatAutogradFn`` (RGB and the dense feature
+image) or, with a feature target, through the training step of ``record_training``.
 """
 from __future__ import annotations
 
@@ -259,8 +259,11 @@ def _uncached(ext):
 
 
 class _TileRenderAutogradFn(torch.autograd.Function):
-    """RGB render with gradients for geometry and MLP weights (scannet/cumodel.py:219-378).  The forward is the
-    ordinary f32 render; the backward re-traverses the frame (``render_tiles_backward_tilecenter_full``)."""
+    """RGB render with gradients for geometry and MLP weights (scannet/cumodel.py:219-378).  In tile-centre order with
+    8x8 tiles and the released MLP the forward keeps the frame's training steps (``TileExt.train_forward``, the f32
+    render's bits) and the backward works on them; every other frame is rendered as usual and its backward traverses
+    it again (``render_tiles_backward_tilecenter_full``, in per-pixel order the records of every pixel's own depth
+    order)."""
 
     @staticmethod
     def forward(ctx, rays_o, rays_d, positions, log_scales, quats, culled_prim_indices, tile_offsets, freq, att,

@@ -5,7 +5,8 @@ The exact high-resolution feature blend is sampled with the bilinear down-sampli
 (``F.interpolate(..., mode="bilinear", align_corners=False)``) without ever materialising the 512-D image; only
 int8 signs of the residual and scalar loss partials are kept.  Geometry, alpha and the MLP are constants of this
 loss (scannet/record_feature_loss.py:1-6).  The kernels are libmlpsp_hip's ``mlpsp_stream_feature_l1`` and
-``mlpsp_feature_attribute_gradients``.
+``mlpsp_feature_attribute_gradients``.  The scene module's training step computes the same loss and gradient from tile
+steps (``ops.train_feature_l1``); these functions are for callers that hold per-pixel records, as the reference's are.
 """
 from __future__ import annotations
 

@@ -539,7 +539,8 @@ class TileExt:
                                       any_tile=False, counts_only=False, name="render_tiles_mlp_records"):
         """[rgb, alpha, ids, x6, raw, masks, gates, offsets]: one record per hit and pixel, in each
         pixel's compositing order.  ``x`` = the 15 scene tensors + two adjoint placeholders that the
-        forward-only mode never reads (scannet/csr_training.py:37-39).  ``render_order`` (not in the reference):
+        forward-only mode never reads (scannet/csr_training.py:37-39).  ``render_order`` (not in the reference, and no
+        longer what the scene module trains on: for callers that want records of the very image a render gives):
         image and records in the rounding of ``render_tiles_forward_tilecenter`` instead of the record kernels'
         own; see :meth:`records_forward_matches_render`."""
         _chk(len(x) == 17, "Expected 15 scene inputs and RGB/T adjoints")
@@ -585,8 +586,8 @@ class TileExt:
     def records_forward_matches_render(freq, W1, b1, W2, b2, tile):
         """True if ``render_tiles_training_records(..., render_order=True)`` is available for this frame: 8x8 tiles
         and the 72->32->32->4 MLP with six frequencies in 16-byte aligned f32 tensors.  Its rgb/alpha are then the
-        bits of ``render_tiles_forward_tilecenter``, and a differentiable render can keep the records of its
-        forward pass for the backward instead of traversing the frame again."""
+        bits of ``render_tiles_forward_tilecenter``; a differentiable render takes :meth:`train_forward` under the same
+        condition and keeps the steps of its forward pass for the backward instead of traversing the frame again."""
         return (int(tile) == 8 and freq.numel() == 6 and tuple(W1.shape[1:]) == (32, 72) and tuple(W2.shape[1:]) == (32, 32)
                 and all(t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (W1, b1, W2, b2)))
 
