@@ -94,7 +94,7 @@ def train_steps(args, scene, frames, proj, thr, W, H, sc, dev):
     feature_dim = 0 if scene.feat_attr is None else int(scene.feat_attr.shape[-1])
     feature_target = None
     if feature_dim:
-        # record-based step with the streamed feature loss against a quarter-resolution target
+        # step with the streamed feature loss against a quarter-resolution target
         params.append(scene.feat_attr)
         opt = torch.optim.Adam(params, lr=1e-4, fused=True)
         feature_target = (torch.randn(H // 4, W // 4, feature_dim, device=dev, generator=gen) * 0.05).half()
@@ -444,10 +444,10 @@ def main() -> int:
     ap.add_argument("--poses", type=int, default=32)
     ap.add_argument("--dense-feature-loss", action="store_true",
                     help="with --train on a feature workload: the dense feature image under autograd (the reference's "
-                         "legacy training backend) instead of the record-based streamed loss")
+                         "legacy training backend) instead of the streamed loss")
     ap.add_argument("--train", action="store_true",
                     help="time full training steps instead (f32 render with autograd, L1 image loss, backward through "
-                         "the record pipeline, Adam on all nine parameter tensors); prints its own JSON line")
+                         "the training steps, Adam on all nine parameter tensors); prints its own JSON line")
     ap.add_argument("--wake-seconds", type=float, default=1.0,
                     help="untimed rendering before the warm-up steps, to bring an idle GPU to its sustained clocks")
     ap.add_argument("--min-seconds", type=float, default=0.5,

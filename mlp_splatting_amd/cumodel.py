@@ -832,7 +832,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
 
     def _forward_csr_training(self, ray_o, ray_d, score_threshold, bg_color, view_matrix, proj_matrix,
                               culled_prim_indices, tile_offsets, return_feature, feature_target, device):
-        """(rgb, streamed feature L1 loss) through the record-based training function
+        """(rgb, streamed feature L1 loss) through the training function of ``record_training``
         (scannet/cumodel.py:1098-1108)."""
         self._forget_parameters()
         W, H = self.image_size
