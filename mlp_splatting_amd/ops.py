@@ -887,6 +887,8 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
             break
         pool_steps = chunks * _lib.STEP_CHUNK
         del workspace                       # (too small: its memory is free for the next)
+    else:                                   # (the walk does not depend on the room: the second asks for what the first did)
+        raise RuntimeError("mlpsp_train_forward: the frame asked for more steps than it had asked for")
     return rgb, alpha, TrainFrame(workspace, pairs, W, H, chunks, status, steps, records)
 
 

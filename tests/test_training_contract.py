@@ -156,3 +156,33 @@ def test_the_streamed_loss_refuses_attributes_that_are_no_rows_of_channels(shape
         assert _loss_geometry(torch.empty(N, 5, 6, device="cuda"), target, (image,), W, H) == (2, 3, 6, 5)
         with pytest.raises(ValueError, match="1/4/5-slot renderer"):
             _loss_geometry(torch.empty(shape, device="cuda"), target, (image,), W, H)
+
+
+@pytest.mark.parametrize("asked,calls", [((4,), 1), ((9, 9), 2), ((9, 10), None)])
+def test_no_frame_comes_back_without_room_for_its_steps(monkeypatch, asked, calls):
+    made = []
+
+    class Lib:
+        def mlpsp_train_workspace_bytes(self, *_a):
+            return 256
+
+        def mlpsp_train_forward_f32(self, *_a):
+            made.append(asked[len(made)])
+            return 0
+    empty = torch.empty
+
+    def chunks_asked(*shape, **kw):             # (the workspace: the kernels count the chunks that they drew)
+        t = empty(*shape, **kw)
+        if t.dtype == torch.uint8:
+            t.view(torch.int32)[:3] = torch.tensor([asked[min(len(made), 1)], 0, 3])
+        return t
+    monkeypatch.setattr(ops._lib, "load", Lib)
+    monkeypatch.setattr(ops, "_stream", lambda _d: 0)
+    monkeypatch.setattr(ops.torch, "empty", chunks_asked)
+    x = torch.zeros(1)
+    args = (x, x, x, x.int(), x.int(), x, x, [x] * 6, W, H, 1e-3, 64, 8 * ops._lib.STEP_CHUNK)
+    if calls is None:
+        with pytest.raises(RuntimeError, match="more steps"):
+            ops.train_forward(*args)
+    else:
+        assert ops.train_forward(*args)[2].chunks == asked[-1] and len(made) == calls
