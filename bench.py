@@ -80,8 +80,8 @@ def dense_culling_cpu_torch(positions, log_scales, view, proj, W, H, tile, thr):
 
 
 def train_steps(args, scene, frames, proj, thr, W, H, sc, dev):
-    """One training step = scene(...) under autograd -> L1 loss against a fixed image -> backward (records
-    forward, reverse compositing, grouped weight gradients in IEEE f32) -> Adam step on every parameter."""
+    """One training step = scene(...) under autograd -> L1 loss against a fixed image -> backward (forward on
+    tile steps, reverse compositing, weight gradients grouped by primitive in IEEE f32) -> Adam step on every parameter."""
     import torch
     scene.train()
     scene.render_precision = "f32"
