@@ -48,6 +48,8 @@ def prepare_primitives(positions, log_scales, quats):
     """[N,3],[N,3],[N,4] -> opaque per-primitive geometry records (uint8 [N*64])."""
     positions, log_scales, quats = _f32c(positions, "positions"), _f32c(log_scales, "log_scales"), _f32c(quats, "quats")
     n = positions.shape[0]
+    if positions.numel() != 3 * n or log_scales.numel() < 3 * n or quats.numel() < 4 * n:
+        raise RuntimeError("positions, log_scales and quats must have the same primitive count")
     rec = torch.empty(max(n, 1) * _lib.PRIM_RECORD_BYTES, dtype=torch.uint8, device=positions.device)
     code = _lib.load().mlpsp_prepare_primitives(_ptr(positions), _ptr(log_scales), _ptr(quats), n, _ptr(rec),
                                                 _stream(positions.device))
@@ -646,6 +648,8 @@ def pack_mfma_weights(W1, b1, W2, b2, W3, b3, bf16=True):
     n = W1.shape[0]
     if tuple(W1.shape[1:]) != (32, 72) or tuple(W2.shape[1:]) != (32, 32) or tuple(W3.shape[1:]) != (4, 32):
         raise RuntimeError("the matrix-core path supports the 72->32->32->4 MLP only")
+    if min(W2.shape[0], W3.shape[0]) < n or min(b1.numel(), b2.numel()) < 32 * n or b3.numel() < 4 * n:
+        raise RuntimeError("MLP tensors must have the same primitive count")
     lib = _lib.load()
     packed = torch.empty(lib.mlpsp_mfma_pack_bytes(n), dtype=torch.uint8, device=W1.device)
     if all(w.is_cuda and w.dtype == torch.float16 for w in (W1, b1, W2, b2, W3, b3)):

@@ -171,6 +171,17 @@ class TileExt:
         _chk(att.is_cuda and att.dtype == torch.float32 and att.dim() == 1, "attenuation must be CUDA float32 1-D")
 
     @staticmethod
+    def _check_mlps(positions, freq, att, ws):
+        """No tensor ends before what the exact kernels read of it: the MLPs of as many primitives as W1 has, in W2's
+        width, and at least those of ``positions``.  (Element counts and one message: this stands in front of a frame.)"""
+        W1, b1, W2, b2, W3, b3 = ws
+        held, hidden, F = W1.shape[0], W2.shape[1], freq.numel()
+        units = held * hidden
+        _chk(3 * held >= positions.numel() and att.numel() >= F and W1.numel() >= 12 * F * units and b1.numel() >= units
+             and W2.numel() >= hidden * units and b2.numel() >= units and W3.numel() >= 4 * units and b3.numel() >= 4 * held,
+             "MLP tensors must be [N,H,12F], [N,H], [N,H,H], [N,H], [N,4,H], [N,4] for the primitive count of positions")
+
+    @staticmethod
     def _weights_f32(ws, allow_low_precision):
         W1 = ws[0]
         _chk(all(w.is_cuda for w in ws), "MLP tensors must be CUDA tensors")
@@ -200,6 +211,8 @@ class TileExt:
         F = freq.shape[0]
         _chk(W1.shape[2] == 6 * F * 2, "Encoded dim must be 6*F*2")
         _chk(W2.shape[1] <= hidden_limit, f"{name} currently supports hidden_dim <= {hidden_limit}")
+        _chk(rays_d.shape[0] >= rays_o.shape[0], "rays_d must be a CUDA float32 [B,3] tensor")
+        self._check_mlps(positions, freq, att, ws)
         geo = (rays_o.contiguous(), rays_d.contiguous(), positions.contiguous(), log_scales.contiguous(),
                quats.contiguous())
         return geo, cand, offsets, freq.contiguous(), att.contiguous(), ws, (Wimg, Himg, TW, TH, float(thr))
@@ -420,6 +433,13 @@ class TileExt:
                                                threshold)
             if binned is None:
                 return None
+        # (what is looked at here and below hides behind the binning and the sort; rays that came through the prologue,
+        # geometry that became records and MLPs that became operand blocks were held to their sizes there)
+        if tile_pyramids is None:
+            floats = 3 * width * height
+            for t, what in ((rays_o, "rays_o"), (unit_dirs, "rays_d")):
+                _chk(t.is_cuda and t.dtype == torch.float32 and t.numel() >= floats and t.is_contiguous(),
+                     f"{what} must be a CUDA float32 [B,3] tensor")
         cand, offsets, counts, tail, cap, scale, held, ends = binned
         if ends is not None and precision == "f32":
             raise ValueError("lists in segments are for frames on the matrix cores")
@@ -435,6 +455,11 @@ class TileExt:
             order, _ = ops.sort_tiles(rays_o, unit_dirs, rec, cand, offsets, width, height, 8, 8, _lib.KEY_TSTAR,
                                       self.max_tile_prims, cull_threshold=threshold, frame_records=frame_records,
                                       tile_pyramids=tile_pyramids, tile_ends=ends, ids_ascend=True)
+            if precision == "f32":
+                self._check_mlps(positions, freq, att, ws)
+            else:
+                _chk(3 * ws[0].shape[0] >= positions.numel() and att.numel() >= freq.numel(),
+                     "MLP tensors must have the primitive count of positions")
             fmap, pool_ran_out = None, 0
             if precision != "f32":
                 packed = self._packed_weights(list(ws), precision == "bf16")
