@@ -10,7 +10,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-from .ops import _check, _f32c, _ptr, _stream, num_tiles
+from .ops import _check, _f32c, _primitives, _ptr, _stream, num_tiles
 
 
 @torch.no_grad()
@@ -28,7 +28,7 @@ def ray_cone_candidates(ray_o, ray_d, positions, log_scales, width, height, tile
     if ray_o.device != device or ray_d.device != device:
         raise ValueError("device mismatch")
     ray_o, ray_d = _f32c(ray_o, "ray_o"), _f32c(ray_d, "ray_d")
-    positions, log_scales = _f32c(positions.detach(), "positions"), _f32c(log_scales.detach(), "log_scales")
+    positions, log_scales = _primitives(positions.detach(), log_scales.detach())
     lib = _lib.load()
     n, T = positions.shape[0], num_tiles(width, height, tile_size, tile_size)
     offsets = torch.empty(T + 1, dtype=torch.int32, device=device)

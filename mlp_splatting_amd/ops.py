@@ -44,12 +44,20 @@ def num_tiles(W: int, H: int, TW: int, TH: int) -> int:
     return ((W + TW - 1) // TW) * ((H + TH - 1) // TH)
 
 
+def _primitives(positions, log_scales):
+    """(positions, log-scales) as the kernels take them: contiguous f32 [N, 3], the second no shorter than the first."""
+    positions, log_scales = _f32c(positions, "positions"), _f32c(log_scales, "log_scales")
+    if positions.numel() != 3 * positions.shape[0] or log_scales.numel() < positions.numel():
+        raise RuntimeError("positions and log_scales must be [N, 3] of the same primitive count")
+    return positions, log_scales
+
+
 def prepare_primitives(positions, log_scales, quats):
     """[N,3],[N,3],[N,4] -> opaque per-primitive geometry records (uint8 [N*64])."""
-    positions, log_scales, quats = _f32c(positions, "positions"), _f32c(log_scales, "log_scales"), _f32c(quats, "quats")
-    n = positions.shape[0]
-    if positions.numel() != 3 * n or log_scales.numel() < 3 * n or quats.numel() < 4 * n:
-        raise RuntimeError("positions, log_scales and quats must have the same primitive count")
+    positions, log_scales = _primitives(positions, log_scales)
+    quats, n = _f32c(quats, "quats"), positions.shape[0]
+    if quats.numel() < 4 * n:
+        raise RuntimeError("quats must be [N, 4] of the primitive count of positions")
     rec = torch.empty(max(n, 1) * _lib.PRIM_RECORD_BYTES, dtype=torch.uint8, device=positions.device)
     code = _lib.load().mlpsp_prepare_primitives(_ptr(positions), _ptr(log_scales), _ptr(quats), n, _ptr(rec),
                                                 _stream(positions.device))
@@ -172,7 +180,7 @@ def bin_legacy(positions, log_scales, view_matrices, proj_matrix, W: int, H: int
     Returns (culled_prim_indices int32 [P], tile_offsets int32 [T+1]); ids ascend inside a tile.
     ``with_longest`` appends the length of the longest tile list (known from the same read-back).
     """
-    positions, log_scales = _f32c(positions, "positions"), _f32c(log_scales, "log_scales")
+    positions, log_scales = _primitives(positions, log_scales)
     dev = positions.device
     vm = view_matrices.detach().to("cpu", torch.float32).reshape(-1, 4, 4).contiguous()
     pm = proj_matrix.detach().to("cpu", torch.float32).reshape(4, 4).contiguous()
@@ -241,7 +249,7 @@ def bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, W: int, 
     between calls whose launches follow each other on one stream; the candidate, offset and scratch buffers are
     then allocated once and handed out again while their sizes stay the same (four allocations less between the
     end of one frame and the first launch of the next)."""
-    positions, log_scales = _f32c(positions, "positions"), _f32c(log_scales, "log_scales")
+    positions, log_scales = _primitives(positions, log_scales)
     dev = positions.device
     on_device = (tile_view_ids is None and all(m.is_cuda and m.dtype == torch.float32 and m.numel() == 16 and
                                                m.is_contiguous() for m in (view_matrices, proj_matrix)))
@@ -296,7 +304,7 @@ def bin_segments_async(positions, log_scales, view_matrix, proj_matrix, W: int, 
     t's list -- the same ids in the same order -- is ``candidates[tile_offsets[t]:tile_ends[t]]``; a list longer
     than ``stride`` keeps its first ``stride`` entries.  :func:`sort_tiles` and :func:`render_tilecenter_mfma` take
     such lists with ``tile_ends``.  ``counts``, ``reuse``: as in :func:`bin_legacy_async`."""
-    positions, log_scales = _f32c(positions, "positions"), _f32c(log_scales, "log_scales")
+    positions, log_scales = _primitives(positions, log_scales)
     dev = positions.device
     for m in (view_matrix, proj_matrix):
         if not (m.is_cuda and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()):

@@ -103,3 +103,18 @@ def test_a_queued_frame_refuses_rays_its_kernels_would_misread(ext, precision):
                 x[i] = change(x[i])
                 with pytest.raises(RuntimeError, match="float32"):
                     _queued(ext, x, precision)
+
+
+@pytest.mark.parametrize("shapes", [((N, 3), (N - 1, 3)), ((N, 2), (N, 3)), ((N, 3), (N, 2)), ((N,), (N,))], ids=str)
+def test_binning_refuses_primitives_that_do_not_go_together(ext, shapes):
+    from mlp_splatting_amd.camera import ray_cone_candidates
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        p, s = (torch.empty(x, device="cuda") for x in shapes)
+        rays, eye = torch.empty(W * H, 3, device="cuda"), torch.empty(4, 4, device="cuda")
+        for call in (lambda: ops.bin_legacy(p, s, eye, eye, W, H, 8, 1e-3),
+                     lambda: ops.bin_legacy_async(p, s, eye, eye, W, H, 8, 1e-3, 64),
+                     lambda: ops.bin_segments_async(p, s, eye, eye, W, H, 8, 1e-3),
+                     lambda: ray_cone_candidates(rays, rays, p, s, W, H, 8, 1e-3),
+                     lambda: ops.prepare_primitives(p, s, torch.empty(N, 4, device="cuda"))):
+            with pytest.raises(RuntimeError, match="primitive count"):
+                call()
