@@ -203,7 +203,7 @@ class Workload:
                 ro, rd = syn.pinhole_rays(self.W, self.H, self.f, c2w)
                 frames.append((t(ro), t(rd), t(syn.view_matrix(c2w))[None], None))
             # A pose whose fullest tile exceeds the 1,536-candidate capacity is an error of the path, not a frame
-            # (the reference raises, and so does this build); the headline scene was constructed so that all 32 poses
+            # (the reference raises, and so does this renderer); the headline scene was constructed so that all 32 poses
             # fit, the literally specified smaller scenes were not.  Such poses are left out and counted.
             fitting = []
             with torch.no_grad():
@@ -465,7 +465,7 @@ def main() -> int:
                          "readings of a profiled run are scaled by")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path (each GPU box has one GPU); "
+        print("bench.py measures one GPU: a frame is rendered and trained on one device; "
               "run with --gpus 1", file=sys.stderr)
         return 2
 

@@ -116,7 +116,7 @@ class TileExt:
     def __getattr__(self, name):
         if name in _BACKWARD_ONLY:
             def _missing(*_a, **_k):
-                raise NotImplementedError(f"{name} is one of the reference's fused backward entry points, which this build does not provide")
+                raise NotImplementedError(f"{name} is one of the reference's fused backward entry points, which mlp_splatting_amd does not provide")
             return _missing
         raise AttributeError(name)
 

@@ -10,7 +10,7 @@ if ROOT not in sys.path:
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs an MI355X (run with -m gpu)")
 
 
 @pytest.fixture(scope="session")
@@ -26,7 +26,7 @@ def device():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from mlp_splatting_amd import _lib
-    _lib.load()  # the HIP library must be there on a GPU box: no fallback
+    _lib.load()  # the HIP library must be there where a GPU is: no fallback
     return torch.device("cuda", 0)
 
 

@@ -3,7 +3,7 @@ renderer and what the CPU oracle returns for it (tile lists, sorted order and ke
 the matrix-core emulations of the image).
 
 The reference renderer exists only as CUDA and holds no output vectors of its own, so these vectors come from
-this build's CPU restatement; they pin it (and the HIP path, which tests/test_golden_frame.py holds to the same
+the CPU restatement; they pin it (and the HIP path, which tests/test_golden_frame.py holds to the same
 bits without the oracle at run time) against drifting, not against the reference.
 
     python tests/golden/make_frame_fixture.py

@@ -1,6 +1,6 @@
 """Parity at the full sizes of the benchmark configurations (50k / 200k primitives, up to 2400x1360).
 
-Where the oracle finishes a frame in seconds on the box's host cores it is the checker, bit for bit; beyond
+Where the oracle finishes a frame in seconds on the host cores the image is held to it, bit for bit; beyond
 that the tests use properties that hold at any size: sortedness and idempotence of the per-tile order, the
 image being independent of the conservative culling, alpha in [0, 1], linearity of the feature image in the
 attributes and its closed form for constant attributes (gates sum to one, so feat = alpha * v).

@@ -125,7 +125,7 @@ def test_per_pixel_order_gradients_match_float64_autograd_over_its_records(devic
 
 
 def test_reference_style_per_pixel_backward_through_count_and_emit(device, oracle_mod, monkeypatch):
-    """The reference's own mode-0 backward (scannet/cumodel.py:297-364), spelled out against this build's entry
+    """The reference's own mode-0 backward (scannet/cumodel.py:297-364), spelled out against these entry
     points: count -> exclusive scan -> emit -> torch autograd through the MLP of the emitted (prim_id, x6) with the
     emitted adjoints of (rgb, sigma_raw).  It must give the gradients of the scene module's per-pixel backward."""
     from mlp_splatting_amd.cumodel import _encode_x6, _mlp_forward_indexed
