@@ -3,17 +3,18 @@
 // grouped gradient kernels (scannet/primitive_gemm.py:101-183) in one pipeline whose unit is a step, not a record.
 //
 // The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal
-// length.  A wavefront walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
+// length.  A wavefront (f32 weights: a workgroup) walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
 // (the primitive goes on in the next chunk) or head row (it ended here).  Two more launches add the rows of the primitives
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.14 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients 6.8 (12.8), joining rows 0.20 and zeros 0.48 (0.8).
+// 0.14 (sort 1.7, gathers 2.85), geometry 0.18 (1.3), weight gradients 4.7 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
 #include "mlpsp_train.hpp"
 #include "mlpsp_vjp16.hpp"
+#include "mlpsp_vjp32.hpp"
 
 namespace mlpsp {
 
@@ -270,14 +271,17 @@ __device__ __forceinline__ void geometry_store(const float v[15], float qw, floa
                         r12 * (2.f * qy) + r20 * (2.f * qx) + r21 * (2.f * qy);
 }
 
-__global__ __launch_bounds__(256) void train_geometry_kernel(
+// A workgroup per chunk, the steps of a run to its wavefronts in turn: one for chunks of 16 steps, four for 256.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void train_geometry_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float* __restrict__ falloff, const float* __restrict__ logs, const float* __restrict__ quats,
     float* __restrict__ rows, GeoGrads out) {
-  const int chunk = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), l = threadIdx.x & 63;
-  if (chunk >= num_chunks) return;
+  __shared__ float s_sum[2][WAVES][16];
+  const int chunk = (int)blockIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63;
   const int chunk_end = min(S, (chunk + 1) * chunk_steps);
-  for (int pos = chunk * chunk_steps; pos < chunk_end;) {
+  int turn = 0;
+  for (int pos = chunk * chunk_steps; pos < chunk_end; turn ^= 1) {
     const StepRun run = step_run(ix, pos, chunk_end);
     const size_t p = (size_t)run.p;
     const float qw = quats[p * 4], qx = quats[p * 4 + 1], qy = quats[p * 4 + 2], qz = quats[p * 4 + 3];
@@ -286,7 +290,7 @@ __global__ __launch_bounds__(256) void train_geometry_kernel(
 #pragma unroll
     for (int k = 0; k < 15; ++k) v[k] = 0.f;
 #pragma unroll 2
-    for (int k = run.begin; k < run.end; ++k) {
+    for (int k = run.begin + wave; k < run.end; k += WAVES) {
       const int4 at = ix.step[k];
       const float4 c = reinterpret_cast<const float4*>(records + (size_t)at.x * kStepBytes + kStepPlaneC)[l];
       const float a = falloff[(size_t)at.y * 64 + l];
@@ -308,13 +312,26 @@ __global__ __launch_bounds__(256) void train_geometry_kernel(
 #pragma unroll
       for (int k = 0; k < 15; ++k) v[k] += __shfl_xor(v[k], d);
     }
-    if (run.complete) {
-      if (l == 0) geometry_store(v, qw, qx, qy, qz, p, out);
-    } else if (l < 15) {
+    if (l < 15) {
       float mine = v[0];
 #pragma unroll
       for (int k = 1; k < 15; ++k) mine = (l == k) ? v[k] : mine;
-      run_row(rows, run, chunk, num_chunks)[kGradFloats + l] = mine;
+      s_sum[turn][wave][l] = mine;
+    }
+    if constexpr (WAVES > 1) __syncthreads();      // (the one barrier of a turn: the next writes the other half)
+    if (wave == 0) {
+      float total = 0.f;
+      if (l < 15) {
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) total += s_sum[turn][w][l];
+      }
+      if (!run.complete) {
+        if (l < 15) run_row(rows, run, chunk, num_chunks)[kGradFloats + l] = total;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 15; ++k) v[k] = __shfl(total, k);
+        if (l == 0) geometry_store(v, qw, qx, qy, qz, p, out);
+      }
     }
     pos = run.end;
   }
@@ -377,6 +394,35 @@ __device__ __forceinline__ void walk_run(const StepIndex& ix, const StepRun& run
   }
 }
 
+// ... or one half of every STRIDE-th step, from `first` on.
+template <int STRIDE, typename Work>
+__device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int end, int half, const unsigned char* __restrict__ records,
+                                            const float4* __restrict__ d4, const float* __restrict__ rays_d, int n, int g, int W,
+                                            int pixels, Work&& work) {
+  if (first >= end) return;
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  const auto where = [&](int k) { return ix.step[min(k, end - 1) + zero]; };
+  const auto record = [&](int4 v) {
+    return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y), 0,
+                                                      __builtin_amdgcn_readfirstlane(v.w)), half, n, g, W, pixels);
+  };
+  StepRecord ahead = record(where(first));
+  int4 next = where(first + STRIDE);
+  for (int k = first; k < end; k += STRIDE) {
+    StepRecord r = ahead;
+    if (k + STRIDE < end) {
+      ahead = record(next);
+      next = where(k + 2 * STRIDE);
+    }
+    const bool adjoint = r.d.x != 0.f || r.d.y != 0.f || r.d.z != 0.f || r.d.w != 0.f;
+    if (__ballot(adjoint) == 0ull) continue;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r.x[c] = adjoint ? r.x[c] : 0.f;
+    work(r);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp16_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
@@ -409,248 +455,44 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 }
 
 // ---------------------------------------------------------------------------------------------
-// MLP weight gradients in IEEE f32 (v_mfma_f32_32x32x2_f32, exact fma chains).
-//
-// f32 MFMAs and vector instructions do not overlap on this chip, so a block of 32 records costs the sum of both, and
-// every product is issued in the one orientation its consumer reads, or in two where that is cheaper than a transpose
-// through LDS:
-//   * lane (n, g) encodes the three inputs of group g of record n (18 pairs, none twice); one half-wave swap per pair
-//     yields the operands of two K-steps.  The encoding is also parked in LDS, row = record, where the W1 gradient reads
-//     it with the encoding index in the lane.
-//   * layer 1 "record-major" (record in the lane, units 2i + g in register i: the operand order of layer 2), its rectified
-//     tile parked in LDS for the W2 gradient; layer 2 "unit-major" (unit in the lane, records in the registers), straight
-//     into the W3 gradient; D2 in both orientations (two MFMAs each); D1 unit-major.
-//   * a weight-gradient product contracts over records: both operands name, in register i of lane group g, record
-//     8 (i / 4) + 4 g + i % 4.
-//   * the last 8 of the 72 encoding columns go into one 16x16x4 product per register -- its four k-slots are (units 0..15,
-//     units 16..31) x (record of g = 0, of g = 1); B holds the 8 columns twice, for k even and for k odd, zero elsewhere
-//     -- 32 clocks instead of 64; the 4x32 W3 gradient into 4x4x1 products, 9 clocks instead of 64.
-// Registers hold all weight operands, LDS (15 KB) what changes orientation: two wavefronts per SIMD.  Per block 118
-// MFMAs of 64 clocks and the small ones, ~800 vector instructions.
+// MLP weight gradients in f32: the blocks of mlpsp_vjp32.hpp.  A workgroup per chunk, half a step to a wavefront.
 // ---------------------------------------------------------------------------------------------
-struct VjpF32Lds {
-  static constexpr int LE = 76, LH = 36;
-  __attribute__((aligned(16))) float enc[32 * LE];    // [record][36 g + 2 t + (0 sin, 1 cos)], columns 72..75 zero
-  __attribute__((aligned(16))) float h1[32 * LH];     // [record][16 g + i] = unit 2i + g
-  __attribute__((aligned(16))) float d3[32 * 4];      // [record][output]
-  __attribute__((aligned(16))) int32_t mask[2][32];
-  __attribute__((aligned(16))) float bias1[2][16];    // [g][i] = b1[2i + g]
-};
-typedef float vf32x4 __attribute__((ext_vector_type(4)));
-
-struct VjpF32Operands {
-  float w1[36], w2[16], w2t[16], w3r[2], w3u[2], bias2;
-  __device__ __forceinline__ void load(const float* __restrict__ W1, const float* __restrict__ b1,
-                                       const float* __restrict__ W2, const float* __restrict__ b2,
-                                       const float* __restrict__ W3, size_t p, int lane, VjpF32Lds& s) {
-    asm volatile("" : "+v"(lane));
-    const int n = lane & 31, g = lane >> 5;
-    const int hid = mfma32_hidden_row(n);
-    const vf32x4* __restrict__ r1 = reinterpret_cast<const vf32x4*>(W1 + p * 2304 + hid * 72 + 36 * g);
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-      const vf32x4 v = r1[q];
-      w1[4 * q] = v[0];
-      w1[4 * q + 1] = v[1];
-      w1[4 * q + 2] = v[2];
-      w1[4 * q + 3] = v[3];
-    }
-    const float* __restrict__ row = W2 + p * 1024 + n * 32 + g;
-    const float* __restrict__ col = W2 + p * 1024 + g * 32 + n;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      w2[i] = row[2 * i];
-      w2t[i] = col[64 * i];
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      w3r[j] = W3[p * 128 + (2 * j + g) * 32 + hid];
-      w3u[j] = W3[p * 128 + (2 * j + g) * 32 + n];
-    }
-    bias2 = b2[p * 32 + n];
-    if (n < 16) s.bias1[g][n] = b1[p * 32 + 2 * n + g];
-  }
-};
-
-struct VjpF32Sums {
-  vf32x16 gw1[2], gw2;
-  vf32x4 gw1e, gw3;
-  float gb1, gb2, gb3[4];
-  __device__ __forceinline__ void clear() {
-    gw1[0] = gw1[1] = gw2 = splat16(0.f);
-    gw1e = gw3 = vf32x4{0.f, 0.f, 0.f, 0.f};
-    gb1 = gb2 = gb3[0] = gb3[1] = gb3[2] = gb3[3] = 0.f;
-  }
-};
-
-__device__ __forceinline__ vf32x16 mfma_f32(float a, float b, vf32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-// v where bit `bit` of word is set, else +0
-__device__ __forceinline__ float where_bit(float v, uint32_t word, int bit) {
-  return __uint_as_float(__float_as_uint(v) & (uint32_t)__builtin_amdgcn_sbfe((int)word, bit, 1));
-}
-
-__device__ __forceinline__ void vjp_f32_block(const VjpF32Operands& w, VjpF32Sums& sum, VjpF32Lds& s, const StepRecord& r,
-                                              const float* __restrict__ freq, const float* __restrict__ att, float scale,
-                                              int lane) {
-  // (made opaque: the addresses below are one or two registers plus immediates as long as they are formed here, and
-  // fifty registers when they are hoisted out of the loop over the blocks one by one)
-  asm volatile("" : "+v"(lane));
-  const int n = lane & 31, g = lane >> 5;
-  const vf32x16 zero = splat16(0.f);
-  const float inf = relu_limit();
-  const vf32x4 d = {r.d.x * scale, r.d.y * scale, r.d.z * scale, r.d.w * scale};
-  const float d_op[2] = {g ? d[1] : d[0], g ? d[3] : d[2]};     // k-slot g of K-step j = output 2j + g
-  if (g == 0) {
-    *reinterpret_cast<vf32x4*>(&s.d3[4 * n]) = d;
-#pragma unroll
-    for (int o = 0; o < 4; ++o) sum.gb3[o] += d[o];
-  }
-  s.mask[g][n] = (int32_t)(g ? r.mask2 : r.mask1);
-
-  // ---- encoding and layer 1, record-major
-  vf32x16 a1;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const vf32x4 v = *reinterpret_cast<const vf32x4*>(&s.bias1[g][4 * q]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a1[4 * q + k] = v[k];
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    __builtin_amdgcn_sched_barrier(0);
-    float sn[6], cs[6];
-    encode_component(r.x[c], freq, att, sn, cs);
-#pragma unroll
-    for (int f = 0; f < 6; f += 2)
-      *reinterpret_cast<vf32x4*>(&s.enc[n * VjpF32Lds::LE + 36 * g + 2 * (6 * c + f)]) = vf32x4{sn[f], cs[f], sn[f + 1], cs[f + 1]};
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-      float lo = sn[f], hi = cs[f];
-      half_swap(lo, hi);       // lo: pair 6c + f of inputs 0..2 (sin in lanes g = 0, cos in g = 1), hi: of inputs 3..5
-      a1 = mfma_f32(w.w1[6 * c + f], lo, a1);
-      a1 = mfma_f32(w.w1[18 + 6 * c + f], hi, a1);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) a1[i] = relu_f32(a1[i], inf);
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    *reinterpret_cast<vf32x4*>(&s.h1[n * VjpF32Lds::LH + 16 * g + 4 * q]) = vf32x4{a1[4 * q], a1[4 * q + 1], a1[4 * q + 2], a1[4 * q + 3]};
-
-  __builtin_amdgcn_sched_barrier(0);     // (the phases one after the other: interleaved they need 100 registers more)
-  // ---- D2 record-major -> D1 unit-major
-  vf32x16 t2 = mfma_f32(w.w3r[0], d_op[0], zero);
-  t2 = mfma_f32(w.w3r[1], d_op[1], t2);
-  const uint32_t word2 = r.mask2 >> g;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) t2[i] = where_bit(t2[i], word2, 2 * i);
-  vf32x16 dd1 = mfma_f32(t2[0], w.w2t[0], zero);
-#pragma unroll
-  for (int i = 1; i < 16; ++i) dd1 = mfma_f32(t2[i], w.w2t[i], dd1);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int4 m = *reinterpret_cast<const int4*>(&s.mask[0][8 * q + 4 * g]);
-    dd1[4 * q] = where_bit(dd1[4 * q], (uint32_t)m.x, n);
-    dd1[4 * q + 1] = where_bit(dd1[4 * q + 1], (uint32_t)m.y, n);
-    dd1[4 * q + 2] = where_bit(dd1[4 * q + 2], (uint32_t)m.z, n);
-    dd1[4 * q + 3] = where_bit(dd1[4 * q + 3], (uint32_t)m.w, n);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  // ---- layer 2 unit-major, straight into the W3 gradient
-  vf32x16 e = mfma_f32(a1[0], w.w2[0], splat16(w.bias2));
-#pragma unroll
-  for (int i = 1; i < 16; ++i) e = mfma_f32(a1[i], w.w2[i], e);
-  const float* d3 = &s.d3[16 * g + (lane & 3)];
-#pragma unroll
-  for (int i = 0; i < 16; ++i)
-    sum.gw3 = __builtin_amdgcn_mfma_f32_4x4x1f32(d3[4 * (8 * (i >> 2) + (i & 3))], relu_f32(e[i], inf), sum.gw3, 0, 0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  // ---- D2 unit-major and the W2 gradient
-  vf32x16 dd2 = mfma_f32(d_op[0], w.w3u[0], zero);
-  dd2 = mfma_f32(d_op[1], w.w3u[1], dd2);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int4 m = *reinterpret_cast<const int4*>(&s.mask[1][8 * q + 4 * g]);
-    dd2[4 * q] = where_bit(dd2[4 * q], (uint32_t)m.x, n);
-    dd2[4 * q + 1] = where_bit(dd2[4 * q + 1], (uint32_t)m.y, n);
-    dd2[4 * q + 2] = where_bit(dd2[4 * q + 2], (uint32_t)m.z, n);
-    dd2[4 * q + 3] = where_bit(dd2[4 * q + 3], (uint32_t)m.w, n);
-  }
-  // register i of lane group g is record 8 (i / 4) + 4 g + i % 4.  The 8 last encoding columns: k-slot l / 16 of a 16x16x4
-  // product takes the units 16 (k & 1) + 0..15 of record group k >> 1
-  const float* h1 = &s.h1[4 * g * VjpF32Lds::LH + 16 * (n & 1) + (n >> 1)];
-  const float* enc = &s.enc[4 * g * VjpF32Lds::LE + n];
-  const float* enc_last = &s.enc[4 * g * VjpF32Lds::LE + (((lane >> 3) & 1) == ((lane >> 4) & 1) ? 64 + (lane & 7) : 72)];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-    const int row = 8 * (i >> 2) + (i & 3);
-    sum.gw1[0] = mfma_f32(dd1[i], enc[row * VjpF32Lds::LE], sum.gw1[0]);
-    sum.gw1[1] = mfma_f32(dd1[i], enc[row * VjpF32Lds::LE + 32], sum.gw1[1]);
-    sum.gw1e = __builtin_amdgcn_mfma_f32_16x16x4f32(dd1[i], enc_last[row * VjpF32Lds::LE], sum.gw1e, 0, 0, 0);
-    sum.gw2 = mfma_f32(dd2[i], h1[row * VjpF32Lds::LH], sum.gw2);
-    sum.gb1 += dd1[i];
-    sum.gb2 += dd2[i];
-  }
-}
-
-__device__ __forceinline__ bool vjp_f32_store(const VjpF32Sums& sum, const GradRows& out, float inv, int lane) {
-  const int n = lane & 31, g = lane >> 5;
-  bool bad = false;
-  const auto put = [&](float* dst, float v) {
-    bad |= !(__builtin_fabsf(v) <= 3.4028235e38f);
-    *dst = v;
-  };
-  const auto column = [](int k) { return (k & 1) * 36 + 18 * (k / 36) + ((k % 36) >> 1); };   // of encoding index k
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = 8 * (i >> 2) + 4 * g + (i & 3);
-    put(out.W1 + row * 72 + column(n), sum.gw1[0][i] * inv);
-    put(out.W1 + row * 72 + column(32 + n), sum.gw1[1][i] * inv);
-    put(out.W2 + row * 32 + n, sum.gw2[i] * inv);
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = (lane & 8 ? 16 : 0) + 4 * (lane >> 4) + r;
-    put(out.W1 + row * 72 + column(64 + (lane & 7)), sum.gw1e[r] * inv);
-    const float v = sum.gw3[r] + __shfl_xor(sum.gw3[r], 32);
-    if (g == 0) put(out.W3 + r * 32 + n, v * inv);
-  }
-  const float gb1 = sum.gb1 + __shfl_xor(sum.gb1, 32), gb2 = sum.gb2 + __shfl_xor(sum.gb2, 32);
-  put((g ? out.b2 : out.b1) + n, (g ? gb2 : gb1) * inv);
-#pragma unroll
-  for (int o = 0; o < 4; ++o) {
-    float v = sum.gb3[o];
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-    if (lane == o) put(out.b3 + o, v * inv);
-  }
-  return bad;
-}
-
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp_f32_kernel(
+__global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp_f32_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int H, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
     int32_t* __restrict__ nonfinite) {
-  __shared__ VjpF32Lds s;
-  const int lane = threadIdx.x, n = lane & 31, g = lane >> 5, chunk = blockIdx.x;
-  const int chunk_end = min(S, (chunk + 1) * chunk_steps);
-  if (g == 0) *reinterpret_cast<vf32x4*>(&s.enc[n * VjpF32Lds::LE + 72]) = vf32x4{0.f, 0.f, 0.f, 0.f};
+  __shared__ Vjp32Lds s;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, g = lane >> 5;
+  const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
+  const SplitUnits u;
+  float factor[6];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) factor[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(freq[f] * att[f])));
+  if (t < 4) s.zero[t] = 0u;
   bool bad = false;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);
-    VjpF32Operands w;
-    w.load(W1, b1, W2, b2, W3, (size_t)run.p, lane, s);
-    VjpF32Sums sum;
+    vjp32_load(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane, s, u);
+    Vjp32Sums sum;
     sum.clear();
-    walk_run(ix, run, records, d4, rays_d, n, g, W, W * H,
-             [&](const StepRecord& r) { vjp_f32_block(w, sum, s, r, freq, att, scale, lane); });
-    bad |= vjp_f32_store(sum, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, lane);
+    __syncthreads();
+    int turn = wave / 4;
+    walk_halves<kVjp32Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
+      // (the two wavefronts of a SIMD take turns at priority, or one of them is blocks ahead when the other ends: 5.56 ms
+      // for the gradient call instead of 5.40)
+      if (turn & 1) __builtin_amdgcn_s_setprio(1);
+      else __builtin_amdgcn_s_setprio(0);
+      ++turn;
+      vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factor, scale, lane, u);
+    });
+    const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
+    if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
+    __syncthreads();
+    bad |= vjp32_store(s, waves, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t);
     pos = run.end;
+    __syncthreads();
   }
   if (__ballot(bad) != 0ull && lane == 0) atomicOr(nonfinite, 1);
 }
@@ -717,6 +559,12 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
 inline int train_chunk_steps(int64_t S) {
   const int64_t per = S / 8192;
   return per >= 16 ? 16 : per <= 4 ? 4 : (int)per;
+}
+// ... of the f32 kernel, whose workgroup of eight wavefronts fills a CU: 256 (2,048 records to a wavefront; 128: 5.58 instead of
+// 5.52 ms), fewer where that would leave fewer than eight chunks for each of the 256 CUs, 16 at the least.
+inline int train_chunk_steps_f32(int64_t S) {
+  const int64_t per = S / 2048 / kVjp32Waves * kVjp32Waves;
+  return per >= 32 * kVjp32Waves ? 32 * kVjp32Waves : per <= 2 * kVjp32Waves ? 2 * kVjp32Waves : (int)per;
 }
 
 // The sorted steps, then head and tail rows of every chunk.
@@ -848,20 +696,26 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
   const GradRows grads{gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
   const GeoGrads geo{grad_positions_dev, grad_log_scales_dev, grad_quats_dev};
   const int S = (int)num_steps;
-  if (t.num_chunks > 0) {
-#define MLPSP_TRAIN_VJP(KERNEL)                                                                                         \
-  hipLaunchKernelGGL(KERNEL, dim3((unsigned)t.num_chunks), dim3(64), 0, s, ix, S, t.chunk_steps, t.num_chunks, sp.records, \
+  const int chunk_steps = precision == 0 ? train_chunk_steps_f32(S) : t.chunk_steps;
+  const int num_chunks = (int)(((int64_t)S + chunk_steps - 1) / chunk_steps);      // (the rows are carved for the shorter chunks)
+  if (num_chunks > 0) {
+#define MLPSP_TRAIN_VJP(KERNEL, THREADS)                                                                                \
+  hipLaunchKernelGGL(KERNEL, dim3((unsigned)num_chunks), dim3(THREADS), 0, s, ix, S, chunk_steps, num_chunks, sp.records, \
                      (const float4*)d4_dev, rays_d_dev, width, height, freq_dev, att_dev, W1, b1, W2, b2, W3, scale,   \
                      t.rows, grads, nonfinite_dev)
-    if (precision == 0) MLPSP_TRAIN_VJP(train_vjp_f32_kernel);
-    else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>));
-    else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>));
+    if (precision == 0) MLPSP_TRAIN_VJP(train_vjp_f32_kernel, 64 * kVjp32Waves);
+    else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>), 64);
+    else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>), 64);
 #undef MLPSP_TRAIN_VJP
     MLPSP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(train_geometry_kernel, dim3((unsigned)((t.num_chunks + 3) / 4)), dim3(256), 0, s, ix, S, t.chunk_steps,
-                       t.num_chunks, sp.records, falloff_dev, log_scales_dev, quats_dev, t.rows, geo);
+#define MLPSP_TRAIN_GEOMETRY(WAVES)                                                                                     \
+  hipLaunchKernelGGL(train_geometry_kernel<WAVES>, dim3((unsigned)num_chunks), dim3(64 * WAVES), 0, s, ix, S, chunk_steps, \
+                     num_chunks, sp.records, falloff_dev, log_scales_dev, quats_dev, t.rows, geo)
+    if (precision == 0) MLPSP_TRAIN_GEOMETRY(4);
+    else MLPSP_TRAIN_GEOMETRY(1);
+#undef MLPSP_TRAIN_GEOMETRY
     MLPSP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)t.num_chunks, 4), dim3(256), 0, s, ix, S, t.chunk_steps, t.num_chunks,
+    hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)num_chunks, 4), dim3(256), 0, s, ix, S, chunk_steps, num_chunks,
                        t.rows, quats_dev, grads, geo, nonfinite_dev);
     MLPSP_LAUNCH_CHECK();
   }

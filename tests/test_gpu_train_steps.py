@@ -259,6 +259,58 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
     assert not bool(torch.isfinite(ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)[0]))
 
 
+@pytest.mark.parametrize("tiles", [1, 3, 4, 5, 15, 16, 17, 31, 129, 255])
+def test_f32_weight_gradients_of_runs_of_every_length(device, tiles):
+    """The f32 kernel deals a run's half steps to eight wavefronts and cuts the steps into chunks of 16 to 256: runs of one
+    primitive that are a little shorter and longer than those, three in a row, against float64 over the same steps.  An f32
+    gradient is a sum of up to 16,000 products of two factors that are f32 sums of up to 72 terms themselves: a few units of
+    2^-24 each, 1e-6 of the norm.  A phase is an f32 product of two roundings, and moves its sine by as much: 2^-23 times the
+    largest phase."""
+    import numpy as np
+    from mlp_splatting_amd import ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    n, width, height = 3, 8 * tiles, 8
+    sc = syn.make_scene(n, 32, seed=5, log_scale_mean=2.5)
+    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
+    sc.b3[:, 3] = -6.0
+    c2w = syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0))
+    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, c2w)
+    cand, off = np.tile(np.arange(n, dtype=np.int32), tiles), np.arange(tiles + 1, dtype=np.int32) * n
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats, cand, off, sc.freq,
+                                        sc.att, *sc.mlp())]
+    ext = TileExt()
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0, render_order=True)
+    _, _, frame = ext.train_forward(base, width, height, 1e-3)
+    assert frame.steps == n * tiles
+    g = torch.Generator().manual_seed(6)
+    g_rgb, g_t = torch.randn(width * height, 3, generator=g).to(device), torch.randn(width * height, generator=g).to(device)
+    d4, falloff = ops.train_reverse(frame, base[6], g_rgb, g_t)
+    got, flag = ops.train_gradients(frame, ops.train_group(frame, base[6], n), d4, falloff, base[1], base[7], base[8], base[9:15],
+                                    base[3], base[4], 0, 1.0)
+    assert int(flag) == 0
+    # d4 is [tile, step of the tile, lane]; the records are [pixel, hit], and every pixel hits all three, in the tile's order
+    ids, x6 = records[2].view(-1, n), records[3].view(-1, n, 6)
+    assert records[2].numel() == n * width * height
+    pixel = torch.arange(width * height, device=device)
+    tile, lane = (pixel % width) // 8, pixel // width * 8 + pixel % 8
+    adjoint = d4.view(tiles, n, 64, 4)[tile[:, None], torch.arange(n, device=device)[None], lane[:, None]].double()
+    W1, b1, W2, b2, W3, _ = (w.double() for w in base[9:15])
+    for p in range(n):
+        at = (ids == p).nonzero(as_tuple=True)
+        phase = (x6[at].double()[:, :, None] * base[7].double() * base[8].double()).reshape(-1, 36)
+        enc, d = torch.cat([phase.sin(), phase.cos()], 1), adjoint[at]
+        z1 = enc @ W1[p].T + b1[p]
+        bound = 1e-6 + 2.0 ** -23 * float(phase.abs().max())
+        h1 = z1.clamp(min=0.0)
+        z2 = h1 @ W2[p].T + b2[p]
+        d2 = (d @ W3[p]) * (z2 > 0)
+        d1 = (d2 @ W2[p]) * (z1 > 0)
+        want = [d1.T @ enc, d1.sum(0), d2.T @ h1, d2.sum(0), d.T @ z2.clamp(min=0.0), d.sum(0)]
+        for i, (a, b) in enumerate(zip(got, want)):
+            assert float((a[p].double() - b).norm()) <= bound * float(b.norm()), (p, i)
+
+
 # every tile by a team (40 and 1,681 tiles), then most by one wavefront (2,050 tiles, in rows of 50 and one of 2,050)
 @pytest.mark.parametrize("width,height", [(61, 40), (328, 325), (400, 325), (16397, 5)])
 def test_tiles_of_every_length_take_the_chunks_they_need(device, width, height):
