@@ -15,8 +15,7 @@
 // moved into operand position by one half-wave swap per sin/cos pair; the same swap brings the 32 layer-2
 // outputs of a pixel onto its own lane for the 4-wide output layer, which runs on the vector ALU with
 // scalar weight operands.
-// With 16 hidden units the same tiles are half filled: A rows 16..31 are zero, accumulator registers 8..15 are
-// never read, layer 2 is eight instructions.  The order of every sum is unchanged.
+// 16 hidden units run on the 16x16x4 form (mlp_wave_mfma16x4 below).
 #pragma once
 #include "mlpsp_device.hpp"
 
@@ -35,6 +34,13 @@ __device__ __forceinline__ void half_swap(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
   a = r[0];
   b = r[1];
+}
+
+// Exchanges the odd rows of 16 lanes of a with the even rows of b.
+__device__ __forceinline__ void row_swap(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
 }
 
 // 16 consecutive floats at src + 16 g, as loaded (c[q] = floats 4q .. 4q+3)  ->  element i = src[2i + g]
@@ -56,67 +62,37 @@ __device__ __forceinline__ void interleave16(const mf32x4 c4[4], float v[16]) {
   }
 }
 
-// 8 consecutive floats at src + 8 g, as loaded  ->  element i = src[2i + g], i < 8 (the rest of v is left alone).
-__device__ __forceinline__ void interleave8(const mf32x4 c4[2], float v[16]) {
-  float c[8];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    c[4 * q + 0] = c4[q][0];
-    c[4 * q + 1] = c4[q][1];
-    c[4 * q + 2] = c4[q][2];
-    c[4 * q + 3] = c4[q][3];
-  }
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    half_swap(c[2 * t], c[2 * t + 1]);   // c[2t] = (src[2t], src[2t+1]), c[2t+1] = (src[8+2t], src[9+2t])
-    v[t] = c[2 * t];
-    v[4 + t] = c[2 * t + 1];
-  }
-}
-template <int H>
-__device__ __forceinline__ void interleave(const mf32x4 c4[H / 8], float v[16]) {
-  if constexpr (H == 32) interleave16(c4, v);
-  else interleave8(c4, v);
-}
-
 // What one lane loads of a primitive's layers 1 and 2, as the loads deliver it: row `hid` of W1 (its half g) and
 // the first bias vector (its half g); the same row of W2 and the second bias vector.  Requesting is separate from
 // using, and layer 1 from layer 2: a caller can have the next primitive's layer-1 operands under way while it
 // evaluates this one, and layer 2's arrive behind layer 1's instructions anyway.
-template <int H>
 struct MlpLayer1 {
-  mf32x4 a1[9], b1[H / 8];
+  mf32x4 a1[9], b1[4];
 };
-template <int H>
 struct MlpLayer2 {
-  mf32x4 a2[H / 8], b2[H / 8];
+  mf32x4 a2[4], b2[4];
 };
 // Hidden unit whose weight row lane (m, g) supplies.
 __device__ __forceinline__ int mfma32_hidden_row(int m) { return 8 * (m >> 3) + 2 * (m & 3) + ((m >> 2) & 1); }
-template <int H>
 __device__ __forceinline__ void request_layer1(const float* __restrict__ W1, const float* __restrict__ b1, int p,
-                                               MlpLayer1<H>& o) {
-  constexpr int IN = 72, HALF = 36;
+                                               MlpLayer1& o) {
   const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
-  const int hid = mfma32_hidden_row(m);
-  const int row = hid < H ? hid : 0;                       // unused rows read row 0 and supply zeros
-  const mf32x4* __restrict__ s1 = reinterpret_cast<const mf32x4*>(W1 + (size_t)p * (H * IN) + row * IN + HALF * g);
+  const mf32x4* __restrict__ s1 =
+      reinterpret_cast<const mf32x4*>(W1 + (size_t)p * (32 * 72) + mfma32_hidden_row(m) * 72 + 36 * g);
 #pragma unroll
   for (int q = 0; q < 9; ++q) o.a1[q] = s1[q];
-  const mf32x4* __restrict__ sb1 = reinterpret_cast<const mf32x4*>(b1 + (size_t)p * H + (H / 2) * g);
+  const mf32x4* __restrict__ sb1 = reinterpret_cast<const mf32x4*>(b1 + (size_t)p * 32 + 16 * g);
 #pragma unroll
-  for (int q = 0; q < H / 8; ++q) o.b1[q] = sb1[q];
+  for (int q = 0; q < 4; ++q) o.b1[q] = sb1[q];
 }
-template <int H>
 __device__ __forceinline__ void request_layer2(const float* __restrict__ W2, const float* __restrict__ b2, int p,
-                                               MlpLayer2<H>& o) {
+                                               MlpLayer2& o) {
   const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
-  const int hid = mfma32_hidden_row(m);
-  const int row = hid < H ? hid : 0;
-  const mf32x4* __restrict__ s2 = reinterpret_cast<const mf32x4*>(W2 + (size_t)p * (H * H) + row * H + (H / 2) * g);
-  const mf32x4* __restrict__ sb2 = reinterpret_cast<const mf32x4*>(b2 + (size_t)p * H + (H / 2) * g);
+  const mf32x4* __restrict__ s2 =
+      reinterpret_cast<const mf32x4*>(W2 + (size_t)p * (32 * 32) + mfma32_hidden_row(m) * 32 + 16 * g);
+  const mf32x4* __restrict__ sb2 = reinterpret_cast<const mf32x4*>(b2 + (size_t)p * 32 + 16 * g);
 #pragma unroll
-  for (int q = 0; q < H / 8; ++q) {
+  for (int q = 0; q < 4; ++q) {
     o.a2[q] = s2[q];
     o.b2[q] = sb2[q];
   }
@@ -187,8 +163,17 @@ __device__ __forceinline__ void encode_component(float x, const float* __restric
 // per 16-byte read.  Written and read by one wavefront: no barrier.  (36 registers less than keeping them: a fourth
 // wavefront per SIMD.)
 struct DirOperands {
-  mf32x4 q[9][64];       // [i]: blocks 0 and 1 of pairs 2i and 2i + 1 = (b0[2i], b1[2i], b0[2i+1], b1[2i+1])
-};
+  mf32x4 q[9][64];       // [i]: pairs 2i and 2i + 1.  32 hidden units: blocks 0 and 1 of either = (b0[2i], b1[2i], b0[2i+1],
+};                       // b1[2i+1]); 16: blocks 0 .. 3 of the two together (mlp_wave_mfma16x4)
+// Four values of every pixel, exchanged between the four rows of 16 lanes: afterwards lane (c, q) holds in v[b] what lane
+// (c, b) = pixel 16 b + c had in v[q].
+__device__ __forceinline__ void row_transpose(float v[4]) {
+  half_swap(v[0], v[2]);
+  half_swap(v[1], v[3]);
+  row_swap(v[0], v[1]);
+  row_swap(v[2], v[3]);
+}
+template <int HID = 32>
 __device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz, const float* __restrict__ freq,
                                                  const float* __restrict__ att, DirOperands& d) {
   const int lane = threadIdx.x & 63;
@@ -196,10 +181,16 @@ __device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz
   for (int c = 0; c < 3; ++c) {
     float s[6], co[6];
     encode_component(c == 0 ? x3[0] : c == 1 ? x3[1] : x3[2], freq, att, s, co);
+    if constexpr (HID == 32) {
 #pragma unroll
-    for (int f = 0; f < 6; ++f) half_swap(s[f], co[f]);
+      for (int f = 0; f < 6; ++f) half_swap(s[f], co[f]);
+    }
 #pragma unroll
-    for (int f = 0; f < 6; f += 2) d.q[3 * c + f / 2][lane] = mf32x4{s[f], co[f], s[f + 1], co[f + 1]};
+    for (int f = 0; f < 6; f += 2) {
+      float v[4] = {s[f], co[f], s[f + 1], co[f + 1]};
+      if constexpr (HID == 16) row_transpose(v);
+      d.q[3 * c + f / 2][lane] = mf32x4{v[0], v[1], v[2], v[3]};
+    }
   }
 }
 
@@ -208,32 +199,30 @@ __device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz
 // operands as request_layer1() loaded them; layer2(w2) requests those of layer 2.
 // REC selects the record kernels' layer-2 rounding (bias added after a chain started at zero); MASKS fills
 // masks[0..1] with the ReLU masks of the lane's pixel.
-template <bool REC = false, bool MASKS = REC, int HID = 32, typename RequestLayer2>
-__device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, RequestLayer2&& layer2, const float x6[6],
+template <bool REC = false, bool MASKS = REC, typename RequestLayer2>
+__device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1& w1, RequestLayer2&& layer2, const float x6[6],
                                                      const float* __restrict__ freq, const float* __restrict__ att,
                                                      const float* __restrict__ W3, const float* __restrict__ b3, int p,
                                                      const DirOperands& dir, float out[4], uint32_t* masks = nullptr) {
-  static_assert(HID == 32 || HID == 16, "hidden width of the matrix-core f32 evaluation");
-  constexpr int H = HID, R = H / 2;   // R: accumulator registers in use (hidden units 2i + g)
-  const int lane = threadIdx.x & 63, m = lane & 31, g = lane >> 5;
-  const bool row_used = mfma32_hidden_row(m) < H;          // (always, with 32 hidden units)
+  constexpr int H = 32, R = H / 2;    // R: accumulator registers (hidden units 2i + g)
+  const int lane = threadIdx.x & 63, g = lane >> 5;
   const float inf = relu_limit();
 
   // A operands: lane (m, g) supplies row hid, k = g of every instruction.
   float a1[36];
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
-    a1[4 * q + 0] = row_used ? w1.a1[q][0] : 0.f;
-    a1[4 * q + 1] = row_used ? w1.a1[q][1] : 0.f;
-    a1[4 * q + 2] = row_used ? w1.a1[q][2] : 0.f;
-    a1[4 * q + 3] = row_used ? w1.a1[q][3] : 0.f;
+    a1[4 * q + 0] = w1.a1[q][0];
+    a1[4 * q + 1] = w1.a1[q][1];
+    a1[4 * q + 2] = w1.a1[q][2];
+    a1[4 * q + 3] = w1.a1[q][3];
   }
-  float bias1[16] = {};
-  interleave<H>(w1.b1, bias1);
+  float bias1[16];
+  interleave16(w1.b1, bias1);
 
   mf32x16 d0, d1;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) d0[i] = d1[i] = (i < R) ? bias1[i] : 0.f;
+  for (int i = 0; i < 16; ++i) d0[i] = d1[i] = bias1[i];
   // (the lane index is made opaque so that the reads stay here and are not hoisted out of the primitive loop)
   int ll = lane;
   asm volatile("" : "+v"(ll));
@@ -245,7 +234,7 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, R
     d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i + 1], q[2], d0, 0, 0, 0);
     d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[2 * i + 1], q[3], d1, 0, 0, 0);
   }
-  MlpLayer2<HID> w2;
+  MlpLayer2 w2;
 #pragma unroll
   for (int c = 3; c < 6; ++c) {
     // (layer 2's operands are requested behind five sixths of layer 1, and not before: 32 registers)
@@ -261,16 +250,12 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, R
     }
   }
 
-  float a2[16] = {}, bias2[16] = {};
-  interleave<H>(w2.a2, a2);
-  interleave<H>(w2.b2, bias2);
-  if constexpr (H != 32) {
-#pragma unroll
-    for (int i = 0; i < R; ++i) a2[i] = row_used ? a2[i] : 0.f;
-  }
+  float a2[16], bias2[16];
+  interleave16(w2.a2, a2);
+  interleave16(w2.b2, bias2);
   mf32x16 e0, e1;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) e0[i] = e1[i] = (REC || i >= R) ? 0.f : bias2[i];
+  for (int i = 0; i < 16; ++i) e0[i] = e1[i] = REC ? 0.f : bias2[i];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     e0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[i], relu_f32(d0[i], inf), e0, 0, 0, 0);
@@ -315,6 +300,82 @@ __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1<HID>& w1, R
   }
 }
 
+// The 72->16->16->4 MLP, the same contract: v_mfma_f32_16x16x4_f32 is four consecutive links of the chain, k = 0 .. 3 (one
+// rounding each, as the 32x32x2's two), in 32 clocks, and has no half-filled rows: four column blocks of 16 pixels, 18
+// instructions a block for layer 1 and four for layer 2, 2,816 clocks per evaluation where half-filled 32x32x2 tiles take
+// 5,632 (frame of 5,000 primitives, 160x120: 268 -> 242 us; nine exchanges of rows more take back a tenth).  Lane (c, q) = (lane % 16, lane / 16) of an accumulator tile holds column c and rows 4 q + r in register r; with row
+// 4 q + r = hidden unit 4 r + q that is the operand (k = q) of the next layer's r-th instruction.
+__device__ __forceinline__ void mlp_wave_mfma16x4(const float x6[6], const float* __restrict__ freq, const float* __restrict__ att,
+                                                  const float* __restrict__ W1, const float* __restrict__ b1,
+                                                  const float* __restrict__ W2, const float* __restrict__ b2,
+                                                  const float* __restrict__ W3, const float* __restrict__ b3, int p,
+                                                  const DirOperands& dir, float out[4]) {
+  const int lane = threadIdx.x & 63, c16 = lane & 15, q = lane >> 4;
+  const int unit = 4 * (c16 & 3) + (c16 >> 2);
+  const float inf = relu_limit();
+  // W1: k-slots 0 .. 3 of instruction j = sine and cosine of pairs 2 j, 2 j + 1: every other entry of a half row
+  const mf32x4* __restrict__ s1 = reinterpret_cast<const mf32x4*>(W1 + (size_t)p * (16 * 72) + unit * 72 + 36 * (q & 1));
+  float a1[18];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const mf32x4 v = s1[i];
+    a1[2 * i] = q & 2 ? v[1] : v[0];
+    a1[2 * i + 1] = q & 2 ? v[3] : v[2];
+  }
+  float bias1[4], a2[4], bias2[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    bias1[i] = b1[(size_t)p * 16 + 4 * i + q];
+    a2[i] = W2[(size_t)p * 256 + unit * 16 + 4 * i + q];
+    bias2[i] = b2[(size_t)p * 16 + 4 * i + q];
+  }
+  mf32x4 d[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) d[b] = mf32x4{bias1[0], bias1[1], bias1[2], bias1[3]};
+  int ll = lane;                         // (opaque: the reads stay here and are not hoisted out of the primitive loop)
+  asm volatile("" : "+v"(ll));
+#pragma unroll
+  for (int j = 0; j < 9; ++j) {
+    const mf32x4 x = dir.q[j][ll];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[j], x[b], d[b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int c = 3; c < 6; ++c) {
+    float sn[6], cs[6];
+    encode_component(x6[c], freq, att, sn, cs);
+#pragma unroll
+    for (int f = 0; f < 6; f += 2) {
+      float v[4] = {sn[f], cs[f], sn[f + 1], cs[f + 1]};
+      row_transpose(v);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) d[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[3 * c + f / 2], v[b], d[b], 0, 0, 0);
+    }
+  }
+  mf32x4 e[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) e[b] = mf32x4{bias2[0], bias2[1], bias2[2], bias2[3]};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) e[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[i], relu_f32(d[b][i], inf), e[b], 0, 0, 0);
+  // output layer on the lane's own pixel
+  const float* __restrict__ w3 = W3 + (size_t)p * 64;
+  const float* __restrict__ bb3 = b3 + (size_t)p * 4;
+  float acc[4] = {bb3[0], bb3[1], bb3[2], bb3[3]};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float h[4] = {relu_f32(e[0][i], inf), relu_f32(e[1][i], inf), relu_f32(e[2][i], inf), relu_f32(e[3][i], inf)};
+    row_transpose(h);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[k] = fmaf(w3[k * 16 + 4 * i + u], h[u], acc[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) out[k] = acc[k];
+}
+
 // The same with the operands requested here.
 template <bool REC = false, bool MASKS = REC, int HID = 32>
 __device__ __forceinline__ void mlp_wave_mfma32(const float x6[6], const float* __restrict__ freq,
@@ -323,13 +384,18 @@ __device__ __forceinline__ void mlp_wave_mfma32(const float x6[6], const float* 
                                                 const float* __restrict__ b2, const float* __restrict__ W3,
                                                 const float* __restrict__ b3, int p, const DirOperands& dir,
                                                 float out[4], uint32_t* masks = nullptr) {
-  MlpLayer1<HID> w1;
-  request_layer1<HID>(W1, b1, p, w1);
-  const auto layer2 = [&](MlpLayer2<HID>& w2) {
-    __builtin_amdgcn_sched_barrier(0);
-    request_layer2<HID>(W2, b2, p, w2);
-  };
-  mlp_wave_mfma32_with<REC, MASKS, HID>(w1, layer2, x6, freq, att, W3, b3, p, dir, out, masks);
+  static_assert(HID == 32 || (HID == 16 && !REC && !MASKS), "hidden width of the matrix-core f32 evaluation");
+  if constexpr (HID == 16) {
+    mlp_wave_mfma16x4(x6, freq, att, W1, b1, W2, b2, W3, b3, p, dir, out);
+  } else {
+    MlpLayer1 w1;
+    request_layer1(W1, b1, p, w1);
+    const auto layer2 = [&](MlpLayer2& w2) {
+      __builtin_amdgcn_sched_barrier(0);
+      request_layer2(W2, b2, p, w2);
+    };
+    mlp_wave_mfma32_with<REC, MASKS>(w1, layer2, x6, freq, att, W3, b3, p, dir, out, masks);
+  }
 }
 
 }  // namespace mlpsp

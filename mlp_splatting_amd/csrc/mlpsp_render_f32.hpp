@@ -205,7 +205,7 @@ __device__ __forceinline__ void render_item_f32(
     if (valid) gt = load3(stats.gt_rgb, pix);
   }
   HitEmitter em = hit_emitter_begin(hp, wslot, start, tile);
-  encode_direction(rd.x, rd.y, rd.z, freq, att, s_dir);
+  encode_direction<HT>(rd.x, rd.y, rd.z, freq, att, s_dir);
 
   walk_tile_f32(
       order, start, end, N, prims, valid, ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, thr, s_walk,
@@ -317,7 +317,7 @@ __device__ __forceinline__ void render_team_item_f32(
   PixelAcc acc = {0.f, 0.f, 0.f, 1.f, 0.f, 0.f};
   unsigned n_proc = 0, n_proc_hit = 0, n_hits = 0;
   TeamSlots slots{wslot * hp.table_stride + (start >> 4) + tile, 0, 0, 0, 0};
-  if (k == 0) encode_direction(rd.x, rd.y, rd.z, freq, att, s.dir);
+  if (k == 0) encode_direction<HT>(rd.x, rd.y, rd.z, freq, att, s.dir);
 
   int p_mine = 0;
   float gates[4];
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // multiple of four, one wavefront on each SIMD of a CU (3, 6 and 8 were slower than 4, 2 as well); twelve where the items
 // are no more than the CUs.  Else the mixed kernel with a team for each of the last 1,024 items -- for all of them up to
 // 1,280 --, which shortens the tail of the launch: what is left when the queue is empty lasts a third as long.  Frame in us,
-// one wavefront per item / teams of four / mixed: 96 items 690 / 315 (of twelve 264), 300 items hidden 16 495 / 268, 588
+// one wavefront per item / teams of four / mixed: 96 items 690 / 315 (of twelve 264), 300 items hidden 16 455 / 260, 588
 // items 780 / 512, 1,200 items 1,020 / 744 / 785, 1,610 items 980 / 901 / 841, 2,214 items 1,086 / 1,070 / 985, 4,860 items
 // 1,840 / 2,128 / 1,766, 12,750 items 4,034 / 5,065 / 3,945; with 768 and 1,536 instead of 1,024 items 4,020 and 3,955.
 // MLPSP_F32_AHEAD=0 / 1 / 2 in the environment: a wavefront per item throughout / four / twelve (comparison runs, tests).
