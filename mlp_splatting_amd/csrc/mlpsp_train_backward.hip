@@ -3,8 +3,9 @@
 // grouped gradient kernels (scannet/primitive_gemm.py:101-183) in one pipeline whose unit is a step, not a record.
 //
 // The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal
-// length.  A wavefront (f32 weights: a workgroup) walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the primitive's steps all lie in the chunk, else to the chunk's tail row
-// (the primitive goes on in the next chunk) or head row (it ended here).  Two more launches add the rows of the primitives
+// length.  A workgroup walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the
+// primitive's steps all lie in the chunk, else to the chunk's tail row (the primitive goes on in the next chunk) or head row
+// (it ended here).  Two more launches add the rows of the primitives
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
@@ -14,6 +15,7 @@
 #include "mlpsp_mlp_mfma32.hpp"
 #include "mlpsp_train.hpp"
 #include "mlpsp_vjp16.hpp"
+#include "mlpsp_vjp16_steps.hpp"
 #include "mlpsp_vjp32.hpp"
 
 namespace mlpsp {
@@ -271,13 +273,13 @@ __device__ __forceinline__ void geometry_store(const float v[15], float qw, floa
                         r12 * (2.f * qy) + r20 * (2.f * qx) + r21 * (2.f * qy);
 }
 
-// A workgroup per chunk, the steps of a run to its wavefronts in turn: one for chunks of 16 steps, four for 256.
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void train_geometry_kernel(
+// A workgroup per chunk, the steps of a run to its wavefronts in turn.
+constexpr int kGeoWaves = 4;
+__global__ __launch_bounds__(64 * kGeoWaves) void train_geometry_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float* __restrict__ falloff, const float* __restrict__ logs, const float* __restrict__ quats,
     float* __restrict__ rows, GeoGrads out) {
-  __shared__ float s_sum[2][WAVES][16];
+  __shared__ float s_sum[2][kGeoWaves][16];
   const int chunk = (int)blockIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63;
   const int chunk_end = min(S, (chunk + 1) * chunk_steps);
   int turn = 0;
@@ -290,7 +292,7 @@ __global__ __launch_bounds__(64 * WAVES) void train_geometry_kernel(
 #pragma unroll
     for (int k = 0; k < 15; ++k) v[k] = 0.f;
 #pragma unroll 2
-    for (int k = run.begin + wave; k < run.end; k += WAVES) {
+    for (int k = run.begin + wave; k < run.end; k += kGeoWaves) {
       const int4 at = ix.step[k];
       const float4 c = reinterpret_cast<const float4*>(records + (size_t)at.x * kStepBytes + kStepPlaneC)[l];
       const float a = falloff[(size_t)at.y * 64 + l];
@@ -318,12 +320,12 @@ __global__ __launch_bounds__(64 * WAVES) void train_geometry_kernel(
       for (int k = 1; k < 15; ++k) mine = (l == k) ? v[k] : mine;
       s_sum[turn][wave][l] = mine;
     }
-    if constexpr (WAVES > 1) __syncthreads();      // (the one barrier of a turn: the next writes the other half)
+    __syncthreads();                   // (the one barrier of a turn: the next writes the other half)
     if (wave == 0) {
       float total = 0.f;
       if (l < 15) {
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) total += s_sum[turn][w][l];
+        for (int w = 0; w < kGeoWaves; ++w) total += s_sum[turn][w][l];
       }
       if (!run.complete) {
         if (l < 15) run_row(rows, run, chunk, num_chunks)[kGradFloats + l] = total;
@@ -338,9 +340,11 @@ __global__ __launch_bounds__(64 * WAVES) void train_geometry_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// MLP weight gradients, 16-bit operands: the block of mlpsp_vjp16.hpp over the two halves of a step
+// MLP weight gradients, 16-bit operands: the blocks of mlpsp_vjp16_steps.hpp.  A workgroup per chunk, half a step to a wavefront.
 // ---------------------------------------------------------------------------------------------
-// What lane (n, g) needs of record n of half h of a step: its group's three inputs, the output adjoints, the masks.
+// What lane (n, g) needs of record n of half h of a step: its group's three inputs (the ray direction, the hit offset), the
+// output adjoints, the masks.  Each lane asks for its own inputs only: chosen behind the loads of both, every request was
+// waited for as soon as it was made (f32 / 16-bit gradient call of 648,000 steps 5.40 -> 5.32 / 2.32 -> 2.18 ms).
 struct StepRecord {
   float x[3];
   float4 d;
@@ -353,68 +357,35 @@ __device__ __forceinline__ StepRecord step_record(const unsigned char* __restric
   const int px = 32 * half + n;
   const unsigned char* __restrict__ rec = records + (size_t)at.x * kStepBytes;
   r.d = d4[(size_t)at.y * 64 + px];
-  const float4 c = reinterpret_cast<const float4*>(rec + kStepPlaneC)[px];
-  r.mask1 = __float_as_uint(c.w);
+  const unsigned char* offset = rec + kStepPlaneC + 16 * px;
+  const float* dir = rays_d + 3 * (size_t)min(at.w + (px >> 3) * W + (px & 7), pixels - 1);      // (whatever it is outside the image)
+  const Float3 x = load3(g ? reinterpret_cast<const float*>(offset) : dir, 0);
+  r.x[0] = x.x;
+  r.x[1] = x.y;
+  r.x[2] = x.z;
+  r.mask1 = *reinterpret_cast<const uint32_t*>(offset + 12);
   r.mask2 = reinterpret_cast<const uint32_t*>(rec + kStepPlaneD)[px];
-  const Float3 dir = load3(rays_d, min(at.w + (px >> 3) * W + (px & 7), pixels - 1));   // (whatever it is outside the image)
-  r.x[0] = g ? c.x : dir.x;
-  r.x[1] = g ? c.y : dir.y;
-  r.x[2] = g ? c.z : dir.z;
   return r;
 }
-// The blocks of a run -- both halves of its steps -- in turn: work(record) for those that have an adjoint.  A record is
-// requested while the one before it is worked on, and where a step's parts lie one step before that (a vector load, so
-// that it is waited for in the order of the requests): with both read for one block, the 16-bit kernel took 2.16 instead
-// of 2.06 ms (648,000 steps).  Records without an adjoint get inputs of zero, whatever ray their lane has.
-template <typename Work>
-__device__ __forceinline__ void walk_run(const StepIndex& ix, const StepRun& run, const unsigned char* __restrict__ records,
-                                         const float4* __restrict__ d4, const float* __restrict__ rays_d, int n, int g, int W,
-                                         int pixels, Work&& work) {
-  int zero = 0;
-  asm volatile("" : "+v"(zero));
-  const auto where = [&](int k) { return ix.step[min(k, run.end - 1) + zero]; };
-  const auto uniform = [](int4 v) {
-    return make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y), 0, __builtin_amdgcn_readfirstlane(v.w));
-  };
-  const int blocks = 2 * (run.end - run.begin);
-  int4 at = uniform(where(run.begin)), next = where(run.begin + 1);
-  StepRecord ahead = step_record(records, d4, rays_d, at, 0, n, g, W, pixels);
-  for (int q = 0; q < blocks; ++q) {
-    StepRecord r = ahead;
-    if (q & 1) {
-      at = uniform(next);
-      next = where(run.begin + (q >> 1) + 2);
-    }
-    if (q + 1 < blocks) ahead = step_record(records, d4, rays_d, at, (q + 1) & 1, n, g, W, pixels);
-    const bool adjoint = r.d.x != 0.f || r.d.y != 0.f || r.d.z != 0.f || r.d.w != 0.f;
-    if (__ballot(adjoint) == 0ull) continue;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) r.x[c] = adjoint ? r.x[c] : 0.f;
-    work(r);
-  }
-}
-
-// ... or one half of every STRIDE-th step, from `first` on.
+// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on, 64 at the most; work(record) for those that
+// have an adjoint.  Lane i asks for where the i-th of them lies; the next record is under way while one is worked on (two or
+// three: no faster).  Records without an adjoint get inputs of zero, whatever ray their lane has.
 template <int STRIDE, typename Work>
 __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int end, int half, const unsigned char* __restrict__ records,
                                             const float4* __restrict__ d4, const float* __restrict__ rays_d, int n, int g, int W,
                                             int pixels, Work&& work) {
-  if (first >= end) return;
-  int zero = 0;
-  asm volatile("" : "+v"(zero));
-  const auto where = [&](int k) { return ix.step[min(k, end - 1) + zero]; };
-  const auto record = [&](int4 v) {
-    return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y), 0,
-                                                      __builtin_amdgcn_readfirstlane(v.w)), half, n, g, W, pixels);
+  const int count = (end - first + STRIDE - 1) / STRIDE;
+  if (count <= 0) return;
+  const int4 where = ix.step[min(first + STRIDE * (n + 32 * g), end - 1)];
+  const auto record = [&](int i) {
+    const int k = min(i, count - 1);
+    return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readlane(where.x, k), __builtin_amdgcn_readlane(where.y, k), 0,
+                                                      __builtin_amdgcn_readlane(where.w, k)), half, n, g, W, pixels);
   };
-  StepRecord ahead = record(where(first));
-  int4 next = where(first + STRIDE);
-  for (int k = first; k < end; k += STRIDE) {
-    StepRecord r = ahead;
-    if (k + STRIDE < end) {
-      ahead = record(next);
-      next = where(k + 2 * STRIDE);
-    }
+  StepRecord next = record(0);
+  for (int i = 0; i < count; ++i) {
+    StepRecord r = next;
+    next = record(i + 1);          // (at the end the last one again: under a condition the request is waited for)
     const bool adjoint = r.d.x != 0.f || r.d.y != 0.f || r.d.z != 0.f || r.d.w != 0.f;
     if (__ballot(adjoint) == 0ull) continue;
 #pragma unroll
@@ -424,32 +395,49 @@ __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int 
 }
 
 template <typename T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp16_kernel(
+__global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp16_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int H, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
     int32_t* __restrict__ nonfinite) {
-  __shared__ __attribute__((aligned(16))) Vjp16Operands<T> w;
-  __shared__ __attribute__((aligned(16))) Vjp16Masks s_mask;
-  const int lane = threadIdx.x, n = lane & 31, g = lane >> 5, chunk = blockIdx.x;
-  const int chunk_end = min(S, (chunk + 1) * chunk_steps);
-  w.select(lane);
+  __shared__ Vjp16StepsLds<T> lds;
+  Vjp16Shared<T>& s = lds.s;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, g = lane >> 5;
+  const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   float kf[6];
 #pragma unroll
-  for (int f = 0; f < 6; ++f) kf[f] = (freq[f] * att[f]) * 0.159154943f;
+  for (int f = 0; f < 6; ++f)
+    kf[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((freq[f] * att[f]) * 0.159154943f)));
   bool bad = false;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);
-    w.load(W1, b1, W2, b2, W3, (size_t)run.p, lane);
-    Vjp16Sums sum;
+    vjp16_load<T>(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane, s);
+    if (t < 4) s.zero[t] = 0u;
+    Vjp16StepSums sum;
     sum.clear();
-    walk_run(ix, run, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
-      s_mask.put(g, n, g ? r.mask2 : r.mask1);
-      vjp16_block<T, true>(w, sum, r.x, g ? make_float4(0.f, 0.f, 0.f, 0.f) : r.d, true, s_mask, r.mask2, kf, scale, lane);
+    __syncthreads();
+    int turn = wave / 4;
+    walk_halves<kVjp16Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
+      // (as in the f32 kernel)
+      if (turn & 1) __builtin_amdgcn_s_setprio(1);
+      else __builtin_amdgcn_s_setprio(0);
+      ++turn;
+      vjp16_step_block<T>(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, kf, scale, lane);
     });
-    bad |= vjp16_store(sum, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, lane);
+    // two wavefronts to a row: the second half of them adds to the first
+    const int waves = min(2 * (run.end - run.begin), kVjp16Waves), slots = min(waves, kVjp16Slots);
+    __syncthreads();
+    if (wave < slots) vjp16_park<false>(sum, lds.sums[wave], lane);
+    if (waves > slots) {
+      __syncthreads();
+      if (wave >= slots && wave < waves) vjp16_park<true>(sum, lds.sums[wave - slots], lane);
+    }
+    __syncthreads();
+    bad |= store_row_sums(lds.sums[0], kGradFloats, slots, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
+                          64 * kVjp16Waves);
     pos = run.end;
+    __syncthreads();
   }
   if (__ballot(bad) != 0ull && lane == 0) atomicOr(nonfinite, 1);
 }
@@ -490,7 +478,8 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
     if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
     __syncthreads();
-    bad |= vjp32_store(s, waves, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t);
+    bad |= store_row_sums(reinterpret_cast<const float*>(&s.wave[0]), sizeof(Vjp32Wave) / 4, waves,
+                          run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t, 64 * kVjp32Waves);
     pos = run.end;
     __syncthreads();
   }
@@ -501,7 +490,8 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
 // One workgroup per chunk and quarter of a row: the sum of the rows of the primitive whose steps begin in the chunk and go
 // on in the next (its tail row here, tails in between, the head row of its last chunk); nothing if there is none.  What
 // lasts is a primitive with steps in most tiles, hundreds of rows one after the other: sixteen of them are in flight, and
-// its columns are shared out (one workgroup and eight in flight: 0.35 ms at 650,000 steps; now 0.21).
+// its columns are shared out (one workgroup and eight in flight, chunks of 64 steps: 0.35 ms at 650,000 steps; 0.21; with
+// chunks of 256 steps 0.03).
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, int chunk_steps, int num_chunks,
                                                          const float* __restrict__ rows, const float* __restrict__ quats,
@@ -553,18 +543,12 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
   }
 }
 
-// Steps per chunk: 16 (1,024 records, the length of an f32 accumulation), fewer where that would leave fewer than eight
-// chunks for each of the chip's 1,024 SIMDs -- the launch then lasts as long as its longest chunks --, but four at the
-// least: every chunk loads 14 KB of weights and writes as much.
+// Steps per chunk, whose workgroup of eight wavefronts fills a CU: 256 (up to 2,048 records to a wavefront;
+// 128: 5.58 instead of 5.52 ms in f32 at 648,000 steps), fewer where that would leave fewer than eight chunks for each of the
+// 256 CUs, 16 at the least.
 inline int train_chunk_steps(int64_t S) {
-  const int64_t per = S / 8192;
-  return per >= 16 ? 16 : per <= 4 ? 4 : (int)per;
-}
-// ... of the f32 kernel, whose workgroup of eight wavefronts fills a CU: 256 (2,048 records to a wavefront; 128: 5.58 instead of
-// 5.52 ms), fewer where that would leave fewer than eight chunks for each of the 256 CUs, 16 at the least.
-inline int train_chunk_steps_f32(int64_t S) {
-  const int64_t per = S / 2048 / kVjp32Waves * kVjp32Waves;
-  return per >= 32 * kVjp32Waves ? 32 * kVjp32Waves : per <= 2 * kVjp32Waves ? 2 * kVjp32Waves : (int)per;
+  const int64_t per = S / 2048 / 8 * 8;
+  return per >= 256 ? 256 : per <= 16 ? 16 : (int)per;
 }
 
 // The sorted steps, then head and tail rows of every chunk.
@@ -639,7 +623,8 @@ MLPSP_API int mlpsp_train_group(const int32_t* tile_offsets_dev, int64_t num_pai
     }
     int32_t* hist = (int32_t*)p;
     p += (size_t)blocks * (1 << width_bits) * 4;
-    if ((size_t)(p - (unsigned char*)scratch_dev) > t.bytes) return MLPSP_E_SCRATCH;      // (cannot be: 4 KB of rows per step)
+    // (cannot be: 110 bytes of rows per step at least, 34 of these)
+    if ((size_t)(p - (unsigned char*)scratch_dev) > t.bytes) return MLPSP_E_SCRATCH;
     hipLaunchKernelGGL(step_list_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, tile_offsets_dev, sp.tile_base,
                        sp.chunk_table, sp.ids, (int)T, width, ceil_div(width, 8), keys[0], info);
     MLPSP_LAUNCH_CHECK();
@@ -696,24 +681,19 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
   const GradRows grads{gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
   const GeoGrads geo{grad_positions_dev, grad_log_scales_dev, grad_quats_dev};
   const int S = (int)num_steps;
-  const int chunk_steps = precision == 0 ? train_chunk_steps_f32(S) : t.chunk_steps;
-  const int num_chunks = (int)(((int64_t)S + chunk_steps - 1) / chunk_steps);      // (the rows are carved for the shorter chunks)
+  const int chunk_steps = t.chunk_steps, num_chunks = t.num_chunks;
   if (num_chunks > 0) {
 #define MLPSP_TRAIN_VJP(KERNEL, THREADS)                                                                                \
   hipLaunchKernelGGL(KERNEL, dim3((unsigned)num_chunks), dim3(THREADS), 0, s, ix, S, chunk_steps, num_chunks, sp.records, \
                      (const float4*)d4_dev, rays_d_dev, width, height, freq_dev, att_dev, W1, b1, W2, b2, W3, scale,   \
                      t.rows, grads, nonfinite_dev)
     if (precision == 0) MLPSP_TRAIN_VJP(train_vjp_f32_kernel, 64 * kVjp32Waves);
-    else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>), 64);
-    else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>), 64);
+    else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>), 64 * kVjp16Waves);
+    else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>), 64 * kVjp16Waves);
 #undef MLPSP_TRAIN_VJP
     MLPSP_LAUNCH_CHECK();
-#define MLPSP_TRAIN_GEOMETRY(WAVES)                                                                                     \
-  hipLaunchKernelGGL(train_geometry_kernel<WAVES>, dim3((unsigned)num_chunks), dim3(64 * WAVES), 0, s, ix, S, chunk_steps, \
-                     num_chunks, sp.records, falloff_dev, log_scales_dev, quats_dev, t.rows, geo)
-    if (precision == 0) MLPSP_TRAIN_GEOMETRY(4);
-    else MLPSP_TRAIN_GEOMETRY(1);
-#undef MLPSP_TRAIN_GEOMETRY
+    hipLaunchKernelGGL(train_geometry_kernel, dim3((unsigned)num_chunks), dim3(64 * kGeoWaves), 0, s, ix, S, chunk_steps,
+                       num_chunks, sp.records, falloff_dev, log_scales_dev, quats_dev, t.rows, geo);
     MLPSP_LAUNCH_CHECK();
     hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)num_chunks, 4), dim3(256), 0, s, ix, S, chunk_steps, num_chunks,
                        t.rows, quats_dev, grads, geo, nonfinite_dev);

@@ -1,6 +1,6 @@
 // Weight gradients of the per-primitive 72->32->32->4 MLP over blocks of 32 records of one primitive, in 16-bit operands
-// with f32 accumulation: what the grouped kernel over a CSR of records (mlpsp_grouped_vjp.hip) and the kernel over
-// training steps (mlpsp_train_backward.hip) share.
+// with f32 accumulation: the grouped kernel over a CSR of records (mlpsp_grouped_vjp.hip), and what the kernel over
+// training steps (mlpsp_vjp16_steps.hpp) takes from it.
 #pragma once
 #include "mlpsp_device.hpp"
 #include "mlpsp_mfma16.hpp"

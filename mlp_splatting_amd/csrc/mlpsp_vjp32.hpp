@@ -10,7 +10,7 @@
 //                           W1                 b1                 W2                 b2                 W3
 //   647,988 steps   3.9e-7 -> 2.3e-7   2.8e-7 -> 1.1e-7   3.4e-7 -> 2.0e-7   3.7e-7 -> 1.0e-7   2.8e-7 -> 1.1e-7
 //    51,614 steps   1.9e-7 -> 1.1e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.0e-7   2.2e-7 -> 0.8e-7   1.7e-7 -> 1.1e-7
-// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.44 -> 5.40 ms, 0.72 -> 0.55 ms.
+// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.44 -> 5.32 ms, 0.72 -> 0.55 ms.
 //
 // Bound by the ~1,250 vector instructions of a block (half of them sines and cosines, a sixth the splits), two wavefronts to
 // a SIMD: 256 registers with the weights in LDS.  A wavefront with its own weights in registers spills (6.7 ms, waiting for
@@ -495,13 +495,15 @@ __device__ __forceinline__ void vjp32_park(const Vjp32Sums& sum, float* row, int
     if (lane == o) out.b3[o] = v;
   }
 }
-// The sums of the first `waves` wavefronts, added up by the workgroup and stored; returns whether a value was not finite.
-__device__ __forceinline__ bool vjp32_store(const Vjp32Lds& s, int waves, const GradRows& out, float inv, int t) {
+// The sums in `rows` rows of LDS, `stride` floats apart, added up by the workgroup and stored; returns whether a value was not
+// finite.
+__device__ __forceinline__ bool store_row_sums(const float* first, int stride, int rows, const GradRows& out, float inv, int t,
+                                               int threads) {
   asm volatile("" : "+v"(t));
   bool bad = false;
-  for (int k = t; k < kGradFloats / 4; k += 64 * kVjp32Waves) {
+  for (int k = t; k < kGradFloats / 4; k += threads) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < waves; ++w) v += reinterpret_cast<const f32x4*>(&s.wave[w])[k];
+    for (int w = 0; w < rows; ++w) v += *reinterpret_cast<const f32x4*>(first + w * stride + 4 * k);
     v *= inv;
 #pragma unroll
     for (int q = 0; q < 4; ++q) bad |= !(__builtin_fabsf(v[q]) <= 3.4028235e38f);

@@ -259,13 +259,15 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
     assert not bool(torch.isfinite(ops.train_feature_l1(frame, base[6], used, target, 1.5, 2.0)[0]))
 
 
+@pytest.mark.parametrize("precision", [0, 1, 2])
 @pytest.mark.parametrize("tiles", [1, 3, 4, 5, 15, 16, 17, 31, 129, 255])
-def test_f32_weight_gradients_of_runs_of_every_length(device, tiles):
-    """The f32 kernel deals a run's half steps to eight wavefronts and cuts the steps into chunks of 16 to 256: runs of one
+def test_weight_gradients_of_runs_of_every_length(device, tiles, precision):
+    """The kernels deal a run's half steps to eight wavefronts and cut the steps into chunks of 16 to 256: runs of one
     primitive that are a little shorter and longer than those, three in a row, against float64 over the same steps.  An f32
     gradient is a sum of up to 16,000 products of two factors that are f32 sums of up to 72 terms themselves: a few units of
     2^-24 each, 1e-6 of the norm.  A phase is an f32 product of two roundings, and moves its sine by as much: 2^-23 times the
-    largest phase."""
+    largest phase.  In 16 bits (1: fp16, 2: bf16) every factor and what it was computed from, eight tensors at the most, is
+    rounded once, by 2^-11 or 2^-8 of it; the adjoints are scaled by 256 and stay above what fp16 holds in full."""
     import numpy as np
     from mlp_splatting_amd import ops, synthetic as syn
     from mlp_splatting_amd.tile_ext import TileExt
@@ -287,7 +289,7 @@ def test_f32_weight_gradients_of_runs_of_every_length(device, tiles):
     g_rgb, g_t = torch.randn(width * height, 3, generator=g).to(device), torch.randn(width * height, generator=g).to(device)
     d4, falloff = ops.train_reverse(frame, base[6], g_rgb, g_t)
     got, flag = ops.train_gradients(frame, ops.train_group(frame, base[6], n), d4, falloff, base[1], base[7], base[8], base[9:15],
-                                    base[3], base[4], 0, 1.0)
+                                    base[3], base[4], precision, 256.0 if precision else 1.0)
     assert int(flag) == 0
     # d4 is [tile, step of the tile, lane]; the records are [pixel, hit], and every pixel hits all three, in the tile's order
     ids, x6 = records[2].view(-1, n), records[3].view(-1, n, 6)
@@ -301,7 +303,7 @@ def test_f32_weight_gradients_of_runs_of_every_length(device, tiles):
         phase = (x6[at].double()[:, :, None] * base[7].double() * base[8].double()).reshape(-1, 36)
         enc, d = torch.cat([phase.sin(), phase.cos()], 1), adjoint[at]
         z1 = enc @ W1[p].T + b1[p]
-        bound = 1e-6 + 2.0 ** -23 * float(phase.abs().max())
+        bound = (1e-6, 8 * 2.0 ** -11, 8 * 2.0 ** -8)[precision] + 2.0 ** -23 * float(phase.abs().max())
         h1 = z1.clamp(min=0.0)
         z2 = h1 @ W2[p].T + b2[p]
         d2 = (d @ W3[p]) * (z2 > 0)
