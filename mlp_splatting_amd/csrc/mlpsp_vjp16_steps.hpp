@@ -6,7 +6,7 @@
 // instructions and ~250 vector instructions a block instead of 30 and 350.
 //
 // Bound by the vector instructions (the 36 sines and cosines are a third of their time).  Eight wavefronts, two to a SIMD, hold
-// everything in 179 registers; twelve spill 24 words and sixteen 224 (gradient call of 648,000 steps 2.18, 2.29 and 4.7 ms;
+// everything in 184 registers; twelve spill 24 words and sixteen 224 (gradient call of 648,000 steps 2.12, 2.23 and 4.7 ms;
 // with the block of mlpsp_vjp16.hpp, a wavefront to a chunk of 64 steps, 2.54).
 #pragma once
 #include "mlpsp_device.hpp"
@@ -90,9 +90,9 @@ struct Vjp16StepSums {
   }
 };
 __device__ __forceinline__ Pack8 transpose_tile(const Pack8& v, Vjp16Wave& s, int n, int g) {
-  const char* const from = reinterpret_cast<const char*>(&s.tile[4 * g + ((n >> 2) & 3)][8 * (n >> 4) + 2 * (n & 3)]);
-  *reinterpret_cast<u32x4*>(&s.tile[n][8 * g]) = v.s[0];
-  *reinterpret_cast<u32x4*>(&s.tile[n][8 * g + 4]) = v.s[1];
+  const char* const from = tile_reads(s.tile, n, g);
+  *reinterpret_cast<u32x4*>(&s.tile[n][tile_place(2 * g, n)]) = v.s[0];
+  *reinterpret_cast<u32x4*>(&s.tile[n][tile_place(2 * g + 1, n)]) = v.s[1];
   return Pack8{{read_records(from, 0, 64), read_records(from, 1, 64)}};
 }
 __device__ __forceinline__ f32x4 tail_product(u32x4 a, u32x4 b, f32x4 c, __bf16) {
@@ -140,7 +140,7 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
       const float rev = t < 18 ? x[t < 18 ? t / 6 : 0] * kf[t % 6] : 0.f;
       e[d] = t < 18 ? Ops<T>::pack2(__builtin_amdgcn_sinf(rev), __builtin_amdgcn_cosf(rev)) : 0u;
     }
-    if (k < 4) *reinterpret_cast<u32x4*>(&s.enc[n][8 * ((2 * g + (k >> 1)) ^ ((n >> 1) & 3)) + 4 * ((k & 1) ^ ((n >> 3) & 1))]) = e;
+    if (k < 4) *reinterpret_cast<u32x4*>(&s.enc[n][enc_place(2 * g + (k >> 1), k & 1, n)]) = e;
     else *reinterpret_cast<u32x2*>(&s.enc_tail[n][2 * g]) = u32x2{e[0], e[1]};
     a1 = Ops<T>::mfma(w.w1[k][lane], e, a1);
   }
@@ -158,8 +158,7 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
   }
   sum.gw2 = mma2<T>(d2t, h1t, sum.gw2);
   // ---- the W1 gradient (addresses as in vjp32_block)
-  const int rec = 4 * g + ((n >> 2) & 3), piece = (n >> 4) ^ ((rec >> 1) & 3);
-  const char* const row = reinterpret_cast<const char*>(s.enc[rec]);
+  const int rec = 4 * g + ((n >> 2) & 3);
   const bool last = ((n >> 1) & 1) == (n >> 4);
   const char* const last0 = last ? reinterpret_cast<const char*>(&s.enc_tail[rec][2 * (n & 1)]) : reinterpret_cast<const char*>(w.zero);
   const int last_row = last ? 16 : 0;
@@ -167,8 +166,7 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
   for (int k = 0; k < 2; ++k) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const char* const at = row + 32 * (piece ^ (2 * c));
-      sum.gw1[c] = Ops<T>::mfma(d1.s[k], read_records(at + 8 * (n & 3), at + (8 * (n & 3) ^ 16), k, Vjp16Wave::kRowBytes), sum.gw1[c]);
+      sum.gw1[c] = Ops<T>::mfma(d1.s[k], read_records(enc_reads(s.enc, c, n, g), k, Vjp16Wave::kRowBytes), sum.gw1[c]);
     }
     sum.gw1e = tail_product(d1.s[k], read_records(last0, k, last_row), sum.gw1e, T{});
   }

@@ -10,7 +10,7 @@
 //                           W1                 b1                 W2                 b2                 W3
 //   647,988 steps   3.9e-7 -> 2.3e-7   2.8e-7 -> 1.1e-7   3.4e-7 -> 2.0e-7   3.7e-7 -> 1.0e-7   2.8e-7 -> 1.1e-7
 //    51,614 steps   1.9e-7 -> 1.1e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.0e-7   2.2e-7 -> 0.8e-7   1.7e-7 -> 1.1e-7
-// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.44 -> 5.32 ms, 0.72 -> 0.55 ms.
+// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.44 -> 5.25 ms, 0.72 -> 0.55 ms.
 //
 // Bound by the ~1,250 vector instructions of a block (half of them sines and cosines, a sixth the splits), two wavefronts to
 // a SIMD: 256 registers with the weights in LDS.  A wavefront with its own weights in registers spills (6.7 ms, waiting for
@@ -109,12 +109,11 @@ __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4&
 constexpr int kVjp32Waves = 8;
 struct Vjp32Wave {
   // Columns of the encoding: pair t of group g (sin, cos) is word 16 g + t of a record's 32 for t < 16, and word
-  // 2 g + (t - 16) of its tail.  The 8-word pieces of a row are exchanged by bits 1, 2 of the record's number and their
-  // 4-word halves by bit 3, so that transposed reads (four records by sixteen columns per sixteen lanes) meet no bank twice.
+  // 2 g + (t - 16) of its tail; enc_place says where in the record's row.
   __attribute__((aligned(16))) unsigned enc[3][32][32];
   __attribute__((aligned(16))) unsigned enc_tail[3][32][4];
   union {
-    __attribute__((aligned(16))) unsigned tile[32][16];   // one plane: word 8 g + d of a record = registers 2 d, 2 d + 1 of group g
+    __attribute__((aligned(16))) unsigned tile[32][16];   // one plane: word 8 g + d of a record (tile_place) = registers 2 d, 2 d + 1 of group g
     __attribute__((aligned(16))) float d3[32][4];         // [record][output]
   };
   __attribute__((aligned(16))) uint32_t mask1[32];
@@ -150,10 +149,22 @@ __device__ __forceinline__ u32x4 read_records(const char* row0, int s, int row) 
   const u32x2 a = read_transposed(row0 + (16 * s) * row), b = read_transposed(row0 + (16 * s + 8) * row);
   return u32x4{a[0], a[1], b[0], b[1]};
 }
-// ... with its own address for records 8 on
-__device__ __forceinline__ u32x4 read_records(const char* row0, const char* row8, int s, int row) {
-  const u32x2 a = read_transposed(row0 + (16 * s) * row), b = read_transposed(row8 + (16 * s + 8) * row);
-  return u32x4{a[0], a[1], b[0], b[1]};
+// Where 16 bytes of a record lie in its row of `tile` (quarter q of 64 bytes) and of `enc` (half h of 32 bytes b), in words: a
+// store of 16 bytes a lane and a transposed read then reach every bank equally often (13 and 2.2 clocks; in order a store to
+// `tile` takes 32).  The same for records eight apart, whose reads differ by a constant.
+__device__ __forceinline__ int tile_place(int q, int record) { return 4 * (q ^ ((record >> 1) & 3)); }
+__device__ __forceinline__ int enc_place(int b, int h, int record) {
+  return 8 * (b ^ ((record & 2) | ((record >> 2) & 1))) + 4 * (h ^ (record & 1));
+}
+// This lane's address of transposed reads: record 4 g + (lane / 4) % 4, columns 16 (n / 16) + 4 (lane % 4) on
+__device__ __forceinline__ const char* tile_reads(const unsigned (*tile)[16], int n, int g) {
+  const int rec = 4 * g + ((n >> 2) & 3);
+  return reinterpret_cast<const char*>(&tile[rec][tile_place(2 * (n >> 4) + ((n >> 1) & 1), rec) + 2 * (n & 1)]);
+}
+// ... columns 32 c further on
+__device__ __forceinline__ const char* enc_reads(const unsigned (*enc)[32], int c, int n, int g) {
+  const int rec = 4 * g + ((n >> 2) & 3);
+  return reinterpret_cast<const char*>(&enc[rec][enc_place((n >> 4) + 2 * c, (n >> 1) & 1, rec) + 2 * (n & 1)]);
 }
 
 // The primitive's weights into LDS, by the whole workgroup: nine pieces of 64 lanes, a piece to a wavefront.
@@ -263,12 +274,15 @@ __device__ __forceinline__ float where_bit(float v, uint32_t word, int bit) {
 }
 // A tile whose lanes are records, transposed through LDS a plane at a time (a wavefront's LDS operations complete in order).
 __device__ __forceinline__ Split8 transpose_tile(const Split8& v, Vjp32Wave& s, int n, int g) {
-  const char* const from = reinterpret_cast<const char*>(&s.tile[4 * g + ((n >> 2) & 3)][8 * (n >> 4) + 2 * (n & 3)]);
+  asm volatile("" : "+v"(n));            // (or the addresses are kept from one transposition to the next, and registers spill)
+  unsigned* const to = &s.tile[n][tile_place(2 * g, n)];
+  unsigned* const to1 = &s.tile[n][tile_place(2 * g + 1, n)];
+  const char* const from = tile_reads(s.tile, n, g);
   Split8 r;
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    *reinterpret_cast<u32x4*>(&s.tile[n][8 * g]) = v.p[p].s[0];
-    *reinterpret_cast<u32x4*>(&s.tile[n][8 * g + 4]) = v.p[p].s[1];
+    *reinterpret_cast<u32x4*>(to) = v.p[p].s[0];
+    *reinterpret_cast<u32x4*>(to1) = v.p[p].s[1];
 #pragma unroll
     for (int k = 0; k < 2; ++k) r.p[p].s[k] = read_records(from, k, 64);
   }
@@ -306,7 +320,7 @@ __device__ __forceinline__ void vjp32_encode(float x, const float (&factor)[6], 
     e.p[2][t & 3] = v.l;
     if ((t & 3) == 3) {
       const int k = t >> 2;
-      unsigned* const to = &s.enc[0][n][8 * ((2 * g + (k >> 1)) ^ ((n >> 1) & 3)) + 4 * ((k & 1) ^ ((n >> 3) & 1))];
+      unsigned* const to = &s.enc[0][n][enc_place(2 * g + (k >> 1), k & 1, n)];
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(to + 1024 * p) = e.p[p];
       done(k, e);
@@ -394,8 +408,7 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   __builtin_amdgcn_sched_barrier(0);
   // ---- layer 1 rectified, beside the first half of the W1 gradient.  This lane's addresses of transposed reads: record
   // rec = 4 g + (lane / 4) % 4 (and 8 on), columns 32 c + 16 (n / 16) + 4 (lane % 4) on
-  const int rec = 4 * g + ((n >> 2) & 3), piece = (n >> 4) ^ ((rec >> 1) & 3);
-  const char* const row = reinterpret_cast<const char*>(s.enc[0][rec]);
+  const int rec = 4 * g + ((n >> 2) & 3);
   // of the last columns: units 0..15 (n < 16) take them in the low half of the columns, units 16..31 in the high half
   const bool last = ((n >> 1) & 1) == (n >> 4);
   const char* const last0 = last ? reinterpret_cast<const char*>(&s.enc_tail[0][rec][2 * (n & 1)]) : reinterpret_cast<const char*>(w.zero);
@@ -403,12 +416,10 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   const auto gradient1 = [&](int k) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const char* const at = row + 32 * (piece ^ (2 * c));
+      const char* const at = enc_reads(s.enc[0], c, n, g);
       u32x4 b[3];
 #pragma unroll
-      for (int p = 0; p < 3; ++p)
-        b[p] = read_records(at + 8 * (n & 3) + p * Vjp32Wave::kPlaneBytes, at + (8 * (n & 3) ^ 16) + p * Vjp32Wave::kPlaneBytes, k,
-                            Vjp32Wave::kRowBytes);
+      for (int p = 0; p < 3; ++p) b[p] = read_records(at + p * Vjp32Wave::kPlaneBytes, k, Vjp32Wave::kRowBytes);
       sum.gw1[c] = mfma_split_onto(d1.p[0].s[k], d1.p[1].s[k], d1.p[2].s[k], b[0], b[1], b[2], sum.gw1[c]);
     }
     bf16x8 b[3];
