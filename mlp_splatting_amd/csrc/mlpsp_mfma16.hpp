@@ -214,10 +214,16 @@ __device__ __forceinline__ void encode_direction_words(float rdx, float rdy, flo
 
 // Bits 4s+d and 16+4s+d of a lane's partial ReLU mask from the rectified operand word (s, d): a half that is
 // not zero is an active unit (the rounded activation the next layer really multiplies).
-__device__ __forceinline__ unsigned relu_mask_bits(unsigned rectified, int shift) {
+// ones: 1 in both halves, hidden from the compiler (hidden_ones): a minimum with a known 1 it takes for a test against zero,
+// which it does half by half in six instructions instead of one.
+__device__ __forceinline__ unsigned hidden_ones() {
+  unsigned ones = 0x00010001u;
+  asm("" : "+s"(ones));
+  return ones;
+}
+__device__ __forceinline__ unsigned relu_mask_bits(unsigned rectified, unsigned ones, int shift) {
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-  const u16x2 one = {1, 1};
-  const u16x2 nz = __builtin_elementwise_min(__builtin_bit_cast(u16x2, rectified), one);
+  const u16x2 nz = __builtin_elementwise_min(__builtin_bit_cast(u16x2, rectified), __builtin_bit_cast(u16x2, ones));
   return __builtin_bit_cast(unsigned, nz) << shift;
 }
 
@@ -312,6 +318,7 @@ __device__ __forceinline__ unsigned long long mlp_wave_mfma16(const unsigned cha
   const HalfPair hx = both_halves(dx), hy = both_halves(dy), hz = both_halves(dz);
   float o_blk[2][4];
   unsigned m_blk[2][2] = {{0u, 0u}, {0u, 0u}};
+  const unsigned ones = MASKS ? hidden_ones() : 0u;
   const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -357,7 +364,8 @@ __device__ __forceinline__ unsigned long long mlp_wave_mfma16(const unsigned cha
       // rounded, as the B operand
       // (its B operand is constant, three zero words and the (1, 1) word: the compiler keeps it in four registers
       // across the primitive loop, which there is room for)
-      const unsigned z0 = 0u, z1 = 0u, z2 = 0u;
+      unsigned z0 = 0u, z1 = 0u, z2 = 0u;
+      if constexpr (MASKS) asm("" : "+v"(z0), "+v"(z1), "+v"(z2));       // (where there is no room it is spilled: 16 bytes read back per block)
       f32x16 d2 = Ops<T>::mfma(a1[4], u32x4{z0, z1, z2, one_word}, zero16);
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -365,7 +373,7 @@ __device__ __forceinline__ unsigned long long mlp_wave_mfma16(const unsigned cha
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           bw[d] = relu_packed(Ops<T>::pack2(d1[8 * s + 2 * d], d1[8 * s + 2 * d + 1]));
-          if constexpr (MASKS) m_blk[b][0] |= relu_mask_bits(bw[d], 4 * s + d);
+          if constexpr (MASKS) m_blk[b][0] |= relu_mask_bits(bw[d], ones, 4 * s + d);
         }
         d2 = Ops<T>::mfma(a2[s], bw, d2);
       }
@@ -378,7 +386,7 @@ __device__ __forceinline__ unsigned long long mlp_wave_mfma16(const unsigned cha
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           bw[d] = relu_packed(Ops<T>::pack2(d2[8 * s + 2 * d], d2[8 * s + 2 * d + 1]));
-          if constexpr (MASKS) m_blk[b][1] |= relu_mask_bits(bw[d], 4 * s + d);
+          if constexpr (MASKS) m_blk[b][1] |= relu_mask_bits(bw[d], ones, 4 * s + d);
         }
         d3 = layer3_small<T>(a3[s], bw, d3);
       }
