@@ -219,6 +219,7 @@ struct StepIndex {
 
 constexpr int kGeoFloats = 16;                            // 15 geometry sums, one pad
 constexpr int kRowFloats = kGradFloats + kGeoFloats;      // of a head or tail row
+constexpr int kTrainChunk = 128;                          // steps of a chunk, at the most (train_chunk_steps)
 
 // A chunk's run of one primitive: steps [begin, end), and where its sums belong.
 struct StepRun {
@@ -367,13 +368,14 @@ __device__ __forceinline__ StepRecord step_record(const unsigned char* __restric
   r.mask2 = reinterpret_cast<const uint32_t*>(rec + kStepPlaneD)[px];
   return r;
 }
-// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on, 64 at the most; work(record) for those that
+// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on; work(record) for those that
 // have an adjoint.  Lane i asks for where the i-th of them lies; the next record is under way while one is worked on (two or
 // three: no faster).  Records without an adjoint get inputs of zero, whatever ray their lane has.
 template <int STRIDE, typename Work>
 __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int end, int half, const unsigned char* __restrict__ records,
                                             const float4* __restrict__ d4, const float* __restrict__ rays_d, int n, int g, int W,
                                             int pixels, Work&& work) {
+  static_assert(kTrainChunk <= 64 * STRIDE, "a lane for every step");
   const int count = (end - first + STRIDE - 1) / STRIDE;
   if (count <= 0) return;
   const int4 where = ix.step[min(first + STRIDE * (n + 32 * g), end - 1)];
@@ -417,24 +419,14 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
     Vjp16StepSums sum;
     sum.clear();
     __syncthreads();
-    int turn = wave / 4;
     walk_halves<kVjp16Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
-      // (as in the f32 kernel)
-      if (turn & 1) __builtin_amdgcn_s_setprio(1);
-      else __builtin_amdgcn_s_setprio(0);
-      ++turn;
       vjp16_step_block<T>(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, kf, scale, lane);
     });
-    // two wavefronts to a row: the second half of them adds to the first
-    const int waves = min(2 * (run.end - run.begin), kVjp16Waves), slots = min(waves, kVjp16Slots);
+    const int waves = min(2 * (run.end - run.begin), kVjp16Waves);
     __syncthreads();
-    if (wave < slots) vjp16_park<false>(sum, lds.sums[wave], lane);
-    if (waves > slots) {
-      __syncthreads();
-      if (wave >= slots && wave < waves) vjp16_park<true>(sum, lds.sums[wave - slots], lane);
-    }
+    if (wave < waves) vjp16_park(sum, lds.sums[wave], lane);
     __syncthreads();
-    bad |= store_row_sums(lds.sums[0], kGradFloats, slots, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
+    bad |= store_row_sums(lds.sums[0], kGradFloats, waves, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
                           64 * kVjp16Waves);
     pos = run.end;
     __syncthreads();
@@ -468,8 +460,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     __syncthreads();
     int turn = wave / 4;
     walk_halves<kVjp32Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
-      // (the two wavefronts of a SIMD take turns at priority, or one of them is blocks ahead when the other ends: 5.56 ms
-      // for the gradient call instead of 5.40)
+      // (a wavefront's blocks take turns at priority: 5.22 ms for the gradient call instead of 5.25)
       if (turn & 1) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(0);
       ++turn;
@@ -543,12 +534,12 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
   }
 }
 
-// Steps per chunk, whose workgroup of eight wavefronts fills a CU: 256 (up to 2,048 records to a wavefront;
-// 128: 5.58 instead of 5.52 ms in f32 at 648,000 steps), fewer where that would leave fewer than eight chunks for each of the
-// 256 CUs, 16 at the least.
+// Steps per chunk: as many as a wavefront has lanes for (twice that is no faster), fewer where that would leave fewer than four
+// chunks for each of the 512 workgroups that run at once, 16 at the least.  Gradient call in us, f32, a half, as much and
+// twice as much of that rule at 51,600 steps: 483, 484, 518.
 inline int train_chunk_steps(int64_t S) {
   const int64_t per = S / 2048 / 8 * 8;
-  return per >= 256 ? 256 : per <= 16 ? 16 : (int)per;
+  return per >= kTrainChunk ? kTrainChunk : per <= 16 ? 16 : (int)per;
 }
 
 // The sorted steps, then head and tail rows of every chunk.
@@ -623,7 +614,7 @@ MLPSP_API int mlpsp_train_group(const int32_t* tile_offsets_dev, int64_t num_pai
     }
     int32_t* hist = (int32_t*)p;
     p += (size_t)blocks * (1 << width_bits) * 4;
-    // (cannot be: 110 bytes of rows per step at least, 34 of these)
+    // (cannot be: 220 bytes of rows per step at least, 34 of these)
     if ((size_t)(p - (unsigned char*)scratch_dev) > t.bytes) return MLPSP_E_SCRATCH;
     hipLaunchKernelGGL(step_list_kernel, dim3((unsigned)((T + 3) / 4)), dim3(256), 0, s, tile_offsets_dev, sp.tile_base,
                        sp.chunk_table, sp.ids, (int)T, width, ceil_div(width, 8), keys[0], info);

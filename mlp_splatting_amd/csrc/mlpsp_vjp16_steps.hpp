@@ -5,9 +5,10 @@
 // ds_read_b64_tr_b16 instead of being computed in both orientations or transposed by the matrix core: 16 large matrix
 // instructions and ~250 vector instructions a block instead of 30 and 350.
 //
-// Bound by the vector instructions (the 36 sines and cosines are a third of their time).  Eight wavefronts, two to a SIMD, hold
-// everything in 184 registers; twelve spill 24 words and sixteen 224 (gradient call of 648,000 steps 2.12, 2.23 and 4.7 ms;
-// with the block of mlpsp_vjp16.hpp, a wavefront to a chunk of 64 steps, 2.54).
+// Bound by the vector instructions (the 36 sines and cosines are a third of their time).  Four wavefronts to a workgroup and
+// two workgroups to a CU: while one changes primitives the other works, and two wavefronts to a SIMD hold everything in 186
+// registers.  Gradient call of 648,000 steps: 1.90 ms; one workgroup of eight 2.12, four of two 2.31, three of four 2.9 (168
+// registers: spills); with the block of mlpsp_vjp16.hpp, a wavefront to a chunk of 64 steps, 2.54.
 #pragma once
 #include "mlpsp_device.hpp"
 #include "mlpsp_mfma16.hpp"
@@ -16,7 +17,7 @@
 
 namespace mlpsp {
 
-constexpr int kVjp16Waves = 8, kVjp16Slots = kVjp16Waves / 2;
+constexpr int kVjp16Waves = 4;
 // As Vjp32Wave, one plane.
 struct Vjp16Wave {
   __attribute__((aligned(16))) unsigned enc[32][32];
@@ -38,7 +39,7 @@ struct Vjp16Shared {
 template <typename T>
 union Vjp16StepsLds {
   Vjp16Shared<T> s;
-  __attribute__((aligned(16))) float sums[kVjp16Slots][kGradFloats];    // two wavefronts to a row
+  __attribute__((aligned(16))) float sums[kVjp16Waves][kGradFloats];    // in the end
 };
 
 // The primitive's weights into LDS, by the first six wavefronts.
@@ -48,18 +49,18 @@ __device__ __forceinline__ void vjp16_load(const float* __restrict__ W1, const f
                                            Vjp16Shared<T>& s) {
   asm volatile("" : "+v"(lane));         // (or the addresses are formed ahead of the loop over the runs, one by one)
   const int n = lane & 31, g = lane >> 5;
-  if (wave < 5) {
+  for (int q = wave; q < 5; q += kVjp16Waves) {
     const float* __restrict__ row = W1 + p * 2304 + n * 72 + 18 * g;
     u32x4 v;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const int t = 4 * wave + d;
+      const int t = 4 * q + d;
       v[d] = t < 18 ? Ops<T>::pack2(row[t < 18 ? t : 0], row[36 + (t < 18 ? t : 0)]) : 0u;
     }
-    s.w1[wave][lane] = v;
+    s.w1[q][lane] = v;
   }
-  if (wave == 4 || wave == 5) {
-    const int k = wave - 4;
+  if (wave == 1 || wave == 2) {
+    const int k = wave - 1;
     const float* __restrict__ row = W2 + p * 1024 + n * 32 + 16 * k + 4 * g;
     const float* __restrict__ col = W2 + p * 1024 + n;
     u32x4 a, b;
@@ -72,7 +73,7 @@ __device__ __forceinline__ void vjp16_load(const float* __restrict__ W1, const f
     s.w2[k][lane] = a;
     s.w2t[k][lane] = b;
   }
-  if (wave == 5) {
+  if (wave == 3) {
     const float* __restrict__ r = W3 + p * 128 + hidden_unit_of_row(n);
     s.w3r[lane] = g ? u32x2{0u, 0u} : u32x2{Ops<T>::pack2(r[0], r[32]), Ops<T>::pack2(r[64], r[96])};
     (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
@@ -172,35 +173,33 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
   }
 }
 
-// A wavefront's sums to a row of LDS, in the order of a packed row of gradients; ADD: onto what is there.
-template <bool ADD>
+// A wavefront's sums to a row of LDS, in the order of a packed row of gradients.
 __device__ __forceinline__ void vjp16_park(const Vjp16StepSums& sum, float* to, int lane) {
   asm volatile("" : "+v"(lane));
   const int n = lane & 31, g = lane >> 5;
   const GradRows out = packed_grad_rows(to);
-  const auto put = [](float* at, float v) { *at = ADD ? *at + v : v; };
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int r = 8 * (i >> 2) + 4 * g + (i & 3);
-    put(out.W1 + r * 72 + enc_feature(n), sum.gw1[0][i]);
-    put(out.W1 + r * 72 + enc_feature(32 + n), sum.gw1[1][i]);
-    put(out.W2 + hidden_unit(r & 15, r >> 4) * 32 + tile_unit(n), sum.gw2[i]);
+    out.W1[r * 72 + enc_feature(n)] = sum.gw1[0][i];
+    out.W1[r * 72 + enc_feature(32 + n)] = sum.gw1[1][i];
+    out.W2[hidden_unit(r & 15, r >> 4) * 32 + tile_unit(n)] = sum.gw2[i];
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    put(out.W1 + ((lane & 8 ? 16 : 0) + 4 * (lane >> 4) + r) * 72 + enc_feature(64 + (lane & 7)), sum.gw1e[r]);
+    out.W1[((lane & 8 ? 16 : 0) + 4 * (lane >> 4) + r) * 72 + enc_feature(64 + (lane & 7))] = sum.gw1e[r];
     const float v = sum.gw3[r] + __shfl_xor(sum.gw3[r], 32);
-    if (g == 0) put(out.W3 + r * 32 + n, v);
+    if (g == 0) out.W3[r * 32 + n] = v;
   }
   const float gb1 = sum.gb1[0] + __shfl_xor(sum.gb1[0], 32), gb2 = sum.gb2[0] + __shfl_xor(sum.gb2[0], 32);
-  if (g == 0) put(out.b1 + n, gb1);
-  else put(out.b2 + hidden_unit(n & 15, n >> 4), gb2);
+  if (g == 0) out.b1[n] = gb1;
+  else out.b2[hidden_unit(n & 15, n >> 4)] = gb2;
 #pragma unroll
   for (int o = 0; o < 4; ++o) {
     float v = sum.gb3[o];
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-    if (lane == o) put(out.b3 + o, v);
+    if (lane == o) out.b3[o] = v;
   }
 }
 

@@ -8,13 +8,14 @@
 // takes six instructions of 32 clocks instead of eight of 64, and rounds its accumulator six times instead of sixteen.
 // Error of the gradients against float64, 2-norm over 2-norm, f32 chains of v_mfma_f32_32x32x2_f32 -> here:
 //                           W1                 b1                 W2                 b2                 W3
-//   647,988 steps   3.9e-7 -> 2.3e-7   2.8e-7 -> 1.1e-7   3.4e-7 -> 2.0e-7   3.7e-7 -> 1.0e-7   2.8e-7 -> 1.1e-7
-//    51,614 steps   1.9e-7 -> 1.1e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.0e-7   2.2e-7 -> 0.8e-7   1.7e-7 -> 1.1e-7
-// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.44 -> 5.25 ms, 0.72 -> 0.55 ms.
+//   647,988 steps   3.9e-7 -> 2.4e-7   2.8e-7 -> 1.5e-7   3.4e-7 -> 2.1e-7   3.7e-7 -> 1.1e-7   2.8e-7 -> 1.4e-7
+//    51,614 steps   1.9e-7 -> 1.2e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.1e-7   2.2e-7 -> 0.7e-7   1.7e-7 -> 1.0e-7
+// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.45 -> 5.17 ms, 0.72 -> 0.48 ms.
 //
 // Bound by the ~1,250 vector instructions of a block (half of them sines and cosines, a sixth the splits), two wavefronts to
 // a SIMD: 256 registers with the weights in LDS.  A wavefront with its own weights in registers spills (6.7 ms, waiting for
-// its spills behind the records requested ahead), alone on its SIMD it is no faster for 512 registers (7.0).
+// its spills behind the records requested ahead), alone on its SIMD it is no faster for 512 registers (7.0).  The two belong to
+// different workgroups, one of which works while the other changes primitives (one workgroup of eight: 5.23 and 0.52 ms).
 //
 // Per block (lane (n, g) = record n, half g of its inputs; D(a, b) has the rows of a in its registers):
 //   d2        D(W3, d): record in the lane, unit 8 (i / 4) + 4 g + i % 4 in register i, in f32 products
@@ -105,32 +106,32 @@ __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4&
   return Ops<__bf16>::mfma(ha, hb, acc);
 }
 
-// A workgroup of eight wavefronts fills a CU, two to a SIMD: 28 KB of operands that all of them read, 16 KB of each one's own.
-constexpr int kVjp32Waves = 8;
-struct Vjp32Wave {
-  // Columns of the encoding: pair t of group g (sin, cos) is word 16 g + t of a record's 32 for t < 16, and word
-  // 2 g + (t - 16) of its tail; enc_place says where in the record's row.
-  __attribute__((aligned(16))) unsigned enc[3][32][32];
-  __attribute__((aligned(16))) unsigned enc_tail[3][32][4];
-  union {
-    __attribute__((aligned(16))) unsigned tile[32][16];   // one plane: word 8 g + d of a record (tile_place) = registers 2 d, 2 d + 1 of group g
-    __attribute__((aligned(16))) float d3[32][4];         // [record][output]
+// A workgroup of four wavefronts, two workgroups to a CU: 23 KB of operands that its wavefronts read, 14 KB of each one's own.
+constexpr int kVjp32Waves = 4;
+union Vjp32Wave {
+  struct {
+    // Columns of the encoding: pair t of group g (sin, cos) is word 16 g + t of a record's 32 for t < 16, and word
+    // 2 g + (t - 16) of its tail; enc_place says where in the record's row.
+    __attribute__((aligned(16))) unsigned enc[3][32][32];
+    __attribute__((aligned(16))) unsigned enc_tail[3][32][4];
+    __attribute__((aligned(16))) uint32_t mask1[32];
   };
-  __attribute__((aligned(16))) uint32_t mask1[32];
+  // (in the encoding's first half of plane 0, which is not written yet or, of the records 16 on, read again)
+  __attribute__((aligned(16))) unsigned tile[32][16];   // one plane: word 8 g + d of a record (tile_place) = registers 2 d, 2 d + 1 of group g
+  __attribute__((aligned(16))) float d3[32][4];         // [record][output]
+  __attribute__((aligned(16))) float sums[kGradFloats]; // in the end
   static constexpr int kRowBytes = 128, kPlaneBytes = 4096;
 };
-static_assert(sizeof(Vjp32Wave) >= kGradFloats * 4, "a wavefront's sums lie there in the end");
 struct Vjp32Lds {
   u32x4 w1[3][4][64];            // W1[n][..]: slots 2 d, 2 d + 1 of K-step s = pair 4 s + d
   u32x4 w1_tail[4][64];          // pairs 16, 17 of two planes
-  u32x4 w2[3][2][64];            // W2[n][unit(8 s + j, g)]
-  u32x4 w2t[3][2][64];           // W2[unit(8 s + j, g)][n]
+  unsigned w2[3][32][16];        // W2[n][..]: 16 bytes 2 s + g (tile_place) = unit(8 s + j, g)
   float w3[2][64];               // W3[2 j + g][n]
   float bias1[32], bias2[32];
   __attribute__((aligned(16))) unsigned zero[4];
   Vjp32Wave wave[kVjp32Waves];
 };
-static_assert(sizeof(Vjp32Lds) <= 163840, "a workgroup per CU");
+static_assert(2 * sizeof(Vjp32Lds) <= 163840, "two workgroups per CU");
 // W1 column of encoding column k = 2 w + (0 sin, 1 cos)
 __device__ __forceinline__ int enc_feature(int k) {
   const int w = k >> 1, g = w < 32 ? w >> 4 : (w - 32) >> 1, t = w < 32 ? w & 15 : 16 + (w & 1);
@@ -167,7 +168,7 @@ __device__ __forceinline__ const char* enc_reads(const unsigned (*enc)[32], int 
   return reinterpret_cast<const char*>(&enc[rec][enc_place((n >> 4) + 2 * c, (n >> 1) & 1, rec) + 2 * (n & 1)]);
 }
 
-// The primitive's weights into LDS, by the whole workgroup: nine pieces of 64 lanes, a piece to a wavefront.
+// The primitive's weights into LDS, by the whole workgroup.
 __device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
                                            const float* __restrict__ b2, const float* __restrict__ W3, size_t p, int wave, int lane,
                                            Vjp32Lds& s, const SplitUnits& u) {
@@ -175,49 +176,36 @@ __device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const f
   const int n = lane & 31, g = lane >> 5;
   const float* __restrict__ row1 = W1 + p * 2304 + n * 72 + 18 * g;
   const auto pair = [&](int t) { return split2(row1[t], row1[36 + t], u); };
-  if (wave < 4) {
-    u32x4 v[3];
+  u32x4 v[3];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const Split2 x = pair(4 * wave + d);
+    v[0][d] = x.h;
+    v[1][d] = x.m;
+    v[2][d] = x.l;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s.w1[k][wave][lane] = v[k];
+  if (wave < 2) {
+    const float* __restrict__ row2 = W2 + p * 1024 + n * 32 + 16 * wave + 4 * g;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const Split2 x = pair(4 * wave + d);
+      const int j = 2 * d + (d & 2 ? 4 : 0);
+      const Split2 x = split2(row2[j], row2[j + 1], u);
       v[0][d] = x.h;
       v[1][d] = x.m;
       v[2][d] = x.l;
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) s.w1[k][wave][lane] = v[k];
-  } else {
-    const int k = wave & 1;        // K-step
-    float v[8];
-    if (wave < 6) {
-      const float* __restrict__ row = W2 + p * 1024 + n * 32 + 16 * k + 4 * g;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = row[j + (j & 4)];
-    } else {
-      const float* __restrict__ col = W2 + p * 1024 + (16 * k + 4 * g) * 32 + n;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = col[(j + (j & 4)) * 32];
-    }
-    u32x4 w[3];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const Split2 x = split2(v[2 * d], v[2 * d + 1], u);
-      w[0][d] = x.h;
-      w[1][d] = x.m;
-      w[2][d] = x.l;
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) (wave < 6 ? s.w2 : s.w2t)[q][k][lane] = w[q];
-  }
-  if (wave == 7) {
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(&s.w2[k][n][tile_place(2 * wave + g, n)]) = v[k];
+  } else if (wave == 2) {
     const Split2 x = pair(16), y = pair(17);
     s.w1_tail[0][lane] = u32x4{x.h, y.h, 0u, 0u};        // h h: against (h, m)
     s.w1_tail[1][lane] = u32x4{x.l, y.l, 0u, 0u};        // l h: against (h, m)
     s.w1_tail[2][lane] = u32x4{x.m, y.m, x.h, y.h};      // m m, h l: against (m, l)
     s.w1_tail[3][lane] = u32x4{x.h, y.h, x.m, y.m};      // h m, m h: against (m, h)
-  }
-  if (wave == 0) (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
-  if (wave == 1) {
+  } else {
+    (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
 #pragma unroll
     for (int j = 0; j < 2; ++j) s.w3[j][lane] = W3[p * 128 + (2 * j + g) * 32 + n];
   }
@@ -288,12 +276,28 @@ __device__ __forceinline__ Split8 transpose_tile(const Split8& v, Vjp32Wave& s, 
   }
   return r;
 }
-__device__ __forceinline__ Split8 read_operand(const u32x4 (*b)[2][64], int lane) {
+// The operands of layer 2, W2[n][unit(8 s + j, g)] and, transposed, W2[unit(8 s + j, g)][n]
+__device__ __forceinline__ Split8 read_w2(const Vjp32Lds& w, int lane) {
+  asm volatile("" : "+v"(lane));
+  const int n = lane & 31, g = lane >> 5;
+  Split8 r;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const unsigned* const from = &w.w2[0][n][tile_place(2 * k + g, n)];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) r.p[p].s[k] = *reinterpret_cast<const u32x4*>(from + 512 * p);
+  }
+  return r;
+}
+__device__ __forceinline__ Split8 read_w2_transposed(const Vjp32Lds& w, int lane) {
+  asm volatile("" : "+v"(lane));
+  const int n = lane & 31, g = lane >> 5, row = 4 * g + ((n >> 2) & 3);
+  const char* const from = reinterpret_cast<const char*>(&w.w2[0][row][tile_place(2 * (n >> 4) + (n & 1), row) + (n & 2)]);
   Split8 r;
 #pragma unroll
   for (int p = 0; p < 3; ++p)
 #pragma unroll
-    for (int k = 0; k < 2; ++k) r.p[p].s[k] = b[p][k][lane];
+    for (int k = 0; k < 2; ++k) r.p[p].s[k] = read_records(from + 2048 * p, k, 64);
   return r;
 }
 struct SplitOperand {
@@ -360,7 +364,7 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   SplitAcc t1;
   t1.big = t1.small = splat16(0.f);
   SplitOperand e, e0, e1, e2, e3;
-  mma_split(d2, read_operand(w.w2t, lane), t1);
+  mma_split(d2, read_w2_transposed(w, lane), t1);
   vjp32_encode<0>(x[0], factor, s, n, g, u, e, [&](int, const SplitOperand& v) { e0 = v; });
   __builtin_amdgcn_sched_barrier(0);
   vf32x16 tsum = t1.sum();
@@ -453,7 +457,7 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   SplitAcc o2;
   o2.big = splat16(bias2);
   o2.small = splat16(0.f);
-  mma_split(h1, read_operand(w.w2, lane), o2);
+  mma_split(h1, read_w2(w, lane), o2);
   const u32x2 ones = {Ops<__bf16>::kOneWord, Ops<__bf16>::kOneWord};
 #pragma unroll
   for (int k = 0; k < 2; ++k) {

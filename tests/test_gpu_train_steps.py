@@ -262,7 +262,7 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
 @pytest.mark.parametrize("precision", [0, 1, 2])
 @pytest.mark.parametrize("tiles", [1, 3, 4, 5, 15, 16, 17, 31, 129, 255])
 def test_weight_gradients_of_runs_of_every_length(device, tiles, precision):
-    """The kernels deal a run's half steps to eight wavefronts and cut the steps into chunks of 16 to 256: runs of one
+    """The kernels deal a run's half steps to four wavefronts and cut the steps into chunks of 16 to 128: runs of one
     primitive that are a little shorter and longer than those, three in a row, against float64 over the same steps.  An f32
     gradient is a sum of up to 16,000 products of two factors that are f32 sums of up to 72 terms themselves: a few units of
     2^-24 each, 1e-6 of the norm.  A phase is an f32 product of two roundings, and moves its sine by as much: 2^-23 times the
