@@ -18,8 +18,8 @@ namespace mlpsp {
 // kernels spend a full 64-lane ray/ellipsoid test on each.  Here, where one LANE handles one
 // candidate, the tile's rays are enclosed in the pyramid of its four corner rays (verified against
 // every ray of the tile), and a candidate whose threshold ellipsoid {x : (x-c)^T A (x-c) < -2 ln thr}
-// lies entirely beyond one of the pyramid's four faces can be hit by no ray of the tile.  For a face
-// with inward normal n through the common origin o that is  n.(c-o) < 0  and
+// lies entirely beyond one of the pyramid's four faces, or of four planes through its edges, can be hit by no ray of the tile.
+// For a plane with inward normal n through the common origin o that is  n.(c-o) < 0  and
 // (n.(c-o))^2 >= -2 ln thr * sum_k s_k^2 (R^T n)_k^2, tested with a 2 % margin on the radius, far
 // above f32 rounding.  Such an entry is written as ~id (negative) AFTER the tile's sorted survivors, in
 // reverse list order: the render kernels skip negative ids, so the image is unchanged bit for bit, and only the
@@ -50,7 +50,7 @@ struct SortLds {
 // key_tstar(), so the key of a candidate costs one quaternion rotation (the ray direction's) instead of two, with
 // the same bits.  For the culling test the record carries e = c - o and the world-space covariance
 // S = R diag(s^2) R^T, so that the support of the threshold ellipsoid along a face normal n is the quadratic form
-// n^T S n (six multiply-adds against per-tile products of the normal) instead of a rotation of n per face.  S is
+// n^T S n instead of a rotation of n per face.  S is
 // stored as six bf16 values rounded so that the stored matrix minus the exact one is positive semi-definite
 // (off-diagonal entries to nearest, every diagonal entry raised by its row's rounding errors plus 1e-5 of the
 // trace, then rounded up): the quadratic form never comes out smaller than the exact one, i.e. the test stays
@@ -157,7 +157,6 @@ __device__ __forceinline__ float key_depth_hoisted(float dx, float dy, float dz,
 struct TilePyramid {
   float ox, oy, oz;        // the tile's common origin (corner 0's)
   float n[4][3];           // inward normals
-  float q[4][6];           // nx^2, ny^2, nz^2, 2 nx ny, 2 nx nz, 2 ny nz of each
   int faces;               // bit j: face j may be used (0: no culling for this tile)
 };
 __device__ __forceinline__ float lane_value(float v, int lane) {
@@ -221,7 +220,6 @@ __device__ __forceinline__ TilePyramid tile_pyramid(const float* __restrict__ ra
   nx *= sgn;
   ny *= sgn;
   nz *= sgn;
-  const float prod[6] = {nx * nx, ny * ny, nz * nz, 2.f * (nx * ny), 2.f * (nx * nz), 2.f * (ny * nz)};
   float nlen[4];
   int ok = 0x10;
 #pragma unroll
@@ -230,8 +228,6 @@ __device__ __forceinline__ TilePyramid tile_pyramid(const float* __restrict__ ra
     py.n[f][1] = lane_value(ny, f);
     py.n[f][2] = lane_value(nz, f);
     nlen[f] = lane_value(len, f);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) py.q[f][k] = lane_value(prod[k], f);
     ok |= ((__ballot(usable) >> f) & 1ull) ? (1 << f) : 0;
   }
   for (int k = lane; k < g.TW * g.TH; k += 64) {
@@ -256,18 +252,17 @@ __device__ __forceinline__ TilePyramid tile_pyramid(const float* __restrict__ ra
   return py;
 }
 
-// The pyramid of a tile as the frame prologue leaves it for the sort: the four normals, the origin, the usable
-// faces, the products of the normals' components (forty words).  Built once per tile there; a sort that is not handed such records builds the pyramid in each of a tile's
+// The pyramid of a tile as the frame prologue leaves it for the sort: the four normals, the origin and the
+// usable faces.  Built once per tile there; a sort that is not handed such records builds the pyramid in each of a tile's
 // wavefronts, whose strided reads of the tile's 64 rays (12-byte stride over eight image rows, by all four
 // wavefronts) measured 18 us of the 134 us launch at 12,750 tiles.
 struct alignas(32) TilePyramidRec {
   float n[4][3];
   float ox, oy, oz;
   int faces;
-  float q[4][6];
+  float unused[24];        // (the record's size is part of the C ABI)
 };
-static_assert(sizeof(TilePyramidRec) == MLPSP_TILE_PYRAMID_BYTES && MLPSP_TILE_PYRAMID_BYTES == 40 * 4,
-              "forty words per tile");
+static_assert(sizeof(TilePyramidRec) == MLPSP_TILE_PYRAMID_BYTES, "record size");
 // One wavefront per tile; `raw` are the directions before normalisation.
 __device__ __forceinline__ void write_tile_pyramid(const float* __restrict__ rays_o, const float* __restrict__ raw,
                                                    const TileGeom& g, int tile, TilePyramidRec* __restrict__ out) {
@@ -276,26 +271,18 @@ __device__ __forceinline__ void write_tile_pyramid(const float* __restrict__ ray
   RawDirs{raw}.get(pc, dx, dy, dz);
   const TilePyramid py = tile_pyramid(rays_o, RawDirs{raw}, g, tile, dx, dy, dz);
   if ((threadIdx.x & 63) == 0) {
-    TilePyramidRec r;
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) r.n[f][k] = py.n[f][k];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) r.q[f][k] = py.q[f][k];
-    }
-    r.ox = py.ox;
-    r.oy = py.oy;
-    r.oz = py.oz;
-    r.faces = py.faces;
-    out[tile] = r;
+    float4* to = reinterpret_cast<float4*>(out + tile);
+    to[0] = make_float4(py.n[0][0], py.n[0][1], py.n[0][2], py.n[1][0]);
+    to[1] = make_float4(py.n[1][1], py.n[1][2], py.n[2][0], py.n[2][1]);
+    to[2] = make_float4(py.n[2][2], py.n[3][0], py.n[3][1], py.n[3][2]);
+    to[3] = make_float4(py.ox, py.oy, py.oz, bits_to_float((uint32_t)py.faces));
   }
 }
 // A record as a wavefront holds it: lane j has word j (one coalesced load), and the words are taken out of that
 // register with v_readlane, the way tile_pyramid() hands out what its lanes computed.
 __device__ __forceinline__ float pyramid_record_word(const TilePyramidRec* __restrict__ record) {
   const int lane = threadIdx.x & 63;
-  return reinterpret_cast<const float*>(record)[lane < 40 ? lane : 0];
+  return reinterpret_cast<const float*>(record)[lane & 15];
 }
 __device__ __forceinline__ TilePyramid pyramid_from_word(float word) {
   TilePyramid py;
@@ -309,16 +296,25 @@ __device__ __forceinline__ TilePyramid pyramid_from_word(float word) {
     py.n[f][0] = nx;
     py.n[f][1] = ny;
     py.n[f][2] = nz;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) py.q[f][k] = lane_value(word, 16 + f * 6 + k);
   }
   return py;
 }
 
-// Can no ray of the tile hit the primitive?  True if its threshold ellipsoid lies wholly beyond one usable face.
-// General form: every face normal is taken into the primitive's axes with the rotation matrix of the quaternion,
-// worked out once per candidate (24 instructions + 9 per face, where a quaternion rotation per face costs 21; fused
-// multiply-adds throughout: roundings are free here, the test keeps a margin of 2 % of the radius).
+// Can no ray of the tile hit the primitive?  True if its threshold ellipsoid lies wholly beyond one usable face, or beyond a
+// plane through the edge where two of them meet.  In units of the ellipsoid's support along a face's normal (r n: support 1)
+// the centre is e = r n.(c - o) in front of the face; the normal taken at the edge is the sum of both faces' r n, whose support
+// squared is 2 + 2 rho with rho the product of the two in the ellipsoid's metric.  (The rays of the tile are in front of every
+// plane whose normal is a sum of face normals.)  rho has an error of 7e-7, which counts where it is close to -1, for discs and
+// needles: 4e-6 of the radius squared are added.  The edges' planes take out half to two thirds of what the faces leave that no
+// pixel is hit by: entries tested per tile at the 200,000-primitive 1200x680 frame 86 -> 70, of which 55 hit; render kernel
+// 526 -> 490 us (bf16), 355 -> 333 at 50,000 primitives and 641x479 (fp16), for 2 us of this one's 93.  The best plane
+// through each edge would take out another tenth, for as many instructions again.
+__device__ __forceinline__ bool beyond_edge(const TilePyramid& py, int j, int k, float both, float rho, float r2) {
+  return (((py.faces >> j) & (py.faces >> k)) & 1) && (both * __builtin_fabsf(both) < fmaf(rho, -2.f * r2, -2.000004f * r2));
+}
+// General form: the normals in the primitive's axes, scaled by its semi-axes and the cull radius (41 instructions once per
+// candidate, 28 per face; fused multiply-adds throughout: roundings are free here, the test keeps a margin of 2 % of the
+// radius).
 __device__ __forceinline__ bool outside_pyramid(const TilePyramid& py, const PrimRecord& P, float cull_r2) {
   bool outside = false;
   const float ex = P.cx - py.ox, ey = P.cy - py.oy, ez = P.cz - py.oz;
@@ -327,40 +323,54 @@ __device__ __forceinline__ bool outside_pyramid(const TilePyramid& py, const Pri
   const float x2 = x + x, y2 = y + y, z2 = z + z;
   const float xx = x * x2, yy = y * y2, zz = z * z2, xy = x * y2, xz = x * z2, yz = y * z2;
   const float wx = w * x2, wy = w * y2, wz = w * z2;
-  const float r00 = 1.f - (yy + zz), r01 = xy - wz, r02 = xz + wy;
-  const float r10 = xy + wz, r11 = 1.f - (xx + zz), r12 = yz - wx;
-  const float r20 = xz - wy, r21 = yz + wx, r22 = 1.f - (xx + yy);
-  // squared semi-axes as reciprocals of the precision diagonal (one unit in the last place, far inside the margin;
-  // 1/0 = inf never culls): the record's own s2 words lie in its fourth 16-byte piece, which nothing else here
-  // needs -- a candidate is then three requests instead of four
-  // (with the squared cull radius folded in: beyond a face means dist < 0 and dist^2 > r^2 h^2, i.e.
-  // dist |dist| < -(r^2 h^2): one product and one comparison per face)
-  const float s2x = cull_r2 * __builtin_amdgcn_rcpf(P.mx), s2y = cull_r2 * __builtin_amdgcn_rcpf(P.my),
-              s2z = cull_r2 * __builtin_amdgcn_rcpf(P.mz);
+  // semi-axes as reciprocal roots of the precision diagonal (a unit in the last place, far inside the margin; a support that is
+  // not finite makes e zero or NaN and never culls): the record's own s2 words lie in its fourth 16-byte piece, which nothing
+  // else here needs -- a candidate is then three requests instead of four
+  const float sx = __builtin_amdgcn_rsqf(P.mx), sy = __builtin_amdgcn_rsqf(P.my), sz = __builtin_amdgcn_rsqf(P.mz);
+  const float r00 = sx * (1.f - (yy + zz)), r01 = sy * (xy - wz), r02 = sz * (xz + wy);
+  const float r10 = sx * (xy + wz), r11 = sy * (1.f - (xx + zz)), r12 = sz * (yz - wx);
+  const float r20 = sx * (xz - wy), r21 = sy * (yz + wx), r22 = sz * (1.f - (xx + yy));
+  float l[4][3], r[4], e[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float nx = py.n[j][0], ny = py.n[j][1], nz = py.n[j][2];
-    const float dist = fmaf(nx, ex, fmaf(ny, ey, nz * ez));
-    const float lx = fmaf(r00, nx, fmaf(r10, ny, r20 * nz));
-    const float ly = fmaf(r01, nx, fmaf(r11, ny, r21 * nz));
-    const float lz = fmaf(r02, nx, fmaf(r12, ny, r22 * nz));
-    const float h2 = fmaf(s2x * lx, lx, fmaf(s2y * ly, ly, (s2z * lz) * lz));
-    outside |= ((py.faces >> j) & 1) && (dist * __builtin_fabsf(dist) < -h2);
+    l[j][0] = fmaf(r00, nx, fmaf(r10, ny, r20 * nz));
+    l[j][1] = fmaf(r01, nx, fmaf(r11, ny, r21 * nz));
+    l[j][2] = fmaf(r02, nx, fmaf(r12, ny, r22 * nz));
+    r[j] = __builtin_amdgcn_rsqf(fmaf(l[j][0], l[j][0], fmaf(l[j][1], l[j][1], l[j][2] * l[j][2])));
+    e[j] = r[j] * fmaf(nx, ex, fmaf(ny, ey, nz * ez));
+    outside |= ((py.faces >> j) & 1) && (e[j] * __builtin_fabsf(e[j]) < -cull_r2);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int k = (j + 1) & 3;
+    const float rho = (r[j] * r[k]) * fmaf(l[j][0], l[k][0], fmaf(l[j][1], l[k][1], l[j][2] * l[k][2]));
+    outside |= beyond_edge(py, j, k, e[j] + e[k], rho, cull_r2);
   }
   return outside;
 }
-// With a frame record: the support along n is the quadratic form of the (conservatively rounded) covariance.
+// With a frame record: in the metric of the (conservatively rounded) covariance.
 __device__ __forceinline__ bool outside_pyramid(const TilePyramid& py, const SortRec& R, float cull_r2) {
   bool outside = false;
   const float sxx = bits_to_float(R.s_xx_yy & 0xffff0000u), syy = bits_to_float(R.s_xx_yy << 16);
   const float szz = bits_to_float(R.s_zz_xy & 0xffff0000u), sxy = bits_to_float(R.s_zz_xy << 16);
   const float sxz = bits_to_float(R.s_xz_yz & 0xffff0000u), syz = bits_to_float(R.s_xz_yz << 16);
+  float u[4][3], r[4], e[4];               // u = S n
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const float dist = fmaf(py.n[j][0], R.ex, fmaf(py.n[j][1], R.ey, py.n[j][2] * R.ez));
-    const float h2 = fmaf(py.q[j][0], sxx, fmaf(py.q[j][1], syy, fmaf(py.q[j][2], szz,
-                     fmaf(py.q[j][3], sxy, fmaf(py.q[j][4], sxz, py.q[j][5] * syz)))));
-    outside |= ((py.faces >> j) & 1) && (dist < 0.f) && (dist * dist >= cull_r2 * h2);
+    const float nx = py.n[j][0], ny = py.n[j][1], nz = py.n[j][2];
+    u[j][0] = fmaf(nx, sxx, fmaf(ny, sxy, nz * sxz));
+    u[j][1] = fmaf(nx, sxy, fmaf(ny, syy, nz * syz));
+    u[j][2] = fmaf(nx, sxz, fmaf(ny, syz, nz * szz));
+    r[j] = __builtin_amdgcn_rsqf(fmaf(nx, u[j][0], fmaf(ny, u[j][1], nz * u[j][2])));
+    e[j] = r[j] * fmaf(nx, R.ex, fmaf(ny, R.ey, nz * R.ez));
+    outside |= ((py.faces >> j) & 1) && (e[j] * __builtin_fabsf(e[j]) < -cull_r2);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int k = (j + 1) & 3;
+    const float rho = (r[j] * r[k]) * fmaf(py.n[k][0], u[j][0], fmaf(py.n[k][1], u[j][1], py.n[k][2] * u[j][2]));
+    outside |= beyond_edge(py, j, k, e[j] + e[k], rho, cull_r2);
   }
   return outside;
 }

@@ -418,6 +418,52 @@ def test_conservative_tile_culling_never_drops_a_hit(device, oracle_mod, name, n
     assert bad == 0
 
 
+@pytest.mark.parametrize("frame_records", [True, False], ids=["frame_records", "full_key"])
+@pytest.mark.parametrize("thin,long", [(0.0, 0.0), (5.0, 0.0), (8.0, 0.0), (0.0, 3.0), (6.0, 2.0)], ids=str)
+def test_planes_through_the_edges_of_a_tile_cull_no_hit(device, thin, long, frame_records):
+    """Balls, discs (one axis e^-thin) and needles (one axis e^long): no culled (tile, primitive) has a ray inside its ellipsoid, in float64 up to 1e-3 of the squared radius (the radius
+    has a margin of 2 %), and some are culled that do not lie beyond one of the four faces."""
+    import math
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=1500, width=48, height=32)
+    sc = fr.scene
+    log_s = sc.log_scales.copy()
+    log_s[:, 0] -= thin
+    log_s[:, 1] += long
+    n, tiles = 1500, (fr.W // 8) * (fr.H // 8)
+    cand = np.tile(np.arange(n, dtype=np.int32), tiles)
+    off = np.arange(tiles + 1, dtype=np.int32) * n
+    ro, rd = _t(fr.rays_o, device), _t(fr.rays_d, device)
+    pos, logs, quat = (_t(a.astype(np.float32), device) for a in (sc.positions, log_s, sc.quats))
+    got, _ = ops.sort_tiles(ro, rd, ops.prepare_primitives(pos, logs, quat), _t(cand, device), _t(off, device), fr.W, fr.H, 8, 8,
+                            cull_threshold=fr.thr, frame_records=frame_records)
+    culled = torch.zeros(tiles, n, dtype=torch.bool, device=device)
+    t, k = (got.view(tiles, n) < 0).nonzero(as_tuple=True)
+    culled[t, (~got.view(tiles, n)[t, k]).long()] = True
+    w, x, y, z = torch.nn.functional.normalize(quat.double(), dim=-1).unbind(-1)
+    axes = torch.stack([1 - 2 * (y * y + z * z), 2 * (x * y - w * z), 2 * (x * z + w * y), 2 * (x * y + w * z),
+                        1 - 2 * (x * x + z * z), 2 * (y * z - w * x), 2 * (x * z - w * y), 2 * (y * z + w * x),
+                        1 - 2 * (x * x + y * y)], -1).view(-1, 3, 3)
+    scale, e = torch.exp(logs.double()), pos.double() - ro[0].double()
+    local = ((e[:, None] @ axes) / scale[:, None])[:, 0]                   # [n, 3], in units of the semi-axes
+    rays = rd.double().view(fr.H // 8, 8, fr.W // 8, 8, 3).permute(0, 2, 1, 3, 4).reshape(tiles, 64, 3)
+    r2, beyond = -2.0 * math.log(fr.thr), torch.zeros(tiles, n, dtype=torch.bool, device=device)
+    for i in range(tiles):
+        d = torch.nn.functional.normalize((rays[i] @ axes) / scale[:, None], dim=-1)      # [n, 64, 3]
+        along = (d * local[:, None]).sum(-1)
+        off_axis = ((local[:, None] - along[..., None] * d) ** 2).sum(-1)
+        hit = ((off_axis < r2 * (1.0 - 1e-3)) & (along > 0)).any(1)
+        assert not bool((hit & culled[i]).any())
+        corners, centre = rays[i][[0, 7, 63, 56]], rays[i].sum(0)
+        for j in range(4):
+            normal = torch.linalg.cross(corners[j], corners[(j + 1) % 4])
+            normal = normal * torch.sign(normal @ centre)
+            support = ((normal @ axes) * scale).norm(dim=-1)
+            beyond[i] |= e @ normal < -math.sqrt(r2) * support
+    # (the faces' own test has a margin: what it takes out lies beyond one of them)
+    assert int((culled & ~beyond).sum()) > 0
+
+
 def test_culling_is_off_for_tiles_with_mixed_origins_or_degenerate_pyramids(device, oracle_mod):
     from mlp_splatting_amd import ops
     fr = Frame("cfg1_5k_160x120", n=1500, width=32, height=24)
