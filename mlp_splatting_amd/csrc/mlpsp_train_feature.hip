@@ -16,11 +16,12 @@
 //
 // All are bound by memory traffic: attribute rows out of L2 in the blend (8 KB per step at 512 channels, four slots), sign
 // rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each).  At 200,000 primitives,
-// 1200x680, a 300x170 target of 512 channels: 0.45, 0.06, 0.42 and 0.28 ms; the record kernels took 4.95 ms for the
+// 1200x680, a 300x170 target of 512 channels: 0.45, 0.06, 0.20 and 0.28 ms; the record kernels took 4.95 ms for the
 // loss and 8.1 ms for the gradient.
 #include <type_traits>
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
+#include "mlpsp_mfma16.hpp"
 #include "mlpsp_train.hpp"
 
 namespace mlpsp {
@@ -78,6 +79,9 @@ inline bool feat_shape(int width, int height, int wf, int hf, int channels, int 
 }
 // Kept for the backward: spans int32[2 (ntx + nty)] | groups of four targets of every tile int32[T] | signs int8[T][NT][Cp]
 // | k float[S][NT / 4][slots][4].  Scratch of the forward: shares float[T][NT][Cp].
+// A sign is the upper byte of a bf16 2, 0 or -2 (the lower one is zero): an integer of kSignUnit, 0 or -kSignUnit.
+constexpr int kSignUnit = 64;
+constexpr float kSignValue = 2.f;        // as bf16
 struct FeatKept {
   int2 *columns, *rows;
   int32_t* groups;
@@ -290,7 +294,7 @@ __global__ __launch_bounds__(256) void train_feature_join_kernel(FeatShape f, Fe
     for (int k = 0; k < 4; ++k) {
       if (c + k < f.C) {
         const float delta = v[k] - (float)want[c + k];
-        signs |= (uint32_t)(uint8_t)(int8_t)((delta > 0.f) - (delta < 0.f)) << (8 * k);
+        signs |= (uint32_t)(uint8_t)(int8_t)(kSignUnit * ((delta > 0.f) - (delta < 0.f))) << (8 * k);
         part += __builtin_fabsf(delta);
       }
     }
@@ -318,7 +322,7 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
   const int c = (int)blockIdx.y * 256 + (lane & (lpr - 1)) * 4;
   const bool channels = c < f.C;
   const int cs = channels ? c : 0;
-  const float norm = (float)((long long)f.WF * f.HF * f.C), scale = adjoint[0];
+  const float norm = (float)((long long)f.WF * f.HF * f.C) * kSignUnit, scale = adjoint[0];
   const size_t k_stride = (size_t)f.NT * SLOTS;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const int p = __builtin_amdgcn_readfirstlane(prim[pos]);
@@ -389,17 +393,116 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
   }
 }
 
+// The same for four slots and rows of 128 channels and more, in sixteens, on the matrix cores: a product of k (four slots x
+// steps and targets) and signs (steps and targets x channels) in 16x16x32 bf16 products.  Exact in its factors: a sign is a
+// bf16 number, k the sum of three (mlpsp_vjp32.hpp), which take three times four of the sixteen rows and have accumulators of
+// their own.  One wavefront = one chunk x 256 channels, eight steps at a time: lane (n, q) has two steps, and of their signs the
+// channels 16 n .. 16 n + 15 -- sixteen bytes of a row a load; product j takes byte j of each, one byte permutation a word.
+// The lanes hold the chunk's steps and their tiles' groups; a step's rows are not behind a chain of reads.
+// Bound by the latency of those rows (2 KB a step at 512 channels), three wavefronts to a SIMD.  648,000 steps, 512 channels:
+// 440 -> 200 us; error against float64 1.4e-7 -> 1.3e-7 of the gradient's norm, of a primitive's 1.4e-7 -> 0.6e-7 (median).
+__global__ __launch_bounds__(256) void train_attr_mfma_kernel(FeatShape f, FeatKept o, const int32_t* __restrict__ prim,
+                                                              const int32_t* __restrict__ first, const int4* __restrict__ step,
+                                                              int S, int chunk_steps, int num_chunks,
+                                                              const float* __restrict__ adjoint, float* __restrict__ rows,
+                                                              float* __restrict__ out) {
+  const int chunk = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
+  if (chunk >= num_chunks) return;
+  const int chunk_begin = chunk * chunk_steps, chunk_end = min(S, chunk_begin + chunk_steps);
+  const int c = (int)blockIdx.y * 256 + 16 * n, cs = c < f.C ? c : 0;
+  const float norm = (float)((long long)f.WF * f.HF * f.C) * kSignValue, scale = adjoint[0];
+  const int4 mine = step[min(chunk_begin + lane, chunk_end - 1)];       // (of up to 64)
+  const int my_groups = o.groups[mine.z], parts = f.NT >> 2;
+  for (int pos = chunk_begin; pos < chunk_end;) {
+    const int p = __builtin_amdgcn_readfirstlane(prim[pos]);
+    const int all_end = first[p + 1], end = min(all_end, chunk_end);
+    const bool goes_on = all_end > chunk_end, complete = first[p] == pos && !goes_on;
+    f32x4 acc[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = pos; i < end; i += 8) {
+      int number[2], tile[2], groups[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int at = i + 2 * q + t, from = min(at, end - 1) - chunk_begin;
+        number[t] = __shfl(mine.y, from);
+        tile[t] = __shfl(mine.z, from);
+        groups[t] = __shfl(my_groups, from);
+        if (at >= end) groups[t] = 0;
+      }
+      for (int g = 0; g < parts && __ballot(groups[0] > g || groups[1] > g) != 0ull; ++g) {
+        u32x4 sign[2][4];
+        float4 k[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int8_t* __restrict__ from = o.signs + ((size_t)tile[t] * f.NT + 4 * g) * f.Cp + cs;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sign[t][r] = *reinterpret_cast<const u32x4*>(from + (size_t)r * f.Cp);
+          k[t] = *reinterpret_cast<const float4*>(o.k + ((size_t)number[t] * parts + g) * 16 + 4 * (n & 3));
+        }
+        // row n of the one operand: part n / 4 of slot n % 4
+        float v[8] = {k[0].x, k[0].y, k[0].z, k[0].w, k[1].x, k[1].y, k[1].z, k[1].w};
+        u32x4 a;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const bool live = groups[d >> 1] > g && n < 12;
+          float x = live ? v[2 * d] : 0.f, y = live ? v[2 * d + 1] : 0.f;
+#pragma unroll
+          for (int part = 0; part < 2; ++part) {
+            const unsigned h = Ops<__bf16>::pack2(x, y);
+            if ((n >> 2) > part) {
+              x -= __uint_as_float(h << 16);
+              y -= __uint_as_float(h & 0xffff0000u);
+            }
+          }
+          a[d] = Ops<__bf16>::pack2(x, y);
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const unsigned byte = 0x040c000cu + 0x01000100u * (unsigned)(j & 3);
+          u32x4 b;
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            b[d] = __builtin_amdgcn_perm(sign[d >> 1][2 * (d & 1) + 1][j >> 2], sign[d >> 1][2 * (d & 1)][j >> 2], byte);
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc[j],
+                                                           0, 0, 0);
+        }
+      }
+    }
+    // rows 4 q + slot of a product lie in lane group q: the three parts added up, slot q to group q
+    float sum[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float even = sum_of_halves(acc[j][0], acc[j][2]), odd = sum_of_halves(acc[j][1], acc[j][3]);
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(even), __float_as_uint(odd), false, false);
+      const unsigned lo = r[0], hi = r[1];
+      sum[j] = __uint_as_float(lo) + __uint_as_float(hi);
+    }
+    if (c < f.C) {
+      float* __restrict__ dst = complete ? out + ((size_t)p * 4 + q) * f.C + c
+                                         : rows + ((size_t)(goes_on ? num_chunks + chunk : chunk) * 4 + q) * f.Cp + c;
+#pragma unroll
+      for (int j = 0; j < 16; j += 4) {
+        float4 v = make_float4(sum[j], sum[j + 1], sum[j + 2], sum[j + 3]);
+        if (complete) v = make_float4(v.x / norm * scale, v.y / norm * scale, v.z / norm * scale, v.w / norm * scale);
+        *reinterpret_cast<float4*>(dst + j) = v;
+      }
+    }
+    pos = end;
+  }
+}
+
 // One workgroup per chunk, lane = four channels of one slot: the rows of the primitive that begins in it and goes on.
 template <bool VEC>
 __global__ __launch_bounds__(256) void train_attr_join_kernel(FeatShape f, const int32_t* __restrict__ prim,
                                                               const int32_t* __restrict__ first, int S, int chunk_steps,
-                                                              int num_chunks, const float* __restrict__ adjoint,
+                                                              int num_chunks, float unit, const float* __restrict__ adjoint,
                                                               const float* __restrict__ rows, float* __restrict__ out) {
   const int cf = blockIdx.x;
   const SpanningRun run = spanning_run(prim, first, S, cf, chunk_steps);
   if (run.p < 0) return;
   const int cl = run.last_chunk;
-  const float norm = (float)((long long)f.WF * f.HF * f.C), scale = adjoint[0];
+  const float norm = (float)((long long)f.WF * f.HF * f.C) * unit, scale = adjoint[0];
   const int quads = f.Cp >> 2;
   for (int i = threadIdx.x; i < quads * f.slots; i += 256) {
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -515,17 +618,23 @@ MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int he
 #define MLPSP_ATTR(SL, VEC)                                                                                              \
   hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, t.prim, t.first, t.step,         \
                      (int)num_steps, per, chunks, lanes_per_row_log2(f.Cp), loss_adjoint_dev, rows_dev, out_dev)
-    if (slots == 1) { if (vec) MLPSP_ATTR(1, true); else MLPSP_ATTR(1, false); }
+    // (fewer channels leave lanes without work)
+    const bool wide = slots == 4 && vec && channels % 16 == 0 && channels >= 128 && ((uintptr_t)kept_dev & 15u) == 0;
+    const float unit = wide ? kSignValue : (float)kSignUnit;
+    if (wide)
+      hipLaunchKernelGGL(train_attr_mfma_kernel, grid, dim3(256), 0, s, f, o, t.prim, t.first, t.step, (int)num_steps, per, chunks,
+                         loss_adjoint_dev, rows_dev, out_dev);
+    else if (slots == 1) { if (vec) MLPSP_ATTR(1, true); else MLPSP_ATTR(1, false); }
     else if (slots == 4) { if (vec) MLPSP_ATTR(4, true); else MLPSP_ATTR(4, false); }
     else { if (vec) MLPSP_ATTR(5, true); else MLPSP_ATTR(5, false); }
 #undef MLPSP_ATTR
     MLPSP_LAUNCH_CHECK();
     if (vec)
       hipLaunchKernelGGL(train_attr_join_kernel<true>, dim3((unsigned)chunks), dim3(256), 0, s, f, t.prim, t.first,
-                         (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
+                         (int)num_steps, per, chunks, unit, loss_adjoint_dev, rows_dev, out_dev);
     else
       hipLaunchKernelGGL(train_attr_join_kernel<false>, dim3((unsigned)chunks), dim3(256), 0, s, f, t.prim, t.first,
-                         (int)num_steps, per, chunks, loss_adjoint_dev, rows_dev, out_dev);
+                         (int)num_steps, per, chunks, unit, loss_adjoint_dev, rows_dev, out_dev);
     MLPSP_LAUNCH_CHECK();
   }
   ZeroRows zero{};
