@@ -8,14 +8,16 @@
 // takes six instructions of 32 clocks instead of eight of 64, and rounds its accumulator six times instead of sixteen.
 // Error of the gradients against float64, 2-norm over 2-norm, f32 chains of v_mfma_f32_32x32x2_f32 -> here:
 //                           W1                 b1                 W2                 b2                 W3
-//   647,988 steps   3.9e-7 -> 2.4e-7   2.8e-7 -> 1.5e-7   3.4e-7 -> 2.1e-7   3.7e-7 -> 1.1e-7   2.8e-7 -> 1.4e-7
+//   647,988 steps   3.9e-7 -> 2.5e-7   2.8e-7 -> 1.5e-7   3.4e-7 -> 2.1e-7   3.7e-7 -> 1.1e-7   2.8e-7 -> 1.5e-7
 //    51,614 steps   1.9e-7 -> 1.2e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.1e-7   2.2e-7 -> 0.7e-7   1.7e-7 -> 1.0e-7
-// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.45 -> 5.17 ms, 0.72 -> 0.48 ms.
+// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.45 -> 4.96 ms, 0.72 -> 0.47 ms.
 //
-// Bound by the ~1,250 vector instructions of a block (half of them sines and cosines, a sixth the splits), two wavefronts to
-// a SIMD: 256 registers with the weights in LDS.  A wavefront with its own weights in registers spills (6.7 ms, waiting for
-// its spills behind the records requested ahead), alone on its SIMD it is no faster for 512 registers (7.0).  The two belong to
-// different workgroups, one of which works while the other changes primitives (one workgroup of eight: 5.23 and 0.52 ms).
+// Bound by the latency of a block's chain -- products, the ~920 vector instructions between them (a third of them sines and
+// cosines, a sixth the splits), LDS --, two wavefronts to a SIMD: 256 registers with the weights in LDS.  (A third of the vector
+// instructions less, by the table of vjp32_sincos, is 3 % of the time.)  A wavefront with its own weights in registers spills
+// (6.7 ms, waiting for its spills behind the records requested ahead), alone on its SIMD it is no faster for 512 registers
+// (7.0).  The two belong to different workgroups, one of which works while the other changes primitives (one workgroup of
+// eight: 5.23 and 0.52 ms instead of 5.17 and 0.48).
 //
 // Per block (lane (n, g) = record n, half g of its inputs; D(a, b) has the rows of a in its registers):
 //   d2        D(W3, d): record in the lane, unit 8 (i / 4) + 4 g + i % 4 in register i, in f32 products
@@ -35,6 +37,7 @@
 namespace mlpsp {
 
 typedef short i16x4v __attribute__((ext_vector_type(4)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
 
 // Pairs of f32 as packed bf16: h + m + l = the pair.
 struct Split2 {
@@ -106,7 +109,7 @@ __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4&
   return Ops<__bf16>::mfma(ha, hb, acc);
 }
 
-// A workgroup of four wavefronts, two workgroups to a CU: 23 KB of operands that its wavefronts read, 14 KB of each one's own.
+// A workgroup of four wavefronts, two workgroups to a CU: 23 KB of operands and 2 KB of turns that its wavefronts read, 14 KB of each one's own.
 constexpr int kVjp32Waves = 4;
 union Vjp32Wave {
   struct {
@@ -129,6 +132,7 @@ struct Vjp32Lds {
   float w3[2][64];               // W3[2 j + g][n]
   float bias1[32], bias2[32];
   __attribute__((aligned(16))) unsigned zero[4];
+  f32x2v circle[256];
   Vjp32Wave wave[kVjp32Waves];
 };
 static_assert(2 * sizeof(Vjp32Lds) <= 163840, "two workgroups per CU");
@@ -221,39 +225,40 @@ struct Vjp32Sums {
   }
 };
 
-// The six (sin, cos) pairs of one input component: encode_component() to the last place but one (pi/2 in two parts instead of
-// three, the phase's factor in one product), without a branch: where one of the phases is out of range, all of the
-// component's values are NaN.
-__device__ __forceinline__ void vjp32_sincos(float x, const float (&factor)[6], float s_out[6], float c_out[6]) {
-  float phase[6];
-#pragma unroll
-  for (int f = 0; f < 6; ++f) phase[f] = x * factor[f];
-  const float reach = fmaxf(fmaxf(fmaxf(__builtin_fabsf(phase[0]), __builtin_fabsf(phase[1])),
-                                  fmaxf(__builtin_fabsf(phase[2]), __builtin_fabsf(phase[3]))),
-                            fmaxf(__builtin_fabsf(phase[4]), __builtin_fabsf(phase[5])));
-  const float stop = reach <= 65536.0f ? 0.f : __builtin_nanf("");
+// The six (sin, cos) pairs of one input component, from a table of 256 turns k 2 pi / 256 and a rotation by the rest, |r| <=
+// pi / 256: sin r = r - r^3 / 6 and cos r = 1 - r^2 / 2 to 2e-12 and 1e-9.  What a pair is off by is the rounding of the two
+// table values and of the two products, 1e-7 as from a polynomial in the reduced phase, in 15 instructions and an LDS read
+// instead of 27 instructions (gradient call 5.11 -> 4.96 and 0.480 -> 0.467 ms).  `limit`: the largest factor; where the component's largest phase is out of range, all of its values are NaN.
+struct CircleTable {
+  float at[256][2];
+  constexpr CircleTable() : at{} {
+    for (int k = 0; k < 256; ++k) {
+      const double x = (k < 128 ? k : k - 256) * (6.283185307179586476925 / 256.0);
+      double sine = 0.0, cosine = 0.0, term = 1.0;      // x^i / i!
+      for (int i = 0; i < 40; ++i) {
+        (i & 1 ? sine : cosine) += i & 2 ? -term : term;
+        term *= x / (i + 1);
+      }
+      at[k][0] = (float)sine;
+      at[k][1] = (float)cosine;
+    }
+  }
+};
+static __device__ const CircleTable kCircle = CircleTable();
+__device__ __forceinline__ void vjp32_sincos(const f32x2v* circle, float x, const float (&factor)[6], float limit, float s_out[6],
+                                             float c_out[6]) {
+  x = __builtin_fabsf(x) * limit <= 65536.0f ? x : __builtin_nanf("");
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
-    const float shifted = fmaf(phase[f], 0.636619772f, 12582912.0f);     // the nearest quarter turn, in the low bits
+    const float phase = x * factor[f];
+    const float shifted = fmaf(phase, 40.7436654f, 12582912.0f);         // the nearest turn, in the low bits
     const float kf = shifted - 12582912.0f;
-    float r = fmaf(kf, -1.57079637f, phase[f]);
-    r = fmaf(kf, 4.37113883e-08f, r) + stop;
-    const float z = r * r;
-    float ps = 2.75573192e-06f;
-    ps = fmaf(ps, z, -1.98412698e-04f);
-    ps = fmaf(ps, z, 8.33333333e-03f);
-    ps = fmaf(ps, z, -1.66666667e-01f);
-    const float s = fmaf(r * z, ps, r);
-    float pc = -2.75573192e-07f;
-    pc = fmaf(pc, z, 2.48015873e-05f);
-    pc = fmaf(pc, z, -1.38888889e-03f);
-    pc = fmaf(pc, z, 4.16666667e-02f);
-    const float c = fmaf(z * z, pc, fmaf(z, -0.5f, 1.0f));
-    const uint32_t q = float_to_bits(shifted);
-    const bool odd = (q & 1u) != 0u;
-    const uint32_t turn = q << 30;             // bit 31: the sine's sign; one more quarter turn: the cosine's
-    s_out[f] = bits_to_float(float_to_bits(odd ? c : s) ^ (turn & 0x80000000u));
-    c_out[f] = bits_to_float(float_to_bits(odd ? s : c) ^ ((turn + 0x40000000u) & 0x80000000u));
+    float r = fmaf(kf, -0.0245436933f, phase);
+    r = fmaf(kf, 6.82990470e-10f, r);
+    const f32x2v at = *reinterpret_cast<const f32x2v*>(reinterpret_cast<const char*>(circle) + ((float_to_bits(shifted) << 3) & 0x7f8u));
+    const float z = r * r, less = -0.5f * z, sine = fmaf(r * z, -0.166666667f, r);
+    s_out[f] = fmaf(at[1], sine, fmaf(at[0], less, at[0]));
+    c_out[f] = fmaf(-at[0], sine, fmaf(at[1], less, at[1]));
   }
 }
 // v where bit `bit` of word is set, else +0
@@ -311,10 +316,10 @@ __device__ __forceinline__ void mfma_split(const SplitOperand& a, const SplitOpe
 }
 // Six pairs of the encoding as operands: e.p[..][t % 4] of K-step t / 4; a finished K-step goes to LDS and to `done`.
 template <int C, typename Done>
-__device__ __forceinline__ void vjp32_encode(float x, const float (&factor)[6], Vjp32Wave& s, int n, int g, const SplitUnits& u,
+__device__ __forceinline__ void vjp32_encode(const f32x2v* circle, float x, const float (&factor)[6], float limit, Vjp32Wave& s, int n, int g, const SplitUnits& u,
                                              SplitOperand& e, Done&& done) {
   float sn[6], cs[6];
-  vjp32_sincos(x, factor, sn, cs);
+  vjp32_sincos(circle, x, factor, limit, sn, cs);
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
     const int t = 6 * C + f;
@@ -336,8 +341,8 @@ __device__ __forceinline__ void vjp32_encode(float x, const float (&factor)[6], 
 // (sched_barrier): mixed by the compiler they need more registers than there are.  (Matrix and vector instructions of a part
 // alternated by hand: no faster; the other wavefront of the SIMD fills the gaps.)
 __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, Vjp32Wave& s, const float x[3], float4 adjoint,
-                                            uint32_t mask1, uint32_t mask2, const float (&factor)[6], float scale, int lane,
-                                            const SplitUnits& u) {
+                                            uint32_t mask1, uint32_t mask2, const float (&factor)[6], float limit, float scale,
+                                            int lane, const SplitUnits& u) {
   asm volatile("" : "+v"(lane));         // (or the addresses are formed ahead of the loop over the blocks, one by one)
   const int n = lane & 31, g = lane >> 5;
   const float inf = relu_limit();
@@ -365,7 +370,7 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   t1.big = t1.small = splat16(0.f);
   SplitOperand e, e0, e1, e2, e3;
   mma_split(d2, read_w2_transposed(w, lane), t1);
-  vjp32_encode<0>(x[0], factor, s, n, g, u, e, [&](int, const SplitOperand& v) { e0 = v; });
+  vjp32_encode<0>(w.circle, x[0], factor, limit, s, n, g, u, e, [&](int, const SplitOperand& v) { e0 = v; });
   __builtin_amdgcn_sched_barrier(0);
   vf32x16 tsum = t1.sum();
   SplitAcc a1;
@@ -377,11 +382,11 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   }
   a1.small = splat16(0.f);
   mfma_split(read_step(w.w1, 0, lane), e0, a1);
-  vjp32_encode<1>(x[1], factor, s, n, g, u, e, [&](int k, const SplitOperand& v) { (k == 1 ? e1 : e2) = v; });
+  vjp32_encode<1>(w.circle, x[1], factor, limit, s, n, g, u, e, [&](int k, const SplitOperand& v) { (k == 1 ? e1 : e2) = v; });
   __builtin_amdgcn_sched_barrier(0);
   mfma_split(read_step(w.w1, 1, lane), e1, a1);
   mfma_split(read_step(w.w1, 2, lane), e2, a1);
-  vjp32_encode<2>(x[2], factor, s, n, g, u, e, [&](int, const SplitOperand& v) { e3 = v; });
+  vjp32_encode<2>(w.circle, x[2], factor, limit, s, n, g, u, e, [&](int, const SplitOperand& v) { e3 = v; });
 #pragma unroll
   for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&s.enc_tail[p][n][2 * g]) = u32x2{e.p[p][0], e.p[p][1]};
   __builtin_amdgcn_sched_barrier(0);
