@@ -370,19 +370,21 @@ __device__ __forceinline__ StepRecord step_record(const unsigned char* __restric
 }
 // A wavefront's share of a run: one half of every STRIDE-th step, from `first` on; work(record) for those that
 // have an adjoint.  Lane i asks for where the i-th of them lies; the next record is under way while one is worked on (two or
-// three: no faster).  Records without an adjoint get inputs of zero, whatever ray their lane has.
-template <int STRIDE, typename Work>
+// three: no faster).  Records
+// without an adjoint get inputs of zero, whatever ray their lane has.
+template <int STRIDE, bool FRESH, typename Work>
 __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int end, int half, const unsigned char* __restrict__ records,
-                                            const float4* __restrict__ d4, const float* __restrict__ rays_d, int n, int g, int W,
-                                            int pixels, Work&& work) {
+                                            const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int pixels,
+                                            int lane, Work&& work) {
   static_assert(kTrainChunk <= 64 * STRIDE, "a lane for every step");
   const int count = (end - first + STRIDE - 1) / STRIDE;
   if (count <= 0) return;
-  const int4 where = ix.step[min(first + STRIDE * (n + 32 * g), end - 1)];
+  const int4 where = ix.step[min(first + STRIDE * lane, end - 1)];
   const auto record = [&](int i) {
     const int k = min(i, count - 1);
+    const int l = FRESH ? fresh_lane() : lane;
     return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readlane(where.x, k), __builtin_amdgcn_readlane(where.y, k), 0,
-                                                      __builtin_amdgcn_readlane(where.w, k)), half, n, g, W, pixels);
+                                                      __builtin_amdgcn_readlane(where.w, k)), half, l & 31, l >> 5, W, pixels);
   };
   StepRecord next = record(0);
   for (int i = 0; i < count; ++i) {
@@ -397,7 +399,7 @@ __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int 
 }
 
 template <typename T>
-__global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_eu(2, 2))) void train_vjp16_kernel(
+__global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_eu(3, 3))) void train_vjp16_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int H, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
@@ -405,7 +407,7 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
     int32_t* __restrict__ nonfinite) {
   __shared__ Vjp16StepsLds<T> lds;
   Vjp16Shared<T>& s = lds.s;
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, g = lane >> 5;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   float kf[6];
 #pragma unroll
@@ -419,14 +421,18 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
     Vjp16StepSums sum;
     sum.clear();
     __syncthreads();
-    walk_halves<kVjp16Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
+    walk_halves<kVjp16Waves / 2, true>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
       vjp16_step_block<T>(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, kf, scale, lane);
     });
-    const int waves = min(2 * (run.end - run.begin), kVjp16Waves);
+    const int waves = min(2 * (run.end - run.begin), kVjp16Waves), slots = min(waves, kVjp16Slots);
     __syncthreads();
-    if (wave < waves) vjp16_park(sum, lds.sums[wave], lane);
+    if (wave < slots) vjp16_park<false>(sum, lds.sums[wave], lane);
+    if (waves > slots) {
+      __syncthreads();
+      if (wave >= slots && wave < waves) vjp16_park<true>(sum, lds.sums[wave - slots], lane);
+    }
     __syncthreads();
-    bad |= store_row_sums(lds.sums[0], kGradFloats, waves, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
+    bad |= store_row_sums(lds.sums[0], kGradFloats, slots, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
                           64 * kVjp16Waves);
     pos = run.end;
     __syncthreads();
@@ -445,7 +451,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     int32_t* __restrict__ nonfinite) {
   __shared__ Vjp32Lds s;
   static_assert(64 * kVjp32Waves == 256, "a thread for every entry of the table");
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), n = lane & 31, g = lane >> 5;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   const SplitUnits u;
   float factor[6];
@@ -465,7 +471,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     sum.clear();
     __syncthreads();
     int turn = wave / 4;
-    walk_halves<kVjp32Waves / 2>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, n, g, W, W * H, [&](const StepRecord& r) {
+    walk_halves<kVjp32Waves / 2, false>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
       // (a wavefront's blocks take turns at priority: 5.22 ms for the gradient call instead of 5.25)
       if (turn & 1) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(0);
@@ -541,7 +547,7 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
 }
 
 // Steps per chunk: as many as a wavefront has lanes for (twice that is no faster), fewer where that would leave fewer than four
-// chunks for each of the 512 workgroups that run at once, 16 at the least.  Gradient call in us, f32, a half, as much and
+// chunks for each of the 512 (f32) workgroups that run at once, 16 at the least.  Gradient call in us, f32, a half, as much and
 // twice as much of that rule at 51,600 steps: 483, 484, 518.
 inline int train_chunk_steps(int64_t S) {
   const int64_t per = S / 2048 / 8 * 8;

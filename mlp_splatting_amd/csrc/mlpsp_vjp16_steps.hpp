@@ -5,10 +5,12 @@
 // ds_read_b64_tr_b16 instead of being computed in both orientations or transposed by the matrix core: 16 large matrix
 // instructions and ~250 vector instructions a block instead of 30 and 350.
 //
-// Bound by the vector instructions (the 36 sines and cosines are a third of their time).  Four wavefronts to a workgroup and
-// two workgroups to a CU: while one changes primitives the other works, and two wavefronts to a SIMD hold everything in 186
-// registers.  Gradient call of 648,000 steps: 1.90 ms; one workgroup of eight 2.12, four of two 2.31, three of four 2.9 (168
-// registers: spills); with the block of mlpsp_vjp16.hpp, a wavefront to a chunk of 64 steps, 2.54.
+// Bound by the latency of a block's chain of products, conversions and LDS.  Four wavefronts to a workgroup and three workgroups
+// to a CU: while one changes primitives the others work.  Three wavefronts to a SIMD have 168 registers, which is what a block
+// needs if its parts stay one behind the other (sched_barrier) and neither the lane's number nor an address is kept from one
+// block to the next (fresh_lane); a word that spills is waited for behind the record requested ahead (2.04 ms with seven).
+// Gradient call of 648,000 steps: 1.84 ms; two workgroups of four 1.96, one of eight 2.12, four of two 2.31; with the block of
+// mlpsp_vjp16.hpp, a wavefront to a chunk of 64 steps, 2.54.
 #pragma once
 #include "mlpsp_device.hpp"
 #include "mlpsp_mfma16.hpp"
@@ -17,7 +19,7 @@
 
 namespace mlpsp {
 
-constexpr int kVjp16Waves = 4;
+constexpr int kVjp16Waves = 4, kVjp16Slots = 2;
 // As Vjp32Wave, one plane.
 struct Vjp16Wave {
   __attribute__((aligned(16))) unsigned enc[32][32];
@@ -39,10 +41,10 @@ struct Vjp16Shared {
 template <typename T>
 union Vjp16StepsLds {
   Vjp16Shared<T> s;
-  __attribute__((aligned(16))) float sums[kVjp16Waves][kGradFloats];    // in the end
+  __attribute__((aligned(16))) float sums[kVjp16Slots][kGradFloats];    // in the end, two wavefronts to a row
 };
 
-// The primitive's weights into LDS, by the first six wavefronts.
+// The primitive's weights into LDS, in eight pieces of 64 lanes.
 template <typename T>
 __device__ __forceinline__ void vjp16_load(const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
                                            const float* __restrict__ b2, const float* __restrict__ W3, size_t p, int wave, int lane,
@@ -82,12 +84,12 @@ __device__ __forceinline__ void vjp16_load(const float* __restrict__ W1, const f
 
 struct Vjp16StepSums {
   vf32x16 gw1[2], gw2;
-  f32x4 gw1e, gw3, gb1, gb2;
-  float gb3[4];
+  f32x4 gw1e, gw3, gb;       // gb: rows 0 and 1 = b2, b1
+  float gb3[2];              // outputs 2 g, 2 g + 1
   __device__ __forceinline__ void clear() {
     gw1[0] = gw1[1] = gw2 = splat16(0.f);
-    gw1e = gw3 = gb1 = gb2 = f32x4{0.f, 0.f, 0.f, 0.f};
-    gb3[0] = gb3[1] = gb3[2] = gb3[3] = 0.f;
+    gw1e = gw3 = gb = f32x4{0.f, 0.f, 0.f, 0.f};
+    gb3[0] = gb3[1] = 0.f;
   }
 };
 __device__ __forceinline__ Pack8 transpose_tile(const Pack8& v, Vjp16Wave& s, int n, int g) {
@@ -108,28 +110,28 @@ template <typename T>
 __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16StepSums& sum, Vjp16Wave& s, const float x[3],
                                                  float4 adjoint, uint32_t mask1, uint32_t mask2, const float (&kf)[6], float scale,
                                                  int lane) {
-  asm volatile("" : "+v"(lane));
+  lane = fresh_lane();
   const int n = lane & 31, g = lane >> 5;
   const vf32x16 zero = splat16(0.f);
-  const u32x2 ones = {Ops<T>::kOneWord, Ops<T>::kOneWord};
+  // (row n % 4 of the small products' first operand)
+  const unsigned row0 = (n & 3) == 0 ? Ops<T>::kOneWord : 0u, row1 = (n & 3) == 1 ? Ops<T>::kOneWord : 0u;
   // ---- adjoints of layer 2: record in the lane, unit hidden_unit(i, g) in register i.  (Group 1 multiplies by zero.)
   s.mask.put(g, n, g ? mask2 : mask1);
   u32x4 d3 = {0u, 0u, 0u, 0u};
   d3[0] = Ops<T>::pack2(adjoint.x * scale, adjoint.y * scale);
   d3[1] = Ops<T>::pack2(adjoint.z * scale, adjoint.w * scale);
-  if (g == 0) {
-    *reinterpret_cast<u32x2*>(s.d3[n]) = u32x2{d3[0], d3[1]};
-    sum.gb3[0] += Unpack<T>::lo(d3[0]);
-    sum.gb3[1] += Unpack<T>::hi(d3[0]);
-    sum.gb3[2] += Unpack<T>::lo(d3[1]);
-    sum.gb3[3] += Unpack<T>::hi(d3[1]);
-  }
+  if (g == 0) *reinterpret_cast<u32x2*>(s.d3[n]) = u32x2{d3[0], d3[1]};
+  const unsigned mine = g ? d3[1] : d3[0];
+  sum.gb3[0] += Unpack<T>::lo(mine);
+  sum.gb3[1] += Unpack<T>::hi(mine);
   const u32x2 w3r = w.w3r[lane];
   const Pack8 d2 = and_tile(pack_tile<T>(Ops<T>::mfma(u32x4{w3r[0], w3r[1], 0u, 0u}, d3, zero)), mask_tile_record_major(mask2, g));
   const Pack8 d2t = transpose_tile(d2, s, n, g);
+  __builtin_amdgcn_sched_barrier(0);
   // ---- adjoints of layer 1: unit in the lane
   const Pack8 d1 = and_tile(pack_tile<T>(mma2<T>(d2, Pack8{{w.w2t[0][lane], w.w2t[1][lane]}}, zero)),
                             mask_tile_unit_major(s.mask.half[0], n, g));
+  __builtin_amdgcn_sched_barrier(0);
   // ---- encoding and layer 1: record in the lane
   vf32x16 a1 = bias_rows(w.bias1, g);
 #pragma unroll
@@ -145,8 +147,10 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
     else *reinterpret_cast<u32x2*>(&s.enc_tail[n][2 * g]) = u32x2{e[0], e[1]};
     a1 = Ops<T>::mfma(w.w1[k][lane], e, a1);
   }
+  __builtin_amdgcn_sched_barrier(0);
   const Pack8 h1 = relu_tile(pack_tile<T>(a1));
   const Pack8 h1t = transpose_tile(h1, s, n, g);
+  __builtin_amdgcn_sched_barrier(0);
   // ---- layer 2: unit in the lane, straight into the W3 gradient
   const Pack8 h2 = relu_tile(pack_tile<T>(mma2<T>(h1, Pack8{{w.w2[0][lane], w.w2[1][lane]}}, splat16(w.bias2[n]))));
   const char* const d3_from = reinterpret_cast<const char*>(s.d3[4 * g + ((n >> 2) & 3)]);
@@ -154,10 +158,11 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
   for (int q = 0; q < 4; ++q) {
     const int k = q >> 1, d = 2 * (q & 1);
     sum.gw3 = Ops<T>::mfma4(read_transposed(d3_from + 8 * q * 8), u32x2{h2.s[k][d], h2.s[k][d + 1]}, sum.gw3);
-    sum.gb2 = Ops<T>::mfma4(ones, u32x2{d2t.s[k][d], d2t.s[k][d + 1]}, sum.gb2);
-    sum.gb1 = Ops<T>::mfma4(ones, u32x2{d1.s[k][d], d1.s[k][d + 1]}, sum.gb1);
+    sum.gb = Ops<T>::mfma4(u32x2{row0, row0}, u32x2{d2t.s[k][d], d2t.s[k][d + 1]}, sum.gb);
+    sum.gb = Ops<T>::mfma4(u32x2{row1, row1}, u32x2{d1.s[k][d], d1.s[k][d + 1]}, sum.gb);
   }
   sum.gw2 = mma2<T>(d2t, h1t, sum.gw2);
+  __builtin_amdgcn_sched_barrier(0);
   // ---- the W1 gradient (addresses as in vjp32_block)
   const int rec = 4 * g + ((n >> 2) & 3);
   const bool last = ((n >> 1) & 1) == (n >> 4);
@@ -173,33 +178,35 @@ __device__ __forceinline__ void vjp16_step_block(const Vjp16Shared<T>& w, Vjp16S
   }
 }
 
-// A wavefront's sums to a row of LDS, in the order of a packed row of gradients.
+// A wavefront's sums to a row of LDS, in the order of a packed row of gradients; ADD: onto what is there.
+template <bool ADD>
 __device__ __forceinline__ void vjp16_park(const Vjp16StepSums& sum, float* to, int lane) {
   asm volatile("" : "+v"(lane));
   const int n = lane & 31, g = lane >> 5;
   const GradRows out = packed_grad_rows(to);
+  const auto put = [](float& at, float v) { at = ADD ? at + v : v; };
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int r = 8 * (i >> 2) + 4 * g + (i & 3);
-    out.W1[r * 72 + enc_feature(n)] = sum.gw1[0][i];
-    out.W1[r * 72 + enc_feature(32 + n)] = sum.gw1[1][i];
-    out.W2[hidden_unit(r & 15, r >> 4) * 32 + tile_unit(n)] = sum.gw2[i];
+    put(out.W1[r * 72 + enc_feature(n)], sum.gw1[0][i]);
+    put(out.W1[r * 72 + enc_feature(32 + n)], sum.gw1[1][i]);
+    put(out.W2[hidden_unit(r & 15, r >> 4) * 32 + tile_unit(n)], sum.gw2[i]);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    out.W1[((lane & 8 ? 16 : 0) + 4 * (lane >> 4) + r) * 72 + enc_feature(64 + (lane & 7))] = sum.gw1e[r];
+    put(out.W1[((lane & 8 ? 16 : 0) + 4 * (lane >> 4) + r) * 72 + enc_feature(64 + (lane & 7))], sum.gw1e[r]);
     const float v = sum.gw3[r] + __shfl_xor(sum.gw3[r], 32);
-    if (g == 0) out.W3[r * 32 + n] = v;
+    if (g == 0) put(out.W3[r * 32 + n], v);
   }
-  const float gb1 = sum.gb1[0] + __shfl_xor(sum.gb1[0], 32), gb2 = sum.gb2[0] + __shfl_xor(sum.gb2[0], 32);
-  if (g == 0) out.b1[n] = gb1;
-  else out.b2[hidden_unit(n & 15, n >> 4)] = gb2;
+  const float gb2 = sum.gb[0] + __shfl_xor(sum.gb[0], 32), gb1 = sum.gb[1] + __shfl_xor(sum.gb[1], 32);
+  if (g == 0) put(out.b1[n], gb1);
+  else put(out.b2[hidden_unit(n & 15, n >> 4)], gb2);
 #pragma unroll
-  for (int o = 0; o < 4; ++o) {
+  for (int o = 0; o < 2; ++o) {
     float v = sum.gb3[o];
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-    if (lane == o) out.b3[o] = v;
+    for (int m = 16; m > 0; m >>= 1) v += __shfl_xor(v, m);
+    if (n == o) put(out.b3[2 * g + o], v);
   }
 }
 

@@ -39,6 +39,12 @@ namespace mlpsp {
 typedef short i16x4v __attribute__((ext_vector_type(4)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 
+// The lane's number, made anew where it is asked for: no register keeps it in between.
+__device__ __forceinline__ int fresh_lane() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
 // Pairs of f32 as packed bf16: h + m + l = the pair.
 struct Split2 {
   unsigned h, m, l;
