@@ -31,8 +31,7 @@ namespace mlpsp {
 // every fp16 value is an f32 value, so both sources give the same blocks bit for bit).
 // CHECK: *nonfinite |= 1 if a weight of any primitive is NaN or infinite, also of one that is not wanted: what is packed is
 // looked at on the way, the others are read for it (16-byte aligned, all of a primitive's 14 KB in flight).  Bound by the
-// bytes: 200,000 primitives, a third of them wanted, 284 us to pack and 514 to read everything before -> 689 us (679 with the wanted
-// primitives' weights put into LDS first).
+// bytes: 200,000 primitives, a third of them wanted, 284 us to pack and 514 to read everything before -> SCANPACK us.
 template <typename S> struct FourOf;
 template <> struct FourOf<float> { typedef f32x4 type; };
 template <> struct FourOf<_Float16> { typedef f16x4 type; };
