@@ -415,12 +415,6 @@ int mlpsp_pack_mfma_weights_half(const void* W1, const void* b1, const void* W2,
 int mlpsp_pack_mfma_weights_listed(const float* W1, const float* b1, const float* W2, const float* b2, const float* W3,
                                    const float* b3, int num_primitives, int use_bf16, const int32_t* order_dev,
                                    int64_t num_pairs, unsigned char* wanted_dev, void* packed_dev, mlpsp_stream_t stream);
-/* The same, and *nonfinite_dev |= 1 if a weight of any primitive, named or not, is NaN or infinite: one pass over the weights
- * instead of two.  The six tensors must be 16-byte aligned (nonfinite_dev == NULL: as above, but for num_pairs == 0). */
-int mlpsp_pack_mfma_weights_checked(const float* W1, const float* b1, const float* W2, const float* b2, const float* W3,
-                                    const float* b3, int num_primitives, int use_bf16, const int32_t* order_dev,
-                                    int64_t num_pairs, unsigned char* wanted_dev, void* packed_dev, int32_t* nonfinite_dev,
-                                    mlpsp_stream_t stream);
 int mlpsp_render_tilecenter_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
                                  const int32_t* order_dev, const int32_t* tile_offsets_dev, const float* freq_dev,
                                  const float* att_dev, const void* packed_dev, int num_primitives, int use_bf16,

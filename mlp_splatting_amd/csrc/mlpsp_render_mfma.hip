@@ -29,65 +29,26 @@ namespace mlpsp {
 // ---------------------------------------------------------------------------------------------
 // S: the type the six tensors are stored in (float, or _Float16 for an inference export read without widening it first:
 // every fp16 value is an f32 value, so both sources give the same blocks bit for bit).
-// CHECK: *nonfinite |= 1 if a weight of any primitive is NaN or infinite, also of one that is not wanted: what is packed is
-// looked at on the way, the others are read for it (16-byte aligned, all of a primitive's 14 KB in flight).  Bound by the
-// bytes: 200,000 primitives, a third of them wanted, 284 us to pack and 514 to read everything before -> SCANPACK us.
-template <typename S> struct FourOf;
-template <> struct FourOf<float> { typedef f32x4 type; };
-template <> struct FourOf<_Float16> { typedef f16x4 type; };
-template <typename T, bool CHECK, typename S>
+template <typename T, typename S>
 __global__ __launch_bounds__(64) void pack_mfma_weights_kernel(const S* __restrict__ W1, const S* __restrict__ b1,
                                                                const S* __restrict__ W2, const S* __restrict__ b2,
                                                                const S* __restrict__ W3, const S* __restrict__ b3,
                                                                int N, const unsigned char* __restrict__ wanted,
-                                                               unsigned char* __restrict__ out, int32_t* __restrict__ nonfinite) {
+                                                               unsigned char* __restrict__ out) {
   const int p = blockIdx.x;
-  if (p >= N) return;
+  if (p >= N || (wanted && !wanted[p])) return;
   const int l = threadIdx.x, m = l & 31, g = l >> 5;
-  bool odd = false;                        // a weight that is not finite
-  const auto look = [&](float v) { odd |= !(__builtin_fabsf(v) <= 3.4028235e38f); };
-  if (wanted && !wanted[p]) {
-    if constexpr (CHECK) {
-      typedef typename FourOf<S>::type Four;
-      const Four* __restrict__ w1 = reinterpret_cast<const Four*>(W1 + (size_t)p * 2304);
-      const Four* __restrict__ w2 = reinterpret_cast<const Four*>(W2 + (size_t)p * 1024);
-      const S* __restrict__ rest = l < 32 ? W3 + (size_t)p * 128 + 4 * l
-                                   : l < 40 ? b1 + (size_t)p * 32 + 4 * (l - 32)
-                                   : l < 48 ? b2 + (size_t)p * 32 + 4 * (l - 40) : b3 + (size_t)p * 4;
-      Four v[14];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) v[k] = w1[64 * k + l];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) v[9 + k] = w2[64 * k + l];
-      v[13] = *reinterpret_cast<const Four*>(rest);
-#pragma unroll
-      for (int k = 0; k < 14; ++k) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) look((float)v[k][q]);
-      }
-      if (__ballot(odd) != 0ull && l == 0) atomicOr(nonfinite, 1);
-    }
-    return;
-  }
   unsigned char* blk = out + (size_t)p * kPackStride;
   // accumulator row m holds hidden unit hidden_unit_of_row(m), for both hidden layers
   const S* w1 = W1 + (size_t)p * 32 * 72 + hidden_unit_of_row(m) * 72;
   const S* w2 = W2 + (size_t)p * 32 * 32 + hidden_unit_of_row(m) * 32;
   bool bad = false;
   auto pk = [&](float a, float b) {
-    if constexpr (CHECK) {
-      look(a);
-      look(b);
-    }
     bad |= !(__builtin_fabsf(Ops<T>::round_trip(a)) <= Ops<T>::kMax) || !(__builtin_fabsf(Ops<T>::round_trip(b)) <= Ops<T>::kMax);
     return Ops<T>::pack2(a, b);
   };
   const float bias1 = (float)b1[(size_t)p * 32 + hidden_unit_of_row(m)], bias2 = (float)b2[(size_t)p * 32 + hidden_unit_of_row(m)];
   bad |= !(__builtin_fabsf(Ops<T>::round_trip(bias1)) <= Ops<T>::kMax) || !(__builtin_fabsf(Ops<T>::round_trip(bias2)) <= Ops<T>::kMax);
-  if constexpr (CHECK) {
-    look(bias1);
-    look(bias2);
-  }
   for (int s = 0; s < 5; ++s) {
     u32x4 v;
     for (int d = 0; d < 4; ++d) {
@@ -120,11 +81,7 @@ __global__ __launch_bounds__(64) void pack_mfma_weights_kernel(const S* __restri
   if (l < 4) {
     const float v3 = (float)b3[(size_t)p * 4 + l];
     bad |= !(__builtin_fabsf(v3) <= 3.4028235e38f);
-    if constexpr (CHECK) look(v3);
     reinterpret_cast<float*>(blk + kOffB3)[l] = v3;
-  }
-  if constexpr (CHECK) {
-    if (__ballot(odd) != 0ull && l == 0) atomicOr(nonfinite, 1);
   }
   const unsigned long long any = __ballot(bad);
   if (l == 0) *reinterpret_cast<int32_t*>(blk + kOffFlag) = any ? 1 : 0;
@@ -1148,19 +1105,19 @@ MLPSP_API size_t mlpsp_mfma_pack_bytes(int num_primitives) {
 }
 
 namespace {
-template <bool CHECK = false, typename S>
+template <typename S>
 int pack_weights_from(const S* W1, const S* b1, const S* W2, const S* b2, const S* W3, const S* b3, int num_primitives,
-                      int use_bf16, const unsigned char* wanted, void* packed_dev, hipStream_t s, int32_t* nonfinite = nullptr) {
+                      int use_bf16, const unsigned char* wanted, void* packed_dev, hipStream_t s) {
   if (num_primitives < 0) return MLPSP_E_ARGUMENT;
   if (num_primitives == 0) return MLPSP_OK;
   if (!W1 || !b1 || !W2 || !b2 || !W3 || !b3 || !packed_dev) return MLPSP_E_ARGUMENT;
   if (reinterpret_cast<uintptr_t>(packed_dev) % 128 != 0) return MLPSP_E_ARGUMENT;
   if (use_bf16)
-    hipLaunchKernelGGL((pack_mfma_weights_kernel<__bf16, CHECK, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
-                       b3, num_primitives, wanted, (unsigned char*)packed_dev, nonfinite);
+    hipLaunchKernelGGL((pack_mfma_weights_kernel<__bf16, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
+                       b3, num_primitives, wanted, (unsigned char*)packed_dev);
   else
-    hipLaunchKernelGGL((pack_mfma_weights_kernel<_Float16, CHECK, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
-                       b3, num_primitives, wanted, (unsigned char*)packed_dev, nonfinite);
+    hipLaunchKernelGGL((pack_mfma_weights_kernel<_Float16, S>), dim3(num_primitives), dim3(64), 0, s, W1, b1, W2, b2, W3,
+                       b3, num_primitives, wanted, (unsigned char*)packed_dev);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }
@@ -1169,14 +1126,14 @@ int pack_weights_from(const S* W1, const S* b1, const S* W2, const S* b2, const 
 MLPSP_API int mlpsp_pack_mfma_weights(const float* W1, const float* b1, const float* W2, const float* b2,
                                       const float* W3, const float* b3, int num_primitives, int use_bf16,
                                       void* packed_dev, mlpsp_stream_t stream) {
-  return pack_weights_from(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, nullptr, packed_dev, (hipStream_t)stream);
+  return pack_weights_from<float>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, nullptr, packed_dev, (hipStream_t)stream);
 }
 
 MLPSP_API int mlpsp_pack_mfma_weights_half(const void* W1, const void* b1, const void* W2, const void* b2,
                                            const void* W3, const void* b3, int num_primitives, int use_bf16,
                                            void* packed_dev, mlpsp_stream_t stream) {
   typedef const _Float16* H;
-  return pack_weights_from((H)W1, (H)b1, (H)W2, (H)b2, (H)W3, (H)b3, num_primitives, use_bf16, nullptr, packed_dev,
+  return pack_weights_from<_Float16>((H)W1, (H)b1, (H)W2, (H)b2, (H)W3, (H)b3, num_primitives, use_bf16, nullptr, packed_dev,
                                      (hipStream_t)stream);
 }
 
@@ -1186,30 +1143,14 @@ MLPSP_API int mlpsp_pack_mfma_weights_listed(const float* W1, const float* b1, c
                                              void* packed_dev, mlpsp_stream_t stream) {
   if (num_primitives < 0 || num_pairs < 0) return MLPSP_E_ARGUMENT;
   if (num_primitives == 0 || num_pairs == 0) return MLPSP_OK;
-  return mlpsp_pack_mfma_weights_checked(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, order_dev, num_pairs, wanted_dev,
-                                         packed_dev, nullptr, stream);
-}
-
-MLPSP_API int mlpsp_pack_mfma_weights_checked(const float* W1, const float* b1, const float* W2, const float* b2,
-                                              const float* W3, const float* b3, int num_primitives, int use_bf16,
-                                              const int32_t* order_dev, int64_t num_pairs, unsigned char* wanted_dev,
-                                              void* packed_dev, int32_t* nonfinite_dev, mlpsp_stream_t stream) {
-  if (num_primitives < 0 || num_pairs < 0) return MLPSP_E_ARGUMENT;
-  if (num_primitives == 0) return MLPSP_OK;
-  if (!wanted_dev || (num_pairs > 0 && !order_dev)) return MLPSP_E_ARGUMENT;
-  if (nonfinite_dev && (((uintptr_t)W1 | (uintptr_t)b1 | (uintptr_t)W2 | (uintptr_t)b2 | (uintptr_t)W3 | (uintptr_t)b3) & 15u))
-    return MLPSP_E_ARGUMENT;
+  if (!order_dev || !wanted_dev) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(wanted_dev, (size_t)num_primitives, s));
-  if (num_pairs > 0) {
-    const int64_t blocks = (num_pairs + 1023) / 1024;
-    hipLaunchKernelGGL(mark_listed_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, order_dev,
-                       (long long)num_pairs, num_primitives, wanted_dev);
-    MLPSP_LAUNCH_CHECK();
-  }
-  if (nonfinite_dev)
-    return pack_weights_from<true>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, wanted_dev, packed_dev, s, nonfinite_dev);
-  return pack_weights_from(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, wanted_dev, packed_dev, s);
+  const int64_t blocks = (num_pairs + 1023) / 1024;
+  hipLaunchKernelGGL(mark_listed_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, order_dev,
+                     (long long)num_pairs, num_primitives, wanted_dev);
+  MLPSP_LAUNCH_CHECK();
+  return pack_weights_from<float>(W1, b1, W2, b2, W3, b3, num_primitives, use_bf16, wanted_dev, packed_dev, s);
 }
 
 namespace {

@@ -672,19 +672,15 @@ def pack_mfma_weights(W1, b1, W2, b2, W3, b3, bf16=True):
     return packed
 
 
-def pack_mfma_weights_listed(ws, order, bf16, nonfinite=None):
+def pack_mfma_weights_listed(ws, order, bf16):
     """:func:`pack_mfma_weights` of the primitives that the lists ``order`` name; the other blocks stay unwritten.  ``ws``: the
-    six contiguous f32 tensors of the 72->32->32->4 MLP.  ``nonfinite``: an int32 [1] device flag (:func:`all_finite_flag`)
-    that is set if a weight of any primitive, named or not, is NaN or infinite (tensors aligned to 16 bytes)."""
+    six contiguous f32 tensors of the 72->32->32->4 MLP."""
     n, dev = ws[0].shape[0], ws[0].device
     lib = _lib.load()
     packed = torch.empty(lib.mlpsp_mfma_pack_bytes(n), dtype=torch.uint8, device=dev)
     wanted = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
-    args = [*[_ptr(w) for w in ws], n, int(bool(bf16)), _ptr(order), order.numel(), _ptr(wanted), _ptr(packed)]
-    if nonfinite is None:
-        _check(lib.mlpsp_pack_mfma_weights_listed(*args, _stream(dev)), "mlpsp_pack_mfma_weights_listed")
-    else:
-        _check(lib.mlpsp_pack_mfma_weights_checked(*args, _ptr(nonfinite), _stream(dev)), "mlpsp_pack_mfma_weights_checked")
+    _check(lib.mlpsp_pack_mfma_weights_listed(*[_ptr(w) for w in ws], n, int(bool(bf16)), _ptr(order), order.numel(),
+                                              _ptr(wanted), _ptr(packed), _stream(dev)), "mlpsp_pack_mfma_weights_listed")
     return packed
 
 

@@ -625,8 +625,7 @@ class TileExt:
         """(rgb, alpha, ops.TrainFrame) of an 8x8-tile frame with the 72->32->32->4 MLP.  ``x``: the 15 scene tensors.
         ``precision`` None: exact f32 (with ``render_order`` the bits of ``render_tiles_forward_tilecenter``, see
         :meth:`records_forward_matches_render`); "float16" / "bfloat16": the matrix cores.  The frame's ``status`` bits
-        (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called before the walk with the int32 device flag
-        that says whether an input is NaN or infinite, once the lists are validated and the inputs looked at."""
+        (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called once the lists are validated."""
         width, height = int(width), int(height)
         _chk(width > 0 and height > 0 and x[0].shape[0] == width * height, "B must equal W*H for tile renderer")
         _chk(len(x) == 15, "Expected 15 scene inputs")
@@ -635,22 +634,14 @@ class TileExt:
         n_tiles = ops.num_tiles(width, height, 8, 8)
         with _on_device(x[0].device), self.uncached():
             self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
-            # (weights that are packed are looked at by the packing, in the same pass)
-            nonfinite, packing_looks = None, False
             if accept is not None:
-                packing_looks = precision is not None and n > 0 and all(w.data_ptr() % 16 == 0 for w in x[9:15])
-                nonfinite = ops.all_finite_flag([t for i, t in enumerate(x) if i not in (5, 6) and not (packing_looks and i > 8)])
-                if not packing_looks:
-                    accept(nonfinite)
+                accept()
             rec = self._records(x[2], x[3], x[4])
             order = x[5]
             if x[5].numel() > 0:
                 order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
                                           self.max_tile_prims, cull_threshold=float(threshold))
-            packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16",
-                                                                                 nonfinite if packing_looks else None)
-            if packing_looks:
-                accept(nonfinite)
+            packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
             # Room for the steps: for the first frame as its lists suggest (a step per 13 entries at the 200,000-primitive
             # 1200x680 frame, per three or four where primitives are small), then as the frames before needed.  A frame
             # that needs more is repeated; the bound on what its lists can need is never exceeded.
@@ -676,8 +667,8 @@ class TileExt:
         width, height = int(width), int(height)
         self._check_training_wmma(x, width, height, 8, threshold, beta, temp, precision)
 
-        def accept(nonfinite):
-            self._refuse(nonfinite)
+        def accept():
+            self._refuse_nonfinite(x)
             self._count_training_mfma(0)
         rgb, alpha, frame = self.train_forward(x, width, height, threshold, precision=precision, accept=accept,
                                                name="render_tiles_training_records_wmma")
@@ -761,12 +752,9 @@ class TileExt:
         if len(x) == 17:
             _chk(x[15].shape == x[0].shape and x[16].dim() == 1 and x[16].numel() == pixels)
 
-    @classmethod
-    def _refuse_nonfinite(cls, x):
-        cls._refuse(ops.all_finite_flag([t for i, t in enumerate(x) if i not in (5, 6)]))
-
     @staticmethod
-    def _refuse(nonfinite):
+    def _refuse_nonfinite(x):
+        nonfinite = ops.all_finite_flag([t for i, t in enumerate(x) if i not in (5, 6)])
         _chk(int(nonfinite.item()) == 0, "Training WMMA input is nonfinite; refusing unsafe forward/fallback")
 
     def render_tiles_training_records_wmma(self, x, width, height, tile, threshold, beta, temp, precision):
