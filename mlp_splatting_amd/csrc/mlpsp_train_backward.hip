@@ -9,7 +9,7 @@
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.14 (sort 1.7, gathers 2.85), geometry 0.18 (1.3), weight gradients 4.7 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
+// 0.14 (sort 1.7, gathers 2.85), geometry 0.18 (1.3), weight gradients 4.6 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
