@@ -547,7 +547,7 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
 }
 
 // Steps per chunk: as many as a wavefront has lanes for (twice that is no faster), fewer where that would leave fewer than four
-// chunks for each of the 512 (f32) workgroups that run at once, 16 at the least.  Gradient call in us, f32, a half, as much and
+// chunks for each of the 512 workgroups that run at once (f32; 768 in 16 bits), 16 at the least.  Gradient call in us, f32, a half, as much and
 // twice as much of that rule at 51,600 steps: 483, 484, 518.
 inline int train_chunk_steps(int64_t S) {
   const int64_t per = S / 2048 / 8 * 8;
