@@ -7,6 +7,8 @@
 // `render_order`, the record kernels' rounding of layer 2 without).  Bound by the MLP; the steps add 3.3 KB of contiguous
 // stores per hit step.  200,000 primitives, 1200x680, f32: 3.9 ms, against 4.0 + 6.0 of the record forward's two walks;
 // 20,000 primitives, 320x240: 1.24 ms with a wavefront per tile, 0.87 with teams (see train_plan).
+#include <type_traits>
+
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mfma16.hpp"
@@ -39,10 +41,14 @@ struct TrainScene {
   float thr;
   int max_hits;
 };
+// In f32 the walk parks 16 entries at a time: four workgroups' LDS is then a CU's (40,960 bytes each; three with 64), and at 128
+// registers, with fifteen spills outside the products, four wavefronts run on a SIMD.  Forward of the 20,000-primitive 320x240
+// frame, all teams, 776 -> 676 us; of 200,000 at 1200x680 4.01 as before.  (The f32 renders gain or lose: frame of 200,000 0.5 %
+// faster, feature frame of 30,000 with its hit records 4 % slower.)
 template <typename T>
 struct TrainItemLds {
   typename TrainDir<T>::type dir;
-  WalkLds walk;
+  WalkLdsOf<std::is_same_v<T, float> ? 16 : 64> walk;
 };
 template <typename T, int TEAM>
 struct TrainTeamLds {
@@ -267,7 +273,7 @@ __device__ __forceinline__ void train_forward_body(const TrainScene& c, const St
       const float *__restrict__ att
 #define MLPSP_TRAIN_TAIL int N, int W, int H, int ntx, int nty, float thr, int max_hits, StepPool sp, TrainOut out, int body
 template <bool REC>
-__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(3, 3))) void train_forward_f32_kernel(
+__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_f32_kernel(
     MLPSP_TRAIN_PARAMS, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, const float* __restrict__ b3, MLPSP_TRAIN_TAIL) {
   const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, nullptr, N, W, H, ntx, nty, thr, max_hits};
