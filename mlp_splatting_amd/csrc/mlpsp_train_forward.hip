@@ -43,8 +43,9 @@ struct TrainScene {
 };
 // In f32 the walk parks 16 entries at a time: four workgroups' LDS is then a CU's (40,960 bytes each; three with 64), and at 128
 // registers, with fifteen spills outside the products, four wavefronts run on a SIMD.  Forward of the 20,000-primitive 320x240
-// frame, all teams, 776 -> 676 us; of 200,000 at 1200x680 4.01 as before.  (The f32 renders gain or lose: frame of 200,000 0.5 %
-// faster, feature frame of 30,000 with its hit records 4 % slower.)
+// frame, all teams: 776 -> 676 us for one camera, 582 -> 573 in the mean of five as traced; 200,000 at 1200x680 4.01 ms as before:
+// there the matrix and vector pipes, which exclude each other, are taken.  (The f32 renders: frame of 200,000 0.5 % faster,
+// feature frame of 30,000 with its hit records up to 4 % slower.)
 template <typename T>
 struct TrainItemLds {
   typename TrainDir<T>::type dir;
