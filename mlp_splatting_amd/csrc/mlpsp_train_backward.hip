@@ -450,7 +450,6 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
     int32_t* __restrict__ nonfinite) {
   __shared__ Vjp32Lds s;
-  static_assert(64 * kVjp32Waves == 256, "a thread for every entry of the table");
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   const SplitUnits u;
@@ -462,7 +461,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
   for (int f = 0; f < 6; ++f) limit = fmaxf(limit, __builtin_fabsf(factor[f]));
   limit = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(limit)));
   if (t < 4) s.zero[t] = 0u;
-  s.circle[t] = f32x2v{kCircle.at[t][0], kCircle.at[t][1]};
+  for (int k = t; k < kCircleEntries; k += 64 * kVjp32Waves) s.circle[k] = f32x2v{kCircle.at[k][0], kCircle.at[k][1]};
   bool bad = false;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);

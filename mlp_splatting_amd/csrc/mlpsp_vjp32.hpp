@@ -115,8 +115,9 @@ __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4&
   return Ops<__bf16>::mfma(ha, hb, acc);
 }
 
-// A workgroup of four wavefronts, two workgroups to a CU: 23 KB of operands and 2 KB of turns that its wavefronts read, 14 KB of each one's own.
+// A workgroup of four wavefronts, two workgroups to a CU: 22 KB of operands and 2.5 KB of turns that its wavefronts read, 14 KB of each one's own.
 constexpr int kVjp32Waves = 4;
+constexpr int kCircleEntries = 320;       // of vjp32_sincos' table
 union Vjp32Wave {
   struct {
     // Columns of the encoding: pair t of group g (sin, cos) is word 16 g + t of a record's 32 for t < 16, and word
@@ -133,12 +134,13 @@ union Vjp32Wave {
 };
 struct Vjp32Lds {
   u32x4 w1[3][4][64];            // W1[n][..]: slots 2 d, 2 d + 1 of K-step s = pair 4 s + d
-  u32x4 w1_tail[4][64];          // pairs 16, 17 of two planes
+  u32x4 w1_tail[2][64];          // pairs 16, 17 of two planes
+  u32x2 w1_tail1[2][64];         // ... of one, against zeros for the other
   unsigned w2[3][32][16];        // W2[n][..]: 16 bytes 2 s + g (tile_place) = unit(8 s + j, g)
   float w3[2][64];               // W3[2 j + g][n]
   float bias1[32], bias2[32];
   __attribute__((aligned(16))) unsigned zero[4];
-  f32x2v circle[256];
+  f32x2v circle[kCircleEntries];
   Vjp32Wave wave[kVjp32Waves];
 };
 static_assert(2 * sizeof(Vjp32Lds) <= 163840, "two workgroups per CU");
@@ -210,10 +212,10 @@ __device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const f
     for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(&s.w2[k][n][tile_place(2 * wave + g, n)]) = v[k];
   } else if (wave == 2) {
     const Split2 x = pair(16), y = pair(17);
-    s.w1_tail[0][lane] = u32x4{x.h, y.h, 0u, 0u};        // h h: against (h, m)
-    s.w1_tail[1][lane] = u32x4{x.l, y.l, 0u, 0u};        // l h: against (h, m)
-    s.w1_tail[2][lane] = u32x4{x.m, y.m, x.h, y.h};      // m m, h l: against (m, l)
-    s.w1_tail[3][lane] = u32x4{x.h, y.h, x.m, y.m};      // h m, m h: against (m, h)
+    s.w1_tail1[0][lane] = u32x2{x.h, y.h};               // h h: against (h, m)
+    s.w1_tail1[1][lane] = u32x2{x.l, y.l};               // l h: against (h, m)
+    s.w1_tail[0][lane] = u32x4{x.m, y.m, x.h, y.h};      // m m, h l: against (m, l)
+    s.w1_tail[1][lane] = u32x4{x.h, y.h, x.m, y.m};      // h m, m h: against (m, h)
   } else {
     (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
 #pragma unroll
@@ -231,22 +233,25 @@ struct Vjp32Sums {
   }
 };
 
-// The six (sin, cos) pairs of one input component, from a table of 256 turns k 2 pi / 256 and a rotation by the rest, |r| <=
-// pi / 256: sin r = r - r^3 / 6 and cos r = 1 - r^2 / 2 to 2e-12 and 1e-9.  What a pair is off by is the rounding of the two
-// table values and of the two products, 1e-7 as from a polynomial in the reduced phase, in 15 instructions and an LDS read
-// instead of 27 instructions (gradient call 5.11 -> 4.96 and 0.480 -> 0.467 ms).  `limit`: the largest factor; where the component's largest phase is out of range, all of its values are NaN.
+// The six (sin, cos) pairs of one input component, from the sine and cosine of the nearest of 256 turns k 2 pi / 256 and a
+// rotation by the rest, |r| <= pi / 256: sin r = r - r^3 / 6 and cos r - 1 = -r^2 / 2 to 2e-12 and 1e-9.  The table holds the
+// sine of 320 turns -- a cosine is the sine of the turn 64 further on -- as its f32 value and what that leaves over, which is
+// added to the rotation's terms before the value itself: what a pair is off by is the rounding of that last sum.  Against
+// float64 over phases up to 30: 1.5e-8 rms, 3.2e-8 at the most; det_sincos 2.1e-8 and 9.2e-8; a table without remainders
+// 2.5e-8 and 8.9e-8.  17 instructions a pair and one LDS read of two entries, det_sincos 27.  `limit`: the largest factor;
+// where the component's largest phase is out of range, all of its values are NaN.
 struct CircleTable {
-  float at[256][2];
+  float at[kCircleEntries][2];
   constexpr CircleTable() : at{} {
-    for (int k = 0; k < 256; ++k) {
+    for (int k = 0; k < kCircleEntries; ++k) {
       const double x = (k < 128 ? k : k - 256) * (6.283185307179586476925 / 256.0);
-      double sine = 0.0, cosine = 0.0, term = 1.0;      // x^i / i!
-      for (int i = 0; i < 40; ++i) {
-        (i & 1 ? sine : cosine) += i & 2 ? -term : term;
-        term *= x / (i + 1);
+      double sine = 0.0, term = x;                       // x^i / i!
+      for (int i = 1; i < 40; i += 2) {
+        sine += i & 2 ? -term : term;
+        term *= x * x / ((i + 1) * (i + 2));
       }
       at[k][0] = (float)sine;
-      at[k][1] = (float)cosine;
+      at[k][1] = (float)(sine - (double)at[k][0]);
     }
   }
 };
@@ -261,10 +266,11 @@ __device__ __forceinline__ void vjp32_sincos(const f32x2v* circle, float x, cons
     const float kf = shifted - 12582912.0f;
     float r = fmaf(kf, -0.0245436933f, phase);
     r = fmaf(kf, 6.82990470e-10f, r);
-    const f32x2v at = *reinterpret_cast<const f32x2v*>(reinterpret_cast<const char*>(circle) + ((float_to_bits(shifted) << 3) & 0x7f8u));
+    const f32x2v* const at = reinterpret_cast<const f32x2v*>(reinterpret_cast<const char*>(circle) + ((float_to_bits(shifted) << 3) & 0x7f8u));
+    const f32x2v sv = at[0], cv = at[64];
     const float z = r * r, less = -0.5f * z, sine = fmaf(r * z, -0.166666667f, r);
-    s_out[f] = fmaf(at[1], sine, fmaf(at[0], less, at[0]));
-    c_out[f] = fmaf(-at[0], sine, fmaf(at[1], less, at[1]));
+    s_out[f] = sv[0] + fmaf(cv[0], sine, fmaf(sv[0], less, sv[1]));
+    c_out[f] = cv[0] + fmaf(-sv[0], sine, fmaf(cv[0], less, cv[1]));
   }
 }
 // v where bit `bit` of word is set, else +0
@@ -401,10 +407,11 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   mfma_split(read_step(w.w1, 3, lane), e3, a1);
   {
     const u32x4 hm = {e.p[0][0], e.p[0][1], e.p[1][0], e.p[1][1]};
-    a1.big = Ops<__bf16>::mfma(w.w1_tail[0][lane], hm, a1.big);
-    a1.small = Ops<__bf16>::mfma(w.w1_tail[1][lane], hm, a1.small);
-    a1.small = Ops<__bf16>::mfma(w.w1_tail[2][lane], u32x4{e.p[1][0], e.p[1][1], e.p[2][0], e.p[2][1]}, a1.small);
-    a1.small = Ops<__bf16>::mfma(w.w1_tail[3][lane], u32x4{e.p[1][0], e.p[1][1], e.p[0][0], e.p[0][1]}, a1.small);
+    const u32x2 wh = w.w1_tail1[0][lane], wl = w.w1_tail1[1][lane];
+    a1.big = Ops<__bf16>::mfma(u32x4{wh[0], wh[1], 0u, 0u}, hm, a1.big);
+    a1.small = Ops<__bf16>::mfma(u32x4{wl[0], wl[1], 0u, 0u}, hm, a1.small);
+    a1.small = Ops<__bf16>::mfma(w.w1_tail[0][lane], u32x4{e.p[1][0], e.p[1][1], e.p[2][0], e.p[2][1]}, a1.small);
+    a1.small = Ops<__bf16>::mfma(w.w1_tail[1][lane], u32x4{e.p[1][0], e.p[1][1], e.p[0][0], e.p[0][1]}, a1.small);
   }
   {
     vf32x16 v = tsum;
