@@ -453,13 +453,12 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   const SplitUnits u;
-  float factor[6];
+  PhaseFactors factors;
 #pragma unroll
-  for (int f = 0; f < 6; ++f) factor[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(freq[f] * att[f])));
-  float limit = 0.f;
-#pragma unroll
-  for (int f = 0; f < 6; ++f) limit = fmaxf(limit, __builtin_fabsf(factor[f]));
-  limit = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(limit)));
+  for (int f = 0; f < 6; ++f) {
+    factors.freq[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(freq[f])));
+    factors.att[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(att[f])));
+  }
   if (t < 4) s.zero[t] = 0u;
   for (int k = t; k < kCircleEntries; k += 64 * kVjp32Waves) s.circle[k] = f32x2v{kCircle.at[k][0], kCircle.at[k][1]};
   bool bad = false;
@@ -475,7 +474,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
       if (turn & 1) __builtin_amdgcn_s_setprio(1);
       else __builtin_amdgcn_s_setprio(0);
       ++turn;
-      vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factor, limit, scale, lane, u);
+      vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, scale, lane, u);
     });
     const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
     if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);

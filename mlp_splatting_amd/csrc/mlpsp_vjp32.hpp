@@ -238,8 +238,15 @@ struct Vjp32Sums {
 // sine of 320 turns -- a cosine is the sine of the turn 64 further on -- as its f32 value and what that leaves over, which is
 // added to the rotation's terms before the value itself: what a pair is off by is the rounding of that last sum.  Against
 // float64 over phases up to 30: 1.5e-8 rms, 3.2e-8 at the most; det_sincos 2.1e-8 and 9.2e-8; a table without remainders
-// 2.5e-8 and 8.9e-8.  17 instructions a pair and one LDS read of two entries, det_sincos 27.  `limit`: the largest factor;
-// where the component's largest phase is out of range, all of its values are NaN.
+// 2.5e-8 and 8.9e-8.  20 instructions a pair and one LDS read of two entries, det_sincos 27.
+//
+// The phase is the forward's, (x freq) att with both roundings: with the factors multiplied first, the sine of a phase of 100
+// is that of another number by 1e-5, and the gradient is off by 2.6e-6 of its norm.  Out of range (|phase| > 65536: a pair of
+// NaN, as in det_sincos) without a comparison: the phase times the largest float / 65536 is infinite exactly there, and zero
+// times that is added to the rest.
+struct PhaseFactors {
+  float freq[6], att[6];
+};
 struct CircleTable {
   float at[kCircleEntries][2];
   constexpr CircleTable() : at{} {
@@ -256,16 +263,15 @@ struct CircleTable {
   }
 };
 static __device__ const CircleTable kCircle = CircleTable();
-__device__ __forceinline__ void vjp32_sincos(const f32x2v* circle, float x, const float (&factor)[6], float limit, float s_out[6],
-                                             float c_out[6]) {
-  x = __builtin_fabsf(x) * limit <= 65536.0f ? x : __builtin_nanf("");
+__device__ __forceinline__ void vjp32_sincos(const f32x2v* circle, float x, const PhaseFactors& k, float s_out[6], float c_out[6]) {
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
-    const float phase = x * factor[f];
+    const float phase = (x * k.freq[f]) * k.att[f];
     const float shifted = fmaf(phase, 40.7436654f, 12582912.0f);         // the nearest turn, in the low bits
     const float kf = shifted - 12582912.0f;
     float r = fmaf(kf, -0.0245436933f, phase);
     r = fmaf(kf, 6.82990470e-10f, r);
+    r = fmaf(phase * 0x1.fffffep111f, 0.f, r);
     const f32x2v* const at = reinterpret_cast<const f32x2v*>(reinterpret_cast<const char*>(circle) + ((float_to_bits(shifted) << 3) & 0x7f8u));
     const f32x2v sv = at[0], cv = at[64];
     const float z = r * r, less = -0.5f * z, sine = fmaf(r * z, -0.166666667f, r);
@@ -328,10 +334,10 @@ __device__ __forceinline__ void mfma_split(const SplitOperand& a, const SplitOpe
 }
 // Six pairs of the encoding as operands: e.p[..][t % 4] of K-step t / 4; a finished K-step goes to LDS and to `done`.
 template <int C, typename Done>
-__device__ __forceinline__ void vjp32_encode(const f32x2v* circle, float x, const float (&factor)[6], float limit, Vjp32Wave& s, int n, int g, const SplitUnits& u,
+__device__ __forceinline__ void vjp32_encode(const f32x2v* circle, float x, const PhaseFactors& factors, Vjp32Wave& s, int n, int g, const SplitUnits& u,
                                              SplitOperand& e, Done&& done) {
   float sn[6], cs[6];
-  vjp32_sincos(circle, x, factor, limit, sn, cs);
+  vjp32_sincos(circle, x, factors, sn, cs);
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
     const int t = 6 * C + f;
@@ -353,7 +359,7 @@ __device__ __forceinline__ void vjp32_encode(const f32x2v* circle, float x, cons
 // (sched_barrier): mixed by the compiler they need more registers than there are.  (Matrix and vector instructions of a part
 // alternated by hand: no faster; the other wavefront of the SIMD fills the gaps.)
 __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, Vjp32Wave& s, const float x[3], float4 adjoint,
-                                            uint32_t mask1, uint32_t mask2, const float (&factor)[6], float limit, float scale,
+                                            uint32_t mask1, uint32_t mask2, const PhaseFactors& factors, float scale,
                                             int lane, const SplitUnits& u) {
   asm volatile("" : "+v"(lane));         // (or the addresses are formed ahead of the loop over the blocks, one by one)
   const int n = lane & 31, g = lane >> 5;
@@ -382,7 +388,7 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   t1.big = t1.small = splat16(0.f);
   SplitOperand e, e0, e1, e2, e3;
   mma_split(d2, read_w2_transposed(w, lane), t1);
-  vjp32_encode<0>(w.circle, x[0], factor, limit, s, n, g, u, e, [&](int, const SplitOperand& v) { e0 = v; });
+  vjp32_encode<0>(w.circle, x[0], factors, s, n, g, u, e, [&](int, const SplitOperand& v) { e0 = v; });
   __builtin_amdgcn_sched_barrier(0);
   vf32x16 tsum = t1.sum();
   SplitAcc a1;
@@ -394,11 +400,11 @@ __device__ __forceinline__ void vjp32_block(const Vjp32Lds& w, Vjp32Sums& sum, V
   }
   a1.small = splat16(0.f);
   mfma_split(read_step(w.w1, 0, lane), e0, a1);
-  vjp32_encode<1>(w.circle, x[1], factor, limit, s, n, g, u, e, [&](int k, const SplitOperand& v) { (k == 1 ? e1 : e2) = v; });
+  vjp32_encode<1>(w.circle, x[1], factors, s, n, g, u, e, [&](int k, const SplitOperand& v) { (k == 1 ? e1 : e2) = v; });
   __builtin_amdgcn_sched_barrier(0);
   mfma_split(read_step(w.w1, 1, lane), e1, a1);
   mfma_split(read_step(w.w1, 2, lane), e2, a1);
-  vjp32_encode<2>(w.circle, x[2], factor, limit, s, n, g, u, e, [&](int, const SplitOperand& v) { e3 = v; });
+  vjp32_encode<2>(w.circle, x[2], factors, s, n, g, u, e, [&](int, const SplitOperand& v) { e3 = v; });
 #pragma unroll
   for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(&s.enc_tail[p][n][2 * g]) = u32x2{e.p[p][0], e.p[p][1]};
   __builtin_amdgcn_sched_barrier(0);

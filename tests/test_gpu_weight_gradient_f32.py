@@ -70,3 +70,37 @@ def test_sines_and_cosines_are_rounded_once(device, reach):
     for got, want in ((sine, phase.sin()), (cosine, phase.cos())):
         error = got.double() - want
         assert float(error.abs().max()) <= PAIR_MAX and float(error.square().mean().sqrt()) <= PAIR_RMS
+
+
+def _attenuated(device):
+    """Frequencies and attenuations of an annealed encoding: neither product with an input is exact."""
+    gen = torch.Generator().manual_seed(2)
+    return 100.5 ** (torch.arange(6) / 5), 0.3 + 0.7 * torch.rand(6, generator=gen)
+
+
+def test_phases_are_those_of_the_forward(device):
+    """(x freq) att with both roundings, and nothing else: to the rounding of a pair, at phases of up to 60."""
+    freq, att = _attenuated(device)
+    rays = torch.rand(1024, 3, generator=torch.Generator().manual_seed(3)) * 2 - 1
+    sine, cosine, flag = _encoding(device, rays, freq, att, 1024)
+    phase = ((rays[:, :, None] * freq) * att).double()
+    assert flag == 0
+    for got, want in ((sine, phase.sin()), (cosine, phase.cos())):
+        assert float((got.double() - want).abs().max()) <= PAIR_MAX
+
+
+def test_a_phase_out_of_range_ends_its_own_pair(device):
+    """65536 is the last phase that the forward takes; the float behind it gives NaN, and so do infinities and NaN."""
+    freq = 2.0 ** torch.arange(6)
+    edge = 65536.0 / 32
+    beyond = float(torch.nextafter(torch.tensor(edge), torch.tensor(1e9)))
+    taken = torch.tensor([[edge, -edge, 0.0], [1e-30, -0.0, 2.0]])
+    refused = torch.tensor([[beyond, -beyond, 1.0], [4 * edge, 1e30, -1e38], [float("inf"), float("-inf"), float("nan")]])
+    for rays in (taken, refused):
+        sine, cosine, flag = _encoding(device, rays, freq, torch.ones(6), rays.shape[0])
+        phase = (rays[:, :, None] * freq).double()
+        phase = torch.where(phase.abs() <= 65536, phase, float("nan"))
+        assert flag == int(bool(phase.isnan().any()))
+        for got, want in ((sine, phase.sin()), (cosine, phase.cos())):
+            assert torch.equal(got.isnan(), want.isnan())
+            assert float((got.double() - want).nan_to_num().abs().max()) <= PAIR_MAX
