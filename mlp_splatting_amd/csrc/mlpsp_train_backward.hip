@@ -465,24 +465,31 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);
     vjp32_load(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane, s, u);
-    Vjp32Sums sum;
-    sum.clear();
-    __syncthreads();
-    int turn = wave / 4;
-    walk_halves<kVjp32Waves / 2, false>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
-      // (a wavefront's blocks take turns at priority: 5.22 ms for the gradient call instead of 5.25)
-      if (turn & 1) __builtin_amdgcn_s_setprio(1);
-      else __builtin_amdgcn_s_setprio(0);
-      ++turn;
-      vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, scale, lane, u);
-    });
-    const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
-    if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
-    __syncthreads();
-    bad |= store_row_sums(reinterpret_cast<const float*>(&s.wave[0]), sizeof(Vjp32Wave) / 4, waves,
-                          run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t, 64 * kVjp32Waves);
+    // The adjoints lifted first; sums that this takes out of range are formed again without.
+    for (float by = scale * kVjp32Lift;; by = scale) {
+      Vjp32Sums sum;
+      sum.clear();
+      __syncthreads();
+      int turn = wave / 4;
+      walk_halves<kVjp32Waves / 2, false>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
+        // (a wavefront's blocks take turns at priority: 5.22 ms for the gradient call instead of 5.25)
+        if (turn & 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
+        ++turn;
+        vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, by, lane, u);
+      });
+      const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
+      if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
+      __syncthreads();
+      const bool beyond = store_row_sums(reinterpret_cast<const float*>(&s.wave[0]), sizeof(Vjp32Wave) / 4, waves,
+                                         run_dest(rows, grads, run, chunk, num_chunks), 1.f / by, t, 64 * kVjp32Waves);
+      if (!__syncthreads_or(beyond)) break;
+      if (by == scale) {
+        bad = true;
+        break;
+      }
+    }
     pos = run.end;
-    __syncthreads();
   }
   if (__ballot(bad) != 0ull && lane == 0) atomicOr(nonfinite, 1);
 }

@@ -3,7 +3,7 @@
 //
 // Why.  v_mfma_f32_32x32x2_f32 does 32 multiply-adds per clock and SIMD and keeps the vector ALU from working meanwhile; the
 // bf16 instruction does 512 beside it.  x = h + m + l with h = bf16(x), m = bf16(x - h), l = x - h - m is exact (three times
-// eight significant bits, down to 2^-100), and of the nine products of two such sums the six of weight 2^-16 and more are
+// eight significant bits, of numbers down to 2^-100; kVjp32Lift), and of the nine products of two such sums the six of weight 2^-16 and more are
 // kept: what is dropped is below 2^-24 of the product, a rounding of the f32 product itself.  A sum over K = 16 terms then
 // takes six instructions of 32 clocks instead of eight of 64, and rounds its accumulator six times instead of sixteen.
 // Error of the gradients against float64, 2-norm over 2-norm, f32 chains of v_mfma_f32_32x32x2_f32 -> here:
@@ -117,6 +117,10 @@ __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4&
 
 // A workgroup of four wavefronts, two workgroups to a CU: 22 KB of operands and 2.5 KB of turns that its wavefronts read, 14 KB of each one's own.
 constexpr int kVjp32Waves = 4;
+// The third part of a number below 2^-100 is lost.  The adjoints, which scale with the loss, are multiplied by this first and
+// their sums divided by it, which changes no bit of a number in range: with adjoints of 2^-120 (2^-112) the W1 gradient was off
+// by 4e-3 (1.5e-5) of its norm, with f32 products by 4e-7 (3e-8).  Weights and encodings below 2^-100 stay as they are.
+constexpr float kVjp32Lift = 0x1p32f;
 constexpr int kCircleEntries = 320;       // of vjp32_sincos' table
 union Vjp32Wave {
   struct {

@@ -104,3 +104,44 @@ def test_a_phase_out_of_range_ends_its_own_pair(device):
         for got, want in ((sine, phase.sin()), (cosine, phase.cos())):
             assert torch.equal(got.isnan(), want.isnan())
             assert float((got.double() - want).nan_to_num().abs().max()) <= PAIR_MAX
+
+
+@pytest.mark.parametrize("power", [-120, -112, -100, 40, 100, 110])
+def test_gradients_scale_with_the_adjoints(device, power):
+    """A loss scaled by a power of two has gradients scaled by it, bit for bit.  Where the sums of a chunk (16 of 16 steps for
+    each primitive, of two rows at the ends) fall below the smallest normal number, each is rounded to 2^-149 by half of that,
+    and those that stay above may be rounded the other way for it, 2^-24 of the largest each."""
+    import numpy as np
+    from mlp_splatting_amd import ops
+    base, frame = _frame(device, 256, [np.arange(3)] * 256, 3)
+    groups = ops.train_group(frame, base[6], 3)
+    gen = torch.Generator(device=device).manual_seed(4)
+    d4 = torch.randn(frame.steps, 64, 4, device=device, generator=gen)
+    scaled = (d4.double() * 2.0 ** power).float()
+    d4 = (scaled.double() * 2.0 ** -power).float()
+    falloff = torch.zeros(frame.steps, 64, device=device)
+    grads = [ops.train_gradients(frame, groups, d, falloff, base[1], base[7], base[8], base[9:15], base[3], base[4], 0, 1.0)
+             for d in (d4, scaled)]
+    assert int(grads[0][1]) == int(grads[1][1]) == 0
+    for want, got in zip(grads[0][0][:6], grads[1][0]):
+        want, got = want.double() * 2.0 ** power, got.double()
+        bound = 18 * (2.0 ** -150 + 2.0 ** -24 * float(want.abs().max())) if power < -80 else 0.0
+        assert float(want.abs().max()) > 0 and float((got - want).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 3e38])
+def test_sums_out_of_range_are_refused(device, value):
+    """... and of the numbers that f32 holds none is refused: a finite adjoint of 3e38 by itself is taken."""
+    import numpy as np
+    from mlp_splatting_amd import ops
+    base, frame = _frame(device, 40, [np.arange(3)] * 40, 3)
+    groups = ops.train_group(frame, base[6], 3)
+    for copies in (1, 2):
+        d4 = torch.zeros(frame.steps, 64, 4, device=device)
+        d4[60:60 + 3 * copies:3, 5, 1] = value              # one primitive, one or two of its tiles
+        got, flag = ops.train_gradients(frame, groups, d4, torch.zeros(frame.steps, 64, device=device), base[1], base[7],
+                                        base[8], base[9:15], base[3], base[4], 0, 1.0)
+        taken = value == 3e38 and copies == 1
+        assert int(flag) == int(not taken)
+        if taken:
+            assert sorted(got[5].flatten().tolist())[-1] == torch.tensor(value).item()
