@@ -470,12 +470,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
       Vjp32Sums sum;
       sum.clear();
       __syncthreads();
-      int turn = wave / 4;
       walk_halves<kVjp32Waves / 2, false>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
-        // (a wavefront's blocks take turns at priority: 5.22 ms for the gradient call instead of 5.25)
-        if (turn & 1) __builtin_amdgcn_s_setprio(1);
-        else __builtin_amdgcn_s_setprio(0);
-        ++turn;
         vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, by, lane, u);
       });
       const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
