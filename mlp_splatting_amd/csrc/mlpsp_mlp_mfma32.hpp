@@ -64,8 +64,7 @@ __device__ __forceinline__ void interleave16(const mf32x4 c4[4], float v[16]) {
 
 // What one lane loads of a primitive's layers 1 and 2, as the loads deliver it: row `hid` of W1 (its half g) and
 // the first bias vector (its half g); the same row of W2 and the second bias vector.  Requesting is separate from
-// using, and layer 1 from layer 2: a caller can have the next primitive's layer-1 operands under way while it
-// evaluates this one, and layer 2's arrive behind layer 1's instructions anyway.
+// using, and layer 1 from layer 2: those of layer 2 arrive behind layer 1's instructions.
 struct MlpLayer1 {
   mf32x4 a1[9], b1[4];
 };
@@ -194,9 +193,6 @@ __device__ __forceinline__ void encode_direction(float rdx, float rdy, float rdz
   }
 }
 
-// All 64 lanes must be active.  x6 is the lane's own pixel's input (components 0..2 enter through dir,
-// which encode_direction() made from them); out is the lane's own pixel's output.  `w1` = the primitive's layer-1
-// operands as request_layer1() loaded them; layer2(w2) requests those of layer 2.
 // `mask` shifted left by BITS, the lowest of which say whether the rectified value r is positive: the highest of them does, as the
 // sign of 0 - r (+0 where r is a zero), the other is r's.  Two instructions a value; compared, selected and or-ed they are three,
 // each of the slower kind, and layer 1's accumulators need not outlive layer 2 (168 -> 146 registers; training forward of the
@@ -206,13 +202,17 @@ __device__ __forceinline__ uint32_t push_positive(uint32_t mask, float r) {
   return __builtin_amdgcn_alignbit(mask, float_to_bits(0.f - r), 32 - BITS);
 }
 
-// REC selects the record kernels' layer-2 rounding (bias added after a chain started at zero); MASKS fills
-// masks[0..1] with the ReLU masks of the lane's pixel.
-template <bool REC = false, bool MASKS = REC, typename RequestLayer2>
+// All 64 lanes must be active.  x6 is the lane's own pixel's input (components 0..2 enter through dir,
+// which encode_direction() made from them); out is the lane's own pixel's output.  `w1` = the primitive's layer-1
+// operands as request_layer1() loaded them; layer2(w2) requests those of layer 2.  REC selects the record kernels' layer-2
+// rounding (bias added after a chain started at zero); MASKS fills masks[0..1] with the ReLU masks of the lane's pixel.
+// (mlp_wave_mfma32 is the one caller.  With its requests written here the compiler places them otherwise: the f32 frame and the
+// training forward are 0.4 to 0.7 % slower.)
+template <bool REC, bool MASKS, typename RequestLayer2>
 __device__ __forceinline__ void mlp_wave_mfma32_with(const MlpLayer1& w1, RequestLayer2&& layer2, const float x6[6],
                                                      const float* __restrict__ freq, const float* __restrict__ att,
                                                      const float* __restrict__ W3, const float* __restrict__ b3, int p,
-                                                     const DirOperands& dir, float out[4], uint32_t* masks = nullptr) {
+                                                     const DirOperands& dir, float out[4], uint32_t* masks) {
   constexpr int H = 32, R = H / 2;    // R: accumulator registers (hidden units 2i + g)
   const int lane = threadIdx.x & 63, g = lane >> 5;
   const float inf = relu_limit();
