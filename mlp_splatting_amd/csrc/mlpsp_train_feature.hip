@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
   }
 }
 
-// The same for four slots and rows of 128 channels and more, in sixteens, on the matrix cores: a product of k (four slots x
+// The same for four slots and sixteens of channels on the matrix cores (attr_on_matrix_cores): a product of k (four slots x
 // steps and targets) and signs (steps and targets x channels) in 16x16x32 bf16 products.  Exact in its factors: a sign is a
 // bf16 number, k the sum of three (mlpsp_vjp32.hpp), which take three times four of the sixteen rows and have accumulators of
 // their own.  One wavefront = one chunk x 256 channels, eight steps at a time: lane (n, q) has two steps, and of their signs the
@@ -530,6 +530,17 @@ inline int attr_chunk_steps(int64_t S, int C) {
   const int64_t per = S * ceil_div(C, 256) / 16384;
   return per >= 64 ? 64 : per <= 4 ? 4 : (int)per;
 }
+// Which of the two attribute kernels (four slots).  A lane of the matrix-core kernel takes sixteen signs a load, hence sixteens
+// of channels, and a product eight steps; the other kernel takes one, two or four steps at a time, for rows of up to 256, 128
+// and 64 channels.  Whole gradient call in us, f32 FMA / matrix cores, by steps of a chunk:
+//     64 channels    4: 49 / 58      12:  54 / 64     43: 114 / 118
+//    128             4: 58 / 70      12:  73 / 73     16:  88 / 80      43: 226 / 174
+//    192 (256)       4: 58 / 62      5:   68 / 68 (73 / 76)      7: 78 / 71 (84 / 79)     43: 361 / 217 (404 / 270)
+//    272 (512)       4: 63 / 74 (74 / 89)     7: 74 / 70 (86 / 85)     10: 93 / 80 (106 / 95)     64: 592 / 344 (740 / 506)
+//    528             7: 78 / 80      11: 100 / 88     36: 260 / 160
+inline bool attr_on_matrix_cores(int channels, int Cp, int chunk_steps) {
+  return channels % 16 == 0 && channels > 64 && chunk_steps >= 7 * (64 >> lanes_per_row_log2(Cp));
+}
 
 }  // namespace mlpsp
 
@@ -618,8 +629,7 @@ MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int he
 #define MLPSP_ATTR(SL, VEC)                                                                                              \
   hipLaunchKernelGGL((train_attr_kernel<SL, VEC>), grid, dim3(256), 0, s, f, o, t.prim, t.first, t.step,         \
                      (int)num_steps, per, chunks, lanes_per_row_log2(f.Cp), loss_adjoint_dev, rows_dev, out_dev)
-    // (fewer channels leave lanes without work)
-    const bool wide = slots == 4 && vec && channels % 16 == 0 && channels >= 128 && ((uintptr_t)kept_dev & 15u) == 0;
+    const bool wide = slots == 4 && vec && attr_on_matrix_cores(channels, f.Cp, per) && ((uintptr_t)kept_dev & 15u) == 0;
     const float unit = wide ? kSignValue : (float)kSignUnit;
     if (wide)
       hipLaunchKernelGGL(train_attr_mfma_kernel, grid, dim3(256), 0, s, f, o, t.prim, t.first, t.step, (int)num_steps, per, chunks,

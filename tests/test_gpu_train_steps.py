@@ -77,7 +77,7 @@ def test_reduced_forward_steps_are_those_of_its_records(device, oracle_mod, prec
     (8, 4, 64, 4), (8, 4, 67, 5), (8, 4, 516, 1),     # a quarter; one, two and four lane groups; more than one wavefront
     (13, 7, 130, 5),       # a ratio that is no whole number
     (3, 2, 256, 4),        # more pixels than a tile between two targets: tiles without one
-    (33, 17, 144, 4), (8, 4, 128, 4), (13, 7, 528, 4),      # four slots of sixteens of channels: on the matrix cores
+    (33, 17, 144, 4), (8, 4, 128, 4), (13, 7, 528, 4),      # sixteens of channels, whole and with a remainder
     (1, 1, 3, 1)])
 @pytest.mark.parametrize("half", [False, True])
 def test_feature_loss_of_steps_is_that_of_records(device, oracle_mod, wf, hf, channels, slots, half):
