@@ -55,3 +55,30 @@ def ulp_diff(a, b):
     ia = np.where(ia < 0x80000000, ia, 0x80000000 - ia)
     ib = np.where(ib < 0x80000000, ib, 0x80000000 - ib)
     return np.abs(ia - ib)
+
+
+def tile_row(device, tiles, n, tile, prim, mlp=None):
+    """(scene tensors, width, height) of a row of ``tiles`` tiles with the lists that ``tile`` (ascending) and ``prim`` name
+    entry by entry; every one of the ``n`` primitives hits every pixel.  ``mlp``: the six weights, broadcast over primitives."""
+    from conftest import to_dev
+    width, height = 8 * tiles, 8
+    sc = syn.make_scene(n, 32, seed=5, log_scale_mean=2.5)
+    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
+    sc.b3[:, 3] = -6.0
+    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
+    off = np.searchsorted(tile, np.arange(tiles + 1)).astype(np.int32)
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats,
+                                        np.asarray(prim, dtype=np.int32), off, sc.freq, sc.att, *sc.mlp())]
+    for t, v in zip(base[9:15], mlp or ()):
+        t.copy_(v.to(device).expand_as(t))
+    return base, width, height
+
+
+def ragged_lists(tiles, n, steps):
+    """(tile, primitive) of together ``steps`` list entries: primitive p lies in about the share (p + 1) / n of the tiles, so
+    that runs of one tile and of nearly all of them end at any place."""
+    rng = np.random.default_rng(7)
+    score = rng.random((tiles, n)) * n - (np.arange(n) + 1.0)
+    listed = np.zeros(tiles * n, dtype=bool)
+    listed[np.argsort(score, axis=None)[:steps]] = True
+    return np.nonzero(listed.reshape(tiles, n))

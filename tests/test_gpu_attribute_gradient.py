@@ -1,39 +1,12 @@
 """The feature-attribute gradient of training steps where its kernels part, against the gradient from per-pixel records: a
 chunk holds steps x (256s of channels, rounded up) / 16,384 of the sorted steps, between 4 and 64, and the matrix-core kernel
 takes rows of more than 64 channels in sixteens where it holds seven and more (fourteen up to 128 channels), eight at a time."""
-import numpy as np
 import pytest
 import torch
 
-from conftest import to_dev
+from helpers import ragged_lists, tile_row
 
 pytestmark = pytest.mark.gpu
-
-
-def _frame(device, tiles, n, steps):
-    """A row of tiles and lists of together ``steps`` entries, all of which hit: primitive p lies in the share (p + 1) / n of
-    the tiles, about, so that runs of one tile and of nearly all are cut at any place."""
-    from mlp_splatting_amd import synthetic as syn
-    from mlp_splatting_amd.tile_ext import TileExt
-    width, height = 8 * tiles, 8
-    sc = syn.make_scene(n, 32, seed=5, log_scale_mean=2.5)
-    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
-    sc.b3[:, 3] = -6.0
-    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
-    rng = np.random.default_rng(7)
-    score = rng.random((tiles, n)) * n - (np.arange(n) + 1.0)
-    listed = np.zeros(tiles * n, dtype=bool)
-    listed[np.argsort(score, axis=None)[:steps]] = True
-    tile, prim = np.nonzero(listed.reshape(tiles, n))
-    off = np.searchsorted(tile, np.arange(tiles + 1)).astype(np.int32)
-    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats,
-                                        prim.astype(np.int32), off, sc.freq, sc.att, *sc.mlp())]
-    ext = TileExt()
-    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
-    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0)
-    _, _, frame = ext.train_forward(base, width, height, 1e-3, render_order=False)
-    assert frame.steps == steps
-    return base, records, frame, width, height
 
 
 #                        tiles, primitives, steps, channels          steps of a chunk
@@ -51,7 +24,13 @@ def _frame(device, tiles, n, steps):
     (2048, 56, 114688, 80), (2048, 56, 114688, 144)])       # 7: FMA up to 128 channels, matrix cores above
 def test_attribute_gradients_at_the_edges_of_chunks_and_kernels(device, tiles, n, steps, channels):
     from mlp_splatting_amd import ops, primitive_csr, record_feature_loss
-    base, records, frame, width, height = _frame(device, tiles, n, steps)
+    from mlp_splatting_amd.tile_ext import TileExt
+    base, width, height = tile_row(device, tiles, n, *ragged_lists(tiles, n, steps))
+    ext = TileExt()
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0)
+    _, _, frame = ext.train_forward(base, width, height, 1e-3, render_order=False)
+    assert frame.steps == steps
     gen = torch.Generator(device=device).manual_seed(7)
     attributes = torch.randn(n, 4, channels, device=device, generator=gen) * 0.05
     # (targets far outside what the attributes blend to: no residual is near zero, where two sums may differ in sign)

@@ -263,12 +263,12 @@ def test_attributes_that_no_target_samples_may_be_anything(device, oracle_mod, v
 @pytest.mark.parametrize("precision", [0, 1, 2])
 @pytest.mark.parametrize("tiles", [1, 3, 4, 5, 15, 16, 17, 31, 129, 255])
 def test_weight_gradients_of_runs_of_every_length(device, tiles, precision):
-    """The kernels deal a run's half steps to four wavefronts and cut the steps into chunks of 16 to 128: runs of one
-    primitive that are a little shorter and longer than those, three in a row, against float64 over the same steps.  An f32
-    gradient is a sum of up to 16,000 products of two factors that are f32 sums of up to 72 terms themselves: a few units of
-    2^-24 each, 1e-6 of the norm.  A phase is an f32 product of two roundings, and moves its sine by as much: 2^-23 times the
-    largest phase.  In 16 bits (1: fp16, 2: bf16) every factor and what it was computed from, eight tensors at the most, is
-    rounded once, by 2^-11 or 2^-8 of it; the adjoints are scaled by 256 and stay above what fp16 holds in full."""
+    """The kernels deal a run's half steps to four wavefronts and cut the steps into chunks, here of 16 (those of more are
+    test_gpu_weight_gradients.py's): runs of one primitive that are a little shorter and longer, three in a row, against float64
+    over the same steps and the forward's phases.  An f32 gradient is a sum of up to 16,000 products of two factors that are f32
+    sums of up to 72 terms themselves: a few units of 2^-24 each, 1e-6 of the norm.  In 16 bits (1: fp16, 2: bf16) every factor
+    and what it was computed from, eight tensors at the most, is rounded once, by 2^-11 or 2^-8 of it, and a phase moves its sine
+    by two roundings, 2^-23 times the largest phase; the adjoints are scaled by 256 and stay above what fp16 holds in full."""
     import numpy as np
     from mlp_splatting_amd import ops, synthetic as syn
     from mlp_splatting_amd.tile_ext import TileExt
@@ -301,10 +301,11 @@ def test_weight_gradients_of_runs_of_every_length(device, tiles, precision):
     W1, b1, W2, b2, W3, _ = (w.double() for w in base[9:15])
     for p in range(n):
         at = (ids == p).nonzero(as_tuple=True)
-        phase = (x6[at].double()[:, :, None] * base[7].double() * base[8].double()).reshape(-1, 36)
+        phase = ((x6[at][:, :, None] * base[7]) * base[8]).reshape(-1, 36).double()
         enc, d = torch.cat([phase.sin(), phase.cos()], 1), adjoint[at]
         z1 = enc @ W1[p].T + b1[p]
-        bound = (1e-6, 8 * 2.0 ** -11, 8 * 2.0 ** -8)[precision] + 2.0 ** -23 * float(phase.abs().max())
+        bound = (1e-6, 8 * 2.0 ** -11, 8 * 2.0 ** -8)[precision]
+        bound += 2.0 ** -23 * float(phase.abs().max()) if precision else 0.0
         h1 = z1.clamp(min=0.0)
         z2 = h1 @ W2[p].T + b2[p]
         d2 = (d @ W3[p]) * (z2 > 0)

@@ -1,45 +1,35 @@
-"""The parts of the f32 weight-gradient kernel of training steps, each against float64: the encoding that it forms anew."""
+"""The weight-gradient kernels of training steps against float64: the encoding that the f32 kernel forms anew, its range, and
+sums over chunks of every length."""
+import numpy as np
 import pytest
 import torch
 
-from conftest import to_dev
+from helpers import ragged_lists, tile_row
 
 pytestmark = pytest.mark.gpu
 
 
-def _frame(device, tiles, lists, n, mlp=None, log_scale_mean=2.5):
-    """(base, frame) of a row of ``tiles`` tiles; ``lists[t]``: the primitives of tile t, each of which hits all its pixels."""
-    import numpy as np
-    from mlp_splatting_amd import synthetic as syn
+def _frame(device, tiles, n, tile, prim, mlp=None):
     from mlp_splatting_amd.tile_ext import TileExt
-    width, height = 8 * tiles, 8
-    sc = syn.make_scene(n, 32, seed=5, log_scale_mean=log_scale_mean)
-    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
-    sc.b3[:, 3] = -6.0
-    c2w = syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0))
-    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, c2w)
-    cand = np.concatenate(lists).astype(np.int32)
-    off = np.concatenate([[0], np.cumsum([len(v) for v in lists])]).astype(np.int32)
-    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats, cand, off, sc.freq,
-                                        sc.att, *sc.mlp())]
-    if mlp is not None:
-        for t, v in zip(base[9:15], mlp):
-            t.copy_(v.to(device).expand_as(t))
+    base, width, height = tile_row(device, tiles, n, tile, prim, mlp)
     _, _, frame = TileExt().train_forward(base, width, height, 1e-3)
-    assert frame.steps == cand.size
+    assert frame.steps == len(tile)
     return base, frame
+
+
+def _every_tile(tiles, n):
+    return np.repeat(np.arange(tiles), n), np.tile(np.arange(n), tiles)
 
 
 def _encoding(device, rays, freq, att, tiles):
     """(sines, cosines, flag) of the phases of ``rays`` [tiles, 3], read off the W1 gradient of one record a primitive whose
     hidden adjoints are all 1: [tiles, 3, 6] each, the value of every hidden unit compared."""
-    import numpy as np
     from mlp_splatting_amd import ops
     eye = torch.eye(32)
     first = torch.zeros(4, 32)
     first[0] = 1.0
     mlp = (torch.zeros(32, 72), torch.ones(32), eye, torch.ones(32), first, torch.tensor([0.0, 0.0, 0.0, -6.0]))
-    base, frame = _frame(device, tiles, [np.array([t]) for t in range(tiles)], tiles, mlp)
+    base, frame = _frame(device, tiles, tiles, np.arange(tiles), np.arange(tiles), mlp)
     tile = torch.arange(tiles, device=device)
     lane = 7 * tile % 64
     d4 = torch.zeros(tiles, 64, 4, device=device)
@@ -111,9 +101,8 @@ def test_gradients_scale_with_the_adjoints(device, power):
     """A loss scaled by a power of two has gradients scaled by it, bit for bit.  Where the sums of a chunk (16 of 16 steps for
     each primitive, of two rows at the ends) fall below the smallest normal number, each is rounded to 2^-149 by half of that,
     and those that stay above may be rounded the other way for it, 2^-24 of the largest each."""
-    import numpy as np
     from mlp_splatting_amd import ops
-    base, frame = _frame(device, 256, [np.arange(3)] * 256, 3)
+    base, frame = _frame(device, 256, 3, *_every_tile(256, 3))
     groups = ops.train_group(frame, base[6], 3)
     gen = torch.Generator(device=device).manual_seed(4)
     d4 = torch.randn(frame.steps, 64, 4, device=device, generator=gen)
@@ -132,9 +121,8 @@ def test_gradients_scale_with_the_adjoints(device, power):
 @pytest.mark.parametrize("value", [float("nan"), float("inf"), 3e38])
 def test_sums_out_of_range_are_refused(device, value):
     """... and of the numbers that f32 holds none is refused: a finite adjoint of 3e38 by itself is taken."""
-    import numpy as np
     from mlp_splatting_amd import ops
-    base, frame = _frame(device, 40, [np.arange(3)] * 40, 3)
+    base, frame = _frame(device, 40, 3, *_every_tile(40, 3))
     groups = ops.train_group(frame, base[6], 3)
     for copies in (1, 2):
         d4 = torch.zeros(frame.steps, 64, 4, device=device)
@@ -145,3 +133,62 @@ def test_sums_out_of_range_are_refused(device, value):
         assert int(flag) == int(not taken)
         if taken:
             assert sorted(got[5].flatten().tolist())[-1] == torch.tensor(value).item()
+
+
+def _two_parts(v):
+    """``v`` as the sum of two bf16 numbers: an f32 operand without its third part."""
+    v = v.float()
+    high = v.bfloat16().float()
+    return (high + (v - high).bfloat16().float()).double()
+
+
+# Steps of a chunk: steps / 2048 in eights, between 16 and 128.
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("tiles,n,steps", [(2500, 40, 49151), (2500, 40, 49152), (3300, 40, 65536 + 17), (6700, 40, 131072 + 50),
+                                           (13200, 40, 262144 - 1), (13200, 40, 262144), (15100, 40, 300001)])
+def test_weight_gradients_of_chunks_of_every_length(device, tiles, n, steps, precision):
+    """A pixel in 25 has an adjoint, so that blocks without one lie among the others.  An f32 gradient is the sum of up to
+    25,000 products, in chains of up to 64 blocks x 12 roundings whose sums, 100 at the most, are added up in turn.  k roundings
+    of a sum that grows to s, as a random walk does, add up to sqrt(k / 2) s 2^-24 / sqrt(12): 5.7 units of 2^-24 for a chain,
+    2 for its sums, 2 for the factors' own; twelve, which is less than what is lost with the third part of any one operand.  In
+    16 bits every factor and what it was computed from, eight tensors at the most, is rounded once, and a phase by a few units
+    of 2^-24."""
+    from mlp_splatting_amd import ops
+    from mlp_splatting_amd.tile_ext import TileExt
+    base, width, height = tile_row(device, tiles, n, *ragged_lists(tiles, n, steps))
+    ext = TileExt()
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0, render_order=True)
+    _, _, frame = ext.train_forward(base, width, height, 1e-3)
+    assert frame.steps == steps and records[2].numel() == 64 * steps
+    gen = torch.Generator(device=device).manual_seed(9)
+    d4 = torch.randn(steps, 64, 4, device=device, generator=gen)
+    d4 *= torch.rand(steps, 64, 1, device=device, generator=gen) < 0.04
+    got, flag = ops.train_gradients(frame, ops.train_group(frame, base[6], n), d4, torch.zeros(steps, 64, device=device), base[1],
+                                    base[7], base[8], base[9:15], base[3], base[4], precision, 256.0 if precision else 1.0)
+    assert int(flag) == 0
+    # d4 is [step of a tile, lane], the records are [pixel, hit] in the tile's order
+    pixel = torch.repeat_interleave(torch.arange(width * height, device=device), records[7].diff())
+    hit = torch.arange(64 * steps, device=device) - records[7][:-1][pixel]
+    at = (base[6].long()[pixel % width // 8] + hit) * 64 + pixel // width * 8 + pixel % 8
+    live = (d4.view(-1, 4)[at] != 0).any(1).nonzero()[:, 0]
+    ids, x6, d4 = records[2][live], records[3][live], d4.view(-1, 4)[at[live]]
+    active = (records[5][live][:, :, None] >> torch.arange(32, dtype=torch.int32, device=device)) & 1
+    W1, b1, W2, b2, W3, _ = (w.double() for w in base[9:15])
+    for p in range(n):
+        mine = ids == p
+        phase = ((x6[mine][:, :, None] * base[7]) * base[8]).reshape(-1, 36).double()
+        enc, d, on = torch.cat([phase.sin(), phase.cos()], 1), d4[mine].double(), active[mine].double()
+        bound = (12 * 2.0 ** -24, 8 * 2.0 ** -11, 8 * 2.0 ** -8)[precision]
+        bound += 2.0 ** -23 * float(phase.abs().max()) if precision else 0.0
+        h1 = (enc @ W1[p].T + b1[p]).clamp(min=0.0)
+        h2 = (h1 @ W2[p].T + b2[p]).clamp(min=0.0)
+        d2 = (d @ W3[p]) * on[:, 1]
+        d1 = (d2 @ W2[p]) * on[:, 0]
+        want = [d1.T @ enc, d1.sum(0), d2.T @ h1, d2.sum(0), d.T @ h2, d.sum(0)]
+        for i, (a, b) in enumerate(zip(got, want)):
+            assert float((a[p].double() - b).norm()) <= bound * float(b.norm()), (p, i)
+        if precision == 0:
+            for i, less in ((0, d1.T @ _two_parts(enc)), (0, _two_parts(d1).T @ enc), (2, d2.T @ _two_parts(h1)),
+                            (2, _two_parts(d2).T @ h1)):
+                assert float((less - want[i]).norm()) > bound * float(want[i].norm()), (p, i)
