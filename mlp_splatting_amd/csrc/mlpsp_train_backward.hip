@@ -9,7 +9,7 @@
 // that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.14 (sort 1.7, gathers 2.85), geometry 0.18 (1.3), weight gradients 4.6 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
+// 0.14 (sort 1.7, gathers 2.85), geometry 0.16 (1.3), weight gradients 5.1 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -493,8 +493,8 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
 // One workgroup per chunk and quarter of a row: the sum of the rows of the primitive whose steps begin in the chunk and go
 // on in the next (its tail row here, tails in between, the head row of its last chunk); nothing if there is none.  What
 // lasts is a primitive with steps in most tiles, hundreds of rows one after the other: sixteen of them are in flight, and
-// its columns are shared out (one workgroup and eight in flight, chunks of 64 steps: 0.35 ms at 650,000 steps; 0.21; with
-// chunks of 256 steps 0.03).
+// its columns are shared out (650,000 steps in chunks of 64: one workgroup and eight in flight 0.35 ms, this 0.21; in chunks of
+// 128 as now 0.035).
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, int chunk_steps, int num_chunks,
                                                          const float* __restrict__ rows, const float* __restrict__ quats,
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(256) void train_join_kernel(StepIndex ix, int S, in
 
 // Steps per chunk: as many as a wavefront has lanes for (twice that is no faster), fewer where that would leave fewer than four
 // chunks for each of the 512 workgroups that run at once (f32; 768 in 16 bits), 16 at the least.  Gradient call in us, f32, a half, as much and
-// twice as much of that rule at 51,600 steps: 483, 484, 518.
+// twice as much of that rule at 51,600 steps: 494, 489, 526.
 inline int train_chunk_steps(int64_t S) {
   const int64_t per = S / 2048 / 8 * 8;
   return per >= kTrainChunk ? kTrainChunk : per <= 16 ? 16 : (int)per;

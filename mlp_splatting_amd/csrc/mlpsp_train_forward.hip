@@ -6,7 +6,8 @@
 // Geometry, order, activations and compositing are the f32 expressions of the render (f32 MLP: its bits with
 // `render_order`, the record kernels' rounding of layer 2 without).  Bound by the MLP; the steps add 3.3 KB of contiguous
 // stores per hit step.  200,000 primitives, 1200x680, f32: 3.9 ms, against 4.0 + 6.0 of the record forward's two walks;
-// 20,000 primitives, 320x240: 1.24 ms with a wavefront per tile, 0.87 with teams (see train_plan).
+// 20,000 primitives, 320x240: 0.57 ms in teams of four (five cameras; with three wavefronts to a SIMD 0.87 for one of them, and
+// 1.24 with a wavefront per tile, see train_plan).
 #include <type_traits>
 
 #include "mlpsp_device.hpp"

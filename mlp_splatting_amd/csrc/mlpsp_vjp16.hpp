@@ -32,7 +32,8 @@ constexpr int kGradFloats = 3524;   // W1 2304 | b1 32 | W2 1024 | b2 32 | W3 12
 // that transposes through LDS.  The 4x32 gradient of W3 and the bias gradient of layer 2 are 4x4x4 products: their 4 rows
 // would fill an eighth of a 32x32 tile.  Bound by the ~350 vector instructions of a block: a wavefront that is alone on its
 // SIMD issues them at half the rate, so the weight operands lie in LDS and two wavefronts fit (252 registers; with the
-// operands in registers 342 and one wavefront).  648,000 steps of 64 records: 3.18 -> 2.06 ms.
+// operands in registers 342 and one wavefront; over training steps, which ran these blocks before mlpsp_vjp16_steps.hpp, the one
+// took 2.06 ms for 648,000 steps, the other 3.18).
 //
 // k-slot order of the encoding (both the X operand of layer 1 and W1's operand): lane group g owns input
 // components 3g..3g+2; its slot q = 8 s + j of K-step s (q < 36) is pair t = q / 2 = 6 c + f (component

@@ -6,18 +6,22 @@
 // eight significant bits, of numbers down to 2^-100; kVjp32Lift), and of the nine products of two such sums the six of weight 2^-16 and more are
 // kept: what is dropped is below 2^-24 of the product, a rounding of the f32 product itself.  A sum over K = 16 terms then
 // takes six instructions of 32 clocks instead of eight of 64, and rounds its accumulator six times instead of sixteen.
-// Error of the gradients against float64, 2-norm over 2-norm, f32 chains of v_mfma_f32_32x32x2_f32 -> here:
-//                           W1                 b1                 W2                 b2                 W3
-//   647,988 steps   3.9e-7 -> 2.5e-7   2.8e-7 -> 1.5e-7   3.4e-7 -> 2.1e-7   3.7e-7 -> 1.1e-7   2.8e-7 -> 1.5e-7
-//    51,614 steps   1.9e-7 -> 1.2e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 1.1e-7   2.2e-7 -> 0.7e-7   1.7e-7 -> 1.0e-7
-// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.45 -> 4.96 ms, 0.72 -> 0.47 ms.
+// Error of the gradients against float64 at the same f32 phases, 2-norm over 2-norm, and of a primitive's W1 gradient in the
+// median and at the most, f32 chains of v_mfma_f32_32x32x2_f32 -> here:
+//                           W1                 b1                 W2                 b2                 W3           a primitive's W1
+//   647,988 steps   3.9e-7 -> 2.3e-7   2.8e-7 -> 1.5e-7   3.4e-7 -> 1.8e-7   3.7e-7 -> 1.1e-7   2.8e-7 -> 1.5e-7   3.7e-7 -> 2.8e-7, 2.4e-6 -> 1.3e-6
+//    51,614 steps   1.9e-7 -> 1.0e-7   2.3e-7 -> 1.1e-7   2.1e-7 -> 0.9e-7   2.2e-7 -> 0.7e-7   1.7e-7 -> 1.0e-7   1.9e-7 -> 1.3e-7, 4.2e-7 -> 4.0e-7
+//   3 x 4,096       6.2e-7 -> 4.7e-7   6.8e-7 -> 3.9e-7   7.4e-7 -> 4.8e-7   8.8e-7 -> 4.0e-7   9.3e-7 -> 3.7e-7
+// The part of it along the gradient (a bias of all elements together) is at most 2e-7 of the norm, of either sign, also where
+// all adjoints have one sign; of the f32 chains as much, for b3 9e-7.
+// Time of the whole gradient call (200,000 primitives, 1200x680 / 20,000, 320x240): 7.42 -> 5.11 ms, 0.72 -> 0.49 ms.
 //
-// Bound by the latency of a block's chain -- products, the ~920 vector instructions between them (a third of them sines and
-// cosines, a sixth the splits), LDS --, two wavefronts to a SIMD: 256 registers with the weights in LDS.  (A third of the vector
-// instructions less, by the table of vjp32_sincos, is 3 % of the time.)  A wavefront with its own weights in registers spills
-// (6.7 ms, waiting for its spills behind the records requested ahead), alone on its SIMD it is no faster for 512 registers
-// (7.0).  The two belong to different workgroups, one of which works while the other changes primitives (one workgroup of
-// eight: 5.23 and 0.52 ms instead of 5.17 and 0.48).
+// Bound by the latency of a block's chain -- products, the ~1,090 vector instructions beside them (a third of them sines and
+// cosines, a sixth the splits), LDS --, two wavefronts to a SIMD: 256 registers with the weights in LDS.  (Sines and cosines by
+// det_sincos: 1,250 instructions instead of 920 with a table without remainders, and 3 % of the time.)  A wavefront with its own
+// weights in registers spills (6.7 ms, waiting for its spills behind the records requested ahead), alone on its SIMD it is no
+// faster for 512 registers (7.0).  The two belong to different workgroups, one of which works while the other changes primitives
+// (one workgroup of eight: 5.23 and 0.52 ms instead of 5.17 and 0.48).
 //
 // Per block (lane (n, g) = record n, half g of its inputs; D(a, b) has the rows of a in its registers):
 //   d2        D(W3, d): record in the lane, unit 8 (i / 4) + 4 g + i % 4 in register i, in f32 products
@@ -104,7 +108,8 @@ __device__ __forceinline__ void mma_split(const Split8& a, const Split8& b, Spli
 #pragma unroll
   for (int s = 0; s < 2; ++s) mfma_split(a.p[0].s[s], a.p[1].s[s], a.p[2].s[s], b.p[0].s[s], b.p[1].s[s], b.p[2].s[s], acc);
 }
-// ... onto one accumulator that is large against any one product
+// ... onto one accumulator that is large against any one product: nothing of it can be cut off by the product beside it (the
+// bias that is left is measured above)
 __device__ __forceinline__ vf32x16 mfma_split_onto(const u32x4& ha, const u32x4& ma, const u32x4& la, const u32x4& hb,
                                                    const u32x4& mb, const u32x4& lb, vf32x16 acc) {
   acc = Ops<__bf16>::mfma(la, hb, acc);
