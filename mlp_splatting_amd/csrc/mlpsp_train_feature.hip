@@ -396,7 +396,8 @@ __global__ __launch_bounds__(256) void train_attr_kernel(FeatShape f, FeatKept o
 // The same for four slots and sixteens of channels on the matrix cores (attr_on_matrix_cores): a product of k (four slots x
 // steps and targets) and signs (steps and targets x channels) in 16x16x32 bf16 products.  Exact in its factors: a sign is a
 // bf16 number, k the sum of three (mlpsp_vjp32.hpp), which take three times four of the sixteen rows and have accumulators of
-// their own.  One wavefront = one chunk x 256 channels, eight steps at a time: lane (n, q) has two steps, and of their signs the
+// their own.  (A k below 2^-100 loses the third; its gradient, divided by the number of residuals, lies at the end of f32's range.)
+// One wavefront = one chunk x 256 channels, eight steps at a time: lane (n, q) has two steps, and of their signs the
 // channels 16 n .. 16 n + 15 -- sixteen bytes of a row a load; product j takes byte j of each, one byte permutation a word.
 // The lanes hold the chunk's steps and their tiles' groups; a step's rows are not behind a chain of reads.
 // Bound by the latency of those rows (2 KB a step at 512 channels), three wavefronts to a SIMD.  648,000 steps, 512 channels:
