@@ -148,7 +148,9 @@ __device__ __forceinline__ void step_store(const StepPool& sp, int slot, int lan
   if (lane == 0) sp.ids[slot] = p;
 }
 // Zero rows of the primitives that have no step, in every gradient tensor: a wavefront takes eight primitives, so that a
-// row of a few floats fills its stores too.  Bound by the stores (6.3 TB/s for a plain fill on this card).
+// row of a few floats fills its stores too.  Bound by the stores (6.3 TB/s for a plain fill on this card) where it is a launch
+// of its own; the weight gradient kernels, which leave memory three quarters idle, do it beside their products (BESIDE: past the
+// caches, where what they read lies; a launch of its own is 2 % slower that way).
 struct ZeroRows {
   float* base[9];
   int len[9];        // floats per primitive
@@ -158,13 +160,16 @@ struct ZeroRows {
     len[count++] = floats;
   }
 };
-static __global__ __launch_bounds__(256) void zero_rows_kernel(const int32_t* __restrict__ first, int N, ZeroRows z) {
-  const int p0 = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * 8, lane = threadIdx.x & 63;
+constexpr int kZeroGroup = 8;          // primitives a wavefront takes at a time
+template <bool BESIDE>
+__device__ __forceinline__ void zero_rows(const int32_t* __restrict__ first, int N, const ZeroRows& z, int group, int lane) {
+  const int p0 = group * kZeroGroup;
   if (p0 >= N) return;
   const int p = min(p0 + (lane & 7), N - 1);
   const unsigned empty = (unsigned)__ballot(lane < 8 && p0 + lane < N && first[p] == first[p + 1]);
   if (empty == 0u) return;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  typedef float quad __attribute__((ext_vector_type(4)));
+  const quad zero = {0.f, 0.f, 0.f, 0.f};
   for (int a = 0; a < z.count; ++a) {
     float* __restrict__ dst = z.base[a] + (size_t)p0 * z.len[a];
     const bool quads = (z.len[a] & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
@@ -173,18 +178,22 @@ static __global__ __launch_bounds__(256) void zero_rows_kernel(const int32_t* __
       for (unsigned todo = empty; todo; todo &= todo - 1u) {
         const size_t at = (size_t)__builtin_ctz(todo) * n;
         for (int i = lane; i < n; i += 64) {
-          if (quads) reinterpret_cast<float4*>(dst)[at + i] = zero;
-          else dst[at + i] = 0.f;
+          if (!quads) dst[at + i] = 0.f;
+          else if (BESIDE) __builtin_nontemporal_store(zero, reinterpret_cast<quad*>(dst) + at + i);
+          else reinterpret_cast<quad*>(dst)[at + i] = zero;
         }
       }
     } else {
       for (int i = lane; i < 8 * n; i += 64) {
         if (!((empty >> (i / n)) & 1u)) continue;
-        if (quads) reinterpret_cast<float4*>(dst)[i] = zero;
+        if (quads) reinterpret_cast<quad*>(dst)[i] = zero;
         else dst[i] = 0.f;
       }
     }
   }
+}
+static __global__ __launch_bounds__(256) void zero_rows_kernel(const int32_t* __restrict__ first, int N, ZeroRows z) {
+  zero_rows<false>(first, N, z, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), threadIdx.x & 63);
 }
 inline void launch_zero_rows(const int32_t* first, int N, const ZeroRows& z, hipStream_t s) {
   hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)((N + 31) / 32)), dim3(256), 0, s, first, N, z);

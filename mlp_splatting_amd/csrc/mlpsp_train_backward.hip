@@ -5,11 +5,11 @@
 // The steps are sorted by primitive (S = 0.65 M at the 200,000-primitive 1200x680 frame) and cut into chunks of equal
 // length.  A workgroup walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the
 // primitive's steps all lie in the chunk, else to the chunk's tail row (the primitive goes on in the next chunk) or head row
-// (it ended here).  Two more launches add the rows of the primitives
-// that span chunks and write the zeros of those without a step.  No atomics, a fixed order of every sum.
+// (it ended here).  One more launch adds the rows of the primitives that span chunks; the zeros of those without a step are
+// written by the weight gradient kernels too.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.14 (sort 1.7, gathers 2.85), geometry 0.16 (1.3), weight gradients 5.1 (12.8), joining rows 0.03 and zeros 0.48 (0.8).
+// 0.14 (sort 1.7, gathers 2.85), geometry 0.16 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -398,13 +398,23 @@ __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int 
   }
 }
 
+// A wavefront's share of the rows of primitives without a step, stored before it turns to its chunk: the chunks begin at
+// different times, and the stores go on beside the products of the others.  The whole call at 648,000 steps of 200,000
+// primitives with these 2.8 GB in a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 /
+// 1.70; at the end of a chunk as at its beginning, a primitive per block of products 5.34 and 1.83.
+template <int WAVES>
+__device__ __forceinline__ void zero_share(const StepIndex& ix, int N, const ZeroRows& zero, int chunk, int num_chunks, int wave,
+                                           int lane) {
+  for (int group = chunk * WAVES + wave; group * kZeroGroup < N; group += num_chunks * WAVES) zero_rows<true>(ix.first, N, zero, group, lane);
+}
+
 template <typename T>
 __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_eu(3, 3))) void train_vjp16_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int H, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
-    int32_t* __restrict__ nonfinite) {
+    int32_t* __restrict__ nonfinite, int N, ZeroRows zero) {
   __shared__ Vjp16StepsLds<T> lds;
   Vjp16Shared<T>& s = lds.s;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -413,6 +423,7 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
   for (int f = 0; f < 6; ++f)
     kf[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((freq[f] * att[f]) * 0.159154943f)));
+  zero_share<kVjp16Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
   bool bad = false;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);
@@ -448,7 +459,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int H, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
-    int32_t* __restrict__ nonfinite) {
+    int32_t* __restrict__ nonfinite, int N, ZeroRows zero) {
   __shared__ Vjp32Lds s;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
@@ -461,6 +472,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
   }
   if (t < 4) s.zero[t] = 0u;
   for (int k = t; k < kCircleEntries; k += 64 * kVjp32Waves) s.circle[k] = f32x2v{kCircle.at[k][0], kCircle.at[k][1]};
+  zero_share<kVjp32Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
   bool bad = false;
   for (int pos = chunk * chunk_steps; pos < chunk_end;) {
     const StepRun run = step_run(ix, pos, chunk_end);
@@ -685,11 +697,21 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
   const GeoGrads geo{grad_positions_dev, grad_log_scales_dev, grad_quats_dev};
   const int S = (int)num_steps;
   const int chunk_steps = t.chunk_steps, num_chunks = t.num_chunks;
+  ZeroRows zero{};
+  zero.add(gW1_dev, 2304);
+  zero.add(gb1_dev, 32);
+  zero.add(gW2_dev, 1024);
+  zero.add(gb2_dev, 32);
+  zero.add(gW3_dev, 128);
+  zero.add(gb3_dev, 4);
+  zero.add(grad_positions_dev, 3);
+  zero.add(grad_log_scales_dev, 3);
+  zero.add(grad_quats_dev, 4);
   if (num_chunks > 0) {
 #define MLPSP_TRAIN_VJP(KERNEL, THREADS)                                                                                \
   hipLaunchKernelGGL(KERNEL, dim3((unsigned)num_chunks), dim3(THREADS), 0, s, ix, S, chunk_steps, num_chunks, sp.records, \
                      (const float4*)d4_dev, rays_d_dev, width, height, freq_dev, att_dev, W1, b1, W2, b2, W3, scale,   \
-                     t.rows, grads, nonfinite_dev)
+                     t.rows, grads, nonfinite_dev, num_primitives, zero)
     if (precision == 0) MLPSP_TRAIN_VJP(train_vjp_f32_kernel, 64 * kVjp32Waves);
     else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>), 64 * kVjp16Waves);
     else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>), 64 * kVjp16Waves);
@@ -701,18 +723,9 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
     hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)num_chunks, 4), dim3(256), 0, s, ix, S, chunk_steps, num_chunks,
                        t.rows, quats_dev, grads, geo, nonfinite_dev);
     MLPSP_LAUNCH_CHECK();
+  } else {
+    launch_zero_rows(t.first, num_primitives, zero, s);
+    MLPSP_LAUNCH_CHECK();
   }
-  ZeroRows zero{};
-  zero.add(gW1_dev, 2304);
-  zero.add(gb1_dev, 32);
-  zero.add(gW2_dev, 1024);
-  zero.add(gb2_dev, 32);
-  zero.add(gW3_dev, 128);
-  zero.add(gb3_dev, 4);
-  zero.add(grad_positions_dev, 3);
-  zero.add(grad_log_scales_dev, 3);
-  zero.add(grad_quats_dev, 4);
-  launch_zero_rows(t.first, num_primitives, zero, s);
-  MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }

@@ -192,3 +192,26 @@ def test_weight_gradients_of_chunks_of_every_length(device, tiles, n, steps, pre
             for i, less in ((0, d1.T @ _two_parts(enc)), (0, _two_parts(d1).T @ enc), (2, d2.T @ _two_parts(h1)),
                             (2, _two_parts(d2).T @ h1)):
                 assert float((less - want[i]).norm()) > bound * float(want[i].norm()), (p, i)
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+@pytest.mark.parametrize("tiles,n", [(1, 1), (1, 7), (1, 8), (1, 33), (17, 4099), (40, 999)])
+def test_primitives_without_a_step_get_zeros(device, monkeypatch, tiles, n, precision):
+    """The wavefronts of the chunks share out the rows of all primitives, eight at a time: fewer groups than wavefronts and
+    more, a last group that is not full; every third primitive has steps."""
+    from mlp_splatting_amd import ops
+    listed = np.arange(0, min(n, 96), 3)
+    tile, prim = np.repeat(np.arange(tiles), len(listed)), np.tile(listed, tiles)
+    base, frame = _frame(device, tiles, n, tile, prim)
+    groups = ops.train_group(frame, base[6], n)
+    d4, falloff = torch.ones(frame.steps, 64, 4, device=device), torch.ones(frame.steps, 64, device=device)
+    monkeypatch.setattr(torch, "empty_like", lambda t: torch.full_like(t, float("nan")))
+    grads, flag = ops.train_gradients(frame, groups, d4, falloff, base[1], base[7], base[8], base[9:15], base[3], base[4],
+                                      precision, 1.0)
+    monkeypatch.undo()
+    without = torch.ones(n, dtype=torch.bool, device=device)
+    without[torch.from_numpy(listed).to(device)] = False
+    assert int(flag) == 0
+    for i, g in enumerate(grads):
+        assert bool(torch.isfinite(g).all()) and not bool(g[without].any()), i
+    assert bool((grads[5][~without] != 0).all())
