@@ -57,8 +57,13 @@ struct FiniteScanInputs {
   int count;
 };
 
+// Bound by memory: 2.86 GB of inputs at 200,000 primitives 481 -> 411 us, 6.95 TB/s, against a load at a time in 8,192 blocks that
+// come and go.  Eight loads on their way per thread and blocks that all run at once (512 blocks 419 us, 1,024 483, 2,048 455),
+// past the caches (471 us with 512 blocks through them).
+constexpr int kScanAhead = 8, kScanBlocks = 768;
 __global__ __launch_bounds__(256) void finite_scan_kernel(FiniteScanInputs in, int32_t* __restrict__ flag) {
-  bool bad = false;
+  uint32_t most = 0u;                // the largest of the magnitudes, as bits: 0x7f800000 and more are not finite
+  const auto look = [&](float v) { most = max(most, __float_as_uint(v) & 0x7fffffffu); };
   const long long stride = (long long)blockDim.x * gridDim.x, first = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   for (int t = 0; t < in.count; ++t) {
     const float* __restrict__ src = in.pointers[t];
@@ -67,14 +72,26 @@ __global__ __launch_bounds__(256) void finite_scan_kernel(FiniteScanInputs in, i
     const long long head = min(n, (long long)(((16 - (reinterpret_cast<uintptr_t>(src) & 15)) & 15) / 4));
     const long long quads = (n - head) / 4;
     const f32x4* __restrict__ mid = reinterpret_cast<const f32x4*>(src + head);
-    for (long long i = first; i < quads; i += stride) {
-      const f32x4 v = mid[i];
-      bad |= not_finite(v[0]) || not_finite(v[1]) || not_finite(v[2]) || not_finite(v[3]);
+    long long i = first;
+    for (; i + (kScanAhead - 1) * stride < quads; i += kScanAhead * stride) {
+      f32x4 v[kScanAhead];
+#pragma unroll
+      for (int k = 0; k < kScanAhead; ++k) v[k] = __builtin_nontemporal_load(mid + i + k * stride);
+#pragma unroll
+      for (int k = 0; k < kScanAhead; ++k) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) look(v[k][q]);
+      }
     }
-    for (long long i = first; i < head; i += stride) bad |= not_finite(src[i]);
-    for (long long i = head + 4 * quads + first; i < n; i += stride) bad |= not_finite(src[i]);
+    for (; i < quads; i += stride) {
+      const f32x4 v = mid[i];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) look(v[q]);
+    }
+    for (long long i = first; i < head; i += stride) look(src[i]);
+    for (long long i = head + 4 * quads + first; i < n; i += stride) look(src[i]);
   }
-  if (__ballot(bad) != 0ull && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
+  if (__ballot(most >= 0x7f800000u) != 0ull && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
 }
 
 template <typename T, bool EMIT>
@@ -304,7 +321,7 @@ MLPSP_API int mlpsp_all_finite(const float* const* arrays_dev, const int64_t* le
   MLPSP_HIP_TRY(clear_async(flag_dev, sizeof(int32_t), s));
   if (in.count == 0) return MLPSP_OK;
   const long long want = (largest / 4 + 255) / 256;
-  const unsigned blocks = (unsigned)(want < 1 ? 1 : (want > 8192 ? 8192 : want));
+  const unsigned blocks = (unsigned)(want < 1 ? 1 : (want > kScanBlocks ? kScanBlocks : want));
   hipLaunchKernelGGL(finite_scan_kernel, dim3(blocks), dim3(256), 0, s, in, flag_dev);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
