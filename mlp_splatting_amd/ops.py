@@ -354,7 +354,7 @@ def compact_segments(order, tile_offsets, tile_ends):
 
 def sort_tiles(rays_o, rays_d, records, candidates, tile_offsets, W, H, TW, TH, family=_lib.KEY_TSTAR,
                capacity=TILE_CAPACITY_DEFAULT, want_keys=False, cull_threshold=0.0, frame_records=None,
-               tile_pyramids=None, tile_ends=None, ids_ascend=False):
+               tile_pyramids=None, tile_ends=None, ids_ascend=False, out=None):
     """Materialised per-tile depth order: (sorted_ids [P], sorted_keys [P] | None).
 
     With ``cull_threshold`` (the render's score threshold) candidates that provably hit no ray of their
@@ -367,12 +367,13 @@ def sort_tiles(rays_o, rays_d, records, candidates, tile_offsets, W, H, TW, TH, 
     ``tile_ends``: the int32 [T] ends of lists that lie in segments (:func:`bin_segments_async`); the sorted lists
     come back in the same places, what lies between them is not written.  ``ids_ascend``: the caller vouches that
     the ids of every list ascend, as the binning entry points write them (same output, no gather of the ids at the
-    end; lists in any other order must leave it False)."""
+    end; lists in any other order must leave it False).  ``out``: an int32 tensor of the candidates' size for the sorted
+    ids."""
     dev = rays_o.device
     if tile_ends is not None and not (tile_ends.is_cuda and tile_ends.dtype == torch.int32 and tile_ends.is_contiguous()
                                       and tile_ends.numel() == tile_offsets.numel() - 1):
         raise ValueError("tile_ends must be a contiguous int32 device tensor with one entry per tile")
-    sorted_ids = torch.empty_like(candidates)
+    sorted_ids = torch.empty_like(candidates) if out is None else out
     keys = torch.empty(candidates.numel(), dtype=torch.float32, device=dev) if want_keys else None
     if candidates.numel() == 0:
         return sorted_ids, keys
@@ -481,12 +482,14 @@ def training_records(rays_o, rays_d, records, order, tile_offsets, freq, att, W1
     return rgb, alpha, ids, x6, raw, masks, gates, offsets
 
 
-def all_finite_flag(tensors):
+def all_finite_flag(tensors, flag=None):
     """int32 device flag [1]: 1 if any element of the float32 tensors (at most 16, one device) is NaN or infinite.
-    One fused scan; reading the flag is the caller's (single) synchronisation."""
+    One fused scan; reading the flag is the caller's (single) synchronisation.  ``flag``: an int32 [1] device tensor to
+    write it to."""
     tensors = [t for t in tensors if t.numel()]
     dev = tensors[0].device if tensors else torch.device("cuda", torch.cuda.current_device())
-    flag = torch.empty(1, dtype=torch.int32, device=dev)
+    if flag is None:
+        flag = torch.empty(1, dtype=torch.int32, device=dev)
     for t in tensors:
         if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == dev):
             raise RuntimeError("all_finite_flag expects contiguous float32 CUDA tensors on one device")
@@ -871,19 +874,43 @@ class TrainFrame:
         return frame
 
 
+# A frame whose lists are queued has these bytes in front of its workspace: what is read back together with the workspace's
+# first words -- the counts of the binning (int64 [4]) and the flag of the look at its inputs (int32) -- in one copy.
+_TRAIN_HEADER = 256
+
+
+class TrainBuffer:
+    """Header and workspace of a differentiable frame with room for ``pool_steps`` steps."""
+    __slots__ = ("bytes", "pairs", "pool_steps", "counts", "flag")
+
+    def __init__(self, pairs, W, H, pool_steps, device):
+        nbytes = _lib.load().mlpsp_train_workspace_bytes(int(pairs), W, H, int(pool_steps))
+        self.pairs, self.pool_steps = int(pairs), int(pool_steps)
+        self.bytes = torch.empty(_TRAIN_HEADER + nbytes, dtype=torch.uint8, device=device)
+        self.counts, self.flag = self.bytes[:32].view(torch.int64), self.bytes[32:36].view(torch.int32)
+
+
 def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W, H, threshold, max_hits, pool_steps,
-                  render_order=True, packed=None, bf16=False):
+                  render_order=True, packed=None, bf16=False, buffer=None, settle=None):
     """Forward of a differentiable frame -> (rgb, alpha, :class:`TrainFrame`); one read-back (12 bytes).  ``ws``: the six
     f32 weight tensors (exact MLP); ``packed``: their matrix-core operand copy instead.  ``pool_steps``: steps to make
-    room for; a frame that needs more is repeated once with what it asked for."""
+    room for; a frame that needs more is repeated once with what it asked for.  ``buffer``: a :class:`TrainBuffer` of
+    these sizes whose header is read back with the frame's words and given to ``settle(counts, flag)``; where that returns
+    False this returns None."""
     dev = rays_o.device
     lib = _lib.load()
     pairs, n = int(order.numel()), ws[0].shape[0]
+    if buffer is not None and (buffer.pairs, buffer.pool_steps) != (pairs, int(pool_steps)):
+        raise ValueError("the frame's buffer was made for other lists")
     rgb = torch.empty(W * H, 3, dtype=torch.float32, device=dev)
     alpha = torch.empty(W * H, 1, dtype=torch.float32, device=dev)
     for _ in range(2):
-        nbytes = lib.mlpsp_train_workspace_bytes(pairs, W, H, int(pool_steps))
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        if buffer is None:
+            nbytes = lib.mlpsp_train_workspace_bytes(pairs, W, H, int(pool_steps))
+            workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        else:
+            workspace = buffer.bytes[_TRAIN_HEADER:]
+            nbytes = workspace.numel()
         head = (_ptr(rays_o), _ptr(rays_d), _ptr(records), _ptr(order), _ptr(tile_offsets), pairs, _ptr(freq), _ptr(att))
         if packed is None:
             code = lib.mlpsp_train_forward_f32(*head, *[_ptr(w) for w in ws], n, W, H, float(threshold), int(max_hits),
@@ -894,10 +921,17 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
                                                 1 if bf16 else 0, _ptr(workspace), nbytes, _ptr(rgb), _ptr(alpha),
                                                 _stream(dev))
         _check(code, "mlpsp_train_forward")
-        chunks, status, steps = workspace[:12].view(torch.int32).tolist()
+        if buffer is None:
+            chunks, status, steps = workspace[:12].view(torch.int32).tolist()
+        else:
+            words = buffer.bytes[:_TRAIN_HEADER + 12].view(torch.int32).tolist()
+            if not settle([a & 0xffffffff | b << 32 for a, b in zip(words[0:8:2], words[1:8:2])], words[8]):
+                return None
+            chunks, status, steps = words[-3:]
         if chunks * _lib.STEP_CHUNK <= pool_steps or pool_steps < 0:
             break
         pool_steps = chunks * _lib.STEP_CHUNK
+        buffer = None
         del workspace                       # (too small: its memory is free for the next)
     else:                                   # (the walk does not depend on the room: the second asks for what the first did)
         raise RuntimeError("mlpsp_train_forward: the frame asked for more steps than it had asked for")

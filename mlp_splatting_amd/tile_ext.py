@@ -63,6 +63,16 @@ class QueuedFrame:
         self.host = self.landed = self.counts = None
 
 
+class QueuedLists:
+    """Tile lists whose binning is queued and whose counts have not been read back (:meth:`TileExt.train_lists_queued`).
+    ``again()``: the lists by way of the host.  ``pyramids``: the ray pyramids of the frame's tiles, where they are there."""
+    __slots__ = ("candidates", "offsets", "buffer", "scale", "again", "pyramids")
+
+    def __init__(self, candidates, offsets, buffer, scale, again):
+        self.candidates, self.offsets, self.buffer, self.scale, self.again = candidates, offsets, buffer, scale, again
+        self.pyramids = None
+
+
 class TileExt:
     """Forward entry points of the tile renderer on one MI355X."""
 
@@ -620,12 +630,46 @@ class TileExt:
     # a differentiable frame in training steps (no counterpart in the reference; what its record entry points, reverse
     # walk and grouped gradients compute, with the step -- tile x primitive -- as the unit of storage)
     # ------------------------------------------------------------------------------------------
+    def train_lists_queued(self, positions, log_scales, view_matrices, proj_matrix, width, height, threshold, again):
+        """The lists of a differentiable frame, queued: its binning starts while the host prepares the rest of the frame,
+        and what it counted comes back with the frame's own read-back.  A :class:`QueuedLists` for :meth:`train_forward`,
+        or None before a frame has shown how many candidates and steps there are.  ``again()`` -> (candidates, offsets)
+        by way of the host, for the frame whose estimate was too small."""
+        width, height = int(width), int(height)
+        with self._lock:
+            cap, scale, room = self._queue_capacity, self._queue_scratch_scale, self._steps_per_tile
+        if cap <= 0 or room is None or positions.shape[0] == 0:
+            return None
+        with _on_device(positions.device):
+            buffer = ops.TrainBuffer(cap, width, height, int(ops.num_tiles(width, height, 8, 8) * room), positions.device)
+            cand, offsets, _ = ops.bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, width, height, 8,
+                                                    float(threshold), cap, scratch_scale=scale, counts=buffer.counts)
+        return QueuedLists(cand, offsets, buffer, scale, again)
+
+    def _settle_lists(self, queued, counts, name):
+        """Whether queued lists are what they should be, by their counts; the estimates for the frames to come."""
+        pairs, longest, _, guard = counts
+        cap = queued.buffer.pairs
+        with self._lock:
+            if guard and pairs <= cap:
+                self._queue_scratch_scale = queued.scale * 4
+            elif pairs > 0.9 * cap:
+                self._queue_capacity = max(self._queue_capacity, int(pairs * 1.3) + 65536)
+        if guard:
+            return False
+        if longest > self.max_tile_prims:
+            raise RuntimeError(f"{name}: tile candidate capacity {self.max_tile_prims} exceeded (maximum observed tile length "
+                               f"{longest}); refusing to truncate or use an inconsistent forward/backward order")
+        return True
+
     def train_forward(self, x, width, height, threshold, *, render_order=True, precision=None,
-                      name="render_tiles_mlp_records", accept=None):
+                      name="render_tiles_mlp_records", accept=None, queued=None):
         """(rgb, alpha, ops.TrainFrame) of an 8x8-tile frame with the 72->32->32->4 MLP.  ``x``: the 15 scene tensors.
         ``precision`` None: exact f32 (with ``render_order`` the bits of ``render_tiles_forward_tilecenter``, see
         :meth:`records_forward_matches_render`); "float16" / "bfloat16": the matrix cores.  The frame's ``status`` bits
-        (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called once the lists are validated."""
+        (1 numeric, 2 hit capacity) are the caller's to judge.  ``accept``: called once the lists are validated.
+        ``queued``: the :class:`QueuedLists` of this frame, whose lists ``x`` holds; a frame that finds them too short is
+        repeated with lists by way of the host, which then stand in ``x`` (a list)."""
         width, height = int(width), int(height)
         _chk(width > 0 and height > 0 and x[0].shape[0] == width * height, "B must equal W*H for tile renderer")
         _chk(len(x) == 15, "Expected 15 scene inputs")
@@ -633,26 +677,34 @@ class TileExt:
         _chk(x[7].numel() == 6 and tuple(x[9].shape[1:]) == (32, 72), "training steps require the 72->32->32->4 MLP")
         n_tiles = ops.num_tiles(width, height, 8, 8)
         with _on_device(x[0].device), self.uncached():
-            self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
-            if accept is not None:
-                accept()
-            rec = self._records(x[2], x[3], x[4])
-            order = x[5]
-            if x[5].numel() > 0:
-                order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
-                                          self.max_tile_prims, cull_threshold=float(threshold))
-            packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
-            # Room for the steps: for the first frame as its lists suggest (a step per 13 entries at the 200,000-primitive
-            # 1200x680 frame, per three or four where primitives are small), then as the frames before needed.  A frame
-            # that needs more is repeated; the bound on what its lists can need is never exceeded.
-            with self._lock:
-                room = self._steps_per_tile
-            if room is None:
-                room = min(96.0, 0.5 * x[5].numel() / n_tiles + _lib.STEP_CHUNK)
-            pool = int(n_tiles * room)
-            rgb, alpha, frame = ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height,
-                                                  float(threshold), self.max_hits, pool, render_order=render_order,
-                                                  packed=packed, bf16=precision == "bfloat16")
+            done = None
+            if queued is not None:
+                done = self._train_forward_queued(x, n, width, height, float(threshold), render_order, precision, name, accept,
+                                                  queued)
+                if done is None:
+                    x[5:7] = queued.again()
+            if done is None:
+                self._validate(x[5], x[6], n_tiles, self.max_tile_prims, n, name)
+                if accept is not None:
+                    accept()
+                rec = self._records(x[2], x[3], x[4])
+                order = x[5]
+                if x[5].numel() > 0:
+                    order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR,
+                                              self.max_tile_prims, cull_threshold=float(threshold))
+                packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
+                # Room for the steps: for the first frame as its lists suggest (a step per 13 entries at the 200,000-primitive
+                # 1200x680 frame, per three or four where primitives are small), then as the frames before needed.  A frame
+                # that needs more is repeated; the bound on what its lists can need is never exceeded.
+                with self._lock:
+                    room = self._steps_per_tile
+                if room is None:
+                    room = min(96.0, 0.5 * x[5].numel() / n_tiles + _lib.STEP_CHUNK)
+                pool = int(n_tiles * room)
+                done = ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height,
+                                         float(threshold), self.max_hits, pool, render_order=render_order,
+                                         packed=packed, bf16=precision == "bfloat16")
+            rgb, alpha, frame = done
             needed = 1.25 * frame.chunks * _lib.STEP_CHUNK / n_tiles
             # A quarter more than was needed, a sixty-fourth less with every frame that needs less: a training set's cameras
             # come in any order, and room for the largest of them is to be there when it comes round again.
@@ -660,18 +712,51 @@ class TileExt:
                 self._steps_per_tile = max(needed, (self._steps_per_tile or 0.0) * (63 / 64))
         return rgb, alpha, frame
 
-    def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision):
+    def _train_forward_queued(self, x, n, width, height, threshold, render_order, precision, name, accept, queued):
+        """The queued half of :meth:`train_forward`: sort, packing and forward behind the binning without a look at it, and
+        everything that is to be judged read back at once.  None if the lists were too short (nothing was rendered)."""
+        _chk(x[5] is queued.candidates and x[6] is queued.offsets)
+        buffer = queued.buffer
+        judge = None if accept is None else accept(buffer.flag)
+        rec = self._records(x[2], x[3], x[4])
+        # (behind the lists' end nothing is written, and the packing looks at every entry)
+        out = None if precision is None else torch.full_like(x[5], -1)
+        order, _ = ops.sort_tiles(x[0], x[1], rec, x[5], x[6], width, height, 8, 8, _lib.KEY_TSTAR, self.max_tile_prims,
+                                  cull_threshold=threshold, tile_pyramids=queued.pyramids, ids_ascend=True, out=out)
+        packed = None if precision is None else ops.pack_mfma_weights_listed(x[9:15], order, precision == "bfloat16")
+
+        def settle(counts, flag):
+            if not self._settle_lists(queued, counts, name):
+                return False
+            if judge is not None:
+                judge(flag)
+            return True
+        return ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height, threshold, self.max_hits,
+                                 buffer.pool_steps, render_order=render_order, packed=packed, bf16=precision == "bfloat16",
+                                 buffer=buffer, settle=settle)
+
+    def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision, queued=None):
         """:meth:`train_forward` on the matrix cores under the contract and policy of
         :meth:`render_tiles_training_records_wmma`: non-finite inputs are refused, a numeric overflow discards the
         reduced-precision pass and repeats the frame in f32, hit capacity raises; same counters."""
         width, height = int(width), int(height)
         self._check_training_wmma(x, width, height, 8, threshold, beta, temp, precision)
 
-        def accept():
-            self._refuse_nonfinite(x)
+        inputs = [t for i, t in enumerate(x) if i not in (5, 6)]
+
+        def judge(flag):
+            _chk(int(flag) == 0, "Training WMMA input is nonfinite; refusing unsafe forward/fallback")
             self._count_training_mfma(0)
+
+        def accept(flag=None):
+            """A look at the inputs: judged at once, or by what is returned, with the value that ``flag`` is to hold."""
+            if flag is None:
+                judge(ops.all_finite_flag(inputs).item())
+            else:
+                ops.all_finite_flag(inputs, flag)
+            return judge
         rgb, alpha, frame = self.train_forward(x, width, height, threshold, precision=precision, accept=accept,
-                                               name="render_tiles_training_records_wmma")
+                                               name="render_tiles_training_records_wmma", queued=queued)
         if frame.status & 2:
             self._count_training_mfma(4)
             raise RuntimeError(f"Training WMMA hit capacity {self.max_hits} exceeded; refusing truncated records")
@@ -679,6 +764,8 @@ class TileExt:
             self._count_training_mfma(1)
             warnings.warn("Training WMMA numeric overflow: discarding both mixed passes and rerunning the whole "
                           "FP32 record forward")
+            if queued is not None and x[5] is queued.candidates:
+                x[5:7] = queued.again()      # (what validates lists takes no candidates behind their end)
             del frame
             rgb, alpha, frame = self.train_forward(x, width, height, threshold, render_order=False)
             self.refuse_overflow(frame)
@@ -696,7 +783,8 @@ class TileExt:
     @classmethod
     def backward_from_steps(cls, frame, groups, x, grad_rgb, grad_t, dtype=torch.float32):
         """The nine gradients of :meth:`render_tiles_backward_tilecenter_full` from a frame's steps; ``x``: the scene
-        tensors of the forward, ``groups``: ``ops.train_group`` of the frame.  Non-finite policy of
+        tensors of the forward, ``groups``: ``ops.train_group`` of the frame, or what returns it (the sort's small launches
+        then are queued while the device works on the reverse walk).  Non-finite policy of
         ``primitive_gemm.grouped_weight_gradients``."""
         from . import primitive_gemm
         # (what saved-tensor hooks hand back is a tensor of their making: it is held to the forward's contract again)
@@ -707,6 +795,8 @@ class TileExt:
                  "The image adjoints must be contiguous FP32 CUDA tensors [B, 3] and [B]")
         with _on_device(x[0].device), torch.no_grad():
             d4, falloff = ops.train_reverse(frame, x[6], grad_rgb, grad_t)
+            if callable(groups):
+                groups = groups()
 
             def launch(operand_dtype, scale):
                 return ops.train_gradients(frame, groups, d4, falloff, x[1], x[7], x[8], x[9:15], x[3], x[4],
