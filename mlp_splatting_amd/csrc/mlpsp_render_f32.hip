@@ -50,15 +50,18 @@ MLPSP_API int mlpsp_render_tilecenter_f32(const float* rays_o_dev, const float* 
 #define MLPSP_F32_ARGS                                                                                            \
   rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, \
       b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, out_t_dev, ctr, 0.f, 0.f, HitPool{}
+#define MLPSP_F32_TEAM(HT, TEAM)                                                                                     \
+  hipLaunchKernelGGL((render_team_f32_kernel<HT, 0, TEAM>), dim3(plan.grid), dim3(64 * TEAM), 0, s, MLPSP_F32_ARGS)
 #define MLPSP_F32_GO(HT)                                                                                          \
   do {                                                                                                            \
-    if (plan.twelve)                                                                                              \
-      hipLaunchKernelGGL((render_team_f32_kernel<HT, 0, 12>), dim3(plan.grid), dim3(768), 0, s, MLPSP_F32_ARGS);    \
+    if (plan.team == 12) MLPSP_F32_TEAM(HT, 12);                                                                  \
+    else if (plan.team == 8) MLPSP_F32_TEAM(HT, 8);                                                               \
+    else if (plan.team == 4) MLPSP_F32_TEAM(HT, 4);                                                               \
     else                                                                                                          \
       hipLaunchKernelGGL((render_mixed_f32_kernel<HT, 0>), dim3(plan.grid), dim3(256), 0, s, MLPSP_F32_ARGS, plan.body); \
   } while (0)
   if (use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    const PlanF32 plan = plan_f32(g, wpt, items);
+    const PlanF32 plan = plan_f32(g, wpt, items, false);
     if (hidden == 32) MLPSP_F32_GO(32);
     else MLPSP_F32_GO(16);
   }
@@ -66,6 +69,7 @@ MLPSP_API int mlpsp_render_tilecenter_f32(const float* rays_o_dev, const float* 
   else if (hidden == 16 && num_frequencies == 6) MLPSP_F32_LAUNCH(16, 6);
   else MLPSP_F32_LAUNCH(0, 0);
 #undef MLPSP_F32_GO
+#undef MLPSP_F32_TEAM
 #undef MLPSP_F32_ARGS
 #undef MLPSP_F32_LAUNCH
   MLPSP_LAUNCH_CHECK();

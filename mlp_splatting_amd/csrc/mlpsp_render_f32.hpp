@@ -408,8 +408,11 @@ __device__ __forceinline__ void render_team_item_f32(
   }
 }
 
+// Every item by a team.  Twelve wavefronts: three on a SIMD, as many as a workgroup of that size leaves room for.  Four and eight:
+// four on a SIMD, 128 registers (EMIT 0: at most twelve bytes spilled), 34 KB of LDS and less.
+constexpr int team_waves_per_simd(int team) { return team == 12 ? 3 : 4; }
 template <int HT, int EMIT, int TEAM>
-__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_team_f32_kernel(
+__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(team_waves_per_simd(TEAM), team_waves_per_simd(TEAM)))) void render_team_f32_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const float* __restrict__ freq,
     const float* __restrict__ att, const float* __restrict__ W1, const float* __restrict__ b1,
@@ -457,27 +460,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 }
 
 // Launch of `items` 64-pixel items on the matrix cores.  An evaluation keeps its SIMD's matrix core busy, so a team is a
-// multiple of four, one wavefront on each SIMD of a CU (3, 6 and 8 were slower than 4, 2 as well); twelve where the items
-// are no more than the CUs.  Else the mixed kernel with a team for each of the last 1,024 items -- for all of them up to
-// 1,280 --, which shortens the tail of the launch: what is left when the queue is empty lasts a third as long.  Frame in us,
-// one wavefront per item / teams of four / mixed: 96 items 690 / 315 (of twelve 264), 300 items hidden 16 455 / 260, 588
-// items 780 / 512, 1,200 items 1,020 / 744 / 785, 1,610 items 980 / 901 / 841, 2,214 items 1,086 / 1,070 / 985, 4,860 items
-// 1,840 / 2,128 / 1,766, 12,750 items 4,034 / 5,065 / 3,945; with 768 and 1,536 instead of 1,024 items 4,020 and 3,955.
+// multiple of four, one wavefront on each SIMD of a CU (3 and 6 were slower than 4, 2 as well): twelve where the items are no more
+// than the CUs; eight up to 640 items, two tiles to a CU and four wavefronts to a SIMD; four up to 1,920.  Above, the mixed kernel
+// with a team for each of the last 1,024 items, which shortens the tail of the launch: what is left when the queue is empty
+// lasts a third as long.  With hit records the kernels of four wavefronts to a SIMD spill 44 bytes and more: the mixed kernel from
+// 641 items on, all teams up to 1,280.  Whole frames in us (5,000 to 50,000 primitives; the mixed kernel's three wavefronts to a
+// SIMD as teams throughout below 1,280 items):
+//                 hidden 32                            hidden 16               hidden 32, feature image of 67 channels
+//      items   twelve  eight  four  mixed   items   eight  four  mixed    items   twelve  eight  four  mixed
+//        180     240    247    276     --     180     213   240     --      180     416    431   472     --
+//        272     282    261    276    280     272     211   230    230      272     460    440   463    455
+//        400     330    310    331    335     300     225   245    244      400     544    525   554    543
+//        500     499    452    472    476     588     356   364    362      500     802    765   809    789
+//        690     547    509    506    511     960     446   426    456      690   1,472  1,416 1,400  1,364
+//      1,200     796    679    687    704   1,200     476   457    474    1,344   1,264  1,149 1,154  1,163
+//      1,610     967    804    770    824   1,610     580   544    556    1,610   1,382  1,218 1,184  1,228
+//      2,016   1,134    949    935    922   2,560     793   731    706    2,016   1,625  1,430 1,378  1,381
+// 12,750 items by a wavefront each / mixed 4,034 / 3,945; with 768 and 1,536 instead of 1,024 items 4,020 and 3,955.
 // MLPSP_F32_AHEAD=0 / 1 / 2 in the environment: a wavefront per item throughout / four / twelve (comparison runs, tests).
 struct PlanF32 {
-  bool twelve;
+  int team;          // wavefronts of the kernel that gives every item a team; 0: the mixed kernel
   int body;          // workgroups per XCD with an item per wavefront (mixed kernel)
   unsigned grid;
 };
-inline PlanF32 plan_f32(const TileGeom& g, int waves_per_tile, int64_t items) {
+inline PlanF32 plan_f32(const TileGeom& g, int waves_per_tile, int64_t items, bool records) {
   const unsigned slots = superblock_grid(g.ntx, g.nty) * (unsigned)waves_per_tile;
   const char* e = getenv("MLPSP_F32_AHEAD");
   const int forced = e && e[0] >= '0' && e[0] <= '2' ? e[0] - '0' : -1;
-  if (forced == 2 || (forced < 0 && items <= 256)) return PlanF32{true, 0, slots};
+  const int team = forced == 2 || (forced < 0 && items <= 256) ? 12
+                   : forced < 0 && items <= 640               ? 8
+                   : !records && (forced == 1 || (forced < 0 && items <= 1920)) ? 4 : 0;
+  if (team != 0) return PlanF32{team, 0, slots};
   const int per_xcd = (int)(slots / kNumXcd);
   const int teams = forced == 0 ? 0 : forced == 1 || items <= 1280 ? per_xcd : min(per_xcd, 1024 / kNumXcd);
   const int body = forced == 0 ? (per_xcd + 3) / 4 : (per_xcd - teams) / 4;
-  return PlanF32{false, body, (unsigned)(kNumXcd * (body + max(0, per_xcd - 4 * body)))};
+  return PlanF32{0, body, (unsigned)(kNumXcd * (body + max(0, per_xcd - 4 * body)))};
 }
 
 // Whether the matrix-core f32 evaluation applies: the 72->32->32->4 or 72->16->16->4 shape, weight arrays that can be

@@ -186,16 +186,18 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
   rays_o_dev, rays_d_dev, (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, \
       b2, W3, b3, num_primitives, g, wpt, threshold, out_rgb_dev, out_alpha_dev, (float*)nullptr,                   \
       (unsigned long long*)nullptr, gating_beta, gating_temp, hp
+#define MLPSP_EMIT_TEAM(EM, TEAM)                                                                                   \
+  hipLaunchKernelGGL((render_team_f32_kernel<32, EM, TEAM>), dim3(plan.grid), dim3(64 * TEAM), 0, s, MLPSP_EMIT_ARGS)
 #define MLPSP_EMIT_GO(EM)                                                                                         \
   do {                                                                                                            \
-    if (plan.twelve)                                                                                              \
-      hipLaunchKernelGGL((render_team_f32_kernel<32, EM, 12>), dim3(plan.grid), dim3(768), 0, s, MLPSP_EMIT_ARGS);  \
+    if (plan.team == 12) MLPSP_EMIT_TEAM(EM, 12);                                                                 \
+    else if (plan.team == 8) MLPSP_EMIT_TEAM(EM, 8);                                                              \
     else                                                                                                          \
       hipLaunchKernelGGL((render_mixed_f32_kernel<32, EM>), dim3(plan.grid), dim3(256), 0, s, MLPSP_EMIT_ARGS, plan.body); \
   } while (0)
   const bool gated = feat_slots > 1;
   if (hidden == 32 && use_mfma32(hidden, num_frequencies, W1, b1, W2, b2)) {
-    const PlanF32 plan = plan_f32(g, wpt, items);
+    const PlanF32 plan = plan_f32(g, wpt, items, true);
     if (gated) MLPSP_EMIT_GO(2);
     else MLPSP_EMIT_GO(1);
   } else if (hidden == 32 && num_frequencies == 6) {
@@ -206,6 +208,7 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
     else MLPSP_EMIT_LAUNCH(0, 0, 1);
   }
 #undef MLPSP_EMIT_GO
+#undef MLPSP_EMIT_TEAM
 #undef MLPSP_EMIT_ARGS
 #undef MLPSP_EMIT_LAUNCH
   MLPSP_LAUNCH_CHECK();

@@ -936,3 +936,31 @@ def test_async_binning_with_device_matrices_equals_host_matrices(device, oracle_
         np.testing.assert_array_equal(off, want_off)
         np.testing.assert_array_equal(cand, want_cand)
         assert longest == int(np.diff(want_off).max())
+
+
+@pytest.mark.parametrize("hidden", [16, 32])
+@pytest.mark.parametrize("columns,rows", [(16, 16), (257, 1), (40, 16), (641, 1), (48, 40), (113, 17)])
+def test_teams_of_every_size_give_the_bits_of_a_wavefront_per_item(device, oracle_mod, monkeypatch, hidden, columns, rows):
+    """Both ends of the item counts of teams of twelve, eight and four: image, alpha, and at hidden 32 the feature image, whose
+    records the teams draw, against MLPSP_F32_AHEAD=0 (which the test above holds to the oracle); edge tiles are cut."""
+    from mlp_splatting_amd import ops
+    width, height = 8 * columns - 3, 8 * rows - 5
+    fr = Frame("cfg1_5k_160x120", n=600, hidden=hidden, width=width, height=height, feature_dim=24 if hidden == 32 else 0,
+               feature_slots=4, eye=(0.5, -0.3, -0.9))
+    sc = fr.scene
+    cand, off = fr.oracle_lists(oracle_mod)
+    rec = ops.prepare_primitives(_t(sc.positions, device), _t(sc.log_scales, device), _t(sc.quats, device))
+    ro, rd, c, o = _t(fr.rays_o, device), _t(fr.rays_d, device), _t(cand, device), _t(off, device)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8, cull_threshold=fr.thr)
+    args = [ro, rd, rec, order, o, _t(sc.freq, device), _t(sc.att, device), *[_t(w, device) for w in sc.mlp()]]
+    dims = (fr.W, fr.H, 8, 8, fr.thr)
+
+    def images():
+        out = list(ops.render_tilecenter_f32(*args, *dims, with_t=True))
+        return out + list(ops.render_tilecenter_feat_f32(*args, attributes, 1.5, 2.0, *dims)) if hidden == 32 else out
+    attributes = torch.randn(600, 4, 24, device=device, generator=torch.Generator(device=device).manual_seed(1))
+    got = images()
+    monkeypatch.setenv("MLPSP_F32_AHEAD", "0")
+    for a, b in zip(got, images()):
+        assert torch.equal(a, b)
+    assert 0.05 < float(got[1].mean())
