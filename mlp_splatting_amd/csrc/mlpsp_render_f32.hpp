@@ -462,10 +462,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // Launch of `items` 64-pixel items on the matrix cores.  An evaluation keeps its SIMD's matrix core busy, so a team is a
 // multiple of four, one wavefront on each SIMD of a CU (3 and 6 were slower than 4, 2 as well): twelve where the items are no more
 // than the CUs; eight up to 640 items, two tiles to a CU and four wavefronts to a SIMD; four up to 1,920.  Above, the mixed kernel
-// with a team for each of the last 1,024 items, which shortens the tail of the launch: what is left when the queue is empty
-// lasts a third as long.  With hit records the kernels of four wavefronts to a SIMD spill 44 bytes and more: the mixed kernel from
-// 641 items on, all teams up to 1,280.  Whole frames in us (5,000 to 50,000 primitives; the mixed kernel's three wavefronts to a
-// SIMD as teams throughout below 1,280 items):
+// with a team for each of the last items, which shortens the tail of the launch: what is left when the queue is empty lasts a
+// third as long.  With hit records the kernels of four wavefronts to a SIMD spill 44 bytes and more: the mixed kernel from
+// 641 items on.  Whole frames in us (5,000 to 50,000 primitives; the mixed kernel's three wavefronts to a
+// SIMD as teams throughout below 1,280 items, else with 1,024 teams):
 //                 hidden 32                            hidden 16               hidden 32, feature image of 67 channels
 //      items   twelve  eight  four  mixed   items   eight  four  mixed    items   twelve  eight  four  mixed
 //        180     240    247    276     --     180     213   240     --      180     416    431   472     --
@@ -476,7 +476,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 //      1,200     796    679    687    704   1,200     476   457    474    1,344   1,264  1,149 1,154  1,163
 //      1,610     967    804    770    824   1,610     580   544    556    1,610   1,382  1,218 1,184  1,228
 //      2,016   1,134    949    935    922   2,560     793   731    706    2,016   1,625  1,430 1,378  1,381
-// 12,750 items by a wavefront each / mixed 4,034 / 3,945; with 768 and 1,536 instead of 1,024 items 4,020 and 3,955.
+// How many of the last items: a CU that is ahead takes one more of them, and a wavefront's item lasts a millisecond of the four
+// that 12,750 items take.  With a wavefront per item throughout 4,034 us; with teams for the last
+//      items    1,024   1,536   2,048   2,560   3,072
+//      2,560    1,032   1,022   1,051   1,066   1,064
+//      4,860    1,780   1,733   1,765   1,799   1,809
+//      8,000    2,525   2,452   2,473   2,470   2,506
+//     12,750    3,971   3,965   3,919   3,927   3,962
+//     30,000    8,206   8,219   8,235   8,245   8,281
+// and with a feature image of 67 channels 1,523 / 1,492 / 1,507 at 2,560 items, 3,605 / 3,534 / 3,557 at 8,000.
 // MLPSP_F32_AHEAD=0 / 1 / 2 in the environment: a wavefront per item throughout / four / twelve (comparison runs, tests).
 struct PlanF32 {
   int team;          // wavefronts of the kernel that gives every item a team; 0: the mixed kernel
@@ -492,7 +500,7 @@ inline PlanF32 plan_f32(const TileGeom& g, int waves_per_tile, int64_t items, bo
                    : !records && (forced == 1 || (forced < 0 && items <= 1920)) ? 4 : 0;
   if (team != 0) return PlanF32{team, 0, slots};
   const int per_xcd = (int)(slots / kNumXcd);
-  const int teams = forced == 0 ? 0 : forced == 1 || items <= 1280 ? per_xcd : min(per_xcd, 1024 / kNumXcd);
+  const int teams = forced == 0 ? 0 : forced == 1 ? per_xcd : min(per_xcd, (items <= 8192 ? 1536 : 2048) / kNumXcd);
   const int body = forced == 0 ? (per_xcd + 3) / 4 : (per_xcd - teams) / 4;
   return PlanF32{0, body, (unsigned)(kNumXcd * (body + max(0, per_xcd - 4 * body)))};
 }

@@ -717,11 +717,18 @@ __global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4)
 #define MLPSP_RENDER_WAVES 4
 #endif
 constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
-// Tiles at the end of the launch that get a workgroup each (RGB only): as many as there are workgroups on the chip, so
-// that what is left when the queue is empty are teams, which finish a tile in a third of the time.  Frame, in us, without
-// and with it: 3,150 tiles 277 -> 266, 4,860 tiles 502 -> 479; at 12,750 tiles 661 either way.  Not where another frame
-// follows on the heels of this one: its wavefronts take the places that the last tiles leave.
-constexpr int kLastRound = 1024;
+// Tiles at the end of the launch that get a workgroup each (RGB only), as a team, which finishes a tile in a third of the time:
+// the wavefronts' tiles are long against the launch, and what a CU still has to do when the queue is empty differs by as much.
+// Not where another frame follows on the heels of this one: its wavefronts take the places that the last tiles leave.  Frame in
+// us, bf16, with teams for so many of the last tiles:
+//     tiles     none   1,024   1,536   2,048   2,560   3,072
+//     2,560      242     235     233     234     239     240
+//     3,150      265     253     258     262     268     272
+//     4,860      344     344     324     329     335     338   (fp16, threshold 1e-3: 463 / 454 / 449 / 458 / 464 / 466)
+//     8,000      439     432     428     428     427     432
+//    12,750      642     632     631     628     630     636   (fp16: 748 / 734 / 733 / 726 / 725 / 730)
+//    30,000    1,273   1,262      --   1,262      --   1,272
+inline int last_round(int64_t tiles) { return tiles < 4096 ? 1024 : tiles <= 8192 ? 1536 : 2048; }
 // MIXED: the workgroups from `body` on (per XCD) take one tile each, as a team.
 template <typename T, int SP, bool MIXED>
 __global__ __launch_bounds__(64 * kRenderWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_tilecenter_mfma_kernel(
@@ -1165,7 +1172,7 @@ void launch_mfma(dim3 grid, hipStream_t s, const float* rays_o, const float* ray
                  unsigned long long* ctr, int slots, float beta, float temp, const HitPool& hp) {
   const int per_xcd = (int)(grid.x / kNumXcd);       // slots
   int body = per_xcd / kRenderWaves;                 // workgroups with a tile per wavefront
-  if (MIXED) body = max(0, per_xcd - kLastRound / kNumXcd) / kRenderWaves;
+  if (MIXED) body = max(0, per_xcd - last_round(T) / kNumXcd) / kRenderWaves;
   hipLaunchKernelGGL((render_tilecenter_mfma_kernel<E, SP, MIXED>), dim3(kNumXcd * (body + per_xcd - body * kRenderWaves)), dim3(64 * kRenderWaves), 0, s, rays_o, rays_d,
                      (const PrimRecord*)prims, order, offsets, ends, freq, att, (const unsigned char*)packed, N, W, H, ntx,
                      body, T, thr, rgb, alpha, status, ctr, slots, beta, temp, hp);
@@ -1261,7 +1268,7 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
   // 4 / 8 wavefronts per tile: 300 tiles 187 / 161 / 150 / 142 / 130, 972 tiles 235 / 207 / 192 / 180 / 190, 1,200 tiles
   // 236 / 209 / 196 / 202 / 209, 1,610 tiles 234 / 219 / 231 / 220 / 241, 2,214 tiles 242 / 245 / 251 / 249 / 277.
   const int64_t team = 4096 / T;
-  const bool mixed = T <= 2 * 4096 && !overlapped;     // (see kLastRound)
+  const bool mixed = !overlapped;                      // (see last_round)
 #define MLPSP_MFMA_TEAM(TT, TEAM)                                                                                       \
   hipLaunchKernelGGL((render_team_mfma_kernel<TT, TEAM>), dim3(grid.x), dim3(64 * TEAM), 0, s, rays_o_dev, rays_d_dev,      \
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev, att_dev,             \
