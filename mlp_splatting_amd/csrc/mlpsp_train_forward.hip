@@ -6,8 +6,7 @@
 // Geometry, order, activations and compositing are the f32 expressions of the render (f32 MLP: its bits with
 // `render_order`, the record kernels' rounding of layer 2 without).  Bound by the MLP; the steps add 3.3 KB of contiguous
 // stores per hit step.  200,000 primitives, 1200x680, f32: 3.9 ms, against 4.0 + 6.0 of the record forward's two walks;
-// 20,000 primitives, 320x240: 0.57 ms in teams of four (five cameras; with three wavefronts to a SIMD 0.87 for one of them, and
-// 1.24 with a wavefront per tile, see train_plan).
+// 20,000 primitives, 320x240: 0.57 to 0.69 ms by camera, in teams of four (see train_plan).
 #include <type_traits>
 
 #include "mlpsp_device.hpp"
@@ -251,7 +250,8 @@ __device__ __forceinline__ void train_tile_team(const int tile, const int k, con
 // A wavefront per tile, four tiles to a workgroup, but for the last ones: the workgroups from `body` on (per XCD) take a tile
 // each, as a team.
 constexpr int kTrainTeam = 4;
-static_assert(kTrainTeam <= kStepChunk, "a round of a team begins one chunk at most");
+constexpr int kTrainLarge = 8;           // a team's wavefronts where tiles are few
+static_assert(kTrainTeam <= kStepChunk && kTrainLarge <= kStepChunk, "a round of a team begins one chunk at most");
 template <typename T, bool REC>
 __device__ __forceinline__ void train_forward_body(const TrainScene& c, const StepPool& sp, const TrainOut& out, int body) {
   union Lds {
@@ -267,6 +267,14 @@ __device__ __forceinline__ void train_forward_body(const TrainScene& c, const St
   if (alone) train_tile<T, REC>(tile, l, s.item[wave], c, sp, out);
   else train_tile_team<T, REC, kTrainTeam>(tile, wave, l, s.team, c, sp, out);
 }
+// Every tile by a team.
+template <typename T, bool REC, int TEAM>
+__device__ __forceinline__ void train_forward_teams(const TrainScene& c, const StepPool& sp, const TrainOut& out) {
+  __shared__ TrainTeamLds<T, TEAM> s;
+  const int tile = superblock_tile(blockIdx.x, c.ntx, c.nty);
+  if (tile < 0) return;
+  train_tile_team<T, REC, TEAM>(tile, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)threadIdx.x & 63, s, c, sp, out);
+}
 // (The kernels take their pointers one by one, __restrict__: as members of an argument structure the output layer's weights,
 // the same for all lanes, would be read through the vector memory path behind the stores of the steps.)
 #define MLPSP_TRAIN_PARAMS                                                                                             \
@@ -274,40 +282,52 @@ __device__ __forceinline__ void train_forward_body(const TrainScene& c, const St
       const int32_t *__restrict__ order, const int32_t *__restrict__ offsets, const float *__restrict__ freq,           \
       const float *__restrict__ att
 #define MLPSP_TRAIN_TAIL int N, int W, int H, int ntx, int nty, float thr, int max_hits, StepPool sp, TrainOut out, int body
-template <bool REC>
-__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_f32_kernel(
+// TEAM: every tile by a team of so many wavefronts; 0: most by one (train_forward_body).
+constexpr int train_workgroup(int team) { return 64 * (team == 0 ? kTrainTeam : team); }
+template <bool REC, int TEAM>
+__global__ __launch_bounds__(train_workgroup(TEAM)) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_f32_kernel(
     MLPSP_TRAIN_PARAMS, const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
     const float* __restrict__ b2, const float* __restrict__ W3, const float* __restrict__ b3, MLPSP_TRAIN_TAIL) {
   const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, W1, b1, W2, b2, W3, b3, nullptr, N, W, H, ntx, nty, thr, max_hits};
-  train_forward_body<float, REC>(c, sp, out, body);
+  if constexpr (TEAM == 0) train_forward_body<float, REC>(c, sp, out, body);
+  else train_forward_teams<float, REC, TEAM>(c, sp, out);
 }
-template <typename T>
-__global__ __launch_bounds__(64 * kTrainTeam) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_mfma_kernel(
+template <typename T, int TEAM>
+__global__ __launch_bounds__(train_workgroup(TEAM)) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_mfma_kernel(
     MLPSP_TRAIN_PARAMS, const unsigned char* __restrict__ packed, MLPSP_TRAIN_TAIL) {
   const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, packed,
                      N, W, H, ntx, nty, thr, max_hits};
-  train_forward_body<T, false>(c, sp, out, body);
+  if constexpr (TEAM == 0) train_forward_body<T, false>(c, sp, out, body);
+  else train_forward_teams<T, false, TEAM>(c, sp, out);
 }
 #undef MLPSP_TRAIN_PARAMS
 #undef MLPSP_TRAIN_TAIL
-// A team for each of the last 1,024 tiles, and for every tile of an image of up to 2,048: the launch then ends with tiles that
-// last a third as long.  Forward in us, f32 / fp16 operands, a wavefront per tile, 1,024 teams, teams throughout:
-//     300 tiles    641 / 245        294 / 125        294 / 125
-//   1,200         1,242 / 426        992 / 369        877 / 303
-//   1,530                            818 / 322        754 / 272
-//   1,900                          1,097 / 393      1,010 / 332
-//   2,214         1,194 / 424      1,049 / 361      1,093 / 370
-//   4,800         1,783 / 639      1,666 / 572      2,091 / 671
-//  12,750         4,211 / 1,356    3,977 / 1,307    5,396 / 1,695
-// 768 and 1,536 teams are within 3 % of 1,024 from 3,000 tiles on.
+// A team of eight for every tile up to 640 tiles (two workgroups to a CU), of four up to 2,048; above, teams of four for the last
+// tiles, so that a CU that is ahead can take one more of them: a wavefront's tile lasts a millisecond of the four that 12,750 take
+// in f32.  Forward in us, f32 / fp16 operands:
+//     tiles    a wavefront per tile   teams of eight    of four    for the last 1,024   1,536          2,048          2,560          3,072
+//       300       641 / 245             240 / 101      259 / 115
+//       500                             441 / 164      470 / 179
+//     1,000                             643 / 228      644 / 227
+//     1,610                             812 / 284      763 / 263
+//     2,016                             973 / 334      906 / 311
+//     2,560                           1,102 / --     1,012 / --     1,043 / 362    1,011 / 335    1,003 / 328
+//     3,150                                                         1,265 / 402    1,172 / 386    1,185 / 392    1,202 / 396    1,224 / 394
+//     4,860     1,783 / 639                                         1,855 / 574    1,708 / 532    1,719 / 537    1,759 / 547    1,770 / 544
+//     8,000                                                         2,579 / 775    2,473 / 759    2,490 / 758    2,446 / 751    2,468 / 763
+//    12,750     4,211 / 1,356                        5,396 / 1,695  4,001 / 1,181  3,984 / 1,183  3,915 / 1,179  3,906 / 1,160  3,924 / 1,173
+//    30,000                                                         8,215          8,204          8,209          8,197          8,231
 struct TrainPlan {
-  int body;
+  int team;          // wavefronts of every tile's team; 0: the mixed kernel
+  int body;          // its workgroups per XCD with a tile per wavefront
   unsigned grid;
 };
 inline TrainPlan train_plan(int ntx, int nty, int64_t T) {
-  const int per_xcd = (int)(superblock_grid(ntx, nty) / kNumXcd);
-  const int teams = T <= 2048 ? per_xcd : min(per_xcd, 1024 / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
-  return TrainPlan{body, (unsigned)(kNumXcd * (body + per_xcd - kTrainTeam * body))};
+  const unsigned slots = superblock_grid(ntx, nty);
+  if (T <= 2048) return TrainPlan{T <= 640 ? kTrainLarge : kTrainTeam, 0, slots};
+  const int per_xcd = (int)(slots / kNumXcd);
+  const int teams = min(per_xcd, (T < 2816 ? 2048 : T <= 6400 ? 1536 : 2560) / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
+  return TrainPlan{0, body, (unsigned)(kNumXcd * (body + per_xcd - kTrainTeam * body))};
 }
 
 // tile_base = exclusive sums of tile_steps, head[2] = their total; one workgroup (12,750 tiles: 6 us).
@@ -399,14 +419,21 @@ MLPSP_API int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(f.sp.head, 64 * sizeof(int32_t), s));
   const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
-#define MLPSP_TRAIN_LAUNCH(REC)                                                                                        \
-  hipLaunchKernelGGL(train_forward_f32_kernel<REC>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \
+#define MLPSP_TRAIN_TEAM(REC, TEAM)                                                                                    \
+  hipLaunchKernelGGL((train_forward_f32_kernel<REC, TEAM>), dim3(plan.grid), dim3(train_workgroup(TEAM)), 0, s, rays_o_dev, rays_d_dev, \
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev, W1, b1, W2, b2,  \
                      W3, b3, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp,                      \
                      TrainOut{out_rgb_dev, out_alpha_dev}, plan.body)
+#define MLPSP_TRAIN_LAUNCH(REC)                                    \
+  do {                                                             \
+    if (plan.team == 0) MLPSP_TRAIN_TEAM(REC, 0);                  \
+    else if (plan.team == kTrainTeam) MLPSP_TRAIN_TEAM(REC, kTrainTeam); \
+    else MLPSP_TRAIN_TEAM(REC, kTrainLarge);                       \
+  } while (0)
   if (render_order) MLPSP_TRAIN_LAUNCH(false);
   else MLPSP_TRAIN_LAUNCH(true);
 #undef MLPSP_TRAIN_LAUNCH
+#undef MLPSP_TRAIN_TEAM
   MLPSP_LAUNCH_CHECK();
   return train_scan(f, s);
 }
@@ -428,14 +455,21 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(f.sp.head, 64 * sizeof(int32_t), s));
   const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
-#define MLPSP_TRAIN_LAUNCH(T)                                                                                          \
-  hipLaunchKernelGGL(train_forward_mfma_kernel<T>, dim3(plan.grid), dim3(64 * kTrainTeam), 0, s, rays_o_dev, rays_d_dev, \
+#define MLPSP_TRAIN_TEAM(T, TEAM)                                                                                      \
+  hipLaunchKernelGGL((train_forward_mfma_kernel<T, TEAM>), dim3(plan.grid), dim3(train_workgroup(TEAM)), 0, s, rays_o_dev, rays_d_dev, \
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,                \
                      (const unsigned char*)packed_dev, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp, \
                      TrainOut{out_rgb_dev, out_alpha_dev}, plan.body)
+#define MLPSP_TRAIN_LAUNCH(T)                                      \
+  do {                                                             \
+    if (plan.team == 0) MLPSP_TRAIN_TEAM(T, 0);                    \
+    else if (plan.team == kTrainTeam) MLPSP_TRAIN_TEAM(T, kTrainTeam); \
+    else MLPSP_TRAIN_TEAM(T, kTrainLarge);                         \
+  } while (0)
   if (use_bf16) MLPSP_TRAIN_LAUNCH(__bf16);
   else MLPSP_TRAIN_LAUNCH(_Float16);
 #undef MLPSP_TRAIN_LAUNCH
+#undef MLPSP_TRAIN_TEAM
   MLPSP_LAUNCH_CHECK();
   return train_scan(f, s);
 }

@@ -435,3 +435,26 @@ def test_cameras_that_come_round_again_are_not_rendered_twice(device, oracle_mod
         if turn == 0:
             asked.clear()
     assert len(asked) == 3 * 5
+
+
+# teams of eight, of four, and most tiles by one wavefront with 2,048, 1,536 and 2,560 teams behind them
+@pytest.mark.parametrize("columns,rows", [(40, 16), (641, 1), (32, 64), (41, 50), (53, 54), (80, 81)])
+@pytest.mark.parametrize("precision", [None, "float16", "bfloat16"])
+def test_the_forward_of_every_team_size_is_that_of_the_records(device, oracle_mod, columns, rows, precision):
+    """Image and alpha bit for bit, and the number of steps, of the same frame in per-pixel records, whose walk knows no teams."""
+    import numpy as np
+    from mlp_splatting_amd.tile_ext import TileExt
+    width, height = 8 * columns - 3, 8 * rows - 5
+    fr, base = _scene(device, oracle_mod, 400, width, height, 0.6, False)
+    ext = TileExt()
+    rgb, alpha, frame = ext.train_forward(base, width, height, fr.thr, precision=precision)
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    if precision is None:
+        records = ext.render_tiles_training_records(x, width, height, 8, fr.thr, 1.5, 2.0, render_order=True)
+    else:
+        records = ext.render_tiles_training_records_wmma(x, width, height, 8, fr.thr, 1.5, 2.0, precision)
+    assert torch.equal(rgb, records[0]) and torch.equal(alpha.reshape(-1), records[1].reshape(-1))
+    offsets = records[7].cpu().numpy()
+    pixel = np.repeat(np.arange(width * height), np.diff(offsets))
+    tile = pixel // width // 8 * columns + pixel % width // 8
+    assert frame.steps == len(np.unique(tile.astype(np.int64) * 400 + records[2].cpu().numpy()))
