@@ -272,6 +272,21 @@ template <> struct RenderTable<__bf16> { static constexpr bool kUse = true; SinC
 // (feat_gemm_kernel below).
 // Register budget: 128 VGPRs, i.e. four wavefronts per SIMD (a dozen values spill; measured 4.5 % faster
 // than the 146 registers and three wavefronts the compiler picks on its own).
+// A lane's coefficients of record rs: its weight w, its gates times w in gt (none with one slot).
+template <int SP>
+__device__ __forceinline__ void store_coefficients(const HitPool& hp, int rs, int l, int p, int slots, float w, const float gt[4]) {
+  unsigned* __restrict__ coef = reinterpret_cast<unsigned*>(hp.records + (size_t)rs * hp.record_bytes);
+  if constexpr (SP == 4) {
+    const unsigned c01 = (slots > 1) ? Ops<_Float16>::pack2(gt[0], gt[1]) : Ops<_Float16>::pack2(w, 0.f);
+    const unsigned c23 = Ops<_Float16>::pack2(gt[2], gt[3]);
+    *reinterpret_cast<uint2*>(coef + l * 2) = make_uint2(c01, c23);
+  } else {
+    const u32x4 c = {Ops<_Float16>::pack2(w, gt[0]), Ops<_Float16>::pack2(gt[1], gt[2]),
+                     Ops<_Float16>::pack2(gt[3], 0.f), 0u};
+    *reinterpret_cast<u32x4*>(coef + l * 4) = c;
+  }
+  if (l == 0) hp.hit_ids[rs] = p;
+}
 // One tile, rendered by the calling wavefront (lane l = pixel l of the tile); s_dir: LDS of this wavefront alone.
 template <typename T, int SP>
 __device__ __forceinline__ void render_tile_mfma(
@@ -442,19 +457,7 @@ __device__ __forceinline__ void render_tile_mfma(
             else fast_tetra_gates<true>(w, h.qlx, h.qly, h.qlz, k, gate_t, gt);
           }
           const int rs = hit_emitter_next(hp, em, l);
-          if (rs >= 0) {
-            unsigned* __restrict__ coef = reinterpret_cast<unsigned*>(hp.records + (size_t)rs * hp.record_bytes);
-            if constexpr (SP == 4) {
-              const unsigned c01 = (slots > 1) ? Ops<_Float16>::pack2(gt[0], gt[1]) : Ops<_Float16>::pack2(w, 0.f);
-              const unsigned c23 = Ops<_Float16>::pack2(gt[2], gt[3]);
-              *reinterpret_cast<uint2*>(coef + l * 2) = make_uint2(c01, c23);
-            } else {
-              const u32x4 c = {Ops<_Float16>::pack2(w, gt[0]), Ops<_Float16>::pack2(gt[1], gt[2]),
-                               Ops<_Float16>::pack2(gt[3], 0.f), 0u};
-              *reinterpret_cast<u32x4*>(coef + l * 4) = c;
-            }
-            if (l == 0) hp.hit_ids[rs] = p;
-          }
+          if (rs >= 0) store_coefficients<SP>(hp, rs, l, p, slots, w, gt);
         }
         live = in_image & __ballot(acc.trans >= kTransmittanceFloor);
         if (live == 0ull) {
@@ -496,7 +499,9 @@ __device__ __forceinline__ void render_tile_mfma(
 // chain, with the chip mostly idle.  320x240, 20,000 primitives, bf16: 166 -> 127 us with three wavefronts per tile (all of
 // them resident); then the SIMDs' issue slots are two thirds busy and the rest is the spread of the tiles.  Requesting the
 // next entry's weights a round ahead changes nothing there.  The price is the second pass over the opacities and up to
-// TEAM - 1 entries evaluated behind the last one that counts.
+// TEAM - 1 entries evaluated behind the last one that counts.  With the records of a feature image, whose slots the team draws
+// together: bf16 feature frame of 300 tiles 266 -> 190 us, 500 334 -> 237, 1,200 372 -> 327, 1,610 350 -> 330, 4,860 569 -> 550,
+// 12,750 1,443 -> 1,435.
 // ---------------------------------------------------------------------------------------------
 template <int TEAM>
 struct TeamRound {
@@ -504,23 +509,26 @@ struct TeamRound {
   float colour[TEAM - 1][3][64];      // of wavefronts 1..: wavefront 0 has its own in registers
 };
 
-template <int TEAM>
+template <int SP, int TEAM>
 struct TeamLds {
   DirWords dir;
-  OriginLds<0> org;
+  OriginLds<SP> org;
   TeamRound<TEAM> round[2];
+  unsigned long long mask[2][SP > 0 ? TEAM : 1];      // lanes that hit a wavefront's entry
+  int chunk;                                          // (team_slot)
 };
 
-template <typename T, int TEAM>
+// SP as in render_tile_mfma: each wavefront writes the record of its own entry.
+template <typename T, int SP, int TEAM>
 __device__ __forceinline__ void render_tile_team(
-    const int tile, const int k, const int l, TeamLds<TEAM>& lds, const SinCosTable* table, const float* __restrict__ rays_o,
+    const int tile, const int k, const int l, TeamLds<SP, TEAM>& lds, const SinCosTable* table, const float* __restrict__ rays_o,
     const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims, const int32_t* __restrict__ order,
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends, const float* __restrict__ freq,
     const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W, int H, int ntx, float thr,
     float* __restrict__ out_rgb, float* __restrict__ out_alpha, int32_t* __restrict__ status,
-    unsigned long long* __restrict__ counters) {
+    unsigned long long* __restrict__ counters, int slots, float beta, float temp, const HitPool& hp) {
   DirWords& s_dir = lds.dir;
-  OriginLds<0>& s_org = lds.org;
+  OriginLds<SP>& s_org = lds.org;
   TeamRound<TEAM>(&s_round)[2] = lds.round;
   float kf[3];
   phase_scales(freq, att, l >> 5, kf);
@@ -551,7 +559,9 @@ __device__ __forceinline__ void render_tile_team(
               oz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(roz), lane0));
   const float reach = 4e-6f * __builtin_sqrtf(fmaxf(-2.f * __logf(thr), 0.f));
   const bool one_origin = __ballot(valid && !(rox == ox && roy == oy && roz == oz)) == 0ull;
+  const float gate_t = temp * 1.44269504f;
   const int start = offsets[tile], end = ends[tile];
+  TeamSlots em{(start >> 4) + tile, 0, 0, 0, 0};
   float trans = 1.f, cr = 0.f, cg = 0.f, cb = 0.f;
   unsigned long long live = in_image;
   int buf = 0;
@@ -568,6 +578,13 @@ __device__ __forceinline__ void render_tile_team(
       *reinterpret_cast<f32x4*>(&s_org.e[l][0]) = f32x4{o.vx, o.vy, o.vz, o.vlx};
       *reinterpret_cast<f32x4*>(&s_org.e[l][4]) = f32x4{o.vly, o.vlz, thr - band_for(o, thr, reach), thr + band_for(o, thr, reach)};
     }
+    if constexpr (SP > 0) {
+      if (slots > 1 && l % TEAM == k && id_lane >= 0 && id_lane < N) {
+        const PrimRecord& P = prims[id_lane];
+        *reinterpret_cast<f32x4*>(&s_org.e[l][8]) =
+            f32x4{gate_t * gate_factor(P.lgx, beta), gate_t * gate_factor(P.lgy, beta), gate_t * gate_factor(P.lgz, beta), 0.f};
+      }
+    }
     const int rounds = ((int)__builtin_popcountll(todo) + TEAM - 1) / TEAM;
     for (int i = 0; i < k; ++i) todo &= todo - 1ull;
     FastRegs q;
@@ -579,8 +596,9 @@ __device__ __forceinline__ void render_tile_team(
     }
     team_barrier();
     for (int r = 0; r < rounds; ++r) {
-      float keep = 1.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+      float keep = 1.f, o[4] = {0.f, 0.f, 0.f, 0.f}, ql[3] = {0.f, 0.f, 0.f};
       unsigned long long mask = 0ull, hit_bad = 0ull, mlp_bad = 0ull;     // mlp_bad: of any lane's pixel
+      const int j_now = j, p_now = p;
       const bool mine = todo != 0ull;
       if (mine) {
         const FastRec R = fast_arrived(q);
@@ -601,8 +619,13 @@ __device__ __forceinline__ void render_tile_team(
         HitInfo h;
         const HitMasks test = hit_fast(ot, rdx, rdy, rdz, R.r, thr_lo, thr_hi, h);
         mask = test.hit & live;
+        if constexpr (SP > 0) {
+          ql[0] = h.qlx;
+          ql[1] = h.qly;
+          ql[2] = h.qlz;
+          asm volatile("" : "+v"(ql[0]), "+v"(ql[1]), "+v"(ql[2]));
+        }
         asm volatile("" : "+v"(h.dx), "+v"(h.dy), "+v"(h.dz), "+v"(h.decay));   // R is used up here
-        const int p_now = p;
 #pragma unroll
         for (int i = 0; i < TEAM; ++i) todo &= todo - 1ull;
         if (todo != 0ull) {
@@ -638,7 +661,13 @@ __device__ __forceinline__ void render_tile_team(
         }
       }
       TeamRound<TEAM>& round = s_round[buf];
+      const unsigned long long* const s_mask = lds.mask[buf];
+      if constexpr (SP > 0) {
+        if (l == 0) lds.mask[buf][k] = mask;
+      }
       buf ^= 1;
+      int kept = 0, rank = -1;
+      float w_mine = 0.f;
       round.keep[k][l] = keep;
       if (k > 0) {
 #pragma unroll
@@ -655,6 +684,16 @@ __device__ __forceinline__ void render_tile_team(
           bad |= (blended & hit_bad) | (blended != 0ull ? mlp_bad : 0ull);
           n_proc_hit += blended != 0ull;
           n_hits += __popcll(blended);
+          if constexpr (SP > 0) {
+            rank = blended != 0ull ? kept : -1;
+            w_mine = lane_in(blended) ? fmaf(-trans, keep, trans) : 0.f;
+          }
+        }
+        if constexpr (SP > 0) {
+          const unsigned long long m = s_mask[i];
+          const unsigned long long um = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)m) |
+                                        ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32);
+          kept += (um & open) != 0ull;
         }
         if (lane_in(open)) {
           if (k == 0) {
@@ -664,6 +703,18 @@ __device__ __forceinline__ void render_tile_team(
             cb = fmaf(w, i == 0 ? o[2] : round.colour[i > 0 ? i - 1 : 0][2][l], cb);
           }
           trans = trans * let;
+        }
+      }
+      if constexpr (SP > 0) {
+        const int rs = team_slot<HitGroups, true>(em, kept, rank, k, l, hp.counters, hp.chunk_table, hp.pool_chunks, lds.chunk);
+        if (rs >= 0) {
+          float gt[4] = {0.f, 0.f, 0.f, 0.f};       // w times the gates
+          if (slots > 1) {
+            const f32x4 factors = *reinterpret_cast<const f32x4*>(&s_org.e[j_now][8]);
+            if (__builtin_fabsf(gate_t) <= kGateExponents) fast_tetra_gates<false>(w_mine, ql[0], ql[1], ql[2], factors, gate_t, gt);
+            else fast_tetra_gates<true>(w_mine, ql[0], ql[1], ql[2], factors, gate_t, gt);
+          }
+          store_coefficients<SP>(hp, rs, l, p_now, slots, w_mine, gt);
         }
       }
       live = in_image & __ballot(trans >= kTransmittanceFloor);
@@ -679,6 +730,9 @@ __device__ __forceinline__ void render_tile_team(
     store3(out_rgb, pix, cr, cg, cb);
     out_alpha[pix] = 1.f - trans;
   }
+  if constexpr (SP > 0) {
+    if (k == 0 && l == 0) hp.item_hits[tile] = em.count;
+  }
   // (a NaN among the outputs of a hit, which the largest of them does not show)
   bad |= __ballot(!(__builtin_fabsf((cr + cg) + (cb + trans)) <= 3.4028235e38f));
   if (bad != 0ull && l == 0) atomicExch(status, 1);
@@ -690,14 +744,14 @@ __device__ __forceinline__ void render_tile_team(
 }
 
 // Every tile by a team of TEAM wavefronts.
-template <typename T, int TEAM>
+template <typename T, int SP, int TEAM>
 __global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_team_mfma_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const int32_t* __restrict__ order, const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends,
     const float* __restrict__ freq, const float* __restrict__ att, const unsigned char* __restrict__ packed, int N, int W,
     int H, int ntx, int num_tiles, float thr, float* __restrict__ out_rgb, float* __restrict__ out_alpha,
-    int32_t* __restrict__ status, unsigned long long* __restrict__ counters) {
-  __shared__ __attribute__((aligned(16))) TeamLds<TEAM> lds;
+    int32_t* __restrict__ status, unsigned long long* __restrict__ counters, int slots, float beta, float temp, HitPool hp) {
+  __shared__ __attribute__((aligned(16))) TeamLds<SP, TEAM> lds;
   __shared__ RenderTable<T> s_table;
   const int tile = superblock_tile(blockIdx.x, ntx, num_tiles / ntx);
   if (tile < 0) return;
@@ -706,9 +760,9 @@ __global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4)
     fill_sincos_table<T>(s_table.t);
     table = &s_table.t;
   }
-  render_tile_team<T, TEAM>(tile, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)threadIdx.x & 63, lds, table,
-                            rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr, out_rgb,
-                            out_alpha, status, counters);
+  render_tile_team<T, SP, TEAM>(tile, __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), (int)threadIdx.x & 63, lds, table,
+                                rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr, out_rgb,
+                                out_alpha, status, counters, slots, beta, temp, hp);
 }
 
 // Four wavefronts = four tiles per workgroup: they share nothing but the sin/cos table, which they fill together
@@ -717,7 +771,7 @@ __global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4)
 #define MLPSP_RENDER_WAVES 4
 #endif
 constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
-// Tiles at the end of the launch that get a workgroup each (RGB only), as a team, which finishes a tile in a third of the time:
+// Tiles at the end of the launch that get a workgroup each, as a team, which finishes a tile in a third of the time:
 // the wavefronts' tiles are long against the launch, and what a CU still has to do when the queue is empty differs by as much.
 // Not where another frame follows on the heels of this one: its wavefronts take the places that the last tiles leave.  Frame in
 // us, bf16, with teams for so many of the last tiles:
@@ -728,6 +782,7 @@ constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
 //     8,000      439     432     428     428     427     432
 //    12,750      642     632     631     628     630     636   (fp16: 748 / 734 / 733 / 726 / 725 / 730)
 //    30,000    1,273   1,262      --   1,262      --   1,272
+// (The renders with feature records have the same tail.)
 inline int last_round(int64_t tiles) { return tiles < 4096 ? 1024 : tiles <= 8192 ? 1536 : 2048; }
 // MIXED: the workgroups from `body` on (per XCD) take one tile each, as a team.
 template <typename T, int SP, bool MIXED>
@@ -746,7 +801,7 @@ __global__ __launch_bounds__(64 * kRenderWaves) __attribute__((amdgpu_waves_per_
   struct NoTeam {};
   union Lds {
     TileLds tiles;
-    typename std::conditional<MIXED, TeamLds<kRenderWaves>, NoTeam>::type team;
+    typename std::conditional<MIXED, TeamLds<SP, kRenderWaves>, NoTeam>::type team;
   };
   __shared__ __attribute__((aligned(16))) Lds lds;
   DirWords(&s_dir)[kRenderWaves] = lds.tiles.dir;
@@ -765,9 +820,9 @@ __global__ __launch_bounds__(64 * kRenderWaves) __attribute__((amdgpu_waves_per_
     if (unit >= body) {
       const int tile = superblock_tile_of(xcd, body * kRenderWaves + (unit - body), ntx, num_tiles / ntx);
       if (tile >= 0)
-        render_tile_team<T, kRenderWaves>(tile, __builtin_amdgcn_readfirstlane(wave), (int)threadIdx.x & 63, lds.team, table,
-                                          rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr,
-                                          out_rgb, out_alpha, status, counters);
+        render_tile_team<T, SP, kRenderWaves>(tile, __builtin_amdgcn_readfirstlane(wave), (int)threadIdx.x & 63, lds.team, table,
+                                              rays_o, rays_d, prims, order, offsets, ends, freq, att, packed, N, W, H, ntx, thr,
+                                              out_rgb, out_alpha, status, counters, slots, beta, temp, hp);
       return;
     }
   }
@@ -1269,25 +1324,29 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
   // 236 / 209 / 196 / 202 / 209, 1,610 tiles 234 / 219 / 231 / 220 / 241, 2,214 tiles 242 / 245 / 251 / 249 / 277.
   const int64_t team = 4096 / T;
   const bool mixed = !overlapped;                      // (see last_round)
-#define MLPSP_MFMA_TEAM(TT, TEAM)                                                                                       \
-  hipLaunchKernelGGL((render_team_mfma_kernel<TT, TEAM>), dim3(grid.x), dim3(64 * TEAM), 0, s, rays_o_dev, rays_d_dev,      \
+#define MLPSP_MFMA_TEAM(TT, SP, TEAM)                                                                                   \
+  hipLaunchKernelGGL((render_team_mfma_kernel<TT, SP, TEAM>), dim3(grid.x), dim3(64 * TEAM), 0, s, rays_o_dev, rays_d_dev,      \
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev, att_dev,             \
                      (const unsigned char*)packed_dev, num_primitives, width, height, ntx, (int)T, threshold, out_rgb_dev,  \
-                     out_alpha_dev, status_dev, ctr)
+                     out_alpha_dev, status_dev, ctr, feat_slots, gating_beta, gating_temp, hp)
 #define MLPSP_MFMA_GO(TT, SP, MIXED)                                                                              \
   launch_mfma<TT, SP, MIXED>(grid, s, rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, ends, freq_dev,   \
                       att_dev, packed_dev, num_primitives, width, height, ntx, (int)T, threshold,                 \
                       out_rgb_dev, out_alpha_dev, status_dev, ctr, feat_slots, gating_beta, gating_temp, hp)
-#define MLPSP_MFMA_SP(TT)                 \
-  do {                                    \
-    if (sp == 0 && team >= 8) MLPSP_MFMA_TEAM(TT, 8); \
-    else if (sp == 0 && team >= 4) MLPSP_MFMA_TEAM(TT, 4); \
-    else if (sp == 0 && team == 3) MLPSP_MFMA_TEAM(TT, 3); \
-    else if (sp == 0 && team == 2) MLPSP_MFMA_TEAM(TT, 2); \
-    else if (sp == 0 && mixed) MLPSP_MFMA_GO(TT, 0, true); \
-    else if (sp == 0) MLPSP_MFMA_GO(TT, 0, false); \
-    else if (sp == 4) MLPSP_MFMA_GO(TT, 4, false); \
-    else MLPSP_MFMA_GO(TT, 8, false);            \
+#define MLPSP_MFMA_SIZE(TT, SP)                           \
+  do {                                                    \
+    if (team >= 8) MLPSP_MFMA_TEAM(TT, SP, 8);            \
+    else if (team >= 4) MLPSP_MFMA_TEAM(TT, SP, 4);       \
+    else if (team == 3) MLPSP_MFMA_TEAM(TT, SP, 3);       \
+    else if (team == 2) MLPSP_MFMA_TEAM(TT, SP, 2);       \
+    else if (mixed) MLPSP_MFMA_GO(TT, SP, true);          \
+    else MLPSP_MFMA_GO(TT, SP, false);                    \
+  } while (0)
+#define MLPSP_MFMA_SP(TT)                     \
+  do {                                        \
+    if (sp == 0) MLPSP_MFMA_SIZE(TT, 0);      \
+    else if (sp == 4) MLPSP_MFMA_SIZE(TT, 4); \
+    else MLPSP_MFMA_SIZE(TT, 8);              \
   } while (0)
   if (stage != 2) {
     if (use_bf16) MLPSP_MFMA_SP(__bf16);
@@ -1295,6 +1354,8 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
     MLPSP_LAUNCH_CHECK();
   }
 #undef MLPSP_MFMA_SP
+#undef MLPSP_MFMA_SIZE
+#undef MLPSP_MFMA_TEAM
 #undef MLPSP_MFMA_GO
   if (sp != 0 && stage != 1) {
     const dim3 ggrid(superblock_grid(ntx, ceil_div(height, 8)), (unsigned)ceil_div(feat_channels, 128 * kGemmNcb)), gblock(256);

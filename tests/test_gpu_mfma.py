@@ -423,3 +423,33 @@ def test_outputs_beyond_f32_are_reported(device, oracle_mod, width, height, row,
     b2[:] = 10.0                       # every hidden unit is active
     W3[:, row] = value if value is not None else np.where(np.arange(32) % 3, 3e38, -3e38)
     assert render()
+
+
+@pytest.mark.parametrize("columns,rows", [(20, 15), (32, 32), (35, 35), (45, 40), (60, 40)])
+@pytest.mark.parametrize("slots,bf16", [(4, True), (5, False), (1, True)])
+def test_feature_frames_of_every_team_size_are_those_of_a_wavefront_per_tile(device, oracle_mod, columns, rows, slots, bf16):
+    """Teams of eight, four, three and two, and of four for the last tiles: image, alpha and feature image bit for bit those of
+    the same tiles at the top of an image whose last tiles, which are empty, take the teams."""
+    from mlp_splatting_amd import ops
+    width, height, channels, extra = 8 * columns, 8 * rows, 40, 8 * (9000 // columns)
+    fr = Frame("cfg1_5k_160x120", n=1200, hidden=32, width=width, height=height, feature_dim=channels, feature_slots=slots)
+    sc = fr.scene
+    cand, off = fr.oracle_lists(oracle_mod)
+    rec = ops.prepare_primitives(*[to_dev(a, device) for a in (sc.positions, sc.log_scales, sc.quats)])
+    mlp = [to_dev(a, device) for a in (sc.freq, sc.att, *sc.mlp())]
+    shape = (1200, channels) if slots == 1 else (1200, slots, channels)
+    attributes = torch.randn(*shape, device=device, generator=torch.Generator(device=device).manual_seed(2))
+
+    def images(more):
+        pad = lambda a: to_dev(np.concatenate([a, np.repeat(a[:1], more * width, 0)]), device)
+        ro, rd = pad(fr.rays_o), pad(fr.rays_d)
+        offsets = to_dev(np.concatenate([off, np.full(more // 8 * columns, off[-1], off.dtype)]), device)
+        order, _ = ops.sort_tiles(ro, rd, rec, to_dev(cand, device), offsets, width, height + more, 8, 8, cull_threshold=fr.thr)
+        rgb, alpha, feat, bad = ops.render_tilecenter_mfma_feat(ro, rd, rec, order, offsets, *mlp, attributes, 1.5, 2.0, width,
+                                                                height + more, fr.thr, bf16=bf16)
+        assert not bad
+        return [t[:width * height] for t in (rgb, alpha, feat)]
+    got, want = images(0), images(extra)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert float(got[1].mean()) > 0.05 and float(got[2].abs().max()) > 0.1
