@@ -964,3 +964,28 @@ def test_teams_of_every_size_give_the_bits_of_a_wavefront_per_item(device, oracl
     for a, b in zip(got, images()):
         assert torch.equal(a, b)
     assert 0.05 < float(got[1].mean())
+
+
+@pytest.mark.parametrize("tile", [8, 16])
+def test_a_feature_frame_whose_record_pool_ran_out_is_repeated(device, oracle_mod, monkeypatch, tile):
+    """With the first pool too small, by choice: the image of the frame that had room, from the exact and the matrix-core render."""
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=600, hidden=32, width=61, height=43, tile=tile, feature_dim=24, feature_slots=4)
+    sc = fr.scene
+    cand, off = fr.oracle_lists(oracle_mod)
+    rec = ops.prepare_primitives(_t(sc.positions, device), _t(sc.log_scales, device), _t(sc.quats, device))
+    ro, rd, c, o = _t(fr.rays_o, device), _t(fr.rays_d, device), _t(cand, device), _t(off, device)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, tile, tile, cull_threshold=fr.thr)
+    args = [ro, rd, rec, order, o, _t(sc.freq, device), _t(sc.att, device), *[_t(w, device) for w in sc.mlp()],
+            _t(sc.feat_attr, device), 1.5, 2.0, fr.W, fr.H]
+
+    def images():
+        out = list(ops.render_tilecenter_feat_f32(*args, tile, tile, fr.thr))
+        return out + list(ops.render_tilecenter_mfma_feat(*args, fr.thr)[:3]) if tile == 8 else out
+    assert ops._feat_pool_sizes(1000, 2048) == (-1,) and len(ops._feat_pool_sizes(1 << 23, 512)) == 2
+    want = images()
+    tried = []
+    monkeypatch.setattr(ops, "_feat_pool_sizes", lambda *_a: tried.append(1) or (64, -1))
+    for a, b in zip(images(), want):
+        assert torch.equal(a, b)
+    assert len(tried) == (2 if tile == 8 else 1) and float(want[1].mean()) > 0.05
