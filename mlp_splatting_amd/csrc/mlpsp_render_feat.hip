@@ -8,7 +8,7 @@
 //      the primitives that hit and per pixel the weight w and the four gates (hit records,
 //      mlpsp_hitrec.hpp): float[K][64] with K = 5 (w, g0..g3) or 1 (w), w = -1 where the primitive missed;
 //   2. feat_accumulate_kernel turns the roles around: lane = channel.  A 256-thread block owns one
-//      64-pixel item, a wavefront 128 channels of 32 or 16 of its pixels.  Per record the attribute rows
+//      64-pixel item, a wavefront up to 128 channels of 32 or 16 of its pixels.  Per record the attribute rows
 //      are two coalesced loads per slot, the per-pixel weight and gates are wave-uniform scalar operands, a
 //      pixel the primitive missed costs one scalar branch, and every output row is written exactly once.
 #include "mlpsp_device.hpp"
@@ -21,17 +21,35 @@ namespace mlpsp {
 
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-// SLOTS = 1, 4 or 5; mix as np_tile_kernels.cu:6037-6070.  PX: pixels per wavefront, 16 or 32; 64 / PX wavefronts share
-// 128 channels.  Bound by latency: a record is its slot, then its rows and weights, then two to ten operations per hit.
+// The mix of a primitive's attribute rows r by a pixel's gates g (np_tile_kernels.cu:6037-6070).
+template <int SLOTS>
+__device__ __forceinline__ float feat_mix(const float r[SLOTS], float g0, float g1, float g2, float g3) {
+  if constexpr (SLOTS == 1) return r[0];
+  constexpr int k = SLOTS == 5 ? 1 : 0;
+  float m = SLOTS == 5 ? fmaf(g0, r[k], r[0]) : fmaf(g0, r[k], 0.f);
+  m = fmaf(g1, r[k + 1], m);
+  m = fmaf(g2, r[k + 2], m);
+  return fmaf(g3, r[k + 3], m);
+}
+
+// SLOTS = 1, 4 or 5.  PX: pixels per wavefront, 16 or 32; 64 / PX wavefronts share
+// 128 channels.  Bound by latency and, with wave-uniform weights and gates (an operand out of a scalar register costs an
+// instruction twice its time), by the two to ten operations per hit and 64 channels.
 // Few pixels per wavefront mean more wavefronts (all four of a block have channels at 128 already) on smaller
 // accumulators (58 to 73 registers at 16 pixels, 150 at 64), at the price of fetching the rows 64 / PX times.
 // 333x251, 30,000 primitives, 67 channels: 433 us with 64 pixels and one slot fetch per record, 187 us with 16.
 // Fetching the next record's rows ahead gained nothing at either size.
-template <int SLOTS, int PX>
+//
+// HALVES: 64 channels or 128.  TAIL (64 channels, 16 pixels): the up to 4 TAIL channels behind them, with a lane's 4 TAIL-th of
+// the wavefront for each of 16 / TAIL pixels at a time, TAIL times: the few channels of a ragged count then cost a few
+// operations per hit and not as many as the first 64 (67 channels as above: 146 us; in the frame no channel count below 81
+// is slower than with 128 of them reckoned, and 81 or more have no such form).
+template <int SLOTS, int PX, int HALVES, int TAIL>
 __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __restrict__ feat_attr, int C, HitPool hp,
                                                               const int32_t* __restrict__ offsets, TileGeom g,
                                                               int waves_per_tile, float* __restrict__ out_feat) {
-  constexpr int kShare = 64 / PX;
+  static_assert(TAIL == 0 || (HALVES == 1 && PX == 16 && (TAIL == 1 || TAIL == 2 || TAIL == 4)), "a tail of up to 16 channels");
+  constexpr int kShare = 64 / PX, kTailChannels = 4 * TAIL, kTailPixels = TAIL ? 16 / TAIL : 0;
   // (the render's mapping: what a tile's wavefront wrote lies in this XCD's L2)
   const int unit = (int)(blockIdx.x / kNumXcd), wslot = unit % waves_per_tile;
   const int tile = superblock_tile_of((int)(blockIdx.x % kNumXcd), unit / waves_per_tile, g.ntx, g.nty);
@@ -42,12 +60,19 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
   const int hits = hp.item_hits[tile * waves_per_tile + wslot];
   const int table_base = wslot * hp.table_stride + (offsets[tile] >> 4) + tile;
   const int ca = c0 + l, cb = c0 + 64 + l;
-  const bool has_a = ca < C, has_b = cb < C;
+  const bool has_a = ca < C, has_b = HALVES == 2 && cb < C;
+  const int ct = c0 + 64 + (TAIL ? l % (TAIL ? kTailChannels : 1) : 0), tail_px = TAIL ? l / (TAIL ? kTailChannels : 1) : 0;
+  const bool has_t = TAIL > 0 && ct < C;
   constexpr bool GATED = SLOTS > 1;
 
-  float acc[PX][2];
+  float acc[PX][HALVES], tail[TAIL ? TAIL : 1];
 #pragma unroll
-  for (int px = 0; px < PX; ++px) acc[px][0] = acc[px][1] = 0.f;
+  for (int px = 0; px < PX; ++px) {
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) acc[px][h] = 0.f;
+  }
+#pragma unroll
+  for (int q = 0; q < TAIL; ++q) tail[q] = 0.f;
 
   int slots = 0, ids = 0;               // of 64 records, one per lane
   for (int m = 0; m < hits; ++m) {
@@ -57,13 +82,22 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
     }
     const int rs = __builtin_amdgcn_readlane(slots, m & 63), p = __builtin_amdgcn_readlane(ids, m & 63);
     const float* __restrict__ rows = feat_attr + (size_t)p * SLOTS * C;
-    float ra[SLOTS], rb[SLOTS];
+    float ra[SLOTS], rb[SLOTS], rt[SLOTS];
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s) {
       ra[s] = has_a ? rows[(size_t)s * C + ca] : 0.f;
       rb[s] = has_b ? rows[(size_t)s * C + cb] : 0.f;
+      rt[s] = has_t ? rows[(size_t)s * C + ct] : 0.f;
     }
     const float* __restrict__ rec = reinterpret_cast<const float*>(hp.records + (size_t)rs * hp.record_bytes) + px0;
+    float wt[TAIL ? TAIL : 1], gt[TAIL ? TAIL : 1][4];
+#pragma unroll
+    for (int q = 0; q < TAIL; ++q) {
+      const int px = q * kTailPixels + tail_px;
+      wt[q] = rec[px];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) gt[q][k] = GATED ? rec[64 * (k + 1) + px] : 0.f;
+    }
     // weights and gates of 8 pixels at a time: wave-uniform 32-byte scalar loads, issued unconditionally
     // so that their latency overlaps the previous group's arithmetic
 #pragma unroll
@@ -79,49 +113,38 @@ __global__ __launch_bounds__(256) void feat_accumulate_kernel(const float* __res
         const int px = 8 * q + j;
         const float w = w8[j];
         if (w >= 0.f) {
-          float ma, mb;
-          if constexpr (SLOTS == 1) {
-            ma = ra[0];
-            mb = rb[0];
-          } else {
-            const float g0 = g8[0][j], g1 = g8[1][j], g2 = g8[2][j], g3 = g8[3][j];
-            if constexpr (SLOTS == 4) {
-              ma = fmaf(g0, ra[0], 0.f);
-              mb = fmaf(g0, rb[0], 0.f);
-              ma = fmaf(g1, ra[1], ma);
-              mb = fmaf(g1, rb[1], mb);
-              ma = fmaf(g2, ra[2], ma);
-              mb = fmaf(g2, rb[2], mb);
-              ma = fmaf(g3, ra[3], ma);
-              mb = fmaf(g3, rb[3], mb);
-            } else {
-              ma = fmaf(g0, ra[1], ra[0]);
-              mb = fmaf(g0, rb[1], rb[0]);
-              ma = fmaf(g1, ra[2], ma);
-              mb = fmaf(g1, rb[2], mb);
-              ma = fmaf(g2, ra[3], ma);
-              mb = fmaf(g2, rb[3], mb);
-              ma = fmaf(g3, ra[4], ma);
-              mb = fmaf(g3, rb[4], mb);
-            }
-          }
-          acc[px][0] = fmaf(w, ma, acc[px][0]);
-          acc[px][1] = fmaf(w, mb, acc[px][1]);
+          acc[px][0] = fmaf(w, feat_mix<SLOTS>(ra, g8[0][j], g8[1][j], g8[2][j], g8[3][j]), acc[px][0]);
+          if constexpr (HALVES == 2)
+            acc[px][1] = fmaf(w, feat_mix<SLOTS>(rb, g8[0][j], g8[1][j], g8[2][j], g8[3][j]), acc[px][1]);
         }
       }
+    }
+#pragma unroll
+    for (int q = 0; q < TAIL; ++q) {
+      const float v = fmaf(wt[q], feat_mix<SLOTS>(rt, gt[q][0], gt[q][1], gt[q][2], gt[q][3]), tail[q]);
+      tail[q] = wt[q] >= 0.f ? v : tail[q];
     }
   }
 
   const int tx = tile % g.ntx, ty = tile / g.ntx;
-#pragma unroll
-  for (int px = 0; px < PX; ++px) {
+  const auto row = [&](int px) -> float* {          // a pixel's row of the image, null outside
     const int slot = wslot * 64 + px0 + px;
     const int x = tx * g.TW + slot % g.TW, y = ty * g.TH + slot / g.TW;
-    if (slot < g.TW * g.TH && x < g.W && y < g.H) {
-      float* __restrict__ dst = out_feat + (size_t)(y * g.W + x) * C;
+    return slot < g.TW * g.TH && x < g.W && y < g.H ? out_feat + (size_t)(y * g.W + x) * C : nullptr;
+  };
+#pragma unroll
+  for (int px = 0; px < PX; ++px) {
+    if (float* __restrict__ dst = row(px)) {
       if (has_a) dst[ca] = acc[px][0];
-      if (has_b) dst[cb] = acc[px][1];
+      if constexpr (HALVES == 2) {
+        if (has_b) dst[cb] = acc[px][1];
+      }
     }
+  }
+#pragma unroll
+  for (int q = 0; q < TAIL; ++q) {
+    float* __restrict__ dst = row(q * kTailPixels + tail_px);
+    if (dst && has_t) dst[ct] = tail[q];
   }
 }
 
@@ -212,8 +235,8 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
 #undef MLPSP_EMIT_ARGS
 #undef MLPSP_EMIT_LAUNCH
   MLPSP_LAUNCH_CHECK();
-#define MLPSP_ACC_LAUNCH(SL, PX)                                                                                    \
-  hipLaunchKernelGGL((feat_accumulate_kernel<SL, PX>), dim3(superblock_grid(g.ntx, g.nty) * (unsigned)wpt,            \
+#define MLPSP_ACC_LAUNCH(SL, PX, HALVES, TAIL)                                                                      \
+  hipLaunchKernelGGL((feat_accumulate_kernel<SL, PX, HALVES, TAIL>), dim3(superblock_grid(g.ntx, g.nty) * (unsigned)wpt,            \
                      (unsigned)ceil_div(feat_channels, 8 * PX)), dim3(256), 0, s, feat_attr_dev, feat_channels, hp,   \
                      tile_offsets_dev, g, wpt, out_feat_dev)
   // 16 pixels per wavefront unless the rows are long and the launch fills the chip anyway: four times the wavefronts for
@@ -227,13 +250,23 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
   //   12,750   5,408 / 5,678  5,464 / 5,659  6,602 / 6,404  6,667 / 6,380  7,847 / 7,722  8,970 / 8,389
   // (384 channels are one and a half of the 256 that a workgroup of 32-pixel wavefronts takes.)
   const bool sixteen = feat_channels <= 128 || items <= 3072;
-  if (feat_slots == 4) {
-    if (sixteen) MLPSP_ACC_LAUNCH(4, 16); else MLPSP_ACC_LAUNCH(4, 32);
-  } else if (feat_slots == 5) {
-    if (sixteen) MLPSP_ACC_LAUNCH(5, 16); else MLPSP_ACC_LAUNCH(5, 32);
-  } else {
-    if (sixteen) MLPSP_ACC_LAUNCH(1, 16); else MLPSP_ACC_LAUNCH(1, 32);
-  }
+  // Up to 80 channels reckon only those that there are (in fours behind the 64th).  Whole frame of 333x251 and 30,000
+  // primitives in us, 128 channels reckoned / as here (96 channels, the same kernel on both sides: 962 / 962):
+  //    16 channels   957 / 914      40   960 / 909      64   959 / 915      67   961 / 922      72   960 / 926      80   960 / 930
+  //    800x640 and 100,000:  33   3,506 / 3,452      70   3,510 / 3,314
+#define MLPSP_ACC_GO(SL)                                          \
+  do {                                                            \
+    if (!sixteen) MLPSP_ACC_LAUNCH(SL, 32, 2, 0);                 \
+    else if (feat_channels <= 64) MLPSP_ACC_LAUNCH(SL, 16, 1, 0); \
+    else if (feat_channels <= 68) MLPSP_ACC_LAUNCH(SL, 16, 1, 1); \
+    else if (feat_channels <= 72) MLPSP_ACC_LAUNCH(SL, 16, 1, 2); \
+    else if (feat_channels <= 80) MLPSP_ACC_LAUNCH(SL, 16, 1, 4); \
+    else MLPSP_ACC_LAUNCH(SL, 16, 2, 0);                          \
+  } while (0)
+  if (feat_slots == 4) MLPSP_ACC_GO(4);
+  else if (feat_slots == 5) MLPSP_ACC_GO(5);
+  else MLPSP_ACC_GO(1);
+#undef MLPSP_ACC_GO
 #undef MLPSP_ACC_LAUNCH
   MLPSP_LAUNCH_CHECK();
   // status_dev[0] = 1 if the record pool was too small (the feature image is then incomplete)

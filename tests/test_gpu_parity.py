@@ -770,6 +770,28 @@ def test_feature_pixels_per_wavefront_give_the_same_bits(device, oracle_mod, slo
         _assert_bits(whole[:, first:first + 100], feature(fa[..., first:first + 100]), "feat")
 
 
+@pytest.mark.parametrize("slots", [1, 4, 5])
+def test_feature_channels_behind_the_64th_give_the_same_bits(device, oracle_mod, slots):
+    """Up to 80 channels take kernels that reckon 64 and 0, 4, 8 or 16 more; 81 and more reckon all 128."""
+    from mlp_splatting_amd import ops
+    fr = Frame("cfg1_5k_160x120", n=900, width=93, height=61, feature_dim=96, feature_slots=max(slots, 4))
+    sc = fr.scene
+    fa = sc.feat_attr if slots > 1 else np.ascontiguousarray(sc.feat_attr[:, 0])
+    cand, off = fr.oracle_lists(oracle_mod)
+    rec = ops.prepare_primitives(_t(sc.positions, device), _t(sc.log_scales, device), _t(sc.quats, device))
+    ro, rd, c, o = _t(fr.rays_o, device), _t(fr.rays_d, device), _t(cand, device), _t(off, device)
+    order, _ = ops.sort_tiles(ro, rd, rec, c, o, fr.W, fr.H, 8, 8)
+
+    def feature(rows):
+        return ops.render_tilecenter_feat_f32(ro, rd, rec, order, o, _t(sc.freq, device), _t(sc.att, device),
+                                              *[_t(w, device) for w in sc.mlp()], _t(np.ascontiguousarray(rows), device),
+                                              1.3, 2.2, fr.W, fr.H, 8, 8, fr.thr)[2].cpu().numpy()
+    whole = feature(fa)
+    assert np.abs(whole[..., 60:]).max() > 1e-3
+    for channels in (1, 63, 64, 65, 68, 69, 72, 73, 80, 81):
+        _assert_bits(whole[..., :channels], feature(fa[..., :channels]), f"{channels} channels")
+
+
 @pytest.mark.parametrize("with_feat", [False, True])
 def test_per_pixel_render_is_bit_exact(device, oracle_mod, with_feat):
     from mlp_splatting_amd import ops
