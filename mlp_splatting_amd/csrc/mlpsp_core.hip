@@ -155,8 +155,17 @@ __global__ __launch_bounds__(256) void frame_prologue_kernel(const float* __rest
 // PYR: the tiles' ray pyramids come from records (the frame prologue's) instead of being built here.
 // Tile t's list is cand[offsets[t] .. ends[t]) (ends = offsets + 1 for lists that follow one another without gaps).
 // ASC: the ids of every list ascend (sort_one_tile_from).
+// Bound by its vector instructions, two thirds of them the face test and the key of a candidate.  Eight wavefronts per SIMD
+// (seven where the ids are looked up again) hide the gather of a round's records better than asking for them a round
+// ahead did with six (200,000 primitives, 1200x680, lists of 560; all calls by events):
+//   a vote and a barrier per round, survivors compacted in LDS, a permutation and an order beside them (27 KB)   95 us
+//   keys in registers, one sum of all votes, words laid out by bucket, ranks straight to the output (19 KB)      86
+//   ... and records asked for in their own round, eight wavefronts per SIMD                                      80
+//   ... and sums and ranges in the operands of the additions instead of through LDS, culled entries counted alone 75
+//   ... and the pyramid in vector registers, out of LDS every round                                              71
+// 641x479, 50,000 primitives: 46 -> 36; 800x450, 100,000: 51 -> 39; 2400x1360 without records of the pyramids: 138 -> 108.
 template <bool PYR, bool ASC = false>
-__global__ __launch_bounds__(kSortThreads) void sort_tiles_kernel(
+__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(ASC ? 8 : 7))) void sort_tiles_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,
     const SortRec* __restrict__ frame, const TilePyramidRec* __restrict__ pyramids, const int32_t* __restrict__ cand,
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ ends, TileGeom g, int family, int capacity,

@@ -10,7 +10,7 @@ namespace mlpsp {
 // 64-bit word (key bits << 32 | list index): keys are positive floats, whose bit patterns order
 // like their values, and the list index in the low word makes equal keys keep list order, which
 // is what a stable radix sort on the key alone yields.  The words are ordered in LDS: normally by a
-// counting pass into 256 key buckets followed by ranking inside each bucket, else (keys piled up in few
+// counting pass into 512 key buckets followed by ranking inside each bucket, else (keys piled up in few
 // buckets) by a bitonic network on the next power of two, padded with all-ones words.
 //
 // Optional conservative culling (cull_threshold in (0,1)): a candidate list comes from a bounding
@@ -28,19 +28,52 @@ namespace mlpsp {
 constexpr int kSortThreads = 256;
 constexpr int kRankPairsMax = 64 * 1024;   // in-bucket comparisons beyond which the sorting network is used instead
 
-// The workgroup's LDS for one tile's sort (27 KB at 2048 entries, 14 KB at 1024).
+// Lane l's sum of the first l + 1 lanes' words (the first 32 lanes', with HALF), and the smallest and the largest word of a
+// wavefront in its last lane: in the operands of the additions themselves, not through LDS with an address per step.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t from_lane(uint32_t otherwise, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)otherwise, (int)x, CTRL, ROWS, 0xf, false);
+}
+template <bool HALF>
+__device__ __forceinline__ uint32_t sum_up_to_lane(uint32_t x) {
+  x += from_lane<0x111, 0xf>(0u, x);                     // row_shr:1, 2, 4, 8: within 16 lanes
+  x += from_lane<0x112, 0xf>(0u, x);
+  x += from_lane<0x114, 0xf>(0u, x);
+  x += from_lane<0x118, 0xf>(0u, x);
+  x += from_lane<0x142, 0xa>(0u, x);                     // row_bcast:15 into rows 1 and 3
+  if constexpr (!HALF) x += from_lane<0x143, 0xc>(0u, x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ void range_in_last_lane(uint32_t& lo, uint32_t& hi) {
+#define MLPSP_RANGE_STEP(CTRL, ROWS)                 \
+  lo = min(lo, from_lane<CTRL, ROWS>(0xffffffffu, lo)); \
+  hi = max(hi, from_lane<CTRL, ROWS>(0u, hi))
+  MLPSP_RANGE_STEP(0x111, 0xf);
+  MLPSP_RANGE_STEP(0x112, 0xf);
+  MLPSP_RANGE_STEP(0x114, 0xf);
+  MLPSP_RANGE_STEP(0x118, 0xf);
+  MLPSP_RANGE_STEP(0x142, 0xa);
+  MLPSP_RANGE_STEP(0x143, 0xc);
+#undef MLPSP_RANGE_STEP
+}
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {      // of the mask's lanes, those before this one
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// The workgroup's LDS for one tile's sort (18.9 KB at 2048 entries).
 template <int kSortMax>
 struct SortLds {
   // a power of two: the sorting network pads a list to the next power of two inside key[]; a multiple of the
-  // workgroup: every thread handles kSortMax / kSortThreads entries; perm[] and order[] hold 16-bit positions
-  static_assert((kSortMax & (kSortMax - 1)) == 0 && kSortMax % kSortThreads == 0 && kSortMax <= 65536,
+  // workgroup: every thread handles kSortMax / kSortThreads entries, and one wavefront adds up all kSortMax / 64 votes;
+  // counts and offsets of the buckets are 16-bit halves
+  static_assert((kSortMax & (kSortMax - 1)) == 0 && kSortMax % kSortThreads == 0 && kSortMax <= 4096,
                 "capacity of the in-LDS tile sort");
   unsigned long long key[kSortMax];
-  int wave_cnt[2][kSortThreads / 64];
-  int cnt[kSortThreads], off[kSortThreads];
-  uint16_t perm[kSortMax], order[kSortMax];
-  uint32_t kmin, kmax;
-  int flags, pairs;
+  int2 bucket[kSortThreads];               // of two buckets each: offsets, counts
+  uint32_t vote[kSortMax / 64];                // [round][wavefront]: ordinary survivors | late ones << 16
+  uint32_t lo[kSortThreads / 64], hi[kSortThreads / 64];
+  uint32_t sum[kSortThreads / 64], pairs[kSortThreads / 64];
+  float4 pyramid[kSortThreads / 64][4];    // each wavefront's own: four normals, origin, faces (TilePyramidRec's words)
 };
 
 // Per-frame, per-primitive record of the sort (64 bytes, one cache line per candidate): what the key and the culling
@@ -263,6 +296,16 @@ struct alignas(32) TilePyramidRec {
   float unused[24];        // (the record's size is part of the C ABI)
 };
 static_assert(sizeof(TilePyramidRec) == MLPSP_TILE_PYRAMID_BYTES, "record size");
+__device__ __forceinline__ void pyramid_to_pieces(const TilePyramid& py, float4* to) {
+  to[0] = make_float4(py.n[0][0], py.n[0][1], py.n[0][2], py.n[1][0]);
+  to[1] = make_float4(py.n[1][1], py.n[1][2], py.n[2][0], py.n[2][1]);
+  to[2] = make_float4(py.n[2][2], py.n[3][0], py.n[3][1], py.n[3][2]);
+  to[3] = make_float4(py.ox, py.oy, py.oz, bits_to_float((uint32_t)py.faces));
+}
+__device__ __forceinline__ TilePyramid pyramid_from_pieces(const float4* from) {
+  const float4 a = from[0], b = from[1], c = from[2], d = from[3];
+  return TilePyramid{d.x, d.y, d.z, {{a.x, a.y, a.z}, {a.w, b.x, b.y}, {b.z, b.w, c.x}, {c.y, c.z, c.w}}, (int)float_to_bits(d.w)};
+}
 // One wavefront per tile; `raw` are the directions before normalisation.
 __device__ __forceinline__ void write_tile_pyramid(const float* __restrict__ rays_o, const float* __restrict__ raw,
                                                    const TileGeom& g, int tile, TilePyramidRec* __restrict__ out) {
@@ -271,11 +314,7 @@ __device__ __forceinline__ void write_tile_pyramid(const float* __restrict__ ray
   RawDirs{raw}.get(pc, dx, dy, dz);
   const TilePyramid py = tile_pyramid(rays_o, RawDirs{raw}, g, tile, dx, dy, dz);
   if ((threadIdx.x & 63) == 0) {
-    float4* to = reinterpret_cast<float4*>(out + tile);
-    to[0] = make_float4(py.n[0][0], py.n[0][1], py.n[0][2], py.n[1][0]);
-    to[1] = make_float4(py.n[1][1], py.n[1][2], py.n[2][0], py.n[2][1]);
-    to[2] = make_float4(py.n[2][2], py.n[3][0], py.n[3][1], py.n[3][2]);
-    to[3] = make_float4(py.ox, py.oy, py.oz, bits_to_float((uint32_t)py.faces));
+    pyramid_to_pieces(py, reinterpret_cast<float4*>(out + tile));
   }
 }
 // A record as a wavefront holds it: lane j has word j (one coalesced load), and the words are taken out of that
@@ -480,215 +519,188 @@ __device__ __forceinline__ void sort_one_tile_from(SortLds<kSortMax>& lds, const
     float cull_r2, int num_prims, int32_t* __restrict__ sorted_ids, float* __restrict__ sorted_keys, int start, int len,
     int n) {
   auto& s_key = lds.key;
-  auto& s_wave_cnt = lds.wave_cnt;
-  auto& s_cnt = lds.cnt;
-  auto& s_off = lds.off;
-  auto& s_perm = lds.perm;
-  auto& s_order = lds.order;
-  auto& s_kmin = lds.kmin;
-  auto& s_kmax = lds.kmax;
-  auto& s_flags = lds.flags;
-  auto& s_pairs = lds.pairs;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // (the wavefront's index as a scalar)
 
   // Every candidate id this thread will handle is requested up front (at most kSortMax / kSortThreads of them),
-  // and the first round's geometry record right behind; each round of the key loop then requests the next round's
-  // record.  An id outside [0, num_prims) (lists that were never validated) reads record 0, is never culled and
+  // and the first round's geometry record right behind.  An id outside [0, num_prims) (lists that were never validated) reads record 0, is never culled and
   // sorts last with the invalid key; it is passed on unchanged, and the render kernels skip it.
   constexpr int kRounds = kSortMax / kSortThreads;
   int my_id[kRounds];
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) my_id[r] = (tid + r * kSortThreads < n) ? cand[start + tid + r * kSortThreads] : 0;
-  typename Source::Rec P_buf[2];                         // this round's record and the next round's
-  P_buf[0] = src.load(((unsigned)my_id[0] < (unsigned)num_prims) ? my_id[0] : 0);
+  typename Source::Rec P = src.load(((unsigned)my_id[0] < (unsigned)num_prims) ? my_id[0] : 0);
 
   // ---- the tile's ray pyramid (only when culling is requested), while those loads are on their way: every
-  //      wavefront builds it for itself -- four faces among its lanes, one ray of the tile per lane -- so no barrier
-  //      is needed for the verdict
-  // (PYR is a compile-time choice: with both forms behind one run-time branch, or with the record read as sixteen
-  // scalar words, the compiler keeps the pyramid in vector registers for the candidate loop -- 96 registers instead of
-  // 72 and a wavefront less per SIMD.  A record therefore arrives in ONE vector register, a word per lane, and the
-  // sixteen words the face test needs are taken out of it with v_readlane: they are scalar operands of its
-  // multiply-adds and stay in scalar registers over the rounds.)
-  TilePyramid py = {};
-  float pyramid_word = 0.f;
+  //      wavefront has its own in LDS -- from the record, or built with four faces among its lanes and one ray of the
+  //      tile per lane -- so no barrier is needed, and reads it there every round.  (Out of LDS it arrives in vector
+  //      registers: an operand out of a scalar register costs the multiply-adds of the face test twice their time, and
+  //      kept over the rounds the words cost a wavefront or three per SIMD.  12,750 tiles, lists of 560: words in
+  //      scalar registers, from v_readlane every round, 76 us; out of LDS every round 72; kept 80.)
   int faces = 0;
   if (cull_r2 > 0.f) {
     if constexpr (PYR) {
-      pyramid_word = pyramid_record_word(pyramids + tile);
-      faces = (int)float_to_bits(lane_value(pyramid_word, 15));
+      const float word = pyramid_record_word(pyramids + tile);
+      faces = (int)float_to_bits(lane_value(word, 15));
+      if (lane < 16) reinterpret_cast<float*>(lds.pyramid[wave])[lane] = word;
     } else {
-      py = tile_pyramid(rays_o, UnitDirs{rays_d}, g, tile, dx, dy, dz);
-      faces = py.faces;
+      const TilePyramid built = tile_pyramid(rays_o, UnitDirs{rays_d}, g, tile, dx, dy, dz);
+      faces = built.faces;
+      if (lane == 0) pyramid_to_pieces(built, lds.pyramid[wave]);
     }
   }
 
-  // ---- keys.  Survivors with an ordinary key are compacted to the front of s_key in list order; survivors
-  //      whose key is the invalid key or larger go to the back of s_key, last slot first (the "late" stream: all
-  //      of them normally carry the invalid key, and a stable sort leaves those in list order after everything
-  //      else); culled entries are written straight to the end of the tile's output, last one first.
+  // ---- keys, kept in registers: what is culled and what lies past the list carries a word above every key's bits.
+  //      A round ends in a vote on each wavefront's survivors, ordinary and late ones (key at or above the invalid
+  //      key: normally all of them carry that very key), and nothing waits between the rounds.
+  constexpr uint32_t kNoEntry = 0xfffffffeu, kCulled = 0xffffffffu;
+  constexpr int kWaves = kSortThreads / 64;
   const uint32_t invalid_bits = float_to_bits(kInvalidKey);
-  if (tid == 0) {
-    s_kmin = 0xffffffffu;
-    s_kmax = 0u;
-    s_flags = 0;
-    s_pairs = 0;
-  }
-  // ordinary survivors so far in the low half, late ones in the high half (block-uniform; a list holds at most
-  // kSortMax <= 65,535 entries, so the halves never carry into each other): one sum serves both streams
-  int survivors = 0;
+  uint32_t kb[kRounds];
   uint32_t key_lo = 0xffffffffu, key_hi = 0u;
-  bool odd_late = false;
+  unsigned long long odd_late = 0ull;
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
-    if (r * kSortThreads >= n) break;
-    const int round = r & 1;
+    kb[r] = kNoEntry;
+    if (r * kSortThreads >= n) continue;
     const int i = r * kSortThreads + tid;
-    bool keep = false, outside = false;
-    float key = 0.f;
-    const typename Source::Rec& P = P_buf[r & 1];
     const int p = my_id[r];
-    if (r + 1 < kRounds && i + kSortThreads < n)
-      P_buf[(r + 1) & 1] = src.load(((unsigned)my_id[r + 1] < (unsigned)num_prims) ? my_id[r + 1] : 0);
+    if (r > 0) P = src.load(((unsigned)p < (unsigned)num_prims) ? p : 0);
     const bool known = (unsigned)p < (unsigned)num_prims;
-    if constexpr (PYR) py = pyramid_from_word(pyramid_word);
+    // (read anew every round: the fence keeps the sixteen words from taking registers across the rounds)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    TilePyramid py = pyramid_from_pieces(lds.pyramid[wave]);
+    py.faces = faces;
     if (i < n) {
-      outside = faces && known && outside_pyramid(py, P, cull_r2);
-      keep = !outside;
-      if (keep) key = !known ? kInvalidKey : src.key(family, dx, dy, dz, P);
+      const bool outside = faces && known && outside_pyramid(py, P, cull_r2);
+      kb[r] = outside ? kCulled : float_to_bits(!known ? kInvalidKey : src.key(family, dx, dy, dz, P));
     }
-    const uint32_t kb = float_to_bits(key);
-    const bool late = keep && kb >= invalid_bits;
-    const bool front = keep && !late;
-    // (the builtin on the predicates themselves: __ballot() takes an int, and the predicate's way through a
-    // register and back is two vector instructions per vote)
-    const unsigned long long mf = __builtin_amdgcn_ballot_w64(front), ml = __builtin_amdgcn_ballot_w64(late);
-    if (lane == 0) s_wave_cnt[round][wave] = __popcll(mf) | (__popcll(ml) << 16);
-    __syncthreads();                                     // (the two count buffers alternate: one barrier per round)
-    int before = survivors, total = 0;
-#pragma unroll
-    for (int v = 0; v < kSortThreads / 64; ++v) {
-      const int c = __builtin_amdgcn_readfirstlane(s_wave_cnt[round][v]);     // (the same word in every lane)
-      before += (v < wave) ? c : 0;
-      total += c;
-    }
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const int f_before = (before & 0xffff) + __popcll(mf & below);
-    const int l_before = (before >> 16) + __popcll(ml & below);
-    const unsigned long long entry = ((unsigned long long)kb << 32) | (unsigned)(ASC ? p : i);
-    if (front) {
-      s_key[f_before] = entry;
-    } else if (late) {
-      s_key[kSortMax - 1 - l_before] = entry;
-    } else if (i < n) {
-      const int pos = start + n - 1 - (i - (f_before + l_before));
-      sorted_ids[pos] = ~p;
-      if (sorted_keys) sorted_keys[pos] = kInvalidKey;
-    }
-    // range of the ordinary keys (per lane here, combined after the loop), and whether any late key is not the
-    // invalid key itself
-    key_lo = front ? min(key_lo, kb) : key_lo;
-    key_hi = front ? max(key_hi, kb) : key_hi;
-    odd_late |= late && kb != invalid_bits;
-    survivors += total;
+    // (the builtin on the comparisons themselves: a vote on more takes the predicate through a register and back)
+    const unsigned long long front = __builtin_amdgcn_ballot_w64(kb[r] < invalid_bits),
+                             in_order = __builtin_amdgcn_ballot_w64(kb[r] <= invalid_bits),
+                             kept = __builtin_amdgcn_ballot_w64(kb[r] < kNoEntry);
+    if (lane == 0) lds.vote[r * kWaves + wave] = (uint32_t)(__popcll(front) | (__popcll(kept & ~front) << 16));
+    // range of the ordinary keys, and whether any late key is not the invalid key itself
+    key_lo = min(key_lo, kb[r]);
+    key_hi = max(key_hi, kb[r] < invalid_bits ? kb[r] : 0u);
+    odd_late |= kept & ~in_order;
   }
-  int nv = survivors & 0xffff, nl = survivors >> 16;
-  {
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-      key_lo = min(key_lo, (uint32_t)__shfl_xor((int)key_lo, d));
-      key_hi = max(key_hi, (uint32_t)__shfl_xor((int)key_hi, d));
-    }
-    if (lane == 0) {                                     // one pair of LDS atomics per wavefront
-      atomicMin(&s_kmin, key_lo);
-      atomicMax(&s_kmax, key_hi);
-    }
-    if (__ballot(odd_late) && lane == 0) atomicOr(&s_flags, 1);
+  range_in_last_lane(key_lo, key_hi);
+  if (lane == 63) {
+    lds.lo[wave] = key_lo;
+    lds.hi[wave] = odd_late ? kCulled : key_hi;
   }
+  lds.bucket[tid] = make_int2(0, 0);
   __syncthreads();
 
+  // survivors before each round's share of this wavefront (a list holds at most kSortMax <= 4096 entries, so the halves
+  // never carry into each other): one sum serves both streams
+  static_assert(kRounds * kWaves == 32 || kRounds * kWaves == 64, "a lane for every vote");
+  constexpr bool kHalf = kRounds * kWaves == 32;
+  const uint32_t own_vote = lane < kWaves * ((n + kSortThreads - 1) / kSortThreads) ? lds.vote[lane] : 0u;
+  const uint32_t upto = sum_up_to_lane<kHalf>(own_vote), before_all = upto - own_vote;
+  const uint32_t survivors = (uint32_t)__builtin_amdgcn_readlane((int)upto, kHalf ? 31 : 63);
+  int nv = (int)(survivors & 0xffffu);
+  const int nl = (int)(survivors >> 16);
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+#pragma unroll
+  for (int v = 0; v < kWaves; ++v) {                     // (the same words in every lane)
+    kmin = min(kmin, (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.lo[v]));
+    kmax = max(kmax, (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.hi[v]));
+  }
+  const bool odd = kmax == kCulled;
+
   // ---- order of the ordinary survivors.  Usual case: a counting pass into 512 buckets that are linear in the
-  //      key bits between the smallest and the largest key (monotone, so bucket order is key order), then every
-  //      entry ranks itself among the entries of its own bucket by its (key, list position) word.  The work of
-  //      that last step is the sum of the squared bucket sizes; when keys pile up in few buckets (or a late key
-  //      is not the invalid key, which the late stream's list order would misplace) the bitonic network below
-  //      sorts instead.
-  // (two buckets per thread: their counts, offsets and cursors are 16-bit halves of one word -- a list holds at
-  // most kSortMax <= 65,535 entries, so a half never carries into its neighbour)
+  //      key bits between the smallest and the largest key (monotone, so bucket order is key order), the words laid out
+  //      bucket by bucket, then every entry ranks itself among those of its own bucket and goes straight to its place in
+  //      the output.  The work of that last step is the sum of the squared bucket sizes; when keys pile up in few buckets
+  //      (or a late key is not the invalid key, so that the late ones are no longer in order as they stand) the
+  //      bitonic network below sorts instead.
+  // (two buckets per thread: their counts and offsets are 16-bit halves of one word)
   constexpr int kBuckets = 2 * kSortThreads;
-  const uint32_t kmin = s_kmin;
-  const float bucket_scale = (float)kBuckets / ((float)(s_kmax - kmin) + 1.f);
-  auto bucket_of = [&](unsigned long long w) {
-    const int b = (int)((float)((uint32_t)(w >> 32) - kmin) * bucket_scale);
+  const float bucket_scale = (float)kBuckets * __builtin_amdgcn_rcpf((float)(kmax - kmin) + 1.f);
+  auto bucket_of = [&](uint32_t bits) {
+    const int b = (int)((float)(bits - kmin) * bucket_scale);
     return b < kBuckets - 1 ? b : kBuckets - 1;
   };
   auto half_of = [](int word, int b) { return (word >> ((b & 1) << 4)) & 0xffff; };
   auto one_in = [](int b) { return 1 << ((b & 1) << 4); };
-  bool network = (s_flags & 1) != 0;
-  const bool ranked = !network && nv > 1;
-  if (ranked) {
-    s_cnt[tid] = 0;
-    __syncthreads();
-    for (int i = tid; i < nv; i += kSortThreads) {
-      const int b = bucket_of(s_key[i]);
-      atomicAdd(&s_cnt[b >> 1], one_in(b));
+  bool network = odd;
+  int at[kRounds];                                       // an ordinary entry's bucket and its number in there
+  auto out = [&](int pos, int id, float key) {
+    sorted_ids[start + pos] = id;
+    if (sorted_keys) sorted_keys[start + pos] = key;
+  };
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    at[r] = 0;
+    if (r * kSortThreads >= n) continue;
+    const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)before_all, r * kWaves + wave);
+    if (kb[r] < invalid_bits && !network) {
+      const int b = bucket_of(kb[r]);
+      at[r] = b | (half_of(atomicAdd(&lds.bucket[b >> 1].y, one_in(b)), b) << 16);
     }
-    __syncthreads();
-    const int c0 = s_cnt[tid] & 0xffff, c1 = (s_cnt[tid] >> 16) & 0xffff;
-    const int c = c0 + c1;
-    int incl = c, pairs = c0 * c0 + c1 * c1;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d);
-      if (lane >= d) incl += up;
-    }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) pairs += __shfl_xor(pairs, d);
-    if (lane == 63) s_wave_cnt[0][wave] = incl;
-    if (lane == 0) atomicAdd(&s_pairs, pairs);
-    __syncthreads();
-    int base = 0;
-#pragma unroll
-    for (int v = 0; v < kSortThreads / 64; ++v) base += (v < wave) ? s_wave_cnt[0][v] : 0;
-    const int excl = base + incl - c;
-    s_off[tid] = excl | ((excl + c0) << 16);
-    s_cnt[tid] = excl | ((excl + c0) << 16);             // from here on: the buckets' fill cursors
-    network = s_pairs > kRankPairsMax;
-    __syncthreads();
-    if (!network) {
-      for (int i = tid; i < nv; i += kSortThreads) {
-        const int b = bucket_of(s_key[i]);
-        s_perm[half_of(atomicAdd(&s_cnt[b >> 1], one_in(b)), b)] = (uint16_t)i;
-      }
-      __syncthreads();
-      for (int a = tid; a < nv; a += kSortThreads) {
-        const int ia = s_perm[a];
-        const unsigned long long wa = s_key[ia];
-        const int b = bucket_of(wa);
-        const int lo = half_of(s_off[b >> 1], b), hi = half_of(s_cnt[b >> 1], b);   // the cursor ended at the bucket's end
-        int r = 0;
-        for (int q = lo; q < hi; ++q) r += (s_key[s_perm[q]] < wa) ? 1 : 0;
-        s_order[lo + r] = (uint16_t)ia;
-      }
+    const unsigned long long culled = __builtin_amdgcn_ballot_w64(kb[r] == kCulled);
+    const int culled_before = r * kSortThreads + wave * 64 - (int)(before & 0xffffu) - (int)(before >> 16);
+    if (kb[r] == kCulled) out(n - 1 - culled_before - lanes_below(culled), ~my_id[r], kInvalidKey);
+    if (nl > 0 && !network) {                            // late ones: in list order behind all others
+      const unsigned long long late = __builtin_amdgcn_ballot_w64(kb[r] == invalid_bits);
+      if (kb[r] == invalid_bits) out(nv + (int)(before >> 16) + lanes_below(late), my_id[r], kInvalidKey);
     }
   }
-  if (network) {
-    // the late entries join the others (through registers: the two regions can overlap)
-    unsigned long long moved[kSortMax / kSortThreads];
-#pragma unroll
-    for (int v = 0; v < kSortMax / kSortThreads; ++v) {
-      const int j = tid + v * kSortThreads;
-      moved[v] = (j < nl) ? s_key[kSortMax - 1 - j] : 0ull;
+  if (!network) {
+    __syncthreads();
+    const int both = lds.bucket[tid].y;
+    const int c0 = both & 0xffff, c1 = (both >> 16) & 0xffff;
+    const int c = c0 + c1;
+    const uint32_t upto_c = sum_up_to_lane<false>((uint32_t)c), pairs = sum_up_to_lane<false>((uint32_t)(c0 * c0 + c1 * c1));
+    if (lane == 63) {
+      lds.sum[wave] = upto_c;
+      lds.pairs[wave] = pairs;
     }
     __syncthreads();
+    uint32_t base = 0u, all_pairs = 0u;
 #pragma unroll
-    for (int v = 0; v < kSortMax / kSortThreads; ++v) {
-      const int j = tid + v * kSortThreads;
-      if (j < nl) s_key[nv + j] = moved[v];
+    for (int v = 0; v < kWaves; ++v) {
+      base += (v < wave) ? (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.sum[v]) : 0u;
+      all_pairs += (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.pairs[v]);
     }
-    nv += nl;
-    nl = 0;
+    const int excl = (int)(base + upto_c) - c;
+    lds.bucket[tid].x = excl | ((excl + c0) << 16);
+    network = all_pairs > (uint32_t)kRankPairsMax;
+    __syncthreads();
+  }
+  if (!network) {
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r * kSortThreads >= n) continue;
+      const int i = r * kSortThreads + tid, b = at[r] & 0xffff;
+      if (kb[r] < invalid_bits)
+        s_key[half_of(lds.bucket[b >> 1].x, b) + (at[r] >> 16)] = ((unsigned long long)kb[r] << 32) | (unsigned)(ASC ? my_id[r] : i);
+    }
+    __syncthreads();
+    for (int a = tid; a < nv; a += kSortThreads) {
+      const unsigned long long wa = s_key[a];
+      const int b = bucket_of((uint32_t)(wa >> 32));
+      const int2 two = lds.bucket[b >> 1];
+      const int lo = half_of(two.x, b), hi = lo + half_of(two.y, b);
+      int rank = 0;
+      for (int q = lo; q < hi; ++q) rank += (s_key[q] < wa) ? 1 : 0;
+      out(lo + rank, ASC ? (int)(wa & 0xffffffffu) : cand[start + (int)(wa & 0xffffffffu)], bits_to_float((uint32_t)(wa >> 32)));
+    }
+  } else {
+    // the words in any order (they are all different); late ones too unless they are in their places already
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+      if (r * kSortThreads >= n) continue;
+      const int i = r * kSortThreads + tid;
+      const bool front = kb[r] < invalid_bits, late = !front && kb[r] < kNoEntry;
+      const unsigned long long mf = __builtin_amdgcn_ballot_w64(front), ml = __builtin_amdgcn_ballot_w64(late);
+      const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)before_all, r * kWaves + wave);
+      const int slot = front ? (int)(before & 0xffffu) + lanes_below(mf) : nv + (int)(before >> 16) + lanes_below(ml);
+      if (front || (late && odd)) s_key[slot] = ((unsigned long long)kb[r] << 32) | (unsigned)(ASC ? my_id[r] : i);
+    }
+    if (odd) nv += nl;
     int npad = 2;
     while (npad < nv) npad <<= 1;
     for (int i = nv + tid; i < npad; i += kSortThreads) s_key[i] = ~0ull;
@@ -720,20 +732,14 @@ __device__ __forceinline__ void sort_one_tile_from(SortLds<kSortMax>& lds, const
         }
       }
     }
-  }
-  __syncthreads();
-
-  const bool through_order = ranked && !network;
-  for (int i = tid; i < len; i += kSortThreads) {
-    if (i < nv + nl) {
-      const unsigned long long w = (i >= nv) ? s_key[kSortMax - 1 - (i - nv)] : s_key[through_order ? s_order[i] : i];
-      sorted_ids[start + i] = ASC ? (int)(w & 0xffffffffu) : cand[start + (int)(w & 0xffffffffu)];
-      if (sorted_keys) sorted_keys[start + i] = bits_to_float((uint32_t)(w >> 32));
-    } else if (i >= n) {
-      sorted_ids[start + i] = cand[start + i];     // beyond the sort capacity: list order, never culled
-      if (sorted_keys) sorted_keys[start + i] = kInvalidKey;
+    __syncthreads();
+    for (int i = tid; i < nv; i += kSortThreads) {
+      const unsigned long long w = s_key[i];
+      out(i, ASC ? (int)(w & 0xffffffffu) : cand[start + (int)(w & 0xffffffffu)], bits_to_float((uint32_t)(w >> 32)));
     }
   }
+  // beyond the sort capacity: list order, never culled
+  for (int i = n + tid; i < len; i += kSortThreads) out(i, cand[start + i], kInvalidKey);
 }
 
 template <int kSortMax, bool PYR, bool ASC = false>

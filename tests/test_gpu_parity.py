@@ -360,6 +360,38 @@ def test_sort_is_the_stable_key_order_for_every_key_distribution(device, oracle_
     _assert_bits(keys, want_keys, "sort keys")
 
 
+@pytest.mark.parametrize("records", ["pyramids, ids ascend", "pyramids", "none"])
+@pytest.mark.parametrize("n", [65, 255, 256, 257, 511, 513, 1025, 1793, 2047, 2048])
+def test_sort_at_the_ends_of_its_rounds(device, oracle_mod, n, records):
+    """One tile, a list that ends at, before or behind a round of 256: ordinary keys, invalid ones and culled entries in every
+    wavefront's share.  The kept ones as the oracle's stable sort has them, the culled ones behind them, last one first."""
+    from mlp_splatting_amd import ops
+    rng = np.random.default_rng(n)
+    fr = Frame("cfg1_5k_160x120", n=8, width=8, height=8, eye=(0, 0, -2.0), target=(0, 0, 0))
+    pos = rng.uniform(-0.1, 0.1, (n, 3))
+    behind = rng.random(n) < 0.2                                     # by less than their size: not culled
+    pos[:, 2] = np.where(behind, rng.uniform(-2.3, -2.1, n), rng.uniform(-1.0, 3.0, n))
+    pos[:, 0] += np.where(rng.random(n) < 0.3, 4.0, 0.0)             # far beside the tile
+    log_s = np.where(behind[:, None], -1.0, rng.uniform(-3.0, -2.0, (n, 3))).astype(np.float32)
+    pos = pos.astype(np.float32)
+    quat = rng.normal(size=(n, 4)).astype(np.float32)
+    quat /= np.linalg.norm(quat, axis=1, keepdims=True)
+    cand, off = np.arange(n, dtype=np.int32), np.array([0, n], np.int32)
+    rec = ops.prepare_primitives(_t(pos, device), _t(log_s, device), _t(quat, device))
+    ro, rd = _t(fr.rays_o, device), _t(fr.rays_d, device)
+    more = {} if records == "none" else {"tile_pyramids": ops.frame_prologue(ro, rd, 8, 8)[1]}
+    ids, keys = ops.sort_tiles(ro, rd, rec, _t(cand, device), _t(off, device), 8, 8, 8, 8, capacity=2048, want_keys=True,
+                               cull_threshold=1e-2, ids_ascend="ascend" in records, **more)
+    want_ids, want_keys = oracle_mod.sort_tiles(fr.rays_o, fr.rays_d, pos, log_s, quat, cand, off, 8, 8, 8, 8, capacity=2048)
+    ids, keys = ids.cpu().numpy(), keys.cpu().numpy()
+    gone = ~ids[ids < 0]
+    assert 0.15 < gone.size / n < 0.6 and np.array_equal(gone, np.sort(gone)[::-1])
+    kept = ~np.isin(want_ids, gone)
+    np.testing.assert_array_equal(ids[:n - gone.size], want_ids[kept])
+    _assert_bits(keys[:n - gone.size], want_keys[kept], "sort keys")
+    assert (want_keys[kept] == np.float32(1e30)).any()
+
+
 @pytest.mark.parametrize("name,n,width,height,tile,eye", [
     ("cfg1_5k_160x120", None, 160, 120, 8, (0.3, -0.2, -0.5)), ("cfg1_5k_160x120", 4000, 100, 76, 16, (1.0, 0.8, -1.2)),
     ("cfg2_50k_640x480", 20000, 200, 136, 8, (-0.7, 0.4, 0.9)), ("cfg1_5k_160x120", 1500, 21, 13, 8, (0.1, 0.1, -0.2))])
