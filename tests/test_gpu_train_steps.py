@@ -361,6 +361,37 @@ def test_tiles_of_every_length_take_the_chunks_they_need(device, width, height):
         assert torch.equal(g, w)
 
 
+@pytest.mark.parametrize("lengths", [(1, 2, 3, 4, 5, 6, 7, 0, 8, 9), (511, 512, 513, 516), (1024, 1, 1025, 1029)])
+def test_the_reverse_walk_of_tiles_of_every_length(device, lengths):
+    """The reverse walk asks for four steps ahead and for the places of 512 at a time: lists that end around these, of
+    primitives that all hit and hardly cover, against the record pipeline.  A step's adjoint behind up to 1,029 others is a
+    chain of as many f32 roundings on either side, 1,029 x 2^-24 = 6e-5 of it at the worst."""
+    import numpy as np
+    from mlp_splatting_amd import ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    n, width, height = max(lengths), 8 * len(lengths), 8
+    sc = syn.make_scene(n, 32, seed=4, log_scale_mean=2.5)
+    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
+    sc.b3[:, 3] = -8.0
+    c2w = syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0))
+    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, c2w)
+    cand = np.concatenate([np.arange(k) for k in lengths]).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats, cand, off, sc.freq,
+                                        sc.att, *sc.mlp())]
+    ext = TileExt(max_hits=2048)
+    x = base + [torch.zeros_like(base[0]), torch.zeros(width * height, device=device)]
+    records = ext.render_tiles_training_records(x, width, height, 8, 1e-3, 1.5, 2.0, render_order=True)
+    rgb, _, frame = ext.train_forward(base, width, height, 1e-3)
+    assert frame.steps == sum(lengths) and torch.equal(rgb, records[0])
+    torch.manual_seed(7)
+    g_rgb, g_t = torch.randn(width * height, 3, device=device), torch.randn(width * height, device=device)
+    want = ext.backward_from_records(records, base[2], base[3], base[4], base[7], base[8], *base[9:15], g_rgb, g_t)
+    got = ext.backward_from_steps(frame, ops.train_group(frame, base[6], n), base, g_rgb, g_t)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert float((g - w).norm()) <= 6e-5 * float(w.norm()), i
+
+
 def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
     """Storage follows the steps, not the tiles: a tile with a hit takes a chunk, and the first frame reserves no more than
     its lists can need."""
