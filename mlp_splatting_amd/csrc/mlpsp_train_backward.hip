@@ -95,8 +95,8 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
 // ---------------------------------------------------------------------------------------------
 // steps sorted by primitive: a stable radix sort of the S primitive numbers in tile order, in digits of equal width (two of
 // nine bits at 200,000 primitives).  A wavefront takes an eighth of its block's steps in rounds of 64, whose equal digits are
-// found with a ballot per bit.  Eight launches, 140 us at 650,000 steps (the two sums over blocks x digits, one workgroup
-// each, 50 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
+// found with a ballot per bit.  Eight launches, 120 us at 650,000 steps (the two sums over blocks x digits, one workgroup
+// each, 27 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSortBlock = 512, kSortBits = 10;
 // Steps of a block: 8,192, a quarter of that where this would leave a chip of 256 CUs fewer than 32 blocks (16 rounds one
@@ -131,39 +131,59 @@ __global__ __launch_bounds__(kSortBlock) void step_hist_kernel(const int32_t* __
   for (int d = threadIdx.x; d < R; d += kSortBlock) hist[d * blocks + blockIdx.x] = s_count[d];
 }
 
-// exclusive sums of n counts, in place; one workgroup
+// exclusive sums of n counts, in place; one workgroup, kSumRounds of 4,096 counts behind one barrier: a round at a time, its
+// loads and two barriers one after the other, the 40,960 counts of 650,000 steps took 26 us instead of 14
+constexpr int kSumRounds = 10;           // what 650,000 steps have
 __global__ __launch_bounds__(1024) void step_sums_kernel(int32_t* __restrict__ v, int n) {
-  __shared__ int s_wave[16];
+  __shared__ int s_wave[2][kSumRounds * 16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   int carry = 0;
-  for (int base = 0; base < n; base += 4096) {
-    const int i = base + 4 * t;
-    int x[4];
+  for (int base = 0, turn = 0; base < n; base += kSumRounds * 4096, turn ^= 1) {
+    int4 x[kSumRounds];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) x[k] = i + k < n ? v[i + k] : 0;
-    const int mine = (x[0] + x[1]) + (x[2] + x[3]);
-    int incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int u = __shfl_up(incl, d);
-      if (lane >= d) incl += u;
+    for (int u = 0; u < kSumRounds; ++u) {
+      const int i = base + 4096 * u + 4 * t;
+      x[u] = i + 3 < n ? *reinterpret_cast<const int4*>(v + i)
+                       : make_int4(i < n ? v[i] : 0, i + 1 < n ? v[i + 1] : 0, i + 2 < n ? v[i + 2] : 0, 0);
     }
-    if (lane == 63) s_wave[wave] = incl;
-    __syncthreads();
-    int before = carry, total = 0;
+    int incl[kSumRounds];
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      before += w < wave ? s_wave[w] : 0;
-      total += s_wave[w];
-    }
-    carry += total;
-    int run = before + incl - mine;
+    for (int u = 0; u < kSumRounds; ++u) {
+      if (base + 4096 * u >= n) break;
+      incl[u] = (x[u].x + x[u].y) + (x[u].z + x[u].w);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (i + k < n) v[i + k] = run;
-      run += x[k];
+      for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl[u], d);
+        if (lane >= d) incl[u] += up;
+      }
+      if (lane == 63) s_wave[turn][16 * u + wave] = incl[u];
     }
-    __syncthreads();
+    __syncthreads();                   // (the one barrier of a turn: the next writes the other half)
+    // lane = wavefront of a round; all rounds' sums up to and with it
+    int total = carry;
+#pragma unroll
+    for (int u = 0; u < kSumRounds; ++u) {
+      if (base + 4096 * u >= n) break;
+      int w = s_wave[turn][16 * u + (lane & 15)];
+      const int own = w;
+#pragma unroll
+      for (int d = 1; d < 16; d <<= 1) {
+        const int up = __shfl_up(w, d);
+        if ((lane & 15) >= d) w += up;
+      }
+      const int i = base + 4096 * u + 4 * t;
+      int run = total + __builtin_amdgcn_readlane(w - own, wave) + incl[u] - ((x[u].x + x[u].y) + (x[u].z + x[u].w));
+      total += __builtin_amdgcn_readlane(w, 15);
+      const int4 out = make_int4(run, run + x[u].x, run + x[u].x + x[u].y, run + x[u].x + x[u].y + x[u].z);
+      if (i + 3 < n) {
+        *reinterpret_cast<int4*>(v + i) = out;
+      } else {
+        if (i < n) v[i] = out.x;
+        if (i + 1 < n) v[i + 1] = out.y;
+        if (i + 2 < n) v[i + 2] = out.z;
+      }
+    }
+    carry = total;
   }
 }
 

@@ -392,6 +392,36 @@ def test_the_reverse_walk_of_tiles_of_every_length(device, lengths):
         assert float((g - w).norm()) <= 6e-5 * float(w.norm()), i
 
 
+@pytest.mark.parametrize("n,tiles,listed", [(2, 1, 1), (40, 700, 40), (70_000, 700, 40), (600_000, 1030, 80)])
+def test_steps_are_sorted_by_primitive(device, n, tiles, listed):
+    """The stable sort of a frame's steps, with fewer counts than the sums over blocks and digits take at a time (4,096), with
+    several times and, at 600,000 primitives and 82,400 steps, with more than ten times as many (41 blocks x 1,024 digits)."""
+    import numpy as np
+    from mlp_splatting_amd import ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    width, height, rng = 8 * tiles, 8, np.random.default_rng(n)
+    lists = np.stack([np.sort(rng.choice(n, listed, replace=False)) for _ in range(tiles)]).astype(np.int32)
+    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
+    positions = np.array([0.0, 0.0, 9.0], np.float32) + 0.1 * rng.standard_normal((n, 3)).astype(np.float32)
+    quats = np.tile(np.array([1.0, 0.0, 0.0, 0.0], np.float32), (n, 1))
+    sc = syn.make_scene(1, 32, seed=0)
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), positions, np.full((n, 3), 2.5, np.float32), quats,
+                                        lists.reshape(-1), np.arange(tiles + 1, dtype=np.int32) * listed, sc.freq, sc.att)]
+    base += [torch.zeros((n,) + w.shape[1:], device=device) for w in sc.mlp()]
+    base[14][:, 3] = -8.0
+    _, _, frame = TileExt().train_forward(base, width, height, 1e-3)
+    steps = frame.steps
+    assert steps == tiles * listed
+    words = ops.train_group(frame, base[6], n).view(torch.int32).cpu().numpy()
+    ends = np.cumsum([(k + 63) // 64 * 64 for k in (n + 1, steps, 4 * steps)])      # parts in units of 256 bytes
+    first, prim, step = words[:n + 1], words[ends[0]:ends[0] + steps], words[ends[1]:ends[1] + 4 * steps].reshape(-1, 4)
+    order = np.argsort(lists.reshape(-1), kind="stable")
+    tile = order // listed                             # (a tile's steps come in the order of their depths: listed to a tile)
+    assert (prim == lists.reshape(-1)[order]).all() and (step[:, 1] // listed == tile).all()
+    assert (step[:, 2] == tile).all() and (step[:, 3] == 8 * tile).all() and (np.sort(step[:, 1]) == np.arange(steps)).all()
+    assert (first == np.searchsorted(prim, np.arange(n + 1))).all()
+
+
 def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
     """Storage follows the steps, not the tiles: a tile with a hit takes a chunk, and the first frame reserves no more than
     its lists can need."""
