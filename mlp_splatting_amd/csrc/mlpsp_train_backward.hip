@@ -274,6 +274,32 @@ __device__ __forceinline__ StepRun step_run(const StepIndex& ix, int pos, int ch
   r.complete = all_begin == pos && !r.goes_on;
   return r;
 }
+// The same out of LDS, where a chunk's workgroup keeps the primitives of its steps, of the one before them and of the one behind
+// (-1: there is none): `first` of the primitive is not looked up, and nothing of memory is waited for.
+struct ChunkPrims {
+  int prim[kTrainChunk + 2];
+};
+__device__ __forceinline__ void load_chunk(const StepIndex& ix, int S, int begin, int end, int t, int threads, ChunkPrims& s) {
+  for (int k = t; k < end - begin + 2; k += threads) {
+    const int i = begin - 1 + k;
+    s.prim[k] = i >= 0 && i < S ? ix.prim[i] : -1;
+  }
+}
+__device__ __forceinline__ StepRun chunk_run(const ChunkPrims& s, int pos, int chunk_begin, int chunk_end, int lane) {
+  static_assert(kTrainChunk <= 128, "two looks");
+  asm volatile("" : "+v"(lane));         // (or addresses are formed ahead of the loop over the runs and kept)
+  const int n = chunk_end - chunk_begin, at = pos - chunk_begin;        // prim[at + 1] is that of step pos
+  StepRun r;
+  r.p = __builtin_amdgcn_readfirstlane(s.prim[at + 1]);
+  const int near = at + lane, far = near + 64;
+  const unsigned long long a = __ballot(near >= n || s.prim[min(near, n) + 1] != r.p);
+  const unsigned long long b = __ballot(far >= n || s.prim[min(far, n) + 1] != r.p);
+  r.begin = pos;
+  r.end = a ? pos + (int)__builtin_ctzll(a) : b ? pos + 64 + (int)__builtin_ctzll(b) : chunk_end;
+  r.goes_on = r.end == chunk_end && __builtin_amdgcn_readfirstlane(s.prim[n + 1]) == r.p;
+  r.complete = !r.goes_on && __builtin_amdgcn_readfirstlane(s.prim[at]) != r.p;
+  return r;
+}
 // head rows come first, then tail rows
 __device__ __forceinline__ float* run_row(float* rows, const StepRun& r, int chunk, int num_chunks) {
   return rows + (size_t)(r.goes_on ? num_chunks + chunk : chunk) * kRowFloats;
@@ -406,28 +432,31 @@ __device__ __forceinline__ StepRecord step_record(const unsigned char* __restric
   r.mask2 = reinterpret_cast<const uint32_t*>(rec + kStepPlaneD)[px];
   return r;
 }
-// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on; work(record) for those that
-// have an adjoint.  Lane i asks for where the i-th of them lies; the next record is under way while one is worked on (two or
-// three: no faster).  Records
-// without an adjoint get inputs of zero, whatever ray their lane has.
-template <int STRIDE, bool FRESH, typename Work>
-__device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int end, int half, const unsigned char* __restrict__ records,
-                                            const float4* __restrict__ d4, const float* __restrict__ rays_d, int W, int pixels,
-                                            int lane, Work&& work) {
+// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on.  Lane i asks for where the i-th of them lies
+// (walk_steps), the first record is requested beside the run's weights (walk_record), and walk_halves has the next record under
+// way while one is worked on (two or three: no faster): work(record) for those that have an adjoint.  Records without one get
+// inputs of zero, whatever ray their lane has.  A wavefront without a step (first >= end) asks for the last one's and drops it.
+template <int STRIDE>
+__device__ __forceinline__ int4 walk_steps(const StepIndex& ix, int first, int end, int lane) {
   static_assert(kTrainChunk <= 64 * STRIDE, "a lane for every step");
+  asm volatile("" : "+v"(lane));         // (as in chunk_run)
+  return ix.step[min(first + STRIDE * lane, end - 1)];
+}
+__device__ __forceinline__ StepRecord walk_record(const int4& where, int k, int half, const unsigned char* __restrict__ records,
+                                                  const float4* __restrict__ d4, const float* __restrict__ rays_d, int W,
+                                                  int pixels, int lane) {
+  return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readlane(where.x, k), __builtin_amdgcn_readlane(where.y, k), 0,
+                                                    __builtin_amdgcn_readlane(where.w, k)), half, lane & 31, lane >> 5, W, pixels);
+}
+template <int STRIDE, bool FRESH, typename Work>
+__device__ __forceinline__ void walk_halves(const int4& where, StepRecord next, int first, int end, int half,
+                                            const unsigned char* __restrict__ records, const float4* __restrict__ d4,
+                                            const float* __restrict__ rays_d, int W, int pixels, int lane, Work&& work) {
   const int count = (end - first + STRIDE - 1) / STRIDE;
-  if (count <= 0) return;
-  const int4 where = ix.step[min(first + STRIDE * lane, end - 1)];
-  const auto record = [&](int i) {
-    const int k = min(i, count - 1);
-    const int l = FRESH ? fresh_lane() : lane;
-    return step_record(records, d4, rays_d, make_int4(__builtin_amdgcn_readlane(where.x, k), __builtin_amdgcn_readlane(where.y, k), 0,
-                                                      __builtin_amdgcn_readlane(where.w, k)), half, l & 31, l >> 5, W, pixels);
-  };
-  StepRecord next = record(0);
   for (int i = 0; i < count; ++i) {
     StepRecord r = next;
-    next = record(i + 1);          // (at the end the last one again: under a condition the request is waited for)
+    // (at the end the last one again: under a condition the request is waited for)
+    next = walk_record(where, min(i + 1, count - 1), half, records, d4, rays_d, W, pixels, FRESH ? fresh_lane() : lane);
     const bool adjoint = r.d.x != 0.f || r.d.y != 0.f || r.d.z != 0.f || r.d.w != 0.f;
     if (__ballot(adjoint) == 0ull) continue;
 #pragma unroll
@@ -436,10 +465,11 @@ __device__ __forceinline__ void walk_halves(const StepIndex& ix, int first, int 
   }
 }
 
-// A wavefront's share of the rows of primitives without a step, stored before it turns to its chunk: the chunks begin at
-// different times, and the stores go on beside the products of the others.  The whole call at 648,000 steps of 200,000
-// primitives with these 2.8 GB in a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 /
-// 1.70; at the end of a chunk as at its beginning, a primitive per block of products 5.34 and 1.83.
+// A wavefront's share of the rows of primitives without a step, stored behind its chunk: the chunks end at different times, and
+// the stores go on beside the products of the others.  The whole call at 648,000 steps of 200,000 primitives with these 2.8 GB in
+// a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 / 1.70; a primitive per block of
+// products 5.34 and 1.83.  Ahead of the chunk its first record is waited for behind the stores: the f32 kernel of 80,000 steps
+// takes 676 us instead of 663.
 template <int WAVES>
 __device__ __forceinline__ void zero_share(const StepIndex& ix, int N, const ZeroRows& zero, int chunk, int num_chunks, int wave,
                                            int lane) {
@@ -454,6 +484,7 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
     int32_t* __restrict__ nonfinite, int N, ZeroRows zero) {
   __shared__ Vjp16StepsLds<T> lds;
+  __shared__ ChunkPrims prims;
   Vjp16Shared<T>& s = lds.s;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
@@ -461,18 +492,26 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
   for (int f = 0; f < 6; ++f)
     kf[f] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((freq[f] * att[f]) * 0.159154943f)));
-  zero_share<kVjp16Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
+  const int chunk_begin = chunk * chunk_steps, first = wave >> 1;
+  load_chunk(ix, S, chunk_begin, chunk_end, t, 64 * kVjp16Waves, prims);
+  __syncthreads();
+  StepRun run = chunk_run(prims, chunk_begin, chunk_begin, chunk_end, lane);
+  Vjp16Request weights = vjp16_request(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane);
+  int4 where = walk_steps<kVjp16Waves / 2>(ix, run.begin + first, run.end, lane);
   bool bad = false;
-  for (int pos = chunk * chunk_steps; pos < chunk_end;) {
-    const StepRun run = step_run(ix, pos, chunk_end);
-    vjp16_load<T>(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane, s);
+  for (;;) {
+    StepRecord record = walk_record(where, 0, wave & 1, records, d4, rays_d, W, W * H, lane);
+    vjp16_load<T>(weights, wave, lane, s);
     if (t < 4) s.zero[t] = 0u;
     Vjp16StepSums sum;
     sum.clear();
     __syncthreads();
-    walk_halves<kVjp16Waves / 2, true>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
+    walk_halves<kVjp16Waves / 2, true>(where, record, run.begin + first, run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
       vjp16_step_block<T>(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, kf, scale, lane);
     });
+    const StepRun next = run.end < chunk_end ? chunk_run(prims, run.end, chunk_begin, chunk_end, lane) : run;
+    weights = vjp16_request(W1, b1, W2, b2, W3, (size_t)next.p, wave, lane);
+    where = walk_steps<kVjp16Waves / 2>(ix, next.begin + first, next.end, lane);
     const int waves = min(2 * (run.end - run.begin), kVjp16Waves), slots = min(waves, kVjp16Slots);
     __syncthreads();
     if (wave < slots) vjp16_park<false>(sum, lds.sums[wave], lane);
@@ -483,9 +522,11 @@ __global__ __launch_bounds__(64 * kVjp16Waves) __attribute__((amdgpu_waves_per_e
     __syncthreads();
     bad |= store_row_sums(lds.sums[0], kGradFloats, slots, run_dest(rows, grads, run, chunk, num_chunks), 1.f / scale, t,
                           64 * kVjp16Waves);
-    pos = run.end;
+    if (run.end >= chunk_end) break;
+    run = next;
     __syncthreads();
   }
+  zero_share<kVjp16Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
   if (__ballot(bad) != 0ull && lane == 0) atomicOr(nonfinite, 1);
 }
 
@@ -499,6 +540,7 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
     const float* __restrict__ b2, const float* __restrict__ W3, float scale, float* __restrict__ rows, GradRows grads,
     int32_t* __restrict__ nonfinite, int N, ZeroRows zero) {
   __shared__ Vjp32Lds s;
+  __shared__ ChunkPrims prims;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int chunk = blockIdx.x, chunk_end = min(S, (chunk + 1) * chunk_steps);
   const SplitUnits u;
@@ -510,32 +552,47 @@ __global__ __launch_bounds__(64 * kVjp32Waves) __attribute__((amdgpu_waves_per_e
   }
   if (t < 4) s.zero[t] = 0u;
   for (int k = t; k < kCircleEntries; k += 64 * kVjp32Waves) s.circle[k] = f32x2v{kCircle.at[k][0], kCircle.at[k][1]};
-  zero_share<kVjp32Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
+  const int chunk_begin = chunk * chunk_steps, first = wave >> 1;
+  load_chunk(ix, S, chunk_begin, chunk_end, t, 64 * kVjp32Waves, prims);
+  __syncthreads();
+  StepRun run = chunk_run(prims, chunk_begin, chunk_begin, chunk_end, lane);
+  Vjp32Request weights = vjp32_request(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane);
+  int4 where = walk_steps<kVjp32Waves / 2>(ix, run.begin + first, run.end, lane);
   bool bad = false;
-  for (int pos = chunk * chunk_steps; pos < chunk_end;) {
-    const StepRun run = step_run(ix, pos, chunk_end);
-    vjp32_load(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane, s, u);
-    // The adjoints lifted first; sums that this takes out of range are formed again without.
-    for (float by = scale * kVjp32Lift;; by = scale) {
-      Vjp32Sums sum;
-      sum.clear();
-      __syncthreads();
-      walk_halves<kVjp32Waves / 2, false>(ix, run.begin + (wave >> 1), run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
-        vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, by, lane, u);
-      });
-      const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
-      if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
-      __syncthreads();
-      const bool beyond = store_row_sums(reinterpret_cast<const float*>(&s.wave[0]), sizeof(Vjp32Wave) / 4, waves,
-                                         run_dest(rows, grads, run, chunk, num_chunks), 1.f / by, t, 64 * kVjp32Waves);
-      if (!__syncthreads_or(beyond)) break;
-      if (by == scale) {
-        bad = true;
-        break;
-      }
+  // The adjoints lifted first; a run whose sums this takes out of range is gone through again without.
+  float by = scale * kVjp32Lift;
+  for (;;) {
+    const StepRecord record = walk_record(where, 0, wave & 1, records, d4, rays_d, W, W * H, lane);
+    vjp32_load(weights, wave, lane, s, u);
+    Vjp32Sums sum;
+    sum.clear();
+    __syncthreads();
+    walk_halves<kVjp32Waves / 2, false>(where, record, run.begin + first, run.end, wave & 1, records, d4, rays_d, W, W * H, lane, [&](const StepRecord& r) {
+      vjp32_block(s, sum, s.wave[wave], r.x, r.d, r.mask1, r.mask2, factors, by, lane, u);
+    });
+    StepRun next = run.end < chunk_end ? chunk_run(prims, run.end, chunk_begin, chunk_end, lane) : run;
+    weights = vjp32_request(W1, b1, W2, b2, W3, (size_t)next.p, wave, lane);
+    where = walk_steps<kVjp32Waves / 2>(ix, next.begin + first, next.end, lane);
+    const int waves = min(2 * (run.end - run.begin), kVjp32Waves);
+    if (wave < waves) vjp32_park(sum, reinterpret_cast<float*>(&s.wave[wave]), lane);
+    __syncthreads();
+    const bool beyond = store_row_sums(reinterpret_cast<const float*>(&s.wave[0]), sizeof(Vjp32Wave) / 4, waves,
+                                       run_dest(rows, grads, run, chunk, num_chunks), 1.f / by, t, 64 * kVjp32Waves);
+    if (lane == 0) s.beyond[wave] = __ballot(beyond) != 0ull;
+    __syncthreads();
+    const bool again = __builtin_amdgcn_readfirstlane(s.beyond[0] | s.beyond[1] | s.beyond[2] | s.beyond[3]) != 0;
+    if (again && by != scale) {
+      by = scale;
+      weights = vjp32_request(W1, b1, W2, b2, W3, (size_t)run.p, wave, lane);
+      where = walk_steps<kVjp32Waves / 2>(ix, run.begin + first, run.end, lane);
+      continue;
     }
-    pos = run.end;
+    bad |= again;
+    if (run.end >= chunk_end) break;
+    by = scale * kVjp32Lift;
+    run = next;
   }
+  zero_share<kVjp32Waves>(ix, N, zero, chunk, num_chunks, wave, lane);
   if (__ballot(bad) != 0ull && lane == 0) atomicOr(nonfinite, 1);
 }
 

@@ -44,41 +44,42 @@ union Vjp16StepsLds {
   __attribute__((aligned(16))) float sums[kVjp16Slots][kGradFloats];    // in the end, two wavefronts to a row
 };
 
-// The primitive's weights into LDS, in eight pieces of 64 lanes.
-template <typename T>
-__device__ __forceinline__ void vjp16_load(const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
-                                           const float* __restrict__ b2, const float* __restrict__ W3, size_t p, int wave, int lane,
-                                           Vjp16Shared<T>& s) {
+// What a lane loads of a primitive's weights, as Vjp32Request: of W1 the pairs 4 wave .. 4 wave + 3; then wavefront 0 the pairs 16
+// and 17, 1 and 2 rows and columns of W2, 3 W3 and the biases.
+struct Vjp16Request {
+  f32x4 sines, cosines, a, b;
+  float c[8];
+};
+__device__ __forceinline__ Vjp16Request vjp16_request(const float* __restrict__ W1, const float* __restrict__ b1,
+                                                      const float* __restrict__ W2, const float* __restrict__ b2,
+                                                      const float* __restrict__ W3, size_t p, int wave, int lane) {
   asm volatile("" : "+v"(lane));         // (or the addresses are formed ahead of the loop over the runs, one by one)
+  const int n = lane & 31, g = lane >> 5, k = wave == 2 ? 1 : 0;
+  const float* row1 = W1 + p * 2304 + n * 72 + 18 * g;
+  const float* a = wave == 0 ? row1 + 14 : W2 + p * 1024 + n * 32 + 16 * k + 4 * g;
+  Vjp16Request r{load4_here(row1 + 4 * wave), load4_here(row1 + 36 + 4 * wave), load4_here(a), load4_here(wave == 0 ? a + 36 : a + 8), {}};
+  const float *col = W2 + p * 1024 + n, *out = W3 + p * 128 + hidden_unit_of_row(n), *bias = (g ? b2 : b1) + p * 32 + n;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r.c[i] = load_here(wave == 3 ? (i < 4 ? out + 32 * i : bias) : col + hidden_unit(8 * k + i, g) * 32);
+  return r;
+}
+// The primitive's weights into LDS, by the whole workgroup.
+template <typename T>
+__device__ __forceinline__ void vjp16_load(const Vjp16Request& r, int wave, int lane, Vjp16Shared<T>& s) {
+  asm volatile("" : "+v"(lane));         // (as in vjp16_request)
   const int n = lane & 31, g = lane >> 5;
-  for (int q = wave; q < 5; q += kVjp16Waves) {
-    const float* __restrict__ row = W1 + p * 2304 + n * 72 + 18 * g;
-    u32x4 v;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int t = 4 * q + d;
-      v[d] = t < 18 ? Ops<T>::pack2(row[t < 18 ? t : 0], row[36 + (t < 18 ? t : 0)]) : 0u;
-    }
-    s.w1[q][lane] = v;
-  }
-  if (wave == 1 || wave == 2) {
-    const int k = wave - 1;
-    const float* __restrict__ row = W2 + p * 1024 + n * 32 + 16 * k + 4 * g;
-    const float* __restrict__ col = W2 + p * 1024 + n;
-    u32x4 a, b;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const int j = 2 * d + (d & 2 ? 4 : 0);
-      a[d] = Ops<T>::pack2(row[j], row[j + 1]);
-      b[d] = Ops<T>::pack2(col[hidden_unit(8 * k + 2 * d, g) * 32], col[hidden_unit(8 * k + 2 * d + 1, g) * 32]);
-    }
-    s.w2[k][lane] = a;
-    s.w2t[k][lane] = b;
-  }
-  if (wave == 3) {
-    const float* __restrict__ r = W3 + p * 128 + hidden_unit_of_row(n);
-    s.w3r[lane] = g ? u32x2{0u, 0u} : u32x2{Ops<T>::pack2(r[0], r[32]), Ops<T>::pack2(r[64], r[96])};
-    (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
+  s.w1[wave][lane] = u32x4{Ops<T>::pack2(r.sines[0], r.cosines[0]), Ops<T>::pack2(r.sines[1], r.cosines[1]),
+                           Ops<T>::pack2(r.sines[2], r.cosines[2]), Ops<T>::pack2(r.sines[3], r.cosines[3])};
+  if (wave == 0) {
+    s.w1[4][lane] = u32x4{Ops<T>::pack2(r.a[2], r.b[2]), Ops<T>::pack2(r.a[3], r.b[3]), 0u, 0u};
+  } else if (wave < 3) {
+    s.w2[wave - 1][lane] = u32x4{Ops<T>::pack2(r.a[0], r.a[1]), Ops<T>::pack2(r.a[2], r.a[3]),
+                                 Ops<T>::pack2(r.b[0], r.b[1]), Ops<T>::pack2(r.b[2], r.b[3])};
+    s.w2t[wave - 1][lane] = u32x4{Ops<T>::pack2(r.c[0], r.c[1]), Ops<T>::pack2(r.c[2], r.c[3]),
+                                  Ops<T>::pack2(r.c[4], r.c[5]), Ops<T>::pack2(r.c[6], r.c[7])};
+  } else {
+    s.w3r[lane] = g ? u32x2{0u, 0u} : u32x2{Ops<T>::pack2(r.c[0], r.c[1]), Ops<T>::pack2(r.c[2], r.c[3])};
+    (g ? s.bias2 : s.bias1)[n] = r.c[4];
   }
 }
 

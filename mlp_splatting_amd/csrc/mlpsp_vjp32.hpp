@@ -146,13 +146,15 @@ struct Vjp32Lds {
   u32x4 w1_tail[2][64];          // pairs 16, 17 of two planes
   u32x2 w1_tail1[2][64];         // ... of one, against zeros for the other
   unsigned w2[3][32][16];        // W2[n][..]: 16 bytes 2 s + g (tile_place) = unit(8 s + j, g)
-  float w3[2][64];               // W3[2 j + g][n]
-  float bias1[32], bias2[32];
+  __attribute__((aligned(16))) float w3[2][64];      // W3[2 j + g][n]: as it lies
+  __attribute__((aligned(16))) float bias1[32], bias2[32];
   __attribute__((aligned(16))) unsigned zero[4];
+  int beyond[kVjp32Waves];       // a wavefront's sums are not all finite
   f32x2v circle[kCircleEntries];
   Vjp32Wave wave[kVjp32Waves];
 };
-static_assert(2 * sizeof(Vjp32Lds) <= 163840, "two workgroups per CU");
+constexpr int kVjp32RestLds = 528;        // of the kernel's own: the primitives of a chunk's steps
+static_assert(2 * (sizeof(Vjp32Lds) + kVjp32RestLds) <= 163840, "two workgroups per CU");
 // W1 column of encoding column k = 2 w + (0 sin, 1 cos)
 __device__ __forceinline__ int enc_feature(int k) {
   const int w = k >> 1, g = w < 32 ? w >> 4 : (w - 32) >> 1, t = w < 32 ? w & 15 : 16 + (w & 1);
@@ -189,18 +191,47 @@ __device__ __forceinline__ const char* enc_reads(const unsigned (*enc)[32], int 
   return reinterpret_cast<const char*>(&enc[rec][enc_place((n >> 4) + 2 * c, (n >> 1) & 1, rec) + 2 * (n & 1)]);
 }
 
-// The primitive's weights into LDS, by the whole workgroup.
-__device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const float* __restrict__ b1, const float* __restrict__ W2,
-                                           const float* __restrict__ b2, const float* __restrict__ W3, size_t p, int wave, int lane,
-                                           Vjp32Lds& s, const SplitUnits& u) {
+// Four floats that need not be aligned to more than one.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef const __attribute__((address_space(1))) f32x4u* Float4Address;
+// (An address of unknown origin: out of a tensor that nothing is written to, the load would be put off until its value is used.)
+__device__ __forceinline__ f32x4 load4_here(const float* p) {
+  uintptr_t at = reinterpret_cast<uintptr_t>(p);
+  asm volatile("" : "+v"(at));
+  return f32x4(*(Float4Address)at);
+}
+__device__ __forceinline__ float load_here(const float* p) {
+  uintptr_t at = reinterpret_cast<uintptr_t>(p);
+  asm volatile("" : "+v"(at));
+  return *(const __attribute__((address_space(1))) float*)at;
+}
+// What a lane loads of a primitive's weights, asked for while the sums of the primitive before are put away, as is where its
+// steps lie (a chain of six look-ups from one primitive to the next otherwise; kernel at 80,000 steps 675 -> 651 us, at 650,000
+// 5.54 -> 5.49 ms, the 16-bit one 1.53 -> 1.52): the workgroup's four wavefronts share them out, each with the same four loads (no branch: where paths meet, loads are waited for).  Of W1,
+// lane (n, g): pairs 4 wave .. 4 wave + 3; then wavefronts 0 and 1 rows of W2, 2 the pairs 16 and 17 (as elements 2 and 3: the
+// four behind them may lie outside the tensor), 3 W3, b1 and b2 as they lie.
+struct Vjp32Request {
+  f32x4 sines, cosines, a, b;
+};
+__device__ __forceinline__ Vjp32Request vjp32_request(const float* __restrict__ W1, const float* __restrict__ b1,
+                                                      const float* __restrict__ W2, const float* __restrict__ b2,
+                                                      const float* __restrict__ W3, size_t p, int wave, int lane) {
   asm volatile("" : "+v"(lane));         // (as in vjp32_block)
   const int n = lane & 31, g = lane >> 5;
-  const float* __restrict__ row1 = W1 + p * 2304 + n * 72 + 18 * g;
-  const auto pair = [&](int t) { return split2(row1[t], row1[36 + t], u); };
+  const float* row1 = W1 + p * 2304 + n * 72 + 18 * g;
+  const float* tail = lane < 32 ? W3 + p * 128 + 4 * lane : lane < 40 ? b1 + p * 32 + 4 * (lane - 32) : b2 + p * 32 + 4 * (min(lane, 47) - 40);
+  const float* a = wave < 2 ? W2 + p * 1024 + n * 32 + 16 * wave + 4 * g : wave == 2 ? row1 + 14 : tail;
+  const float* b = wave < 2 ? a + 8 : wave == 2 ? a + 36 : a;
+  return Vjp32Request{load4_here(row1 + 4 * wave), load4_here(row1 + 36 + 4 * wave), load4_here(a), load4_here(b)};
+}
+// The primitive's weights into LDS, by the whole workgroup.
+__device__ __forceinline__ void vjp32_load(const Vjp32Request& r, int wave, int lane, Vjp32Lds& s, const SplitUnits& u) {
+  asm volatile("" : "+v"(lane));         // (as in vjp32_block)
+  const int n = lane & 31, g = lane >> 5;
   u32x4 v[3];
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
-    const Split2 x = pair(4 * wave + d);
+    const Split2 x = split2(r.sines[d], r.cosines[d], u);
     v[0][d] = x.h;
     v[1][d] = x.m;
     v[2][d] = x.l;
@@ -208,11 +239,10 @@ __device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const f
 #pragma unroll
   for (int k = 0; k < 3; ++k) s.w1[k][wave][lane] = v[k];
   if (wave < 2) {
-    const float* __restrict__ row2 = W2 + p * 1024 + n * 32 + 16 * wave + 4 * g;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      const int j = 2 * d + (d & 2 ? 4 : 0);
-      const Split2 x = split2(row2[j], row2[j + 1], u);
+      const f32x4& from = d < 2 ? r.a : r.b;
+      const Split2 x = split2(from[2 * (d & 1)], from[2 * (d & 1) + 1], u);
       v[0][d] = x.h;
       v[1][d] = x.m;
       v[2][d] = x.l;
@@ -220,15 +250,13 @@ __device__ __forceinline__ void vjp32_load(const float* __restrict__ W1, const f
 #pragma unroll
     for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(&s.w2[k][n][tile_place(2 * wave + g, n)]) = v[k];
   } else if (wave == 2) {
-    const Split2 x = pair(16), y = pair(17);
+    const Split2 x = split2(r.a[2], r.b[2], u), y = split2(r.a[3], r.b[3], u);
     s.w1_tail1[0][lane] = u32x2{x.h, y.h};               // h h: against (h, m)
     s.w1_tail1[1][lane] = u32x2{x.l, y.l};               // l h: against (h, m)
     s.w1_tail[0][lane] = u32x4{x.m, y.m, x.h, y.h};      // m m, h l: against (m, l)
     s.w1_tail[1][lane] = u32x4{x.h, y.h, x.m, y.m};      // h m, m h: against (m, h)
-  } else {
-    (g ? s.bias2 : s.bias1)[n] = (g ? b2 : b1)[p * 32 + n];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) s.w3[j][lane] = W3[p * 128 + (2 * j + g) * 32 + n];
+  } else if (lane < 48) {
+    reinterpret_cast<f32x4*>(lane < 32 ? &s.w3[0][0] : lane < 40 ? s.bias1 - 32 * 4 : s.bias2 - 40 * 4)[lane] = r.a;
   }
 }
 struct Vjp32Sums {
