@@ -9,7 +9,7 @@
 // written by the weight gradient kernels too.  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.14 (sort 1.7, gathers 2.85), geometry 0.16 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
+// 0.12 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -264,18 +264,8 @@ struct StepRun {
   int p, begin, end;
   bool complete, goes_on;
 };
-__device__ __forceinline__ StepRun step_run(const StepIndex& ix, int pos, int chunk_end) {
-  StepRun r;
-  r.p = __builtin_amdgcn_readfirstlane(ix.prim[pos]);
-  const int all_begin = ix.first[r.p], all_end = ix.first[r.p + 1];
-  r.begin = pos;
-  r.end = min(all_end, chunk_end);
-  r.goes_on = all_end > chunk_end;
-  r.complete = all_begin == pos && !r.goes_on;
-  return r;
-}
-// The same out of LDS, where a chunk's workgroup keeps the primitives of its steps, of the one before them and of the one behind
-// (-1: there is none): `first` of the primitive is not looked up, and nothing of memory is waited for.
+// A chunk's workgroup keeps the primitives of its steps in LDS, and those of the step before and of the one behind (-1: there is
+// none): where a run ends is seen without a look-up that would have to be waited for.
 struct ChunkPrims {
   int prim[kTrainChunk + 2];
 };
@@ -299,6 +289,13 @@ __device__ __forceinline__ StepRun chunk_run(const ChunkPrims& s, int pos, int c
   r.goes_on = r.end == chunk_end && __builtin_amdgcn_readfirstlane(s.prim[n + 1]) == r.p;
   r.complete = !r.goes_on && __builtin_amdgcn_readfirstlane(s.prim[at]) != r.p;
   return r;
+}
+// Where the steps first, first + STRIDE, ... of a run lie, a step in each lane; the last one's in those that have none.
+template <int STRIDE>
+__device__ __forceinline__ int4 walk_steps(const StepIndex& ix, int first, int end, int lane) {
+  static_assert(kTrainChunk <= 64 * STRIDE, "a lane for every step");
+  asm volatile("" : "+v"(lane));         // (as in chunk_run)
+  return ix.step[min(first + STRIDE * lane, end - 1)];
 }
 // head rows come first, then tail rows
 __device__ __forceinline__ float* run_row(float* rows, const StepRun& r, int chunk, int num_chunks) {
@@ -338,52 +335,76 @@ __device__ __forceinline__ void geometry_store(const float v[15], float qw, floa
                         r12 * (2.f * qy) + r20 * (2.f * qx) + r21 * (2.f * qy);
 }
 
-// A workgroup per chunk, the steps of a run to its wavefronts in turn.
-constexpr int kGeoWaves = 4;
+// The wavefront's sum, in its last lane: row_shr 1, 2, 4 and 8, then row_bcast 15 and 31, in the additions' own operands.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float plus_lane(float v) {
+  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float sum_in_last_lane(float v) {
+  v = plus_lane<0x111, 0xf>(v);
+  v = plus_lane<0x112, 0xf>(v);
+  v = plus_lane<0x114, 0xf>(v);
+  v = plus_lane<0x118, 0xf>(v);
+  v = plus_lane<0x142, 0xa>(v);
+  return plus_lane<0x143, 0xc>(v);
+}
+// A workgroup per chunk, the steps of a run to its wavefronts in turn.  Bound by memory (1,280 bytes a step) where there are many
+// steps, by the chain of look-ups, loads and sums of a run where there are few: a lane knows where a step lies, four steps are asked
+// for together, and a run's 15 sums do not go through LDS.  650,000 steps: 185 -> 174 us, 4.8 TB/s; 80,000: 36 -> 28.
+constexpr int kGeoWaves = 4, kGeoAhead = 4;
 __global__ __launch_bounds__(64 * kGeoWaves) void train_geometry_kernel(
     StepIndex ix, int S, int chunk_steps, int num_chunks, const unsigned char* __restrict__ records,
     const float* __restrict__ falloff, const float* __restrict__ logs, const float* __restrict__ quats,
     float* __restrict__ rows, GeoGrads out) {
-  __shared__ float s_sum[2][kGeoWaves][16];
+  __shared__ __attribute__((aligned(16))) float s_sum[2][kGeoWaves][16];
+  __shared__ ChunkPrims prims;
   const int chunk = (int)blockIdx.x, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63;
-  const int chunk_end = min(S, (chunk + 1) * chunk_steps);
+  const int chunk_begin = chunk * chunk_steps, chunk_end = min(S, chunk_begin + chunk_steps);
+  load_chunk(ix, S, chunk_begin, chunk_end, threadIdx.x, 64 * kGeoWaves, prims);
+  __syncthreads();
   int turn = 0;
-  for (int pos = chunk * chunk_steps; pos < chunk_end; turn ^= 1) {
-    const StepRun run = step_run(ix, pos, chunk_end);
+  for (int pos = chunk_begin; pos < chunk_end; turn ^= 1) {
+    const StepRun run = chunk_run(prims, pos, chunk_begin, chunk_end, l);
     const size_t p = (size_t)run.p;
+    const int4 where = walk_steps<kGeoWaves>(ix, run.begin + wave, run.end, l);
+    const int count = (run.end - run.begin - wave + kGeoWaves - 1) / kGeoWaves;
     const float qw = quats[p * 4], qx = quats[p * 4 + 1], qy = quats[p * 4 + 2], qz = quats[p * 4 + 3];
     const float mx = det_exp(-2.f * logs[p * 3]), my = det_exp(-2.f * logs[p * 3 + 1]), mz = det_exp(-2.f * logs[p * 3 + 2]);
-    float v[15];
+    float v[16];
 #pragma unroll
-    for (int k = 0; k < 15; ++k) v[k] = 0.f;
-#pragma unroll 2
-    for (int k = run.begin + wave; k < run.end; k += kGeoWaves) {
-      const int4 at = ix.step[k];
-      const float4 c = reinterpret_cast<const float4*>(records + (size_t)at.x * kStepBytes + kStepPlaneC)[l];
-      const float a = falloff[(size_t)at.y * 64 + l];
-      const float dx = c.x, dy = c.y, dz = c.z;
-      const Vec3 q = quat_rotate_conj(qw, qx, qy, qz, Vec3{dx, dy, dz});
-      const float gx = -a * mx * q.x, gy = -a * my * q.y, gz = -a * mz * q.z;
-      v[0] += gx;
-      v[1] += gy;
-      v[2] += gz;
-      v[3] += a * mx * q.x * q.x;
-      v[4] += a * my * q.y * q.y;
-      v[5] += a * mz * q.z * q.z;
-      v[6] += dx * gx; v[7] += dx * gy; v[8] += dx * gz;
-      v[9] += dy * gx; v[10] += dy * gy; v[11] += dy * gz;
-      v[12] += dz * gx; v[13] += dz * gy; v[14] += dz * gz;
+    for (int k = 0; k < 16; ++k) v[k] = 0.f;
+    for (int first = 0; first < count; first += kGeoAhead) {
+      float4 offset[kGeoAhead];
+      float fall[kGeoAhead];
+#pragma unroll
+      for (int u = 0; u < kGeoAhead; ++u) {
+        const int k = min(first + u, count - 1);
+        offset[u] = reinterpret_cast<const float4*>(records + (size_t)__builtin_amdgcn_readlane(where.x, k) * kStepBytes + kStepPlaneC)[l];
+        fall[u] = falloff[(size_t)__builtin_amdgcn_readlane(where.y, k) * 64 + l];
+      }
+#pragma unroll
+      for (int u = 0; u < kGeoAhead; ++u) {
+        if (first + u >= count) break;
+        const float a = fall[u], dx = offset[u].x, dy = offset[u].y, dz = offset[u].z;
+        const Vec3 q = quat_rotate_conj(qw, qx, qy, qz, Vec3{dx, dy, dz});
+        const float gx = -a * mx * q.x, gy = -a * my * q.y, gz = -a * mz * q.z;
+        v[0] += gx;
+        v[1] += gy;
+        v[2] += gz;
+        v[3] += a * mx * q.x * q.x;
+        v[4] += a * my * q.y * q.y;
+        v[5] += a * mz * q.z * q.z;
+        v[6] += dx * gx; v[7] += dx * gy; v[8] += dx * gz;
+        v[9] += dy * gx; v[10] += dy * gy; v[11] += dy * gz;
+        v[12] += dz * gx; v[13] += dz * gy; v[14] += dz * gz;
+      }
     }
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
+    for (int k = 0; k < 15; ++k) v[k] = sum_in_last_lane(v[k]);
+    if (l == 63) {
 #pragma unroll
-      for (int k = 0; k < 15; ++k) v[k] += __shfl_xor(v[k], d);
-    }
-    if (l < 15) {
-      float mine = v[0];
-#pragma unroll
-      for (int k = 1; k < 15; ++k) mine = (l == k) ? v[k] : mine;
-      s_sum[turn][wave][l] = mine;
+      for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<float4*>(&s_sum[turn][wave][4 * k]) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
     }
     __syncthreads();                   // (the one barrier of a turn: the next writes the other half)
     if (wave == 0) {
@@ -396,7 +417,7 @@ __global__ __launch_bounds__(64 * kGeoWaves) void train_geometry_kernel(
         if (l < 15) run_row(rows, run, chunk, num_chunks)[kGradFloats + l] = total;
       } else {
 #pragma unroll
-        for (int k = 0; k < 15; ++k) v[k] = __shfl(total, k);
+        for (int k = 0; k < 15; ++k) v[k] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(total), k));
         if (l == 0) geometry_store(v, qw, qx, qy, qz, p, out);
       }
     }
@@ -432,16 +453,10 @@ __device__ __forceinline__ StepRecord step_record(const unsigned char* __restric
   r.mask2 = reinterpret_cast<const uint32_t*>(rec + kStepPlaneD)[px];
   return r;
 }
-// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on.  Lane i asks for where the i-th of them lies
-// (walk_steps), the first record is requested beside the run's weights (walk_record), and walk_halves has the next record under
-// way while one is worked on (two or three: no faster): work(record) for those that have an adjoint.  Records without one get
-// inputs of zero, whatever ray their lane has.  A wavefront without a step (first >= end) asks for the last one's and drops it.
-template <int STRIDE>
-__device__ __forceinline__ int4 walk_steps(const StepIndex& ix, int first, int end, int lane) {
-  static_assert(kTrainChunk <= 64 * STRIDE, "a lane for every step");
-  asm volatile("" : "+v"(lane));         // (as in chunk_run)
-  return ix.step[min(first + STRIDE * lane, end - 1)];
-}
+// A wavefront's share of a run: one half of every STRIDE-th step, from `first` on (walk_steps).  The first record is requested
+// beside the run's weights (walk_record), and walk_halves has the next record under way while one is worked on (two or three: no
+// faster): work(record) for those that have an adjoint.  Records without one get inputs of zero, whatever ray their lane has.  A
+// wavefront without a step (first >= end) asks for the last one's and drops it.
 __device__ __forceinline__ StepRecord walk_record(const int4& where, int k, int half, const unsigned char* __restrict__ records,
                                                   const float4* __restrict__ d4, const float* __restrict__ rays_d, int W,
                                                   int pixels, int lane) {
