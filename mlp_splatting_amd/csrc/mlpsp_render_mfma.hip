@@ -17,7 +17,7 @@
 #include "mlpsp_team.hpp"
 
 // 32-channel accumulator tiles per wavefront of the feature GEMM: a block of four wavefronts covers 128 x this many
-// channels of a tile (2: three blocks per CU instead of two, a few percent faster than 4 on 512 channels)
+// channels of a tile (2: four blocks per CU instead of two; with three it was a few percent faster than 4 on 512 channels)
 #ifndef MLPSP_GEMM_NCB
 #define MLPSP_GEMM_NCB 2
 #endif
@@ -868,11 +868,15 @@ __global__ __launch_bounds__(256) void pack_feat_kernel(const SRC* __restrict__ 
 //
 // The product is bound by the latency of its operand loads, not by the matrix cores (13 K-steps per tile on
 // average, each needing 4 KB of attributes per record from L2), so the operands go through LDS in chunks of
-// kGemmChunk records: all 256 threads request the chunk's attribute rows (the block's channel slice, up to 4 KB per
+// 16 records (8 of eight slots): all 256 threads request the chunk's attribute rows (the block's channel slice, up to 4 KB per
 // record for 4 slots) and its coefficient records (contiguous in the pool: a pool chunk is kHitChunk records) at
-// once -- ten or more 16-byte loads in flight per thread instead of one K-step's -- then write them to LDS, and
-// after a barrier the wavefronts multiply out of LDS (8-byte or 16-byte reads, lanes on consecutive addresses).
-// Two or three blocks share a CU, so one block's loads overlap another's multiplications and stores.  (Holding the
+// once -- ten 16-byte loads in flight per thread instead of one K-step's -- then write them to
+// LDS, and after a barrier the wavefronts multiply out of LDS (8-byte or 16-byte reads, lanes on consecutive addresses).
+// Four blocks share a CU, so one block's loads overlap another's multiplications and stores: the chunk is a quarter of a CU's LDS
+// to the byte, so what names the records -- pool places, primitives -- lies in the wavefronts' lanes, requested a window ahead, and
+// is read out with v_readlane (a wavefront's loads are of one row at a time); the rows' loads stand under no condition, and LDS
+// addresses are formed anew, which keeps the kernel at 124 registers.  1200x680, 200,000 primitives, 512 channels: three blocks
+// with the names in LDS 641 us, this 591; both slices of a tile side by side, for the coefficients in L2: 599.  (Holding the
 // next chunk's loads in registers across the multiplication measured slower: the registers cost a block per CU.)
 // K-slot j of lane group g is (record 16/SP * step + g * 8/SP + j / SP, slot j % SP).
 template <int SP>
@@ -880,8 +884,9 @@ struct GemmChunk {
   static constexpr int kRecords = 64 / SP;      // 16 records of 4 slots, 8 records of 8: K = 64 per chunk
 };
 
-template <int SP, int NCB>
-__global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restrict__ attr, HitPool hp,
+// WIDE: rows start on 16-byte boundaries.
+template <int SP, int NCB, bool WIDE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 3, 4))) void feat_gemm_kernel(const unsigned* __restrict__ attr, HitPool hp,
                                                         const int32_t* __restrict__ offsets, int C, int W, int H,
                                                         int ntx, int per_xcd, int num_tiles,
                                                         float* __restrict__ out_feat) {
@@ -889,7 +894,7 @@ __global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restri
   // and a primitive's attribute row is fetched into that L2 once for all of them
   const int tile = superblock_tile(blockIdx.x, ntx, num_tiles / ntx);
   if (tile < 0) return;
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 5, m = l & 31;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), l = threadIdx.x & 63, g = l >> 5, m = l & 31;
   constexpr int EPL = 8 / SP;         // records per lane group and K-step
   constexpr int STEP = 2 * EPL;       // records per K-step (one MFMA per accumulator tile)
   constexpr int DW = SP / 2;          // dwords per (record, pixel) and per (primitive, channel)
@@ -897,12 +902,12 @@ __global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restri
   constexpr int kSlice = 128 * NCB;   // channels per block
   constexpr int kRowDw = kSlice * DW; // dwords of one record's attribute row slice in LDS
   constexpr int kCoefDw = 64 * DW;    // dwords of one coefficient record
-  constexpr int kStage = 512;         // records whose pool slot and primitive id are staged in LDS at a time
+  constexpr int kWindow = 64;         // records whose pool slot and primitive id a wavefront's lanes hold at a time
+  static_assert(kWindow % R == 0 && kRowDw / 4 % 64 == 0, "whole chunks; a wavefront loads from one row at a time");
   static_assert(kHitChunk % R == 0, "a chunk of the product lies inside one chunk of the record pool");
   __shared__ __attribute__((aligned(16))) unsigned s_b[R * kRowDw];
   __shared__ __attribute__((aligned(16))) unsigned s_a[R * kCoefDw];
-  __shared__ int s_slot[kStage / R];  // pool slot of the first record of each staged chunk
-  __shared__ int s_prim[kStage];
+  static_assert(4 * (sizeof(s_a) + sizeof(s_b)) <= 163840 || NCB != 2, "four workgroups to a CU");
   const int slice0 = (int)blockIdx.y * kSlice;           // first channel of the block
   const int c0 = slice0 + wave * (32 * NCB);
   const bool active = c0 < C;              // a wavefront without channels still helps staging and meets the barriers
@@ -919,47 +924,51 @@ __global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restri
 
   // dwords of an attribute row that belong to this block's slice and exist: [0, row_dw)
   const int row_dw = min(kSlice, C - slice0) * DW;
-  const bool wide = ((C * DW) & 3) == 0;                // rows start on 16-byte boundaries
   constexpr int kBLoads = R * kRowDw / 4 / 256;          // 16-byte pieces of the chunk's rows per thread
   constexpr int kALoads = R * kCoefDw / 4 / 256;         // ... of its coefficient records
   static_assert(kBLoads * 256 * 4 == R * kRowDw && kALoads * 256 * 4 == R * kCoefDw, "whole pieces per thread");
 
-  for (int base = 0; base < hits; base += kStage) {
-    const int n = min(kStage, hits - base);
-    // record -> primitive id (and chunk -> pool slot) once per block, so that the chunk loop below has a single
-    // level of global loads to wait for
-    for (int k = threadIdx.x; k < n; k += 256) {
-      const int rs = hit_slot(hp, table_base, base + k);
-      if ((k & (R - 1)) == 0) s_slot[k / R] = rs;
-      s_prim[k] = hp.hit_ids[rs];
+  // Places of the records' pool chunks, 64 at a time, one in each lane, and the primitives of a window of 64 records, the next
+  // window's requested while this one is worked on.
+  constexpr int kSpan = 64 * kHitChunk;
+  const auto places = [&](int base) { return hp.chunk_table[table_base + min(base + kHitChunk * l, hits - 1) / kHitChunk]; };
+  const auto primitive = [&](int places, int record) {
+    return hp.hit_ids[__shfl(places, (record & (kSpan - 1)) / kHitChunk) * kHitChunk + record % kHitChunk];
+  };
+  int chunks = 0, prim = 0;
+  for (int base = 0; base < hits; base += kWindow) {
+    const int n = min(kWindow, hits - base);
+    if ((base & (kSpan - 1)) == 0) {
+      chunks = places(base);
+      prim = primitive(chunks, min(base + l, hits - 1));
     }
-    __syncthreads();
-    // requests chunk e0 of the staged records into registers (records past the end of the list as zeros)
+    const int next_prim = primitive(chunks, min(base + kWindow + l, hits - 1));     // (of another span: looked up there)
+    // Requests chunk e0 of the window into registers.  Records past the end of the list: the last one's rows -- its own tile's,
+    // so nothing that could not stand beside a zero -- against coefficients of zero.  WIDE: pieces past the end of a row are its
+    // first again, for channels that are not stored, so that no load stands under a condition.
     auto request = [&](int e0, u32x4 (&vb)[kBLoads], u32x4 (&va)[kALoads]) {
-      const int nrec = min(R, n - e0);
+      const int nrec = min(R, n - e0), dw = (int)(threadIdx.x % (kRowDw / 4)) * 4;
 #pragma unroll
       for (int i = 0; i < kBLoads; ++i) {
-        const int piece = threadIdx.x + 256 * i;           // 16-byte piece of the chunk's row slices
-        const int rec = piece / (kRowDw / 4), dw = (piece % (kRowDw / 4)) * 4;
-        vb[i] = u32x4{0u, 0u, 0u, 0u};
-        if (rec < nrec && dw < row_dw) {
-          const unsigned* __restrict__ src = attr + ((size_t)s_prim[e0 + rec] * C + slice0) * DW + dw;
-          if (wide && dw + 3 < row_dw) {
-            vb[i] = *reinterpret_cast<const u32x4*>(src);
-          } else {
+        const int rec = min((64 * wave + 256 * i) / (kRowDw / 4), nrec - 1);
+        const unsigned* __restrict__ row = attr + ((size_t)__builtin_amdgcn_readlane(prim, e0 + rec) * C + slice0) * DW;
+        if constexpr (WIDE) {
+          vb[i] = *reinterpret_cast<const u32x4*>(row + (dw < row_dw ? dw : 0));
+        } else {
+          vb[i] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (dw + j < row_dw) vb[i][j] = src[j];
-          }
+          for (int j = 0; j < 4; ++j)
+            if (dw + j < row_dw) vb[i][j] = row[dw + j];
         }
       }
       const unsigned* __restrict__ coef =
-          reinterpret_cast<const unsigned*>(hp.records + (size_t)s_slot[e0 / R] * hp.record_bytes);
+          reinterpret_cast<const unsigned*>(
+              hp.records + (size_t)(__builtin_amdgcn_readlane(chunks, ((base + e0) & (kSpan - 1)) / kHitChunk) * kHitChunk + e0 % kHitChunk) * hp.record_bytes);
 #pragma unroll
-      for (int i = 0; i < kALoads; ++i) {
-        const int piece = threadIdx.x + 256 * i;
-        va[i] = (piece / (kCoefDw / 4) < nrec) ? *reinterpret_cast<const u32x4*>(coef + piece * 4) : u32x4{0u, 0u, 0u, 0u};
-      }
+      for (int i = 0; i < kALoads; ++i) va[i] = *reinterpret_cast<const u32x4*>(coef + (threadIdx.x + 256 * i) * 4);
+#pragma unroll
+      for (int i = 0; i < kALoads; ++i)          // (what lies behind the list's end was never written)
+        if ((int)(threadIdx.x + 256 * i) / (kCoefDw / 4) >= nrec) va[i] = u32x4{0u, 0u, 0u, 0u};
     };
     for (int e0 = 0; e0 < n; e0 += R) {
       const int nrec = min(R, n - e0);
@@ -973,6 +982,8 @@ __global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restri
       __syncthreads();
       // ---- multiply
       if (active) {
+        int m = l & 31, g = l >> 5;
+        asm volatile("" : "+v"(m), "+v"(g));      // (or the addresses are formed ahead of the loop and spilled)
 #pragma unroll
         for (int ks = 0; ks < R / STEP; ++ks) {
           if (ks * STEP >= nrec) break;
@@ -1014,6 +1025,7 @@ __global__ __launch_bounds__(256) void feat_gemm_kernel(const unsigned* __restri
       }
       __syncthreads();
     }
+    prim = next_prim;
   }
   if (!active) return;
 
@@ -1359,11 +1371,12 @@ MLPSP_API int mlpsp_render_tilecenter_mfma_feat(const float* rays_o_dev, const f
 #undef MLPSP_MFMA_GO
   if (sp != 0 && stage != 1) {
     const dim3 ggrid(superblock_grid(ntx, ceil_div(height, 8)), (unsigned)ceil_div(feat_channels, 128 * kGemmNcb)), gblock(256);
-#define MLPSP_FEAT_GEMM(SP)                                                                                       \
-  hipLaunchKernelGGL((feat_gemm_kernel<SP, kGemmNcb>), ggrid, gblock, 0, s, (const unsigned*)packed_feat_dev, hp, \
+#define MLPSP_FEAT_GEMM(SP, WIDE)                                                                                 \
+  hipLaunchKernelGGL((feat_gemm_kernel<SP, kGemmNcb, WIDE>), ggrid, gblock, 0, s, (const unsigned*)packed_feat_dev, hp, \
                      tile_offsets_dev, feat_channels, width, height, ntx, per_xcd, (int)T, out_feat_dev)
-    if (sp == 4) MLPSP_FEAT_GEMM(4);
-    else MLPSP_FEAT_GEMM(8);
+    if (sp != 4) MLPSP_FEAT_GEMM(8, true);
+    else if (feat_channels % 2 == 0) MLPSP_FEAT_GEMM(4, true);
+    else MLPSP_FEAT_GEMM(4, false);
 #undef MLPSP_FEAT_GEMM
     MLPSP_LAUNCH_CHECK();
     // status_dev[1] = 1 if the record pool was too small (the feature image is then incomplete)

@@ -282,6 +282,37 @@ def test_matrix_core_feature_image_on_a_ragged_frame(device, oracle_mod, channel
     assert scale > 1e-2 and 0 < err <= TOL[True] * max(1.0, scale)
 
 
+@pytest.mark.parametrize("slots,channels", [(4, 64), (4, 37), (5, 64)])
+@pytest.mark.parametrize("lengths", [(0, 1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 127, 128, 129), (1023, 3, 1024, 1025, 1100)])
+def test_feature_product_of_tiles_of_every_length(device, lengths, slots, channels):
+    """The product looks up 64 records at a time, the places of 1,024, and multiplies chunks of 16 (8 of five slots): lists that
+    end around these, of primitives that all hit and hardly cover, each with its attribute in one channel -- a record lost or
+    taken twice moves a channel of at most 30 by a thirtieth -- against the exact path.  fp16 operands move an opacity's logit, a
+    sum of 32 products of numbers below 1, by 32 x 2^-11 / 2 at the most: 1 % of the weight."""
+    from mlp_splatting_amd import synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    n, width, height = max(lengths), 8 * len(lengths), 8
+    sc = syn.make_scene(n, 32, seed=4, log_scale_mean=2.5)
+    sc.positions[:] = np.array([0.0, 0.0, 9.0]) + 0.1 * sc.positions
+    sc.b3[:, 3] = -6.0
+    ro, rd = syn.pinhole_rays(width, height, 2.0 * width, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
+    cand = np.concatenate([np.arange(n - k, n) for k in lengths]).astype(np.int32)
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    x = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats, cand, off, sc.freq,
+                                     sc.att, *sc.mlp())]
+    fa = torch.zeros(n, slots, channels, device=device)
+    fa[torch.arange(n), :, torch.arange(n) % channels] = 1.0
+    ext = TileExt()
+    _, alpha, feat = ext.render_tiles_rgb_wmma_with_feat(x, fa, 1.0, 4.0, width, height, 1e-3, False)
+    exact = ext.render_tiles_forward_tilecenter_with_feat(*x, fa, 1.0, 4.0, width, height, 8, 8, 1e-3)
+    assert ext.rgb_wmma_safety_stats()[1] == 0 and 0 < float(alpha.max()) < 0.999       # (no tile ends before its list)
+    for tile, length in enumerate(lengths):
+        at = torch.arange(width * height, device=device).view(height, width)[:, 8 * tile:8 * tile + 8].reshape(-1)
+        got, want = feat[at], exact[2][at]
+        assert float(want.max()) > 0 or length == 0
+        assert float((got - want).abs().max()) <= 0.015 * float(want.max()), (tile, length)
+
+
 def test_matrix_core_feature_render_with_separate_origins(device, oracle_mod):
     from mlp_splatting_amd import ops
     fr = Frame("cfg1_5k_160x120", n=1200, hidden=32, width=56, height=40, feature_dim=72, feature_slots=4)
