@@ -550,12 +550,15 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  *   (mlpsp_train_scratch_bytes(num_steps, num_primitives) bytes, 256-byte aligned; all of it is scratch of the call).
  * mlpsp_train_gradients: the nine gradients, written whole, from a scratch_dev that mlpsp_train_group has filled.
  *   precision, scale: as mlpsp_grouped_vjp; nonfinite_dev[0] becomes 1 if a weight gradient is not finite.
+ *   _beside: and zeros into the rows (row_floats floats each) of rows_dev that belong to primitives without a step.
  *
  * mlpsp_train_feature_l1 / _gradients: the streamed feature L1 loss of mlpsp_stream_feature_l1 and its attribute gradient
  *   (mlpsp_feature_attribute_gradients, times the loss adjoint loss_adjoint_dev[0]) from the steps; arguments as there, beta
  *   and temp as in the record forward.  mlpsp_train_feature_bytes returns the size of kept_dev (what the gradients need,
  *   256-byte aligned) and fills share_bytes (shares_dev, scratch of the loss), loss_partials (floats; their sum is the loss)
- *   and row_bytes (rows_dev, scratch of the gradients); 0 = invalid shape.  scratch_dev: filled by mlpsp_train_group. */
+ *   and row_bytes (rows_dev, scratch of the gradients); 0 = invalid shape.  scratch_dev: filled by mlpsp_train_group.
+ *   mlpsp_train_feature_gradients_listed leaves the rows of primitives without a step as they are (for
+ *   mlpsp_train_gradients_beside, which waits for products, not for memory, and writes them in passing). */
 #define MLPSP_STEP_CHUNK 8
 size_t mlpsp_train_workspace_bytes(int64_t num_pairs, int width, int height, int64_t pool_steps);
 int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
@@ -586,6 +589,15 @@ int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int width, int h
                           float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev, float* gb3_dev,
                           float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev,
                           int32_t* nonfinite_dev, mlpsp_stream_t stream);
+int mlpsp_train_gradients_beside(int64_t num_steps, int64_t num_pairs, int width, int height,
+                          const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,
+                          const float* falloff_dev, const float* rays_d_dev, const float* freq_dev,
+                          const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2,
+                          const float* W3, const float* log_scales_dev, const float* quats_dev, int num_primitives,
+                          int precision, float scale, void* scratch_dev, size_t scratch_bytes, float* gW1_dev,
+                          float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev, float* gb3_dev,
+                          float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev,
+                          int32_t* nonfinite_dev, float* rows_dev, int row_floats, mlpsp_stream_t stream);
 
 size_t mlpsp_train_feature_bytes(int width, int height, int target_width, int target_height, int channels, int slots,
                                  int64_t num_steps, size_t* share_bytes, int64_t* loss_partials, size_t* row_bytes);
@@ -596,6 +608,10 @@ int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t num_pairs, i
                            float temp, void* kept_dev, size_t kept_bytes, float* shares_dev, float* loss_partials_dev,
                            mlpsp_stream_t stream);
 int mlpsp_train_feature_gradients(int64_t num_steps, int width, int height,
+                                  int target_width, int target_height, int channels, int slots, const void* kept_dev,
+                                  size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes, int num_primitives,
+                                  const float* loss_adjoint_dev, float* rows_dev, float* out_dev, mlpsp_stream_t stream);
+int mlpsp_train_feature_gradients_listed(int64_t num_steps, int width, int height,
                                   int target_width, int target_height, int channels, int slots, const void* kept_dev,
                                   size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes, int num_primitives,
                                   const float* loss_adjoint_dev, float* rows_dev, float* out_dev, mlpsp_stream_t stream);

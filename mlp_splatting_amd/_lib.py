@@ -106,9 +106,12 @@ SIGNATURES = {
     "mlpsp_train_scratch_bytes": (_sz, [_i64, _i]),
     "mlpsp_train_group": (_i, [_vp, _i64, _i, _i, _vp, _sz, _i64, _i, _vp, _sz, _vp]),
     "mlpsp_train_gradients": (_i, [_i64, _i64, _i, _i, _vp, _sz] + [_vp] * 12 + [_i, _i, _f, _vp, _sz] + [_vp] * 11),
+    "mlpsp_train_gradients_beside": (_i, [_i64, _i64, _i, _i, _vp, _sz] + [_vp] * 12 + [_i, _i, _f, _vp, _sz] + [_vp] * 11
+                                     + [_i, _vp]),
     "mlpsp_train_feature_bytes": (_sz, [_i] * 6 + [_i64, _vp, _vp, _vp]),
     "mlpsp_train_feature_l1": (_i, [_vp, _i64, _i, _i, _vp, _sz, _i64, _vp, _vp, _vp] + [_i] * 5 + [_f, _f, _vp, _sz, _vp, _vp, _vp]),
     "mlpsp_train_feature_gradients": (_i, [_i64] + [_i] * 6 + [_vp, _sz, _vp, _sz, _i] + [_vp] * 4),
+    "mlpsp_train_feature_gradients_listed": (_i, [_i64] + [_i] * 6 + [_vp, _sz, _vp, _sz, _i] + [_vp] * 4),
     "mlpsp_records_reverse": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _vp, _vp, _vp, _vp, _vp]),
 }
 

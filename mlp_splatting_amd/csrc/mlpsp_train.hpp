@@ -152,8 +152,8 @@ __device__ __forceinline__ void step_store(const StepPool& sp, int slot, int lan
 // of its own; the weight gradient kernels, which leave memory three quarters idle, do it beside their products (BESIDE: past the
 // caches, where what they read lies; a launch of its own is 2 % slower that way).
 struct ZeroRows {
-  float* base[9];
-  int len[9];        // floats per primitive
+  float* base[10];
+  int len[10];       // floats per primitive
   int count;
   void add(float* p, int floats) {
     base[count] = p;

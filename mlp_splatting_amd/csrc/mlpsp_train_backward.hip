@@ -484,7 +484,7 @@ __device__ __forceinline__ void walk_halves(const int4& where, StepRecord next, 
 // the stores go on beside the products of the others.  The whole call at 648,000 steps of 200,000 primitives with these 2.8 GB in
 // a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 / 1.70; a primitive per block of
 // products 5.34 and 1.83.  Ahead of the chunk its first record is waited for behind the stores: the f32 kernel of 80,000 steps
-// takes 676 us instead of 663.
+// takes 676 us instead of 663.  With the rows of the attributes' gradient (512 channels, four slots: 1.3 GB more) fp16 1.52 -> 1.62.
 template <int WAVES>
 __device__ __forceinline__ void zero_share(const StepIndex& ix, int N, const ZeroRows& zero, int chunk, int num_chunks, int wave,
                                            int lane) {
@@ -776,7 +776,8 @@ MLPSP_API int mlpsp_train_group(const int32_t* tile_offsets_dev, int64_t num_pai
   return MLPSP_OK;
 }
 
-MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int width,
+namespace {
+int train_gradients(int64_t num_steps, int64_t num_pairs, int width,
                                     int height, const void* workspace_dev, size_t workspace_bytes, const float* d4_dev,
                                     const float* falloff_dev, const float* rays_d_dev, const float* freq_dev,
                                     const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2,
@@ -784,7 +785,7 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
                                     int precision, float scale, void* scratch_dev, size_t scratch_bytes, float* gW1_dev,
                                     float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev, float* gb3_dev,
                                     float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev,
-                                    int32_t* nonfinite_dev, mlpsp_stream_t stream) {
+                                    int32_t* nonfinite_dev, float* rows_dev, int row_floats, hipStream_t s) {
   const int64_t T = checked_num_tiles(width, height, 8, 8);
   if (T <= 0 || num_pairs < 0 || num_pairs > 2147483647LL || num_steps < 0 || num_steps > 2147483647LL || num_primitives <= 0)
     return MLPSP_E_ARGUMENT;
@@ -800,7 +801,6 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
        (uintptr_t)gb1_dev | (uintptr_t)gW2_dev | (uintptr_t)gb2_dev | (uintptr_t)gW3_dev | (uintptr_t)gb3_dev) & 15u)
     return MLPSP_E_ARGUMENT;
   const StepPool sp = step_pool_carve(const_cast<void*>(workspace_dev), workspace_bytes, num_pairs, T);
-  hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(nonfinite_dev, sizeof(int32_t), s));
   const StepIndex ix{t.prim, t.first, t.step};
   const GradRows grads{gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev, gb3_dev};
@@ -817,6 +817,7 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
   zero.add(grad_positions_dev, 3);
   zero.add(grad_log_scales_dev, 3);
   zero.add(grad_quats_dev, 4);
+  if (rows_dev) zero.add(rows_dev, row_floats);
   if (num_chunks > 0) {
 #define MLPSP_TRAIN_VJP(KERNEL, THREADS)                                                                                \
   hipLaunchKernelGGL(KERNEL, dim3((unsigned)num_chunks), dim3(THREADS), 0, s, ix, S, chunk_steps, num_chunks, sp.records, \
@@ -838,4 +839,34 @@ MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int wi
     MLPSP_LAUNCH_CHECK();
   }
   return MLPSP_OK;
+}
+}  // namespace
+
+MLPSP_API int mlpsp_train_gradients(int64_t num_steps, int64_t num_pairs, int width, int height, const void*
+    workspace_dev, size_t workspace_bytes, const float* d4_dev, const float* falloff_dev, const float* rays_d_dev, const
+    float* freq_dev, const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2, const
+    float* W3, const float* log_scales_dev, const float* quats_dev, int num_primitives, int precision, float scale, void*
+    scratch_dev, size_t scratch_bytes, float* gW1_dev, float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev,
+    float* gb3_dev, float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev, int32_t* nonfinite_dev,
+    mlpsp_stream_t stream) {
+  return train_gradients(num_steps, num_pairs, width, height, workspace_dev, workspace_bytes, d4_dev, falloff_dev,
+                         rays_d_dev, freq_dev, att_dev, W1, b1, W2, b2, W3, log_scales_dev, quats_dev, num_primitives,
+                         precision, scale, scratch_dev, scratch_bytes, gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev,
+                         gb3_dev, grad_positions_dev, grad_log_scales_dev, grad_quats_dev, nonfinite_dev, nullptr, 0,
+                         (hipStream_t)stream);
+}
+
+MLPSP_API int mlpsp_train_gradients_beside(int64_t num_steps, int64_t num_pairs, int width, int height, const void*
+    workspace_dev, size_t workspace_bytes, const float* d4_dev, const float* falloff_dev, const float* rays_d_dev, const
+    float* freq_dev, const float* att_dev, const float* W1, const float* b1, const float* W2, const float* b2, const
+    float* W3, const float* log_scales_dev, const float* quats_dev, int num_primitives, int precision, float scale, void*
+    scratch_dev, size_t scratch_bytes, float* gW1_dev, float* gb1_dev, float* gW2_dev, float* gb2_dev, float* gW3_dev,
+    float* gb3_dev, float* grad_positions_dev, float* grad_log_scales_dev, float* grad_quats_dev, int32_t* nonfinite_dev,
+    float* rows_dev, int row_floats, mlpsp_stream_t stream) {
+  if (!rows_dev || row_floats <= 0) return MLPSP_E_ARGUMENT;
+  return train_gradients(num_steps, num_pairs, width, height, workspace_dev, workspace_bytes, d4_dev, falloff_dev,
+                         rays_d_dev, freq_dev, att_dev, W1, b1, W2, b2, W3, log_scales_dev, quats_dev, num_primitives,
+                         precision, scale, scratch_dev, scratch_bytes, gW1_dev, gb1_dev, gW2_dev, gb2_dev, gW3_dev,
+                         gb3_dev, grad_positions_dev, grad_log_scales_dev, grad_quats_dev, nonfinite_dev, rows_dev,
+                         row_floats, (hipStream_t)stream);
 }

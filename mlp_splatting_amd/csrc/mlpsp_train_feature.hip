@@ -15,9 +15,10 @@
 //   train_attr_join_kernel      rows of primitives that span chunks
 //
 // All are bound by memory traffic: attribute rows out of L2 in the blend (8 KB per step at 512 channels, four slots), sign
-// rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each).  At 200,000 primitives,
-// 1200x680, a 300x170 target of 512 channels: 0.45, 0.06, 0.20 and 0.28 ms; the record kernels took 4.95 ms for the
-// loss and 8.1 ms for the gradient.
+// rows (2 KB) in the gradient; then come the zeros of the primitives without a step (8 KB each), in a launch of their own or,
+// where weight gradients are asked for too, by their kernel (_listed: 0.26 ms less here, 0.10 more there, and what comes next
+// does not meet the last of them on their way).  At 200,000 primitives, 1200x680, a 300x170 target of 512 channels: 0.45, 0.06,
+// 0.20 and 0.26 ms; the record kernels took 4.95 ms for the loss and 8.1 ms for the gradient.
 #include <type_traits>
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
@@ -606,11 +607,11 @@ MLPSP_API int mlpsp_train_feature_l1(const int32_t* tile_offsets_dev, int64_t nu
   return MLPSP_OK;
 }
 
-MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int height,
-                                            int target_width, int target_height, int channels, int slots,
-                                            const void* kept_dev, size_t kept_bytes, const void* scratch_dev,
-                                            size_t scratch_bytes, int num_primitives, const float* loss_adjoint_dev,
-                                            float* rows_dev, float* out_dev, mlpsp_stream_t stream) {
+namespace {
+int train_feature_gradients(int64_t num_steps, int width, int height, int target_width, int target_height, int channels, int slots,
+                            const void* kept_dev, size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes,
+                            int num_primitives, const float* loss_adjoint_dev, float* rows_dev, float* out_dev, bool zeros,
+                            hipStream_t s) {
   FeatShape f;
   if (!feat_shape(width, height, target_width, target_height, channels, slots, f) || num_steps < 0 ||
       num_steps > 2147483647LL || num_primitives < 0)
@@ -622,7 +623,6 @@ MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int he
   if (num_primitives == 0) return MLPSP_OK;
   if (!loss_adjoint_dev || !out_dev || (num_steps > 0 && (!rows_dev || ((uintptr_t)rows_dev & 15u))))
     return MLPSP_E_ARGUMENT;
-  hipStream_t s = (hipStream_t)stream;
   const bool vec = channels % 4 == 0 && ((uintptr_t)out_dev & 15u) == 0;
   const int per = attr_chunk_steps(num_steps, channels), chunks = (int)((num_steps + per - 1) / per);
   if (chunks > 0) {
@@ -648,9 +648,24 @@ MLPSP_API int mlpsp_train_feature_gradients(int64_t num_steps, int width, int he
                          (int)num_steps, per, chunks, unit, loss_adjoint_dev, rows_dev, out_dev);
     MLPSP_LAUNCH_CHECK();
   }
+  if (!zeros) return MLPSP_OK;
   ZeroRows zero{};
   zero.add(out_dev, slots * channels);
   launch_zero_rows(t.first, num_primitives, zero, s);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }
+}  // namespace
+
+#define MLPSP_FEATURE_GRADIENTS(NAME, ZEROS)                                                                                \
+  MLPSP_API int NAME(int64_t num_steps, int width, int height, int target_width, int target_height, int channels, int slots, \
+                     const void* kept_dev, size_t kept_bytes, const void* scratch_dev, size_t scratch_bytes,                 \
+                     int num_primitives, const float* loss_adjoint_dev, float* rows_dev, float* out_dev,                     \
+                     mlpsp_stream_t stream) {                                                                                \
+    return train_feature_gradients(num_steps, width, height, target_width, target_height, channels, slots, kept_dev,         \
+                                   kept_bytes, scratch_dev, scratch_bytes, num_primitives, loss_adjoint_dev, rows_dev,       \
+                                   out_dev, ZEROS, (hipStream_t)stream);                                                     \
+  }
+MLPSP_FEATURE_GRADIENTS(mlpsp_train_feature_gradients, true)
+MLPSP_FEATURE_GRADIENTS(mlpsp_train_feature_gradients_listed, false)
+#undef MLPSP_FEATURE_GRADIENTS

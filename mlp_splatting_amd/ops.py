@@ -971,8 +971,9 @@ def train_reverse(frame, tile_offsets, grad_rgb, grad_t):
     return d4, falloff
 
 
-def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scales, quats, precision, scale):
-    """([gW1, gb1, gW2, gb2, gW3, gb3, grad_positions, grad_log_scales, grad_quats], non-finite flag int32 [1])."""
+def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scales, quats, precision, scale, beside=None):
+    """([gW1, gb1, gW2, gb2, gW3, gb3, grad_positions, grad_log_scales, grad_quats], non-finite flag int32 [1]).  ``beside``: a
+    contiguous f32 tensor [n, ...] whose rows are set to zero where a primitive has no step."""
     dev = rays_d.device
     n = log_scales.shape[0]
     grads = [torch.empty_like(w) for w in ws[:6]]
@@ -980,11 +981,18 @@ def train_gradients(frame, groups, d4, falloff, rays_d, freq, att, ws, log_scale
     if n == 0:
         return grads + geo, torch.zeros(1, dtype=torch.int32, device=dev)
     flag = torch.empty(1, dtype=torch.int32, device=dev)
-    code = _lib.load().mlpsp_train_gradients(
-        frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace), frame.workspace.numel(), _ptr(d4), _ptr(falloff), _ptr(rays_d), _ptr(freq), _ptr(att), *[_ptr(w) for w in ws[:5]],
-        _ptr(log_scales), _ptr(quats), n, int(precision), float(scale), _ptr(groups), groups.numel(),
-        *[_ptr(g) for g in grads], *[_ptr(g) for g in geo], _ptr(flag), _stream(dev))
-    _check(code, "mlpsp_train_gradients")
+    args = [frame.steps, frame.pairs, frame.width, frame.height, _ptr(frame.workspace), frame.workspace.numel(), _ptr(d4),
+            _ptr(falloff), _ptr(rays_d), _ptr(freq), _ptr(att), *[_ptr(w) for w in ws[:5]], _ptr(log_scales), _ptr(quats), n,
+            int(precision), float(scale), _ptr(groups), groups.numel(), *[_ptr(g) for g in grads], *[_ptr(g) for g in geo],
+            _ptr(flag)]
+    if beside is None:
+        _check(_lib.load().mlpsp_train_gradients(*args, _stream(dev)), "mlpsp_train_gradients")
+    else:
+        if not (beside.is_cuda and beside.dtype == torch.float32 and beside.is_contiguous() and beside.shape[0] == n
+                and beside.numel() < n * 2 ** 31):
+            raise RuntimeError("beside must be a contiguous float32 CUDA tensor with a row for every primitive")
+        _check(_lib.load().mlpsp_train_gradients_beside(*args, _ptr(beside), beside.numel() // n, _stream(dev)),
+               "mlpsp_train_gradients_beside")
     return grads + geo, flag
 
 
@@ -1019,8 +1027,9 @@ def train_feature_l1(frame, tile_offsets, attributes, target, beta, temp):
     return partials.sum(), feature, kept
 
 
-def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoint):
-    """d / d attributes of the loss of :func:`train_feature_l1` times ``loss_adjoint`` (f32 device scalar)."""
+def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoint, out=None):
+    """d / d attributes of the loss of :func:`train_feature_l1` times ``loss_adjoint`` (f32 device scalar).  ``out``: where the
+    rows of primitives with a step go; the others are left as they are (``beside`` of :func:`train_gradients`)."""
     for t in (attributes, loss_adjoint):
         if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
             raise RuntimeError("feature attributes and the loss adjoint must be contiguous float32 CUDA tensors")
@@ -1028,8 +1037,13 @@ def train_feature_gradients(frame, groups, feature, kept, attributes, loss_adjoi
         raise RuntimeError("feature attributes and the loss adjoint do not match the loss they belong to")
     dev = kept.device
     rows = torch.empty(feature.row_bytes, dtype=torch.uint8, device=dev)
-    out = torch.empty_like(attributes)
-    _check(_lib.load().mlpsp_train_feature_gradients(
+    listed = out is not None
+    if listed and not (out.dtype == torch.float32 and out.is_contiguous() and out.shape == attributes.shape and out.device == dev):
+        raise RuntimeError("the attributes' gradient must be a contiguous float32 tensor of their shape")
+    if not listed:
+        out = torch.empty_like(attributes)
+    lib = _lib.load()
+    _check((lib.mlpsp_train_feature_gradients_listed if listed else lib.mlpsp_train_feature_gradients)(
         frame.steps, frame.width, frame.height, *feature.target_size, feature.channels, feature.slots,
         _ptr(kept), feature.kept, _ptr(groups), groups.numel(), attributes.shape[0], _ptr(loss_adjoint),
         _ptr(rows), _ptr(out), _stream(dev)), "mlpsp_train_feature_gradients")

@@ -781,11 +781,11 @@ class TileExt:
                                "transmittance termination; refusing to return truncated gradients")
 
     @classmethod
-    def backward_from_steps(cls, frame, groups, x, grad_rgb, grad_t, dtype=torch.float32):
+    def backward_from_steps(cls, frame, groups, x, grad_rgb, grad_t, dtype=torch.float32, beside=None):
         """The nine gradients of :meth:`render_tiles_backward_tilecenter_full` from a frame's steps; ``x``: the scene
         tensors of the forward, ``groups``: ``ops.train_group`` of the frame, or what returns it (the sort's small launches
-        then are queued while the device works on the reverse walk).  Non-finite policy of
-        ``primitive_gemm.grouped_weight_gradients``."""
+        then are queued while the device works on the reverse walk).  ``beside``: as in ``ops.train_gradients``.  Non-finite
+        policy of ``primitive_gemm.grouped_weight_gradients``."""
         from . import primitive_gemm
         # (what saved-tensor hooks hand back is a tensor of their making: it is held to the forward's contract again)
         cls._check_training_f32(x, frame.width, frame.height)
@@ -800,7 +800,7 @@ class TileExt:
 
             def launch(operand_dtype, scale):
                 return ops.train_gradients(frame, groups, d4, falloff, x[1], x[7], x[8], x[9:15], x[3], x[4],
-                                           primitive_gemm._PRECISION_CODE[operand_dtype], scale)
+                                           primitive_gemm._PRECISION_CODE[operand_dtype], scale, beside)
             return primitive_gemm._checked_grouped_vjp(launch, dtype, 4096.0 if dtype == torch.float16 else 1.0)
 
     def training_wmma_safety_stats(self):

@@ -104,6 +104,33 @@ def test_feature_loss_of_steps_is_that_of_records(device, oracle_mod, wf, hf, ch
     torch.testing.assert_close(got, want * 0.75, rtol=1e-4, atol=2e-6 * float(want.abs().max()))
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("away", [False, True])
+@pytest.mark.parametrize("channels,slots", [(8, 4), (67, 5), (300, 1), (1, 1)])
+def test_zeros_of_the_attribute_gradient_beside_the_weight_gradients(device, oracle_mod, channels, slots, away, precision):
+    """Rows of primitives without a step from the weight gradients, the others from the attribute gradient: together what the
+    attribute gradient writes by itself, and the weight gradients are the same."""
+    from mlp_splatting_amd import ops
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr, base = _scene(device, oracle_mod, 300, 33, 17, 0.3, away)
+    _, _, frame = TileExt().train_forward(base, 33, 17, fr.thr)
+    gen = torch.Generator(device=device).manual_seed(8)
+    attributes = torch.randn(300, slots, channels, device=device, generator=gen)
+    target = torch.randn(5, 9, channels, device=device, generator=gen)
+    _, feature, kept = ops.train_feature_l1(frame, base[6], attributes, target, 1.5, 2.0)
+    groups, one = ops.train_group(frame, base[6], 300), torch.ones(1, device=device)
+    d4 = torch.randn(frame.steps, 64, 4, device=device, generator=gen)
+    args = (frame, groups, d4, d4[..., 0].contiguous(), base[1], base[7], base[8], base[9:15], base[3], base[4], precision, 1.0)
+    rows = torch.full_like(attributes, float("nan"))
+    grads, got = ops.train_gradients(*args)[0], ops.train_gradients(*args, rows)[0]
+    assert all(torch.equal(a, b) for a, b in zip(grads, got))
+    used = torch.zeros(300, dtype=torch.bool, device=device)
+    used[groups.view(torch.int32)[320:320 + frame.steps].long()] = True          # (the sorted primitives, behind 301 ints)
+    assert (rows[~used] == 0).all() and rows[used].isnan().all() and bool(used.any()) != away and not bool(used.all())
+    assert ops.train_feature_gradients(frame, groups, feature, kept, attributes, one, rows) is rows
+    assert torch.equal(rows, ops.train_feature_gradients(frame, groups, feature, kept, attributes, one))
+
+
 def test_feature_training_step_of_an_empty_scene(device, oracle_mod):
     from mlp_splatting_amd.record_training import Frame as TrainingFrame, feature_training_step
     fr, base = _scene(device, oracle_mod, 40, 33, 17, 1.0, False)
