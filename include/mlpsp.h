@@ -544,6 +544,8 @@ int mlpsp_geometry_gradients(const int64_t* csr_offsets_dev, const int64_t* reco
  *   2 = a live pixel reached max_hits), steps}.
  *   If MLPSP_STEP_CHUNK times the first word exceeds pool_steps the pool ran out: image and alpha are complete, the steps are not, and
  *   the caller repeats the call with a pool of that size.
+ *   _mfma_checked: and flag_dev[0] |= 1 if an element of the arrays is NaN or infinite (arguments as mlpsp_all_finite, which
+ *   clears the flag first), by the wavefronts that are done with their tiles where tiles are many.
  * mlpsp_train_reverse: reverse compositing; d4_dev [num_steps, 64, 4] = adjoints of the four pre-activation outputs,
  *   falloff_dev [num_steps, 64] = dL/d(decay) * decay.
  * mlpsp_train_group: the steps (num_steps = the third word) sorted by primitive, into the index part of scratch_dev
@@ -573,6 +575,13 @@ int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, c
                              const float* freq_dev, const float* att_dev, const void* packed_dev, int num_primitives,
                              int width, int height, float threshold, int max_hits, int use_bf16, void* workspace_dev,
                              size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev, mlpsp_stream_t stream);
+int mlpsp_train_forward_mfma_checked(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
+                             const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
+                             const float* freq_dev, const float* att_dev, const void* packed_dev, int num_primitives,
+                             int width, int height, float threshold, int max_hits, int use_bf16, void* workspace_dev,
+                             size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev,
+                             const float* const* arrays_dev, const int64_t* lengths, int num_arrays, int32_t* flag_dev,
+                             mlpsp_stream_t stream);
 int mlpsp_train_reverse(const int32_t* tile_offsets_dev, int64_t num_pairs, int width, int height,
                         const void* workspace_dev, size_t workspace_bytes, const float* grad_rgb_dev,
                         const float* grad_t_dev, float* d4_dev, float* falloff_dev, mlpsp_stream_t stream);

@@ -102,6 +102,8 @@ SIGNATURES = {
     "mlpsp_train_workspace_bytes": (_sz, [_i64, _i, _i, _i64]),
     "mlpsp_train_forward_f32": (_i, [_vp] * 5 + [_i64] + [_vp] * 8 + [_i, _i, _i, _f, _i, _i, _vp, _sz, _vp, _vp, _vp]),
     "mlpsp_train_forward_mfma": (_i, [_vp] * 5 + [_i64] + [_vp] * 3 + [_i, _i, _i, _f, _i, _i, _vp, _sz, _vp, _vp, _vp]),
+    "mlpsp_train_forward_mfma_checked": (_i, [_vp] * 5 + [_i64] + [_vp] * 3 + [_i, _i, _i, _f, _i, _i, _vp, _sz, _vp, _vp]
+                                         + [_vp, _vp, _i, _vp, _vp]),
     "mlpsp_train_reverse": (_i, [_vp, _i64, _i, _i, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "mlpsp_train_scratch_bytes": (_sz, [_i64, _i]),
     "mlpsp_train_group": (_i, [_vp, _i64, _i, _i, _vp, _sz, _i64, _i, _vp, _sz, _vp]),

@@ -19,6 +19,7 @@
 // status bits: 1 numeric (non-finite operand, activation or output -- the caller repeats the frame in f32),
 // 2 hit capacity, 4 count/emit disagreement.
 #include "mlpsp_device.hpp"
+#include "mlpsp_finite.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mfma16.hpp"
 #include "mlpsp_record_stage.hpp"
@@ -48,51 +49,6 @@ __device__ __forceinline__ bool not_finite(float v) { return !(__builtin_fabsf(v
 
 template <bool EMIT> struct StageFor { using type = RecordStage<MLPSP_STAGE_K>; };
 template <> struct StageFor<false> { struct type {}; };
-
-// One read-only pass over up to 16 f32 arrays; flag[0] |= 1 if any element is NaN or infinite
-// (training_wmma.cuh:24-60: one fused scan and one read-back instead of a reduction per tensor).
-struct FiniteScanInputs {
-  const float* pointers[16];
-  long long lengths[16];
-  int count;
-};
-
-// Bound by memory: 2.86 GB of inputs at 200,000 primitives 481 -> 411 us, 6.95 TB/s, against a load at a time in 8,192 blocks that
-// come and go.  Eight loads on their way per thread and blocks that all run at once (512 blocks 419 us, 1,024 483, 2,048 455),
-// past the caches (471 us with 512 blocks through them).
-constexpr int kScanAhead = 8, kScanBlocks = 768;
-__global__ __launch_bounds__(256) void finite_scan_kernel(FiniteScanInputs in, int32_t* __restrict__ flag) {
-  uint32_t most = 0u;                // the largest of the magnitudes, as bits: 0x7f800000 and more are not finite
-  const auto look = [&](float v) { most = max(most, __float_as_uint(v) & 0x7fffffffu); };
-  const long long stride = (long long)blockDim.x * gridDim.x, first = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int t = 0; t < in.count; ++t) {
-    const float* __restrict__ src = in.pointers[t];
-    const long long n = in.lengths[t];
-    // 16-byte loads over the aligned middle, scalar loads for the ragged ends
-    const long long head = min(n, (long long)(((16 - (reinterpret_cast<uintptr_t>(src) & 15)) & 15) / 4));
-    const long long quads = (n - head) / 4;
-    const f32x4* __restrict__ mid = reinterpret_cast<const f32x4*>(src + head);
-    long long i = first;
-    for (; i + (kScanAhead - 1) * stride < quads; i += kScanAhead * stride) {
-      f32x4 v[kScanAhead];
-#pragma unroll
-      for (int k = 0; k < kScanAhead; ++k) v[k] = __builtin_nontemporal_load(mid + i + k * stride);
-#pragma unroll
-      for (int k = 0; k < kScanAhead; ++k) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) look(v[k][q]);
-      }
-    }
-    for (; i < quads; i += stride) {
-      const f32x4 v = mid[i];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) look(v[q]);
-    }
-    for (long long i = first; i < head; i += stride) look(src[i]);
-    for (long long i = head + 4 * quads + first; i < n; i += stride) look(src[i]);
-  }
-  if (__ballot(most >= 0x7f800000u) != 0ull && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
-}
 
 template <typename T, bool EMIT>
 __device__ __forceinline__ void records_mfma_body(
@@ -304,25 +260,13 @@ MLPSP_API int mlpsp_records_mfma_emit(const float* rays_o_dev, const float* rays
 
 MLPSP_API int mlpsp_all_finite(const float* const* arrays_dev, const int64_t* lengths, int num_arrays, int32_t* flag_dev,
                                mlpsp_stream_t stream) {
-  if (num_arrays < 0 || num_arrays > 16 || !flag_dev || (num_arrays > 0 && (!arrays_dev || !lengths)))
-    return MLPSP_E_ARGUMENT;
+  if (!flag_dev) return MLPSP_E_ARGUMENT;
   FiniteScanInputs in{};
-  long long largest = 0;
-  for (int t = 0; t < num_arrays; ++t) {
-    if (lengths[t] < 0 || (lengths[t] > 0 && !arrays_dev[t])) return MLPSP_E_ARGUMENT;
-    if (lengths[t] == 0) continue;
-    if ((reinterpret_cast<uintptr_t>(arrays_dev[t]) & 3) != 0) return MLPSP_E_ARGUMENT;
-    in.pointers[in.count] = arrays_dev[t];
-    in.lengths[in.count] = lengths[t];
-    largest = lengths[t] > largest ? lengths[t] : largest;
-    ++in.count;
-  }
+  if (!finite_scan_inputs(arrays_dev, lengths, num_arrays, in)) return MLPSP_E_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(flag_dev, sizeof(int32_t), s));
   if (in.count == 0) return MLPSP_OK;
-  const long long want = (largest / 4 + 255) / 256;
-  const unsigned blocks = (unsigned)(want < 1 ? 1 : (want > kScanBlocks ? kScanBlocks : want));
-  hipLaunchKernelGGL(finite_scan_kernel, dim3(blocks), dim3(256), 0, s, in, flag_dev);
+  launch_finite_scan(in, flag_dev, s);
   MLPSP_LAUNCH_CHECK();
   return MLPSP_OK;
 }

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "mlpsp_device.hpp"
+#include "mlpsp_finite.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mfma16.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -294,11 +295,18 @@ __global__ __launch_bounds__(train_workgroup(TEAM)) __attribute__((amdgpu_waves_
 }
 template <typename T, int TEAM>
 __global__ __launch_bounds__(train_workgroup(TEAM)) __attribute__((amdgpu_waves_per_eu(4, 4))) void train_forward_mfma_kernel(
-    MLPSP_TRAIN_PARAMS, const unsigned char* __restrict__ packed, MLPSP_TRAIN_TAIL) {
+    MLPSP_TRAIN_PARAMS, const unsigned char* __restrict__ packed, MLPSP_TRAIN_TAIL, FiniteScanInputs scan,
+    int32_t* __restrict__ nonfinite) {
   const TrainScene c{rays_o, rays_d, prims, order, offsets, freq, att, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, packed,
                      N, W, H, ntx, nty, thr, max_hits};
-  if constexpr (TEAM == 0) train_forward_body<T, false>(c, sp, out, body);
-  else train_forward_teams<T, false, TEAM>(c, sp, out);
+  if constexpr (TEAM == 0) {
+    train_forward_body<T, false>(c, sp, out, body);
+    const int unit = (int)(blockIdx.x / kNumXcd), workgroup = 64 * kTrainTeam;
+    if (scan.count > 0 && unit < body)
+      finite_scan(scan, (long long)blockIdx.x * workgroup + threadIdx.x, (long long)kNumXcd * body * workgroup, nonfinite);
+  } else {
+    train_forward_teams<T, false, TEAM>(c, sp, out);
+  }
 }
 #undef MLPSP_TRAIN_PARAMS
 #undef MLPSP_TRAIN_TAIL
@@ -329,6 +337,14 @@ inline TrainPlan train_plan(int ntx, int nty, int64_t T) {
   const int teams = min(per_xcd, (T < 2816 ? 2048 : T <= 6400 ? 1536 : 2560) / kNumXcd), body = (per_xcd - teams) / kTrainTeam;
   return TrainPlan{0, body, (unsigned)(kNumXcd * (body + per_xcd - kTrainTeam * body))};
 }
+
+// What a wavefront that is done with its tile may look through for what is not finite, while the others' products leave memory
+// idle; where it would be more -- most tiles in teams, which do not look, and many primitives --, a launch of its own.  Forward
+// and look in us, fp16, in a launch of its own / beside:
+//     50,000 primitives, 4,860 tiles, 212 KB a wavefront   645 /   597      200,000, 12,750, 280 KB   1,609 / 1,416
+//    100,000,            4,860,       424 KB               749 /   695      200,000,  7,000, 635 KB   1,219 / 1,186
+//     30,000,            2,400,     1,060 KB               378 /   385
+constexpr int64_t kScanShare = 768 * 1024;
 
 // tile_base = exclusive sums of tile_steps, head[2] = their total; one workgroup (12,750 tiles: 6 us).
 __global__ __launch_bounds__(1024) void step_scan_kernel(const int32_t* __restrict__ tile_steps, int T,
@@ -438,12 +454,12 @@ MLPSP_API int mlpsp_train_forward_f32(const float* rays_o_dev, const float* rays
   return train_scan(f, s);
 }
 
-MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
-                                       const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
-                                       const float* freq_dev, const float* att_dev, const void* packed_dev,
-                                       int num_primitives, int width, int height, float threshold, int max_hits,
-                                       int use_bf16, void* workspace_dev, size_t workspace_bytes, float* out_rgb_dev,
-                                       float* out_alpha_dev, mlpsp_stream_t stream) {
+namespace {
+int train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev, const int32_t* order_dev,
+                       const int32_t* tile_offsets_dev, int64_t num_pairs, const float* freq_dev, const float* att_dev,
+                       const void* packed_dev, int num_primitives, int width, int height, float threshold, int max_hits,
+                       int use_bf16, void* workspace_dev, size_t workspace_bytes, float* out_rgb_dev, float* out_alpha_dev,
+                       FiniteScanInputs scan, int32_t* nonfinite_dev, hipStream_t s) {
   TrainFrame f;
   const int rc = train_frame(width, height, num_pairs, workspace_dev, workspace_bytes, f);
   if (rc != MLPSP_OK) return rc;
@@ -452,14 +468,18 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
     return MLPSP_E_ARGUMENT;
   if (num_primitives > 0 && (!prim_records_dev || !packed_dev)) return MLPSP_E_ARGUMENT;
   if (((uintptr_t)prim_records_dev % 128) != 0 || ((uintptr_t)packed_dev % 16) != 0) return MLPSP_E_ARGUMENT;
-  hipStream_t s = (hipStream_t)stream;
   MLPSP_HIP_TRY(clear_async(f.sp.head, 64 * sizeof(int32_t), s));
   const TrainPlan plan = train_plan(f.ntx, f.nty, f.T);
+  if (scan.count > 0 && finite_scan_bytes(scan) > kScanShare * kNumXcd * kTrainTeam * plan.body) {
+    launch_finite_scan(scan, nonfinite_dev, s);
+    MLPSP_LAUNCH_CHECK();
+    scan.count = 0;
+  }
 #define MLPSP_TRAIN_TEAM(T, TEAM)                                                                                      \
   hipLaunchKernelGGL((train_forward_mfma_kernel<T, TEAM>), dim3(plan.grid), dim3(train_workgroup(TEAM)), 0, s, rays_o_dev, rays_d_dev, \
                      (const PrimRecord*)prim_records_dev, order_dev, tile_offsets_dev, freq_dev, att_dev,                \
                      (const unsigned char*)packed_dev, num_primitives, width, height, f.ntx, f.nty, threshold, max_hits, f.sp, \
-                     TrainOut{out_rgb_dev, out_alpha_dev}, plan.body)
+                     TrainOut{out_rgb_dev, out_alpha_dev}, plan.body, scan, nonfinite_dev)
 #define MLPSP_TRAIN_LAUNCH(T)                                      \
   do {                                                             \
     if (plan.team == 0) MLPSP_TRAIN_TEAM(T, 0);                    \
@@ -472,4 +492,30 @@ MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* ray
 #undef MLPSP_TRAIN_TEAM
   MLPSP_LAUNCH_CHECK();
   return train_scan(f, s);
+}
+}  // namespace
+
+MLPSP_API int mlpsp_train_forward_mfma(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
+                                       const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
+                                       const float* freq_dev, const float* att_dev, const void* packed_dev,
+                                       int num_primitives, int width, int height, float threshold, int max_hits,
+                                       int use_bf16, void* workspace_dev, size_t workspace_bytes, float* out_rgb_dev,
+                                       float* out_alpha_dev, mlpsp_stream_t stream) {
+  return train_forward_mfma(rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, num_pairs, freq_dev, att_dev,
+                            packed_dev, num_primitives, width, height, threshold, max_hits, use_bf16, workspace_dev,
+                            workspace_bytes, out_rgb_dev, out_alpha_dev, FiniteScanInputs{}, nullptr, (hipStream_t)stream);
+}
+
+MLPSP_API int mlpsp_train_forward_mfma_checked(const float* rays_o_dev, const float* rays_d_dev, const void* prim_records_dev,
+                                       const int32_t* order_dev, const int32_t* tile_offsets_dev, int64_t num_pairs,
+                                       const float* freq_dev, const float* att_dev, const void* packed_dev,
+                                       int num_primitives, int width, int height, float threshold, int max_hits,
+                                       int use_bf16, void* workspace_dev, size_t workspace_bytes, float* out_rgb_dev,
+                                       float* out_alpha_dev, const float* const* arrays_dev,
+                                       const int64_t* lengths, int num_arrays, int32_t* flag_dev, mlpsp_stream_t stream) {
+  FiniteScanInputs scan{};
+  if (!flag_dev || !finite_scan_inputs(arrays_dev, lengths, num_arrays, scan)) return MLPSP_E_ARGUMENT;
+  return train_forward_mfma(rays_o_dev, rays_d_dev, prim_records_dev, order_dev, tile_offsets_dev, num_pairs, freq_dev, att_dev,
+                            packed_dev, num_primitives, width, height, threshold, max_hits, use_bf16, workspace_dev,
+                            workspace_bytes, out_rgb_dev, out_alpha_dev, scan, flag_dev, (hipStream_t)stream);
 }

@@ -490,13 +490,17 @@ def all_finite_flag(tensors, flag=None):
     dev = tensors[0].device if tensors else torch.device("cuda", torch.cuda.current_device())
     if flag is None:
         flag = torch.empty(1, dtype=torch.int32, device=dev)
+    _check(_lib.load().mlpsp_all_finite(*_arrays(tensors, dev), _ptr(flag), _stream(dev)), "mlpsp_all_finite")
+    return flag
+
+
+def _arrays(tensors, dev):
+    """Host arrays of addresses and lengths of what a look for non-finite elements goes through, and their number."""
     for t in tensors:
         if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.device == dev):
             raise RuntimeError("all_finite_flag expects contiguous float32 CUDA tensors on one device")
-    pointers = (C.c_void_p * max(len(tensors), 1))(*[t.data_ptr() for t in tensors])
-    lengths = (C.c_int64 * max(len(tensors), 1))(*[t.numel() for t in tensors])
-    _check(_lib.load().mlpsp_all_finite(pointers, lengths, len(tensors), _ptr(flag), _stream(dev)), "mlpsp_all_finite")
-    return flag
+    return ((C.c_void_p * max(len(tensors), 1))(*[t.data_ptr() for t in tensors]),
+            (C.c_int64 * max(len(tensors), 1))(*[t.numel() for t in tensors]), len(tensors))
 
 
 def training_records_mfma(rays_o, rays_d, records, order, tile_offsets, freq, att, packed, n, W, H, threshold, beta,
@@ -894,12 +898,12 @@ class TrainBuffer:
 
 
 def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W, H, threshold, max_hits, pool_steps,
-                  render_order=True, packed=None, bf16=False, buffer=None, settle=None):
+                  render_order=True, packed=None, bf16=False, buffer=None, settle=None, look=()):
     """Forward of a differentiable frame -> (rgb, alpha, :class:`TrainFrame`); one read-back (12 bytes).  ``ws``: the six
     f32 weight tensors (exact MLP); ``packed``: their matrix-core operand copy instead.  ``pool_steps``: steps to make
     room for; a frame that needs more is repeated once with what it asked for.  ``buffer``: a :class:`TrainBuffer` of
     these sizes whose header is read back with the frame's words and given to ``settle(counts, flag)``; where that returns
-    False this returns None."""
+    False this returns None.  ``look``: with ``packed`` and ``buffer``, tensors whose non-finite elements set its flag."""
     dev = rays_o.device
     lib = _lib.load()
     pairs, n = int(order.numel()), ws[0].shape[0]
@@ -920,9 +924,12 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
                                                1 if render_order else 0, _ptr(workspace), nbytes, _ptr(rgb), _ptr(alpha),
                                                _stream(dev))
         else:
-            code = lib.mlpsp_train_forward_mfma(*head, _ptr(packed), n, W, H, float(threshold), int(max_hits),
-                                                1 if bf16 else 0, _ptr(workspace), nbytes, _ptr(rgb), _ptr(alpha),
-                                                _stream(dev))
+            args = (*head, _ptr(packed), n, W, H, float(threshold), int(max_hits), 1 if bf16 else 0, _ptr(workspace), nbytes,
+                    _ptr(rgb), _ptr(alpha))
+            if look and buffer is not None:
+                code = lib.mlpsp_train_forward_mfma_checked(*args, *_arrays(look, dev), _ptr(buffer.flag), _stream(dev))
+            else:
+                code = lib.mlpsp_train_forward_mfma(*args, _stream(dev))
         _check(code, "mlpsp_train_forward")
         if buffer is None:
             chunks, status, steps = workspace[:12].view(torch.int32).tolist()

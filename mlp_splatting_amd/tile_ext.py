@@ -733,7 +733,7 @@ class TileExt:
             return True
         return ops.train_forward(x[0], x[1], rec, order, x[6], x[7], x[8], x[9:15], width, height, threshold, self.max_hits,
                                  buffer.pool_steps, render_order=render_order, packed=packed, bf16=precision == "bfloat16",
-                                 buffer=buffer, settle=settle)
+                                 buffer=buffer, settle=settle, look=() if judge is None else x[9:15])
 
     def train_forward_wmma(self, x, width, height, threshold, beta, temp, precision, queued=None):
         """:meth:`train_forward` on the matrix cores under the contract and policy of
@@ -742,14 +742,14 @@ class TileExt:
         width, height = int(width), int(height)
         self._check_training_wmma(x, width, height, 8, threshold, beta, temp, precision)
 
-        inputs = [t for i, t in enumerate(x) if i not in (5, 6)]
-
         def judge(flag):
             _chk(int(flag) == 0, "Training WMMA input is nonfinite; refusing unsafe forward/fallback")
             self._count_training_mfma(0)
 
         def accept(flag=None):
-            """A look at the inputs: judged at once, or by what is returned, with the value that ``flag`` is to hold."""
+            """A look at the inputs: judged at once, or by what is returned, with the value that ``flag`` is to hold when the
+            forward, which looks at the weights, is through."""
+            inputs = [t for i, t in enumerate(x) if i not in (5, 6) and (flag is None or not 9 <= i < 15)]
             if flag is None:
                 judge(ops.all_finite_flag(inputs).item())
             else:

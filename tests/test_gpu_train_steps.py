@@ -449,6 +449,47 @@ def test_steps_are_sorted_by_primitive(device, n, tiles, listed):
     assert (first == np.searchsorted(prim, np.arange(n + 1))).all()
 
 
+@pytest.mark.parametrize("columns", [3, 2100])
+def test_the_forward_looks_for_what_is_not_finite(device, columns):
+    """By its wavefronts behind their tiles (2,100 tiles, most in teams, which do not look) or in a launch of its own: every
+    element of arrays that begin at any float and of every length around a wavefront's and a workgroup's reach, the first and
+    the last ones among them; a flag that is set stays set."""
+    from mlp_splatting_amd import ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    n, width, height = 40, 8 * columns, 8
+    sc = syn.make_scene(n, 32, seed=4, log_scale_mean=-1.0)
+    ro, rd = syn.pinhole_rays(width, height, 60.0, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
+    base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats)]
+    order = torch.arange(n, dtype=torch.int32, device=device).repeat(columns)
+    offsets = torch.arange(columns + 1, dtype=torch.int32, device=device) * n
+    freq, att, ws = to_dev(sc.freq, device), to_dev(sc.att, device), [to_dev(w, device) for w in sc.mlp()]
+    records, packed = ops.prepare_primitives(*base[2:5]), ops.pack_mfma_weights(*ws, bf16=False)
+    pool = columns * n + 32 * columns
+    arrays = [torch.ones(length + 3, device=device)[shift:shift + length]
+              for length, shift in ((1, 0), (3, 1), (63, 2), (257, 3), (4 * 64 + 1, 0), (70_001, 1), (3_000_000, 2), (0, 0))]
+
+    def run(flag):
+        seen = []
+        buffer = ops.TrainBuffer(order.numel(), width, height, pool, device)
+        buffer.bytes[:256].zero_()
+        buffer.flag.fill_(flag)
+        out = ops.train_forward(base[0], base[1], records, order, offsets, freq, att, ws, width, height, 1e-3, 128, pool,
+                                packed=packed, buffer=buffer, settle=lambda counts, word: seen.append(word) or True, look=arrays)
+        return out, seen[0]
+    want, flag = run(0)
+    assert flag == 0 and run(1)[1] == 1
+    plain = ops.train_forward(base[0], base[1], records, order, offsets, freq, att, ws, width, height, 1e-3, 128, pool,
+                              packed=packed)
+    assert torch.equal(want[0], plain[0]) and torch.equal(want[1], plain[1]) and want[2].steps == plain[2].steps > 0
+    for array in arrays[:-1]:
+        for at in {0, array.numel() // 2, array.numel() - 1}:
+            for value in (float("nan"), float("-inf")):
+                array[at] = value
+                (rgb, _, _), flag = run(0)
+                assert flag == 1 and torch.equal(rgb, want[0])
+            array[at] = 1.0
+
+
 def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
     """Storage follows the steps, not the tiles: a tile with a hit takes a chunk, and the first frame reserves no more than
     its lists can need."""
