@@ -609,81 +609,92 @@ __global__ __launch_bounds__(kWideThreads) void bin_level1_fill_kernel(
 }
 
 // In-place exclusive scan of data[0..n) by one workgroup; data[n] and *total receive the sum, *largest
-// (if not null) the largest element.  data must be 16-byte aligned.  A pass covers 8 slabs of 4096
+// (if not null) the largest element.  data must be 16-byte aligned.  A pass covers kScanSlabs slabs of 4096
 // elements: thread t owns elements 4t..4t+3 of every slab, so all loads and stores are coalesced 16-byte
-// accesses and the 8 loads of a pass are independent (one memory latency per pass, and one pass covers
-// 32768 elements).  Thread sums are scanned with wavefront shuffles, wavefront totals through LDS.
+// accesses and the loads of a pass are independent and under no condition, where they would be waited for one by one (one
+// memory latency per pass, and one pass covers 53,248 elements).  Thread sums are scanned in the additions' own operands, the
+// elements' halves apart, so that the 256 of a wavefront fit 32 bits; a slab's 16 wavefronts by one of them.  51,000 tiles: 22 us
+// with sums in 64-bit shuffles, two passes and every wavefront adding up all others, 10 so; 1,344 tiles: 4.9, 5.5.
 // (Only the two-call binning, whose caller sizes the candidate buffer from the total, scans with a kernel of its
 // own; the asynchronous entry points place their lists inside the fill passes.)
-constexpr int kScanSlabs = 8;
+constexpr int kScanSlabs = 13;
+__device__ __forceinline__ unsigned sum_up_to_lane32(unsigned x) {
+#define MLPSP_SCAN_STEP(CTRL, ROWS) x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false)
+  MLPSP_SCAN_STEP(0x111, 0xf);           // row_shr:1, 2, 4, 8
+  MLPSP_SCAN_STEP(0x112, 0xf);
+  MLPSP_SCAN_STEP(0x114, 0xf);
+  MLPSP_SCAN_STEP(0x118, 0xf);
+  MLPSP_SCAN_STEP(0x142, 0xa);           // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+  MLPSP_SCAN_STEP(0x143, 0xc);
+#undef MLPSP_SCAN_STEP
+  return x;
+}
 __global__ __launch_bounds__(1024) void exclusive_scan_kernel(int32_t* __restrict__ data, int n,
                                                               long long* __restrict__ total,
                                                               long long* __restrict__ largest) {
-  __shared__ long long s_wave[kScanSlabs][16];
+  static_assert(kScanSlabs <= 16, "a wavefront for every slab");
+  __shared__ long long s_wave[kScanSlabs][16], s_slab[kScanSlabs];
   __shared__ int s_wmax[16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int full = n & ~3;               // (the elements behind the last whole four are the first thread's)
   long long carry = 0;
   int mx = 0;
-  for (int pass0 = 0; pass0 < n; pass0 += kScanSlabs * 4096) {
+  for (int pass0 = 0; pass0 < full; pass0 += kScanSlabs * 4096) {
     int4 v[kScanSlabs];
 #pragma unroll
     for (int u = 0; u < kScanSlabs; ++u) {
-      const int idx = pass0 + u * 4096 + t * 4;
-      if (idx + 3 < n) {
-        v[u] = *reinterpret_cast<const int4*>(data + idx);
-      } else {
-        v[u].x = (idx < n) ? data[idx] : 0;
-        v[u].y = (idx + 1 < n) ? data[idx + 1] : 0;
-        v[u].z = (idx + 2 < n) ? data[idx + 2] : 0;
-        v[u].w = 0;
-      }
+      if (pass0 + u * 4096 >= full) break;           // (of the workgroup)
+      v[u] = *reinterpret_cast<const int4*>(data + min(pass0 + u * 4096 + t * 4, full - 4));
+    }
+#pragma unroll
+    for (int u = 0; u < kScanSlabs; ++u) {
+      if (pass0 + u * 4096 >= full) break;
+      if (pass0 + u * 4096 + t * 4 >= full) v[u] = make_int4(0, 0, 0, 0);
+      mx = max(max(mx, max(v[u].x, v[u].y)), max(v[u].z, v[u].w));
     }
     long long incl[kScanSlabs];
 #pragma unroll
     for (int u = 0; u < kScanSlabs; ++u) {
-      incl[u] = 0;
-      if (pass0 + u * 4096 >= n) {            // slab beyond the data (workgroup-uniform): nothing to scan
-        if (lane == 63) s_wave[u][wave] = 0;
-        continue;
-      }
-      mx = max(max(mx, max(v[u].x, v[u].y)), max(v[u].z, v[u].w));
-      long long x = (long long)v[u].x + v[u].y + v[u].z + v[u].w;
+      if (pass0 + u * 4096 >= full) break;
+      const unsigned low = (v[u].x & 0xffff) + (v[u].y & 0xffff) + (v[u].z & 0xffff) + (v[u].w & 0xffff);
+      const unsigned high = (v[u].x >> 16) + (v[u].y >> 16) + (v[u].z >> 16) + (v[u].w >> 16);
+      incl[u] = sum_up_to_lane32(low) + ((long long)sum_up_to_lane32(high) << 16);
+      if (lane == 63) s_wave[u][wave] = incl[u];
+    }
+    __syncthreads();
+    // (a single slab: every wavefront for itself, without another barrier)
+    const bool single = full - pass0 <= 4096;
+    long long only_before = 0, only_slab = 0;
+    if (single || (wave < kScanSlabs && pass0 + wave * 4096 < full)) {
+      long long* const sums = s_wave[single ? 0 : wave];
+      const long long own = lane < 16 ? sums[lane] : 0;
+      long long x = own;
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
+      for (int d = 1; d < 16; d <<= 1) {
         const long long up = __shfl_up(x, d);
         if (lane >= d) x += up;
       }
-      incl[u] = x;
-      if (lane == 63) s_wave[u][wave] = x;
+      if (single) {
+        only_before = __shfl(x - own, wave);
+        only_slab = __shfl(x, 15);
+      } else {
+        if (lane < 16) sums[lane] = x - own;
+        if (lane == 15) s_slab[wave] = x;
+      }
     }
-    __syncthreads();
-    long long base = carry;
+    if (!single) __syncthreads();
 #pragma unroll
     for (int u = 0; u < kScanSlabs; ++u) {
-      if (pass0 + u * 4096 >= n) continue;
-      long long before = 0, slab = 0;
-#pragma unroll
-      for (int w = 0; w < 16; ++w) {
-        const long long c = s_wave[u][w];
-        before += (w < wave) ? c : 0;
-        slab += c;
-      }
+      if (pass0 + u * 4096 >= full) break;
       const long long own = (long long)v[u].x + v[u].y + v[u].z + v[u].w;
-      const long long e0 = base + before + incl[u] - own;
+      const long long e0 = carry + (single ? only_before : s_wave[u][wave]) + incl[u] - own;
       const int idx = pass0 + u * 4096 + t * 4;
-      const int4 o = make_int4((int)e0, (int)(e0 + v[u].x), (int)(e0 + v[u].x + v[u].y),
-                               (int)(e0 + v[u].x + v[u].y + v[u].z));
-      if (idx + 3 < n) {
-        *reinterpret_cast<int4*>(data + idx) = o;
-      } else {
-        if (idx < n) data[idx] = o.x;
-        if (idx + 1 < n) data[idx + 1] = o.y;
-        if (idx + 2 < n) data[idx + 2] = o.z;
-      }
-      base += slab;
+      if (idx < full)
+        *reinterpret_cast<int4*>(data + idx) = make_int4((int)e0, (int)(e0 + v[u].x), (int)(e0 + v[u].x + v[u].y),
+                                                         (int)(e0 + v[u].x + v[u].y + v[u].z));
+      carry += single ? only_slab : s_slab[u];
     }
-    carry = base;
-    __syncthreads();
+    if (pass0 + kScanSlabs * 4096 < full) __syncthreads();
   }
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) mx = max(mx, __shfl_xor(mx, d));
@@ -692,6 +703,12 @@ __global__ __launch_bounds__(1024) void exclusive_scan_kernel(int32_t* __restric
   if (t == 0) {
     int all_max = 0;
     for (int w = 0; w < 16; ++w) all_max = max(all_max, s_wmax[w]);
+    for (int i = full; i < n; ++i) {
+      const int own = data[i];
+      data[i] = (int32_t)carry;
+      carry += own;
+      all_max = max(all_max, own);
+    }
     data[n] = (int32_t)carry;
     *total = carry;
     if (largest) *largest = all_max;

@@ -1043,3 +1043,18 @@ def test_a_feature_frame_whose_record_pool_ran_out_is_repeated(device, oracle_mo
     for a, b in zip(images(), want):
         assert torch.equal(a, b)
     assert len(tried) == (2 if tile == 8 else 1) and float(want[1].mean()) > 0.05
+
+
+@pytest.mark.parametrize("columns,rows", [(1, 1), (3, 1), (64, 64), (67, 61), (208, 256), (275, 275), (417, 256)])
+def test_offsets_of_many_tiles(device, oracle_mod, columns, rows):
+    """The sums over the tiles' counts take 4,096 of them at a time and 53,248 in a pass, four to a thread: numbers of tiles that
+    end in, at and behind these."""
+    from mlp_splatting_amd import ops, synthetic as syn
+    W, H, thr = 8 * columns, 8 * rows, 1e-3
+    sc = syn.make_scene(120, 32, seed=2, log_scale_mean=-2.0)
+    view, proj = syn.view_matrix(syn.look_at((0.2, -0.1, -0.9)))[None], syn.projection_matrix(0.5 * W, W, H)
+    want, off = oracle_mod.bin_legacy(sc.positions, sc.log_scales, view, proj, W, H, 8, thr)
+    got, got_off = ops.bin_legacy(_t(sc.positions, device), _t(sc.log_scales, device), torch.from_numpy(view),
+                                  torch.from_numpy(proj), W, H, 8, thr)
+    assert len(off) == columns * rows + 1 and np.array_equal(got_off.cpu().numpy(), off)
+    assert np.array_equal(got.cpu().numpy(), want)
