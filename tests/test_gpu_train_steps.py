@@ -490,6 +490,24 @@ def test_the_forward_looks_for_what_is_not_finite(device, columns):
             array[at] = 1.0
 
 
+@pytest.mark.parametrize("columns,rows", [(1, 1), (3, 1), (64, 64), (67, 61), (128, 128), (129, 129)])
+def test_first_steps_of_many_tiles(device, columns, rows):
+    """The sums over the tiles' steps take 4,096 tiles at a time and 16,384 behind a barrier, four to a thread."""
+    from mlp_splatting_amd import ops, synthetic as syn
+    from mlp_splatting_amd.tile_ext import TileExt
+    tiles, width, height = columns * rows, 8 * columns, 8 * rows
+    sc = syn.make_scene(40, 32, seed=4, log_scale_mean=-1.0)
+    view, proj = syn.view_matrix(syn.look_at((0.0, 0.0, -3.0))), syn.projection_matrix(0.5 * width, width, height)
+    ro, rd = syn.pinhole_rays(width, height, 0.5 * width, syn.look_at((0.0, 0.0, -3.0)))
+    ro, rd, pos, logs, quats = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats)]
+    order, offsets = ops.bin_legacy(pos, logs, torch.from_numpy(view)[None], torch.from_numpy(proj), width, height, 8, 1e-3)
+    base = [ro, rd, pos, logs, quats, order, offsets] + [to_dev(a, device) for a in (sc.freq, sc.att, *sc.mlp())]
+    _, _, frame = TileExt().train_forward(base, width, height, 1e-3)
+    words = frame.workspace[256:].view(torch.int32)
+    steps, first = words[:tiles].long(), words[(tiles + 63) // 64 * 64:][:tiles + 1].long()
+    assert frame.steps == int(steps.sum()) > 0 and int(first[0]) == 0 and torch.equal(first[1:], steps.cumsum(0))
+
+
 def test_a_frame_of_small_primitives_keeps_little(device, oracle_mod):
     """Storage follows the steps, not the tiles: a tile with a hit takes a chunk, and the first frame reserves no more than
     its lists can need."""
