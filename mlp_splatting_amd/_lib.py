@@ -20,7 +20,7 @@ TILE_CAPACITY_MAX = 2048
 PIXEL_HIT_CAPACITY = 256
 PRIM_RECORD_BYTES = 128
 MFMA_PACK_BYTES = 7808
-VERSION = 400      # MLPSP_VERSION of include/mlpsp.h: the interface this binding was written against
+VERSION = 401      # MLPSP_VERSION of include/mlpsp.h: the interface this binding was written against
 STEP_CHUNK = 8
 STAGE_STATUS_IS_CLEAR = 4
 STAGE_FRAMES_OVERLAP = 8
