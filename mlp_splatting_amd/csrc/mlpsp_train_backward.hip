@@ -6,7 +6,7 @@
 // length.  A workgroup walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the
 // primitive's steps all lie in the chunk, else to the chunk's tail row (the primitive goes on in the next chunk) or head row
 // (it ended here).  One more launch adds the rows of the primitives that span chunks; the zeros of those without a step are
-// written by the weight gradient kernels too.  No atomics, a fixed order of every sum.
+// written by the weight gradient kernels too, or by a launch of their own where these have few wavefronts (kZeroShare32).  No atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
 // 0.12 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
@@ -485,6 +485,16 @@ __device__ __forceinline__ void walk_halves(const int4& where, StepRecord next, 
 // a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 / 1.70; a primitive per block of
 // products 5.34 and 1.83.  Ahead of the chunk its first record is waited for behind the stores: the f32 kernel of 80,000 steps
 // takes 676 us instead of 663.  With the rows of the attributes' gradient (512 channels, four slots: 1.3 GB more) fp16 1.52 -> 1.62.
+// What a wavefront may be given of them: few steps make few chunks, and the four wavefronts of one would store all rows alone
+// (16 steps of 200,000 primitives 56 ms, in a launch of their own 0.7).  Above it that launch, behind the gradients.  Call in us,
+// a launch / here, at KB per wavefront:
+//   f32    200,000 primitives  4,000 steps  2,761   628 /   649     8,000  1,380   651 / 648    16,000  690   735 /   677
+//           60,000             1,008        3,287   270 /   382     2,400  1,380   267 / 271     4,000  828   274 /   270
+//           20,000             1,008        1,096   169 /   203     2,400    460   166 / 163     8,000  138   193 /   169
+//   fp16   200,000            16,000          690   641 /   652    24,000    460   663 / 678    32,000  345   703 /   701
+//           60,000             1,008        3,287   244 /   358     4,000    828   240 / 243     8,000  414   251 /   243
+//          and 512 attribute channels of four slots, 200,000: 32,000  545   997 / 1,006    48,000  363  1,056 / 1,049    80,000  436  1,165 / 1,116
+constexpr int64_t kZeroShare32 = 1024 * 1024, kZeroShare16 = 448 * 1024;
 template <int WAVES>
 __device__ __forceinline__ void zero_share(const StepIndex& ix, int N, const ZeroRows& zero, int chunk, int num_chunks, int wave,
                                            int lane) {
@@ -818,11 +828,15 @@ int train_gradients(int64_t num_steps, int64_t num_pairs, int width,
   zero.add(grad_log_scales_dev, 3);
   zero.add(grad_quats_dev, 4);
   if (rows_dev) zero.add(rows_dev, row_floats);
+  const int64_t row_bytes = 4LL * (kGradFloats + 10 + (rows_dev ? row_floats : 0));
+  const int64_t room = num_chunks * (precision == 0 ? kZeroShare32 * kVjp32Waves : kZeroShare16 * kVjp16Waves);
+  const bool beside = num_primitives * row_bytes <= room;
   if (num_chunks > 0) {
+    const int zeros_here = beside ? num_primitives : 0;
 #define MLPSP_TRAIN_VJP(KERNEL, THREADS)                                                                                \
   hipLaunchKernelGGL(KERNEL, dim3((unsigned)num_chunks), dim3(THREADS), 0, s, ix, S, chunk_steps, num_chunks, sp.records, \
                      (const float4*)d4_dev, rays_d_dev, width, height, freq_dev, att_dev, W1, b1, W2, b2, W3, scale,   \
-                     t.rows, grads, nonfinite_dev, num_primitives, zero)
+                     t.rows, grads, nonfinite_dev, zeros_here, zero)
     if (precision == 0) MLPSP_TRAIN_VJP(train_vjp_f32_kernel, 64 * kVjp32Waves);
     else if (precision == 1) MLPSP_TRAIN_VJP((train_vjp16_kernel<_Float16>), 64 * kVjp16Waves);
     else MLPSP_TRAIN_VJP((train_vjp16_kernel<__bf16>), 64 * kVjp16Waves);
@@ -834,7 +848,8 @@ int train_gradients(int64_t num_steps, int64_t num_pairs, int width,
     hipLaunchKernelGGL(train_join_kernel, dim3((unsigned)num_chunks, 4), dim3(256), 0, s, ix, S, chunk_steps, num_chunks,
                        t.rows, quats_dev, grads, geo, nonfinite_dev);
     MLPSP_LAUNCH_CHECK();
-  } else {
+  }
+  if (!beside) {
     launch_zero_rows(t.first, num_primitives, zero, s);
     MLPSP_LAUNCH_CHECK();
   }

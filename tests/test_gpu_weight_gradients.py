@@ -215,3 +215,48 @@ def test_primitives_without_a_step_get_zeros(device, monkeypatch, tiles, n, prec
     for i, g in enumerate(grads):
         assert bool(torch.isfinite(g).all()) and not bool(g[without].any()), i
     assert bool((grads[5][~without] != 0).all())
+
+
+@pytest.mark.parametrize("precision,share", [(0, 1 << 20), (1, 448 << 10), (2, 448 << 10)])
+@pytest.mark.parametrize("beside", [False, True])
+def test_zeros_on_both_sides_of_a_wavefronts_share(device, precision, share, beside):
+    """One chunk of 16 steps, four wavefronts: as many primitives as they store the rows of, and one more, whose rows a launch of
+    its own writes."""
+    from mlp_splatting_amd import ops
+    channels = 24 if beside else 0
+    most = 4 * share // (4 * (3524 + 10 + channels))
+    for n in (most, most + 1):
+        base, frame = _frame(device, 1, n, np.zeros(16, int), np.arange(5, 21))
+        groups, d4 = ops.train_group(frame, base[6], n), torch.ones(16, 64, 4, device=device)
+        rows = torch.full((n, max(channels, 1)), float("nan"), device=device)
+        grads, flag = ops.train_gradients(frame, groups, d4, d4[..., 0].contiguous(), base[1], base[7], base[8], base[9:15], base[3],
+                                          base[4], precision, 1.0, *((rows,) if beside else ()))
+        without = torch.ones(n, dtype=torch.bool, device=device)
+        without[5:21] = False
+        assert int(flag) == 0 and bool((grads[5][~without] != 0).all())
+        for g in grads + ([rows] if beside else []):
+            assert not bool(g[without].ne(0).any())
+        assert not beside or bool(rows[~without].isnan().all())
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_few_steps_of_many_primitives_do_not_wait_for_their_zeros(device, precision):
+    """16 steps, a chunk, of 20,000 primitives: 283 MB of zeros, which one workgroup takes 50 times as long for as the whole
+    call of 2,400 steps takes.  With a launch for them it is twice as long; ten times leaves room for a busy host."""
+    from mlp_splatting_amd import ops
+
+    def call(tiles):
+        listed = np.arange(16) * 700
+        base, frame = _frame(device, tiles, 20_000, np.repeat(np.arange(tiles), 16), np.tile(listed, tiles))
+        groups, d4 = ops.train_group(frame, base[6], 20_000), torch.ones(frame.steps, 64, 4, device=device)
+        args = (frame, groups, d4, d4[..., 0].contiguous(), base[1], base[7], base[8], base[9:15], base[3], base[4], precision, 1.0)
+        times = []
+        for _ in range(7):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            ops.train_gradients(*args)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end))
+        return sorted(times)[3]
+    assert call(1) <= 10.0 * call(150)
