@@ -887,7 +887,8 @@ _TRAIN_HEADER = 256
 
 
 class TrainBuffer:
-    """Header and workspace of a differentiable frame with room for ``pool_steps`` steps."""
+    """Header and workspace of a differentiable frame with room for ``pool_steps`` steps.  The frame's forward takes the
+    memory over (:meth:`release`): where it is not what the frame keeps, nothing else may hold it."""
     __slots__ = ("bytes", "pairs", "pool_steps", "counts", "flag")
 
     def __init__(self, pairs, W, H, pool_steps, device):
@@ -896,14 +897,17 @@ class TrainBuffer:
         self.bytes = torch.empty(_TRAIN_HEADER + nbytes, dtype=torch.uint8, device=device)
         self.counts, self.flag = self.bytes[:32].view(torch.int64), self.bytes[32:36].view(torch.int32)
 
+    def release(self):
+        self.bytes = self.counts = self.flag = None
+
 
 def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W, H, threshold, max_hits, pool_steps,
                   render_order=True, packed=None, bf16=False, buffer=None, settle=None, look=()):
     """Forward of a differentiable frame -> (rgb, alpha, :class:`TrainFrame`); one read-back (12 bytes).  ``ws``: the six
     f32 weight tensors (exact MLP); ``packed``: their matrix-core operand copy instead.  ``pool_steps``: steps to make
     room for; a frame that needs more is repeated once with what it asked for.  ``buffer``: a :class:`TrainBuffer` of
-    these sizes whose header is read back with the frame's words and given to ``settle(counts, flag)``; where that returns
-    False this returns None.  ``look``: with ``packed`` and ``buffer``, tensors whose non-finite elements set its flag."""
+    these sizes, given up here, whose header is read back with the frame's words and given to ``settle(counts, flag)``; where
+    that returns False this returns None.  ``look``: with ``packed`` and ``buffer``, tensors whose non-finite elements set its flag."""
     dev = rays_o.device
     lib = _lib.load()
     pairs, n = int(order.numel()), ws[0].shape[0]
@@ -935,6 +939,7 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
             chunks, status, steps = workspace[:12].view(torch.int32).tolist()
         else:
             words = buffer.bytes[:_TRAIN_HEADER + 12].view(torch.int32).tolist()
+            buffer.release()
             if not settle([a & 0xffffffff | b << 32 for a, b in zip(words[0:8:2], words[1:8:2])], words[8]):
                 return None
             chunks, status, steps = words[-3:]

@@ -130,3 +130,42 @@ def test_a_queued_frame_that_overflows_its_operands_is_repeated_in_f32(device, f
         want = _step(scene, *camera, target)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("what", ["room", "lists", "numbers"])
+def test_a_frame_that_is_repeated_gives_its_workspace_up_first(device, fresh, monkeypatch, what):
+    """Too little room for the steps, lists cut short, operands beyond fp16: before the repetition makes its workspace, nothing
+    holds the one it replaces."""
+    import weakref
+    from mlp_splatting_amd import _lib, ops
+    monkeypatch.setenv("MLPSP_CSR_FORWARD_BACKEND", "wmma_fp16")
+    scene, camera = _scene(device, 4), _camera(device, (0.2, -0.1, -0.9))
+    target = torch.randn(11, 15, 4, device=device)
+    _step(scene, *camera, target)
+    ext, lib, made, gone = scene._ensure_tile_ext(), _lib.load(), [], []
+
+    class Buffer(ops.TrainBuffer):
+        def __init__(self, *a):
+            super().__init__(*a)
+            made.append(weakref.ref(self.bytes))
+
+    class Spy:
+        def __getattr__(self, name):
+            if name == "mlpsp_train_workspace_bytes" and made:
+                gone.append([ref() is None for ref in made])
+            return getattr(lib, name)
+    monkeypatch.setattr(ops, "TrainBuffer", Buffer)
+    monkeypatch.setattr(_lib, "load", lambda: Spy())
+    if what == "room":
+        ext._steps_per_tile = 0.5
+    elif what == "lists":
+        ext._queue_capacity = 64
+    else:
+        with torch.no_grad():
+            scene.W2.mul_(1e6)
+    if what == "numbers":
+        with pytest.warns(UserWarning, match="numeric overflow"):
+            _step(scene, *camera, target)
+    else:
+        _step(scene, *camera, target)
+    assert gone == [[True]]
