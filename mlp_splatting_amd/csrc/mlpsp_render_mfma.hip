@@ -263,15 +263,6 @@ template <typename T> struct RenderTable { static constexpr bool kUse = false; u
 template <> struct RenderTable<__bf16> { static constexpr bool kUse = true; SinCosTable t; };
 #endif
 
-// SP = 0: RGB only.  SP = 4 or 8: the kernel also emits, per tile, the compact list of primitives that
-// hit at least one pixel (hit records, mlpsp_hitrec.hpp) and per (such primitive, pixel) the SP compositing
-// coefficients of the gated feature channel, rounded to fp16 (they lie in [0, 1]; fp16 keeps 11
-// significant bits there, bf16 only 8): (w g0, w g1, w g2, w g3) for 4 slots,
-// (w, 0, 0, 0) for one slot, (w, w g0, .., w g3, 0, 0, 0) for 5 slots (np_tile_kernels.cu:6036-6075:
-// feat += w * (base + sum_s g_s attr_s)).  The feature image is then one grouped GEMM over those lists
-// (feat_gemm_kernel below).
-// Register budget: 128 VGPRs, i.e. four wavefronts per SIMD (a dozen values spill; measured 4.5 % faster
-// than the 146 registers and three wavefronts the compiler picks on its own).
 // A lane's coefficients of record rs: its weight w, its gates times w in gt (none with one slot).
 template <int SP>
 __device__ __forceinline__ void store_coefficients(const HitPool& hp, int rs, int l, int p, int slots, float w, const float gt[4]) {
@@ -287,6 +278,15 @@ __device__ __forceinline__ void store_coefficients(const HitPool& hp, int rs, in
   }
   if (l == 0) hp.hit_ids[rs] = p;
 }
+// SP = 0: RGB only.  SP = 4 or 8: the kernel also emits, per tile, the compact list of primitives that
+// hit at least one pixel (hit records, mlpsp_hitrec.hpp) and per (such primitive, pixel) the SP compositing
+// coefficients of the gated feature channel, rounded to fp16 (they lie in [0, 1]; fp16 keeps 11
+// significant bits there, bf16 only 8): (w g0, w g1, w g2, w g3) for 4 slots,
+// (w, 0, 0, 0) for one slot, (w, w g0, .., w g3, 0, 0, 0) for 5 slots (np_tile_kernels.cu:6036-6075:
+// feat += w * (base + sum_s g_s attr_s)).  The feature image is then one grouped GEMM over those lists
+// (feat_gemm_kernel below).
+// Register budget: 128 VGPRs, i.e. four wavefronts per SIMD (a dozen values spill; measured 4.5 % faster
+// than the 146 registers and three wavefronts the compiler picks on its own).
 // One tile, rendered by the calling wavefront (lane l = pixel l of the tile); s_dir: LDS of this wavefront alone.
 template <typename T, int SP>
 __device__ __forceinline__ void render_tile_mfma(
@@ -773,8 +773,8 @@ __global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(4, 4)
 constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
 // Tiles at the end of the launch that get a workgroup each, as a team, which finishes a tile in a third of the time:
 // the wavefronts' tiles are long against the launch, and what a CU still has to do when the queue is empty differs by as much.
-// Not where another frame follows on the heels of this one: its wavefronts take the places that the last tiles leave.  Frame in
-// us, bf16, with teams for so many of the last tiles:
+// Not where another RGB frame follows on the heels of this one (MLPSP_STAGE_FRAMES_OVERLAP): its wavefronts take the places that
+// the last tiles leave.  Frame in us, bf16, with teams for so many of the last tiles:
 //     tiles     none   1,024   1,536   2,048   2,560   3,072
 //     2,560      242     235     233     234     239     240
 //     3,150      265     253     258     262     268     272
@@ -782,7 +782,12 @@ constexpr int kRenderWaves = MLPSP_RENDER_WAVES;
 //     8,000      439     432     428     428     427     432
 //    12,750      642     632     631     628     630     636   (fp16: 748 / 734 / 733 / 726 / 725 / 730)
 //    30,000    1,273   1,262      --   1,262      --   1,272
-// (The renders with feature records have the same tail.)
+//    32,400    1,294   1,275   1,274   1,275      --   1,289
+//    51,000    2,015   2,010   2,000   2,001      --   1,995   (a mosaic of four views 1,528 / 1,521 / 1,520 / 1,523 / -- / 1,521)
+//    93,750    3,630   3,631   3,616   3,610      --   3,604
+// The renders with feature records have the same tail.  Between two of them lies a feature product, and teams make no
+// difference there: two frames in flight, us a frame without / with, 64 channels: 2,700 tiles 285 to 292 / 288 to 296, 5,700
+// 458 to 464 / 452, 12,750 858 to 865 / 864 to 868; 512 channels 1,275 to 1,291 / 1,282 to 1,286.  So these are not told of each other.
 inline int last_round(int64_t tiles) { return tiles < 4096 ? 1024 : tiles <= 8192 ? 1536 : 2048; }
 // MIXED: the workgroups from `body` on (per XCD) take one tile each, as a team.
 template <typename T, int SP, bool MIXED>
