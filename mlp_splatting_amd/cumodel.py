@@ -642,7 +642,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def build_tilecenter_culling_from_tile_views(self, tile_view_ids, view_matrices, proj_matrix,
                                                  score_threshold: float = 1e-3, tile_size: int | None = None):
         """Tile lists when every tile takes its rays from one of K views (scannet/cumodel.py:838-949)."""
-        if getattr(self, "camera_mode", "legacy-centered") == "colmap-native":
+        if self._native_camera():
             return None, None
         if self.image_size is None:
             raise ValueError("image_size must be set before building tile culling.")
@@ -688,13 +688,20 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
                 memo[key] = hit
         return hit[:3]
 
+    def _native_camera(self):
+        """Whether ``camera_mode``, of the instance or of its class, asks for lists from ray cones.  (getattr with a default on
+        a module that lacks the name walks parameters, buffers and submodules first.)"""
+        if "camera_mode" not in self.__dict__ and not hasattr(type(self), "camera_mode"):
+            return False
+        return self.camera_mode == "colmap-native"
+
     def _tile_lists(self, ray_o, ray_d, score_threshold, view_matrix, proj_matrix, culled_prim_indices, tile_offsets,
                     device, allow_native=True):
         W, H = self.image_size
         tile_size = int(self.tile_size)
         num_tiles = ops.num_tiles(W, H, tile_size, tile_size)
         external = (culled_prim_indices is not None) or (tile_offsets is not None)
-        if allow_native and getattr(self, "camera_mode", "legacy-centered") == "colmap-native":
+        if allow_native and self._native_camera():
             if external:
                 raise ValueError("Native camera culling must be derived from the actual rays")
             culled_prim_indices, tile_offsets = ray_cone_candidates(
@@ -768,7 +775,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             plain = self.__dict__
             own_lists = (culled_prim_indices is None and tile_offsets is None and view_matrix is not None
                          and proj_matrix is not None
-                         and plain.get("camera_mode", "legacy-centered") != "colmap-native")
+                         and not self._native_camera())
             with_feat = return_feature and self.feat_attr is not None
             if (own_lists and use_tilecenter and ts == 8 and (with_feat or not return_feature)
                     and feature_target is None and plain.get("queued_frames", True)
@@ -846,7 +853,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         ext, plain = self._ensure_tile_ext(), self.__dict__
         W, H = self.image_size
         own = (culled_prim_indices is None and tile_offsets is None and view_matrix is not None and proj_matrix is not None
-               and plain.get("camera_mode", "legacy-centered") != "colmap-native")
+               and not self._native_camera())
         queued = None
         if own and keeps_steps and plain.get("queued_frames", True) and hasattr(ext, "train_lists_queued"):
             def again():
@@ -1044,7 +1051,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         eligible = (frames_in_flight > 1 and len(frames) > 1 and self.image_size is not None
                     and self._resolve_tile_order_mode() == "tilecenter" and int(self.tile_size) == 8
                     and (with_feat or not return_feature) and plain.get("queued_frames", True)
-                    and plain.get("camera_mode", "legacy-centered") != "colmap-native"
+                    and not self._native_camera()
                     and str(getattr(self, "render_precision", "f32")).lower() in {"bf16", "fp16"}
                     and all(f[2] is not None and f[3] is not None and f[0].shape[0] == W * H for f in frames))
         if not eligible:
@@ -1117,7 +1124,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def render_rgb_alpha_no_grad(self, ray_o, ray_d, score_threshold: float = 1e-3, bg_color=None, view_matrix=None,
                                  proj_matrix=None, collect_w_stats: bool = False, gt_rgb=None):
         """(rgb, alpha) under the tile-centre pipeline (scannet/cumodel.py:1196-1383)."""
-        if getattr(self, "camera_mode", "legacy-centered") == "colmap-native":
+        if self._native_camera():
             raise NotImplementedError("Native camera statistics rendering is not implemented; use forward for RGB/features")
         if self.image_size is None:
             raise ValueError("image_size must be set on NeuralPrimitiveSceneTileCUDA before calling render_rgb_alpha_no_grad.")
@@ -1152,7 +1159,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def render_rgb_t_no_grad(self, ray_o, ray_d, score_threshold: float = 1e-3, bg_color=None, view_matrix=None,
                              proj_matrix=None):
         """(rgb, t, alpha) with t the expected depth (scannet/cumodel.py:1385-1525)."""
-        if getattr(self, "camera_mode", "legacy-centered") == "colmap-native":
+        if self._native_camera():
             raise NotImplementedError("Native camera depth rendering is not implemented; use forward for RGB/features")
         if self.image_size is None:
             raise ValueError("image_size must be set on NeuralPrimitiveSceneTileCUDA before calling render_rgb_t_no_grad.")

@@ -146,6 +146,36 @@ def test_native_camera_mode_uses_ray_cone_lists(device, oracle_mod):
         _call(scene, fr, device, culled_prim_indices=every, tile_offsets=offs)
 
 
+@pytest.mark.parametrize("of_class", [False, True])
+def test_native_camera_mode_of_a_subclass(device, oracle_mod, monkeypatch, of_class):
+    """A class attribute counts as the instance's does: for frames, frames in flight and training steps, the first and later
+    ones, all lists come from ray cones."""
+    from mlp_splatting_amd import cumodel
+    from mlp_splatting_amd.tile_ext import TileExt
+    fr = Frame("cfg1_5k_160x120", n=600, width=40, height=24)
+    monkeypatch.setattr(cumodel, "_tile_ext", TileExt())
+    scene = _scene_from(fr, device)
+    if of_class:
+        scene.__class__ = type("Native", (type(scene),), {"camera_mode": "colmap-native"})
+    else:
+        scene.camera_mode = "colmap-native"
+    cones, real = [], cumodel.ray_cone_candidates
+    monkeypatch.setattr(cumodel, "ray_cone_candidates", lambda *a, **k: cones.append(1) or real(*a, **k))
+    for _ in range(3):
+        _call(scene, fr, device)
+    assert len(cones) == 3
+    scene.train()
+    for _ in range(3):
+        rgb = scene(*[to_dev(r, device) for r in (fr.rays_o, fr.rays_d)], fr.thr, view_matrix=to_dev(fr.view, device),
+                    proj_matrix=to_dev(fr.proj, device))
+        rgb.sum().backward()
+    assert len(cones) == 6
+    scene.eval()
+    scene.render_precision = "bf16"
+    scene.render_frames(_camera_frames(fr, device, 3), fr.thr)
+    assert len(cones) == 9
+
+
 def test_lists_from_the_own_binning_skip_device_validation_but_keep_the_capacity_check(device, oracle_mod, monkeypatch):
     from mlp_splatting_amd import cumodel, ops
     from mlp_splatting_amd.tile_ext import TileExt
