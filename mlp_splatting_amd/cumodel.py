@@ -873,8 +873,8 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             unit_dirs = _unit_directions(ray_d)
             culled_prim_indices, tile_offsets = self._tile_lists(
                 ray_o, ray_d, score_threshold, view_matrix, proj_matrix, culled_prim_indices, tile_offsets, device)
-            if own and keeps_steps and hasattr(ext, "note_frame_pairs"):
-                ext.note_frame_pairs(int(culled_prim_indices.numel()))
+            if own and keeps_steps and hasattr(ext, "note_training_pairs"):
+                ext.note_training_pairs(culled_prim_indices.numel(), W, H)
         freq, att = self._frequency_tables(device)
         return unit_dirs, culled_prim_indices, tile_offsets, freq, att, queued
 

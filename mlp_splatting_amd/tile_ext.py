@@ -93,6 +93,7 @@ class TileExt:
         self._queue_capacity = 0          # candidate-buffer estimate of render_frame_queued (0: not seeded yet)
         self._queue_scratch_scale = 1
         self._steps_per_tile = None       # room the differentiable frame makes for its steps (see train_forward)
+        self._pairs_per_tile = None       # ... and for its candidates, where its lists are queued (see _note_pairs)
 
     # ------------------------------------------------------------------------------------------
     # derived-tensor caches (geometry records, matrix-core operand copies)
@@ -636,25 +637,39 @@ class TileExt:
         or None before a frame has shown how many candidates and steps there are.  ``again()`` -> (candidates, offsets)
         by way of the host, for the frame whose estimate was too small."""
         width, height = int(width), int(height)
+        tiles = ops.num_tiles(width, height, 8, 8)
         with self._lock:
-            cap, scale, room = self._queue_capacity, self._queue_scratch_scale, self._steps_per_tile
-        if cap <= 0 or room is None or positions.shape[0] == 0:
+            cap, scale, room, pairs = self._queue_capacity, self._queue_scratch_scale, self._steps_per_tile, self._pairs_per_tile
+        if cap <= 0 or room is None or pairs is None or positions.shape[0] == 0:
             return None
+        cap = min(cap, int(tiles * pairs) + 65536)
         with _on_device(positions.device):
-            buffer = ops.TrainBuffer(cap, width, height, int(ops.num_tiles(width, height, 8, 8) * room), positions.device)
+            buffer = ops.TrainBuffer(cap, width, height, int(tiles * room), positions.device)
             cand, offsets, _ = ops.bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, width, height, 8,
                                                     float(threshold), cap, scratch_scale=scale, counts=buffer.counts)
         return QueuedLists(cand, offsets, buffer, scale, again)
 
+    def _note_pairs(self, pairs, tiles):
+        """The candidates of a differentiable frame, for the next one's lists.  Frames that are only rendered, or of another
+        size, have estimates of their own: room is per tile, what was needed and three tenths, a sixty-fourth less with every frame
+        that needs less (as the steps' in :meth:`train_forward`)."""
+        with self._lock:
+            if pairs * 1.1 > self._queue_capacity:
+                self._queue_capacity = int(pairs * 1.3) + 65536
+            self._pairs_per_tile = max(1.3 * pairs / tiles, (self._pairs_per_tile or 0.0) * (63 / 64))
+
+    def note_training_pairs(self, pairs: int, width: int, height: int):
+        """Seed the estimate of :meth:`train_lists_queued` from a frame whose lists came by way of the host."""
+        self._note_pairs(int(pairs), ops.num_tiles(int(width), int(height), 8, 8))
+
     def _settle_lists(self, queued, counts, name):
         """Whether queued lists are what they should be, by their counts; the estimates for the frames to come."""
         pairs, longest, _, guard = counts
-        cap = queued.buffer.pairs
-        with self._lock:
-            if guard and pairs <= cap:
+        if guard and pairs <= queued.buffer.pairs:
+            with self._lock:
                 self._queue_scratch_scale = queued.scale * 4
-            elif pairs > 0.9 * cap:
-                self._queue_capacity = max(self._queue_capacity, int(pairs * 1.3) + 65536)
+        else:
+            self._note_pairs(pairs, queued.offsets.numel() - 1)
         if guard:
             return False
         if longest > self.max_tile_prims:

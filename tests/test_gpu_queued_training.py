@@ -169,3 +169,31 @@ def test_a_frame_that_is_repeated_gives_its_workspace_up_first(device, fresh, mo
     else:
         _step(scene, *camera, target)
     assert gone == [[True]]
+
+
+@pytest.mark.parametrize("backend", [None, "wmma_fp16"])
+def test_lists_have_room_for_what_training_frames_needed(device, fresh, monkeypatch, backend):
+    """The lists of a queued training frame hold three tenths more than the frames before needed, a tile, and 65,536: not what a
+    frame of many candidates needed that was only rendered.  One that needs more is repeated, and the next one has the room."""
+    scene = _scene(device, 4 if backend else 0)
+    target = None
+    if backend:
+        monkeypatch.setenv("MLPSP_CSR_FORWARD_BACKEND", backend)
+        target = torch.randn(11, 15, 4, device=device)
+    camera = _camera(device, (0.2, -0.1, -0.9))
+    want = _step(scene, *camera, target)
+    ext = scene._ensure_tile_ext()
+    pairs = ext._queue_capacity                        # (1.3 pairs + 65,536 by the first frame)
+    ext.note_frame_pairs(50_000_000)
+    sizes, whole = [], ext.train_lists_queued
+    monkeypatch.setattr(ext, "train_lists_queued", lambda *a: (lambda q: sizes.append(q.candidates.numel()) or q)(whole(*a)))
+    for _ in range(3):
+        assert all(torch.equal(a, b) for a, b in zip(_step(scene, *camera, target), want))
+    assert len(sizes) == 3 and all(abs(size - pairs) <= 2 for size in sizes)
+    ext._pairs_per_tile *= 64.0
+    _step(scene, *camera, target)
+    assert sizes[3] > sizes[2] and ext._pairs_per_tile < 64.0 * (sizes[0] - 65_536) / 48 * 0.99
+    ext._pairs_per_tile, ext._queue_capacity = 0.0, 256
+    for _ in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(_step(scene, *camera, target), want))
+    assert sizes[4] == 256 and abs(sizes[5] - pairs) <= 2
