@@ -556,13 +556,14 @@ def _feat_shape(feat_attr, allow_half=False):
     return int(slots), int(ch)
 
 
-def _feat_pool_sizes(pairs: int, entry_bytes: int):
+def _feat_pool_sizes(pairs: int, entry_bytes: int, tiles: int = 0):
     """Record-pool sizes to try in turn: the worst case, which cannot run out and needs no look at whether it did, where it
-    is no more than 2 GiB (`entry_bytes`: the records of a list entry); else a quarter of the candidates (at the 200k-primitive benchmark scene 8 % of them hit before
-    their tile saturates; of a scene of few large primitives a third, whose frames were rendered twice: 12,000 primitives at
-    240x184 1.36 ms, now 0.75), then the worst case."""
+    is no more than 2 GiB (`entry_bytes`: the records of a list entry; a tile's last draw can stay 63 of them short of full);
+    else a quarter of the candidates (at the 200k-primitive benchmark scene 8 % of them hit before their tile saturates; of a
+    scene of few large primitives a third, whose frames were rendered twice: 12,000 primitives at 240x184 1.36 ms, now 0.75),
+    then the worst case."""
     first = max(pairs // 4, 1 << 16)
-    return (first, -1) if first < pairs and pairs * entry_bytes > 2 << 30 else (-1,)
+    return (first, -1) if first < pairs and (pairs + 63 * tiles) * entry_bytes > 2 << 30 else (-1,)
 
 
 def render_tilecenter_feat_f32(rays_o, rays_d, records, order, tile_offsets, freq, att, W1, b1, W2, b2, W3, b3,
@@ -579,7 +580,7 @@ def render_tilecenter_feat_f32(rays_o, rays_d, records, order, tile_offsets, fre
     n, hidden, F = W1.shape[0], W2.shape[1], freq.shape[0]
     pairs = int(order.numel())
     waves = (TW * TH + 63) // 64
-    for pool in _feat_pool_sizes(pairs, waves * 256 * (5 if slots > 1 else 1)):
+    for pool in _feat_pool_sizes(pairs, waves * 256 * (5 if slots > 1 else 1), num_tiles(W, H, TW, TH)):
         nbytes = lib.mlpsp_feat_workspace_bytes(pairs, W, H, TW, TH, slots, 0, pool)
         if nbytes == 0:
             raise RuntimeError("mlpsp_feat_workspace_bytes: bad arguments")
@@ -801,7 +802,7 @@ def render_tilecenter_mfma_feat(rays_o, rays_d, records, order, tile_offsets, fr
         launch(workspace, ws_bytes, 2)
         stages(3)
         return rgb, alpha, feat, (bool(flag[0].item()) if check else flag)
-    for pool in _feat_pool_sizes(pairs, 128 * (8 if slots == 5 else 4)):
+    for pool in _feat_pool_sizes(pairs, 128 * (8 if slots == 5 else 4), num_tiles(W, H, 8, 8)):
         ws_bytes = lib.mlpsp_feat_workspace_bytes(pairs, W, H, 8, 8, slots, 1, pool)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         code = launch(workspace, ws_bytes, 0)
@@ -907,7 +908,8 @@ def train_forward(rays_o, rays_d, records, order, tile_offsets, freq, att, ws, W
     f32 weight tensors (exact MLP); ``packed``: their matrix-core operand copy instead.  ``pool_steps``: steps to make
     room for; a frame that needs more is repeated once with what it asked for.  ``buffer``: a :class:`TrainBuffer` of
     these sizes, given up here, whose header is read back with the frame's words and given to ``settle(counts, flag)``; where
-    that returns False this returns None.  ``look``: with ``packed`` and ``buffer``, tensors whose non-finite elements set its flag."""
+    that returns False this returns None.  ``look``: with ``packed`` and ``buffer``, tensors whose non-finite elements set its
+    flag."""
     dev = rays_o.device
     lib = _lib.load()
     pairs, n = int(order.numel()), ws[0].shape[0]

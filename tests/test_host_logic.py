@@ -311,3 +311,25 @@ def test_compact_segments_writes_segment_lists_one_after_the_other():
     assert flat.dtype == torch.int32 and off.dtype == torch.int32
     none, off0 = ops.compact_segments(order, offsets, offsets[:-1].clone())
     assert none.numel() == 0 and off0.tolist() == [0, 0, 0, 0, 0]
+
+
+@pytest.mark.parametrize("width,height", [(320, 240), (2400, 1360), (4000, 3000)])
+@pytest.mark.parametrize("slots,half,tile", [(1, False, 8), (4, False, 8), (5, False, 16), (4, True, 8), (5, True, 8)])
+def test_a_record_pool_that_cannot_run_out_takes_two_gibibytes_at_most(width, height, tile, slots, half):
+    """The pool of the first attempt at a feature frame, by the size of the workspace that it asks for, with few list entries to a
+    tile and many: the worst case where this is 2 GiB and less (its records; their names are a thirty-second more at most), and
+    beyond that only where a quarter of the entries is no less."""
+    from mlp_splatting_amd import _lib, ops
+    waves = (tile * tile + 63) // 64
+    entry = 128 * (8 if slots == 5 else 4) if half else waves * 256 * (5 if slots > 1 else 1)
+    whole = []
+    for pairs in (0, 65_536, 65_537, 200_000, 1_000_000, 4_000_000, 40_000_000):
+        sizes = ops._feat_pool_sizes(pairs, entry, ops.num_tiles(width, height, tile, tile))
+        worst = _lib.load().mlpsp_feat_workspace_bytes(pairs, width, height, tile, tile, slots, int(half), -1)
+        assert sizes[-1] == -1 and worst > 0
+        whole.append(len(sizes) == 1)
+        if whole[-1]:
+            assert pairs <= 65_536 or worst <= (2 << 30) * 33 / 32 + 4 * pairs * waves
+        else:
+            assert sizes[0] == max(pairs // 4, 65_536) and worst > 2 << 30
+    assert whole[0] and not whole[-1] and whole == sorted(whole, reverse=True)
