@@ -109,10 +109,10 @@ def _unit_directions(ray_d):
     return F.normalize(ray_d, dim=-1).contiguous()
 
 
-def _frame_matrix(t):
-    """The matrix as the queued frame takes it: a float32 device tensor stays where it is (the binning reads it
-    there; no copy to the host, no synchronisation), anything else becomes a host copy."""
-    if torch.is_tensor(t) and t.is_cuda and t.dtype == torch.float32 and t.numel() == 16:
+def _frame_matrix(t, device):
+    """The matrix as a queued frame on ``device`` takes it: a float32 tensor of that device stays where it is (the
+    binning reads it there; no copy to the host, no synchronisation), anything else becomes a host copy."""
+    if torch.is_tensor(t) and t.device == device and t.is_cuda and t.dtype == torch.float32 and t.numel() == 16:
         return t.detach().contiguous()
     return _host_matrix(t)
 
@@ -859,13 +859,14 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             def again():
                 return self._tile_lists(ray_o, ray_d, score_threshold, view_matrix, proj_matrix, None, None, device)
             queued = ext.train_lists_queued(self.positions.detach(), self.log_scales.detach(),
-                                            _frame_matrix(view_matrix).reshape(1, 4, 4), _frame_matrix(proj_matrix), W, H,
+                                            _frame_matrix(view_matrix, device).reshape(1, 4, 4),
+                                            _frame_matrix(proj_matrix, device), W, H,
                                             float(score_threshold), again)
         if queued is not None:
             culled_prim_indices, tile_offsets = queued.candidates, queued.offsets
             rays = ray_o.contiguous()
             if (ray_d.is_cuda and ray_d.dtype == torch.float32 and ray_d.dim() == 2 and ray_d.shape[1] == 3
-                    and rays.dtype == torch.float32 and rays.shape == ray_d.shape and rays.is_cuda):
+                    and rays.dtype == torch.float32 and rays.shape == ray_d.shape and rays.device == ray_d.device):
                 unit_dirs, queued.pyramids, _ = ext.frame_prologue(rays, ray_d, int(W), int(H))
             else:
                 unit_dirs = _unit_directions(ray_d)
@@ -978,7 +979,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             positions = positions.contiguous()
         if not log_scales.is_contiguous():
             log_scales = log_scales.contiguous()
-        views, proj = _frame_matrix(view_matrix).reshape(1, 4, 4), _frame_matrix(proj_matrix)
+        views, proj = _frame_matrix(view_matrix, device).reshape(1, 4, 4), _frame_matrix(proj_matrix, device)
         binned = None
         if hasattr(ext, "frame_binning_queued"):
             # (a frame on the matrix cores takes its lists in per-tile segments: one binning launch less)
@@ -999,7 +1000,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         ray_o = ray_o.contiguous()
         if (hasattr(ext, "frame_prologue") and ray_d.is_cuda and ray_d.dtype == torch.float32 and ray_d.dim() == 2
                 and ray_d.shape[1] == 3 and not ray_d.requires_grad and ray_o.dtype == torch.float32
-                and ray_o.shape == ray_d.shape and ray_o.is_cuda):
+                and ray_o.shape == ray_d.shape and ray_o.device == ray_d.device):
             # unit directions and the tiles' ray pyramids for the sort's culling in one launch; with
             # MLPSP_SORT_FRAME_RECORDS=1 also the sort's per-frame records (opt-in: measured 6 us per frame slower than
             # the full key evaluation on one MI355X)

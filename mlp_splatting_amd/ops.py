@@ -239,6 +239,12 @@ def _bin_scratch_bytes(n, K, W, H, tile):
     return got
 
 
+def matrices_on_device(matrices, device):
+    """Whether the binning of primitives on ``device`` can read a camera's matrices where they are."""
+    return all(m.is_cuda and m.device == device and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()
+               for m in matrices)
+
+
 def bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, W: int, H: int, tile: int, threshold: float,
                      cand_capacity: int, tile_view_ids=None, scratch_scale: int = 1, counts=None, reuse=None):
     """:func:`bin_legacy` without any host synchronisation -> (candidates [cand_capacity], tile_offsets [T+1],
@@ -251,8 +257,7 @@ def bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, W: int, 
     end of one frame and the first launch of the next)."""
     positions, log_scales = _primitives(positions, log_scales)
     dev = positions.device
-    on_device = (tile_view_ids is None and all(m.is_cuda and m.dtype == torch.float32 and m.numel() == 16 and
-                                               m.is_contiguous() for m in (view_matrices, proj_matrix)))
+    on_device = tile_view_ids is None and matrices_on_device((view_matrices, proj_matrix), dev)
     if on_device:               # one view, both matrices already on the device: nothing is brought to the host
         vm, pm = view_matrices, proj_matrix
         K = 1
@@ -306,9 +311,8 @@ def bin_segments_async(positions, log_scales, view_matrix, proj_matrix, W: int, 
     such lists with ``tile_ends``.  ``counts``, ``reuse``: as in :func:`bin_legacy_async`."""
     positions, log_scales = _primitives(positions, log_scales)
     dev = positions.device
-    for m in (view_matrix, proj_matrix):
-        if not (m.is_cuda and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()):
-            raise ValueError("view_matrix and proj_matrix must be contiguous float32 device tensors of 16 elements")
+    if not matrices_on_device((view_matrix, proj_matrix), dev):
+        raise ValueError("view_matrix and proj_matrix must be contiguous float32 device tensors of 16 elements")
     n = positions.shape[0]
     T = num_tiles(W, H, tile, tile)
     stride = int(stride)

@@ -365,8 +365,7 @@ class TileExt:
         with self._lock:
             cap, scale = self._queue_capacity, self._queue_scratch_scale
         # (not for screens whose segments would take more than 2 GiB per array: those keep the lists one after the other)
-        segments = (segments and all(m.is_cuda and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()
-                                     for m in (view_matrices, proj_matrix))
+        segments = (segments and ops.matrices_on_device((view_matrices, proj_matrix), positions.device)
                     and ops.num_tiles(int(width), int(height), 8, 8) * self.max_tile_prims <= 1 << 29)
         if cap <= 0 and not segments:
             return None

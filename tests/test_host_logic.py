@@ -333,3 +333,35 @@ def test_a_record_pool_that_cannot_run_out_takes_two_gibibytes_at_most(width, he
         else:
             assert sizes[0] == max(pairs // 4, 65_536) and worst > 2 << 30
     assert whole[0] and not whole[-1] and whole == sorted(whole, reverse=True)
+
+
+def test_matrices_of_another_device_are_brought_to_the_host(monkeypatch):
+    """The binning reads a camera's matrices in place only on the primitives' own device; of another one it would take an
+    address that means nothing there."""
+    from mlp_splatting_amd import ops
+
+    class Matrix:
+        dtype, is_cuda = torch.float32, True
+
+        def __init__(self, device):
+            self.device = torch.device(device)
+
+        def numel(self):
+            return 16
+
+        def is_contiguous(self):
+            return True
+
+        def detach(self):
+            return self
+
+        def contiguous(self):
+            return self
+    here, there = Matrix("cuda:0"), Matrix("cuda:1")
+    assert ops.matrices_on_device((here, here), torch.device("cuda:0"))
+    assert not ops.matrices_on_device((here, there), torch.device("cuda:0"))
+    assert not ops.matrices_on_device((there, here), torch.device("cuda:0"))
+    monkeypatch.setattr(cumodel.torch, "is_tensor", lambda t: isinstance(t, Matrix))
+    monkeypatch.setattr(cumodel, "_host_matrix", lambda t: "host")
+    assert cumodel._frame_matrix(here, torch.device("cuda:0")) is here
+    assert cumodel._frame_matrix(there, torch.device("cuda:0")) == "host"
