@@ -612,12 +612,17 @@ __global__ __launch_bounds__(kWideThreads) void bin_level1_fill_kernel(
 // (if not null) the largest element.  data must be 16-byte aligned.  A pass covers kScanSlabs slabs of 4096
 // elements: thread t owns elements 4t..4t+3 of every slab, so all loads and stores are coalesced 16-byte
 // accesses and the loads of a pass are independent and under no condition, where they would be waited for one by one (one
-// memory latency per pass, and one pass covers 53,248 elements).  Thread sums are scanned in the additions' own operands, the
-// elements' halves apart, so that the 256 of a wavefront fit 32 bits; a slab's 16 wavefronts by one of them.  51,000 tiles: 22 us
-// with sums in 64-bit shuffles, two passes and every wavefront adding up all others, 10 so; 1,344 tiles: 4.9, 5.5.
+// memory latency per pass, and one pass covers 65,536 elements).  Thread sums are scanned in the additions' own operands, the
+// elements' halves apart, so that the 256 of a wavefront fit 32 bits; a slab's 16 wavefronts by one of them.  16 slabs: as many as
+// the 128 registers of a workgroup of this size hold.  Kernel in us (traced; up to 4,096 tiles the lower of runs whose clocks differ),
+// with sums in 64-bit shuffles, 8 slabs and every wavefront adding up all others / so with 8 / with 16:
+//     tiles     300   1,344   4,096   5,040  12,750  20,000  32,768  40,000  51,000  53,300  60,000  100,000
+//     those     4.4     4.6     4.6     5.8     9.0    10.2    13.5    17.4    20.7    21.7    22.9     37.3
+//     8         2.8     2.9     4.0     4.1     5.8     5.8     7.0     8.6    10.0    10.4    10.9     17.2
+//     16        2.9     2.9     4.0     4.1     5.8     5.8     7.0     7.9     9.3     9.8    10.4     15.7
 // (Only the two-call binning, whose caller sizes the candidate buffer from the total, scans with a kernel of its
 // own; the asynchronous entry points place their lists inside the fill passes.)
-constexpr int kScanSlabs = 13;
+constexpr int kScanSlabs = 16;
 __device__ __forceinline__ unsigned sum_up_to_lane32(unsigned x) {
 #define MLPSP_SCAN_STEP(CTRL, ROWS) x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false)
   MLPSP_SCAN_STEP(0x111, 0xf);           // row_shr:1, 2, 4, 8

@@ -1045,9 +1045,10 @@ def test_a_feature_frame_whose_record_pool_ran_out_is_repeated(device, oracle_mo
     assert len(tried) == (2 if tile == 8 else 1) and float(want[1].mean()) > 0.05
 
 
-@pytest.mark.parametrize("columns,rows", [(1, 1), (3, 1), (64, 64), (67, 61), (208, 256), (275, 275), (417, 256)])
+@pytest.mark.parametrize("columns,rows", [(1, 1), (3, 1), (64, 64), (67, 61), (208, 256), (256, 256), (257, 255), (275, 275), (417, 256),
+                                          (512, 257)])
 def test_offsets_of_many_tiles(device, oracle_mod, columns, rows):
-    """The sums over the tiles' counts take 4,096 of them at a time and 53,248 in a pass, four to a thread: numbers of tiles that
+    """The sums over the tiles' counts take 4,096 of them at a time and 65,536 in a pass, four to a thread: numbers of tiles that
     end in, at and behind these."""
     from mlp_splatting_amd import ops, synthetic as syn
     W, H, thr = 8 * columns, 8 * rows, 1e-3
@@ -1057,4 +1058,24 @@ def test_offsets_of_many_tiles(device, oracle_mod, columns, rows):
     got, got_off = ops.bin_legacy(_t(sc.positions, device), _t(sc.log_scales, device), torch.from_numpy(view),
                                   torch.from_numpy(proj), W, H, 8, thr)
     assert len(off) == columns * rows + 1 and np.array_equal(got_off.cpu().numpy(), off)
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("columns,rows,n", [(3, 2, 70_000), (5, 1, 140_000), (2, 2, 65_536)])
+def test_offsets_of_tiles_with_long_lists(device, oracle_mod, columns, rows, n):
+    """Counts of 65,536 and more: both halves of the elements that the sums over tiles add apart, in a slab's whole fours and
+    behind them."""
+    from mlp_splatting_amd import ops, synthetic as syn
+    W, H, thr = 8 * columns, 8 * rows, 1e-3
+    rng = np.random.default_rng(n)
+    pos = (np.array([0.0, 0.0, 4.0]) + rng.uniform(-0.1, 0.1, (n, 3))).astype(np.float32)
+    logs = np.full((n, 3), 1.0, np.float32)              # as wide as the image
+    logs[rng.random(n) < 1e-3] = -9.0                    # a few to some tiles only
+    view, proj = syn.view_matrix(syn.look_at((0.0, 0.0, 0.0), (0.0, 0.0, 1.0)))[None], syn.projection_matrix(0.5 * W, W, H)
+    want, off = oracle_mod.bin_legacy(pos, logs, view, proj, W, H, 8, thr)
+    counts = np.diff(off)
+    assert counts.max() >= (65_536 if n > 65_536 else 65_000) and (n == 65_536 or len(np.unique(counts)) > 1)
+    got, got_off, longest = ops.bin_legacy(_t(pos, device), _t(logs, device), torch.from_numpy(view), torch.from_numpy(proj), W, H,
+                                           8, thr, with_longest=True)
+    assert np.array_equal(got_off.cpu().numpy(), off) and int(longest) == counts.max()
     assert np.array_equal(got.cpu().numpy(), want)
