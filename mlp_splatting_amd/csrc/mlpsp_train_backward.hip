@@ -6,7 +6,8 @@
 // length.  A workgroup walks one chunk; where the primitive changes it writes its sums: straight to the gradients if the
 // primitive's steps all lie in the chunk, else to the chunk's tail row (the primitive goes on in the next chunk) or head row
 // (it ended here).  One more launch adds the rows of the primitives that span chunks; the zeros of those without a step are
-// written by the weight gradient kernels too, or by a launch of their own where these have few wavefronts (kZeroShare32).  No atomics, a fixed order of every sum.
+// written by the weight gradient kernels too, or by a launch of their own where these have few wavefronts (kZeroShare32).  No
+// atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
 // 0.12 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
@@ -95,8 +96,8 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
 // ---------------------------------------------------------------------------------------------
 // steps sorted by primitive: a stable radix sort of the S primitive numbers in tile order, in digits of equal width (two of
 // nine bits at 200,000 primitives).  A wavefront takes an eighth of its block's steps in rounds of 64, whose equal digits are
-// found with a ballot per bit.  Eight launches, 120 us at 650,000 steps (the two sums over blocks x digits, one workgroup
-// each, 27 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
+// found with a ballot per bit.  Eight launches, 110 us at 650,000 steps (the two sums over blocks x digits, one workgroup
+// each, 17 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSortBlock = 512, kSortBits = 10;
 // Steps of a block: 8,192, a quarter of that where this would leave a chip of 256 CUs fewer than 32 blocks (16 rounds one
@@ -131,9 +132,14 @@ __global__ __launch_bounds__(kSortBlock) void step_hist_kernel(const int32_t* __
   for (int d = threadIdx.x; d < R; d += kSortBlock) hist[d * blocks + blockIdx.x] = s_count[d];
 }
 
-// exclusive sums of n counts, in place; one workgroup, kSumRounds of 4,096 counts behind one barrier: a round at a time, its
-// loads and two barriers one after the other, the 40,960 counts of 650,000 steps took 26 us instead of 14
-constexpr int kSumRounds = 10;           // what 650,000 steps have
+// exclusive sums of n counts, in place; one workgroup, kSumRounds of 4,096 counts behind one barrier.  Us a launch (traced,
+// 200,000 primitives), a round at a time, its loads and two barriers one after the other / 6 / 10 / 16 rounds:
+//     steps    1,600   80,000  250,000  650,000  750,000  1,000,000  1,300,000  2,000,000
+//     one        2.1     12.9     37.4     24.3     28.2       36.6       47.2       70.3
+//     6          2.7      4.7     12.6      8.3      9.4       12.4       15.5       23.2
+//     10         3.2      4.9     12.5      8.3     10.5       12.4       15.0       23.7
+//     16         3.9      5.6     11.9      8.2      9.4       11.8       15.9       21.4
+constexpr int kSumRounds = 6;
 __global__ __launch_bounds__(1024) void step_sums_kernel(int32_t* __restrict__ v, int n) {
   __shared__ int s_wave[2][kSumRounds * 16];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;

@@ -347,8 +347,13 @@ inline TrainPlan train_plan(int ntx, int nty, int64_t T) {
 constexpr int64_t kScanShare = 768 * 1024;
 
 // tile_base = exclusive sums of tile_steps, head[2] = their total; one workgroup, four tiles to a thread and up to 16,384 behind
-// one barrier, their counts on the way together (12,750 tiles: consecutive ones to a thread, one load
-// after the other, 14.9 us; so 6.4).
+// one barrier, their counts on the way together.  Us (traced), consecutive tiles to a thread, one load after the other / 2 / 4 / 8
+// rounds behind a barrier:
+//     tiles     300   1,200   4,096  12,750  16,500  20,000  32,768  51,000  100,000
+//     that      3.9     5.9     6.0    14.1    20.4    26.9    59.2    92.8    206.1
+//     2         3.9     5.9     6.0     6.1     7.8     8.0    10.6    16.5     29.6
+//     4         3.8     5.9     5.9     6.0     8.6     8.7     9.7    15.9     27.2
+//     8         6.4     7.6     7.7     8.4     8.9     9.0     9.5    15.6     28.1
 __global__ __launch_bounds__(1024) void step_scan_kernel(const int32_t* __restrict__ tile_steps, int T,
                                                          int32_t* __restrict__ tile_base, int32_t* __restrict__ head) {
   constexpr int kRounds = 4;
