@@ -422,7 +422,8 @@ def test_the_reverse_walk_of_tiles_of_every_length(device, lengths):
 @pytest.mark.parametrize("n,tiles,listed", [(2, 1, 1), (40, 700, 40), (70_000, 700, 40), (600_000, 1030, 80)])
 def test_steps_are_sorted_by_primitive(device, n, tiles, listed):
     """The stable sort of a frame's steps, with fewer counts than the sums over blocks and digits take at a time (4,096), with
-    several times and, at 600,000 primitives and 82,400 steps, with more than ten times as many (41 blocks x 1,024 digits)."""
+    several times and, at 600,000 primitives and 82,400 steps, with more than ten times as many (41 blocks x 1,024 digits),
+    which are two turns of six."""
     import numpy as np
     from mlp_splatting_amd import ops, synthetic as syn
     from mlp_splatting_amd.tile_ext import TileExt
@@ -449,22 +450,22 @@ def test_steps_are_sorted_by_primitive(device, n, tiles, listed):
     assert (first == np.searchsorted(prim, np.arange(n + 1))).all()
 
 
-@pytest.mark.parametrize("columns", [3, 2100])
-def test_the_forward_looks_for_what_is_not_finite(device, columns):
-    """By its wavefronts behind their tiles (2,100 tiles, most in teams, which do not look) or in a launch of its own: every
-    element of arrays that begin at any float and of every length around a wavefront's and a workgroup's reach, the first and
-    the last ones among them; a flag that is set stays set."""
+@pytest.mark.parametrize("columns,rows", [(3, 1), (2100, 1), (50, 42)])
+def test_the_forward_looks_for_what_is_not_finite(device, columns, rows):
+    """By its wavefronts behind their tiles (2,100 tiles in a row, of which 244 go to teams, which do not look, and 50x42, of which
+    all but 248 do) or, of 3 tiles, in a launch of its own: every element of arrays that begin at any float and of every length around a
+    wavefront's and a workgroup's reach, the first and the last ones among them; a flag that is set stays set."""
     from mlp_splatting_amd import ops, synthetic as syn
     from mlp_splatting_amd.tile_ext import TileExt
-    n, width, height = 40, 8 * columns, 8
+    n, tiles, width, height = 40, columns * rows, 8 * columns, 8 * rows
     sc = syn.make_scene(n, 32, seed=4, log_scale_mean=-1.0)
     ro, rd = syn.pinhole_rays(width, height, 60.0, syn.look_at((0.0, 0.0, -3.0), (0.0, 0.0, 5.0)))
     base = [to_dev(a, device) for a in (ro, syn.normalize_rays(rd), sc.positions, sc.log_scales, sc.quats)]
-    order = torch.arange(n, dtype=torch.int32, device=device).repeat(columns)
-    offsets = torch.arange(columns + 1, dtype=torch.int32, device=device) * n
+    order = torch.arange(n, dtype=torch.int32, device=device).repeat(tiles)
+    offsets = torch.arange(tiles + 1, dtype=torch.int32, device=device) * n
     freq, att, ws = to_dev(sc.freq, device), to_dev(sc.att, device), [to_dev(w, device) for w in sc.mlp()]
     records, packed = ops.prepare_primitives(*base[2:5]), ops.pack_mfma_weights(*ws, bf16=False)
-    pool = columns * n + 32 * columns
+    pool = tiles * n + 32 * tiles
     arrays = [torch.ones(length + 3, device=device)[shift:shift + length]
               for length, shift in ((1, 0), (3, 1), (63, 2), (257, 3), (4 * 64 + 1, 0), (70_001, 1), (3_000_000, 2), (0, 0))]
 
