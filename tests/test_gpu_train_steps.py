@@ -453,8 +453,8 @@ def test_steps_are_sorted_by_primitive(device, n, tiles, listed):
 @pytest.mark.parametrize("columns,rows", [(3, 1), (2100, 1), (50, 42)])
 def test_the_forward_looks_for_what_is_not_finite(device, columns, rows):
     """By its wavefronts behind their tiles (2,100 tiles in a row, of which 244 go to teams, which do not look, and 50x42, of which
-    all but 248 do) or, of 3 tiles, in a launch of its own: every element of arrays that begin at any float and of every length around a
-    wavefront's and a workgroup's reach, the first and the last ones among them; a flag that is set stays set."""
+    all but 248 do) or, of 3 tiles, in a launch of its own: every element of arrays that begin at any float and of every length
+    around a wavefront's and a workgroup's reach, the first and the last ones among them; a flag that is set stays set."""
     from mlp_splatting_amd import ops, synthetic as syn
     from mlp_splatting_amd.tile_ext import TileExt
     n, tiles, width, height = 40, columns * rows, 8 * columns, 8 * rows
