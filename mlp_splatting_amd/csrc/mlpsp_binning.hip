@@ -623,17 +623,6 @@ __global__ __launch_bounds__(kWideThreads) void bin_level1_fill_kernel(
 // (Only the two-call binning, whose caller sizes the candidate buffer from the total, scans with a kernel of its
 // own; the asynchronous entry points place their lists inside the fill passes.)
 constexpr int kScanSlabs = 16;
-__device__ __forceinline__ unsigned sum_up_to_lane32(unsigned x) {
-#define MLPSP_SCAN_STEP(CTRL, ROWS) x += (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false)
-  MLPSP_SCAN_STEP(0x111, 0xf);           // row_shr:1, 2, 4, 8
-  MLPSP_SCAN_STEP(0x112, 0xf);
-  MLPSP_SCAN_STEP(0x114, 0xf);
-  MLPSP_SCAN_STEP(0x118, 0xf);
-  MLPSP_SCAN_STEP(0x142, 0xa);           // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
-  MLPSP_SCAN_STEP(0x143, 0xc);
-#undef MLPSP_SCAN_STEP
-  return x;
-}
 __global__ __launch_bounds__(1024) void exclusive_scan_kernel(int32_t* __restrict__ data, int n,
                                                               long long* __restrict__ total,
                                                               long long* __restrict__ largest) {
@@ -663,7 +652,7 @@ __global__ __launch_bounds__(1024) void exclusive_scan_kernel(int32_t* __restric
       if (pass0 + u * 4096 >= full) break;
       const unsigned low = (v[u].x & 0xffff) + (v[u].y & 0xffff) + (v[u].z & 0xffff) + (v[u].w & 0xffff);
       const unsigned high = (v[u].x >> 16) + (v[u].y >> 16) + (v[u].z >> 16) + (v[u].w >> 16);
-      incl[u] = sum_up_to_lane32(low) + ((long long)sum_up_to_lane32(high) << 16);
+      incl[u] = sum_up_to_lane<false>(low) + ((long long)sum_up_to_lane<false>(high) << 16);
       if (lane == 63) s_wave[u][wave] = incl[u];
     }
     __syncthreads();

@@ -22,6 +22,27 @@ constexpr float kInvalidKey = 1e30f;          // sort key of primitives behind t
 __device__ __forceinline__ float bits_to_float(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t float_to_bits(float x) { return __float_as_uint(x); }
 
+// Lane l's sum of the first l + 1 lanes' words (of its half's, with HALF), and the whole wavefront's in its last lane: in the
+// operands of the additions themselves, not through LDS with an address per step.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t from_lane(uint32_t otherwise, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)otherwise, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t plus(uint32_t x, uint32_t y) { return x + y; }
+__device__ __forceinline__ float plus(float x, uint32_t y) { return x + bits_to_float(y); }
+__device__ __forceinline__ uint32_t word_of(uint32_t x) { return x; }
+__device__ __forceinline__ uint32_t word_of(float x) { return float_to_bits(x); }
+template <bool HALF, typename V>
+__device__ __forceinline__ V sum_up_to_lane(V x) {
+  x = plus(x, from_lane<0x111, 0xf>(0u, word_of(x)));      // row_shr:1, 2, 4, 8: within 16 lanes
+  x = plus(x, from_lane<0x112, 0xf>(0u, word_of(x)));
+  x = plus(x, from_lane<0x114, 0xf>(0u, word_of(x)));
+  x = plus(x, from_lane<0x118, 0xf>(0u, word_of(x)));
+  x = plus(x, from_lane<0x142, 0xa>(0u, word_of(x)));      // row_bcast:15 into rows 1 and 3
+  if constexpr (!HALF) x = plus(x, from_lane<0x143, 0xc>(0u, word_of(x)));  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 // e^x: x < -87 -> 0, x > 88 -> +inf, NaN -> NaN.  k = rint(x log2 e), r = x - k ln2 in two
 // parts, degree-7 Taylor polynomial, scaling by 2^k through the exponent field.
 __device__ __forceinline__ float det_exp(float x) {

@@ -254,6 +254,8 @@ MLPSP_API int mlpsp_render_tilecenter_feat_f32(
   // primitives in us, 128 channels reckoned / as here (96 channels, the same kernel on both sides: 962 / 962):
   //    16 channels   957 / 914      40   960 / 909      64   959 / 915      67   961 / 922      72   960 / 926      80   960 / 930
   //    800x640 and 100,000:  33   3,506 / 3,452      70   3,510 / 3,314
+  // Above, 32 channels behind the 64th, two pixels at a time, are no faster than 64: 84, 88 and 96 channels 1,136 / 1,150, 1,141 /
+  // 1,160 and 1,141 / 1,146 at 30,000 primitives, 3,556 / 3,611, 3,544 / 3,617 and 3,565 / 3,615 at 100,000.
 #define MLPSP_ACC_GO(SL)                                          \
   do {                                                            \
     if (!sixteen) MLPSP_ACC_LAUNCH(SL, 32, 2, 0);                 \

@@ -28,22 +28,7 @@ namespace mlpsp {
 constexpr int kSortThreads = 256;
 constexpr int kRankPairsMax = 64 * 1024;   // in-bucket comparisons beyond which the sorting network is used instead
 
-// Lane l's sum of the first l + 1 lanes' words (the first 32 lanes', with HALF), and the smallest and the largest word of a
-// wavefront in its last lane: in the operands of the additions themselves, not through LDS with an address per step.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t from_lane(uint32_t otherwise, uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)otherwise, (int)x, CTRL, ROWS, 0xf, false);
-}
-template <bool HALF>
-__device__ __forceinline__ uint32_t sum_up_to_lane(uint32_t x) {
-  x += from_lane<0x111, 0xf>(0u, x);                     // row_shr:1, 2, 4, 8: within 16 lanes
-  x += from_lane<0x112, 0xf>(0u, x);
-  x += from_lane<0x114, 0xf>(0u, x);
-  x += from_lane<0x118, 0xf>(0u, x);
-  x += from_lane<0x142, 0xa>(0u, x);                     // row_bcast:15 into rows 1 and 3
-  if constexpr (!HALF) x += from_lane<0x143, 0xc>(0u, x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
+// The smallest and the largest word of a wavefront, in its last lane (as sum_up_to_lane).
 __device__ __forceinline__ void range_in_last_lane(uint32_t& lo, uint32_t& hi) {
 #define MLPSP_RANGE_STEP(CTRL, ROWS)                 \
   lo = min(lo, from_lane<CTRL, ROWS>(0xffffffffu, lo)); \

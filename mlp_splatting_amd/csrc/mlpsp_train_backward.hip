@@ -341,19 +341,6 @@ __device__ __forceinline__ void geometry_store(const float v[15], float qw, floa
                         r12 * (2.f * qy) + r20 * (2.f * qx) + r21 * (2.f * qy);
 }
 
-// The wavefront's sum, in its last lane: row_shr 1, 2, 4 and 8, then row_bcast 15 and 31, in the additions' own operands.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float plus_lane(float v) {
-  return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ float sum_in_last_lane(float v) {
-  v = plus_lane<0x111, 0xf>(v);
-  v = plus_lane<0x112, 0xf>(v);
-  v = plus_lane<0x114, 0xf>(v);
-  v = plus_lane<0x118, 0xf>(v);
-  v = plus_lane<0x142, 0xa>(v);
-  return plus_lane<0x143, 0xc>(v);
-}
 // A workgroup per chunk, the steps of a run to its wavefronts in turn.  Bound by memory (1,280 bytes a step) where there are many
 // steps, by the chain of look-ups, loads and sums of a run where there are few: a lane knows where a step lies, four steps are asked
 // for together, and a run's 15 sums do not go through LDS.  650,000 steps: 185 -> 174 us, 4.8 TB/s; 80,000: 36 -> 28.
@@ -406,7 +393,7 @@ __global__ __launch_bounds__(64 * kGeoWaves) void train_geometry_kernel(
       }
     }
 #pragma unroll
-    for (int k = 0; k < 15; ++k) v[k] = sum_in_last_lane(v[k]);
+    for (int k = 0; k < 15; ++k) v[k] = sum_up_to_lane<false>(v[k]);      // (the last lane has all)
     if (l == 63) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
