@@ -112,7 +112,7 @@ def _unit_directions(ray_d):
 def _frame_matrix(t, device):
     """The matrix as a queued frame on ``device`` takes it: a float32 tensor of that device stays where it is (the
     binning reads it there; no copy to the host, no synchronisation), anything else becomes a host copy."""
-    if torch.is_tensor(t) and t.device == device and t.is_cuda and t.dtype == torch.float32 and t.numel() == 16:
+    if torch.is_tensor(t) and t.get_device() == device.index and t.dtype == torch.float32 and t.numel() == 16:
         return t.detach().contiguous()
     return _host_matrix(t)
 
@@ -453,6 +453,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     """
 
     requires_full_image = True
+    camera_mode = "legacy-centered"      # or "colmap-native", of an instance or a subclass: lists from ray cones
 
     def __init__(self, num_primitives=1024, hidden_dim=32, pe_frequencies=6, initial_positions=None,
                  use_integrated_pe=True, pe_sigma: float = 0.01, min_points: int = 10, tile_size: int = 8,
@@ -642,7 +643,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def build_tilecenter_culling_from_tile_views(self, tile_view_ids, view_matrices, proj_matrix,
                                                  score_threshold: float = 1e-3, tile_size: int | None = None):
         """Tile lists when every tile takes its rays from one of K views (scannet/cumodel.py:838-949)."""
-        if self._native_camera():
+        if self.camera_mode == "colmap-native":
             return None, None
         if self.image_size is None:
             raise ValueError("image_size must be set before building tile culling.")
@@ -688,20 +689,13 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
                 memo[key] = hit
         return hit[:3]
 
-    def _native_camera(self):
-        """Whether ``camera_mode``, of the instance or of its class, asks for lists from ray cones.  (getattr with a default on
-        a module that lacks the name walks parameters, buffers and submodules first.)"""
-        if "camera_mode" not in self.__dict__ and not hasattr(type(self), "camera_mode"):
-            return False
-        return self.camera_mode == "colmap-native"
-
     def _tile_lists(self, ray_o, ray_d, score_threshold, view_matrix, proj_matrix, culled_prim_indices, tile_offsets,
                     device, allow_native=True):
         W, H = self.image_size
         tile_size = int(self.tile_size)
         num_tiles = ops.num_tiles(W, H, tile_size, tile_size)
         external = (culled_prim_indices is not None) or (tile_offsets is not None)
-        if allow_native and self._native_camera():
+        if allow_native and self.camera_mode == "colmap-native":
             if external:
                 raise ValueError("Native camera culling must be derived from the actual rays")
             culled_prim_indices, tile_offsets = ray_cone_candidates(
@@ -775,7 +769,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
             plain = self.__dict__
             own_lists = (culled_prim_indices is None and tile_offsets is None and view_matrix is not None
                          and proj_matrix is not None
-                         and not self._native_camera())
+                         and self.camera_mode != "colmap-native")
             with_feat = return_feature and self.feat_attr is not None
             if (own_lists and use_tilecenter and ts == 8 and (with_feat or not return_feature)
                     and feature_target is None and plain.get("queued_frames", True)
@@ -853,7 +847,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         ext, plain = self._ensure_tile_ext(), self.__dict__
         W, H = self.image_size
         own = (culled_prim_indices is None and tile_offsets is None and view_matrix is not None and proj_matrix is not None
-               and not self._native_camera())
+               and self.camera_mode != "colmap-native")
         queued = None
         if own and keeps_steps and plain.get("queued_frames", True) and hasattr(ext, "train_lists_queued"):
             def again():
@@ -1052,7 +1046,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
         eligible = (frames_in_flight > 1 and len(frames) > 1 and self.image_size is not None
                     and self._resolve_tile_order_mode() == "tilecenter" and int(self.tile_size) == 8
                     and (with_feat or not return_feature) and plain.get("queued_frames", True)
-                    and not self._native_camera()
+                    and self.camera_mode != "colmap-native"
                     and str(getattr(self, "render_precision", "f32")).lower() in {"bf16", "fp16"}
                     and all(f[2] is not None and f[3] is not None and f[0].shape[0] == W * H for f in frames))
         if not eligible:
@@ -1125,7 +1119,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def render_rgb_alpha_no_grad(self, ray_o, ray_d, score_threshold: float = 1e-3, bg_color=None, view_matrix=None,
                                  proj_matrix=None, collect_w_stats: bool = False, gt_rgb=None):
         """(rgb, alpha) under the tile-centre pipeline (scannet/cumodel.py:1196-1383)."""
-        if self._native_camera():
+        if self.camera_mode == "colmap-native":
             raise NotImplementedError("Native camera statistics rendering is not implemented; use forward for RGB/features")
         if self.image_size is None:
             raise ValueError("image_size must be set on NeuralPrimitiveSceneTileCUDA before calling render_rgb_alpha_no_grad.")
@@ -1160,7 +1154,7 @@ class NeuralPrimitiveSceneTileCUDA(nn.Module):
     def render_rgb_t_no_grad(self, ray_o, ray_d, score_threshold: float = 1e-3, bg_color=None, view_matrix=None,
                              proj_matrix=None):
         """(rgb, t, alpha) with t the expected depth (scannet/cumodel.py:1385-1525)."""
-        if self._native_camera():
+        if self.camera_mode == "colmap-native":
             raise NotImplementedError("Native camera depth rendering is not implemented; use forward for RGB/features")
         if self.image_size is None:
             raise ValueError("image_size must be set on NeuralPrimitiveSceneTileCUDA before calling render_rgb_t_no_grad.")

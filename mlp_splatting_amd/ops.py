@@ -241,8 +241,11 @@ def _bin_scratch_bytes(n, K, W, H, tile):
 
 def matrices_on_device(matrices, device):
     """Whether the binning of primitives on ``device`` can read a camera's matrices where they are."""
-    return all(m.is_cuda and m.device == device and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()
-               for m in matrices)
+    index = device.index
+    for m in matrices:          # (get_device: -1 of a tensor in host memory; a frame's first launch waits for this)
+        if not (m.get_device() == index and m.dtype == torch.float32 and m.numel() == 16 and m.is_contiguous()):
+            return False
+    return True
 
 
 def bin_legacy_async(positions, log_scales, view_matrices, proj_matrix, W: int, H: int, tile: int, threshold: float,

@@ -341,10 +341,13 @@ def test_matrices_of_another_device_are_brought_to_the_host(monkeypatch):
     from mlp_splatting_amd import ops
 
     class Matrix:
-        dtype, is_cuda = torch.float32, True
+        dtype = torch.float32
 
-        def __init__(self, device):
-            self.device = torch.device(device)
+        def __init__(self, index):
+            self.index = index
+
+        def get_device(self):
+            return self.index
 
         def numel(self):
             return 16
@@ -357,11 +360,13 @@ def test_matrices_of_another_device_are_brought_to_the_host(monkeypatch):
 
         def contiguous(self):
             return self
-    here, there = Matrix("cuda:0"), Matrix("cuda:1")
+    here, there, host = Matrix(0), Matrix(1), Matrix(-1)
     assert ops.matrices_on_device((here, here), torch.device("cuda:0"))
     assert not ops.matrices_on_device((here, there), torch.device("cuda:0"))
     assert not ops.matrices_on_device((there, here), torch.device("cuda:0"))
+    assert not ops.matrices_on_device((host, here), torch.device("cuda:0"))
     monkeypatch.setattr(cumodel.torch, "is_tensor", lambda t: isinstance(t, Matrix))
     monkeypatch.setattr(cumodel, "_host_matrix", lambda t: "host")
     assert cumodel._frame_matrix(here, torch.device("cuda:0")) is here
     assert cumodel._frame_matrix(there, torch.device("cuda:0")) == "host"
+    assert cumodel._frame_matrix(host, torch.device("cuda:0")) == "host"
