@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256) void frame_prologue_kernel(const float* __rest
 //   ... and records asked for in their own round, eight wavefronts per SIMD                                      80
 //   ... and sums and ranges in the operands of the additions instead of through LDS, culled entries counted alone 75
 //   ... and the pyramid in vector registers, out of LDS every round                                              71
-// 641x479, 50,000 primitives: 46 -> 36; 800x450, 100,000: 51 -> 39; 2400x1360 without records of the pyramids: 138 -> 108.
+// The first of these and the last as traced, on another box: 90 -> 70 (78 to 88 on others, and behind a training step's kernels);
+// 641x479, 50,000 primitives, 47 -> 37.5; 2400x1360 without records of the pyramids 168 -> 132.
 template <bool PYR, bool ASC = false>
 __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(ASC ? 8 : 7))) void sort_tiles_kernel(
     const float* __restrict__ rays_o, const float* __restrict__ rays_d, const PrimRecord* __restrict__ prims,

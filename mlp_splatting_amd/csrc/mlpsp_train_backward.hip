@@ -10,7 +10,7 @@
 // atomics, a fixed order of every sum.
 //
 // Measured at 200,000 primitives, 1200x680, f32, against the record pipeline (ms): reverse 0.47 (1.8), sort and grouping
-// 0.12 (sort 1.7, gathers 2.85), geometry 0.17 (1.3), weight gradients and zeros 5.1 + 0.24 (12.8 and 0.8), joining rows 0.03.
+// 0.11 (sort 1.7, gathers 2.85), geometry 0.16 (1.3), weight gradients with the zeros beside them 5.1 (12.8 and 0.8), joining rows 0.04.
 #include "mlpsp_device.hpp"
 #include "mlpsp_host.hpp"
 #include "mlpsp_mlp_mfma32.hpp"
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64) void train_reverse_kernel(
 // steps sorted by primitive: a stable radix sort of the S primitive numbers in tile order, in digits of equal width (two of
 // nine bits at 200,000 primitives).  A wavefront takes an eighth of its block's steps in rounds of 64, whose equal digits are
 // found with a ballot per bit.  Eight launches, 110 us at 650,000 steps (the two sums over blocks x digits, one workgroup
-// each, 17 of them, the two scatters 60); the library's sort took 22 launches and 200 us with the gather behind it.
+// each, 18 of them, the two scatters 58); the library's sort took 22 launches and 200 us with the gather behind it.
 // ---------------------------------------------------------------------------------------------
 constexpr int kSortBlock = 512, kSortBits = 10;
 // Steps of a block: 8,192, a quarter of that where this would leave a chip of 256 CUs fewer than 32 blocks (16 rounds one
@@ -477,7 +477,7 @@ __device__ __forceinline__ void walk_halves(const int4& where, StepRecord next, 
 // the stores go on beside the products of the others.  The whole call at 648,000 steps of 200,000 primitives with these 2.8 GB in
 // a launch behind it / here / here past the caches: f32 5.54 / 5.31 / 5.30 ms, fp16 1.94 / 1.74 / 1.70; a primitive per block of
 // products 5.34 and 1.83.  Ahead of the chunk its first record is waited for behind the stores: the f32 kernel of 80,000 steps
-// takes 676 us instead of 663.  With the rows of the attributes' gradient (512 channels, four slots: 1.3 GB more) fp16 1.52 -> 1.62.
+// takes 676 us instead of 663.  With the rows of the attributes' gradient (512 channels, four slots: 1.6 GB more) fp16 1.52 -> 1.62.
 // What a wavefront may be given of them: few steps make few chunks, and the four wavefronts of one would store all rows alone
 // (16 steps of 200,000 primitives 56 ms, in a launch of their own 0.7).  Above it that launch, behind the gradients.  Call in us,
 // a launch / here, at KB per wavefront:
