@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) void frame_prologue_kernel(const float* __rest
 //   ... and records asked for in their own round, eight wavefronts per SIMD                                      80
 //   ... and sums and ranges in the operands of the additions instead of through LDS, culled entries counted alone 75
 //   ... and the pyramid in vector registers, out of LDS every round                                              71
-// The first of these and the last as traced, on another box: 90 -> 70 (78 to 88 on others, and behind a training step's kernels);
+// The first of these and the last as traced, on another card: 90 -> 70 (78 to 88 on others, and behind a training step's kernels);
 // 641x479, 50,000 primitives, 47 -> 37.5; 2400x1360 without records of the pyramids 168 -> 132.
 template <bool PYR, bool ASC = false>
 __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(ASC ? 8 : 7))) void sort_tiles_kernel(
